@@ -10,8 +10,8 @@
 //   loads, so a wave streams 64*16 B of K (then V) per step; all G = Hq/Hkv query heads of the kv
 //   head are scored from the same K/V bytes (GQA packing: K/V are read once per kv head, not per q
 //   head). Online softmax in the log2 domain; partitions merge in attn_decode_reduce.
-// prefill (varlen, causal, paged context incl. cached prefix): flash-attention forward on MFMA
-//   16x16x32 bf16. A workgroup holds 16 query rows x up to 8 query heads of one kv head (one wave per
+// prefill (varlen, causal, paged context incl. cached prefix): attention_flash.hip; here the form for head dim
+//   256 (and the V^T image): flash-attention forward on MFMA 16x16x32 bf16. A workgroup holds 16 query rows x up to 8 query heads of one kv head (one wave per
 //   head) so every K/V tile staged in LDS is reused by all heads of the group. K is stored
 //   XOR-swizzled for conflict-free ds_read_b128 B-fragments; V is read with ds_read_b64_tr_b16
 //   (hardware transpose) from a region-swizzled image; P goes register -> LDS -> A-fragment.
@@ -754,11 +754,8 @@ extern "C" int mxk_attn_decode_mfma(const bf16_t* q, int q_stride, const void* k
     return (int)hipErrorInvalidValue;
 }
 
-// KSP = 2 (key split, GW = 4 only: 8 waves): two groups of GW waves share the workgroup's 16 query rows x GW heads and take alternate
-// 64-key tiles (each group stages its own K / V tile), then merge (m, l, O) through LDS. A short prompt chunk runs
-// only ~n_tiles x Hq / GW workgroups (136 for a 270-token chunk of Llama-3-8B, fewer than the CUs), each walking
-// its causal key range one tile at a time: the split halves the longest walk.
-template <int D, int GW, int VT, bool F16, int KVF, int KSP = 1>
+// What attention_flash.hip does not take: head dim 256, and the V^T image (VT = 1, `vmode`) of any head dim.
+template <int D, int GW, int VT, bool F16, int KVF>
 __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restrict__ q,
                                                            const void* __restrict__ kc,
                                                            const void* __restrict__ vc,
@@ -769,10 +766,8 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
                                                            const int* __restrict__ ctx_lens, int Hq, int Hkv,
                                                            int G, int bs, float scale, int window, float softcap,
                                                            bf16_t* __restrict__ out) {
-    static_assert(KSP == 1 || GW == 4, "key split: 2 x 4 waves (the 512-thread launch bound)");
-    constexpr int NWG = GW >= 3 ? GW : 4;     // waves per key group
-    constexpr int NW = NWG * KSP;             // waves per workgroup
-    constexpr int RT = NWG / GW;              // 16-row query tiles per workgroup
+    constexpr int NW = GW >= 3 ? GW : 4;      // waves per workgroup
+    constexpr int RT = NW / GW;               // 16-row query tiles per workgroup
     constexpr int KT = 64;                    // keys per tile
     constexpr int KBYTES = KT * D * 2;
     constexpr int PSTRIDE = (KT + 8) * 2;     // bytes per P row (padded)
@@ -780,19 +775,18 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
     constexpr int VBYTES = VT ? D * VTSTRIDE : KBYTES;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int ksp = KSP > 1 ? wave / NWG : 0;  // key group
-    char* k_lds = smem + ksp * (KBYTES + VBYTES);
+    char* k_lds = smem;
     char* v_lds = k_lds + KBYTES;
-    char* p_lds = smem + KSP * (KBYTES + VBYTES);
-    constexpr int NT_C = NWG * 64;             // threads staging one group's tile
-    const int tid = threadIdx.x - ksp * NT_C;
+    char* p_lds = v_lds + VBYTES;
+    constexpr int NT_C = NW * 64;              // threads staging a tile
+    const int tid = threadIdx.x;
     const int g = lane >> 4, col = lane & 15;
     const int tile = blockIdx.x;
     const int s = tile_seq[tile], q0 = tile_q0[tile];
     if (s < 0) return;  // padding tile of a graph-captured step (uniform across the workgroup)
     const int hq = blockIdx.y * GW + (wave % GW);
     const int kvh = (blockIdx.y * GW) / G;
-    const int rt = KSP > 1 ? 0 : wave / GW;
+    const int rt = wave / GW;
     const int qbeg = cu_q[s], qlen = cu_q[s + 1] - qbeg;
     const int ctx = ctx_lens[s];
     const int pos_off = ctx - qlen;  // position of query 0
@@ -884,21 +878,12 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
             }
         }
     };
-    // key group ksp takes tiles kt_begin + KT (ksp + KSP r); every group runs the same number of rounds (the
-    // barriers below are workgroup-wide), a group past the end idles through its last round
-    const int n_rounds = kv_end > kt_begin ? (kv_end - kt_begin + KSP * KT - 1) / (KSP * KT) : 0;
-    if (kt_begin + ksp * KT < kv_end) load_tile(kt_begin + ksp * KT);
-    for (int r = 0; r < n_rounds; ++r) {
-        const int kt0 = kt_begin + (KSP * r + ksp) * KT;
-        const bool live = kt0 < kv_end;
+    if (kt_begin < kv_end) load_tile(kt_begin);
+    for (int kt0 = kt_begin; kt0 < kv_end; kt0 += KT) {
         // ---- stage this K and V tile (64 keys x D), then request the next one ----
-        if (live) store_tile();
-        if (kt0 + KSP * KT < kv_end) load_tile(kt0 + KSP * KT);
+        store_tile();
+        if (kt0 + KT < kv_end) load_tile(kt0 + KT);
         __syncthreads();
-        if (!live) {
-            __syncthreads();
-            continue;
-        }
         // ---- S = Q K^T : 16 rows x 64 keys ----
         f32x4 sacc[4];
 #pragma unroll
@@ -983,33 +968,6 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
         }
         __syncthreads();
     }
-    if constexpr (KSP > 1) {
-        // ---- merge the key groups: group 1 parks (m, l, O) in the freed tile buffers, group 0 combines ----
-        float* mo = (float*)smem + (wave % GW) * (16 * D + 32);  // [16 rows][D] O, then m[16], l[16]
-        if (ksp == 1) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-#pragma unroll
-                for (int nt = 0; nt < D / 16; ++nt) mo[(4 * g + i) * D + 16 * nt + col] = oacc[nt][i];
-                if (col == 0) {
-                    mo[16 * D + 4 * g + i] = mrow[i];
-                    mo[16 * D + 16 + 4 * g + i] = lrow[i];
-                }
-            }
-        }
-        __syncthreads();
-        if (ksp == 1) return;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float m1 = mo[16 * D + 4 * g + i], l1 = mo[16 * D + 16 + 4 * g + i];
-            const float mn = fmaxf(mrow[i], m1);
-            const float a0 = mn == -INFINITY ? 0.f : exp2f(mrow[i] - mn), a1 = mn == -INFINITY ? 0.f : exp2f(m1 - mn);
-            lrow[i] = lrow[i] * a0 + l1 * a1;
-#pragma unroll
-            for (int nt = 0; nt < D / 16; ++nt)
-                oacc[nt][i] = oacc[nt][i] * a0 + mo[(4 * g + i) * D + 16 * nt + col] * a1;
-        }
-    }
     // ---- write O / l ----
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -1022,21 +980,21 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
     }
 }
 
-template <int D, int GW, int VT, int KVF, int KSP = 1>
+template <int D, int GW, int VT, int KVF>
 static void launch_prefill_t(dim3 grid, int threads, size_t lds, const bf16_t* q, const void* kc, const void* vc,
                              const int* bt, int bt_stride, const int* tile_seq, const int* tile_q0, const int* cu_q,
                              const int* ctx_lens, int Hq, int Hkv, int bs, float scale, int window, float softcap,
                              bf16_t* out, hipStream_t st) {
     MX_ACT_DISPATCH({
-        if (lds > 65536) {  // D=256 tiles / key-split tiles (73-82 KB): opt in to the large LDS allocation once
+        if (lds > 65536) {  // D=256 tiles (73-82 KB): opt in to the large LDS allocation once
             static bool opted = false;
             if (!opted) {
-                (void)hipFuncSetAttribute((const void*)attn_prefill_kernel<D, GW, VT, F16, KVF, KSP>,
+                (void)hipFuncSetAttribute((const void*)attn_prefill_kernel<D, GW, VT, F16, KVF>,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
                 opted = true;
             }
         }
-        attn_prefill_kernel<D, GW, VT, F16, KVF, KSP><<<grid, threads, lds, st>>>(
+        attn_prefill_kernel<D, GW, VT, F16, KVF><<<grid, threads, lds, st>>>(
             q, kc, vc, bt, bt_stride, tile_seq, tile_q0, cu_q, ctx_lens, Hq, Hkv, Hq / Hkv, bs, scale, window,
             softcap, out);
     });
@@ -1051,18 +1009,6 @@ static int launch_prefill(const bf16_t* q, const void* kc, const void* vc, const
     dim3 grid(n_tiles, Hq / GW);
     const size_t lds0 = 2 * 64 * D * 2 + NW * 16 * (64 + 8) * 2;
     const size_t lds1 = 64 * D * 2 + D * (64 + 8) * 2 + NW * 16 * (64 + 8) * 2;
-    // key split when the grid leaves most CUs idle (short prompt chunks): bf16 cache, V image, D = 128, one wave
-    // per head and GW = 4 (2 x 4 waves = 512 threads, the kernel's launch bound; the merge buffer, 4 x (16 D + 32)
-    // floats, fits the two tile buffers)
-    if constexpr (D == 128 && GW == 4) {
-        static const bool ks_on = !getenv("MX_PREFILL_KSPLIT") || atoi(getenv("MX_PREFILL_KSPLIT")) != 0;
-        if (ks_on && vmode == 0 && !kv8 && (long)n_tiles * (Hq / GW) < 256) {
-            launch_prefill_t<D, GW, 0, KVF_BF16, 2>(grid, 2 * NW * 64, 2 * (2 * 64 * D * 2) + 2 * NW * 16 * (64 + 8) * 2,
-                                                 q, kc, vc, bt, bt_stride, tile_seq, tile_q0, cu_q, ctx_lens, Hq, Hkv,
-                                                 bs, scale, window, softcap, out, st);
-            MXK_CHECK_LAUNCH();
-        }
-    }
 #define PFL(VT_, K8_)                                                                                          \
     launch_prefill_t<D, GW, VT_, K8_>(grid, NW * 64, VT_ ? lds1 : lds0, q, kc, vc, bt, bt_stride, tile_seq,    \
                                       tile_q0, cu_q, ctx_lens, Hq, Hkv, bs, scale, window, softcap, out, st)
@@ -1077,7 +1023,9 @@ static int launch_prefill(const bf16_t* q, const void* kc, const void* vc, const
         else if (kv8 == KVF_IQ4_NL) PFL(VT_, KVF_IQ4_NL);                                                       \
         else PFL(VT_, KVF_BF16);                                                                                \
     }
-    if (vmode == 0) PFK(0) else PFK(1)
+    if constexpr (D == 256) {
+        if (vmode == 0) PFK(0) else PFK(1)
+    } else PFK(1)  // (the row image of V at these head dims: attention_flash.hip)
 #undef PFK
 #undef PFL
     MXK_CHECK_LAUNCH();

@@ -1,0 +1,470 @@
+// attention_flash.hip: prompt attention over the paged cache on 32x32x16 MFMA (bf16, fp8 and block-quantised caches),
+// head dims 64 and 128: what mxk_attn_prefill runs except for head dim 256 and the V^T image (attention.hip).
+//
+// A workgroup owns one KV head, RQ consecutive queries of one sequence and a range of key tiles. Its G query heads are
+// packed with the queries into 32-column groups, column = query * G + head: whatever G is, a wave holds 32 of them and
+// every K / V tile in LDS serves them all. The scores are computed transposed, S^T = K Q^T, so that a column is one
+// lane's (two half-waves hold the even and odd 4-key groups): maximum, sum and rescaling are lane-local but for one
+// exchange between the half-waves per tile, and the probabilities are already where the B operand of O^T = V^T P^T wants
+// them when V^T's keys are taken in the same order (S^T's C layout gives a lane keys 8 j + 4 h + i; both operands' k slot
+// (h, e) then means key 8 (e / 4) + 4 h + e % 4 of the 16). Nothing goes through LDS but K and V.
+//
+// K image: row p, 16-byte chunk c at c ^ row bits, read as A fragments (ds_read_b128, 32 rows x 1 chunk a half-wave);
+// V image: row p, 32-byte region r at r ^ row bits, read with ds_read_b64_tr_b16 (4 keys of a dim per lane).
+// Tiles of 64 keys are double-buffered: a tile's 16-byte chunks are requested one tile ahead, wait in registers (where
+// fp8 and block formats are widened to bf16) and are stored to the other buffer, one barrier per tile.
+//
+// A short chunk behind a long context has too few workgroups (7 x 8 for 416 rows of a 32 / 8-head model), so the key
+// range is split over grid.z: every part has at least MIN_TILES tiles, writes (m, l, O) unnormalised in fp32, and
+// attn_flash_merge_kernel combines them; a block of queries that only one part has keys for is finished by that part.
+//
+// Measured, 32 / 8 heads of 128, against the 16-row kernel this replaced (which read each K / V fragment for one 16x16x32
+// product and moved P through LDS): an 8191-token prompt 2400 -> 630 us (873 TFLOP/s), 2048 233 -> 65, 333 18.5 -> 15.5;
+// 416 rows behind 12000 keys 498 -> 140 us in bf16, 788 -> 140 in fp8. Heads of 64, 8191 rows: 1253 -> 360 us. Bound by
+// the vector unit beside the matrix unit (32 exponentials and ~100 other vector operations a lane and tile against 32
+// products); short prompts by the chain of one tile (~1.3 us) times their tiles.
+#include <type_traits>
+
+#include "kvq.h"
+
+#define LOG2E 1.4426950408889634f
+
+namespace {
+
+constexpr int FT = 64;        // keys per tile
+constexpr int MIN_TILES = 16;  // fewest key tiles a part is made for
+
+template <int D>
+MX_DEV int fk_off(int p, int c) {  // K image: byte offset of 16-byte chunk c of row p
+    const int f = D == 128 ? (p & 15) : ((p >> 1) & 7);
+    return p * (2 * D) + ((c ^ f) << 4);
+}
+template <int D>
+MX_DEV int fv_off(int p, int r) {  // V image: byte offset of 32-byte region r (16 dims) of row p
+    const int f = D == 128 ? (p & 7) : ((p >> 1) & 3);
+    return p * (2 * D) + ((r ^ f) << 5);
+}
+
+MX_DEV float half_max(float x) {  // max of the two half-waves' values of a column, in both
+    const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false));
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+MX_DEV float half_sum(float x) {
+    const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false));
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+template <int KVF>
+struct FRaw {
+    using T = typename std::conditional<(KVF >= KVF_Q8_0), KVQRaw, typename std::conditional<KVF == KVF_FP8, uint2, uint4>::type>::type;
+};
+template <int KVF, int D>
+MX_DEV typename FRaw<KVF>::T f_load(const void* base, size_t eo) {
+    if constexpr (KVF >= KVF_Q8_0) return kvq_load<KVF, D>(base, eo);
+    else if constexpr (KVF == KVF_FP8) return *(const uint2*)((const uint8_t*)base + eo);
+    else return *(const uint4*)((const bf16_t*)base + eo);
+}
+template <int KVF>
+MX_DEV uint4 f_widen(const typename FRaw<KVF>::T& w) {
+    if constexpr (KVF >= KVF_Q8_0) return kvq_to_bf16x8<KVF>(w);
+    else if constexpr (KVF == KVF_FP8) return fp8x8_to_bf16x8(w);
+    else return w;
+}
+
+// GEN: sliding window, soft cap, or a scale that is not positive; without it the scale is one FMA with the maximum
+template <int D, int NW, int KVF, bool GEN>
+__global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_flash_kernel(const bf16_t* __restrict__ q, const void* __restrict__ kc,
+                                                             const void* __restrict__ vc, const int* __restrict__ block_tables,
+                                                             int bt_stride, const int* __restrict__ cu_q,
+                                                             const int* __restrict__ ctx_lens, int n_seqs, int T, int Hq, int Hkv,
+                                                             int G, int bs, int bs_sh, float scale, int window, float softcap,
+                                                             bf16_t* __restrict__ out, int f16, float* __restrict__ part_o,
+                                                             float2* __restrict__ part_ml) {
+    constexpr int NT = 64 * NW;
+    constexpr int IMG = FT * D * 2;              // one K or V image
+    constexpr int CH = FT * D / 8;               // 8-element chunks per image
+    constexpr int NCH = CH / NT;                 // per thread
+    static_assert(CH % NT == 0, "whole chunks per thread");
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int h = lane >> 5, col = lane & 31;
+    const int RQ = 32 * NW / G;                  // queries per workgroup
+    const int kvh = blockIdx.x, part = blockIdx.z, n_parts = gridDim.z;
+
+    // ---- which queries: blocks of RQ of the sequences in order, the last one first (it sees the most keys) ----
+    int total = 0;
+    for (int b = 0; b < n_seqs; b += 64) {
+        const int i = b + lane;
+        total += wave_sum_i(i < n_seqs ? (cu_q[i + 1] - cu_q[i] + RQ - 1) / RQ : 0);
+    }
+    int want = total - 1 - (int)blockIdx.y;
+    if (want < 0) return;  // uniform: the grid is sized for the most blocks that n_seqs sequences can have
+    int s = 0;
+    for (int b = 0; b < n_seqs; b += 64) {
+        const int i = b + lane;
+        int n = i < n_seqs ? (cu_q[i + 1] - cu_q[i] + RQ - 1) / RQ : 0, acc = n;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int x = __shfl_up(acc, o, 64);
+            if (lane >= o) acc += x;
+        }
+        const unsigned long long m = __ballot(acc > want);
+        if (m) {
+            const int l = __ffsll(m) - 1;
+            s = b + l;
+            want -= __shfl(acc - n, l, 64);
+            break;
+        }
+        want -= __shfl(acc, 63, 64);
+    }
+    s = __builtin_amdgcn_readfirstlane(s);
+    const int q0 = __builtin_amdgcn_readfirstlane(want) * RQ;
+    const int qbeg = cu_q[s], qlen = cu_q[s + 1] - qbeg, ctx = ctx_lens[s], pos_off = ctx - qlen;
+    const int* bt = block_tables + (size_t)s * bt_stride;
+
+    // ---- which keys ----
+    const int kv_end = min(ctx, pos_off + min(qlen, q0 + RQ));
+    const int kt_begin = GEN && window > 0 ? max(0, pos_off + q0 - window + 1) / FT * FT : 0;
+    const int n_tiles = kv_end > kt_begin ? (kv_end - kt_begin + FT - 1) / FT : 0;
+    const int per = max(MIN_TILES, (n_tiles + n_parts - 1) / n_parts);
+    const int live = max(1, (n_tiles + per - 1) / per);
+    const int r = wave * 32 + col;               // this lane's column
+    const int qi = q0 + r / G, hq = kvh * G + r % G;
+    const bool real = r < RQ * G && qi < qlen;
+    const size_t orow = (size_t)(qbeg + (real ? qi : 0)) * Hq + hq;  // row of out / of a part's results
+    if (part >= live) {
+        if (real && h == 0) part_ml[(size_t)part * T * Hq + orow] = make_float2(-INFINITY, 0.f);
+        return;
+    }
+    const int t0 = part * per, t1 = min(n_tiles, t0 + per);
+
+    // Q^T as B operand: lane = column, 8 dims 16 ks + 8 h (columns past the end repeat a real one, never stored)
+    bf16x8 qf[D / 16];
+    {
+        const bf16_t* qp = q + ((size_t)(qbeg + min(qi, qlen - 1)) * Hq + kvh * G + r % G) * D + 8 * h;
+#pragma unroll
+        for (int ks = 0; ks < D / 16; ++ks) qf[ks] = *(const bf16x8*)(qp + 16 * ks);
+    }
+    f32x16 o[D / 32];
+#pragma unroll
+    for (int i = 0; i < D / 32; ++i)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) o[i][j] = 0.f;
+    float m_run = -INFINITY, l_run = 0.f;
+    const float qs = scale * LOG2E;
+    const float sc_l2 = softcap * LOG2E, sc_inv = softcap > 0.f ? 1.f / (softcap * LOG2E) : 0.f;
+    const int qpos = pos_off + qi;
+    // the wave's smallest query position (uniform): tiles that end before it need no mask
+    const int wq0 = pos_off + min(q0 + wave * 32 / G, qlen - 1);
+    const int wq1 = pos_off + min(q0 + min(RQ - 1, (wave * 32 + 31) / G), qlen - 1);
+
+    // A tile's chunks: block ids one tile before their rows, rows one tile before they are stored. Rows past the last
+    // key repeat it: no column sees them.
+    typename FRaw<KVF>::T kr[NCH], vr[NCH];
+    int blk[NCH], off[NCH];
+    const size_t page = (size_t)Hkv * bs * D;
+    auto find_rows = [&](int t) {
+#pragma unroll
+        for (int j = 0; j < NCH; ++j) off[j] = min(kt_begin + t * FT + (int)(threadIdx.x + j * NT) / (D / 8), kv_end - 1);
+        int bi[NCH];
+        if (bs_sh >= 0) {
+#pragma unroll
+            for (int j = 0; j < NCH; ++j) bi[j] = off[j] >> bs_sh;
+        } else {
+#pragma unroll
+            for (int j = 0; j < NCH; ++j) bi[j] = off[j] / bs;
+        }
+#pragma unroll
+        for (int j = 0; j < NCH; ++j) {
+            blk[j] = bt[bi[j]];
+            off[j] -= bi[j] * bs;
+        }
+    };
+    auto load_rows = [&]() {
+#pragma unroll
+        for (int j = 0; j < NCH; ++j) {
+            const size_t eo = blk[j] * page + (size_t)((kvh * bs + off[j]) * D + (int)(threadIdx.x + j * NT) % (D / 8) * 8);
+            kr[j] = f_load<KVF, D>(kc, eo);
+            vr[j] = f_load<KVF, D>(vc, eo);
+        }
+    };
+    auto store_rows = [&](int buf) {
+        char* kb = smem + buf * (2 * IMG);
+#pragma unroll
+        for (int j = 0; j < NCH; ++j) {
+            const int id = threadIdx.x + j * NT;
+            const int p = id / (D / 8), c = id % (D / 8);
+            *(uint4*)(kb + fk_off<D>(p, c)) = f_widen<KVF>(kr[j]);
+            *(uint4*)(kb + IMG + fv_off<D>(p, c >> 1) + 16 * (c & 1)) = f_widen<KVF>(vr[j]);
+        }
+    };
+    const int i16 = lane & 15, dh = (lane >> 4) & 1;
+    // The fences keep the fragment reads ahead of what they wait behind: K's before the first product, V's first before the
+    // softmax, its others one k-step ahead of their products (left alone, the scheduler puts every read next to its use).
+    auto work = [&](int t) {
+        const char* kb = smem + (t & 1) * (2 * IMG);
+        const char* vb = kb + IMG;
+        const int kt0 = kt_begin + t * FT;
+        f32x16 sc[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) sc[u][j] = 0.f;
+        bf16x8 kf[D / 16][2];
+        constexpr int KB = NW == 8 ? D / 32 : D / 64;  // k-steps read together (registers: a thread of 4 waves stages twice as much)
+        auto read_k = [&](int k0) {
+#pragma unroll
+            for (int ks = k0; ks < k0 + KB; ++ks)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) kf[ks][u] = *(const bf16x8*)(kb + fk_off<D>(32 * u + col, 2 * ks + h));
+        };
+        read_k(0);
+#pragma unroll
+        for (int k0 = 0; k0 < D / 16; k0 += KB) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (k0 + KB < D / 16) read_k(k0 + KB);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int ks = k0; ks < k0 + KB; ++ks)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) sc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ks][u], qf[ks], sc[u], 0, 0, 0);
+        }
+        bf16x8 vf[4][D / 32];
+        auto read_v = [&](int ks) {
+            const int row = 16 * ks + 4 * h + (i16 >> 2);
+#pragma unroll
+            for (int mt = 0; mt < D / 32; ++mt) {
+                const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (MX_LDS s16x4*)(vb + fv_off<D>(row, 2 * mt + dh) + 8 * (i16 & 3))));
+                const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (MX_LDS s16x4*)(vb + fv_off<D>(row + 8, 2 * mt + dh) + 8 * (i16 & 3))));
+                const u32x4 w4 = {lo[0], lo[1], hi[0], hi[1]};
+                vf[ks][mt] = __builtin_bit_cast(bf16x8, w4);
+            }
+        };
+        __builtin_amdgcn_sched_barrier(0);
+        read_v(0);
+        __builtin_amdgcn_sched_barrier(0);
+        float mul = qs;
+        if constexpr (GEN) {
+            mul = 1.f;
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int j = 0; j < 16; ++j) {
+                    const float v = sc[u][j] * qs;
+                    sc[u][j] = softcap > 0.f ? sc_l2 * tanhf(v * sc_inv) : v;
+                }
+        }
+        if (kt0 + FT - 1 > wq0 || (GEN && window > 0 && kt0 <= wq1 - window)) {
+            const int d = qpos - kt0 - 4 * h;  // (a real column's position is below ctx: later keys hide there too)
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int j = 0; j < 16; ++j) {
+                    const int kp = 32 * u + 8 * (j >> 2) + (j & 3);
+                    if (kp > d || (GEN && window > 0 && kp <= d - window)) sc[u][j] = -INFINITY;
+                }
+        }
+        // (med3 with infinity is the maximum without the quieting of its inputs that fmaxf asks for)
+        float mx[2] = {sc[0][0], sc[1][0]};
+#pragma unroll
+        for (int j = 1; j < 16; ++j)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) mx[u] = __builtin_amdgcn_fmed3f(mx[u], sc[u][j], INFINITY);
+        const float m_new = fmaxf(m_run, half_max(fmaxf(mx[0], mx[1])) * mul);
+        if (__any(m_new > m_run)) {
+            const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);
+            l_run *= alpha;
+#pragma unroll
+            for (int i = 0; i < D / 32; ++i)
+#pragma unroll
+                for (int j = 0; j < 16; ++j) o[i][j] *= alpha;
+            m_run = m_new;
+        }
+        const float m_use = m_run == -INFINITY ? 0.f : m_run;
+        float ls[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            const int u = ks >> 1, j0 = 8 * (ks & 1);
+            if (ks < 3) read_v(ks + 1);
+            u32x4 pw;
+#pragma unroll
+            for (int j = 0; j < 8; j += 2) {
+                const float p0 = __builtin_amdgcn_exp2f(fmaf(sc[u][j0 + j], mul, -m_use));
+                const float p1 = __builtin_amdgcn_exp2f(fmaf(sc[u][j0 + j + 1], mul, -m_use));
+                ls[j & 2] += p0;
+                ls[(j & 2) + 1] += p1;
+                pw[j >> 1] = pack_bf16x2(p0, p1);
+            }
+            const bf16x8 pf = __builtin_bit_cast(bf16x8, pw);
+#pragma unroll
+            for (int mt = 0; mt < D / 32; ++mt) o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[ks][mt], pf, o[mt], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        l_run += (ls[0] + ls[1]) + (ls[2] + ls[3]);
+    };
+
+    if (t0 < t1) {
+        find_rows(t0);
+        load_rows();
+        find_rows(min(t0 + 1, t1 - 1));
+        store_rows(t0 & 1);
+        load_rows();
+        find_rows(min(t0 + 2, t1 - 1));
+        __syncthreads();
+        for (int t = t0; t < t1; ++t) {
+            // the other buffer was last read while tile t - 1 was worked on, before the barrier that ended that round;
+            // half of the waves store first and half work first, so that one's matrix products run beside the other's loads
+            auto stage = [&]() {
+                if (t + 1 >= t1) return;
+                store_rows((t + 1) & 1);
+                load_rows();  // (past the end: the last tile's rows once more, not stored)
+                find_rows(min(t + 3, t1 - 1));
+            };
+            const bool first = wave < NW / 2;
+            if (first) stage();
+            if (kt_begin + t * FT <= wq1) work(t);  // (uniform per wave) tiles past the wave's last query carry nothing
+            if (!first) stage();
+            __syncthreads();
+        }
+    }
+    l_run = half_sum(l_run);
+    auto pack2 = [f16](float a, float b) { return f16 ? pack_act2<true>(a, b) : pack_act2<false>(a, b); };
+    if (live == 1) {
+        if (!real) return;
+        if (n_parts > 1 && h == 0) part_ml[orow] = make_float2(0.f, -1.f);  // finished here: the merge leaves the row alone
+        const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
+#pragma unroll
+        for (int mt = 0; mt < D / 32; ++mt)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                *(uint2*)(out + orow * D + 32 * mt + 8 * g + 4 * h) =
+                    make_uint2(pack2(o[mt][4 * g] * inv, o[mt][4 * g + 1] * inv),
+                               pack2(o[mt][4 * g + 2] * inv, o[mt][4 * g + 3] * inv));
+        return;
+    }
+    if (!real) return;
+    const size_t pr = (size_t)part * T * Hq + orow;
+    if (h == 0) part_ml[pr] = make_float2(m_run, l_run);
+#pragma unroll
+    for (int mt = 0; mt < D / 32; ++mt)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            *(float4*)(part_o + pr * D + 32 * mt + 8 * g + 4 * h) =
+                make_float4(o[mt][4 * g], o[mt][4 * g + 1], o[mt][4 * g + 2], o[mt][4 * g + 3]);
+}
+
+// out rows from the parts' (m, l, O): D / 8 lanes a row, 8 dims each. A row that one part finished alone (l < 0 in part 0)
+// is left as it is, parts without a visible key (m = -inf) are not read.
+template <int D>
+__global__ __launch_bounds__(256) void attn_flash_merge_kernel(const float* __restrict__ part_o, const float2* __restrict__ part_ml,
+                                                               int n_parts, const int* __restrict__ cu_q, int n_seqs, int T, int Hq,
+                                                               bf16_t* __restrict__ out, int f16) {
+    constexpr int LPR = D / 8;
+    const long row = (long)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
+    const int d0 = threadIdx.x % LPR * 8;
+    if (row >= (long)min(T, cu_q[n_seqs]) * Hq) return;  // rows past the step's last query belong to nobody
+    const size_t stride = (size_t)T * Hq;
+    float mx = -INFINITY;
+    for (int p = 0; p < n_parts; ++p) {
+        const float2 ml = part_ml[p * stride + row];
+        if (p == 0 && ml.y < 0.f) return;
+        mx = fmaxf(mx, ml.x);
+    }
+    float ls = 0.f, acc[8] = {};
+    for (int p = 0; p < n_parts; ++p) {
+        const float2 ml = part_ml[p * stride + row];
+        if (ml.x == -INFINITY) continue;
+        const float a = exp2f(ml.x - mx);
+        ls += ml.y * a;
+        const float4* po = (const float4*)(part_o + (p * stride + row) * D + d0);
+        const float4 x = po[0], y = po[1];
+        acc[0] += x.x * a;
+        acc[1] += x.y * a;
+        acc[2] += x.z * a;
+        acc[3] += x.w * a;
+        acc[4] += y.x * a;
+        acc[5] += y.y * a;
+        acc[6] += y.z * a;
+        acc[7] += y.w * a;
+    }
+    const float inv = ls > 0.f ? 1.f / ls : 0.f;
+    uint32_t w[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        w[e] = f16 ? pack_act2<true>(acc[2 * e] * inv, acc[2 * e + 1] * inv) : pack_act2<false>(acc[2 * e] * inv, acc[2 * e + 1] * inv);
+    *(uint4*)(out + row * D + d0) = make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+template <int D, int NW, int KVF>
+int launch_flash(const bf16_t* q, const void* kc, const void* vc, const int* bt, int bt_stride, const int* cu_q, const int* ctx_lens,
+                 int n_seqs, int T, int Hq, int Hkv, int bs, float scale, int window, float softcap, bf16_t* out, int n_parts,
+                 float* part_o, float2* part_ml, hipStream_t st) {
+    const int G = Hq / Hkv, RQ = 32 * NW / G;
+    const long blocks = (long)T / RQ + min(n_seqs, T);
+    if (blocks > 65535) return (int)hipErrorInvalidValue;
+    const dim3 grid(Hkv, (unsigned)blocks, n_parts);
+    constexpr int LDS = 4 * FT * D * 2;
+    const int sh = (bs & (bs - 1)) ? -1 : __builtin_ctz(bs);
+    const bool gen = window > 0 || softcap > 0.f || !(scale > 0.f);
+#define FL(GEN_)                                                                                                             \
+    do {                                                                                                                     \
+        static const hipError_t once = hipFuncSetAttribute((const void*)attn_flash_kernel<D, NW, KVF, GEN_>,            \
+                                                           hipFuncAttributeMaxDynamicSharedMemorySize, LDS);                 \
+        if (once != hipSuccess) return (int)once;                                                                            \
+        attn_flash_kernel<D, NW, KVF, GEN_><<<grid, 64 * NW, LDS, st>>>(q, kc, vc, bt, bt_stride, cu_q, ctx_lens, n_seqs, \
+                                                                             T, Hq, Hkv, G, bs, sh, scale, window, softcap,  \
+                                                                             out, g_mx_act_f16, part_o, part_ml);                          \
+    } while (0)
+    if (gen) FL(true);
+    else FL(false);
+    if (n_parts > 1)
+        attn_flash_merge_kernel<D><<<(unsigned)(((long)T * Hq * (D / 8) + 255) / 256), 256, 0, st>>>(part_o, part_ml, n_parts, cu_q,
+                                                                                               n_seqs, T, Hq, out, g_mx_act_f16);
+#undef FL
+    MXK_CHECK_LAUNCH();
+}
+
+template <int D, int NW>
+int dispatch_flash(const bf16_t* q, const void* kc, const void* vc, const int* bt, int bt_stride, const int* cu_q, const int* ctx_lens,
+                   int n_seqs, int T, int Hq, int Hkv, int bs, float scale, int window, float softcap, bf16_t* out, int n_parts,
+                   float* part_o, float2* part_ml, int kvf, hipStream_t st) {
+#define FD(F_)                                                                                                                \
+    case F_:                                                                                                                  \
+        return launch_flash<D, NW, F_>(q, kc, vc, bt, bt_stride, cu_q, ctx_lens, n_seqs, T, Hq, Hkv, bs, scale, window, softcap, \
+                                       out, n_parts, part_o, part_ml, st)
+    switch (kvf) {
+        FD(KVF_BF16);
+        FD(KVF_FP8);
+        FD(KVF_Q8_0);
+        FD(KVF_Q4_0);
+        FD(KVF_Q4_1);
+        FD(KVF_Q5_0);
+        FD(KVF_Q5_1);
+        FD(KVF_IQ4_NL);
+    }
+#undef FD
+    return (int)hipErrorInvalidValue;
+}
+
+}  // namespace
+
+// q bf16 [T, Hq, D]; sequences cu_q [n_seqs + 1] with contexts ctx_lens; keys and values from the paged caches. waves: 4 or 8
+// per workgroup (the caller's plan). n_parts > 1 needs part_o fp32 [n_parts, T, Hq, D] and part_ml float2 [n_parts, T, Hq].
+extern "C" int mxk_attn_flash(const bf16_t* q, const void* kc, const void* vc, const int* bt, int bt_stride, const int* cu_q,
+                              const int* ctx_lens, int n_seqs, int T, int Hq, int Hkv, int D, int bs, float scale, int window,
+                              float softcap, bf16_t* out, int waves, int n_parts, float* part_o, float2* part_ml, int kvf, hipStream_t st) {
+    if (T <= 0 || n_seqs <= 0) return 0;
+    if (Hkv <= 0 || Hq % Hkv || Hq / Hkv > 128 || bs <= 0 || n_parts < 1 || n_parts > 64) return (int)hipErrorInvalidValue;
+    if (n_parts > 1 && (!part_o || !part_ml)) return (int)hipErrorInvalidValue;
+#define FW(D_, W_) \
+    if (D == D_ && waves == W_)  \
+        return dispatch_flash<D_, W_>(q, kc, vc, bt, bt_stride, cu_q, ctx_lens, n_seqs, T, Hq, Hkv, bs, scale, window, softcap, out, n_parts, part_o, part_ml, kvf, st)
+    FW(128, 4);
+    FW(128, 8);
+    FW(64, 4);
+    FW(64, 8);
+#undef FW
+    return (int)hipErrorInvalidValue;
+}

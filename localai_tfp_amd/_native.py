@@ -62,6 +62,7 @@ KERNEL_SIGS = {
     "mxk_attn_decode_mfma": [P, I, P, P, P, I, P, I, I, I, I, I, F, I, F, I, I, P, I, P, P, I, P, P],
     "mxk_attn_prefill": [P, P, P, P, I, P, P, I, P, P, I, I, I, I, F, I, F, P, I, I, P],
     "mxk_probe_tr16": [P, P],
+    "mxk_attn_flash": [P, P, P, P, I, P, P, I, I, I, I, I, I, F, I, F, P, I, I, P, P, I, P],
     "mxk_attn_prefill_rows": [I, I],
     "mxk_sample": [P, I, I, I, P, P, P, P, P, I, P, P, P, P],
     "mxk_sample_topk_split": [P, I, I, I, P, I, P, P, P, P, I, I, P, P, P, P, P, P, P, P],

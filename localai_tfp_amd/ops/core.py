@@ -436,6 +436,36 @@ def prefill_tiles(q_lens, rows_per_tile: int):
 ATTN_VMODE = int(__import__("os").environ.get("MX_ATTN_VMODE", "0"))
 
 
+CU_COUNT = 256
+FLASH_SPLIT_KEYS = 2048  # contexts from which a grid that leaves compute units idle splits its keys
+
+
+def flash_plan(T: int, n_seqs: int, Hq: int, Hkv: int, D: int, block_size: int, table_width: int, window: int,
+               ctx_lens_host=None):
+    """(waves per workgroup, key parts) of attention_flash.hip for T prompt rows, or None where the other prompt kernel
+    runs (head dim 256, and what neither takes). A workgroup holds 32 * waves / G queries of one KV head.
+
+    Measured on Llama-3-8B heads (32 / 8 x 128): 4 waves, two workgroups on a compute unit, beat 8 at every size that does
+    not fill the chip twice over with 8 (333 rows 15.5 against 20 us, 2048 rows 65 against 76; 8191 rows 675 against 630).
+    A grid of fewer than two workgroups per compute unit is split over its keys where the context is long: 416 rows behind
+    12000 keys 275 -> 140 us, 289 behind 2000 58 -> 41; the merge launch costs 2-3 us where it has nothing to merge, so
+    contexts that are known to be short (ctx_lens_host; else what the block tables can hold) do not ask for it."""
+    if D not in (64, 128) or Hkv <= 0 or Hq % Hkv:
+        return None
+    G = Hq // Hkv
+    if G > 128 or (G > 8 and G % 8) or (D == 64 and G in (3, 5, 6, 7)):
+        return None
+    blocks = lambda waves: T // (32 * waves // G) + min(n_seqs, T)  # noqa: E731
+    if D == 128 and blocks(8) * Hkv >= 2 * CU_COUNT:
+        return (8, 1) if blocks(8) <= 65535 else None
+    base = blocks(4) * Hkv
+    keys = max(ctx_lens_host) if ctx_lens_host else block_size * table_width
+    if window > 0:
+        keys = min(keys, window + 32 * 4 // G)
+    parts = max(1, min(16, 2 * CU_COUNT // base)) if keys >= FLASH_SPLIT_KEYS else 1
+    return (4, parts) if blocks(4) <= 65535 else None
+
+
 def attn_prefill(q: torch.Tensor, k_cache, v_cache, block_tables: torch.Tensor, cu_q: torch.Tensor,
                  ctx_lens: torch.Tensor, scale: float, out: torch.Tensor, q_lens_host=None, ctx_lens_host=None,
                  vmode: int | None = None, window: int = 0, softcap: float = 0.0, tiles=None):
@@ -445,13 +475,31 @@ def attn_prefill(q: torch.Tensor, k_cache, v_cache, block_tables: torch.Tensor, 
     T, Hq, D = q.shape
     if T == 0:
         return out
+    if q.is_cuda:
+        vmode = ATTN_VMODE if vmode is None else int(vmode)
+        plan = flash_plan(T, cu_q.numel() - 1, Hq, k_cache.shape[1], D, k_cache.shape[2], block_tables.shape[1], window,
+                          ctx_lens_host) if vmode == 0 else None
+        if plan is not None:
+            waves, parts = plan
+            po = ml = None
+            if parts > 1:
+                po = torch.empty((parts, T, Hq, D), dtype=torch.float32, device=q.device)
+                ml = torch.empty((parts, T, Hq, 2), dtype=torch.float32, device=q.device)
+            N.ensure_act(out.dtype)
+            N.kcall("mxk_attn_flash", q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), block_tables.data_ptr(),
+                    block_tables.stride(0), cu_q.data_ptr(), ctx_lens.data_ptr(), cu_q.numel() - 1, T, Hq,
+                    k_cache.shape[1], D, k_cache.shape[2], float(scale), int(window), float(softcap), out.data_ptr(),
+                    waves, parts, N.ptr(po), N.ptr(ml), kv_format(k_cache), N.stream_ptr())
+            return out
+        if D != 256:
+            vmode = 1
     if tiles is not None and q.is_cuda:
         Hkv, bs = k_cache.shape[1], k_cache.shape[2]
         N.ensure_act(out.dtype)
         N.kcall("mxk_attn_prefill", q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), block_tables.data_ptr(),
                 block_tables.stride(0), tiles[0].data_ptr(), tiles[1].data_ptr(), int(tiles[0].numel()),
                 cu_q.data_ptr(), ctx_lens.data_ptr(), Hq, Hkv, D, bs, float(scale), int(window), float(softcap),
-                out.data_ptr(), ATTN_VMODE if vmode is None else int(vmode), kv_format(k_cache), N.stream_ptr())
+                out.data_ptr(), vmode, kv_format(k_cache), N.stream_ptr())
         return out
     Hkv, bs = k_cache.shape[1], k_cache.shape[2]
     cu = cu_q.tolist() if q_lens_host is None else None
@@ -473,8 +521,8 @@ def attn_prefill(q: torch.Tensor, k_cache, v_cache, block_tables: torch.Tensor, 
     N.ensure_act(out.dtype)
     N.kcall("mxk_attn_prefill", q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), block_tables.data_ptr(),
             block_tables.stride(0), tiles[0].data_ptr(), tiles[1].data_ptr(), len(seqs), cu_q.data_ptr(),
-            ctx_lens.data_ptr(), Hq, Hkv, D, bs, float(scale), int(window), float(softcap), out.data_ptr(),
-            ATTN_VMODE if vmode is None else int(vmode), kv_format(k_cache), N.stream_ptr())
+            ctx_lens.data_ptr(), Hq, Hkv, D, bs, float(scale), int(window), float(softcap), out.data_ptr(), vmode,
+            kv_format(k_cache), N.stream_ptr())
     return out
 
 

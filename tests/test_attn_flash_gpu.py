@@ -1,0 +1,105 @@
+"""Prompt attention of csrc/kernels/attention_flash.hip against the fp32 reference, at the edges of its query blocks, key
+tiles and key parts, and the plan that chooses it (ops/core.py flash_plan)."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from localai_tfp_amd.ops import core as K
+from localai_tfp_amd.ops import kvq as KQ
+
+
+def _case(Hq, Hkv, D, q_lens, pre, bs=16, fmt="bf16", seed=0):
+    g = torch.Generator().manual_seed(seed)
+    ctx = [a + b for a, b in zip(q_lens, pre)]
+    nb = sum(-(-c // bs) for c in ctx) + 2
+    ids = (torch.randperm(nb - 1, generator=g) + 1).tolist()
+    bt = torch.zeros(len(ctx), max(1, max(-(-c // bs) for c in ctx)), dtype=torch.int32)
+    for s, c in enumerate(ctx):
+        n = -(-c // bs)
+        bt[s, :n] = torch.tensor(ids[:n], dtype=torch.int32)
+        ids = ids[n:]
+    kc, vc = (torch.randn(nb, Hkv, bs, D, generator=g) for _ in range(2))
+    if fmt in KQ.FORMATS:
+        f = KQ.FORMATS[fmt]
+        kc, vc = (KQ.tag(torch.from_numpy(KQ.quantize_rows(t.reshape(-1, D), f)).view(nb, Hkv, bs, -1), f) for t in (kc, vc))
+    else:
+        kc, vc = (t.to(torch.float8_e4m3fn if fmt == "fp8" else torch.bfloat16) for t in (kc, vc))
+    q = torch.randn(sum(q_lens), Hq, D, generator=g).to(torch.bfloat16)
+    return q, kc, vc, bt, torch.tensor(np.concatenate([[0], np.cumsum(q_lens)]), dtype=torch.int32), torch.tensor(ctx, dtype=torch.int32)
+
+
+def _check(Hq, Hkv, D, q_lens, pre, window=0, softcap=0.0, scale=None, plan=None, monkeypatch=None, **kw):
+    q, kc, vc, bt, cu, ctx = _case(Hq, Hkv, D, q_lens, pre, **kw)
+    scale = D ** -0.5 if scale is None else scale
+    want = torch.zeros(q.shape)
+    for s, n in enumerate(q_lens):
+        if n:
+            c, r = int(ctx[s]), slice(int(cu[s]), int(cu[s]) + n)
+            want[r] = K._attn_ref_one(q[r], kc, vc, bt[s], c, c - n, scale, kc.shape[2], window, softcap).nan_to_num(0.0)
+    if plan is not None:
+        monkeypatch.setattr(K, "flash_plan", lambda *a, **k: plan)
+    kd, vd = kc.cuda(), vc.cuda()
+    if hasattr(kc, "kvf"):
+        kd.kvf, vd.kvf = kc.kvf, vc.kvf
+    out = torch.full(q.shape, float("nan"), dtype=torch.float16, device="cuda")
+    K.attn_prefill(q.cuda(), kd, vd, bt.cuda(), cu.cuda(), ctx.cuda(), scale, out, window=window, softcap=softcap)
+    got = out.cpu().float()
+    # probabilities and outputs are rounded to 16 bits once each (2^-9, 2^-11): over a row of summed values the relative
+    # error stays below 4 x 2^-9
+    assert float((got - want).norm() / want.norm()) < 4 * 2 ** -9
+    assert torch.isfinite(got).all()
+
+
+def test_plan_takes_what_the_kernel_takes():
+    p = K.flash_plan
+    assert p(100, 1, 32, 8, 256, 16, 64, 0) is None and p(100, 1, 12, 4, 64, 16, 64, 0) is None  # the other kernel's / refused
+    assert p(100, 1, 30, 8, 128, 16, 64, 0) is None
+    assert p(333, 1, 32, 8, 128, 16, 512, 0, [333]) == (4, 1)  # known to be short: no parts
+    assert p(333, 1, 32, 8, 128, 16, 512, 0) == (4, 5) and p(333, 1, 32, 8, 128, 16, 512, 0, []) == (4, 5)
+    assert p(333, 1, 32, 8, 128, 16, 512, 256) == (4, 1)  # a window hides what lies further back
+    assert p(8191, 1, 32, 8, 128, 16, 512, 0) == (8, 1) and p(8191, 1, 32, 8, 64, 16, 512, 0) == (4, 1)
+    assert all(1 <= p(t, s, 8 * g, 8, 128, 16, 4096, 0)[1] <= 16 for t in (1, 17, 500, 4000) for s in (1, 9, 200) for g in (1, 2, 3, 5, 7, 8, 16))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Hq,Hkv,D", [(32, 8, 128), (8, 8, 128), (6, 2, 128), (28, 4, 128), (16, 1, 128), (32, 8, 64), (4, 2, 64), (40, 1, 128)])
+def test_query_blocks_and_key_tiles(Hq, Hkv, D):
+    """Blocks of queries and tiles of keys that end just before, at and after an edge; sequences without rows between others."""
+    _check(Hq, Hkv, D, [1, 31, 0, 33, 64, 65, 0], [0, 33, 5, 31, 0, 63, 9])
+    _check(Hq, Hkv, D, [130], [127], bs=24)  # pages that are no power of two
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("waves,parts", [(4, 1), (8, 1), (4, 2), (8, 3), (4, 16)])
+@pytest.mark.parametrize("D", [64, 128])
+def test_key_parts(waves, parts, D, monkeypatch):
+    """Sequences that one part finishes beside others that several share (parts hold at least 16 tiles of 64 keys)."""
+    _check(8, 2, D, [70, 5, 40], [1100, 0, 3000], plan=(waves, parts), monkeypatch=monkeypatch)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", ["fp8", "q8_0", "q4_0", "q4_1", "q5_0", "q5_1", "iq4_nl"])
+def test_cache_formats(fmt, monkeypatch):
+    _check(8, 2, 128, [70, 33], [61, 1500], fmt=fmt)
+    _check(8, 2, 64, [70, 33], [61, 1500], fmt=fmt, plan=(8, 2), monkeypatch=monkeypatch)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("window,softcap,scale", [(50, 0.0, None), (64, 0.0, None), (1, 0.0, None), (0, 20.0, None), (130, 30.0, None), (0, 0.0, -0.05)])
+def test_windows_caps_and_scales(window, softcap, scale, monkeypatch):
+    _check(8, 2, 128, [90, 40], [300, 0], window=window, softcap=softcap, scale=scale)
+    _check(8, 2, 128, [90, 40], [3000, 0], window=window, softcap=softcap, scale=scale, plan=(4, 3), monkeypatch=monkeypatch)
+
+
+@pytest.mark.gpu
+def test_infinite_scores_behave_like_the_reference():
+    """A key of infinite score makes its row NaN, and no other row."""
+    q, kc, vc, bt, cu, ctx = _case(4, 1, 128, [80], [0])
+    kc[bt[0, 40 // 16], 0, 40 % 16] = float("inf")
+    q[:, :, :] = q.abs() + 0.1
+    out = torch.zeros(q.shape, dtype=torch.float16, device="cuda")
+    K.attn_prefill(q.cuda(), kc.cuda(), vc.cuda(), bt.cuda(), cu.cuda(), ctx.cuda(), 1 / math.sqrt(128), out)
+    got = out.cpu().float()
+    assert torch.isfinite(got[:40]).all() and torch.isnan(got[40:]).all()
