@@ -180,13 +180,17 @@ __global__ __launch_bounds__(NG == 8 ? 512 / GPW : 256 * KS) void qmm2_kernel(co
     constexpr int NW = NG / WN;
     const int nw = cg % NW, mw = cg / NW;
 
-    // XCD-aware bijective remap: consecutive logical ids (the row tiles and splits of one column panel)
-    // run on one XCD and share its L2
+    // XCD-aware bijective remap: consecutive logical ids (q2_tile_of) run on one XCD and share its L2
     const int nwg = gridDim.x, bid = blockIdx.x;
     const int xcd = bid & 7, q8 = nwg >> 3, r8 = nwg & 7;
     const int lid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (bid >> 3);
-    const int mt = lid % n_mt;
-    const int rest = lid / n_mt;
+    int mt, rest;
+    if constexpr (GR) {  // (row tiles of experts: how many there are is known on the device)
+        mt = lid % n_mt;
+        rest = lid / n_mt;
+    } else {
+        q2_tile_of(lid, n_mt, nwg / n_mt, mt, rest);
+    }
     const int split = rest % splits;
     const int ct = rest / splits;
 

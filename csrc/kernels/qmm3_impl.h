@@ -43,12 +43,12 @@ __global__ __launch_bounds__(512) void qmm3_kernel(const uint16_t* __restrict__ 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int h = lane >> 5, col = lane & 31;
 
-    // XCD-aware bijective remap (as qmm2): the row tiles and splits of one column panel share an XCD's L2
+    // XCD-aware bijective remap (as qmm2, q2_tile_of)
     const int nwg = gridDim.x, bid = blockIdx.x;
     const int xcd = bid & 7, q8 = nwg >> 3, r8 = nwg & 7;
     const int lid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (bid >> 3);
-    const int mt = lid % n_mt;
-    const int rest = lid / n_mt;
+    int mt, rest;
+    q2_tile_of(lid, n_mt, nwg / n_mt, mt, rest);
     const int split = rest % splits;
     const int ct = rest / splits;
     const int nsb = K >> 8;

@@ -14,6 +14,7 @@ numerics oracle for the HIP kernels.
 """
 from __future__ import annotations
 
+import functools
 import logging
 import os
 
@@ -604,6 +605,46 @@ def _split_for(tiles: int, K: int, can_split: bool) -> int:
     return splits
 
 
+# Row tiles of GEMMs beyond the load-time autotuner's buckets: (wm, ks, wn, us per 10^6 of rows x columns x K of a tile)
+LARGE_M = 512
+_LARGE_TILES = ((6, 17, 1, 0.421), (7, 17, 1, 0.415), (4, 17, 1, 0.458), (6, 1, 1, 0.508), (4, 2, 1, 0.526),
+                (2, 2, 1, 0.633))
+# bytes a 32-column group stages per 64-k tile and per super-block header (csrc/kernels/qmm2_fmt.h QB, HB)
+_STAGE_BYTES = {int(QType.Q4_K): (1024, 512), int(QType.Q5_K): (1024, 1536), int(QType.Q6_K): (1536, 640),
+                int(QType.Q3_K): (1024, 1536), int(QType.Q2_K): (1024, 640), int(QType.MX4F): (1024, 1024),
+                int(QType.MX5F): (1280, 1024), int(QType.Q8_0): (2176, 0)}
+
+
+@functools.lru_cache(maxsize=4096)
+def _large_plan(M: int, N_: int, K: int, qtype: int, can_split: bool):
+    """qmm2 plan of a GEMM of more than LARGE_M rows: the least of
+        6.6 + rounds * tile * K / splits * c  (+ 2.4e-6 * M * N * splits where partial sums meet in atomics)   us
+    over the tiles whose ring fits the LDS for the format, rounds = workgroups / 256 with a last round that is r full
+    counted as 0.6 + 0.4 r (a half-empty chip clocks and feeds its tiles faster). The constants are a fit to 13 shapes
+    (1024 x 4096 .. 57344 x 8192) at 12 row counts 528 .. 8191: the plan picked is within 1 % of the best of 40 candidates
+    on average (18 % at worst), where one 128 x 128 tile for every shape was 16 % off (76 %). Wide tiles (256 columns)
+    win where there are rounds enough: gate|up 28672 x 4096 at 8191 rows 2182 -> 1733 us (1.11 PFLOP/s), 1024 276 -> 252;
+    narrow outputs take 64-row tiles: 1024 x 4096 at 1024 rows 31 -> 22 us."""
+    qb, hb = _STAGE_BYTES[qtype]
+    best = None
+    for wm, ks, wn, c in _LARGE_TILES:
+        bm, ng = 32 * wm * wn, 8 if ks == 17 else 4
+        if 4 * (bm * 128 + ng * qb) + 2 * ng * hb > 160 * 1024:
+            continue
+        for s in (1, 2, 4) if can_split else (1,):
+            if s > 1 and (K // 256) // s < 2:
+                continue
+            wgs = -(-M // bm) * -(-N_ // (32 * ng)) * s
+            full, rem = divmod(wgs, CU_COUNT)
+            rounds = full + (0.6 + 0.4 * rem / CU_COUNT if rem else 0.0)
+            t = 6.6 + rounds * bm * 32 * ng * 256 * -(-(K // 256) // s) * c * 1e-6
+            if s > 1:
+                t += 2.4e-6 * M * N_ * s
+            if best is None or t < best[0]:
+                best = (t, ("q2", wm, ks, wn, s))
+    return best[1]
+
+
 def _gemm_pick(M: int, N_: int, K: int, qtype: int, can_split: bool):
     """Untuned fallback plan ("q3", wm, splits) | ("q2", wm, ks, wn, splits) for a t32 GEMM — shapes the load-time
     autotuner (ops/autotune.py) did not time. The rule follows the tuned Llama-3-8B table
@@ -613,6 +654,8 @@ def _gemm_pick(M: int, N_: int, K: int, qtype: int, can_split: bool):
         return ("q3", *_qmm3_shape(M, N_, K, can_split))
     if QMM2 and M >= QMM2_MIN_M:
         return ("q2", *_qmm2_shape(M, N_, K, can_split))
+    if M > LARGE_M:
+        return _large_plan(M, N_, K, qtype, can_split)
     nct = -(-N_ // 128)
     wide = N_ >= 16384
     if M <= 64 or (not wide and K < 8192 and M <= 256):

@@ -1,0 +1,46 @@
+"""GEMM plans beyond the autotuner's buckets (ops/linear.py _large_plan) and the banded tile order they run in."""
+import pytest
+import torch
+
+from localai_tfp_amd.formats.gguf import QType
+from localai_tfp_amd.ops import linear as L
+from localai_tfp_amd.ops import quant as Q
+
+QTYPES = [QType.Q4_K, QType.Q5_K, QType.Q6_K, QType.Q3_K, QType.Q2_K, QType.Q8_0]
+
+
+def test_plans_are_compiled_tiles():
+    for qt in L._STAGE_BYTES:
+        for m in (513, 640, 1000, 2049, 8191, 40000):
+            for n, k in ((32, 256), (1024, 4096), (4096, 14336), (28672, 4096), (2080, 512)):
+                for split in (False, True):
+                    kind, wm, ks, wn, s = L._gemm_pick(m, n, k, qt, split)
+                    assert kind == "q2" and (wm, ks, wn) in L.QMM2_CONFIGS and s in (1, 2, 4)
+                    assert s == 1 or (split and (k // 256) // s >= 2)
+                    assert not (ks == 17 and wm == 7 and qt not in (int(QType.Q4_K), int(QType.Q2_K), int(QType.MX4F)))
+                    assert not (ks == 17 and wm >= 6 and qt == int(QType.Q8_0))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("qt", QTYPES)
+@pytest.mark.parametrize("M,n", [(513, 32), (769, 416), (1025, 1056), (2100, 288)])
+def test_large_plan_product(qt, M, n):
+    """Whole and partial bands of row tiles, tails of rows and columns, plans that split K and plans that do not."""
+    import numpy as np
+    k = 1536
+    raw = Q.random_quantized(np.random.default_rng(M + n), int(qt), n, k).reshape(n, -1)
+    W = L.QWeight.from_ggml(raw, int(qt), n, k, "cuda", t32=True)
+    dense = torch.from_numpy(Q.dequantize(raw.reshape(-1), int(qt), (k, n)).reshape(n, k).copy())
+    assert W.to_t32()
+    x = (torch.randn(M, k, generator=torch.Generator().manual_seed(1)) * 0.5).half()
+    want = x.double() @ dense.double().t()
+    for zeroed in (False, True):
+        out = torch.zeros(M, n, device="cuda")
+        L.qmatmul(W, x.cuda(), L.EPI_F32, out, out_zeroed=zeroed)
+        # weights are rounded to f16 once (2^-11), products summed in fp32
+        assert float((out.cpu().double() - want).norm() / want.norm()) < 2 ** -10
+    act = torch.zeros(M, n // 2, device="cuda", dtype=torch.float16)
+    L.qmatmul(W, x.cuda(), L.EPI_SWIGLU, act)
+    y = want.view(M, -1, 2, 16)
+    g = (torch.nn.functional.silu(y[:, :, 0]) * y[:, :, 1]).reshape(M, -1)
+    assert float((act.cpu().double() - g).norm() / g.norm()) < 4 * 2 ** -10
