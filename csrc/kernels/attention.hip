@@ -305,30 +305,110 @@ MX_DEV int v_lds_off(int p, int nt) {
 // ------------------------------------------------------------------------------------------------
 // decode on MFMA. The VALU kernel above spends its time on the per-position dot products and the
 // 16-lane shuffle reductions (~30% of HBM bandwidth at B=128); here the G query heads of a kv head are
-// the rows of a 16x16x32 bf16 MFMA tile, so QK^T and PV run on the matrix cores and the softmax
-// reductions happen once per 32-key tile.
+// the columns of a 16x16x32 bf16 MFMA tile, so QK^T and PV run on the matrix cores and the softmax
+// happens once per 32-key tile.
 //   workgroup = (kv head, sequence, partition), 4 waves; wave w takes the partition's 32-key tiles
-//   w, w+4, ...: K fragments come straight from the paged cache into MFMA B operands (16-byte loads,
-//   one cached position x 8 dims per lane), V is staged in the wave's LDS slice and read back with
-//   the hardware-transposing ds_read_b64_tr_b16 (same V image as the prefill kernel), P goes
-//   register -> LDS -> A fragment. The 4 waves' (m, l, O) merge through LDS at the end, in the same
-//   partial-result format as attn_decode_kernel (attn_decode_reduce merges partitions).
-// Occupancy, not register double buffering, hides HBM latency: ~9.3 KB of LDS per wave lets 4
+//   w, w+4, ...: K fragments come straight from the paged cache into MFMA A operands (16-byte loads,
+//   one cached position x 8 dims per lane) and S^T = K Q^T leaves a head's scores in four lanes: two lane
+//   swaps give its maximum, the rest is lane-local, and the probabilities are already the B operand of
+//   O^T = V^T P^T when V^T's keys are read in the order S^T's layout has them. V is staged in the wave's LDS
+//   slice and read with the hardware-transposing ds_read_b64_tr_b16 (same V image as the prefill kernel). The 4
+//   waves' (m, l, O) merge through LDS at the end, in the same partial-result format as attn_decode_kernel
+//   (attn_decode_reduce merges partitions).
+// Against the form with heads as rows (4 rows a lane, two 16-lane shuffle reductions per row and tile, P through LDS) and
+// caches widened load by load: bf16 B=128 ctx 65-1021 50.0 -> 45.2 us (4.0 TB/s), B=32 ctx 97-4003 44.5 -> 41.3; q8_0
+// B=9 ctx 3001-24001 155 -> 76 us at 256-key partitions (62 at 1024: 3.3 TB/s), fp8 147 -> 72 (55), q4_0 151 -> 75 (65:
+// 1.7 TB/s, bound by the widening's vector work).
+// Occupancy, not register double buffering, hides HBM latency: 8 KB of LDS per wave lets 4
 // workgroups (16 waves) share a CU, each with one tile's 16 KB of K/V loads in flight.
 template <int D>
-constexpr int dec_wave_lds() { return 32 * D * 2 + 16 * (32 + 8) * 2; }
+constexpr int dec_wave_lds() { return 32 * D * 2; }
+
+// maximum / sum over the lanes l, l ^ 16, l ^ 32, l ^ 48 in each of them
+MX_DEV float quarters_max(float x) {
+    const u32x2 a = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false));
+    x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const u32x2 b = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false));
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+MX_DEV float quarters_sum(float x) {
+    const u32x2 a = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false));
+    x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const u32x2 b = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false));
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
 
 // NW = 16 (1024 threads, one workgroup per CU): the small-batch form — a 512-key partition per workgroup, so a
 // context of <= 512 keys is ONE partition whose workgroup writes the final output (no reduce work for it).
 // TS: debug instantiation writing wall-clock stamps of workgroup (0, 0, 0) wave 0 to ts[0..7] (tools/prof_attn_decode.py)
 // DPF: the K-prefetch form (below; 2 waves / SIMD for its registers, MX_DECODE_PF=0 selects the 4-wave form)
-// 8 cached elements at element offset eo widened to bf16 (fp8 / block-quantised caches)
+// The bytes of one tile of an 8-bit or block-quantised cache as a lane holds them (16 + 16 keys of K, a half row of V),
+// requested one tile ahead: wide loads (8 bytes of K, 16 of V) and one load for all of a row's block scales, not two loads
+// per eight elements. Rows are 4-byte aligned.
+struct __attribute__((packed, aligned(4))) DecU4 { uint32_t x[4]; };
+struct __attribute__((packed, aligned(4))) DecU2 { uint32_t x[2]; };
 template <int KVF, int D>
-MX_DEV uint4 kv_widen8(const void* base, size_t eo) {
-    if constexpr (KVF == KVF_FP8) return fp8x8_to_bf16x8(*(const uint2*)((const uint8_t*)base + eo));
-    else return kvq_to_bf16x8<KVF>(kvq_load<KVF, D>(base, eo));
-}
+struct DecRaw {
+    using Q = KVQ<KVF, D>;
+    static constexpr bool KVQ_ = KVF >= KVF_Q8_0;
+    static constexpr bool B8 = KVF == KVF_FP8 || Q::Q8;              // one byte per element, else four bits
+    static constexpr int ROWB = KVQ_ ? Q::ROWB : D;
+    static constexpr int SB = KVQ_ ? (Q::MIN ? 4 : 2) : 0;           // scale bytes per block of 32
+    static constexpr int KS = D / 32;
+    uint32_t kc[2][KS][B8 ? 2 : 1];
+    uint32_t ks[2][KVQ_ ? (KS * SB + 3) / 4 : 1], kh[2][KVQ_ && Q::HB ? KS : 1];
+    uint32_t vc[D / 2 / (B8 ? 4 : 8)];
+    uint32_t vs[KVQ_ ? (KS / 2 * SB + 3) / 4 : 1], vh[KVQ_ && Q::HB ? D / 64 : 1];
 
+    static MX_DEV void copy(uint32_t* to, const uint8_t* from, int bytes) {
+        int i = 0;
+        for (; i + 16 <= bytes; i += 16) {
+            const DecU4 w = *(const DecU4*)(from + i);
+            for (int j = 0; j < 4; ++j) to[i / 4 + j] = w.x[j];
+        }
+        for (; i + 8 <= bytes; i += 8) {
+            const DecU2 w = *(const DecU2*)(from + i);
+            to[i / 4] = w.x[0];
+            to[i / 4 + 1] = w.x[1];
+        }
+        for (; i + 4 <= bytes; i += 4) to[i / 4] = *(const uint32_t*)(from + i);
+        if (i < bytes) to[i / 4] = *(const uint16_t*)(from + i);
+    }
+    // K row `row`, chunks 32 ks + 8 g
+    MX_DEV void load_k(int t, const void* base, size_t row, int g) {
+        const uint8_t* r = (const uint8_t*)base + row * ROWB;
+#pragma unroll
+        for (int k = 0; k < KS; ++k) copy(kc[t][k], r + (B8 ? 32 * k + 8 * g : 16 * k + 4 * g), B8 ? 8 : 4);
+        if constexpr (KVQ_) copy(ks[t], r + Q::CB + Q::HBB, KS * SB);
+        if constexpr (KVQ_ && Q::HB) copy(kh[t], r + Q::CB, 4 * KS);
+    }
+    // half hf of V row `row`
+    MX_DEV void load_v(const void* base, size_t row, int hf) {
+        const uint8_t* r = (const uint8_t*)base + row * ROWB;
+        constexpr int HC = D / 2 / (B8 ? 1 : 2);
+        copy(vc, r + hf * HC, HC);
+        if constexpr (KVQ_) copy(vs, r + Q::CB + Q::HBB + hf * (KS / 2 * SB), KS / 2 * SB);
+        if constexpr (KVQ_ && Q::HB) copy(vh, r + Q::CB + hf * (D / 16), D / 16);
+    }
+    static MX_DEV uint4 widen(uint32_t c0, uint32_t c1, const uint32_t* sw, int blk, uint32_t hb) {
+        if constexpr (KVF == KVF_FP8) return fp8x8_to_bf16x8(make_uint2(c0, c1));
+        else if constexpr (KVQ_) {
+            KVQRaw w;
+            w.c = make_uint2(c0, c1);
+            w.s = Q::MIN ? sw[blk] : (sw[blk >> 1] >> (16 * (blk & 1))) & 0xFFFF;
+            w.hb = hb;
+            return kvq_to_bf16x8<KVF>(w);
+        } else return make_uint4(0, 0, 0, 0);
+    }
+    MX_DEV bf16x8 k(int t, int k_, int g) const {
+        return __builtin_bit_cast(bf16x8, widen(kc[t][k_][0], B8 ? kc[t][k_][B8 ? 1 : 0] : 0u, ks[t], k_,
+                                                KVQ_ && Q::HB ? (kh[t][KVQ_ && Q::HB ? k_ : 0] >> (8 * g)) & 0xFF : 0u));
+    }
+    MX_DEV uint4 v(int j) const {  // elements 8 j .. of the half row
+        return widen(vc[B8 ? 2 * j : j], B8 ? vc[B8 ? 2 * j + 1 : 0] : 0u, vs, j >> 2,
+                     KVQ_ && Q::HB ? (vh[KVQ_ && Q::HB ? j >> 2 : 0] >> (8 * (j & 3))) & 0xFF : 0u);
+    }
+};
 template <int D, bool F16, int KVF, int NW = 4, bool TS = false, bool DPF = false>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
     (KVF != KVF_BF16 || (DPF && !TS && NW <= 8)) ? 2 : 4, (KVF != KVF_BF16 || (DPF && !TS && NW <= 8)) ? 2 : 4))) void attn_decode_mfma_kernel(
@@ -345,8 +425,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
     }
     DEC_TS(0)
     constexpr int KT = 32;                      // keys per wave tile
-    constexpr int VBYTES = KT * D * 2;
-    constexpr int PSTRIDE = (KT + 8) * 2;       // bytes per P row (padded)
     constexpr int WB = dec_wave_lds<D>();
     constexpr int NVC = KT * D / 8 / 64;        // 16-byte V chunks per lane per tile
     constexpr bool KV8 = KVF != KVF_BF16;       // a cache widened in registers (fp8 or block-quantised)
@@ -387,11 +465,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
     f32x4 oacc[D / 16];
 #pragma unroll
     for (int i = 0; i < D / 16; ++i) oacc[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    float mrow[4], lrow[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) { mrow[i] = -INFINITY; lrow[i] = 0.f; }
+    float mrow = -INFINITY, lrow = 0.f;  // of head `col`; lrow: this lane's keys
     char* v_lds = smem + wave * WB;
-    char* pw = v_lds + VBYTES;
     const char* kc = (const char*)kcv;
     const char* vc = (const char*)vcv;
 
@@ -411,10 +486,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
             const size_t eo = (PF || ok) ? (((size_t)sbt[kk / bs - blk0] * Hkv + kvh) * bs + kk % bs) * D : 0;
 #pragma unroll
             for (int ks = 0; ks < D / 32; ++ks) {
-                if constexpr (KV8) {
-                    kf_[t][ks] = ok ? __builtin_bit_cast(bf16x8, kv_widen8<KVF, D>(kc, eo + 32 * ks + 8 * g))
-                                    : (bf16x8){};
-                } else if constexpr (PF) {
+                if constexpr (PF) {
                     const bf16x8 w = *(const bf16x8*)(kc + (eo + 32 * ks + 8 * g) * ES);
                     kf_[t][ks] = ok ? w : (bf16x8){};
                 } else {
@@ -423,6 +495,20 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
             }
         }
     };
+    // 8-bit and block-quantised caches: a tile's bytes wait in registers (keys past the end: the last one again, P = 0)
+    [[maybe_unused]] DecRaw<KVF, D> raw;
+    auto load_raw = [&](int kt) {
+        auto row_of = [&](int key) {
+            const int kk = min(key, p1 - 1), bi = kk / bs;
+            return ((size_t)sbt[bi - blk0] * Hkv + kvh) * bs + (kk - bi * bs);
+        };
+#pragma unroll
+        for (int t = 0; t < 2; ++t) raw.load_k(t, kc, row_of(kt + 16 * t + col), g);
+        raw.load_v(vc, row_of(kt + (lane >> 1)), lane & 1);
+    };
+    if constexpr (KV8) {
+        if (p_start + wave * KT < p1) load_raw(p_start + wave * KT);
+    }
     [[maybe_unused]] bf16x8 knext[2][D / 32];
     if constexpr (PF) {
         if (p_start + wave * KT < p1) load_k(p_start + wave * KT, knext);
@@ -435,17 +521,30 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
             for (int t = 0; t < 2; ++t)
 #pragma unroll
                 for (int ks = 0; ks < D / 32; ++ks) kf[t][ks] = knext[t][ks];
+        } else if constexpr (KV8) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int ks = 0; ks < D / 32; ++ks) kf[t][ks] = raw.k(t, ks, g);
         } else {
             load_k(kt0, kf);
         }
         // V: bf16 caches go HBM -> LDS by DMA (global_load_lds, no VGPR staging): instruction j fills
         // bytes [1024 j, 1024 j + 1024) of the slice linearly by lane, so each lane fetches the chunk
-        // that the swizzled V image (v_lds_off) places at its slot; fp8 caches widen in registers.
-        [[maybe_unused]] uint4 vv[(KV8 || PF) ? NVC : 1];
+        // that the swizzled V image (v_lds_off) places at its slot; 8-bit caches widen in registers.
+        [[maybe_unused]] uint4 vv[PF ? NVC : 1];
+        if constexpr (KV8) {
 #pragma unroll
-        for (int j = 0; j < NVC; ++j) {
+            for (int j = 0; j < NVC; ++j) {
+                const int p = lane >> 1, c = (lane & 1) * (D / 16) + j;
+                *(uint4*)(v_lds + v_lds_off<D>(p, c >> 1) + 16 * (c & 1)) = raw.v(j);
+            }
+            if (kt0 + NW * KT < p1) load_raw(kt0 + NW * KT);
+        }
+#pragma unroll
+        for (int j = 0; j < (KV8 ? 0 : NVC); ++j) {
             int p, c;
-            if constexpr (KV8 || PF) {
+            if constexpr (PF) {
                 const int id = lane + 64 * j;
                 p = id / (D / 8);
                 c = id % (D / 8);
@@ -460,9 +559,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
             }
             const int key = kt0 + p < p1 ? kt0 + p : kt0;  // past the end: a valid row (P = 0 there)
             const size_t eo = (((size_t)sbt[key / bs - blk0] * Hkv + kvh) * bs + key % bs) * D + c * 8;
-            if constexpr (KV8) {
-                vv[j] = kt0 + p < p1 ? kv_widen8<KVF, D>(vc, eo) : make_uint4(0, 0, 0, 0);
-            } else if constexpr (PF) {
+            if constexpr (PF) {
                 vv[j] = *(const uint4*)(vc + eo * ES);  // rows past the end: a valid row, P = 0 there
             } else {
                 __builtin_amdgcn_global_load_lds((const void*)(vc + eo * ES), (MX_LDS void*)(v_lds + 1024 * j), 16, 0, 0);
@@ -477,80 +574,82 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
             if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NVC + NK) : "memory");
             else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NVC) : "memory");
         }
-        // ---- S = Q K^T : 16 head rows x 32 keys ----
+        // ---- S^T = K Q^T: 2 x 16 keys x 16 head columns; a lane holds keys 16 t + 4 g + i of head `col` ----
         f32x4 sacc[2];
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             sacc[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int ks = 0; ks < D / 32; ++ks)
-                sacc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qf[ks], kf[t][ks], sacc[t], 0, 0, 0);
+                sacc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t][ks], qf[ks], sacc[t], 0, 0, 0);
         }
         if constexpr (TS) {
             if (kt0 == p_start) DEC_TS(3)  // the K tile has landed (first tile of wave 0)
         }
-        if constexpr (KV8 || PF) {  // V -> this wave's LDS slice (the previous tile's reads have returned)
+        if constexpr (PF) {  // V -> this wave's LDS slice (the previous tile's reads have returned)
 #pragma unroll
             for (int j = 0; j < NVC; ++j) {
                 const int id = lane + 64 * j, p = id / (D / 8), c = id % (D / 8);
                 *(uint4*)(v_lds + v_lds_off<D>(p, c >> 1) + 16 * (c & 1)) = vv[j];
             }
         }
-        // ---- online softmax over the tile (rows 4g+i, keys 16t+col) ----
-        float alpha[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float mx = -INFINITY;
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                float v = sacc[t][i] * qs;
-                if (softcap > 0.f) v = sc_l2 * tanhf(v * sc_inv);
-                if (kt0 + 16 * t + col >= p1) v = -INFINITY;
-                sacc[t][i] = v;
-                mx = fmaxf(mx, v);
-            }
-            mx = group_max<16>(mx);
-            const float mn = fmaxf(mrow[i], mx);
-            alpha[i] = mn == -INFINITY ? 1.f : exp2f(mrow[i] - mn);
-            float rs = 0.f;
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const float pv = mn == -INFINITY ? 0.f : exp2f(sacc[t][i] - mn);
-                sacc[t][i] = pv;
-                rs += pv;
-            }
-            lrow[i] = lrow[i] * alpha[i] + group_sum<16>(rs);
-            mrow[i] = mn;
-        }
-#pragma unroll
-        for (int nt = 0; nt < D / 16; ++nt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) oacc[nt][i] *= alpha[i];
+        // ---- online softmax over the tile: the head's maximum over its four lanes, everything else lane-local ----
+        float mx = -INFINITY;
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                *(bf16_t*)(pw + (4 * g + i) * PSTRIDE + (16 * t + col) * 2) = f32_to_bf16(sacc[t][i]);
-        // the V DMA has landed and the P (and fp8 V) writes are visible (PF: the next tile's K may stay in flight)
+            for (int i = 0; i < 4; ++i) {
+                float v = sacc[t][i] * qs;
+                if (softcap > 0.f) v = sc_l2 * tanhf(v * sc_inv);
+                if (kt0 + 16 * t + 4 * g + i >= p1) v = -INFINITY;
+                sacc[t][i] = v;
+                mx = fmaxf(mx, v);
+            }
+        const float mn = fmaxf(mrow, quarters_max(mx));
+        if (__any(mn > mrow)) {
+            const float alpha = mn == -INFINITY ? 1.f : exp2f(mrow - mn);
+            lrow *= alpha;
+#pragma unroll
+            for (int nt = 0; nt < D / 16; ++nt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) oacc[nt][i] *= alpha;
+            mrow = mn;
+        }
+        u32x4 pw;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            float pv[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                pv[i] = mn == -INFINITY ? 0.f : exp2f(sacc[t][i] - mn);
+                lrow += pv[i];
+            }
+            pw[2 * t] = pack_bf16x2(pv[0], pv[1]);
+            pw[2 * t + 1] = pack_bf16x2(pv[2], pv[3]);
+        }
+        // P^T as B operand: k slot (g, e) is key 16 (e / 4) + 4 g + e % 4, and V^T's rows are read in that order
+        const bf16x8 pb = __builtin_bit_cast(bf16x8, pw);
+        // the V DMA has landed and the V writes are visible (PF, 8-bit caches: the next tile's loads may stay in flight)
         if constexpr (PF) {
             if (more) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(NK) : "memory");
             else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        } else if constexpr (KV8) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         } else {
             __builtin_amdgcn_s_waitcnt(0);
         }
         __builtin_amdgcn_wave_barrier();
-        // ---- O += P V ----
-        const bf16x8 pa = *(const bf16x8*)(pw + col * PSTRIDE + 8 * g * 2);
-        const int r0 = 8 * g, q4 = col >> 2, p4 = col & 3;
+        // ---- O^T += V^T P^T ----
+        const int r0 = 4 * g, q4 = col >> 2, p4 = col & 3;
 #pragma unroll
         for (int nt = 0; nt < D / 16; ++nt) {
             const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                 (MX_LDS s16x4*)(v_lds + v_lds_off<D>(r0 + q4, nt) + 8 * p4));
             const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (MX_LDS s16x4*)(v_lds + v_lds_off<D>(r0 + 4 + q4, nt) + 8 * p4));
+                (MX_LDS s16x4*)(v_lds + v_lds_off<D>(r0 + 16 + q4, nt) + 8 * p4));
             const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
             const u32x4 w4 = {l2[0], l2[1], h2[0], h2[1]};
-            oacc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, __builtin_bit_cast(bf16x8, w4), oacc[nt], 0, 0, 0);
+            oacc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w4), pb, oacc[nt], 0, 0, 0);
         }
         __builtin_amdgcn_s_waitcnt(0xc07f);  // the transposed reads have returned before V is rewritten
         __builtin_amdgcn_wave_barrier();
@@ -563,15 +662,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
     float* wml = (float*)(smem + NW * WB) + wave * 32;  // [16 rows] m, [16 rows] l
     // waves past the context's last tile hold nothing (m = -inf, l = 0): neither written nor read
     const int nwa = p1 > p_start ? min(NW, (p1 - p_start + KT - 1) / KT) : 0;
-    if (wave < nwa) {
+    lrow = quarters_sum(lrow);
+    if (wave < nwa && col < G) {  // only the G real heads of the 16 columns
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int r = 4 * g + i;
-            if (r >= G) continue;  // only the G real head rows of the 16-row tile
-#pragma unroll
-            for (int nt = 0; nt < D / 16; ++nt) wo[r * D + 16 * nt + col] = oacc[nt][i];
-            if (col == 0) { wml[r] = mrow[i]; wml[16 + r] = lrow[i]; }
-        }
+        for (int nt = 0; nt < D / 16; ++nt)
+            *(float4*)(wo + col * D + 16 * nt + 4 * g) = make_float4(oacc[nt][0], oacc[nt][1], oacc[nt][2], oacc[nt][3]);
+        if (g == 0) { wml[col] = mrow; wml[16 + col] = lrow; }
     }
     __syncthreads();
     DEC_TS(6)

@@ -103,3 +103,22 @@ def test_infinite_scores_behave_like_the_reference():
     K.attn_prefill(q.cuda(), kc.cuda(), vc.cuda(), bt.cuda(), cu.cuda(), ctx.cuda(), 1 / math.sqrt(128), out)
     got = out.cpu().float()
     assert torch.isfinite(got[:40]).all() and torch.isnan(got[40:]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", ["bf16", "fp8", "q8_0", "q4_0", "q4_1", "q5_0", "q5_1", "iq4_nl"])
+@pytest.mark.parametrize("Hq,Hkv,D", [(32, 8, 128), (8, 1, 64), (6, 2, 128), (16, 1, 128)])
+def test_decode_rows(fmt, Hq, Hkv, D):
+    """One row per sequence: contexts around the 32-key tiles of a wave, the tiles of a workgroup and the partitions."""
+    pre = [0, 31, 32, 33, 126, 127, 128, 512, 700, 1500]
+    q, kc, vc, bt, _, ctx = _case(Hq, Hkv, D, [1] * len(pre), pre, fmt=fmt)
+    want = torch.stack([K._attn_ref_one(q[i:i + 1], kc, vc, bt[i], int(c), int(c) - 1, D ** -0.5, 16)[0] for i, c in enumerate(ctx)])
+    kd, vd = kc.cuda(), vc.cuda()
+    if hasattr(kc, "kvf"):
+        kd.kvf, vd.kvf = kc.kvf, vc.kvf
+    for rows, part in ((slice(None), 256), (slice(None), 128), (slice(None), 1024), (slice(6, 10), 512), (slice(6, 10), 256)):
+        out = torch.full((len(ctx[rows]), Hq, D), float("nan"), dtype=torch.float16, device="cuda")
+        K.attn_decode(q[rows].cuda(), kd, vd, bt[rows].contiguous().cuda(), ctx[rows].cuda(), D ** -0.5, out, part_size=part)
+        got = out.cpu().float()
+        # as for prompts: probabilities and outputs are rounded to 16 bits once each
+        assert float((got - want[rows]).norm() / want[rows].norm()) < 4 * 2 ** -9, part
