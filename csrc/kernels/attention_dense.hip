@@ -52,7 +52,8 @@ __global__ __launch_bounds__(256) void attn_dense_kernel(const uint16_t* __restr
                                                          uint16_t* __restrict__ o, int o_stride, int Sq, int Sk,
                                                          int Hq, int Hkv, const int* __restrict__ qlen_b,
                                                          const int* __restrict__ klen_b, int causal, float scale,
-                                                         int kv_rows, const float* __restrict__ rbias, int rb_ld) {
+                                                         int kv_rows, const float* __restrict__ rbias, int rb_ld,
+                                                         const int* __restrict__ cu) {
     // key tile: 64 keys (D <= 128) or 32 (D = 512: the VAE mid-block's single 512-wide head; K + V tiles 64 KB)
     constexpr int KT = D > 128 ? 32 : 64;
     constexpr int KBYTES = KT * D * 2;
@@ -64,7 +65,9 @@ __global__ __launch_bounds__(256) void attn_dense_kernel(const uint16_t* __restr
     const int g = lane >> 4, col = lane & 15;
     const int b = blockIdx.z, h = blockIdx.y;
     const int kvh = h / (Hq / Hkv);
-    const int qlen = qlen_b ? qlen_b[b] : Sq;
+    // ragged batches: sequence b's rows are cu[b] .. cu[b + 1], keys and queries alike
+    const size_t q_row = cu ? (size_t)cu[b] : (size_t)b * Sq, k_row = cu ? (size_t)cu[b] : (size_t)b * kv_rows;
+    const int qlen = cu ? cu[b + 1] - cu[b] : qlen_b ? qlen_b[b] : Sq;
     const int klen = klen_b ? klen_b[b] : Sk;
     const int row_q0 = blockIdx.x * 64 + wave * 16;
     if (blockIdx.x * 64 >= qlen) return;  // whole workgroup idle (uniform)
@@ -72,15 +75,15 @@ __global__ __launch_bounds__(256) void attn_dense_kernel(const uint16_t* __restr
     int kv_end = klen;
     if (causal) kv_end = min(kv_end, blockIdx.x * 64 + 64 + shift);
     const float qs = scale * LOG2E_D;
-    const uint16_t* kb = k + (size_t)b * kv_rows * k_stride + (size_t)kvh * D;
-    const uint16_t* vb_ = v + (size_t)b * kv_rows * v_stride + (size_t)kvh * D;
+    const uint16_t* kb = k + k_row * k_stride + (size_t)kvh * D;
+    const uint16_t* vb_ = v + k_row * v_stride + (size_t)kvh * D;
 
     u32x4 qf[D / 32];
     {
         const int qi = row_q0 + col;
 #pragma unroll
         for (int ks = 0; ks < D / 32; ++ks) {
-            if (qi < qlen) qf[ks] = *(const u32x4*)(q + ((size_t)b * Sq + qi) * q_stride + (size_t)h * D + 32 * ks + 8 * g);
+            if (qi < qlen) qf[ks] = *(const u32x4*)(q + (q_row + qi) * q_stride + (size_t)h * D + 32 * ks + 8 * g);
             else qf[ks] = (u32x4){0, 0, 0, 0};
         }
     }
@@ -205,7 +208,7 @@ __global__ __launch_bounds__(256) void attn_dense_kernel(const uint16_t* __restr
         const float inv = lrow[i] > 0.f ? 1.f / lrow[i] : 0.f;
 #pragma unroll
         for (int nt = 0; nt < D / 16; ++nt)
-            o[((size_t)b * Sq + qi) * o_stride + (size_t)h * D + 16 * nt + col] = f32_to_act<F16>(oacc[nt][i] * inv);
+            o[(q_row + qi) * o_stride + (size_t)h * D + 16 * nt + col] = f32_to_act<F16>(oacc[nt][i] * inv);
     }
 }
 
@@ -225,13 +228,33 @@ extern "C" int mxk_attn_dense(const uint16_t* q, int q_stride, const uint16_t* k
     MX_ACT_DISPATCH({
         if (D == 512)
             attn_dense_kernel<512, F16><<<grid, 256, 0, st>>>(q, q_stride, k, k_stride, v, v_stride, o, o_stride, Sq, Sk,
-                                                             Hq, Hkv, qlen, klen, causal, scale, kv_rows, rbias, rb_ld);
+                                                             Hq, Hkv, qlen, klen, causal, scale, kv_rows, rbias, rb_ld, nullptr);
         else if (D == 128)
             attn_dense_kernel<128, F16><<<grid, 256, 0, st>>>(q, q_stride, k, k_stride, v, v_stride, o, o_stride, Sq, Sk,
-                                                             Hq, Hkv, qlen, klen, causal, scale, kv_rows, rbias, rb_ld);
+                                                             Hq, Hkv, qlen, klen, causal, scale, kv_rows, rbias, rb_ld, nullptr);
         else
             attn_dense_kernel<64, F16><<<grid, 256, 0, st>>>(q, q_stride, k, k_stride, v, v_stride, o, o_stride, Sq, Sk,
-                                                            Hq, Hkv, qlen, klen, causal, scale, kv_rows, rbias, rb_ld);
+                                                            Hq, Hkv, qlen, klen, causal, scale, kv_rows, rbias, rb_ld, nullptr);
+    });
+    MXK_CHECK_LAUNCH();
+}
+
+// Rows packed without padding (BERT): sequence b of B has rows cu[b] .. cu[b + 1] (at most Smax) of q, k, v and o, and sees
+// its first klen[b] keys; D in {64, 128}.
+extern "C" int mxk_attn_dense_ragged(const uint16_t* q, int q_stride, const uint16_t* k, int k_stride, const uint16_t* v,
+                                     int v_stride, uint16_t* o, int o_stride, int B, int Smax, int H, int D, const int* cu,
+                                     const int* klen, float scale, hipStream_t st) {
+    if (B <= 0 || Smax <= 0) return 0;
+    if ((D != 64 && D != 128) || B > 65535 || !cu || !klen) return (int)hipErrorInvalidValue;
+    if ((q_stride | k_stride | v_stride) & 7) return (int)hipErrorInvalidValue;
+    dim3 grid((Smax + 63) / 64, H, B);
+    MX_ACT_DISPATCH({
+        if (D == 128)
+            attn_dense_kernel<128, F16><<<grid, 256, 0, st>>>(q, q_stride, k, k_stride, v, v_stride, o, o_stride, Smax, Smax,
+                                                             H, H, nullptr, klen, 0, scale, 0, nullptr, 0, cu);
+        else
+            attn_dense_kernel<64, F16><<<grid, 256, 0, st>>>(q, q_stride, k, k_stride, v, v_stride, o, o_stride, Smax, Smax, H,
+                                                            H, nullptr, klen, 0, scale, 0, nullptr, 0, cu);
     });
     MXK_CHECK_LAUNCH();
 }

@@ -1,0 +1,339 @@
+// encoder.hip — post-norm text encoders (BERT) on packed rows: the texts of a batch one after another, no padding rows.
+//
+// A layer is four GEMMs, attention (attention_dense.hip) and two LayerNorms. Batches of few rows are bound by launches
+// and by the time a workgroup waits for its first loads, large ones by the GEMMs and by the passes between them; so
+//   - few rows run whole layers from one call (mxk_enc_layers), with a GEMM that splits K over the waves of a workgroup
+//     and applies bias and GELU to its fp32 sums;
+//   - above, the caller multiplies with the library and the passes between are one kernel each, over 16-bit rows.
+// Measured on BERT-base, against padded rows with fp32 copies around each LayerNorm and a library call per operation: one
+// text of 19 tokens 2024 -> 488 us (87 launches of 4-7 us), 48 texts of 23-401 tokens (6427 rows of 19248 padded) 7317 ->
+// 2574: LayerNorm + casts 74 -> 8.3 us (30 MB: 3.6 TB/s), GELU 40 -> 16 (79 MB: 4.9 TB/s).
+#include "mx_common.h"
+
+#include <type_traits>
+
+namespace {
+
+constexpr int EW = 4;   // rows (waves) per workgroup of the row kernels
+constexpr int GW = 8;   // waves per workgroup of the GEMM
+
+// LayerNorm of one row held by a wave: lane has the 8-element chunks lane + 64 j. Two passes over registers: the
+// variance is a sum of squares about the mean.
+template <int NC, bool F16>
+MX_DEV void ln_row(float (&v)[NC][8], int H, const float* __restrict__ g, const float* __restrict__ b, float eps,
+                   uint16_t* __restrict__ out, int lane) {
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < NC; ++j)
+        if (8 * (lane + 64 * j) < H)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s += v[j][e];
+    const float mean = wave_sum(s) / H;
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < NC; ++j)
+        if (8 * (lane + 64 * j) < H)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ss += (v[j][e] - mean) * (v[j][e] - mean);
+    const float rs = rsqrtf(wave_sum(ss) / H + eps);
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+        const int c = 8 * (lane + 64 * j);
+        if (c >= H) continue;
+        float y[8];
+#pragma unroll
+        for (int e = 0; e < 8; e += 4) {
+            const float4 gv = *(const float4*)(g + c + e);
+            const float4 bv = b ? *(const float4*)(b + c + e) : make_float4(0.f, 0.f, 0.f, 0.f);
+            y[e] = (v[j][e] - mean) * rs * gv.x + bv.x;
+            y[e + 1] = (v[j][e + 1] - mean) * rs * gv.y + bv.y;
+            y[e + 2] = (v[j][e + 2] - mean) * rs * gv.z + bv.z;
+            y[e + 3] = (v[j][e + 3] - mean) * rs * gv.w + bv.w;
+        }
+        *(uint4*)(out + c) = make_uint4(pack_act2<F16>(y[0], y[1]), pack_act2<F16>(y[2], y[3]), pack_act2<F16>(y[4], y[5]),
+                                        pack_act2<F16>(y[6], y[7]));
+    }
+}
+
+template <int NC>
+MX_DEV void add_f32(float (&v)[NC][8], const float* __restrict__ p, int H, int lane) {
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+        const int c = 8 * (lane + 64 * j);
+        if (c >= H) continue;
+        const float4 a = *(const float4*)(p + c), b = *(const float4*)(p + c + 4);
+        v[j][0] += a.x;
+        v[j][1] += a.y;
+        v[j][2] += a.z;
+        v[j][3] += a.w;
+        v[j][4] += b.x;
+        v[j][5] += b.y;
+        v[j][6] += b.z;
+        v[j][7] += b.w;
+    }
+}
+
+template <int NC, bool F16>
+MX_DEV void add_act(float (&v)[NC][8], const uint16_t* __restrict__ p, int H, int lane) {
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+        const int c = 8 * (lane + 64 * j);
+        if (c >= H) continue;
+        const uint4 w = *(const uint4*)(p + c);
+        const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float lo, hi;
+            unpack_act2<F16>(ws[e], lo, hi);
+            v[j][2 * e] += lo;
+            v[j][2 * e + 1] += hi;
+        }
+    }
+}
+
+// x = LN(tok[id] + pos[p] + typ[t]); ids: [3][rows] token, position, type (typ null: no type table)
+template <int NC, bool F16>
+__global__ __launch_bounds__(64 * EW) void enc_embed_kernel(const int* __restrict__ ids, int rows, const float* __restrict__ tok,
+                                                            const float* __restrict__ pos, const float* __restrict__ typ,
+                                                            const float* __restrict__ g, const float* __restrict__ b, int H,
+                                                            float eps, uint16_t* __restrict__ x) {
+    const int row = blockIdx.x * EW + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (row >= rows) return;
+    float v[NC][8] = {};
+    add_f32<NC>(v, tok + (size_t)ids[row] * H, H, lane);
+    add_f32<NC>(v, pos + (size_t)ids[rows + row] * H, H, lane);
+    if (typ) add_f32<NC>(v, typ + (size_t)ids[2 * rows + row] * H, H, lane);
+    ln_row<NC, F16>(v, H, g, b, eps, x + (size_t)row * H, lane);
+}
+
+// x = LN(a + x): the residual sum in fp32, one pass over 16-bit rows
+template <int NC, bool F16>
+__global__ __launch_bounds__(64 * EW) void enc_add_ln_kernel(const uint16_t* __restrict__ a, uint16_t* __restrict__ x, int rows,
+                                                             const float* __restrict__ g, const float* __restrict__ b, int H,
+                                                             float eps) {
+    const int row = blockIdx.x * EW + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (row >= rows) return;
+    float v[NC][8] = {};
+    add_act<NC, F16>(v, a + (size_t)row * H, H, lane);
+    add_act<NC, F16>(v, x + (size_t)row * H, H, lane);
+    ln_row<NC, F16>(v, H, g, b, eps, x + (size_t)row * H, lane);
+}
+
+// y = gelu(y) in place, 8 elements a thread
+template <bool F16>
+__global__ __launch_bounds__(256) void enc_gelu_kernel(uint16_t* __restrict__ y, long n8) {
+    const long i = (long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n8) return;
+    uint4 w = ((uint4*)y)[i];
+    uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        float lo, hi;
+        unpack_act2<F16>(ws[e], lo, hi);
+        ws[e] = pack_act2<F16>(gelu_erf_f(lo), gelu_erf_f(hi));
+    }
+    ((uint4*)y)[i] = make_uint4(ws[0], ws[1], ws[2], ws[3]);
+}
+
+// One text per workgroup -> e [H] fp32. mode 0: mean over its klen rows, 1: first row, 2: last row; then / max(|e|, 1e-12).
+// A thread sums pairs of columns over every 4th row (a text of 400 rows x 768: 0.6 MB).
+template <bool F16>
+__global__ __launch_bounds__(1024) void enc_pool_kernel(const uint16_t* __restrict__ x, const int* __restrict__ cu,
+                                                        const int* __restrict__ klen, int H, int mode, int norm,
+                                                        float* __restrict__ e) {
+    __shared__ float part[4][512];
+    __shared__ float red[16];
+    const int b = blockIdx.x, r0 = cu[b], n = cu[b + 1] - r0, live = klen[b];
+    const int grp = threadIdx.x >> 8, t = threadIdx.x & 255;
+    const int lo = mode == 2 ? n - 1 : 0, hi = mode == 0 ? live : lo + 1;
+    const float cnt = mode == 0 ? (float)max(live, 1) : 1.f;
+    float sq = 0.f;
+    for (int c0 = 0; c0 < H; c0 += 512) {
+        const int c = c0 + 2 * t;
+        float s0 = 0.f, s1 = 0.f;
+        if (c < H)
+            for (int r = lo + grp; r < hi; r += 4) {
+                float a, d;
+                unpack_act2<F16>(*(const uint32_t*)(x + (size_t)(r0 + r) * H + c), a, d);
+                s0 += a;
+                s1 += d;
+            }
+        part[grp][2 * t] = s0;
+        part[grp][2 * t + 1] = s1;
+        __syncthreads();
+        if (threadIdx.x < 512 && c0 + (int)threadIdx.x < H) {
+            const float v = ((part[0][threadIdx.x] + part[1][threadIdx.x]) + (part[2][threadIdx.x] + part[3][threadIdx.x])) / cnt;
+            e[(size_t)b * H + c0 + threadIdx.x] = v;
+            sq += v * v;
+        }
+        __syncthreads();
+    }
+    if (!norm) return;
+    const float ws = wave_sum(sq);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ws;
+    __syncthreads();
+    float tot = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) tot += red[i];  // (waves 8 .. 15 hold no columns)
+    const float nr = fmaxf(sqrtf(tot), 1e-12f);
+    for (int c0 = 0; c0 < H; c0 += 512)
+        if (threadIdx.x < 512 && c0 + (int)threadIdx.x < H) e[(size_t)b * H + c0 + threadIdx.x] /= nr;
+}
+
+template <bool F16>
+MX_DEV f32x4 enc_mfma(uint4 a, uint4 b, f32x4 c) {
+    if constexpr (F16)
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// y[M, N] = act(x[M, K] W[N, K]^T + bias), 16-bit in and out, fp32 sums. A workgroup has 16 columns and 16 MT rows; its 8
+// waves take every 8th 32-wide k-step and their sums meet in LDS. What bounds it is the wait for the first loads: a wave
+// asks for U k-steps at once (all three of K = 768). Rows past M read row M - 1 and are not stored.
+template <int MT, bool F16, bool GELU>
+__global__ __launch_bounds__(64 * GW) void enc_gemm_kernel(const uint16_t* __restrict__ x, int ldx, const uint16_t* __restrict__ W,
+                                                           const uint16_t* __restrict__ bias, uint16_t* __restrict__ y, int ldy,
+                                                           int M, int N, int K) {
+    __shared__ float red[GW * MT * 256];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * 16, m0 = blockIdx.y * (16 * MT), KS = K / 32;
+    const uint16_t* wp = W + (size_t)(n0 + col) * K + 8 * g;
+    const uint16_t* xp[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) xp[t] = x + (size_t)min(m0 + 16 * t + col, M - 1) * ldx + 8 * g;
+    f32x4 acc[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    auto steps = [&](int s, auto uc) {
+        constexpr int U = decltype(uc)::value;
+        uint4 wf[U], xf[U][MT];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            wf[u] = *(const uint4*)(wp + 32 * (s + GW * u));
+#pragma unroll
+            for (int t = 0; t < MT; ++t) xf[u][t] = *(const uint4*)(xp[t] + 32 * (s + GW * u));
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) acc[t] = enc_mfma<F16>(xf[u][t], wf[u], acc[t]);
+    };
+    constexpr int U = MT <= 2 ? 6 : 3;
+    int s = wave;
+    for (; s + GW * (U - 1) < KS; s += GW * U) steps(s, std::integral_constant<int, U>{});
+    if (U > 3 && s + GW * 2 < KS) {
+        steps(s, std::integral_constant<int, 3>{});
+        s += GW * 3;
+    }
+    for (; s < KS; s += GW) steps(s, std::integral_constant<int, 1>{});
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+        *(float4*)(red + ((wave * MT + t) * 64 + lane) * 4) = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < MT * 256; idx += 64 * GW) {
+        const int n = idx & 15, r = idx >> 4, m = m0 + r;
+        if (m >= M) continue;
+        const int e = (r >> 4) * 256 + (((r & 15) >> 2) * 16 + n) * 4 + (r & 3);
+        float v = 0.f;
+#pragma unroll
+        for (int w = 0; w < GW; ++w) v += red[w * MT * 256 + e];
+        if (bias) v += act_to_f32<F16>(bias[n0 + n]);
+        if constexpr (GELU) v = gelu_erf_f(v);
+        y[(size_t)m * ldy + n0 + n] = f32_to_act<F16>(v);
+    }
+}
+
+template <bool F16>
+int enc_gemm(const uint16_t* x, int ldx, const uint16_t* W, const uint16_t* bias, uint16_t* y, int ldy, int M, int N, int K,
+             int gelu, hipStream_t st) {
+    const int mt = min(4, (M + 15) / 16);
+#define EG(MT_)                                                                                                        \
+    if (mt == MT_) {                                                                                                   \
+        const dim3 grid(N / 16, (M + 16 * MT_ - 1) / (16 * MT_));                                                      \
+        if (gelu) enc_gemm_kernel<MT_, F16, true><<<grid, 64 * GW, 0, st>>>(x, ldx, W, bias, y, ldy, M, N, K);          \
+        else enc_gemm_kernel<MT_, F16, false><<<grid, 64 * GW, 0, st>>>(x, ldx, W, bias, y, ldy, M, N, K);              \
+    }
+    EG(1) EG(2) EG(3) EG(4)
+#undef EG
+    return (int)hipGetLastError();
+}
+
+// chunks of a row per lane: H <= 512 NC
+#define ENC_NC(H, ...)                                \
+    do {                                              \
+        if ((H) <= 1024) { constexpr int NC = 2; __VA_ARGS__; } \
+        else { constexpr int NC = 8; __VA_ARGS__; }   \
+    } while (0)
+
+int enc_add_ln(const uint16_t* a, uint16_t* x, int rows, const float* g, const float* b, int H, float eps, hipStream_t st) {
+    MX_ACT_DISPATCH(ENC_NC(H, enc_add_ln_kernel<NC, F16><<<(rows + EW - 1) / EW, 64 * EW, 0, st>>>(a, x, rows, g, b, H, eps)));
+    return (int)hipGetLastError();
+}
+
+bool enc_width_ok(int H) { return H > 0 && H % 8 == 0 && H <= 4096; }
+
+}  // namespace
+
+extern "C" int mxk_attn_dense_ragged(const uint16_t* q, int q_stride, const uint16_t* k, int k_stride, const uint16_t* v,
+                                     int v_stride, uint16_t* o, int o_stride, int B, int Smax, int H, int D, const int* cu,
+                                     const int* klen, float scale, hipStream_t st);
+
+extern "C" int mxk_enc_embed(const int* ids, int rows, const float* tok, const float* pos, const float* typ, const float* g,
+                             const float* b, int H, float eps, uint16_t* x, hipStream_t st) {
+    if (rows <= 0) return 0;
+    if (!enc_width_ok(H)) return (int)hipErrorInvalidValue;
+    MX_ACT_DISPATCH(ENC_NC(H, enc_embed_kernel<NC, F16><<<(rows + EW - 1) / EW, 64 * EW, 0, st>>>(ids, rows, tok, pos, typ, g, b,
+                                                                                                 H, eps, x)));
+    MXK_CHECK_LAUNCH();
+}
+
+extern "C" int mxk_enc_add_ln(const uint16_t* a, uint16_t* x, int rows, const float* g, const float* b, int H, float eps,
+                              hipStream_t st) {
+    if (rows <= 0) return 0;
+    if (!enc_width_ok(H)) return (int)hipErrorInvalidValue;
+    return enc_add_ln(a, x, rows, g, b, H, eps, st);
+}
+
+extern "C" int mxk_enc_gelu(uint16_t* y, long long n, hipStream_t st) {
+    if (n <= 0) return 0;
+    if (n % 8) return (int)hipErrorInvalidValue;
+    const long n8 = n / 8;
+    MX_ACT_DISPATCH(enc_gelu_kernel<F16><<<(unsigned)((n8 + 255) / 256), 256, 0, st>>>(y, n8));
+    MXK_CHECK_LAUNCH();
+}
+
+extern "C" int mxk_enc_pool(const uint16_t* x, const int* cu, const int* klen, int B, int H, int mode, int norm, float* e,
+                            hipStream_t st) {
+    if (B <= 0) return 0;
+    if (H <= 0 || H % 2 || mode < 0 || mode > 2) return (int)hipErrorInvalidValue;
+    MX_ACT_DISPATCH(enc_pool_kernel<F16><<<B, 1024, 0, st>>>(x, cu, klen, H, mode, norm, e));
+    MXK_CHECK_LAUNCH();
+}
+
+// w: 12 device pointers a layer: qkv W, b, output W, b, norm g, b (fp32), up W, b, down W, b, norm g, b (fp32); biases may be
+// null. x [rows][H] in and out; qkv [rows][3 H], attn and proj [rows][H], up [rows][F] are scratch.
+extern "C" int mxk_enc_layers(const void* const* w, int n_layers, uint16_t* x, int rows, int B, int Smax, const int* cu,
+                              const int* klen, int H, int heads, int F, float scale, float eps, uint16_t* qkv, uint16_t* attn,
+                              uint16_t* proj, uint16_t* up, hipStream_t st) {
+    if (rows <= 0 || n_layers <= 0) return 0;
+    if (!enc_width_ok(H) || H % 32 || F % 32 || heads <= 0 || H % heads) return (int)hipErrorInvalidValue;
+    for (int l = 0; l < n_layers; ++l, w += 12) {
+        auto gemm = [&](const uint16_t* a, int i, uint16_t* y, int N, int K, int gelu) {
+            const uint16_t *W = (const uint16_t*)w[i], *b = (const uint16_t*)w[i + 1];
+            int rc = 0;
+            MX_ACT_DISPATCH(rc = enc_gemm<F16>(a, K, W, b, y, N, rows, N, K, gelu, st));
+            return rc;
+        };
+        int rc = gemm(x, 0, qkv, 3 * H, H, 0);
+        if (!rc) rc = mxk_attn_dense_ragged(qkv, 3 * H, qkv + H, 3 * H, qkv + 2 * H, 3 * H, attn, H, B, Smax, heads, H / heads, cu,
+                                            klen, scale, st);
+        if (!rc) rc = gemm(attn, 2, proj, H, H, 0);
+        if (!rc) rc = enc_add_ln(proj, x, rows, (const float*)w[4], (const float*)w[5], H, eps, st);
+        if (!rc) rc = gemm(x, 6, up, F, H, 1);
+        if (!rc) rc = gemm(up, 8, proj, H, F, 0);
+        if (!rc) rc = enc_add_ln(proj, x, rows, (const float*)w[10], (const float*)w[11], H, eps, st);
+        if (rc) return rc;
+    }
+    return 0;
+}

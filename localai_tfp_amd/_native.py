@@ -53,6 +53,13 @@ KERNEL_SIGS = {
     "mxk_set_act_f16": [I],
     "mxk_attn_dense": [P, I, P, I, P, I, P, I, I, I, I, I, I, I, P, P, I, F, I, P, I, P],
     "mxk_get_act_f16": [],
+    # encoder.hip: packed text encoders
+    "mxk_enc_embed": [P, I, P, P, P, P, P, I, F, P, P],
+    "mxk_enc_add_ln": [P, P, I, P, P, I, F, P],
+    "mxk_enc_gelu": [P, C.c_longlong, P],
+    "mxk_enc_pool": [P, P, P, I, I, I, I, P, P],
+    "mxk_enc_layers": [P, I, P, I, I, I, P, P, I, I, I, F, F, P, P, P, P, P],
+    "mxk_attn_dense_ragged": [P, I, P, I, P, I, P, I, I, I, I, I, P, P, F, P],
     "mxk_qgemv": [I, I, P, P, P, P, I, I, I, P, I, P],
     "mxk_dequant_rows": [I, P, P, P, I, I, P, P, I, P],
     "mxk_rope_kv": [P, P, P, P, P, F, I, I, I, I, I, I, P, P, P, I, P, P, F, I, I, P],

@@ -114,3 +114,34 @@ def test_bert_gpu_matches_fp32():
     e = g.embed(seqs).cpu()
     c = BM.BertModel.load(cfg, get, "cpu").embed(seqs)
     assert (e - c).abs().max() < 1e-2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hidden,heads,ffn,pooling", [(256, 4, 1024, "mean"), (128, 1, 160, "last"), (1056, 11, 96, "mean"),
+                                                      (768, 12, 3072, "cls")])
+def test_packed_rows_match_fp32(hidden, heads, ffn, pooling, monkeypatch):
+    """Packed texts (encoder.hip) at the edges of its 16-row tiles, one-call and library GEMMs, against the fp32 encoder: hidden
+    rows within the bound of 16-bit activations (a LayerNorm output of up to ~5 is rounded to 2^-11 of itself some 8 times a
+    layer, 3e-3 each), pooled unit vectors ten times closer. Head dims it does not take (1056 / 11 = 96) run padded."""
+    cfg = BM.BertConfig(vocab=400, hidden=hidden, n_layers=2, n_heads=heads, ffn=ffn, max_pos=256, pooling=pooling, name="t")
+    get = BM.synthetic_bert(cfg, 5)
+    g, c = BM.BertModel.load(cfg, get, "cuda:0"), BM.BertModel.load(cfg, get, "cpu")
+    assert (g._packed_weights([[1]]) is None) == (hidden == 1056)
+    gen = torch.Generator().manual_seed(1)
+    for lens in ([1], [16], [17], [1, 63, 64, 65, 3], [200, 2, 31]):
+        ids = [torch.randint(0, 400, (n,), generator=gen).tolist() for n in lens]
+        want, _ = c.encode(ids)
+        for rows in (0, 4096):  # library GEMMs, the one-call layers
+            monkeypatch.setattr(BM, "ENC_SMALL_ROWS", rows)
+            hid, n = g.encode(ids)
+            assert n.tolist() == lens and hid.shape == want.shape and hid.dtype == torch.float32
+            for b, k in enumerate(lens):
+                assert (hid[b, :k].cpu() - want[b, :k]).abs().max() < 5e-2
+            assert (g.embed(ids).cpu() - c.embed(ids)).abs().max() < 5e-3
+            assert (g.embed(ids, normalize=False).cpu() - c.embed(ids, normalize=False)).abs().max() < 5e-2
+    if hidden != 1056:
+        with pytest.raises(IndexError):
+            g.embed([[400]])
+        with pytest.raises(IndexError):
+            g.embed([[1] * 257])
+    assert g.embed([[5, 6], []]).shape == (2, hidden)
