@@ -6,16 +6,18 @@
 //     and applies bias and GELU to its fp32 sums;
 //   - above, the caller multiplies with the library and the passes between are one kernel each, over 16-bit rows.
 // Measured on BERT-base, against padded rows with fp32 copies around each LayerNorm and a library call per operation: one
-// text of 19 tokens 2024 -> 488 us (87 launches of 4-7 us), 48 texts of 23-401 tokens (6427 rows of 19248 padded) 7317 ->
-// 2574: LayerNorm + casts 74 -> 8.3 us (30 MB: 3.6 TB/s), GELU 40 -> 16 (79 MB: 4.9 TB/s).
+// text of 19 tokens 2019 -> 483 us (87 launches of 4-6 us), 48 texts of 23-401 tokens (6428 rows of 19248 padded) 7147 ->
+// 2278: LayerNorm + casts 74 -> 8.3 us (30 MB: 3.6 TB/s), GELU 40 -> 16 (79 MB: 4.9 TB/s).
 #include "mx_common.h"
 
 #include <type_traits>
 
 namespace {
 
-constexpr int EW = 4;   // rows (waves) per workgroup of the row kernels
-constexpr int GW = 8;   // waves per workgroup of the GEMM
+constexpr int EW = 4;  // rows (waves) per workgroup of the row kernels
+constexpr int GW = 8;  // waves per workgroup of the GEMM
+constexpr int ENC_ACT = 0, ENC_GELU = 1, ENC_PART = 2;  // what the GEMM writes
+__host__ constexpr int enc_parts(int K) { return K >= 2048 ? 4 : 1; }
 
 // LayerNorm of one row held by a wave: lane has the 8-element chunks lane + 64 j. Two passes over registers: the
 // variance is a sum of squares about the mean.
@@ -119,6 +121,22 @@ __global__ __launch_bounds__(64 * EW) void enc_add_ln_kernel(const uint16_t* __r
     ln_row<NC, F16>(v, H, g, b, eps, x + (size_t)row * H, lane);
 }
 
+// x = LN(sum of parts + bias + x); parts [NP][rows][H] fp32
+template <int NC, int NP, bool F16>
+__global__ __launch_bounds__(64 * EW) void enc_parts_ln_kernel(const float* __restrict__ parts,
+                                                               const uint16_t* __restrict__ bias, uint16_t* __restrict__ x, int rows,
+                                                               const float* __restrict__ g, const float* __restrict__ b, int H,
+                                                               float eps) {
+    const int row = blockIdx.x * EW + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (row >= rows) return;
+    float v[NC][8] = {};
+#pragma unroll
+    for (int p = 0; p < NP; ++p) add_f32<NC>(v, parts + ((size_t)p * rows + row) * H, H, lane);
+    if (bias) add_act<NC, F16>(v, bias, H, lane);
+    add_act<NC, F16>(v, x + (size_t)row * H, H, lane);
+    ln_row<NC, F16>(v, H, g, b, eps, x + (size_t)row * H, lane);
+}
+
 // y = gelu(y) in place, 8 elements a thread
 template <bool F16>
 __global__ __launch_bounds__(256) void enc_gelu_kernel(uint16_t* __restrict__ y, long n8) {
@@ -136,83 +154,100 @@ __global__ __launch_bounds__(256) void enc_gelu_kernel(uint16_t* __restrict__ y,
 }
 
 // One text per workgroup -> e [H] fp32. mode 0: mean over its klen rows, 1: first row, 2: last row; then / max(|e|, 1e-12).
-// A thread sums pairs of columns over every 4th row (a text of 400 rows x 768: 0.6 MB).
+// Groups of H / 8 threads (at most 512) take every n-th row, 16 bytes a thread; their sums meet in LDS (H <= 4096). A text of
+// 401 rows x 768 (0.6 MB): 56 us with 4-byte loads of four row groups, 9 with these.
 template <bool F16>
 __global__ __launch_bounds__(1024) void enc_pool_kernel(const uint16_t* __restrict__ x, const int* __restrict__ cu,
                                                         const int* __restrict__ klen, int H, int mode, int norm,
                                                         float* __restrict__ e) {
-    __shared__ float part[4][512];
+    __shared__ __attribute__((aligned(16))) float part[1024 * 8];
     __shared__ float red[16];
     const int b = blockIdx.x, r0 = cu[b], n = cu[b + 1] - r0, live = klen[b];
-    const int grp = threadIdx.x >> 8, t = threadIdx.x & 255;
     const int lo = mode == 2 ? n - 1 : 0, hi = mode == 0 ? live : lo + 1;
+    const int nc = H / 8, ng = 1024 / nc;  // (nc <= 512)
+    const int grp = threadIdx.x / nc, c = threadIdx.x - grp * nc;
+    float s[8] = {};
+    if (grp < ng) {
+        const uint16_t* xp = x + (size_t)r0 * H + 8 * c;
+        auto add = [&](const uint4& w) {
+            const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float a, d;
+                unpack_act2<F16>(ws[i], a, d);
+                s[2 * i] += a;
+                s[2 * i + 1] += d;
+            }
+        };
+        int r = lo + grp;
+        for (; r + 3 * ng < hi; r += 4 * ng) {
+            uint4 w[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) w[u] = *(const uint4*)(xp + (size_t)(r + u * ng) * H);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) add(w[u]);
+        }
+        for (; r < hi; r += ng) add(*(const uint4*)(xp + (size_t)r * H));
+        float* p = part + grp * H + 8 * c;
+        *(float4*)p = make_float4(s[0], s[1], s[2], s[3]);
+        *(float4*)(p + 4) = make_float4(s[4], s[5], s[6], s[7]);
+    }
+    __syncthreads();
     const float cnt = mode == 0 ? (float)max(live, 1) : 1.f;
     float sq = 0.f;
-    for (int c0 = 0; c0 < H; c0 += 512) {
-        const int c = c0 + 2 * t;
-        float s0 = 0.f, s1 = 0.f;
-        if (c < H)
-            for (int r = lo + grp; r < hi; r += 4) {
-                float a, d;
-                unpack_act2<F16>(*(const uint32_t*)(x + (size_t)(r0 + r) * H + c), a, d);
-                s0 += a;
-                s1 += d;
-            }
-        part[grp][2 * t] = s0;
-        part[grp][2 * t + 1] = s1;
-        __syncthreads();
-        if (threadIdx.x < 512 && c0 + (int)threadIdx.x < H) {
-            const float v = ((part[0][threadIdx.x] + part[1][threadIdx.x]) + (part[2][threadIdx.x] + part[3][threadIdx.x])) / cnt;
-            e[(size_t)b * H + c0 + threadIdx.x] = v;
-            sq += v * v;
-        }
-        __syncthreads();
+    for (int i = threadIdx.x; i < H; i += 1024) {
+        float v = 0.f;
+        for (int k = 0; k < ng; ++k) v += part[k * H + i];
+        v /= cnt;
+        part[i] = v;  // (group 0's sums: this thread alone reads them)
+        sq += v * v;
     }
-    if (!norm) return;
-    const float ws = wave_sum(sq);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ws;
+    sq = wave_sum(sq);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = sq;
     __syncthreads();
     float tot = 0.f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) tot += red[i];  // (waves 8 .. 15 hold no columns)
-    const float nr = fmaxf(sqrtf(tot), 1e-12f);
-    for (int c0 = 0; c0 < H; c0 += 512)
-        if (threadIdx.x < 512 && c0 + (int)threadIdx.x < H) e[(size_t)b * H + c0 + threadIdx.x] /= nr;
+    for (int i = 0; i < 16; ++i) tot += red[i];
+    const float nr = norm ? fmaxf(sqrtf(tot), 1e-12f) : 1.f;
+    for (int i = threadIdx.x; i < H; i += 1024) e[(size_t)b * H + i] = part[i] / nr;
 }
 
 template <bool F16>
-MX_DEV f32x4 enc_mfma(uint4 a, uint4 b, f32x4 c) {
+MX_DEV f32x4 enc_mfma(u32x4 a, u32x4 b, f32x4 c) {
     if constexpr (F16)
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
     else
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-// y[M, N] = act(x[M, K] W[N, K]^T + bias), 16-bit in and out, fp32 sums. A workgroup has 16 columns and 16 MT rows; its 8
-// waves take every 8th 32-wide k-step and their sums meet in LDS. What bounds it is the wait for the first loads: a wave
-// asks for U k-steps at once (all three of K = 768). Rows past M read row M - 1 and are not stored.
-template <int MT, bool F16, bool GELU>
-__global__ __launch_bounds__(64 * GW) void enc_gemm_kernel(const uint16_t* __restrict__ x, int ldx, const uint16_t* __restrict__ W,
-                                                           const uint16_t* __restrict__ bias, uint16_t* __restrict__ y, int ldy,
-                                                           int M, int N, int K) {
+// y[M, N] = act(x[M, K] W[N, K]^T + bias), 16-bit in and out, fp32 sums; or, ENC_PART, the fp32 sums of gridDim.z parts of K
+// one after another, which the LayerNorm that follows adds up. A workgroup has 16 columns and 16 MT rows; its 8 waves take
+// every 8th 32-wide k-step and their sums meet in LDS. What bounds it is the wait for the first loads: a wave asks for U
+// k-steps at once (all three of K = 768). 19 rows: K = 768 4.5 us whatever N up to 3072; K = 3072, N = 768 9.4 us with 48
+// workgroups (16 waves in each: the same), 4.5 in four parts. Rows past M read row M - 1 and are not stored.
+template <int MT, bool F16, int OUT>
+__global__ __launch_bounds__(64 * GW) void enc_gemm_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ W,
+                                                           const uint16_t* __restrict__ bias, void* __restrict__ y, int M, int N,
+                                                           int K) {
     __shared__ float red[GW * MT * 256];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
-    const int n0 = blockIdx.x * 16, m0 = blockIdx.y * (16 * MT), KS = K / 32;
+    const int n0 = blockIdx.x * 16, m0 = blockIdx.y * (16 * MT);
+    const int KS = K / 32 * (blockIdx.z + 1) / gridDim.z;
     const uint16_t* wp = W + (size_t)(n0 + col) * K + 8 * g;
     const uint16_t* xp[MT];
 #pragma unroll
-    for (int t = 0; t < MT; ++t) xp[t] = x + (size_t)min(m0 + 16 * t + col, M - 1) * ldx + 8 * g;
+    for (int t = 0; t < MT; ++t) xp[t] = x + (size_t)min(m0 + 16 * t + col, M - 1) * K + 8 * g;
     f32x4 acc[MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
     auto steps = [&](int s, auto uc) {
         constexpr int U = decltype(uc)::value;
-        uint4 wf[U], xf[U][MT];
+        u32x4 wf[U], xf[U][MT];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            wf[u] = *(const uint4*)(wp + 32 * (s + GW * u));
+            wf[u] = *(const u32x4*)(wp + 32 * (s + GW * u));
 #pragma unroll
-            for (int t = 0; t < MT; ++t) xf[u][t] = *(const uint4*)(xp[t] + 32 * (s + GW * u));
+            for (int t = 0; t < MT; ++t) xf[u][t] = *(const u32x4*)(xp[t] + 32 * (s + GW * u));
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -220,7 +255,7 @@ __global__ __launch_bounds__(64 * GW) void enc_gemm_kernel(const uint16_t* __res
             for (int t = 0; t < MT; ++t) acc[t] = enc_mfma<F16>(xf[u][t], wf[u], acc[t]);
     };
     constexpr int U = MT <= 2 ? 6 : 3;
-    int s = wave;
+    int s = K / 32 * blockIdx.z / gridDim.z + wave;
     for (; s + GW * (U - 1) < KS; s += GW * U) steps(s, std::integral_constant<int, U>{});
     if (U > 3 && s + GW * 2 < KS) {
         steps(s, std::integral_constant<int, 3>{});
@@ -238,22 +273,23 @@ __global__ __launch_bounds__(64 * GW) void enc_gemm_kernel(const uint16_t* __res
         float v = 0.f;
 #pragma unroll
         for (int w = 0; w < GW; ++w) v += red[w * MT * 256 + e];
-        if (bias) v += act_to_f32<F16>(bias[n0 + n]);
-        if constexpr (GELU) v = gelu_erf_f(v);
-        y[(size_t)m * ldy + n0 + n] = f32_to_act<F16>(v);
+        if constexpr (OUT == ENC_PART) {
+            ((float*)y)[((size_t)blockIdx.z * M + m) * N + n0 + n] = v;
+        } else {
+            if (bias) v += act_to_f32<F16>(bias[n0 + n]);
+            if constexpr (OUT == ENC_GELU) v = gelu_erf_f(v);
+            ((uint16_t*)y)[(size_t)m * N + n0 + n] = f32_to_act<F16>(v);
+        }
     }
 }
 
-template <bool F16>
-int enc_gemm(const uint16_t* x, int ldx, const uint16_t* W, const uint16_t* bias, uint16_t* y, int ldy, int M, int N, int K,
-             int gelu, hipStream_t st) {
+template <bool F16, int OUT>
+int enc_gemm(const uint16_t* x, const uint16_t* W, const uint16_t* bias, void* y, int M, int N, int K, hipStream_t st) {
     const int mt = min(4, (M + 15) / 16);
-#define EG(MT_)                                                                                                        \
-    if (mt == MT_) {                                                                                                   \
-        const dim3 grid(N / 16, (M + 16 * MT_ - 1) / (16 * MT_));                                                      \
-        if (gelu) enc_gemm_kernel<MT_, F16, true><<<grid, 64 * GW, 0, st>>>(x, ldx, W, bias, y, ldy, M, N, K);          \
-        else enc_gemm_kernel<MT_, F16, false><<<grid, 64 * GW, 0, st>>>(x, ldx, W, bias, y, ldy, M, N, K);              \
-    }
+#define EG(MT_)                                                                                                            \
+    if (mt == MT_)                                                                                                         \
+        enc_gemm_kernel<MT_, F16, OUT><<<dim3(N / 16, (M + 16 * MT_ - 1) / (16 * MT_), OUT == ENC_PART ? enc_parts(K) : 1),    \
+                                         64 * GW, 0, st>>>(x, W, bias, y, M, N, K);
     EG(1) EG(2) EG(3) EG(4)
 #undef EG
     return (int)hipGetLastError();
@@ -306,33 +342,39 @@ extern "C" int mxk_enc_gelu(uint16_t* y, long long n, hipStream_t st) {
 extern "C" int mxk_enc_pool(const uint16_t* x, const int* cu, const int* klen, int B, int H, int mode, int norm, float* e,
                             hipStream_t st) {
     if (B <= 0) return 0;
-    if (H <= 0 || H % 2 || mode < 0 || mode > 2) return (int)hipErrorInvalidValue;
+    if (!enc_width_ok(H) || mode < 0 || mode > 2) return (int)hipErrorInvalidValue;
     MX_ACT_DISPATCH(enc_pool_kernel<F16><<<B, 1024, 0, st>>>(x, cu, klen, H, mode, norm, e));
     MXK_CHECK_LAUNCH();
 }
 
 // w: 12 device pointers a layer: qkv W, b, output W, b, norm g, b (fp32), up W, b, down W, b, norm g, b (fp32); biases may be
-// null. x [rows][H] in and out; qkv [rows][3 H], attn and proj [rows][H], up [rows][F] are scratch.
+// null. x [rows][H] in and out; qkv [rows][3 H], attn [rows][H], up [rows][F] and parts [4][rows][H] fp32 are scratch.
 extern "C" int mxk_enc_layers(const void* const* w, int n_layers, uint16_t* x, int rows, int B, int Smax, const int* cu,
                               const int* klen, int H, int heads, int F, float scale, float eps, uint16_t* qkv, uint16_t* attn,
-                              uint16_t* proj, uint16_t* up, hipStream_t st) {
+                              float* parts, uint16_t* up, hipStream_t st) {
     if (rows <= 0 || n_layers <= 0) return 0;
     if (!enc_width_ok(H) || H % 32 || F % 32 || heads <= 0 || H % heads) return (int)hipErrorInvalidValue;
+    static_assert(enc_parts(32) == 1 && enc_parts(1 << 20) == 4, "parts");
     for (int l = 0; l < n_layers; ++l, w += 12) {
-        auto gemm = [&](const uint16_t* a, int i, uint16_t* y, int N, int K, int gelu) {
-            const uint16_t *W = (const uint16_t*)w[i], *b = (const uint16_t*)w[i + 1];
+        auto at = [&](int i) { return (const uint16_t*)w[i]; };
+        auto ln = [&](int K, int i, int j) {  // x = LN(parts of a product over K + bias i + x) with norm j
+            auto go = [&](auto kern) {
+                kern<<<(rows + EW - 1) / EW, 64 * EW, 0, st>>>(parts, at(i), x, rows, (const float*)w[j], (const float*)w[j + 1], H, eps);
+                return (int)hipGetLastError();
+            };
             int rc = 0;
-            MX_ACT_DISPATCH(rc = enc_gemm<F16>(a, K, W, b, y, N, rows, N, K, gelu, st));
+            MX_ACT_DISPATCH(ENC_NC(H, rc = enc_parts(K) == 1 ? go(enc_parts_ln_kernel<NC, 1, F16>) : go(enc_parts_ln_kernel<NC, 4, F16>)));
             return rc;
         };
-        int rc = gemm(x, 0, qkv, 3 * H, H, 0);
+        int rc = 0;
+        MX_ACT_DISPATCH((rc = enc_gemm<F16, ENC_ACT>(x, at(0), at(1), qkv, rows, 3 * H, H, st)));
         if (!rc) rc = mxk_attn_dense_ragged(qkv, 3 * H, qkv + H, 3 * H, qkv + 2 * H, 3 * H, attn, H, B, Smax, heads, H / heads, cu,
                                             klen, scale, st);
-        if (!rc) rc = gemm(attn, 2, proj, H, H, 0);
-        if (!rc) rc = enc_add_ln(proj, x, rows, (const float*)w[4], (const float*)w[5], H, eps, st);
-        if (!rc) rc = gemm(x, 6, up, F, H, 1);
-        if (!rc) rc = gemm(up, 8, proj, H, F, 0);
-        if (!rc) rc = enc_add_ln(proj, x, rows, (const float*)w[10], (const float*)w[11], H, eps, st);
+        if (!rc) MX_ACT_DISPATCH((rc = enc_gemm<F16, ENC_PART>(attn, at(2), nullptr, parts, rows, H, H, st)));
+        if (!rc) rc = ln(H, 3, 4);
+        if (!rc) MX_ACT_DISPATCH((rc = enc_gemm<F16, ENC_GELU>(x, at(6), at(7), up, rows, F, H, st)));
+        if (!rc) MX_ACT_DISPATCH((rc = enc_gemm<F16, ENC_PART>(up, at(8), nullptr, parts, rows, H, F, st)));
+        if (!rc) rc = ln(F, 9, 10);
         if (rc) return rc;
     }
     return 0;

@@ -26,8 +26,8 @@ from .. import _native as N
 from ..ops import core as K
 from ..ops.linear import ACT_DTYPE
 
-# packed rows up to which encoder.hip runs the layers in one call (BERT-base, whole embed calls: 64 rows 752 us against 1291 with
-# library GEMMs issued from Python, 320 rows 997 against 1314, 512 equal, 640 1415 against 1281)
+# packed rows up to which encoder.hip runs the layers in one call (BERT-base, whole embed calls: 64 rows 662 us against 1332 with
+# library GEMMs issued from Python, 320 rows 1016 against 1362, 512 equal, 640 1501 against 1380)
 ENC_SMALL_ROWS = 448
 
 
@@ -203,11 +203,11 @@ class BertModel:
                 N.ptr(ln_b), H, float(cfg.eps), x.data_ptr(), st)
         scale = 1.0 / math.sqrt(H // cfg.n_heads)
         if R <= ENC_SMALL_ROWS:
-            proj = torch.empty_like(attn)
+            parts = torch.empty(4, R, H, dtype=torch.float32, device=dev)  # fp32 sums of up to four parts of K
             qkv, up = (torch.empty(R, n, dtype=self.dtype, device=dev) for n in (3 * H, Fd))
             ptrs = (ctypes.c_void_p * (12 * cfg.n_layers))(*map(N.ptr, ts[5:]))
             N.kcall("mxk_enc_layers", ptrs, cfg.n_layers, x.data_ptr(), R, B, S, cu_d.data_ptr(), len_d.data_ptr(), H,
-                    cfg.n_heads, Fd, scale, float(cfg.eps), qkv.data_ptr(), attn.data_ptr(), proj.data_ptr(), up.data_ptr(), st)
+                    cfg.n_heads, Fd, scale, float(cfg.eps), qkv.data_ptr(), attn.data_ptr(), parts.data_ptr(), up.data_ptr(), st)
             return x, cu_d, len_d
 
         def linear(a, W, b):
