@@ -2,15 +2,20 @@
 // state_scan). Per sequence and head, over the step's rows in order:
 //     S <- a_t S;   u = c_t (v_t - S^T k_t)  [delta]   or   u = c_t v_t;   S <- S + k_t u^T;   o_t = S^T q_t (+ D v_t)
 // S has N numbers for each of the head's P value columns, fp32, stored column-major: state [slots, H, P, N]. The
-// columns never mix, so a column belongs to LPC neighbouring lanes (4, or the 16 of one DPP row) that each keep NPL
-// consecutive numbers of it in registers for the whole chunk: a step costs 4 NPL vector operations and two LPC-wide
-// sums done with DPP moves, and a lane's part of the state is one contiguous run in memory (a column's lanes read N
-// contiguous floats, a wave's columns are adjacent). k_t and q_t are the same for every column of a head: the block
-// stages them in LDS together with the tokens' decays, write strengths and values, 8 or 16 tokens at a time in two
-// buffers; the next tokens' numbers are requested from memory before the current ones are worked on and wait in
-// registers meanwhile, so memory latency and the barrier are paid once per 8 or 16 steps. The state is read from the
-// sequence's slot unless the chunk starts at position 0, and written back after the chunk's last row: a decode row is
-// a chunk of one, a prompt chunk walks its rows inside one launch.
+// columns never mix, so a column belongs to LPC neighbouring lanes (4, or the 16 of one DPP row) that each keep NPL of its
+// numbers (every LPC-th quadruple) in registers for the whole chunk. k_t and q_t are the same for every column of a head: the
+// block stages them in LDS together with the tokens' decays, write strengths and values, 8 or 16 tokens at a time in two
+// buffers; the next tokens' numbers are requested from memory before the current ones are worked on and wait in registers
+// meanwhile, so memory latency and the barrier are paid once per 8 or 16 steps. The state is read from the sequence's slot
+// unless the chunk starts at position 0, and written back after the chunk's last row: a decode row is a chunk of one, a
+// prompt chunk walks its rows inside one launch.
+// What bounds a prompt is the issue of a step's instructions by the few waves its columns make (1111 rows, 16 heads of 128 x
+// 128: 128 blocks; a step is 32 vector operations a lane and a chain of two sums): the read S^T k uses the undecayed state
+// (its decay is multiplied in after the sum), a step's LDS reads are asked for a step ahead, and output sums over a column's
+// lanes are made for 8 or 16 steps together, transposed on the way (3 operations a step instead of a chain of 4 and a store).
+// Prompts of 301 / 578 / 1111 rows: delta rule 576 -> 250 us, 64 heads of 64 x 128 without it 554 -> 227 (0.2 us a step;
+// most of the gain is that a round's loads no longer wait for each other). Steps of decode rows alone (ONE) stage one token and
+// sum at once: 33 rows 18.0 -> 12.6 and 30.3 -> 22.2 us (6.2 TB/s of states read and written).
 // CHD (gated linear attention): the decay is one number per head and state row, a_t[n], staged beside k_t and q_t:
 // S[n][p] <- a_t[n] S[n][p] + k_t[n] u[p]; with DELTA as well, the delta rule's read follows that per-row decay. A
 // missing write strength means 1, one given as pre-activations (coef_sigmoid, row stride ldc) passes a sigmoid when
@@ -26,6 +31,10 @@ template <int CTRL>
 MX_DEV float dpp_add(float v) {
     return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
 }
+template <int CTRL>
+MX_DEV float dpp_move(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
 // sum over the LPC (4 or 16) neighbouring lanes of a column, returned to each of them
 template <int LPC>
 MX_DEV float lanes_sum(float v) {
@@ -39,7 +48,7 @@ MX_DEV float lanes_sum(float v) {
 }
 
 // grid (column blocks, H, sequences); block = 256 threads = 256 / LPC columns
-template <int NPL, int LPC, bool DELTA, bool CHD>
+template <int NPL, int LPC, bool DELTA, bool CHD, bool ONE>
 __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk, const float* q, int ldq,
                                                          const float* v, int ldv, const float* decay, int ldd,
                                                          const float* coef, int ldc, int coef_sigmoid,
@@ -51,12 +60,12 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk
     constexpr int NT = 256;
     constexpr int NP = NPL * LPC;  // padded N
     constexpr int COLS = NT / LPC;
-    constexpr int TB = NP <= 128 ? 16 : 8;  // tokens staged together
+    constexpr int TB = ONE ? 1 : NP <= 128 ? 16 : 8;  // tokens staged together
     constexpr int NW = CHD ? 3 : 2;  // vectors of N numbers staged per token: k, q (, channel decays)
-    constexpr int KQ_PT = TB * NW * NP / NT, V_PT = (TB * COLS + NT - 1) / NT;
-    __shared__ float kq[2][TB][NW][NP];
+    constexpr int KQ_PT = (TB * NW * NP + NT - 1) / NT, V_PT = (TB * COLS + NT - 1) / NT;
+    __shared__ __attribute__((aligned(16))) float kq[2][TB][NW][NP];
     __shared__ float vs[2][TB][COLS];
-    __shared__ float ac[2][TB][2];
+    __shared__ __attribute__((aligned(8))) float ac[2][TB][2];
     const int cl = threadIdx.x / LPC;
     const int col = blockIdx.x * COLS + cl;
     const int part = threadIdx.x % LPC;
@@ -80,13 +89,14 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk
     // use is replaced by zero afterwards
     const int colc = min(col, PT - 1);
     float* sp = state + (((long)(slot < 0 ? 0 : slot) * H + h) * PT + colc) * N;
-    const bool whole = N == NP && (N & 3) == 0;  // no padding: a lane's run is NPL aligned floats
+    const bool whole = N == NP && (N & 3) == 0;  // no padding: a lane's numbers are NPL / 4 aligned quadruples
+    auto at = [&](int j) { return (j >> 2) * (4 * LPC) + part * 4 + (j & 3); };  // which number of the column S[j] is
     float S[NPL];
     if (whole) {
-        const float4* s4 = (const float4*)(sp + part * NPL);
+        const float4* s4 = (const float4*)sp + part;
 #pragma unroll
         for (int j = 0; j < NPL / 4; ++j) {
-            const float4 x = s4[j];
+            const float4 x = s4[j * LPC];
             S[4 * j] = x.x;
             S[4 * j + 1] = x.y;
             S[4 * j + 2] = x.z;
@@ -94,11 +104,11 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk
         }
     } else {
 #pragma unroll
-        for (int j = 0; j < NPL; ++j) S[j] = sp[min(part * NPL + j, N - 1)];
+        for (int j = 0; j < NPL; ++j) S[j] = sp[min(at(j), N - 1)];
     }
     const bool keep = !fresh && live;
 #pragma unroll
-    for (int j = 0; j < NPL; ++j) S[j] = (keep && part * NPL + j < N) ? S[j] : 0.f;
+    for (int j = 0; j < NPL; ++j) S[j] = (keep && at(j) < N) ? S[j] : 0.f;
     const float* kp = k + (long)g * N;
     const float* qp = q + (long)g * N;
     const float sk = skip ? skip[h] : 0.f;
@@ -106,29 +116,25 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk
     // TB tokens' k, q, value, decay and write strength wait in registers while the TB tokens before them are worked
     // on, then move to LDS: memory latency is paid once per TB steps, and a barrier too
     float st_kq[KQ_PT], st_v[V_PT], st_ac = 0.f;
-    // a round's loads are unconditional (clamped addresses, all in flight together) except that whole groups of NT
-    // loads beyond the round's tokens are skipped by a block-uniform test: a decode row asks for one token's numbers,
-    // not TB copies of them
+    // a round's loads are unconditional (one load from a selected, clamped address; scaled, masked and squashed when they
+    // move to LDS) so that all are in flight together; whole groups of NT loads beyond the round's tokens are skipped by a
+    // block-uniform test: a decode row asks for one token's numbers, not TB copies of them
     auto fetch = [&](int c) {
         const int r0 = row0 + c * TB;
         const int ntc = min(TB, n - c * TB);
 #pragma unroll
         for (int i = 0; i < KQ_PT; ++i) {
-            float x = 0.f;
-            const int idx = threadIdx.x + i * NT;
-            const int e = idx % NP;
+            const int idx = ONE ? min((int)threadIdx.x + i * NT, TB * NW * NP - 1) : threadIdx.x + i * NT;
             if (i * NT < ntc * NW * NP) {
                 const int tt = idx / (NW * NP), w = (idx / NP) % NW;
                 const long row = min(r0 + tt, last);
-                const int ec = min(e, N - 1);
-                if (CHD && w == 2) x = decay[row * ((long)H * N) + (long)h * N + ec];
-                else x = w ? qp[row * ldq + ec] * q_scale : kp[row * ldk + ec];
+                const float* src = CHD && w == 2 ? decay + (long)h * N : w ? qp : kp;
+                const long ld = CHD && w == 2 ? (long)H * N : w ? ldq : ldk;
+                st_kq[i] = src[row * ld + min(idx % NP, N - 1)];
             }
-            st_kq[i] = e < N ? x : 0.f;
         }
 #pragma unroll
         for (int i = 0; i < V_PT; ++i) {
-            st_v[i] = 0.f;
             if (i * NT < ntc * COLS) {
                 const int idx = min(threadIdx.x + i * NT, TB * COLS - 1);
                 const int tt = idx / COLS, cc = idx % COLS;
@@ -138,22 +144,33 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk
         }
         if (threadIdx.x < 2 * TB) {
             const long row = min(r0 + (int)threadIdx.x / 2, last);
-            if (threadIdx.x & 1) {
-                st_ac = coef ? coef[row * ldc + h] : 1.f;
-                if (coef && coef_sigmoid) st_ac = 1.f / (1.f + expf(-st_ac));
-            } else {
-                st_ac = CHD ? 1.f : decay[row * ldd + h];
-            }
+            const bool cf = threadIdx.x & 1;
+            // (what has no source reads the decay and is replaced)
+            const float* src = cf && coef ? coef + row * ldc + h : decay + (CHD ? row * ((long)H * N) + (long)h * N : row * ldd + h);
+            st_ac = *src;
         }
     };
     auto publish = [&](int b) {
 #pragma unroll
-        for (int i = 0; i < KQ_PT; ++i) (&kq[b][0][0][0])[threadIdx.x + i * NT] = st_kq[i];
+        for (int i = 0; i < KQ_PT; ++i) {
+            const int idx = threadIdx.x + i * NT;
+            if (ONE && idx >= TB * NW * NP) continue;
+            (&kq[b][0][0][0])[idx] = idx % NP < N ? ((idx / NP) % NW == 1 ? st_kq[i] * q_scale : st_kq[i]) : 0.f;
+        }
 #pragma unroll
         for (int i = 0; i < V_PT; ++i)
             if (threadIdx.x + i * NT < TB * COLS) (&vs[b][0][0])[threadIdx.x + i * NT] = st_v[i];
-        if (threadIdx.x < 2 * TB) (&ac[b][0][0])[threadIdx.x] = st_ac;
+        if (threadIdx.x < 2 * TB) {
+            float x = st_ac;
+            if (threadIdx.x & 1) x = !coef ? 1.f : coef_sigmoid ? 1.f / (1.f + expf(-x)) : x;
+            else if (CHD) x = 1.f;
+            (&ac[b][0][0])[threadIdx.x] = x;
+        }
     };
+#pragma unroll
+    for (int i = 0; i < KQ_PT; ++i) st_kq[i] = 0.f;  // (tokens past the end are staged as zeros and not worked on)
+#pragma unroll
+    for (int i = 0; i < V_PT; ++i) st_v[i] = 0.f;
     const int nchunks = (n + TB - 1) / TB;
     fetch(0);
     publish(0);
@@ -162,47 +179,90 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk
         const int b = c & 1;
         if (c + 1 < nchunks) fetch(c + 1);
         const int nt = min(TB, n - c * TB);
-        for (int tt = 0; tt < nt; ++tt) {
-            const int row = row0 + c * TB + tt;
-            const float a = ac[b][tt][0], cf = ac[b][tt][1];
-            const float vv = col < P ? vs[b][tt][cl] : live ? 1.f : 0.f;
-            const float* kb = &kq[b][tt][0][part * NPL];
-            const float* qb = &kq[b][tt][1][part * NPL];
+        // a step leaves the lane's share of its output (and of the skip term's value) here: they are summed over the
+        // column's lanes TB at a time
+        float os[TB];
+        // a step's numbers are read from LDS while the step before it is worked on
+        struct Tok {
+            float k[NPL], q[NPL], d[CHD ? NPL : 1], a, cf, v;
+        } tok[2];
+        auto read = [&](int tt, Tok& x) {
+            const float2 y = *(const float2*)ac[b][tt];
+            x.a = y.x;
+            x.cf = y.y;
+            x.v = vs[b][tt][cl];
+#pragma unroll
+            for (int j = 0; j < NPL; j += 4) {
+                *(float4*)(x.k + j) = *(const float4*)&kq[b][tt][0][j * LPC + part * 4];
+                *(float4*)(x.q + j) = *(const float4*)&kq[b][tt][1][j * LPC + part * 4];
+                if constexpr (CHD) *(float4*)(x.d + j) = *(const float4*)&kq[b][tt][NW - 1][j * LPC + part * 4];
+            }
+        };
+        read(0, tok[0]);
+#pragma unroll
+        for (int tt = 0; tt < TB; ++tt) {
+            os[tt] = 0.f;
+            if (tt + 1 < TB && tt + 1 < nt) read(tt + 1, tok[(tt + 1) & 1]);
+            __builtin_amdgcn_sched_barrier(0);
+            if (tt >= nt) continue;
+            const Tok& x = tok[tt & 1];
+            const float a = x.a, cf = x.cf, vv = col < P ? x.v : live ? 1.f : 0.f;
+            const float *kb = x.k, *qb = x.q, *ab = x.d;
             float u;
             if constexpr (DELTA) {
-                float d0 = 0.f, d1 = 0.f;  // two chains instead of one of NPL dependent adds
-                const float* ab = &kq[b][tt][NW - 1][part * NPL];  // (the channel decays; q's row when there are none)
+                if constexpr (CHD) {
 #pragma unroll
-                for (int j = 0; j < NPL; j += 2) {
-                    S[j] *= CHD ? ab[j] : a;
-                    S[j + 1] *= CHD ? ab[j + 1] : a;
-                    d0 += S[j] * kb[j];
-                    d1 += S[j + 1] * kb[j + 1];
+                    for (int j = 0; j < NPL; ++j) S[j] *= ab[j];
                 }
-                u = cf * (vv - lanes_sum<LPC>(d0 + d1));
-            } else if constexpr (CHD) {
-                const float* ab = &kq[b][tt][NW - 1][part * NPL];
+                float d[4] = {0.f, 0.f, 0.f, 0.f};  // four chains of dependent adds
 #pragma unroll
-                for (int j = 0; j < NPL; ++j) S[j] *= ab[j];
-                u = cf * vv;
+                for (int j = 0; j < NPL; ++j) d[j & 3] += S[j] * kb[j];
+                const float dk = lanes_sum<LPC>((d[0] + d[1]) + (d[2] + d[3]));
+                u = cf * (CHD ? vv - dk : vv - a * dk);  // (one decay for all rows: taken out of the sum)
             } else {
-#pragma unroll
-                for (int j = 0; j < NPL; ++j) S[j] *= a;
                 u = cf * vv;
             }
-            float o0 = 0.f, o1 = 0.f;
+            float o[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int j = 0; j < NPL; j += 2) {
+            for (int j = 0; j < NPL; ++j) {
+                if constexpr (!(DELTA && CHD)) S[j] *= CHD ? ab[CHD ? j : 0] : a;
                 S[j] += kb[j] * u;
-                S[j + 1] += kb[j + 1] * u;
-                o0 += S[j] * qb[j];
-                o1 += S[j + 1] * qb[j + 1];
+                o[j & 3] += S[j] * qb[j];
             }
-            const float o = lanes_sum<LPC>(o0 + o1);
-            if (part == 0) {
-                if (col < P) out[(long)row * ldo + (long)h * P + col] = o + sk * vv;
-                else if (live) nout[(long)row * H + h] = o;
+            os[tt] = (o[0] + o[1]) + (o[2] + o[3]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        auto put = [&](int tt, float o) {
+            if (tt >= nt || !live) return;
+            const long row = row0 + c * TB + tt;
+            if (col < P) out[row * ldo + (long)h * P + col] = o + sk * vs[b][tt][cl];
+            else nout[row * H + h] = o;
+        };
+        // sums over the lanes of a column, transposed on the way: lane `part` ends with steps part, part + LPC, ...
+        float o4[ONE ? 1 : TB / 4];
+#pragma unroll
+        for (int j = 0; j < TB / 4; ++j) {
+            const float a0 = part & 1 ? os[4 * j + 1] : os[4 * j], b0 = part & 1 ? os[4 * j] : os[4 * j + 1];
+            const float a1 = part & 1 ? os[4 * j + 3] : os[4 * j + 2], b1 = part & 1 ? os[4 * j + 2] : os[4 * j + 3];
+            const float e0 = a0 + dpp_move<0xB1>(b0), e1 = a1 + dpp_move<0xB1>(b1);  // quad_perm [1, 0, 3, 2]
+            const float f0 = part & 2 ? e1 : e0, f1 = part & 2 ? e0 : e1;
+            o4[j] = f0 + dpp_move<0x4E>(f1);                                          // quad_perm [2, 3, 0, 1]
+            if constexpr (LPC == 16) {
+                o4[j] = dpp_add<0x124>(o4[j]);  // row_ror 4
+                o4[j] = dpp_add<0x128>(o4[j]);  // row_ror 8
             }
+        }
+        if constexpr (ONE) {
+            const float o = lanes_sum<LPC>(os[0]);
+            if (part == 0) put(0, o);
+        } else if constexpr (LPC == 16) {
+            float o = o4[0];
+#pragma unroll
+            for (int j = 1; j < TB / 4; ++j) o = (part >> 2) == j ? o4[j] : o;
+            put(part, o);
+        } else {
+#pragma unroll
+            for (int j = 0; j < TB / 4; ++j) put(4 * j + part, o4[j]);
         }
         // the other buffer was last read while chunk c - 1 was worked on, before the barrier that ended that round
         if (c + 1 < nchunks) publish(b ^ 1);
@@ -210,13 +270,13 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk
     }
     if (slot >= 0 && live) {
         if (whole) {
-            float4* s4 = (float4*)(sp + part * NPL);
+            float4* s4 = (float4*)sp + part;
 #pragma unroll
-            for (int j = 0; j < NPL / 4; ++j) s4[j] = make_float4(S[4 * j], S[4 * j + 1], S[4 * j + 2], S[4 * j + 3]);
+            for (int j = 0; j < NPL / 4; ++j) s4[j * LPC] = make_float4(S[4 * j], S[4 * j + 1], S[4 * j + 2], S[4 * j + 3]);
         } else {
 #pragma unroll
             for (int j = 0; j < NPL; ++j)
-                if (part * NPL + j < N) sp[part * NPL + j] = S[j];
+                if (at(j) < N) sp[at(j)] = S[j];
         }
     }
 }
@@ -308,8 +368,13 @@ extern "C" int mxh_state_scan(const float* k, int ldk, const float* q, int ldq, 
     const int threads = 256;
     const int cols = threads / lpc;
     const dim3 grid((P + (nout ? 1 : 0) + cols - 1) / cols, H, n_seqs);
-#define GO2(NPL, LPC, D_, C_)                                                                                      \
-    state_scan_kernel<NPL, LPC, D_, C_><<<grid, threads, 0, st>>>(k, ldk, q, ldq, v, ldv, decay, ldd, coef, ldc,      \
+#define GO2(NPL, LPC, D_, C_)              \
+    do {                                   \
+        if (n_pf) GO3(NPL, LPC, D_, C_, false); \
+        else GO3(NPL, LPC, D_, C_, true);  \
+    } while (0)
+#define GO3(NPL, LPC, D_, C_, O_)                                                                                  \
+    state_scan_kernel<NPL, LPC, D_, C_, O_><<<grid, threads, 0, st>>>(k, ldk, q, ldq, v, ldv, decay, ldd, coef, ldc,      \
                                                                   coef_sigmoid, skip, state, seq_state, positions,    \
                                                                   n_dec, pf_cu, out, ldo, H, G, N, P, q_scale, nout)
 #define GO(NPL, LPC)                              \
@@ -326,6 +391,7 @@ extern "C" int mxh_state_scan(const float* k, int ldk, const float* q, int ldq, 
     else GO(16, 16);
 #undef GO
 #undef GO2
+#undef GO3
     return (int)hipGetLastError();
 }
 
