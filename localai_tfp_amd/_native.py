@@ -53,6 +53,7 @@ KERNEL_SIGS = {
     "mxk_set_act_f16": [I],
     "mxk_attn_dense": [P, I, P, I, P, I, P, I, I, I, I, I, I, I, P, P, I, F, I, P, I, P],
     "mxk_get_act_f16": [],
+    "mxk_lin16": [P, I, P, P, I, P, I, I, I, I, I, I, P],  # lin16.hip: x, ldx, W, y, ldy, part, parts, M, N, K, f16, acc
     # encoder.hip: packed text encoders
     "mxk_enc_embed": [P, I, P, P, P, P, P, I, F, P, P],
     "mxk_enc_add_ln": [P, P, I, P, P, I, F, P],

@@ -1,6 +1,6 @@
 """Dense 16-bit layers for the non-LLM model families (BERT, Whisper, CLIP/T5 text encoders, UNet /
-MMDiT, VAE, TTS): plain library GEMMs on hipBLASLt with the bias folded into the
-GEMM, fp32 accumulation into the residual stream, and the library's act16 activations.
+MMDiT, VAE, TTS): plain library GEMMs on hipBLASLt (few rows by matrices it is slow on: lin16.hip) with the bias folded into
+the GEMM, fp32 accumulation into the residual stream, and the library's act16 activations.
 
 On CPU everything runs in fp32 (the numerics oracle for the tests)."""
 from __future__ import annotations
@@ -20,6 +20,39 @@ def to_dev(a, device, dtype) -> torch.Tensor:
     if isinstance(a, torch.Tensor):
         return a.to(device=device, dtype=dtype).contiguous()
     return torch.from_numpy(np.ascontiguousarray(a, dtype=np.float32)).to(device).to(dtype).contiguous()
+
+
+def few_rows_parts(M: int, N: int, K: int) -> int:
+    """Parts of K that csrc/kernels/lin16.hip sums for M rows, or 0 where the library multiplies.
+
+    Measured with weights in no cache (bf16, us, here / library): long K and few columns, where the library's choice degrades
+    beyond K = 16384: 4096 x 16384 35-50 / 31-43, x 17408 34-52 / 47-129, x 24576 45-70 / 66-148, x 28672 51-79 / 57-166,
+    2048 x 20480 23-34 / 60-80 (1-64 rows); but 5120 x 20480 49-56 / 50-53 to 16 rows, 8192 x 20480 66-89 / 59-65 to 32. Many
+    columns and up to 8 rows: 28672 x 4096 52-56 / 66, 32000 56-58 / 61, 41024 69-74 / 74-77, 65536 x 2048 52-56 / 67; 16384 x
+    4096 31-32 / 33 and 12288 26 / 24 stay. Parts make one workgroup per compute unit (4096 columns: 1 / 2 / 4 / 8 parts 148 /
+    80 / 50 / 52 us)."""
+    if N % 64 or K % 32 or not 0 < M <= 64:
+        return 0
+    if K > 16384 and N <= 4096:
+        return min(8, 256 // (N // 64))
+    return 1 if N >= 24576 and M <= 8 else 0
+
+
+def _few_rows(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, acc: bool) -> bool:
+    """out (fp32) (+)= x w^T by lin16.hip where few_rows_parts takes it; False: nothing done."""
+    if not (x.is_cuda and x.dim() == 2 and x.dtype == w.dtype and x.dtype in (torch.float16, torch.bfloat16)):
+        return False
+    M, K = x.shape
+    N_ = w.shape[0]
+    parts = few_rows_parts(M, N_, K)
+    if not parts or x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16 or not w.is_contiguous() or w.data_ptr() % 16 \
+            or out.dtype != torch.float32 or out.shape != (M, N_) or out.stride(1) != 1 or out.stride(0) < N_:
+        return False
+    from .. import _native as N
+    part = torch.empty(parts, M, N_, dtype=torch.float32, device=x.device) if parts > 1 else None
+    N.kcall("mxk_lin16", x.data_ptr(), max(K, x.stride(0)), w.data_ptr(), out.data_ptr(), out.stride(0), N.ptr(part), parts, M, N_,
+            K, int(x.dtype == torch.float16), int(acc), N.stream_ptr())
+    return True
 
 
 class Dense:
@@ -71,6 +104,8 @@ class Dense:
             else:
                 torch.mm(x, self.wt, out=out)
             return out
+        if self.b32 is None and _few_rows(x, self.w, out, False):
+            return out
         if _fp32_out_ok(x.dtype):
             if self.b32 is not None:
                 out.copy_(self.b32.expand_as(out))
@@ -91,7 +126,8 @@ class Dense:
         if x.dtype != torch.float32 and _fp32_out_ok(x.dtype) and acc.is_contiguous():
             if self.b32 is not None:
                 acc.add_(self.b32)
-            torch.addmm(acc, x, self.wt, out_dtype=torch.float32, out=acc)
+            if not _few_rows(x, self.w, acc, True):
+                torch.addmm(acc, x, self.wt, out_dtype=torch.float32, out=acc)
             return acc
         acc.add_(self(x).float())
         return acc

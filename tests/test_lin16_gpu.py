@@ -1,0 +1,68 @@
+"""Products of a few 16-bit rows (csrc/kernels/lin16.hip) and the rule that chooses them (ops/dense.py)."""
+import pytest
+import torch
+
+from localai_tfp_amd.ops import dense as D
+
+
+def test_rule():
+    p = D.few_rows_parts
+    assert p(1, 4096, 17408) == p(64, 4096, 20480) == 4 and p(33, 2048, 20480) == 8 and p(8, 1024, 32768) == 8
+    assert p(65, 4096, 20480) == p(33, 4096, 16384) == p(16, 5120, 20480) == p(0, 4096, 20480) == 0
+    assert p(8, 28672, 4096) == 1 and p(9, 28672, 4096) == p(8, 16384, 4096) == 0
+    assert p(4, 4000, 20480) == p(4, 4096, 20488) == 0
+    assert all(0 <= p(m, n, k) <= 8 for m in (1, 64) for n in range(64, 4097, 64) for k in (16416, 40960))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,parts", [(1, 64, 32, 1), (15, 68, 96, 2), (16, 128, 256, 8), (17, 64, 2080, 3), (33, 192, 20480, 4),
+                                         (48, 4, 288, 1), (64, 100, 800, 5), (64, 64, 17408, 8)])
+@pytest.mark.parametrize("acc", [False, True])
+def test_few_rows_match_64_bits(dt, M, N, K, parts, acc):
+    """Ends of row tiles, column panels and k-steps, parts without a step of their own, rows of x and y with room between them.
+    Every product is exact in fp32 and a sum of K terms (and y) is off by at most (K + 1) x 2^-24 of the sum of magnitudes."""
+    from localai_tfp_amd import _native as Nv
+    g = torch.Generator().manual_seed(M + K)
+    x = torch.randn(M, K + 8, generator=g).to(dt).cuda()[:, :K]
+    w = torch.randn(N, K, generator=g).to(dt).cuda()
+    y = torch.randn(M, N + 3, generator=g).cuda()
+    xd, wd, yd = (t.double().cpu() for t in (x, w, y[:, :N]))
+    want = xd @ wd.t() + (yd if acc else 0)
+    mag = xd.abs() @ wd.abs().t() + yd.abs()
+    rest = y[:, N:].clone()
+    part = torch.full((parts, M, N), float("nan"), device="cuda")
+    Nv.kcall("mxk_lin16", x.data_ptr(), x.stride(0), w.data_ptr(), y.data_ptr(), y.stride(0), part.data_ptr(), parts, M, N, K,
+             int(dt == torch.float16), int(acc), Nv.stream_ptr())
+    assert ((y[:, :N].double().cpu() - want).abs() <= (K + 1) * 2 ** -24 * mag).all() and torch.equal(y[:, N:], rest)
+
+
+@pytest.mark.gpu
+def test_dense_routes_few_rows(monkeypatch):
+    """The layer's two entries on the routed shapes against the library's product: the same sums in another order."""
+    g = torch.Generator().manual_seed(0)
+    layer = D.Dense(torch.randn(256, 16416, generator=g) * 0.01, torch.randn(256, generator=g), "cuda", torch.bfloat16)
+    plain = D.Dense(layer.w, None, "cuda", torch.bfloat16)
+    x = torch.randn(33, 16416, generator=g).bfloat16().cuda()
+    start = torch.randn(33, 256, generator=g).cuda()
+    got = [layer.acc(x, start.clone()), plain.into(x, torch.empty(33, 256, device="cuda")), plain.acc(x, start.clone())]
+    monkeypatch.setattr(D, "few_rows_parts", lambda *a: 0)
+    want = [layer.acc(x, start.clone()), plain.into(x, torch.empty(33, 256, device="cuda")), plain.acc(x, start.clone())]
+    mag = 2 * 16417 * 2 ** -24 * (x.double().abs().cpu() @ layer.w.double().abs().t().cpu() + 8)
+    for a, b in zip(got, want):
+        assert ((a.double() - b.double()).abs().cpu() <= mag).all()
+    # a replayed graph allocates its parts once and sums them in the same order every time
+    monkeypatch.undo()
+    y = start.clone()
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        plain.acc(x, y)
+    torch.cuda.current_stream().wait_stream(s)
+    gr = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(gr):
+        plain.acc(x, y)
+    for _ in range(3):
+        y.copy_(start)
+        gr.replay()
+        assert torch.equal(y, got[2])
