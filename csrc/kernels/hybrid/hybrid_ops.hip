@@ -295,8 +295,10 @@ __global__ __launch_bounds__(64) void rope_norm_append_kernel(const float* qi, c
 }
 
 // grid (ceil(C / NT), sequences, ceil(T / CONV_ROWS)): thread = channel. Reads the tails only; conv_tails_kernel
-// rolls them afterwards
-constexpr int CONV_ROWS = 8;
+// rolls them afterwards. TAPS 2 .. 4: the last inputs slide through registers, one read a row (1990 rows of 4352 channels, 4
+// taps: 57 us with a read per tap and row, 19 with these); 0: any number up to 16.
+constexpr int CONV_ROWS = 16;
+template <int TAPS>
 __global__ __launch_bounds__(NT) void causal_conv_kernel(const float* x, int ldx, const float* w, const float* bias,
                                                          int taps, int silu, float* tails, const int* state,
                                                          const int* positions, int n_dec, const int* pf_cu, float* out,
@@ -315,27 +317,39 @@ __global__ __launch_bounds__(NT) void causal_conv_kernel(const float* x, int ldx
     const int t0 = blockIdx.z * CONV_ROWS;
     if (t0 >= n || c >= C) return;
     const int slot = state[s];
-    const int nt = taps - 1;
+    const int nt = (TAPS ? TAPS : taps) - 1;
     const bool fresh = positions[row0] == 0 || slot < 0;
-    float* tail = tails + ((long)(slot < 0 ? 0 : slot) * (nt > 0 ? nt : 1)) * C + c;  // entry i at tail[i * C]
-    float wr[16];
+    const float* tail = tails + ((long)(slot < 0 ? 0 : slot) * (nt > 0 ? nt : 1)) * C + c;  // entry i at tail[i * C]
+    constexpr int WT = TAPS ? TAPS : 16;
+    float wr[WT];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) wr[j] = j < taps ? w[(long)c * taps + j] : 0.f;
+    for (int j = 0; j < WT; ++j) wr[j] = TAPS || j < taps ? w[(long)c * (TAPS ? TAPS : taps) + j] : 0.f;
     const float b = bias ? bias[c] : 0.f;
     const int t1 = min(n, t0 + CONV_ROWS);
-    for (int t = t0; t < t1; ++t) {
-        float acc = b;
+    // input index within the chunk; < 0: carried from earlier steps
+    auto at = [&](int tau) { return tau >= 0 ? x[(long)(row0 + tau) * ldx + c] : fresh ? 0.f : tail[(long)(nt + tau) * C]; };
+    if constexpr (TAPS > 0) {
+        float v[CONV_ROWS + TAPS - 1];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            if (j < taps) {
-                const int tau = t - nt + j;  // input index within the chunk; < 0: carried from earlier steps
-                float v;
-                if (tau >= 0) v = x[(long)(row0 + tau) * ldx + c];
-                else v = fresh ? 0.f : tail[(long)(nt + tau) * C];
-                acc += wr[j] * v;
-            }
+        for (int i = 0; i < TAPS - 1; ++i) v[i] = at(t0 - nt + i);
+#pragma unroll
+        for (int i = 0; i < CONV_ROWS; ++i) v[TAPS - 1 + i] = x[(long)(row0 + min(t0 + i, n - 1)) * ldx + c];
+#pragma unroll
+        for (int i = 0; i < CONV_ROWS; ++i) {
+            if (t0 + i >= t1) break;
+            float acc = b;
+#pragma unroll
+            for (int j = 0; j < TAPS; ++j) acc += wr[j] * v[i + j];
+            out[(long)(row0 + t0 + i) * ldo + c] = silu ? silu_acc(acc) : acc;
         }
-        out[(long)(row0 + t) * ldo + c] = silu ? silu_acc(acc) : acc;
+    } else {
+        for (int t = t0; t < t1; ++t) {
+            float acc = b;
+#pragma unroll
+            for (int j = 0; j < 16; ++j)
+                if (j < taps) acc += wr[j] * at(t - nt + j);
+            out[(long)(row0 + t) * ldo + c] = silu ? silu_acc(acc) : acc;
+        }
     }
 }
 
@@ -512,39 +526,65 @@ __global__ void gated_group_norm_kernel(const float* y, int ldy, const float* ga
 MX_DEV float gelu_tanh_acc(float x) {
     return 0.5f * x * (1.f + tanhf(0.7978845608028654f * (x + 0.044715f * x * x * x)));
 }
-template <bool B16>
+MX_DEV float glu_one(float x, float y, float fac, int act, float limit, float alpha) {
+    if (act == 2) {
+        const float r = fmaxf(fac * x, 0.f);
+        return r * r;
+    }
+    if (act == 4) return 0.5f * x * (1.f + erff(x * 0.7071067811865476f)) * fac;
+    if (act == 3) {
+        const float g = fminf(x, limit), u = fminf(fmaxf(y, -limit), limit);
+        return g * sigmoid_acc(alpha * g) * (u + 1.f) * fac;
+    }
+    return (act == 1 ? gelu_tanh_acc(x) : silu_acc(x)) * y * fac;
+}
+// V elements a thread: 4 where every row, factor group and operand allows 16-byte reads, else 1. Bound by its bytes: 1990 rows of
+// 14336 (285 MB) took 113 us with one element a thread, 84 with four.
+template <bool B16, int V>
 __global__ __launch_bounds__(NT) void glu_kernel(const float* a, int lda, const float* b, int ldb, const float* ba,
                                                  const float* bb, const float* scale, int lds, int group,
                                                  int scale_sigmoid, void* out, int ldo, int F, int act, float limit,
                                                  float alpha) {
-    const int f = blockIdx.y * NT + threadIdx.x, t = blockIdx.x;
+    const int f = (blockIdx.y * NT + threadIdx.x) * V, t = blockIdx.x;
     if (f >= F) return;
-    float fac = 1.f;
+    auto put = [&](const float* v) {
+        if constexpr (V == 4 && B16)
+            *(uint2*)((bf16_t*)out + (long)t * ldo + f) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+        else if constexpr (V == 4)
+            *(float4*)((float*)out + (long)t * ldo + f) = make_float4(v[0], v[1], v[2], v[3]);
+        else
+            st_elem<B16>(out, (long)t * ldo + f, v[0]);
+    };
+    float fac = 1.f, x[V], y[V], r[V];
     if (scale) {
         fac = scale[(long)t * lds + f / group];
         if (scale_sigmoid) fac = sigmoid_acc(fac);
         if (fac == 0.f) {  // an expert the router did not choose: nothing to evaluate
-            st_elem<B16>(out, (long)t * ldo + f, 0.f);
+#pragma unroll
+            for (int e = 0; e < V; ++e) r[e] = 0.f;
+            put(r);
             return;
         }
     }
-    const float x = a[(long)t * lda + f] + (ba ? ba[f] : 0.f);
-    if (act == 2) {
-        const float r = fmaxf(fac * x, 0.f);
-        st_elem<B16>(out, (long)t * ldo + f, r * r);
-        return;
-    }
-    if (act == 4) {
-        st_elem<B16>(out, (long)t * ldo + f, 0.5f * x * (1.f + erff(x * 0.7071067811865476f)) * fac);
-        return;
-    }
-    const float y = b[(long)t * ldb + f] + (bb ? bb[f] : 0.f);
-    if (act == 3) {
-        const float g = fminf(x, limit), u = fminf(fmaxf(y, -limit), limit);
-        st_elem<B16>(out, (long)t * ldo + f, g * sigmoid_acc(alpha * g) * (u + 1.f) * fac);
-        return;
-    }
-    st_elem<B16>(out, (long)t * ldo + f, (act == 1 ? gelu_tanh_acc(x) : silu_acc(x)) * y * fac);
+    auto get = [&](const float* p, float* v) {
+        if constexpr (V == 4) {
+            const float4 w = *(const float4*)p;
+            v[0] = w.x;
+            v[1] = w.y;
+            v[2] = w.z;
+            v[3] = w.w;
+        } else {
+            v[0] = *p;
+        }
+    };
+    get(a + (long)t * lda + f, x);
+#pragma unroll
+    for (int e = 0; e < V; ++e) y[e] = 0.f;
+    if (b) get(b + (long)t * ldb + f, y);
+#pragma unroll
+    for (int e = 0; e < V; ++e)
+        r[e] = glu_one(x[e] + (ba ? ba[f + e] : 0.f), y[e] + (bb ? bb[f + e] : 0.f), fac, act, limit, alpha);
+    put(r);
 }
 
 // one wave per token; lane l holds experts l, l + 64, ... (up to 16 each)
@@ -724,8 +764,14 @@ extern "C" int mxh_causal_conv(const float* x, int ldx, const float* w, const fl
     MXH_CHECK(ldx >= C && ldo >= C && n_dec >= 0 && n_pf >= 0 && n_dec + n_pf > 0 && (n_pf == 0 || pf_cu));
     const int rows = n_pf ? T - n_dec : 1;
     const dim3 grid((C + NT - 1) / NT, n_dec + n_pf, (max(rows, 1) + CONV_ROWS - 1) / CONV_ROWS);
-    causal_conv_kernel<<<grid, NT, 0, st>>>(x, ldx, w, bias, taps, silu, tails, state, positions, n_dec, pf_cu, out,
-                                            ldo, C);
+#define GO(T_)                                                                                                          \
+    causal_conv_kernel<T_><<<grid, NT, 0, st>>>(x, ldx, w, bias, taps, silu, tails, state, positions, n_dec, pf_cu, out, \
+                                                ldo, C)
+    if (taps == 2) GO(2);
+    else if (taps == 3) GO(3);
+    else if (taps == 4) GO(4);
+    else GO(0);
+#undef GO
     if (taps > 1) {
         const dim3 g2((C + NT - 1) / NT, n_dec + n_pf);
         conv_tails_kernel<<<g2, NT, 0, st>>>(x, ldx, taps, tails, state, positions, n_dec, pf_cu, C);
@@ -793,13 +839,16 @@ extern "C" int mxh_glu(const float* a, int lda, const float* b, int ldb, const f
     MXH_CHECK(a && out && lda >= F && ldo >= F && group > 0 && F <= 65535 * NT && act >= 0 && act <= 4);
     MXH_CHECK(act == 2 || act == 4 ? !b : (b && ldb >= F));  // the squared ReLU and the plain gelu have one operand
     MXH_CHECK(!scale || (F % group == 0 && lds >= F / group));
-    const dim3 grid(T, (F + NT - 1) / NT);
-    if (o16)
-        glu_kernel<true><<<grid, NT, 0, st>>>(a, lda, b, ldb, ba, bb, scale, lds, group, scale_sigmoid, out, ldo, F, act,
-                                          limit, alpha);
-    else
-        glu_kernel<false><<<grid, NT, 0, st>>>(a, lda, b, ldb, ba, bb, scale, lds, group, scale_sigmoid, out, ldo, F, act,
-                                          limit, alpha);
+    const bool four = F % 4 == 0 && group % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0 && ldo % 4 == 0 &&
+                      ((uintptr_t)a | (uintptr_t)b | (uintptr_t)out) % 16 == 0;
+#define GO(B, V)                                                                                                      \
+    glu_kernel<B, V><<<dim3(T, (F + NT * V - 1) / (NT * V)), NT, 0, st>>>(a, lda, b, ldb, ba, bb, scale, lds, group, \
+                                                                         scale_sigmoid, out, ldo, F, act, limit, alpha)
+    if (o16 && four) GO(true, 4);
+    else if (o16) GO(true, 1);
+    else if (four) GO(false, 4);
+    else GO(false, 1);
+#undef GO
     return (int)hipGetLastError();
 }
 

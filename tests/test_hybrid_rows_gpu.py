@@ -1,0 +1,95 @@
+"""Kernels of the hybrid decoders (csrc/kernels/hybrid: the recurrence, gated units, convolutions) on the GPU against the same
+steps on the CPU."""
+import types
+
+import pytest
+import torch
+
+from localai_tfp_amd.ops import hybrid as HY
+
+pytestmark = pytest.mark.gpu
+
+
+def _rag(n_dec, chunks, at, slots, dev):
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    cu = [0]
+    for c in chunks:
+        cu.append(cu[-1] + c)
+    pos = [p for p, c in zip(at, [1] * n_dec + chunks) for p in range(p, p + c)]
+    return HY.Ragged(types.SimpleNamespace(
+        T=len(pos), n_decode=n_dec, positions=i32(pos), seq_state=i32(slots), slots=i32([-1] * len(pos)), pf_cu_q=i32(cu),
+        pf_q_lens_host=chunks, pf_ctx_lens_host=[p + c for p, c in zip(at[n_dec:], chunks)], pf_block_tables=None, pf_ctx_lens=None,
+        dec_block_tables=None, dec_seq_lens=None, dec_max_len=0))
+
+
+@pytest.mark.parametrize("N,P", [(16, 64), (32, 5), (33, 16), (64, 17), (128, 16), (100, 33), (256, 20)])
+@pytest.mark.parametrize("delta,channel,nout", [(True, False, False), (False, False, True), (False, True, False), (True, True, False)])
+def test_rounds_of_tokens(N, P, delta, channel, nout):
+    """Chunks that end just before, at and after a round of 8 or 16 tokens, beside decode rows, with and without padding of N.
+    Both sides sum in fp32, in another order: a share of 2^-24 per step and term of sums whose terms shrink with the decay, some
+    40 steps of up to 256 terms, stays below 2e-5 of the largest output."""
+    g = torch.Generator().manual_seed(N)
+    H, G, chunks = 2, 1, [1, 7, 8, 9, 15, 16, 17, 33, 48]
+    n_dec, T = 2, 2 + sum(chunks)
+    k = torch.randn(T, G * N, generator=g) * N ** -0.5
+    q, v = torch.randn(T, G * N, generator=g), torch.randn(T, H * P, generator=g)
+    decay = torch.rand(T, H * N if channel else H, generator=g)
+    coef = torch.rand(T, H, generator=g)
+    skip = None if delta or nout else torch.randn(H, generator=g)  # (no caller has a skip term beside a normaliser)
+    slots = list(range(n_dec + len(chunks)))
+    at = [3, 0] + [0, 5] * 5
+    start = torch.randn(len(slots), H, P + nout, N, generator=g)
+    got = {}
+    for dev in ("cpu", "cuda"):
+        state, out = start.clone().to(dev), torch.zeros(T, H * P, device=dev)
+        no = torch.zeros(T, H, device=dev) if nout else None
+        HY.state_scan(k.to(dev), q.to(dev), v.to(dev), decay.to(dev), coef.to(dev), None if skip is None else skip.to(dev), state,
+                      _rag(n_dec, chunks, at[:len(slots)], slots, dev), out, H, G, N, P, delta, channel, 0.5, False, no)
+        got[dev] = [t.cpu() for t in (out, state, no) if t is not None]
+    for a, b in zip(got["cuda"], got["cpu"]):
+        assert (a - b).abs().max() <= 2e-5 * b.abs().max()
+
+
+@pytest.mark.parametrize("F,group,off", [(4, 4, 0), (260, 4, 0), (2048, 256, 0), (1023, 1023, 0), (1024, 2, 0), (1024, 1024, 1)])
+@pytest.mark.parametrize("act", ["silu", "gelu_tanh", "relu2", "clamped", "gelu"])
+def test_glu_widths(F, group, off, act):
+    """Four elements a thread and one (odd widths, factor groups and offsets), fp32 and 16-bit out, with biases and factors of
+    zero. A handful of fp32 operations and one function of a few units in the last place, whose arguments are sums of numbers up
+    to ~10: 2e-5 of a result (or of 1); two such numbers may round to neighbouring bf16 numbers, 2^-7 of them apart."""
+    g = torch.Generator().manual_seed(F)
+    T = 5
+    y = torch.randn(T, 2 * F + 16, generator=g) * 2
+    ba, bb = torch.randn(F, generator=g), torch.randn(F, generator=g)
+    scale = torch.rand(T, F // group, generator=g)
+    scale[1] = 0.0
+    two = act not in ("relu2", "gelu")
+    res = {}
+    for dev in ("cpu", "cuda"):
+        z = y.to(dev)
+        b = z[:, F + 8 + off:2 * F + 8 + off] if two else None
+        for dt in (torch.float32, torch.bfloat16):
+            out = torch.full((T, F + 8), 7.0, dtype=dt, device=dev)
+            HY.glu(z[:, off:off + F], b, ba.to(dev), bb.to(dev) if two else None, out[:, off:off + F], scale=scale.to(dev),
+                   group=group, act=act, **({"limit": 1.5, "alpha": 1.7} if act == "clamped" else {}))
+            res[dev, dt] = out.float().cpu()
+    a, b = res["cuda", torch.float32], res["cpu", torch.float32]
+    assert ((a - b).abs() <= 2e-5 * (1 + b.abs())).all()
+    a, b = res["cuda", torch.bfloat16], res["cpu", torch.bfloat16]
+    assert ((a - b).abs() <= 2 ** -7 * b.abs() + 2e-5 * (1 + b.abs())).all()
+
+
+@pytest.mark.parametrize("taps", [1, 2, 3, 4, 5])
+def test_conv_blocks_of_rows(taps):
+    """Chunks that end around a block of 16 rows, fresh and carried, beside decode rows: sums of up to five products in fp32."""
+    g = torch.Generator().manual_seed(taps)
+    C, chunks, n_dec = 70, [1, 2, 15, 16, 17, 33], 2
+    T, slots = n_dec + sum(chunks), list(range(n_dec + len(chunks)))
+    x, w, bias = torch.randn(T, C + 3, generator=g), torch.randn(C, taps, generator=g), torch.randn(C, generator=g)
+    at = [4, 0, 0, 7, 0, 9, 0, 3]
+    start = torch.randn(len(slots), max(1, taps - 1), C, generator=g)
+    res = []
+    for dev in ("cpu", "cuda"):
+        tails, out = start.clone().to(dev), torch.zeros(T, C, device=dev)
+        HY.causal_conv(x.to(dev)[:, 3:], w.to(dev), bias.to(dev), tails, _rag(n_dec, chunks, at, slots, dev), out, silu=True)
+        res.append((out.cpu(), tails.cpu()))
+    assert (res[0][0] - res[1][0]).abs().max() < 1e-5 and torch.equal(res[0][1], res[1][1])
