@@ -194,16 +194,18 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const bf16_t* __restri
 
 constexpr int DEC_RED_MAXP = 512;  // partitions whose merge weights fit the reduce kernel's LDS table
 
+// One (sequence, query head) per workgroup. Wave 0 reads the partitions' (m, l) with all its lanes at once and publishes the
+// merge weights through LDS; then groups of D / 4 threads take every n-th partition, four dims a thread and four partitions in
+// flight, and their sums meet in LDS. A chain of memory latencies bounds it: 9 contexts of 3001-24001 in 256-key partitions 9.9 us
+// with one group of D threads, 5.7 with eight of 32.
 template <bool F16>
-__global__ __launch_bounds__(128) void attn_decode_reduce_kernel(const float2* __restrict__ part_ml,
+__global__ __launch_bounds__(256) void attn_decode_reduce_kernel(const float2* __restrict__ part_ml,
                                                                   const float* __restrict__ part_o, int n_parts,
                                                                   int Hq, int D, const int* __restrict__ seq_lens,
                                                                   int part_size, bf16_t* __restrict__ out,
                                                                   int out_stride) {
-    // wave 0 reads the partitions' (m, l) with all its lanes at once and publishes the merge weights through
-    // LDS (a serial loop of dependent loads made this launch as long as the attention itself at batch 1);
-    // every thread then sums its dims over the partitions with independent loads
     __shared__ float wts[DEC_RED_MAXP];
+    __shared__ __attribute__((aligned(16))) float sums[1024];  // [groups][D]
     __shared__ float s_mx, s_ls;
     const int bh = blockIdx.x;
     const int b = bh / Hq, h = bh % Hq;
@@ -226,19 +228,30 @@ __global__ __launch_bounds__(128) void attn_decode_reduce_kernel(const float2* _
     }
     __syncthreads();
     const float mx = s_mx, L = s_ls;
-    for (int d = threadIdx.x; d < D; d += blockDim.x) {
-        float os = 0.f;
-        int p = 0;
-        for (; p + 4 <= min(np, DEC_RED_MAXP); p += 4) {
-            const float o0 = part_o[(pb + p) * D + d], o1 = part_o[(pb + p + 1) * D + d];
-            const float o2 = part_o[(pb + p + 2) * D + d], o3 = part_o[(pb + p + 3) * D + d];
-            os += o0 * wts[p] + o1 * wts[p + 1] + o2 * wts[p + 2] + o3 * wts[p + 3];
-        }
-        for (; p < np; ++p) {
-            const float a = p < DEC_RED_MAXP ? wts[p] : (mx == -INFINITY ? 0.f : exp2f(part_ml[pb + p].x - mx));
-            os += part_o[(pb + p) * D + d] * a;
-        }
-        out[(size_t)b * out_stride + (size_t)h * D + d] = f32_to_act<F16>(L > 0.f ? os / L : 0.f);
+    const int nq = D / 4, groups = 256 / nq, grp = threadIdx.x / nq, d = threadIdx.x % nq * 4;  // (D 64, 128 or 256)
+    float4 os = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto add = [&](const float4& o, float a) {
+        os.x += o.x * a;
+        os.y += o.y * a;
+        os.z += o.z * a;
+        os.w += o.w * a;
+    };
+    auto at = [&](int p) { return *(const float4*)(part_o + (pb + p) * D + d); };
+    int p = grp;
+    for (; p + 3 * groups < min(np, DEC_RED_MAXP); p += 4 * groups) {
+        const float4 o0 = at(p), o1 = at(p + groups), o2 = at(p + 2 * groups), o3 = at(p + 3 * groups);
+        add(o0, wts[p]);
+        add(o1, wts[p + groups]);
+        add(o2, wts[p + 2 * groups]);
+        add(o3, wts[p + 3 * groups]);
+    }
+    for (; p < np; p += groups) add(at(p), p < DEC_RED_MAXP ? wts[p] : (mx == -INFINITY ? 0.f : exp2f(part_ml[pb + p].x - mx)));
+    *(float4*)(sums + grp * D + d) = os;
+    __syncthreads();
+    for (int e = threadIdx.x; e < D; e += 256) {
+        float v = 0.f;
+        for (int k = 0; k < groups; ++k) v += sums[k * D + e];
+        out[(size_t)b * out_stride + (size_t)h * D + e] = f32_to_act<F16>(L > 0.f ? v / L : 0.f);
     }
 }
 
@@ -258,7 +271,7 @@ static int launch_decode(const bf16_t* q, int q_stride, const void* kc, const vo
                                                                        Hkv, bs, scale, window, softcap, part_size,
                                                                        n_parts, out, out_stride, part_ml, part_o);
         if (n_parts > 1)
-            attn_decode_reduce_kernel<F16><<<B * Hkv * G, 128, 0, st>>>(part_ml, part_o, n_parts, Hkv * G, D, seq_lens,
+            attn_decode_reduce_kernel<F16><<<B * Hkv * G, 256, 0, st>>>(part_ml, part_o, n_parts, Hkv * G, D, seq_lens,
                                                                         part_size, out, out_stride);
     });
 #undef DQK
@@ -438,15 +451,15 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
     const int p0 = part * part_size;
     const int* bt = block_tables + (size_t)b * bt_stride;
     const int blk0 = p0 / bs;
-    // the partition's block-table entries are requested before (not after) the sequence length: the
-    // table read does not wait for seq_lens, entries past the context are loaded but never used
-    {
-        const int nbt = min(part_size / bs + 1, bt_stride - blk0);
-        for (int i = threadIdx.x; i < nbt; i += 64 * NW) sbt[i] = bt[blk0 + i];
-    }
+    // the partition's block-table entries (at most 256: one a thread) are requested before the sequence length and wait in a
+    // register: a partition past the context ends as soon as the length is here
+    static_assert(64 * NW >= MAXB, "one entry a thread");
+    const int nbt = min(part_size / bs + 1, bt_stride - blk0);
+    const int bt_entry = (int)threadIdx.x < nbt ? bt[blk0 + threadIdx.x] : 0;
     const int L = seq_lens[b];
     const int p1 = min(L, p0 + part_size);
     if (p0 >= L && part > 0) return;  // uniform: graphs launch n_parts for max_model_len
+    if ((int)threadIdx.x < nbt) sbt[threadIdx.x] = bt_entry;
     DEC_TS(1)
     const int Hq = Hkv * G;
     const int p_start = window > 0 ? max(p0, L - window) : p0;
@@ -809,7 +822,7 @@ static int launch_decode_mfma(const bf16_t* q, int q_stride, const void* kc, con
                                                                           part_size, n_parts, out, out_stride, part_ml,
                                                                           part_o, part_cnt);
         if (n_parts > 1 && !part_cnt)
-            attn_decode_reduce_kernel<F16><<<B * Hkv * G, 128, 0, st>>>(part_ml, part_o, n_parts, Hkv * G, D, seq_lens,
+            attn_decode_reduce_kernel<F16><<<B * Hkv * G, 256, 0, st>>>(part_ml, part_o, n_parts, Hkv * G, D, seq_lens,
                                                                         part_size, out, out_stride);
     });
     MXK_CHECK_LAUNCH();
