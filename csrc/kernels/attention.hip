@@ -329,9 +329,9 @@ MX_DEV int v_lds_off(int p, int nt) {
 //   waves' (m, l, O) merge through LDS at the end, in the same partial-result format as attn_decode_kernel
 //   (attn_decode_reduce merges partitions).
 // Against the form with heads as rows (4 rows a lane, two 16-lane shuffle reductions per row and tile, P through LDS) and
-// caches widened load by load: bf16 B=128 ctx 65-1021 50.0 -> 45.2 us (4.0 TB/s), B=32 ctx 97-4003 44.5 -> 41.3; q8_0
-// B=9 ctx 3001-24001 155 -> 76 us at 256-key partitions (62 at 1024: 3.3 TB/s), fp8 147 -> 72 (55), q4_0 151 -> 75 (65:
-// 1.7 TB/s, bound by the widening's vector work).
+// caches widened load by load: bf16 B=128 ctx 65-1021 53.1 -> 49.2 us at 512-key partitions (44.9 at 1024: 4.1 TB/s), B=9 ctx
+// 3001-24001 95 -> 85; q8_0 B=9 155 -> 64 us (3.2 TB/s), fp8 147 -> 59, q4_0 151 -> 60 (1.8 TB/s, bound by the widening's
+// vector work). Three waves per SIMD instead of two gave the quantised caches 73 -> 64 of that.
 // Occupancy, not register double buffering, hides HBM latency: 8 KB of LDS per wave lets 4
 // workgroups (16 waves) share a CU, each with one tile's 16 KB of K/V loads in flight.
 template <int D>
@@ -422,9 +422,14 @@ struct DecRaw {
                      KVQ_ && Q::HB ? (vh[KVQ_ && Q::HB ? j >> 2 : 0] >> (8 * (j & 3))) & 0xFF : 0u);
     }
 };
+// waves per SIMD: what the registers of each cache format allow without spilling
+template <int KVF, int NW, bool TS, bool DPF>
+constexpr int dec_waves() {
+    return KVF == KVF_IQ4_NL || (KVF == KVF_BF16 && DPF && !TS && NW <= 8) ? 2 : KVF != KVF_BF16 ? 3 : 4;
+}
 template <int D, bool F16, int KVF, int NW = 4, bool TS = false, bool DPF = false>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
-    (KVF != KVF_BF16 || (DPF && !TS && NW <= 8)) ? 2 : 4, (KVF != KVF_BF16 || (DPF && !TS && NW <= 8)) ? 2 : 4))) void attn_decode_mfma_kernel(
+    dec_waves<KVF, NW, TS, DPF>(), dec_waves<KVF, NW, TS, DPF>()))) void attn_decode_mfma_kernel(
     const bf16_t* __restrict__ q, int q_stride, const void* __restrict__ kcv, const void* __restrict__ vcv,
     const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ seq_lens, int Hkv, int G, int bs,
     float scale, int window, float softcap, int part_size, int n_parts, bf16_t* __restrict__ out, int out_stride,
