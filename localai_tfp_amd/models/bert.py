@@ -139,8 +139,8 @@ class BertModel:
 
     # ---- packed rows (GPU) ----
     def _packed_weights(self, ids):
-        """The layers' tensors in the order encoder.hip takes them, or None where the batch runs padded: encoder.hip wants
-        16-bit weights, head dims 64 / 128 and widths in whole 16-byte pieces."""
+        """(tensors, addresses) in the order encoder.hip takes them, or None where the batch runs padded: encoder.hip wants
+        16-bit weights on the GPU, head dims 64 / 128, widths in whole 16-byte pieces and 16-byte aligned rows."""
         cfg, w = self.cfg, self.w
         H = cfg.hidden
         if self.device.type != "cuda" or not any(map(len, ids)) or H % 32 or H > 4096 or cfg.ffn % 32 or H % cfg.n_heads \
@@ -151,22 +151,24 @@ class BertModel:
             if t is None:
                 if need:
                     return None
-            elif t.shape != shape or t.dtype != dtype or not t.is_contiguous():
+            elif t.shape != shape or t.dtype != dtype or not t.is_contiguous() or not t.is_cuda:
                 return None
         for t, need in zip(ts, (1, 1, 0, 1, 0)):
             if t is None:
                 if need:
                     return None
-            elif t.shape[-1] != H or t.dtype != torch.float32 or not t.is_contiguous():
+            elif t.shape[-1] != H or t.dtype != torch.float32 or not t.is_contiguous() or not t.is_cuda:
                 return None
-        return ts
+        ptrs = [None if t is None else t.data_ptr() for t in ts]
+        return None if any(p is not None and p & 15 for p in ptrs) else (ts, ptrs)
 
     def _encode_packed(self, ts, ids, types=None):
         """-> (16-bit rows [R, H] of the texts one after another, first rows [B + 1], lengths [B], both int32 on the device).
         An empty text keeps one row that sees no key, as a padded batch has it."""
-        cfg, dev, w = self.cfg, self.device, self.w
+        cfg, dev = self.cfg, self.device
         B, H, Fd = len(ids), cfg.hidden, cfg.ffn
-        tokens, positions, kinds, ln_g, ln_b = ts[:5]
+        ts, ptrs = ts
+        tokens, positions, kinds = ts[:3]
         lens = np.fromiter((len(x) for x in ids), np.int64, B)
         rows = np.maximum(lens, 1)
         cu = np.zeros(B + 1, np.int64)
@@ -199,14 +201,12 @@ class BertModel:
         attn = torch.empty(R, H, dtype=self.dtype, device=dev)
         N.ensure_act(self.dtype)
         st = N.stream_ptr()
-        N.kcall("mxk_enc_embed", img.data_ptr(), R, tokens.data_ptr(), positions.data_ptr(), N.ptr(kinds), ln_g.data_ptr(),
-                N.ptr(ln_b), H, float(cfg.eps), x.data_ptr(), st)
+        N.kcall("mxk_enc_embed", img.data_ptr(), R, *ptrs[:5], H, float(cfg.eps), x.data_ptr(), st)
         scale = 1.0 / math.sqrt(H // cfg.n_heads)
         if R <= ENC_SMALL_ROWS:
             parts = torch.empty(4, R, H, dtype=torch.float32, device=dev)  # fp32 sums of up to four parts of K
             qkv, up = (torch.empty(R, n, dtype=self.dtype, device=dev) for n in (3 * H, Fd))
-            ptrs = (ctypes.c_void_p * (12 * cfg.n_layers))(*map(N.ptr, ts[5:]))
-            N.kcall("mxk_enc_layers", ptrs, cfg.n_layers, x.data_ptr(), R, B, S, cu_d.data_ptr(), len_d.data_ptr(), H,
+            N.kcall("mxk_enc_layers", (ctypes.c_void_p * (12 * cfg.n_layers))(*ptrs[5:]), cfg.n_layers, x.data_ptr(), R, B, S, cu_d.data_ptr(), len_d.data_ptr(), H,
                     cfg.n_heads, Fd, scale, float(cfg.eps), qkv.data_ptr(), attn.data_ptr(), parts.data_ptr(), up.data_ptr(), st)
             return x, cu_d, len_d
 
