@@ -39,19 +39,25 @@ def few_rows_parts(M: int, N: int, K: int) -> int:
 
 
 def _few_rows(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, acc: bool) -> bool:
-    """out (fp32) (+)= x w^T by lin16.hip where few_rows_parts takes it; False: nothing done."""
+    """out (fp32) (+)= x w^T by lin16.hip where few_rows_parts takes it; False: nothing done, the library's product answers (or
+    refuses) as for any other shape: operands of other devices or widths, rows of x that overlap (a row stride below K, as
+    expanded rows and sliding windows have), and graphs that would need a gradient are its business."""
     if not (x.is_cuda and x.dim() == 2 and x.dtype == w.dtype and x.dtype in (torch.float16, torch.bfloat16)):
         return False
     M, K = x.shape
     N_ = w.shape[0]
     parts = few_rows_parts(M, N_, K)
-    if not parts or x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16 or not w.is_contiguous() or w.data_ptr() % 16 \
+    if not parts or w.device != x.device or out.device != x.device or x.device.index != torch.cuda.current_device() \
+            or tuple(w.shape) != (N_, K) or (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or out.requires_grad)):
+        return False
+    ldx = x.stride(0) if M > 1 else K
+    if x.stride(1) != 1 or ldx < K or ldx % 8 or x.data_ptr() % 16 or not w.is_contiguous() or w.data_ptr() % 16 \
             or out.dtype != torch.float32 or out.shape != (M, N_) or out.stride(1) != 1 or out.stride(0) < N_:
         return False
     from .. import _native as N
     part = torch.empty(parts, M, N_, dtype=torch.float32, device=x.device) if parts > 1 else None
-    N.kcall("mxk_lin16", x.data_ptr(), max(K, x.stride(0)), w.data_ptr(), out.data_ptr(), out.stride(0), N.ptr(part), parts, M, N_,
-            K, int(x.dtype == torch.float16), int(acc), N.stream_ptr())
+    N.kcall("mxk_lin16", x.data_ptr(), ldx, w.data_ptr(), out.data_ptr(), out.stride(0), N.ptr(part), parts, M, N_, K,
+            int(x.dtype == torch.float16), int(acc), N.stream_ptr())
     return True
 
 
@@ -97,7 +103,8 @@ class Dense:
 
     def into(self, x: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
         """out (fp32, contiguous, preallocated) = x W^T + b: 16-bit operands with the fp32 accumulator written as is,
-        fp32 operands in plain fp32. No allocation, so a captured graph sees static addresses."""
+        fp32 operands in plain fp32. `out` is written in place; under capture the parts of a few rows' product (_few_rows)
+        come from the graph's own pool, so a captured graph sees static addresses."""
         if x.dtype == torch.float32:
             if self.b32 is not None:
                 torch.addmm(self.b32, x, self.wt, out=out)

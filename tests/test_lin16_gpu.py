@@ -1,4 +1,6 @@
 """Products of a few 16-bit rows (csrc/kernels/lin16.hip) and the rule that chooses them (ops/dense.py)."""
+import types
+
 import pytest
 import torch
 
@@ -12,6 +14,57 @@ def test_rule():
     assert p(8, 28672, 4096) == 1 and p(9, 28672, 4096) == p(8, 16384, 4096) == 0
     assert p(4, 4000, 20480) == p(4, 4096, 20488) == 0
     assert all(0 <= p(m, n, k) <= 8 for m in (1, 64) for n in range(64, 4097, 64) for k in (16416, 40960))
+
+
+def test_route_takes_only_what_the_kernel_reads(monkeypatch):
+    """What lin16.hip would read past, or from another device, stays with the library's product. On descriptions of tensors: no
+    call may reach a kernel."""
+    from localai_tfp_amd import _native as Nv
+    calls = []
+    monkeypatch.setattr(Nv, "kcall", lambda name, *a: calls.append((name, a)))
+    monkeypatch.setattr(Nv, "stream_ptr", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+
+    def t(shape, strides=None, dev="cuda:0", dtype=torch.bfloat16, ptr=4096, grad=False):
+        strides = strides or (shape[1], 1)
+        return types.SimpleNamespace(shape=torch.Size(shape), dtype=dtype, device=torch.device(dev), is_cuda=dev != "cpu",
+                                     requires_grad=grad, dim=lambda: len(shape), stride=lambda i: strides[i],
+                                     data_ptr=lambda: ptr, is_contiguous=lambda: strides == (shape[1], 1))
+
+    def route(x=None, w=None, out=None):
+        calls.clear()
+        took = D._few_rows(x or t((8, K)), w or t((N, K)), out or t((8, N), dtype=torch.float32), False)
+        assert took == (len(calls) == 1)
+        return took
+    N, K = 24576, 4096
+    assert route() and calls[0][1][1] == K
+    assert route(x=t((8, K), (K + 16, 1))) and calls[0][1][1] == K + 16
+    assert route(x=t((1, K), (0, 1)), out=t((1, N), dtype=torch.float32)) and calls[0][1][1] == K  # one row: no stride to follow
+    for s in (0, 8, K - 8, K + 4):  # expanded rows, windows, rows of which every other is not 16-byte aligned
+        assert not route(x=t((8, K), (s, 1)))
+    assert not route(w=t((N, K), dev="cpu")) and not route(out=t((8, N), dtype=torch.float32, dev="cpu"))
+    assert not route(w=t((N, K), dev="cuda:1")) and not route(w=t((N, K - 32))) and not route(w=t((N, K + 32)))
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    assert not route()
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    assert not route(x=t((8, K), grad=True)) and not route(out=t((8, N), dtype=torch.float32, grad=True))
+    with torch.no_grad():
+        assert route(x=t((8, K), grad=True))
+
+
+@pytest.mark.gpu
+def test_rows_that_overlap_match_the_library():
+    g = torch.Generator().manual_seed(3)
+    layer = D.Dense(torch.randn(64, 16416, generator=g) * 0.01, None, "cuda", torch.bfloat16)
+    row = torch.randn(16416 + 7 * 8, generator=g).bfloat16().cuda()
+    for x in (row[:16416].expand(8, 16416), row.unfold(0, 16416, 8)):
+        want = x.double() @ layer.w.double().t()
+        got = layer.into(x, torch.empty(8, 64, device="cuda"))
+        mag = 16417 * 2 ** -24 * (x.double().abs() @ layer.w.double().abs().t())  # products exact, a sum of K terms in fp32
+        assert ((got.double() - want).abs() <= mag).all()
+        assert ((layer.acc(x, torch.zeros(8, 64, device="cuda")).double() - want).abs() <= mag).all()
+    with pytest.raises(RuntimeError):
+        D.Dense(layer.w.cpu(), None, "cpu", torch.bfloat16).into(row[:16416].expand(8, 16416), torch.empty(8, 64, device="cuda"))
 
 
 @pytest.mark.gpu
