@@ -21,6 +21,10 @@
 
 #define LOG2E 1.4426950408889634f
 
+// Pages a decode partition lists in LDS. A partition that starts inside a page touches part_size / bs + 2 of them at most: 257
+// where the launchers' limit of part_size / bs + 1 <= 256 is met.
+constexpr int DEC_MAXB = 257;
+
 // ------------------------------------------------------------------------------------------------
 template <int D, int G, bool F16, bool KV8>
 __global__ __launch_bounds__(256) void attn_decode_kernel(const bf16_t* __restrict__ q, int q_stride,
@@ -75,8 +79,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const bf16_t* __restri
     // K/V fetch), and K/V are double-buffered in registers: the loads of step i+1 are in flight
     // while step i is scored, so each lane keeps 2*U 16-byte loads outstanding (memory-level
     // parallelism is what bounds this kernel, not VALU).
-    constexpr int MAXB = 256;  // part_size / bs + 1 <= MAXB (host checks)
-    __shared__ int sbt[MAXB];
+    __shared__ int sbt[DEC_MAXB];
     const int* bt = block_tables + (size_t)b * bt_stride;
     using kvec = typename KVVec<KV8>::T;
     constexpr int ES = KV8 ? 1 : 2;  // bytes per cached element
@@ -448,29 +451,29 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
     constexpr bool KV8 = KVF != KVF_BF16;       // a cache widened in registers (fp8 or block-quantised)
     constexpr int ES = KV8 ? 1 : 2;
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    constexpr int MAXB = 256;
-    __shared__ int sbt[MAXB];
+    __shared__ int sbt[DEC_MAXB];
     const int kvh = blockIdx.x, b = blockIdx.y, part = blockIdx.z;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int g = lane >> 4, col = lane & 15;
     const int p0 = part * part_size;
     const int* bt = block_tables + (size_t)b * bt_stride;
     const int blk0 = p0 / bs;
-    // the partition's block-table entries (at most 256: one a thread) are requested before the sequence length and wait in a
-    // register: a partition past the context ends as soon as the length is here
-    static_assert(64 * NW >= MAXB, "one entry a thread");
-    const int nbt = min(part_size / bs + 1, bt_stride - blk0);
+    // the partition's block-table entries (its last page's is (p0 + part_size - 1) / bs: a partition may start inside a page) are
+    // requested before the sequence length and wait in a register: a partition past the context ends as soon as the length is here
+    static_assert(64 * NW >= DEC_MAXB - 1, "one entry a thread, the last one apart");
+    const int nbt = min((p0 + part_size - 1) / bs - blk0 + 1, bt_stride - blk0);
     const int bt_entry = (int)threadIdx.x < nbt ? bt[blk0 + threadIdx.x] : 0;
     const int L = seq_lens[b];
     const int p1 = min(L, p0 + part_size);
     if (p0 >= L && part > 0) return;  // uniform: graphs launch n_parts for max_model_len
     if ((int)threadIdx.x < nbt) sbt[threadIdx.x] = bt_entry;
+    if (64 * NW < DEC_MAXB && nbt == DEC_MAXB && threadIdx.x == 0) sbt[DEC_MAXB - 1] = bt[blk0 + DEC_MAXB - 1];
     DEC_TS(1)
     const int Hq = Hkv * G;
     const int p_start = window > 0 ? max(p0, L - window) : p0;
     const float qs = scale * LOG2E;
     const float sc_l2 = softcap * LOG2E, sc_inv = softcap > 0.f ? 1.f / (softcap * LOG2E) : 0.f;
-    // Q as the A operand: row = head (lane col), k = dims 32 ks + 8 g — requested before the block-table
+    // Q^T as the B operand: column = head (lane col), k = dims 32 ks + 8 g — requested before the block-table
     // barrier so its latency overlaps the table read
     bf16x8 qf[D / 32];
 #pragma unroll

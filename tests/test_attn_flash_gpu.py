@@ -122,3 +122,23 @@ def test_decode_rows(fmt, Hq, Hkv, D):
         got = out.cpu().float()
         # as for prompts: probabilities and outputs are rounded to 16 bits once each
         assert float((got - want[rows]).norm() / want[rows].norm()) < 4 * 2 ** -9, part
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bs,part", [(24, 256), (48, 512), (20, 512), (640, 512), (3, 767)])
+@pytest.mark.parametrize("fmt,impl", [("bf16", "mfma"), ("q8_0", "mfma"), ("fp8", "mfma"), ("bf16", "valu"), ("fp8", "valu")])
+def test_decode_partitions_that_start_inside_a_page(bs, part, fmt, impl):
+    """Pages that do not divide a partition: its keys reach into one page more than its length in pages says (24-key pages, 256
+    keys from key 256 on: pages 10 .. 21). The last of (3, 767) is the 257th, the most that is listed."""
+    pre = [0, part - 1, part, part + 1, 2 * part - 2, 2 * part - 1, 2 * part, 3 * part - 1, 3 * part + 7]
+    q, kc, vc, bt, _, ctx = _case(8, 2, 128, [1] * len(pre), pre, bs=bs, fmt=fmt)
+    want = torch.stack([K._attn_ref_one(q[i:i + 1], kc, vc, bt[i], int(c), int(c) - 1, 128 ** -0.5, bs)[0] for i, c in enumerate(ctx)])
+    kd, vd = kc.cuda(), vc.cuda()
+    if hasattr(kc, "kvf"):
+        kd.kvf, vd.kvf = kc.kvf, vc.kvf
+    for rows in (slice(None), slice(4, 9)):  # (few bf16 rows take more waves a workgroup)
+        out = torch.full((len(ctx[rows]), 8, 128), float("nan"), dtype=torch.float16, device="cuda")
+        K.attn_decode(q[rows].cuda(), kd, vd, bt[rows].contiguous().cuda(), ctx[rows].cuda(), 128 ** -0.5, out, part_size=part, impl=impl)
+        got = out.cpu().float()
+        # as for prompts: probabilities and outputs are rounded to 16 bits once each
+        assert float((got - want[rows]).norm() / want[rows].norm()) < 4 * 2 ** -9
