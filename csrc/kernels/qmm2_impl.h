@@ -42,18 +42,27 @@ namespace {
 
 // 16 agent-coherent (sc1) loads in flight at once and one wait: the relaxed __hip_atomic_load form waits for each
 // load before issuing the next (measured: +10-40 us per GEMM for a 32 x 128 block per wave). Rows past M load row
-// M - 1 (the caller ignores them).
+// M - 1 (the caller ignores them). Loads and wait are ONE asm block with early-clobber outputs: between blocks of their own the
+// compiler would take the registers as written and could move them, or reuse them while the load is still to land.
 MX_DEV void q2_ld16_sc1(float (&v)[16], const float* base, size_t ld, int m0, int M) {
+    const float* p[16];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const float* p = base + (size_t)min(m0 + 8 * (r >> 2) + (r & 3), M - 1) * ld;
-        asm volatile("global_load_dword %0, %1, off sc1" : "=v"(v[r]) : "v"(p) : "memory");
-    }
-    asm volatile("s_waitcnt vmcnt(0)"
-                 : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]),
-                   "+v"(v[8]), "+v"(v[9]), "+v"(v[10]), "+v"(v[11]), "+v"(v[12]), "+v"(v[13]), "+v"(v[14]), "+v"(v[15])
-                 :
-                 : "memory");
+    for (int r = 0; r < 16; ++r) p[r] = base + (size_t)min(m0 + 8 * (r >> 2) + (r & 3), M - 1) * ld;
+    asm volatile(
+        "global_load_dword %0, %16, off sc1\n\tglobal_load_dword %1, %17, off sc1\n\t"
+        "global_load_dword %2, %18, off sc1\n\tglobal_load_dword %3, %19, off sc1\n\t"
+        "global_load_dword %4, %20, off sc1\n\tglobal_load_dword %5, %21, off sc1\n\t"
+        "global_load_dword %6, %22, off sc1\n\tglobal_load_dword %7, %23, off sc1\n\t"
+        "global_load_dword %8, %24, off sc1\n\tglobal_load_dword %9, %25, off sc1\n\t"
+        "global_load_dword %10, %26, off sc1\n\tglobal_load_dword %11, %27, off sc1\n\t"
+        "global_load_dword %12, %28, off sc1\n\tglobal_load_dword %13, %29, off sc1\n\t"
+        "global_load_dword %14, %30, off sc1\n\tglobal_load_dword %15, %31, off sc1\n\t"
+        "s_waitcnt vmcnt(0)"
+        : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7]),
+          "=&v"(v[8]), "=&v"(v[9]), "=&v"(v[10]), "=&v"(v[11]), "=&v"(v[12]), "=&v"(v[13]), "=&v"(v[14]), "=&v"(v[15])
+        : "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]), "v"(p[4]), "v"(p[5]), "v"(p[6]), "v"(p[7]), "v"(p[8]), "v"(p[9]),
+          "v"(p[10]), "v"(p[11]), "v"(p[12]), "v"(p[13]), "v"(p[14]), "v"(p[15])
+        : "memory");
 }
 
 // NS: ring slots (k-tiles of 64): 4, or 8 for the 64-row tiles ("deep ring", ks | 8 in mxk_qmm2) — a 64-row
