@@ -26,9 +26,21 @@ from .. import _native as N
 from ..ops import core as K
 from ..ops.linear import ACT_DTYPE
 
-# packed rows up to which encoder.hip runs the layers in one call (BERT-base, whole embed calls: 64 rows 662 us against 1332 with
-# library GEMMs issued from Python, 320 rows 1016 against 1362, 512 equal, 640 1501 against 1380)
+# packed rows up to which encoder.hip runs the layers in one call; above, the library multiplies
 ENC_SMALL_ROWS = 448
+
+
+def small_rows(hidden: int, ffn: int) -> int:
+    """Packed rows up to which the layers run in one call (encoder.hip's own GEMMs read a layer's weights once per 64 rows, so
+    rows x weights decide; beyond 64 M weights a layer the library's tiles win at any row count).
+
+    Whole embed calls, us, one call / library GEMMs issued from Python (110 us a layer at least): 384 x 1536, 12 layers, 448 rows
+    679 / 1433; 768 x 3072, 12 layers, 64 rows 657 / 1374, 384 1161 / 1363, 512 1275 / 1356, 640 1488 / 1354; 1024 x 4096, 24
+    layers, 64 rows 1428 / 2631, 256 2263 / 2605, 320 2857 / 2624; 1280 x 5120, 8 layers, 128 rows 828 / 910, 192 940 / 906; 1536 x
+    6144, 8 layers, 96 rows 813 / 958, 128 994 / 952; 2048 x 8192, 8 layers, 48 rows 899 / 963, 128 1388 / 947; 3072 x 12288, 4
+    layers, 16 rows 596 / 534, 256 2320 / 883."""
+    weights = 4 * hidden * hidden + 2 * hidden * ffn
+    return min(ENC_SMALL_ROWS, 3_200_000_000 // weights) if weights <= 64_000_000 else 0
 
 
 @dataclass
@@ -203,7 +215,7 @@ class BertModel:
         st = N.stream_ptr()
         N.kcall("mxk_enc_embed", img.data_ptr(), R, *ptrs[:5], H, float(cfg.eps), x.data_ptr(), st)
         scale = 1.0 / math.sqrt(H // cfg.n_heads)
-        if R <= ENC_SMALL_ROWS:
+        if R <= small_rows(H, Fd):
             parts = torch.empty(4, R, H, dtype=torch.float32, device=dev)  # fp32 sums of up to four parts of K
             qkv, up = (torch.empty(R, n, dtype=self.dtype, device=dev) for n in (3 * H, Fd))
             N.kcall("mxk_enc_layers", (ctypes.c_void_p * (12 * cfg.n_layers))(*ptrs[5:]), cfg.n_layers, x.data_ptr(), R, B, S, cu_d.data_ptr(), len_d.data_ptr(), H,

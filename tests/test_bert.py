@@ -99,6 +99,15 @@ def test_http_embeddings_and_rerank(client):
     assert sc == sorted(sc, reverse=True) and j["usage"]["total_tokens"] > 0
 
 
+def test_one_call_layers_are_chosen_by_rows_and_width():
+    """A one-call layer reads its weights once per 64 rows: wide encoders leave it at fewer rows (measured: small_rows)."""
+    rows = BM.small_rows
+    assert rows(384, 1536) == rows(768, 3072) == BM.ENC_SMALL_ROWS
+    assert 192 <= rows(1024, 4096) < 320 and rows(1024, 4096) < rows(1024, 2816) < 384
+    assert 64 <= rows(1280, 5120) < 192 and 64 <= rows(1536, 6144) < 128 and 48 <= rows(2048, 8192) < 96
+    assert rows(3072, 12288) == rows(4096, 16384) == 0
+
+
 @pytest.mark.gpu
 def test_bert_gpu_matches_fp32():
     """GPU path (hipBLASLt GEMMs + attention_dense.hip + norm.hip LayerNorm) vs the fp32 encoder."""
