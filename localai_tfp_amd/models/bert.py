@@ -174,9 +174,10 @@ class BertModel:
         ptrs = [None if t is None else t.data_ptr() for t in ts]
         return None if any(p is not None and p & 15 for p in ptrs) else (ts, ptrs)
 
-    def _encode_packed(self, ts, ids, types=None):
+    def _encode_packed(self, ts, ids, types=None, last=False):
         """-> (16-bit rows [R, H] of the texts one after another, first rows [B + 1], lengths [B], both int32 on the device).
-        An empty text keeps one row that sees no key, as a padded batch has it."""
+        An empty text keeps one row that sees no key, as a padded batch has it: its first one or (last) the batch's last position,
+        which is what the row before the first is there."""
         cfg, dev = self.cfg, self.device
         B, H, Fd = len(ids), cfg.hidden, cfg.ffn
         ts, ptrs = ts
@@ -189,6 +190,8 @@ class BertModel:
         img = np.zeros(3 * R + 2 * B + 1, np.int32)
         tok, pos, typ = img[:R], img[R:2 * R], img[2 * R:3 * R]
         pos[:] = np.arange(R) - np.repeat(cu[:-1], rows)
+        if last:
+            pos[cu[:-1][lens == 0]] = S - 1
 
         def pack(dst, lists, limit, what):
             for i, n in enumerate(lens.tolist()):
@@ -290,8 +293,8 @@ class BertModel:
     def embed(self, ids: list[list[int]], normalize: bool = True) -> torch.Tensor:
         ts = self._packed_weights(ids)
         if ts is not None:
-            x, cu, lens = self._encode_packed(ts, ids)
             mode = {"cls": 1, "rank": 1, "last": 2}.get(self.cfg.pooling, 0)
+            x, cu, lens = self._encode_packed(ts, ids, last=mode == 2)
             e = torch.empty(len(ids), self.cfg.hidden, dtype=torch.float32, device=x.device)
             N.kcall("mxk_enc_pool", x.data_ptr(), cu.data_ptr(), lens.data_ptr(), len(ids), self.cfg.hidden, mode,
                     int(normalize), e.data_ptr(), N.stream_ptr())

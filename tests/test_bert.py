@@ -158,3 +158,15 @@ def test_packed_rows_match_fp32(hidden, heads, ffn, pooling, monkeypatch):
     w = g.w["blk.0.ffn_up.bias"]
     g.w["blk.0.ffn_up.bias"] = torch.cat([w[:1], w])[1:]
     assert g._packed_weights([[1]]) is None and (g.embed([[5, 6]]).cpu() - c.embed([[5, 6]])).abs().max() < 5e-3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pooling", ["mean", "cls", "last"])
+def test_empty_texts_match_the_padded_batch(pooling):
+    """An empty text has a row too: nothing for the mean, its first row, or the batch's last position."""
+    cfg = BM.BertConfig(vocab=400, hidden=128, n_layers=2, n_heads=2, ffn=256, max_pos=64, pooling=pooling, name="t")
+    get = BM.synthetic_bert(cfg, 5)
+    g, c = BM.BertModel.load(cfg, get, "cuda:0"), BM.BertModel.load(cfg, get, "cpu")
+    ids = [[5, 6, 7, 8, 9], [], [11, 12], []]
+    assert g._packed_weights(ids) is not None
+    assert (g.embed(ids).cpu() - c.embed(ids)).abs().max() < 5e-3  # (the bound of test_packed_rows_match_fp32)
