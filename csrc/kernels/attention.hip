@@ -871,7 +871,8 @@ extern "C" int mxk_attn_decode_mfma(const bf16_t* q, int q_stride, const void* k
     return (int)hipErrorInvalidValue;
 }
 
-// What attention_flash.hip does not take: head dim 256, and the V^T image (VT = 1, `vmode`) of any head dim.
+// What attention_flash.hip does not take (ops/core.py flash_plan): head dim 256, with V as rows or (VT = 1, `vmode`) transposed in
+// LDS, and short contexts of head dims 64 / 128 where its wider workgroups lose.
 template <int D, int GW, int VT, bool F16, int KVF>
 __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restrict__ q,
                                                            const void* __restrict__ kc,
@@ -1142,7 +1143,7 @@ static int launch_prefill(const bf16_t* q, const void* kc, const void* vc, const
     }
     if constexpr (D == 256) {
         if (vmode == 0) PFK(0) else PFK(1)
-    } else PFK(1)  // (the row image of V at these head dims: attention_flash.hip)
+    } else PFK(0)
 #undef PFK
 #undef PFL
     MXK_CHECK_LAUNCH();

@@ -441,27 +441,38 @@ FLASH_SPLIT_KEYS = 2048  # contexts from which a grid that leaves compute units 
 
 
 def flash_plan(T: int, n_seqs: int, Hq: int, Hkv: int, D: int, block_size: int, table_width: int, window: int,
-               ctx_lens_host=None):
+               ctx_lens_host=None, softcap: float = 0.0, tiles: bool = False):
     """(waves per workgroup, key parts) of attention_flash.hip for T prompt rows, or None where the other prompt kernel
-    runs (head dim 256, and what neither takes). A workgroup holds 32 * waves / G queries of one KV head.
+    runs (head dim 256, short contexts, and what neither takes). A workgroup holds 32 * waves / G queries of one KV head.
+    ctx_lens_host: the contexts, or a bound on them, where the caller knows them.
 
-    Measured on Llama-3-8B heads (32 / 8 x 128): 4 waves, two workgroups on a compute unit, beat 8 at every size that does
-    not fill the chip twice over with 8 (333 rows 15.5 against 20 us, 2048 rows 65 against 76; 8191 rows 675 against 630).
+    4 waves, two workgroups on a compute unit, unless sequences of 4096 rows and more fill the chip twice over with 8 (Llama-3-8B
+    heads, 32 / 8 x 128, us with 4 / 8: 4096 rows 182 / 172, 8191 616 / 599, but 4 x 2000 183 / 190, 16 x 500 80 / 91, and blocks
+    that are part empty pay twice: 64 x 17 rows 11.7 / 18.4).
     A grid of fewer than two workgroups per compute unit is split over its keys where the context is long: 416 rows behind
-    12000 keys 275 -> 140 us, 289 behind 2000 58 -> 41; the merge launch costs 2-3 us where it has nothing to merge, so
-    contexts that are known to be short (ctx_lens_host; else what the block tables can hold) do not ask for it."""
+    12000 keys 275 -> 140 us, 289 behind 2000 58 -> 41; the merge launch costs 1.5-2 us where it has nothing to merge, so
+    contexts that are known to be short (else what the block tables can hold) do not ask for it.
+    Contexts of one key tile are the 16-row kernel's where its smaller workgroups wait less (us here / there, D 128): few of
+    them 8.6 / 7.4 (33 rows), sequences that its row tiles hold whole 9.4 / 7.4 (64 x 1), 27 / 19 (200 x 1), 17.4 / 14.4 (100 x
+    10), with a soft cap 9.4 / 7.5 (33 rows); not 11.7 / 17.3 (64 x 17), nor beyond what the chip holds at once with more than 4
+    heads a group, 7.4 / 15 (400 x 1, 16 / 1 heads). D 64 only for crowds: 5.8 / 5.6 (1 x 1), 10.5 / 7.6 (100 x 1). It needs `tiles`."""
     if D not in (64, 128) or Hkv <= 0 or Hq % Hkv:
         return None
     G = Hq // Hkv
     if G > 128 or (G > 8 and G % 8) or (D == 64 and G in (3, 5, 6, 7)):
         return None
+    longest = max(ctx_lens_host) if ctx_lens_host else block_size * table_width
+    if tiles and longest <= 64:
+        rt = 16 * max(1, 4 // G)
+        whole = T <= rt * n_seqs
+        waves = (T // rt + n_seqs) * (Hq // min(G, 8)) * max(4, min(G, 8))
+        if whole and G <= 4 and n_seqs * Hkv > 2 * CU_COUNT or (D == 128 or softcap > 0) and waves <= (8.5 if whole else 4) * CU_COUNT:
+            return None
     blocks = lambda waves: T // (32 * waves // G) + min(n_seqs, T)  # noqa: E731
-    if D == 128 and blocks(8) * Hkv >= 2 * CU_COUNT:
+    if D == 128 and T >= 4096 * n_seqs and T // (256 // G) * Hkv >= 2 * CU_COUNT:
         return (8, 1) if blocks(8) <= 65535 else None
     base = blocks(4) * Hkv
-    keys = max(ctx_lens_host) if ctx_lens_host else block_size * table_width
-    if window > 0:
-        keys = min(keys, window + 32 * 4 // G)
+    keys = min(longest, window + 32 * 4 // G) if window > 0 else longest
     parts = max(1, min(16, 2 * CU_COUNT // base)) if keys >= FLASH_SPLIT_KEYS else 1
     return (4, parts) if blocks(4) <= 65535 else None
 
@@ -478,7 +489,7 @@ def attn_prefill(q: torch.Tensor, k_cache, v_cache, block_tables: torch.Tensor, 
     if q.is_cuda:
         vmode = ATTN_VMODE if vmode is None else int(vmode)
         plan = flash_plan(T, cu_q.numel() - 1, Hq, k_cache.shape[1], D, k_cache.shape[2], block_tables.shape[1], window,
-                          ctx_lens_host) if vmode == 0 else None
+                          ctx_lens_host, softcap, tiles is not None) if vmode == 0 else None
         if plan is not None:
             waves, parts = plan
             po = ml = None
@@ -491,8 +502,6 @@ def attn_prefill(q: torch.Tensor, k_cache, v_cache, block_tables: torch.Tensor, 
                     k_cache.shape[1], D, k_cache.shape[2], float(scale), int(window), float(softcap), out.data_ptr(),
                     waves, parts, N.ptr(po), N.ptr(ml), kv_format(k_cache), N.stream_ptr())
             return out
-        if D != 256:
-            vmode = 1
     if tiles is not None and q.is_cuda:
         Hkv, bs = k_cache.shape[1], k_cache.shape[2]
         N.ensure_act(out.dtype)

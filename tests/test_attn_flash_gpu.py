@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 import torch
 
+from localai_tfp_amd import _native as N
 from localai_tfp_amd.ops import core as K
 from localai_tfp_amd.ops import kvq as KQ
 
@@ -30,7 +31,7 @@ def _case(Hq, Hkv, D, q_lens, pre, bs=16, fmt="bf16", seed=0):
     return q, kc, vc, bt, torch.tensor(np.concatenate([[0], np.cumsum(q_lens)]), dtype=torch.int32), torch.tensor(ctx, dtype=torch.int32)
 
 
-def _check(Hq, Hkv, D, q_lens, pre, window=0, softcap=0.0, scale=None, plan=None, monkeypatch=None, **kw):
+def _check(Hq, Hkv, D, q_lens, pre, window=0, softcap=0.0, scale=None, plan=None, monkeypatch=None, tiles=False, **kw):
     q, kc, vc, bt, cu, ctx = _case(Hq, Hkv, D, q_lens, pre, **kw)
     scale = D ** -0.5 if scale is None else scale
     want = torch.zeros(q.shape)
@@ -44,7 +45,12 @@ def _check(Hq, Hkv, D, q_lens, pre, window=0, softcap=0.0, scale=None, plan=None
     if hasattr(kc, "kvf"):
         kd.kvf, vd.kvf = kc.kvf, vc.kvf
     out = torch.full(q.shape, float("nan"), dtype=torch.float16, device="cuda")
-    K.attn_prefill(q.cuda(), kd, vd, bt.cuda(), cu.cuda(), ctx.cuda(), scale, out, window=window, softcap=softcap)
+    if tiles:
+        rows = N.kernels().mxk_attn_prefill_rows(Hq, Hkv)
+        tiles = [torch.tensor(v + [-1], dtype=torch.int32).cuda() for v in K.prefill_tiles(q_lens, rows)]
+        assert K.flash_plan(q.shape[0], len(q_lens), Hq, Hkv, D, kc.shape[2], bt.shape[1], window, ctx.tolist(), softcap, True) is None
+    K.attn_prefill(q.cuda(), kd, vd, bt.cuda(), cu.cuda(), ctx.cuda(), scale, out, q_lens, ctx.tolist(), window=window, softcap=softcap,
+                   tiles=tiles or None)
     got = out.cpu().float()
     # probabilities and outputs are rounded to 16 bits once each (2^-9, 2^-11): over a row of summed values the relative
     # error stays below 4 x 2^-9
@@ -63,12 +69,42 @@ def test_plan_takes_what_the_kernel_takes():
     assert all(1 <= p(t, s, 8 * g, 8, 128, 16, 4096, 0)[1] <= 16 for t in (1, 17, 500, 4000) for s in (1, 9, 200) for g in (1, 2, 3, 5, 7, 8, 16))
 
 
+def test_plan_of_short_contexts_and_of_many_sequences():
+    """Known contexts of one key tile run the 16-row kernel where it is the faster one, and only where its tile lists are at hand; 8
+    waves are for sequences that fill their blocks."""
+    p = K.flash_plan
+    one = lambda T, n, D, ctx, cap=0.0, tiles=True, H=32: p(T, n, H, 8, D, 16, 512, 0, [ctx] * n, cap, tiles)  # noqa: E731
+    assert one(33, 1, 128, 33) is None and one(64, 64, 128, 1) is None and one(200, 200, 128, 1) is None and one(1000, 100, 128, 50) is None
+    assert one(33, 1, 128, 33, tiles=False) == (4, 1) and one(33, 1, 128, 65) == (4, 1) and one(4000, 100, 128, 40) == (4, 1)
+    assert one(17 * 64, 64, 128, 17) == (4, 1) and p(400, 400, 16, 1, 128, 16, 512, 0, [1] * 400, 0.0, True) == (4, 1)
+    assert one(33, 1, 64, 33) == (4, 1) and one(200, 200, 64, 1) is None and one(17 * 64, 64, 64, 17) == (4, 1)
+    assert one(33, 1, 64, 33, 50.0) is None and one(100, 1, 128, 100, 50.0) == (4, 1) and one(4000, 100, 128, 40, 50.0) == (4, 1)
+    assert one(17 * 64, 64, 128, 500) == (4, 1) and one(8000, 16, 128, 500) == (4, 1)  # (8 waves: 1.6 times as long)
+    assert p(100, 1, 32, 8, 128, 16, 4, 0, None, 0.0, True) is None  # (tables of 64 keys are a bound too)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", ["bf16", "fp8", "q8_0", "q4_0", "q4_1", "q5_0", "q5_1", "iq4_nl"])
+@pytest.mark.parametrize("Hq,Hkv,D", [(32, 8, 128), (8, 8, 128), (6, 2, 128), (28, 4, 128), (16, 1, 128), (32, 8, 64), (4, 2, 64), (8, 1, 64)])
+def test_short_contexts_on_the_row_kernel(fmt, Hq, Hkv, D):
+    _check(Hq, Hkv, D, [1, 15, 16, 0, 17, 33, 64], [0, 5, 48, 0, 20, 31, 0], softcap=50.0, tiles=True, fmt=fmt)
+    if Hkv >= 8:  # a crowd of short sequences
+        _check(Hq, Hkv, D, [i % 9 for i in range(120)], [(i * 7) % 50 for i in range(120)], tiles=True, fmt=fmt)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("Hq,Hkv,D", [(32, 8, 128), (8, 8, 128), (6, 2, 128), (28, 4, 128), (16, 1, 128), (32, 8, 64), (4, 2, 64), (40, 1, 128)])
 def test_query_blocks_and_key_tiles(Hq, Hkv, D):
     """Blocks of queries and tiles of keys that end just before, at and after an edge; sequences without rows between others."""
     _check(Hq, Hkv, D, [1, 31, 0, 33, 64, 65, 0], [0, 33, 5, 31, 0, 63, 9])
     _check(Hq, Hkv, D, [130], [127], bs=24)  # pages that are no power of two
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 130])
+def test_which_sequence_a_block_belongs_to(n, monkeypatch):
+    """Up to 64 sequences are found by one scan over the lanes, more in rounds of 64; some have no rows."""
+    _check(8, 2, 128, [(i * 7) % 45 for i in range(n)][::-1] if n > 1 else [40], [(i * 13) % 70 for i in range(n)], plan=(4, 1), monkeypatch=monkeypatch)
 
 
 @pytest.mark.gpu
