@@ -27,6 +27,7 @@ import torch
 from ..utils import roctx
 from ..utils.pinned import PinnedRing
 from ..models.llama import ForwardBatch, LlamaModel, Workspace
+from ..ops.core import flash_plan
 from ..ops.sampling import SamplerBatch
 from .kv_cache import KVCache, LatentCache, SlotPool, make_block_manager
 from .scheduler import ScheduledSeq, Scheduler, SchedulerOutput, needs_host_state
@@ -98,7 +99,7 @@ class EngineConfig:
                                                        "64,128,192,256,288,320,352,384,448,512,768,1024").split(",")
                               if x.strip())
     mixed_graph_seqs: int = 4
-    max_graphs: int = 64
+    max_graphs: int = 128
     attn_part_size: int = 256  # must match ops.core.attn_decode's default
     # dense 16-bit copy of the layer projections for hipBLASLt (ops/linear.py DENSE_MIN_M_*). Off: the K-quant
     # MFMA kernels (qmm2 / qmm3) run every M > 4 GEMM on the quantised weights; MX_DENSE_CACHE=1 restores the copy
@@ -202,7 +203,7 @@ class StepGraph:
     image into a pinned ring buffer and refreshes all inputs with ONE async H2D copy per step.
     """
 
-    def __init__(self, engine: "LLMEngine", B: int, P: int = 0, PS: int = 0, L: int = 0):
+    def __init__(self, engine: "LLMEngine", B: int, P: int = 0, PS: int = 0, L: int = 0, C: int = 0):
         e = engine
         dev = e.device
         self.B, self.P, self.PS = B, P, PS
@@ -250,6 +251,8 @@ class StepGraph:
         if P:
             self.fb.pf_block_tables, self.fb.pf_cu_q, self.fb.pf_ctx_lens = v["pf_bt"], v["pf_cu"], v["pf_ctx"]
             self.fb.pf_tiles = (v["pf_tseq"], v["pf_tq0"])
+            if C:  # every prompt's context is at most C keys: the bound stands for the contexts that a capture cannot know
+                self.fb.pf_ctx_lens_host = [C]
         self.graph = None
         self.logits = None
         self.replay_s = 0.0  # host time inside hipGraphLaunch (profiling)
@@ -461,6 +464,7 @@ class LLMEngine:
         self._thread: threading.Thread | None = None
         self._stop = False
         self.graphs: dict[tuple, StepGraph] = {}
+        self._bounds: dict[int, list] = {}  # _prompt_bounds
         self._graph_pool = None
         self.use_graphs = c.use_graphs and self.device.type == "cuda"
         self.eos_ids = set(getattr(tokenizer, "eos_token_ids", []) or [])
@@ -577,9 +581,8 @@ class LLMEngine:
             for p in c.mixed_graph_tokens:
                 if p > c.max_batched_tokens or top + p > self.ws.max_tokens:
                     continue
-                keys.append((top, p, c.mixed_graph_seqs, 0))
-                if top >= self.SINGLE_PART_B:
-                    keys.append((top, p, c.mixed_graph_seqs, self.SINGLE_PART_CTX))
+                for ctx in (0, self.SINGLE_PART_CTX) if top >= self.SINGLE_PART_B else (0,):
+                    keys += [(top, p, c.mixed_graph_seqs, ctx, *bound) for bound in ((), *((x,) for x in self._prompt_bounds(p)))]
             for k in keys:
                 if len(self.graphs) >= c.max_graphs:
                     break
@@ -960,6 +963,21 @@ class LLMEngine:
     # (models/llama.py SINGLE_PART_*: no partition-merge launch per layer)
     SINGLE_PART_CTX, SINGLE_PART_B = 1024, int(os.environ.get("MX_SINGLE_PART_MIN_B", "64"))
 
+    # mixed steps whose prompts' contexts are all this short replay a graph captured with that bound, whose prompt attention
+    # (ops/core.py flash_plan) does without key parts and their merge launch, or runs the kernel for one key tile. Llama-3-8B
+    # heads, tables of 8192 keys, us a layer without / with the bound: 37 rows 9.1 / 6.6, 333 15.8 / 14.0, 4 x 70 10.0 / 8.3; parts
+    # win from about 1300 keys on (288 rows behind 1100 37.2 / 38.0, 64 behind 1900 35 / 50)
+    PROMPT_CTX = (64, 1280)
+
+    def _prompt_bounds(self, P: int) -> list:
+        """The bounds for which P prompt tokens run another attention plan than without one."""
+        if P not in self._bounds:
+            c, m = self.cfg, self.model
+            plan = lambda host: flash_plan(P, c.mixed_graph_seqs, m.n_heads, m.n_kv, m.cfg.head_dim, c.block_size,  # noqa: E731
+                                           self.max_blocks_per_seq, 0, host, m.cfg.attn_softcap, True)
+            self._bounds[P] = [x for x in self.PROMPT_CTX if P <= x < c.max_model_len and plan([x]) != plan(None)]
+        return self._bounds[P]
+
     def _graph_for(self, n: int) -> StepGraph | None:
         """Decode-only graph of the bucket holding n rows."""
         b = self._dec_bucket(n)
@@ -969,7 +987,7 @@ class LLMEngine:
         return next((x for x in self.cfg.graph_buckets if x >= n and x <= self.cfg.max_num_seqs), None)
 
     def _graph_key(self, plan: dict):
-        """Shape bucket (B, P, PS) whose graph can run this plan, or None (eager)."""
+        """Shape bucket (B, P, PS, L[, C]) whose graph can run this plan, or None (eager)."""
         c = self.cfg
         if not self.use_graphs or "mm" in plan or plan["keep_hidden"]:
             return None
@@ -993,10 +1011,11 @@ class LLMEngine:
         if P is None or B + P > self.ws.max_tokens:
             return None
         # the decode rows of a mixed step: one attention partition per sequence too (no partition-merge launch)
-        if nd and B >= self.SINGLE_PART_B and int(plan["dec_lens"].max()) <= self.SINGLE_PART_CTX and \
-                os.environ.get("MX_MIXED_SINGLE_PART", "1") == "1":
-            return (B, P, c.mixed_graph_seqs, self.SINGLE_PART_CTX)
-        return (B, P, c.mixed_graph_seqs, 0)
+        one = nd and B >= self.SINGLE_PART_B and int(plan["dec_lens"].max()) <= self.SINGLE_PART_CTX and \
+            os.environ.get("MX_MIXED_SINGLE_PART", "1") == "1"
+        key = (B, P, c.mixed_graph_seqs, self.SINGLE_PART_CTX if one else 0)
+        longest = int(plan["pf_ctx"].max())
+        return key + tuple(x for x in self._prompt_bounds(P) if longest <= x)[:1]
 
     def _graph_get(self, key, create: bool = True) -> StepGraph | None:
         if not self.use_graphs:
@@ -1114,15 +1133,14 @@ class LLMEngine:
             from ..ops.core import prefill_tiles
             ts, tq = prefill_tiles([it.n for it in pf], self.model.prefill_rows())
             plan["pf_tseq"], plan["pf_tq0"] = np.asarray(ts, np.int32), np.asarray(tq, np.int32)
-        key = self._graph_key(plan)
+        key, g = self._graph_key(plan), None
         # tensor parallel: a capture runs collectives, so only graphs every rank captured up front
-        # (precapture_graphs: decode buckets) are used; single-rank engines capture on first use
-        g = self._graph_get(key, create=self.tp is None) if key is not None else None
-        if g is None and key is not None and key[3]:
-            # a short-context form that is not captured (tensor parallel replays precaptured buckets only): the
-            # bucket's full-context graph runs the same step
-            key = (key[0], key[1], key[2], 0)
+        # (precapture_graphs: decode buckets) are used; single-rank engines capture on first use. Where a short-context
+        # form is not captured (tensor parallel, or max_graphs reached) the bucket's wider graphs run the same step
+        for key in dict.fromkeys((key, key[:4], key[:3] + (0,))) if key is not None else ():
             g = self._graph_get(key, create=self.tp is None)
+            if g is not None:
+                break
         plan["graph"] = key if g is not None and g.fits(plan) else False
         return plan
 
