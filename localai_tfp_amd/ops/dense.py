@@ -25,17 +25,18 @@ def to_dev(a, device, dtype) -> torch.Tensor:
 def few_rows_parts(M: int, N: int, K: int) -> int:
     """Parts of K that csrc/kernels/lin16.hip sums for M rows, or 0 where the library multiplies.
 
-    Measured with weights in no cache (bf16, us, here / library): long K and few columns, where the library's choice degrades
-    beyond K = 16384: 4096 x 16384 35-50 / 31-43, x 17408 34-52 / 47-129, x 24576 45-70 / 66-148, x 28672 51-79 / 57-166,
-    2048 x 20480 23-34 / 60-80 (1-64 rows); but 5120 x 20480 49-56 / 50-53 to 16 rows, 8192 x 20480 66-89 / 59-65 to 32. Many
-    columns and up to 8 rows: 28672 x 4096 52-56 / 66, 32000 56-58 / 61, 41024 69-74 / 74-77, 65536 x 2048 52-56 / 67; 16384 x
-    4096 31-32 / 33 and 12288 26 / 24 stay. Parts make one workgroup per compute unit (4096 columns: 1 / 2 / 4 / 8 parts 148 /
-    80 / 50 / 52 us)."""
+    Measured with weights in no cache (bf16, f16 alike; us, here / library): long K and few columns, where the library's choice
+    degrades beyond K = 16384: 4096 x 17408 0.75 of the library's time at one row, 0.34-0.4 beyond 32, x 28672 0.96 and 0.4-0.47,
+    3072 0.65-0.9 and 0.3-0.6, 2048 0.25-0.6, 1024 0.22-0.7, 128-512 0.22-1.0; but 64 x 49152 1.06-1.4 beyond 32 rows, 5120 x
+    20480 49-56 / 50-53 to 16 rows, 8192 x 20480 66-89 / 59-65 to 32. Many columns and up to 8 rows: 24576-32768 x 512-2304
+    0.67-1.0, 28672-32768 x 4096 0.84-0.98; 24576 x 4096 1.1, any x 5120 and 8192 up to 1.4, and beyond 32768 columns the library is
+    as good or better at most widths (51200 x 1280 1.14-1.25, 256000 x 2304 1.07-1.17). Parts make one workgroup per compute unit
+    (4096 columns: 1 / 2 / 4 / 8 parts 148 / 80 / 50 / 52 us)."""
     if N % 64 or K % 32 or not 0 < M <= 64:
         return 0
     if K > 16384 and N <= 4096:
-        return min(8, 256 // (N // 64))
-    return 1 if N >= 24576 and M <= 8 else 0
+        return min(8, 256 // (N // 64)) if N >= 128 or K <= 32768 or M <= 32 else 0
+    return 1 if 24576 <= N <= 32768 and M <= 8 and K <= (4096 if N >= 28672 else 2304) else 0
 
 
 def _few_rows(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, acc: bool) -> bool:

@@ -16,6 +16,13 @@ def test_rule():
     assert all(0 <= p(m, n, k) <= 8 for m in (1, 64) for n in range(64, 4097, 64) for k in (16416, 40960))
 
 
+def test_rule_leaves_the_library_what_it_does_better():
+    p = D.few_rows_parts
+    assert p(1, 24576, 2048) == p(8, 28672, 2304) == p(4, 32768, 4096) == 1
+    assert p(1, 24576, 4096) == p(8, 32768, 5120) == p(1, 28672, 8192) == p(8, 51200, 1280) == p(1, 256000, 2304) == p(8, 41024, 4096) == 0
+    assert p(32, 64, 65536) == p(64, 64, 32768) == 8 and p(33, 64, 65536) == 0 and p(64, 128, 65536) == 8
+
+
 def test_route_takes_only_what_the_kernel_reads(monkeypatch):
     """What lin16.hip would read past, or from another device, stays with the library's product. On descriptions of tensors: no
     call may reach a kernel."""
@@ -36,7 +43,7 @@ def test_route_takes_only_what_the_kernel_reads(monkeypatch):
         took = D._few_rows(x or t((8, K)), w or t((N, K)), out or t((8, N), dtype=torch.float32), False)
         assert took == (len(calls) == 1)
         return took
-    N, K = 24576, 4096
+    N, K = 28672, 4096
     assert route() and calls[0][1][1] == K
     assert route(x=t((8, K), (K + 16, 1))) and calls[0][1][1] == K + 16
     assert route(x=t((1, K), (0, 1)), out=t((1, N), dtype=torch.float32)) and calls[0][1][1] == K  # one row: no stride to follow
