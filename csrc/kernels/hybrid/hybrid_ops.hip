@@ -296,8 +296,9 @@ __global__ __launch_bounds__(64) void rope_norm_append_kernel(const float* qi, c
 
 // grid (ceil(C / NT), sequences, ceil(T / CONV_ROWS)): thread = channel. Reads the tails only; conv_tails_kernel
 // rolls them afterwards. TAPS 2 .. 4: the last inputs slide through registers, one read a row (1990 rows of 4352 channels, 4
-// taps: 57 us with a read per tap and row, 19 with these); 0: any number up to 16.
-constexpr int CONV_ROWS = 16;
+// taps: 57 us with a read per tap and row, 19 with these); 0: any number up to 16, where a thread's rows come one after another
+// and half as many take half as long (300 rows of 1000 channels, 5 taps: 19.2 us with 16 rows, 12.1 with 8).
+constexpr int conv_rows(int taps) { return taps >= 2 && taps <= 4 ? 16 : 8; }
 template <int TAPS>
 __global__ __launch_bounds__(NT) void causal_conv_kernel(const float* x, int ldx, const float* w, const float* bias,
                                                          int taps, int silu, float* tails, const int* state,
@@ -314,6 +315,7 @@ __global__ __launch_bounds__(NT) void causal_conv_kernel(const float* x, int ldx
         row0 = n_dec + pf_cu[k];
         n = pf_cu[k + 1] - pf_cu[k];
     }
+    constexpr int CONV_ROWS = conv_rows(TAPS);
     const int t0 = blockIdx.z * CONV_ROWS;
     if (t0 >= n || c >= C) return;
     const int slot = state[s];
@@ -763,7 +765,7 @@ extern "C" int mxh_causal_conv(const float* x, int ldx, const float* w, const fl
     MXH_CHECK(x && w && tails && state && positions && out && C > 0 && taps >= 1 && taps <= 16);
     MXH_CHECK(ldx >= C && ldo >= C && n_dec >= 0 && n_pf >= 0 && n_dec + n_pf > 0 && (n_pf == 0 || pf_cu));
     const int rows = n_pf ? T - n_dec : 1;
-    const dim3 grid((C + NT - 1) / NT, n_dec + n_pf, (max(rows, 1) + CONV_ROWS - 1) / CONV_ROWS);
+    const dim3 grid((C + NT - 1) / NT, n_dec + n_pf, (max(rows, 1) + conv_rows(taps) - 1) / conv_rows(taps));
 #define GO(T_)                                                                                                          \
     causal_conv_kernel<T_><<<grid, NT, 0, st>>>(x, ldx, w, bias, taps, silu, tails, state, positions, n_dec, pf_cu, out, \
                                                 ldo, C)
