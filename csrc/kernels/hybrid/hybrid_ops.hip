@@ -540,8 +540,9 @@ MX_DEV float glu_one(float x, float y, float fac, int act, float limit, float al
     }
     return (act == 1 ? gelu_tanh_acc(x) : silu_acc(x)) * y * fac;
 }
-// V elements a thread: 4 where every row, factor group and operand allows 16-byte reads, else 1. Bound by its bytes: 1990 rows of
-// 14336 (285 MB) took 113 us with one element a thread, 84 with four.
+// V elements a thread: 4 where every row, factor group and operand allows 16-byte reads and there are a million of them, else 1.
+// Many are bound by their bytes: 1990 rows of 14336 (285 MB) took 113 us with one element a thread, 84 with four; few by the chain
+// of one thread: 128 x 2048 2.9 us with one, 3.4 with four; 128 x 14336 5.5 / 4.6.
 template <bool B16, int V>
 __global__ __launch_bounds__(NT) void glu_kernel(const float* a, int lda, const float* b, int ldb, const float* ba,
                                                  const float* bb, const float* scale, int lds, int group,
@@ -841,7 +842,7 @@ extern "C" int mxh_glu(const float* a, int lda, const float* b, int ldb, const f
     MXH_CHECK(a && out && lda >= F && ldo >= F && group > 0 && F <= 65535 * NT && act >= 0 && act <= 4);
     MXH_CHECK(act == 2 || act == 4 ? !b : (b && ldb >= F));  // the squared ReLU and the plain gelu have one operand
     MXH_CHECK(!scale || (F % group == 0 && lds >= F / group));
-    const bool four = F % 4 == 0 && group % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0 && ldo % 4 == 0 &&
+    const bool four = (long)T * F >= 1 << 20 && F % 4 == 0 && group % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0 && ldo % 4 == 0 &&
                       ((uintptr_t)a | (uintptr_t)b | (uintptr_t)out) % 16 == 0;
 #define GO(B, V)                                                                                                      \
     glu_kernel<B, V><<<dim3(T, (F + NT * V - 1) / (NT * V)), NT, 0, st>>>(a, lda, b, ldb, ba, bb, scale, lds, group, \

@@ -93,3 +93,20 @@ def test_conv_blocks_of_rows(taps):
         HY.causal_conv(x.to(dev)[:, 3:], w.to(dev), bias.to(dev), tails, _rag(n_dec, chunks, at, slots, dev), out, silu=True)
         res.append((out.cpu(), tails.cpu()))
     assert (res[0][0] - res[1][0]).abs().max() < 1e-5 and torch.equal(res[0][1], res[1][1])
+
+
+@pytest.mark.parametrize("act", ["silu", "relu2", "clamped", "gelu"])
+def test_glu_of_many_elements(act):
+    """A million numbers and more run four elements a thread where widths and addresses allow it; the bound of test_glu_widths."""
+    g = torch.Generator().manual_seed(2)
+    T, F = 300, 4096
+    a, b, sc = (torch.randn(T, n, generator=g) for n in (F + 1, F, F // 256))
+    for off in (0, 1):
+        for dt in (torch.float32, torch.bfloat16):
+            got = {}
+            for dev in ("cpu", "cuda"):
+                out = torch.empty(T, F, dtype=dt, device=dev)
+                HY.glu(a.to(dev)[:, off:off + F], None if act in HY.GLU_SINGLE else b.to(dev), None, None, out, sc.to(dev), 256, True, act, 2.0, 1.7)
+                got[dev] = out.cpu().float()
+            tol = 2e-5 if dt == torch.float32 else 2 ** -7
+            assert ((got["cuda"] - got["cpu"]).abs() <= tol * got["cpu"].abs().clamp_min(1)).all()
