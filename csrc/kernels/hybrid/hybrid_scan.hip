@@ -14,7 +14,7 @@
 // (its decay is multiplied in after the sum), a step's LDS reads are asked for a step ahead, and output sums over a column's
 // lanes are made for 8 or 16 steps together, transposed on the way (3 operations a step instead of a chain of 4 and a store).
 // Prompts of 301 / 578 / 1111 rows: delta rule 576 -> 250 us, 64 heads of 64 x 128 without it 554 -> 227 (0.2 us a step;
-// most of the gain is that a round's loads no longer wait for each other). Steps of decode rows alone (ONE) stage one token and
+// most of the gain is that a round's loads no longer wait for each other). Decode rows and short chunks (ONE) stage one token and
 // sum at once: 33 rows 18.0 -> 12.6 and 30.3 -> 22.2 us (6.2 TB/s of states read and written).
 // CHD (gated linear attention): the decay is one number per head and state row, a_t[n], staged beside k_t and q_t:
 // S[n][p] <- a_t[n] S[n][p] + k_t[n] u[p]; with DELTA as well, the delta rule's read follows that per-row decay. A
@@ -47,7 +47,7 @@ MX_DEV float lanes_sum(float v) {
     return v;
 }
 
-// grid (column blocks, H, sequences); block = 256 threads = 256 / LPC columns
+// grid (column blocks, H, sequences from s0 on); block = 256 threads = 256 / LPC columns. ONE: rounds of one token
 template <int NPL, int LPC, bool DELTA, bool CHD, bool ONE>
 __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk, const float* q, int ldq,
                                                          const float* v, int ldv, const float* decay, int ldd,
@@ -55,7 +55,7 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk
                                                          const float* skip, float* state, const int* seq_state,
                                                          const int* positions, int n_dec, const int* pf_cu, float* out,
                                                          int ldo, int H, int G, int N, int P, float q_scale,
-                                                         float* nout) {
+                                                         float* nout, int s0) {
     static_assert(LPC == 4 || LPC == 16, "a column's lanes are a quad or a DPP row");
     constexpr int NT = 256;
     constexpr int NP = NPL * LPC;  // padded N
@@ -69,7 +69,7 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk
     const int cl = threadIdx.x / LPC;
     const int col = blockIdx.x * COLS + cl;
     const int part = threadIdx.x % LPC;
-    const int h = blockIdx.y, s = blockIdx.z;
+    const int h = blockIdx.y, s = s0 + blockIdx.z;
     int row0, n;
     if (s < n_dec) {
         row0 = s;
@@ -356,7 +356,7 @@ extern "C" int mxh_state_scan(const float* k, int ldk, const float* q, int ldq, 
                               const float* decay, int decay_rows, const float* coef, int ldc, int coef_sigmoid,
                               const float* skip, float* state, const int* seq_state, const int* positions, int n_dec,
                               const int* pf_cu, int n_pf, float* out, int ldo, int H, int G, int N, int P, int delta,
-                              int channel, float q_scale, float* nout, hipStream_t st) {
+                              int channel, float q_scale, float* nout, int T, hipStream_t st) {
     const int n_seqs = n_dec + n_pf;
     if (n_seqs <= 0) return 0;
     MXH_CHECK(k && q && v && decay && state && seq_state && positions && out && (n_pf == 0 || pf_cu));
@@ -368,15 +368,28 @@ extern "C" int mxh_state_scan(const float* k, int ldk, const float* q, int ldq, 
     const int threads = 256;
     const int cols = threads / lpc;
     const dim3 grid((P + (nout ? 1 : 0) + cols - 1) / cols, H, n_seqs);
+    // Short prompt chunks step token by token as decode rows do (ONE): staging 8 or 16 tokens and reading them ahead costs registers,
+    // which are what keeps states in flight. us, staged / one by one: 8 heads of 128 x 256 with channel decays, 64 chunks of 3
+    // tokens 89 / 30, 16 of 4 26.5 / 11.4, 33 decode rows + 3 tokens 46 / 15; 16 heads of 128 x 128, one chunk of 4 tokens 4.8 / 5.0,
+    // of 8 5.4 / 7.0, with channel decays 8.4 / 7.5.
+    // Decode rows that fill the chip by themselves run as a launch of their own beside longer chunks: 127 rows + 64 tokens, 16 heads of
+    // 128 x 128 66 -> 58 us, with channel decays 165 -> 66; few stay in the chunks' launch (8 rows + 289 tokens 70).
+    const int few = N > 64 ? (!channel ? 4 : n_pf < 8 ? 12 : 16) : channel ? 4 : 3;
+    const bool one = T - n_dec <= (long)few * n_pf, apart = !one && (long)grid.x * H * n_dec >= 4096;
+    const dim3 grid_dec(grid.x, H, n_dec), grid_pf(grid.x, H, apart ? n_pf : n_seqs);
 #define GO2(NPL, LPC, D_, C_)              \
     do {                                   \
-        if (n_pf) GO3(NPL, LPC, D_, C_, false); \
-        else GO3(NPL, LPC, D_, C_, true);  \
+        if (one) {                         \
+            GO3(NPL, LPC, D_, C_, true, grid, 0); \
+            break;                         \
+        }                                  \
+        if (apart) GO3(NPL, LPC, D_, C_, true, grid_dec, 0); \
+        GO3(NPL, LPC, D_, C_, false, grid_pf, apart ? n_dec : 0); \
     } while (0)
-#define GO3(NPL, LPC, D_, C_, O_)                                                                                  \
-    state_scan_kernel<NPL, LPC, D_, C_, O_><<<grid, threads, 0, st>>>(k, ldk, q, ldq, v, ldv, decay, ldd, coef, ldc,      \
+#define GO3(NPL, LPC, D_, C_, O_, GRID, S0)                                                                                  \
+    state_scan_kernel<NPL, LPC, D_, C_, O_><<<GRID, threads, 0, st>>>(k, ldk, q, ldq, v, ldv, decay, ldd, coef, ldc,      \
                                                                   coef_sigmoid, skip, state, seq_state, positions,    \
-                                                                  n_dec, pf_cu, out, ldo, H, G, N, P, q_scale, nout)
+                                                                  n_dec, pf_cu, out, ldo, H, G, N, P, q_scale, nout, S0)
 #define GO(NPL, LPC)                              \
     do {                                          \
         if (delta && channel) GO2(NPL, LPC, true, true); \

@@ -206,7 +206,7 @@ HYBRID_SIGS = {
     "mxh_channel_decay": [P, I, P, F, P, I, I, P, I, P, I, P],
     # k, ldk, q, ldq, v, ldv, decay, coef, skip, state, seq_state, positions, n_dec, pf_cu, n_pf, out, ldo, H, G, N, P,
     # delta, channel, q_scale, normaliser out, stream
-    "mxh_state_scan": [P, I, P, I, P, I, P, I, P, I, I, P, P, P, P, I, P, I, P, I, I, I, I, I, I, I, F, P, P],
+    "mxh_state_scan": [P, I, P, I, P, I, P, I, P, I, I, P, P, P, P, I, P, I, P, I, I, I, I, I, I, I, F, P, I, P],
     # y, ldy, gate, ldg, w, wlen, eps, group, gate_first, out_scale, out, ldo, o16, T, C, sigmoid gate, proj, R, den, den_min,
     # ldd, den_eps, stream
     "mxh_gated_group_norm": [P, I, P, I, P, I, F, I, I, F, P, I, I, I, I, I, P, I, P, P, I, F, P],

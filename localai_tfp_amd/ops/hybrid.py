@@ -893,7 +893,7 @@ def state_scan(k: torch.Tensor, q: torch.Tensor, v: torch.Tensor, decay: torch.T
             coef.stride(0) if coef is not None else 0, int(coef_sigmoid), N.ptr(skip), state.data_ptr(),
             rag.state.data_ptr(),
             rag.positions.data_ptr(), rag.n_dec, N.ptr(rag.pf_cu), rag.n_pf, out.data_ptr(), out.stride(0), H, G, Nk,
-            P, int(delta), int(channel), float(q_scale), N.ptr(norm_out), N.stream_ptr())
+            P, int(delta), int(channel), float(q_scale), N.ptr(norm_out), T, N.stream_ptr())
     return out
 
 

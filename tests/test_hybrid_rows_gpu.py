@@ -50,6 +50,29 @@ def test_rounds_of_tokens(N, P, delta, channel, nout):
         assert (a - b).abs().max() <= 2e-5 * b.abs().max()
 
 
+@pytest.mark.parametrize("H,N,P,n_dec,chunks", [(2, 128, 20, 0, [1]), (2, 128, 20, 3, [2, 9, 1]), (2, 64, 33, 1, [3]), (2, 64, 33, 0, [4]),
+                                                (3, 32, 70, 2, [1] * 6 + [11]), (2, 200, 17, 0, [12, 12]), (16, 128, 64, 64, [37]),
+                                                (16, 128, 64, 64, [3]), (8, 256, 128, 70, [20, 0, 30])])
+@pytest.mark.parametrize("delta,channel", [(True, False), (False, True), (True, True)])
+def test_short_chunks_and_rows_apart(H, N, P, n_dec, chunks, delta, channel):
+    """Chunks that step token by token, whole or among longer ones, and decode rows that run as a launch of their own; the bound of
+    test_rounds_of_tokens."""
+    g = torch.Generator().manual_seed(N + n_dec)
+    T, slots = n_dec + sum(chunks), list(range(n_dec + len(chunks)))[::-1]
+    k, q, v = torch.randn(T, N, generator=g) * N ** -0.5, torch.randn(T, N, generator=g), torch.randn(T, H * P, generator=g)
+    decay, coef = torch.rand(T, H * N if channel else H, generator=g), torch.rand(T, H, generator=g)
+    at = [(i * 3) % 5 for i in range(len(slots))]
+    start = torch.randn(len(slots), H, P, N, generator=g)
+    got = {}
+    for dev in ("cpu", "cuda"):
+        state, out = start.clone().to(dev), torch.zeros(T, H * P, device=dev)
+        HY.state_scan(k.to(dev), q.to(dev), v.to(dev), decay.to(dev), coef.to(dev), None, state, _rag(n_dec, chunks, at, slots, dev), out,
+                      H, 1, N, P, delta, channel, 0.5, False, None)
+        got[dev] = [out.cpu(), state.cpu()]
+    for a, b in zip(got["cuda"], got["cpu"]):
+        assert (a - b).abs().max() <= 2e-5 * b.abs().max()
+
+
 @pytest.mark.parametrize("F,group,off", [(4, 4, 0), (260, 4, 0), (2048, 256, 0), (1023, 1023, 0), (1024, 2, 0), (1024, 1024, 1)])
 @pytest.mark.parametrize("act", ["silu", "gelu_tanh", "relu2", "clamped", "gelu"])
 def test_glu_widths(F, group, off, act):
