@@ -622,11 +622,22 @@ def _large_plan(M: int, N_: int, K: int, qtype: int, can_split: bool):
     over the tiles whose ring fits the LDS for the format, rounds = workgroups / 256 with a last round that is r full
     counted as 0.6 + 0.4 r (a half-empty chip clocks and feeds its tiles faster). The constants are a fit to 13 shapes
     (1024 x 4096 .. 57344 x 8192) at 12 row counts 528 .. 8191: the plan picked is within 1 % of the best of 40 candidates
-    on average (18 % at worst), where one 128 x 128 tile for every shape was 16 % off (76 %). Wide tiles (256 columns)
+    on average (18 % at worst), where one 128 x 128 tile for every shape was 16 % off (76 %). That tile stays where the estimate
+    for another is not 7 % lower, which is what the estimate can be off by (1536 x 8960 at 1024 rows, Q4_K: 64-row tiles estimated at
+    48 us took 52.7, this one 45.8; of the fitted shapes none is left slower than with it). Wide tiles (256 columns)
     win where there are rounds enough: gate|up 28672 x 4096 at 8191 rows 2182 -> 1733 us (1.11 PFLOP/s), 1024 276 -> 252;
     narrow outputs take 64-row tiles: 1024 x 4096 at 1024 rows 31 -> 22 us."""
     qb, hb = _STAGE_BYTES[qtype]
-    best = None
+
+    def cost(wm, ks, wn, c, s):
+        bm, ng = 32 * wm * wn, 8 if ks == 17 else 4
+        full, rem = divmod(-(-M // bm) * -(-N_ // (32 * ng)) * s, CU_COUNT)
+        rounds = full + (0.6 + 0.4 * rem / CU_COUNT if rem else 0.0)
+        t = 6.6 + rounds * bm * 32 * ng * 256 * -(-(K // 256) // s) * c * 1e-6
+        return t + 2.4e-6 * M * N_ * s if s > 1 else t
+    square = next(t for t in _LARGE_TILES if t[:3] == (4, 2, 1))
+    splits = 1 if N_ < 16384 and K < 8192 else _split_for(-(-M // 128) * -(-N_ // 128), K, can_split)
+    best = (0.93 * cost(*square, splits), ("q2", 4, 2, 1, splits))
     for wm, ks, wn, c in _LARGE_TILES:
         bm, ng = 32 * wm * wn, 8 if ks == 17 else 4
         if 4 * (bm * 128 + ng * qb) + 2 * ng * hb > 160 * 1024:
@@ -634,13 +645,8 @@ def _large_plan(M: int, N_: int, K: int, qtype: int, can_split: bool):
         for s in (1, 2, 4) if can_split else (1,):
             if s > 1 and (K // 256) // s < 2:
                 continue
-            wgs = -(-M // bm) * -(-N_ // (32 * ng)) * s
-            full, rem = divmod(wgs, CU_COUNT)
-            rounds = full + (0.6 + 0.4 * rem / CU_COUNT if rem else 0.0)
-            t = 6.6 + rounds * bm * 32 * ng * 256 * -(-(K // 256) // s) * c * 1e-6
-            if s > 1:
-                t += 2.4e-6 * M * N_ * s
-            if best is None or t < best[0]:
+            t = cost(wm, ks, wn, c, s)
+            if t < best[0]:
                 best = (t, ("q2", wm, ks, wn, s))
     return best[1]
 

@@ -44,3 +44,9 @@ def test_large_plan_product(qt, M, n):
     y = want.view(M, -1, 2, 16)
     g = (torch.nn.functional.silu(y[:, :, 0]) * y[:, :, 1]).reshape(M, -1)
     assert float((act.cpu().double() - g).norm() / g.norm()) < 4 * 2 ** -10
+
+
+def test_square_tile_stays_where_the_estimate_is_too_close():
+    pick = lambda m, n, k: L._gemm_pick(m, n, k, int(QType.Q4_K), True)  # noqa: E731
+    assert pick(1024, 1536, 8960) == ("q2", 4, 2, 1, 2) and pick(520, 1536, 8960) == ("q2", 4, 2, 1, 4)
+    assert pick(8191, 28672, 4096)[1:4] == (6, 17, 1) and pick(1024, 1024, 4096)[1:4] == (2, 2, 1)
