@@ -46,7 +46,59 @@ def test_large_plan_product(qt, M, n):
     assert float((act.cpu().double() - g).norm() / g.norm()) < 4 * 2 ** -10
 
 
+def test_real_shapes_pick_every_tile():
+    """What the products below force is what shapes of models ask for."""
+    shapes = ((1024, 4096), (4096, 4096), (6144, 4096), (28672, 4096), (4096, 14336), (1536, 8960), (14336, 8192), (57344, 8192))
+    picks = {L._gemm_pick(m, n, k, int(QType.Q4_K), split) for m in range(513, 8192, 113) for n, k in shapes for split in (False, True)}
+    assert {p[1:4] for p in picks} == {t[:3] for t in L._LARGE_TILES} and {p[4] for p in picks} >= {1, 2, 4}
+
+
 def test_square_tile_stays_where_the_estimate_is_too_close():
     pick = lambda m, n, k: L._gemm_pick(m, n, k, int(QType.Q4_K), True)  # noqa: E731
     assert pick(1024, 1536, 8960) == ("q2", 4, 2, 1, 2) and pick(520, 1536, 8960) == ("q2", 4, 2, 1, 4)
     assert pick(8191, 28672, 4096)[1:4] == (6, 17, 1) and pick(1024, 1024, 4096)[1:4] == (2, 2, 1)
+
+
+_WEIGHTS = {}
+
+
+def _weight(qt, n, k):
+    """(weight on the GPU, its numbers) of a format; Q4_0 / Q5_0 / Q5_1 files load as MX4F / MX5F."""
+    import numpy as np
+    if qt not in _WEIGHTS:
+        raw = Q.random_quantized(np.random.default_rng(n), int(qt), n, k).reshape(n, -1)
+        W = L.QWeight.from_ggml(raw, int(qt), n, k, "cuda", t32=True)
+        assert W.to_t32() and int(W.qtype) in L._STAGE_BYTES
+        _WEIGHTS[qt] = W, torch.from_numpy(Q.dequantize(raw.reshape(-1), int(qt), (k, n)).reshape(n, k).copy())
+    return _WEIGHTS[qt]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("qt", [*QTYPES, QType.Q4_0, QType.Q5_0, QType.Q5_1])
+@pytest.mark.parametrize("tile", [t[:3] for t in L._LARGE_TILES])
+def test_every_tile_in_bands(qt, tile):
+    """Each tile the plans choose from, on five and six row tiles (a band of four and a partial one, its last tile part empty), two
+    column panels of which the second is part empty, whole K and two and three parts of it."""
+    n, k = 288, 1536
+    W, dense = _weight(qt, n, k)
+    wm, ks, wn = tile
+    bm, ng = 32 * wm * wn, 8 if ks == 17 else 4
+    qb, hb = L._STAGE_BYTES[int(W.qtype)]
+    if 4 * (bm * 128 + ng * qb) + 2 * ng * hb > 160 * 1024:
+        pytest.skip("this tile's ring does not fit the LDS for the format (never chosen)")
+    for M in (4 * bm + 33, 6 * bm - 1):
+        x = (torch.randn(M, k, generator=torch.Generator().manual_seed(M)) * 0.5).half()
+        want = x.double() @ dense.double().t()
+        base = torch.randn(M, n, generator=torch.Generator().manual_seed(1))
+        for splits in (1, 2, 4):  # (six super-blocks: 4 asks for three parts of two)
+            out = torch.zeros(M, n, device="cuda")
+            L.run_plan(("q2", *tile, splits), W, x.cuda(), L.EPI_F32, out, True)
+            assert float((out.cpu().double() - want).norm() / want.norm()) < 2 ** -10  # weights rounded to f16 once (2^-11)
+            out = base.cuda()
+            L.run_plan(("q2", *tile, splits), W, x.cuda(), L.EPI_ADD_F32, out, False)
+            assert float((out.cpu().double() - base - want).norm() / want.norm()) < 2 ** -10
+        act = torch.zeros(M, n // 2, device="cuda", dtype=torch.float16)
+        L.run_plan(("q2", *tile, 1), W, x.cuda(), L.EPI_SWIGLU, act, False)
+        y = want.view(M, -1, 2, 16)
+        g = (torch.nn.functional.silu(y[:, :, 0]) * y[:, :, 1]).reshape(M, -1)
+        assert float((act.cpu().double() - g).norm() / g.norm()) < 4 * 2 ** -10
