@@ -22,22 +22,16 @@
 
 #define LOG2E_D 1.4426950408889634f
 
-// K image: row p holds D/8 16-byte chunks; chunk c lives at c ^ f(p) (f < 16: 16 consecutive rows, one chunk
-// column, land in 16 different banks). D = 512 uses the D = 128 swizzle (its rows are 4 x as wide, same banking).
+// Head dim 512. K image: row p holds D/8 16-byte chunks; chunk c lives at c ^ f(p) (f < 16: 16 consecutive rows, one chunk
+// column, land in 16 different banks).
 template <int D>
 MX_DEV int kd_lds_off(int p, int c) {
     const int r = p & 15;
-    int f;
-    if constexpr (D >= 128) f = r ^ (((r + 4) >> 3) & 1);
-    else f = ((r >> 1) & 7) ^ (((r + 4) >> 3) & 1);
-    return p * (D * 2) + ((c ^ (f & (D / 8 - 1))) << 4);
+    return p * (D * 2) + ((c ^ r ^ (((r + 4) >> 3) & 1)) << 4);
 }
 template <int D>
 MX_DEV int vd_lds_off(int p, int nt) {
-    int sv;
-    if constexpr (D >= 128) sv = (p & 3) | (((p >> 3) & 1) << 2);
-    else sv = ((p >> 1) & 1) | (((p >> 3) & 1) << 1);
-    return p * (D * 2) + ((nt ^ sv) << 5);
+    return p * (D * 2) + ((nt ^ ((p & 3) | (((p >> 3) & 1) << 2))) << 5);
 }
 
 template <bool F16>
@@ -58,8 +52,8 @@ __global__ __launch_bounds__(256) void attn_dense_kernel(const uint16_t* __restr
                                                          int Hq, int Hkv, const int* __restrict__ qlen_b,
                                                          const int* __restrict__ klen_b, int causal, float scale,
                                                          int kv_rows, const float* __restrict__ rbias, int rb_ld) {
-    // key tile: 64 keys (D <= 128) or 32 (D = 512: the VAE mid-block's single 512-wide head; K + V tiles 64 KB)
-    constexpr int KT = D > 128 ? 32 : 64;
+    static_assert(D == 512, "smaller head dims: attn_dense_t_kernel");
+    constexpr int KT = 32;  // keys per tile (the VAE mid-block's single 512-wide head; K + V tiles 64 KB)
     constexpr int KBYTES = KT * D * 2;
     constexpr int PSTRIDE = (KT + 8) * 2;
     __shared__ __attribute__((aligned(16))) char smem[2 * KBYTES + 4 * 16 * PSTRIDE];
@@ -97,8 +91,7 @@ __global__ __launch_bounds__(256) void attn_dense_kernel(const uint16_t* __restr
     for (int i = 0; i < 4; ++i) { mrow[i] = -INFINITY; lrow[i] = 0.f; }
     char* pw = smem + 2 * KBYTES + wave * 16 * PSTRIDE;
 
-    // K / V tiles software-pipelined one tile deep: the next tile's 16-byte chunks are requested right after
-    // this tile is staged in LDS, so their latency hides behind this tile's MFMAs and softmax
+    // (a tile is 8 chunks per thread and per operand: asking for the next one ahead would spill, so each loads in place)
     constexpr int CH = KT * D / 8;
     constexpr int NCH = (CH + 255) / 256;  // chunks per thread
     uint4 kr[NCH], vr[NCH];
@@ -116,11 +109,8 @@ __global__ __launch_bounds__(256) void attn_dense_kernel(const uint16_t* __restr
             }
         }
     };
-    // (D = 512: a tile is 8 chunks per thread and per operand; prefetching it would spill, so it loads in place)
-    constexpr bool PF = D <= 128;
-    if (PF && kv_end > 0) load_tile(0);
     for (int kt0 = 0; kt0 < kv_end; kt0 += KT) {
-        if constexpr (!PF) load_tile(kt0);
+        load_tile(kt0);
 #pragma unroll
         for (int j = 0; j < NCH; ++j) {
             const int id = threadIdx.x + 256 * j;
@@ -129,7 +119,6 @@ __global__ __launch_bounds__(256) void attn_dense_kernel(const uint16_t* __restr
             *(uint4*)(k_lds + kd_lds_off<D>(p, c)) = kr[j];
             *(uint4*)(v_lds + vd_lds_off<D>(p, c >> 1) + 16 * (c & 1)) = vr[j];
         }
-        if (PF && kt0 + KT < kv_end) load_tile(kt0 + KT);
         __syncthreads();
         constexpr int NT16 = KT / 16;
         f32x4 sacc[NT16];
