@@ -10,9 +10,9 @@
 //   loads, so a wave streams 64*16 B of K (then V) per step; all G = Hq/Hkv query heads of the kv
 //   head are scored from the same K/V bytes (GQA packing: K/V are read once per kv head, not per q
 //   head). Online softmax in the log2 domain; partitions merge in attn_decode_reduce.
-// prefill (varlen, causal, paged context incl. cached prefix): attention_flash.hip; here the form for head dim
-//   256 (and the V^T image): flash-attention forward on MFMA 16x16x32 bf16. A workgroup holds 16 query rows x up to 8 query heads of one kv head (one wave per
-//   head) so every K/V tile staged in LDS is reused by all heads of the group. K is stored
+// prefill (varlen, causal, paged context incl. cached prefix): attention_flash.hip; here the form for head dim 256 and for
+//   contexts of one key tile (ops/core.py flash_plan): flash-attention forward on MFMA 16x16x32 bf16. A workgroup holds 16 query
+//   rows x up to 8 query heads of one kv head (one wave per head) so every K/V tile staged in LDS is reused by all heads of the group. K is stored
 //   XOR-swizzled for conflict-free ds_read_b128 B-fragments; V is read with ds_read_b64_tr_b16
 //   (hardware transpose) from a region-swizzled image; P goes register -> LDS -> A-fragment.
 #include <type_traits>

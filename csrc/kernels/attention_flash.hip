@@ -1,5 +1,5 @@
 // attention_flash.hip: prompt attention over the paged cache on 32x32x16 MFMA (bf16, fp8 and block-quantised caches),
-// head dims 64 and 128: what mxk_attn_prefill runs except for head dim 256 and the V^T image (attention.hip).
+// head dims 64 and 128, except for contexts of one key tile where attention.hip is the faster (ops/core.py flash_plan).
 //
 // A workgroup owns one KV head, RQ consecutive queries of one sequence and a range of key tiles. Its G query heads are
 // packed with the queries into 32-column groups, column = query * G + head: whatever G is, a wave holds 32 of them and
@@ -15,11 +15,12 @@
 // fp8 and block formats are widened to bf16) and are stored to the other buffer, one barrier per tile.
 //
 // A short chunk behind a long context has too few workgroups (7 x 8 for 416 rows of a 32 / 8-head model), so the key
-// range is split over grid.z: every part has at least MIN_TILES tiles, writes (m, l, O) unnormalised in fp32, and
-// attn_flash_merge_kernel combines them; a block of queries that only one part has keys for is finished by that part.
+// range is split over grid.z: parts of MIN_TILES tiles or more, the last one of what is left (17 tiles: 16 + 1), write (m, l, O)
+// unnormalised in fp32 and attn_flash_merge_kernel combines them; a block of queries that only one part has keys for is
+// finished by that part.
 //
 // Measured, 32 / 8 heads of 128, against the 16-row kernel this replaced (which read each K / V fragment for one 16x16x32
-// product and moved P through LDS): an 8191-token prompt 2400 -> 630 us (873 TFLOP/s), 2048 233 -> 65, 333 18.5 -> 15.5;
+// product and moved P through LDS): an 8191-token prompt 2400 -> 600 us (917 TFLOP/s), 2048 233 -> 65, 333 18.5 -> 14.0;
 // 416 rows behind 12000 keys 498 -> 140 us in bf16, 788 -> 140 in fp8. Heads of 64, 8191 rows: 1253 -> 360 us. Bound by
 // the vector unit beside the matrix unit (32 exponentials and ~100 other vector operations a lane and tile against 32
 // products); short prompts by the chain of one tile (~1.3 us) times their tiles.
@@ -32,7 +33,7 @@
 namespace {
 
 constexpr int FT = 64;        // keys per tile
-constexpr int MIN_TILES = 16;  // fewest key tiles a part is made for
+constexpr int MIN_TILES = 16;  // fewest key tiles of a part that is not a block's last
 
 template <int D>
 MX_DEV int fk_off(int p, int c) {  // K image: byte offset of 16-byte chunk c of row p

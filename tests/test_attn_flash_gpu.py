@@ -111,8 +111,10 @@ def test_which_sequence_a_block_belongs_to(n, monkeypatch):
 @pytest.mark.parametrize("waves,parts", [(4, 1), (8, 1), (4, 2), (8, 3), (4, 16)])
 @pytest.mark.parametrize("D", [64, 128])
 def test_key_parts(waves, parts, D, monkeypatch):
-    """Sequences that one part finishes beside others that several share (parts hold at least 16 tiles of 64 keys)."""
+    """Sequences that one part finishes beside others that several share (parts hold 16 tiles of 64 keys, the last one what is left);
+    contexts of 16 and 17 tiles."""
     _check(8, 2, D, [70, 5, 40], [1100, 0, 3000], plan=(waves, parts), monkeypatch=monkeypatch)
+    _check(8, 2, D, [24, 24, 24], [1000, 1001, 1064], plan=(waves, parts), monkeypatch=monkeypatch)
 
 
 @pytest.mark.gpu
