@@ -18,7 +18,7 @@
 // Masks: `causal` (key position > query position + (Sk - Sq) dropped) and per-batch key lengths
 // `klen` (BERT padding); rows past `qlen[b]` are not written. Optional additive relative-position bias
 // `rbias[h][j - i + Sq - 1]` (fp32, T5's bucketed bias table expanded per offset; shared by the batch).
-#include "mx_common.h"
+#include "attn_tile.h"
 
 #define LOG2E_D 1.4426950408889634f
 
@@ -204,33 +204,6 @@ __global__ __launch_bounds__(256) void attn_dense_kernel(const uint16_t* __restr
 }
 
 // ---- head dims 64 / 128 ----
-template <bool F16>
-MX_DEV f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
-    if constexpr (F16)
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-// 64-key images: K chunk c (16 bytes) of row p, V region r (32 bytes) of row p; both reads are free of bank conflicts
-template <int D>
-MX_DEV int kt_off(int p, int c) {
-    const int f = D == 128 ? (p & 15) : ((p >> 1) & 7);
-    return p * (2 * D) + ((c ^ f) << 4);
-}
-template <int D>
-MX_DEV int vt_off(int p, int r) {
-    const int f = D == 128 ? (p & 7) : ((p >> 1) & 3);
-    return p * (2 * D) + ((r ^ f) << 5);
-}
-MX_DEV float halves_max(float x) {  // over the two half-waves' values of a column, in both
-    const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false));
-    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-MX_DEV float halves_sum(float x) {
-    const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false));
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
 // GEN: a position bias, or a scale that is not positive; without it the scale is one FMA with the maximum
 template <int D, int NW, bool F16, bool GEN>
 __global__ __launch_bounds__(64 * NW, 2) void attn_dense_t_kernel(const uint16_t* __restrict__ q, int q_stride,
@@ -241,7 +214,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dense_t_kernel(const uint16_t
                                                               const int* __restrict__ klen_b, int causal, float scale,
                                                               int kv_rows, const float* __restrict__ rbias, int rb_ld,
                                                               const int* __restrict__ cu) {
-    constexpr int FT = 64, IMG = FT * D * 2;
+    constexpr int FT = AT_KEYS, IMG = FT * D * 2;
     constexpr int NCH = FT * D / 8 / (64 * NW);  // 16-byte chunks of an image per thread
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -292,56 +265,22 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dense_t_kernel(const uint16_t
 #pragma unroll
         for (int j = 0; j < NCH; ++j) {
             const int id = threadIdx.x + 64 * NW * j, p = id / (D / 8), c = id % (D / 8);
-            *(u32x4*)(kb + kt_off<D>(p, c)) = kr[j];
-            *(u32x4*)(kb + IMG + vt_off<D>(p, c >> 1) + 16 * (c & 1)) = vr[j];
+            *(u32x4*)(kb + at_k_off<D>(p, c)) = kr[j];
+            *(u32x4*)(kb + IMG + at_v_off<D>(p, c >> 1) + 16 * (c & 1)) = vr[j];
         }
     };
-    const int i16 = lane & 15, dh = (lane >> 4) & 1;
+    int vo[D / 32];
+    at_v_lane<D>(lane, vo);
     auto work = [&](int t) {
         const char* kb = smem + (t & 1) * (2 * IMG);
         const char* vb = kb + IMG;
         const int kt0 = t * FT;
         f32x16 sc[2];
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int j = 0; j < 16; ++j) sc[u][j] = 0.f;
-        // the fences keep the fragment reads ahead of the products that wait for them
-        constexpr int KB = 2;
-        u32x4 kf[D / 16][2];
-        auto read_k = [&](int k0) {
-#pragma unroll
-            for (int ks = k0; ks < k0 + KB; ++ks)
-#pragma unroll
-                for (int u = 0; u < 2; ++u) kf[ks][u] = *(const u32x4*)(kb + kt_off<D>(32 * u + col, 2 * ks + h));
-        };
-        read_k(0);
-#pragma unroll
-        for (int k0 = 0; k0 < D / 16; k0 += KB) {
-            __builtin_amdgcn_sched_barrier(0);
-            if (k0 + KB < D / 16) read_k(k0 + KB);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int ks = k0; ks < k0 + KB; ++ks)
-#pragma unroll
-                for (int u = 0; u < 2; ++u) sc[u] = mfma32<F16>(kf[ks][u], qf[ks], sc[u]);
-        }
+        at_scores<D, F16, 2>(kb, h, col, qf, sc);
         u32x4 vf[4][D / 32];
-        auto read_v = [&](int ks) {
-            const int row = 16 * ks + 4 * h + (i16 >> 2);
-#pragma unroll
-            for (int mt = 0; mt < D / 32; ++mt) {
-                const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                    (MX_LDS s16x4*)(vb + vt_off<D>(row, 2 * mt + dh) + 8 * (i16 & 3))));
-                const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                    (MX_LDS s16x4*)(vb + vt_off<D>(row + 8, 2 * mt + dh) + 8 * (i16 & 3))));
-                vf[ks][mt] = (u32x4){lo[0], lo[1], hi[0], hi[1]};
-            }
-        };
         __builtin_amdgcn_sched_barrier(0);
-        read_v(0);
+        at_read_v<D>(vb, vo, 0, vf);
         __builtin_amdgcn_sched_barrier(0);
-        const float mul = GEN ? 1.f : qs;
         if constexpr (GEN) {
 #pragma unroll
             for (int u = 0; u < 2; ++u)
@@ -360,42 +299,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dense_t_kernel(const uint16_t
                 for (int j = 0; j < 16; ++j)
                     if (32 * u + 8 * (j >> 2) + (j & 3) > d) sc[u][j] = -INFINITY;
         }
-        float mx[2] = {sc[0][0], sc[1][0]};  // (med3 with infinity: the maximum without the quieting of its inputs)
-#pragma unroll
-        for (int j = 1; j < 16; ++j)
-#pragma unroll
-            for (int u = 0; u < 2; ++u) mx[u] = __builtin_amdgcn_fmed3f(mx[u], sc[u][j], INFINITY);
-        const float m_new = fmaxf(m_run, halves_max(fmaxf(mx[0], mx[1])) * mul);
-        if (__any(m_new > m_run)) {
-            const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);
-            l_run *= alpha;
-#pragma unroll
-            for (int i = 0; i < D / 32; ++i)
-#pragma unroll
-                for (int j = 0; j < 16; ++j) acc[i][j] *= alpha;
-            m_run = m_new;
-        }
-        const float m_use = m_run == -INFINITY ? 0.f : m_run;
-        float ls[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            const int u = ks >> 1, j0 = 8 * (ks & 1);
-            if (ks < 3) read_v(ks + 1);
-            uint32_t pw[4];
-#pragma unroll
-            for (int j = 0; j < 8; j += 2) {
-                const float p0 = __builtin_amdgcn_exp2f(fmaf(sc[u][j0 + j], mul, -m_use));
-                const float p1 = __builtin_amdgcn_exp2f(fmaf(sc[u][j0 + j + 1], mul, -m_use));
-                ls[j & 2] += p0;
-                ls[(j & 2) + 1] += p1;
-                pw[j >> 1] = pack_act2<F16>(p0, p1);
-            }
-            const u32x4 pf = (u32x4){pw[0], pw[1], pw[2], pw[3]};
-#pragma unroll
-            for (int mt = 0; mt < D / 32; ++mt) acc[mt] = mfma32<F16>(vf[ks][mt], pf, acc[mt]);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        l_run += (ls[0] + ls[1]) + (ls[2] + ls[3]);
+        at_softmax_v<D, F16>(vb, vo, sc, GEN ? 1.f : qs, vf, acc, m_run, l_run);
     };
     if (n_tiles > 0) {
         load_rows(0);
@@ -417,7 +321,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dense_t_kernel(const uint16_t
             __syncthreads();
         }
     }
-    l_run = halves_sum(l_run);
+    l_run = at_half_sum(l_run);
     if (!real) return;
     const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
     uint16_t* op = o + (q_row + qi) * o_stride + (size_t)head * D + 4 * h;

@@ -3,14 +3,11 @@
 //
 // A workgroup owns one KV head, RQ consecutive queries of one sequence and a range of key tiles. Its G query heads are
 // packed with the queries into 32-column groups, column = query * G + head: whatever G is, a wave holds 32 of them and
-// every K / V tile in LDS serves them all. The scores are computed transposed, S^T = K Q^T, so that a column is one
-// lane's (two half-waves hold the even and odd 4-key groups): maximum, sum and rescaling are lane-local but for one
-// exchange between the half-waves per tile, and the probabilities are already where the B operand of O^T = V^T P^T wants
-// them when V^T's keys are taken in the same order (S^T's C layout gives a lane keys 8 j + 4 h + i; both operands' k slot
-// (h, e) then means key 8 (e / 4) + 4 h + e % 4 of the 16). Nothing goes through LDS but K and V.
+// every K / V tile in LDS serves them all. The scores are computed transposed (attn_tile.h), so that a column is one lane's (two
+// half-waves hold the even and odd 4-key groups): maximum, sum and rescaling are lane-local but for one exchange between the
+// half-waves per tile, and the probabilities are already where the next product's B operand wants them. Nothing goes through LDS
+// but K and V.
 //
-// K image: row p, 16-byte chunk c at c ^ row bits, read as A fragments (ds_read_b128, 32 rows x 1 chunk a half-wave);
-// V image: row p, 32-byte region r at r ^ row bits, read with ds_read_b64_tr_b16 (4 keys of a dim per lane).
 // Tiles of 64 keys are double-buffered: a tile's 16-byte chunks are requested one tile ahead, wait in registers (where
 // fp8 and block formats are widened to bf16) and are stored to the other buffer, one barrier per tile.
 //
@@ -26,34 +23,15 @@
 // products); short prompts by the chain of one tile (~1.3 us) times their tiles.
 #include <type_traits>
 
+#include "attn_tile.h"
 #include "kvq.h"
 
 #define LOG2E 1.4426950408889634f
 
 namespace {
 
-constexpr int FT = 64;        // keys per tile
+constexpr int FT = AT_KEYS;
 constexpr int MIN_TILES = 16;  // fewest key tiles of a part that is not a block's last
-
-template <int D>
-MX_DEV int fk_off(int p, int c) {  // K image: byte offset of 16-byte chunk c of row p
-    const int f = D == 128 ? (p & 15) : ((p >> 1) & 7);
-    return p * (2 * D) + ((c ^ f) << 4);
-}
-template <int D>
-MX_DEV int fv_off(int p, int r) {  // V image: byte offset of 32-byte region r (16 dims) of row p
-    const int f = D == 128 ? (p & 7) : ((p >> 1) & 3);
-    return p * (2 * D) + ((r ^ f) << 5);
-}
-
-MX_DEV float half_max(float x) {  // max of the two half-waves' values of a column, in both
-    const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false));
-    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-MX_DEV float half_sum(float x) {
-    const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false));
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
 
 // c tanh(v / c) for c = softcap * log2(e), k = 2 / softcap: (1 - e) / (1 + e) with e = exp2(-k |v|). tanhf took half of a capped
 // prompt's time (416 rows behind 100 tokens, 32 / 8 heads of 128: 35.4 us).
@@ -151,11 +129,11 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_flash_kernel(co
     const int t0 = part * per, t1 = min(n_tiles, t0 + per);
 
     // Q^T as B operand: lane = column, 8 dims 16 ks + 8 h (columns past the end repeat a real one, never stored)
-    bf16x8 qf[D / 16];
+    u32x4 qf[D / 16];
     {
         const bf16_t* qp = q + ((size_t)(qbeg + min(qi, qlen - 1)) * Hq + kvh * G + r % G) * D + 8 * h;
 #pragma unroll
-        for (int ks = 0; ks < D / 16; ++ks) qf[ks] = *(const bf16x8*)(qp + 16 * ks);
+        for (int ks = 0; ks < D / 16; ++ks) qf[ks] = *(const u32x4*)(qp + 16 * ks);
     }
     f32x16 o[D / 32];
 #pragma unroll
@@ -206,60 +184,24 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_flash_kernel(co
         for (int j = 0; j < NCH; ++j) {
             const int id = threadIdx.x + j * NT;
             const int p = id / (D / 8), c = id % (D / 8);
-            *(uint4*)(kb + fk_off<D>(p, c)) = f_widen<KVF>(kr[j]);
-            *(uint4*)(kb + IMG + fv_off<D>(p, c >> 1) + 16 * (c & 1)) = f_widen<KVF>(vr[j]);
+            *(uint4*)(kb + at_k_off<D>(p, c)) = f_widen<KVF>(kr[j]);
+            *(uint4*)(kb + IMG + at_v_off<D>(p, c >> 1) + 16 * (c & 1)) = f_widen<KVF>(vr[j]);
         }
     };
-    const int i16 = lane & 15, dh = (lane >> 4) & 1;
-    // The fences keep the fragment reads ahead of what they wait behind: K's before the first product, V's first before the
-    // softmax, its others one k-step ahead of their products (left alone, the scheduler puts every read next to its use).
+    constexpr int KB = NW == 8 ? D / 32 : D / 64;  // K fragments read together (a thread of 4 waves holds twice as much staged)
+    int vo[D / 32];
+    at_v_lane<D>(lane, vo);
     auto work = [&](int t) {
         const char* kb = smem + (t & 1) * (2 * IMG);
         const char* vb = kb + IMG;
         const int kt0 = kt_begin + t * FT;
         f32x16 sc[2];
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int j = 0; j < 16; ++j) sc[u][j] = 0.f;
-        bf16x8 kf[D / 16][2];
-        constexpr int KB = NW == 8 ? D / 32 : D / 64;  // k-steps read together (registers: a thread of 4 waves stages twice as much)
-        auto read_k = [&](int k0) {
-#pragma unroll
-            for (int ks = k0; ks < k0 + KB; ++ks)
-#pragma unroll
-                for (int u = 0; u < 2; ++u) kf[ks][u] = *(const bf16x8*)(kb + fk_off<D>(32 * u + col, 2 * ks + h));
-        };
-        read_k(0);
-#pragma unroll
-        for (int k0 = 0; k0 < D / 16; k0 += KB) {
-            __builtin_amdgcn_sched_barrier(0);
-            if (k0 + KB < D / 16) read_k(k0 + KB);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int ks = k0; ks < k0 + KB; ++ks)
-#pragma unroll
-                for (int u = 0; u < 2; ++u) sc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ks][u], qf[ks], sc[u], 0, 0, 0);
-        }
-        bf16x8 vf[4][D / 32];
-        auto read_v = [&](int ks) {
-            const int row = 16 * ks + 4 * h + (i16 >> 2);
-#pragma unroll
-            for (int mt = 0; mt < D / 32; ++mt) {
-                const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                    (MX_LDS s16x4*)(vb + fv_off<D>(row, 2 * mt + dh) + 8 * (i16 & 3))));
-                const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                    (MX_LDS s16x4*)(vb + fv_off<D>(row + 8, 2 * mt + dh) + 8 * (i16 & 3))));
-                const u32x4 w4 = {lo[0], lo[1], hi[0], hi[1]};
-                vf[ks][mt] = __builtin_bit_cast(bf16x8, w4);
-            }
-        };
+        at_scores<D, false, KB>(kb, h, col, qf, sc);
+        u32x4 vf[4][D / 32];
         __builtin_amdgcn_sched_barrier(0);
-        read_v(0);
+        at_read_v<D>(vb, vo, 0, vf);
         __builtin_amdgcn_sched_barrier(0);
-        float mul = qs;
         if constexpr (GEN) {
-            mul = 1.f;
 #pragma unroll
             for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -278,43 +220,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_flash_kernel(co
                     if (kp > d || (GEN && window > 0 && kp <= d - window)) sc[u][j] = -INFINITY;
                 }
         }
-        // (med3 with infinity is the maximum without the quieting of its inputs that fmaxf asks for)
-        float mx[2] = {sc[0][0], sc[1][0]};
-#pragma unroll
-        for (int j = 1; j < 16; ++j)
-#pragma unroll
-            for (int u = 0; u < 2; ++u) mx[u] = __builtin_amdgcn_fmed3f(mx[u], sc[u][j], INFINITY);
-        const float m_new = fmaxf(m_run, half_max(fmaxf(mx[0], mx[1])) * mul);
-        if (__any(m_new > m_run)) {
-            const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);
-            l_run *= alpha;
-#pragma unroll
-            for (int i = 0; i < D / 32; ++i)
-#pragma unroll
-                for (int j = 0; j < 16; ++j) o[i][j] *= alpha;
-            m_run = m_new;
-        }
-        const float m_use = m_run == -INFINITY ? 0.f : m_run;
-        float ls[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            const int u = ks >> 1, j0 = 8 * (ks & 1);
-            if (ks < 3) read_v(ks + 1);
-            u32x4 pw;
-#pragma unroll
-            for (int j = 0; j < 8; j += 2) {
-                const float p0 = __builtin_amdgcn_exp2f(fmaf(sc[u][j0 + j], mul, -m_use));
-                const float p1 = __builtin_amdgcn_exp2f(fmaf(sc[u][j0 + j + 1], mul, -m_use));
-                ls[j & 2] += p0;
-                ls[(j & 2) + 1] += p1;
-                pw[j >> 1] = pack_bf16x2(p0, p1);
-            }
-            const bf16x8 pf = __builtin_bit_cast(bf16x8, pw);
-#pragma unroll
-            for (int mt = 0; mt < D / 32; ++mt) o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[ks][mt], pf, o[mt], 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        l_run += (ls[0] + ls[1]) + (ls[2] + ls[3]);
+        at_softmax_v<D, false>(vb, vo, sc, GEN ? 1.f : qs, vf, o, m_run, l_run);
     };
 
     if (t0 < t1) {
@@ -341,7 +247,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_flash_kernel(co
             __syncthreads();
         }
     }
-    l_run = half_sum(l_run);
+    l_run = at_half_sum(l_run);
     auto pack2 = [f16](float a, float b) { return f16 ? pack_act2<true>(a, b) : pack_act2<false>(a, b); };
     if (live == 1) {
         if (!real) return;
