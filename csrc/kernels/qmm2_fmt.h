@@ -154,10 +154,11 @@ struct Q2B<MXQ_Q5_K> {
     u32x2 qh0, qh1;  // qh bytes 8 h .. 8 h + 7 of chunks 0 / 1
     u32x2 v0, v1;
     f16x2 sm[2];
-    MX_DEV void load_hdr(const char* hb, int col, int h) {
+    MX_DEV void load_hdr(const char* hb, int col, int h) { load_hdr(hb, hb + 512, col, h); }
+    MX_DEV void load_hdr(const char* hb, const char* qh, int col, int h) {  // qh: the fifth-bit chunks
         hd = *(const u32x4*)(hb + col * 16);
-        qh0 = *(const u32x2*)(hb + 512 + col * 16 + 8 * h);
-        qh1 = *(const u32x2*)(hb + 1024 + col * 16 + 8 * h);
+        qh0 = *(const u32x2*)(qh + col * 16 + 8 * h);
+        qh1 = *(const u32x2*)(qh + 512 + col * 16 + 8 * h);
     }
     MX_DEV void load_q(const char* qb, int col, int h) {
         v0 = *(const u32x2*)(qb + col * 16 + 8 * h);

@@ -6,8 +6,8 @@ badly between its breakpoints (qkv 6144 x 4096: 55 us at M = 384 against 41 us a
 profiles/r5_gemm_curve.md). Instead, every distinct (N, K, block format, epilogue class) of a loaded model is
 timed on the GPU it runs on, for each M bucket the engine produces, over every compiled tile / split
 candidate; the fastest plan per bucket is kept in TUNED and ops/linear.py dispatches from it. A plan is
-("q2", wm, ks, wn, splits) | ("q3", wm, splits) | ("rows", chunk) (row chunks of `chunk`, each dispatched by
-its own bucket). Only kernel choice is tuned: every candidate computes the same product (the GPU tests check
+("q2", wm, ks, wn, splits) | ("q3", wm, splits) | ("qr", wm, gw, kw, splits) | ("rows", chunk) (row chunks of
+`chunk`, each dispatched by its own bucket). Only kernel choice is tuned: every candidate computes the same product (the GPU tests check
 every tile / split / epilogue against the fp32 reference).
 
 Tuning costs ~1-3 s per model (a handful of shapes x buckets x ~40 candidates x ~15 launches); results are
@@ -65,6 +65,11 @@ def candidates(M: int, N: int, K: int, qtype: int, can_split: bool) -> list[tupl
                 continue
             for s in sp:
                 out.append(("q3", wm, s))
+    if M <= L.QMMR_MAX_M:
+        for wm, gw, kw in L.QMMR_CONFIGS:
+            if 32 * wm <= max(32, M):
+                for s in sp:
+                    out.append(("qr", wm, gw, kw, s))
     for c in (128, 256):
         if c < M:
             out.append(("rows", c))

@@ -325,7 +325,8 @@ def row_chunks(M: int, chunk: int | None = None) -> list[tuple[int, int]]:
 
 def run_plan(plan: tuple, W: QWeight, x: torch.Tensor, epi: int, out: torch.Tensor, out_zeroed: bool,
              fuse: "NormFuse | None" = None):
-    """Launch one GEMM plan (ops/autotune.py): ("q3", wm, splits) | ("q2", wm, ks, wn, splits) | ("rows", chunk)."""
+    """Launch one GEMM plan (ops/autotune.py): ("q3", wm, splits) | ("q2", wm, ks, wn, splits) |
+    ("qr", wm, gw, kw, splits) | ("rows", chunk)."""
     M = x.shape[0]
     kind = plan[0]
     if fuse is not None and kind != "q2":
@@ -343,6 +344,9 @@ def run_plan(plan: tuple, W: QWeight, x: torch.Tensor, epi: int, out: torch.Tens
     if kind == "q3":
         N.kcall("mxk_qmm3", int(W.qtype), e, plan[1], x.data_ptr(), x.stride(0), W.data.data_ptr(), M, W.N, W.K,
                 splits, out.data_ptr(), out.stride(0), N.stream_ptr())
+    elif kind == "qr":
+        N.kcall("mxk_qmmr", int(W.qtype), e, plan[1], plan[2], plan[3], x.data_ptr(), x.stride(0), W.data.data_ptr(),
+                M, W.N, W.K, splits, out.data_ptr(), out.stride(0), N.stream_ptr())
     elif kind == "q2" and fuse is not None and fuse.mode & 4:
         f = fuse
         slots, rot, bias, qo, kc, vc, n_off, D, hq, hkv, bsz = f.rope
@@ -593,6 +597,9 @@ if os.environ.get("MX_QMM2_WIDE4", "0") == "1":
 # every t32 block format runs on qmm2 / qmm3 (qmm2_fmt.h decoders)
 QMM2_QTYPES = (int(QType.Q4_K), int(QType.Q6_K), int(QType.Q3_K), int(QType.Q2_K), int(QType.Q5_K), int(QType.Q8_0),
                int(QType.MX4F), int(QType.MX5F))
+# qmmr.hip (wm, gw, kw): 32 wm rows x 32 gw columns a workgroup, kw waves over each super-block of K
+QMMR_CONFIGS = ((1, 4, 4), (1, 2, 4), (1, 1, 4), (1, 4, 2), (1, 2, 2), (2, 2, 4), (2, 4, 2))
+QMMR_MAX_M = 192  # rows up to which the tuner times them (weights are decoded once per row tile)
 QMM2_MIN_M = int(os.environ.get("MX_QMM2_MIN_M", "16"))
 
 
@@ -652,7 +659,7 @@ def _large_plan(M: int, N_: int, K: int, qtype: int, can_split: bool):
 
 
 def _gemm_pick(M: int, N_: int, K: int, qtype: int, can_split: bool):
-    """Untuned fallback plan ("q3", wm, splits) | ("q2", wm, ks, wn, splits) for a t32 GEMM — shapes the load-time
+    """Untuned fallback plan (run_plan) for a t32 GEMM — shapes the load-time
     autotuner (ops/autotune.py) did not time. The rule follows the tuned Llama-3-8B table
     (profiles/r5_gemm_autotune.md): 64-row 8-wave qmm2 tiles for the narrow projections, 128-row tiles for the
     wide ones, qmm3 for the gated FFN at 129-256 rows."""
@@ -664,6 +671,8 @@ def _gemm_pick(M: int, N_: int, K: int, qtype: int, can_split: bool):
         return _large_plan(M, N_, K, qtype, can_split)
     nct = -(-N_ // 128)
     wide = N_ >= 16384
+    if M <= 32:  # qmmr from its table (qmmr.hip): 128 columns a workgroup where they fill the chip, else 64 and K splits
+        return ("qr", 1, 4, 4, 1) if wide else ("qr", 1, 2, 4, _split_for(-(-N_ // 64), K, can_split))
     if M <= 64 or (not wide and K < 8192 and M <= 256):
         return ("q2", 2, 2, 1, _split_for(-(-M // 64) * nct, K, can_split))
     if wide and 128 < M <= 256:

@@ -494,6 +494,38 @@ def test_qmm3(qt, M, wm, splits, monkeypatch):
     assert rel(sw, ref_sw) < 1e-2
 
 
+@pytest.mark.parametrize("qt", [QType.Q4_K, QType.Q6_K, QType.Q3_K, QType.Q2_K, QType.Q5_K, QType.Q8_0, QType.Q4_0, QType.Q5_0])
+@pytest.mark.parametrize("M,wm,gw,kw,splits", [
+    (1, 1, 4, 4, 1), (32, 1, 4, 4, 9), (33, 1, 2, 4, 2), (9, 1, 1, 4, 5), (70, 1, 4, 2, 3), (31, 1, 2, 2, 4),
+    (64, 2, 2, 4, 1), (129, 2, 4, 2, 2)])
+def test_qmmr(qt, M, wm, gw, kw, splits):
+    """qmmr.hip (weights in registers) for every format and epilogue: ragged rows and columns (416 = 13 groups), splits of
+    one to nine super-blocks (odd and even: the two register sets), against the fp32 product of the dequantised weight."""
+    from localai_tfp_amd.ops import linear as L
+    n, k = 416, 2304
+    raw, dense = make_w(qt, n, k, seed=M + 7 * wm)
+    W = QWeight.from_ggml(raw, qt, n, k, DEV, t32=True)
+    assert W.to_t32() and W.layout == "t32"
+    x = torch.randn(M, k, device=DEV).half()
+    ref = x.float().cpu() @ dense.t()
+    plan = ("qr", wm, gw, kw, splits)
+    out = torch.full((M, n), 7.0, device=DEV)
+    L.run_plan((*plan[:-1], 1), W, x, EPI_F32, out, False)
+    assert rel(out, ref) < 5e-3
+    acc = torch.randn(M, n, device=DEV)
+    acc0 = acc.clone()
+    L.run_plan(plan, W, x, EPI_ADD_F32, acc, False)
+    assert rel(acc - acc0, ref) < 5e-3
+    ob = torch.empty(M, n, dtype=torch.float16, device=DEV)
+    L.run_plan((*plan[:-1], 1), W, x, EPI_BF16, ob, False)
+    assert rel(ob, ref) < 5e-3
+    g = ref.reshape(M, n // 32, 2, 16)
+    for epi, act in ((EPI_SWIGLU, torch.nn.functional.silu), (L.EPI_GEGLU, lambda z: torch.nn.functional.gelu(z, approximate="tanh"))):
+        sw = torch.empty(M, n // 2, dtype=torch.float16, device=DEV)
+        L.run_plan((*plan[:-1], 1), W, x, epi, sw, False)
+        assert rel(sw, act(g[:, :, 0].reshape(M, -1)) * g[:, :, 1].reshape(M, -1)) < 1e-2
+
+
 @pytest.mark.parametrize("name,qt,n,k,epi", [
     ("qkv", QType.Q4_K, 6144, 4096, EPI_F32), ("o_proj", QType.Q4_K, 4096, 4096, EPI_ADD_F32),
     ("gate_up", QType.Q4_K, 28672, 4096, EPI_SWIGLU), ("down", QType.Q4_K, 4096, 14336, EPI_ADD_F32),
