@@ -19,59 +19,76 @@ constexpr int GW = 8;  // waves per workgroup of the GEMM
 constexpr int ENC_ACT = 0, ENC_GELU = 1, ENC_PART = 2;  // what the GEMM writes
 __host__ constexpr int enc_parts(int K) { return K >= 2048 ? 4 : 1; }
 
-// LayerNorm of one row held by a wave: lane has the 8-element chunks lane + 64 j. Two passes over registers: the
-// variance is a sum of squares about the mean.
+// A row is held by a wave: lane has the 8-element chunks lane + 64 j. Chunks past H are loaded from the row's last one and count
+// as zero: loads behind a branch are waited for inside it, one after another (LayerNorm of 19 rows after four parts of a product
+// 6.6 -> 4.6 us, the gains and offsets asked for ahead of the sums).
+MX_DEV int enc_chunk(int j, int H, int lane) { return min(8 * (lane + 64 * j), H - 8); }
+MX_DEV bool enc_has(int j, int H, int lane) { return 8 * (lane + 64 * j) < H; }
+
+template <int NC>
+struct LnGain {
+    float4 g[NC][2], b[NC][2];
+    MX_DEV void load(const float* __restrict__ gp, const float* __restrict__ bp, int H, int lane) {
+#pragma unroll
+        for (int j = 0; j < NC; ++j)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int c = enc_chunk(j, H, lane) + 4 * e;
+                g[j][e] = *(const float4*)(gp + c);
+                b[j][e] = bp ? *(const float4*)(bp + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+    }
+};
+
+// LayerNorm of one row. Two passes over registers: the variance is a sum of squares about the mean.
 template <int NC, bool F16>
-MX_DEV void ln_row(float (&v)[NC][8], int H, const float* __restrict__ g, const float* __restrict__ b, float eps,
-                   uint16_t* __restrict__ out, int lane) {
+MX_DEV void ln_row(float (&v)[NC][8], int H, const LnGain<NC>& gb, float eps, uint16_t* __restrict__ out, int lane) {
     float s = 0.f;
 #pragma unroll
     for (int j = 0; j < NC; ++j)
-        if (8 * (lane + 64 * j) < H)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) s += v[j][e];
+        for (int e = 0; e < 8; ++e) s += v[j][e];
     const float mean = wave_sum(s) / H;
     float ss = 0.f;
 #pragma unroll
-    for (int j = 0; j < NC; ++j)
-        if (8 * (lane + 64 * j) < H)
+    for (int j = 0; j < NC; ++j) {
+        float q = 0.f;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) ss += (v[j][e] - mean) * (v[j][e] - mean);
+        for (int e = 0; e < 8; ++e) q += (v[j][e] - mean) * (v[j][e] - mean);
+        ss += enc_has(j, H, lane) ? q : 0.f;
+    }
     const float rs = rsqrtf(wave_sum(ss) / H + eps);
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
-        const int c = 8 * (lane + 64 * j);
-        if (c >= H) continue;
         float y[8];
 #pragma unroll
-        for (int e = 0; e < 8; e += 4) {
-            const float4 gv = *(const float4*)(g + c + e);
-            const float4 bv = b ? *(const float4*)(b + c + e) : make_float4(0.f, 0.f, 0.f, 0.f);
-            y[e] = (v[j][e] - mean) * rs * gv.x + bv.x;
-            y[e + 1] = (v[j][e + 1] - mean) * rs * gv.y + bv.y;
-            y[e + 2] = (v[j][e + 2] - mean) * rs * gv.z + bv.z;
-            y[e + 3] = (v[j][e + 3] - mean) * rs * gv.w + bv.w;
+        for (int e = 0; e < 2; ++e) {
+            const float4 gv = gb.g[j][e], bv = gb.b[j][e];
+            y[4 * e] = (v[j][4 * e] - mean) * rs * gv.x + bv.x;
+            y[4 * e + 1] = (v[j][4 * e + 1] - mean) * rs * gv.y + bv.y;
+            y[4 * e + 2] = (v[j][4 * e + 2] - mean) * rs * gv.z + bv.z;
+            y[4 * e + 3] = (v[j][4 * e + 3] - mean) * rs * gv.w + bv.w;
         }
-        *(uint4*)(out + c) = make_uint4(pack_act2<F16>(y[0], y[1]), pack_act2<F16>(y[2], y[3]), pack_act2<F16>(y[4], y[5]),
-                                        pack_act2<F16>(y[6], y[7]));
+        if (enc_has(j, H, lane))
+            *(uint4*)(out + 8 * (lane + 64 * j)) = make_uint4(pack_act2<F16>(y[0], y[1]), pack_act2<F16>(y[2], y[3]),
+                                                              pack_act2<F16>(y[4], y[5]), pack_act2<F16>(y[6], y[7]));
     }
 }
-
 template <int NC>
 MX_DEV void add_f32(float (&v)[NC][8], const float* __restrict__ p, int H, int lane) {
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
-        const int c = 8 * (lane + 64 * j);
-        if (c >= H) continue;
+        const int c = enc_chunk(j, H, lane);
+        const bool has = enc_has(j, H, lane);
         const float4 a = *(const float4*)(p + c), b = *(const float4*)(p + c + 4);
-        v[j][0] += a.x;
-        v[j][1] += a.y;
-        v[j][2] += a.z;
-        v[j][3] += a.w;
-        v[j][4] += b.x;
-        v[j][5] += b.y;
-        v[j][6] += b.z;
-        v[j][7] += b.w;
+        v[j][0] += has ? a.x : 0.f;
+        v[j][1] += has ? a.y : 0.f;
+        v[j][2] += has ? a.z : 0.f;
+        v[j][3] += has ? a.w : 0.f;
+        v[j][4] += has ? b.x : 0.f;
+        v[j][5] += has ? b.y : 0.f;
+        v[j][6] += has ? b.z : 0.f;
+        v[j][7] += has ? b.w : 0.f;
     }
 }
 
@@ -79,14 +96,12 @@ template <int NC, bool F16>
 MX_DEV void add_act(float (&v)[NC][8], const uint16_t* __restrict__ p, int H, int lane) {
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
-        const int c = 8 * (lane + 64 * j);
-        if (c >= H) continue;
-        const uint4 w = *(const uint4*)(p + c);
+        const uint4 w = *(const uint4*)(p + enc_chunk(j, H, lane));
         const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             float lo, hi;
-            unpack_act2<F16>(ws[e], lo, hi);
+            unpack_act2<F16>(enc_has(j, H, lane) ? ws[e] : 0u, lo, hi);
             v[j][2 * e] += lo;
             v[j][2 * e + 1] += hi;
         }
@@ -101,11 +116,13 @@ __global__ __launch_bounds__(64 * EW) void enc_embed_kernel(const int* __restric
                                                             float eps, uint16_t* __restrict__ x) {
     const int row = blockIdx.x * EW + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (row >= rows) return;
+    LnGain<NC> gb;
+    gb.load(g, b, H, lane);
     float v[NC][8] = {};
     add_f32<NC>(v, tok + (size_t)ids[row] * H, H, lane);
     add_f32<NC>(v, pos + (size_t)ids[rows + row] * H, H, lane);
     if (typ) add_f32<NC>(v, typ + (size_t)ids[2 * rows + row] * H, H, lane);
-    ln_row<NC, F16>(v, H, g, b, eps, x + (size_t)row * H, lane);
+    ln_row<NC, F16>(v, H, gb, eps, x + (size_t)row * H, lane);
 }
 
 // x = LN(a + x): the residual sum in fp32, one pass over 16-bit rows
@@ -115,10 +132,12 @@ __global__ __launch_bounds__(64 * EW) void enc_add_ln_kernel(const uint16_t* __r
                                                              float eps) {
     const int row = blockIdx.x * EW + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (row >= rows) return;
+    LnGain<NC> gb;
+    gb.load(g, b, H, lane);
     float v[NC][8] = {};
     add_act<NC, F16>(v, a + (size_t)row * H, H, lane);
     add_act<NC, F16>(v, x + (size_t)row * H, H, lane);
-    ln_row<NC, F16>(v, H, g, b, eps, x + (size_t)row * H, lane);
+    ln_row<NC, F16>(v, H, gb, eps, x + (size_t)row * H, lane);
 }
 
 // x = LN(sum of parts + bias + x); parts [NP][rows][H] fp32
@@ -129,12 +148,14 @@ __global__ __launch_bounds__(64 * EW) void enc_parts_ln_kernel(const float* __re
                                                                float eps) {
     const int row = blockIdx.x * EW + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (row >= rows) return;
+    LnGain<NC> gb;
+    gb.load(g, b, H, lane);
     float v[NC][8] = {};
 #pragma unroll
     for (int p = 0; p < NP; ++p) add_f32<NC>(v, parts + ((size_t)p * rows + row) * H, H, lane);
     if (bias) add_act<NC, F16>(v, bias, H, lane);
     add_act<NC, F16>(v, x + (size_t)row * H, H, lane);
-    ln_row<NC, F16>(v, H, g, b, eps, x + (size_t)row * H, lane);
+    ln_row<NC, F16>(v, H, gb, eps, x + (size_t)row * H, lane);
 }
 
 // y = gelu(y) in place, 8 elements a thread
