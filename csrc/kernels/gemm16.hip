@@ -1,0 +1,272 @@
+// gemm16.hip — prompts of thousands of rows by quantised weights: the weights are expanded to f16 once (t32_expand) and multiplied by
+// a plain f16 GEMM.
+//
+//   C[M, N] (+)= A[M, K] · B[N, K]^T,   A, B f16, fp32 sums; epilogues as qmm2.hip
+//
+// qmm2's tiles decode the weights of their columns for themselves: beyond some 2000 rows that is done 10 to 40 times over, beside
+// products that want every issue slot (gate|up 28672 x 4096 at 8191 rows: 1750 to 1850 us, 1.04 to 1.1 PFLOP/s). Expanding them
+// first moves 2.6 bytes a weight (80 us there) and leaves a GEMM whose inner loop is products, fragment reads and loads:
+//   * 256 x 256 tiles, four waves of 128 x 128, one on a SIMD: the sums take all 256 accumulation registers. 16 x 16 x 32 products:
+//     32 x 32 x 16 ones of the same tile reach 1.06 PFLOP/s where these reach 1.26 (they write each sum twice as often);
+//   * 64-wide k-tiles by LDS-DMA into five 32 KB slots, A and B apart, so that a tile's successor but one is on its way while the
+//     next waits in LDS. Deeper rings of 32-wide halves, loads through registers or staggered k order changed nothing;
+//   * every product is followed by at most one load or fragment read, and the four waves' loads fall between different products.
+//     The address unit takes 16 cycles a load: issued together, all waves queue behind it with their products (1.26 PFLOP/s;
+//     spread over the tile 1.34, at different places in each wave 1.40);
+//   * the operands are swapped (C^T), so a lane ends with four columns of a row: 16-byte stores, and the residual read a block of
+//     16 rows ahead (read just before each store the epilogue of 4096 columns took 110 us of 310, now 15).
+// Measured at 8191 rows, us, expansion apart: gate|up 28672 x 4096 with SwiGLU 1370 (1.40 PFLOP/s; the library's product without it
+// 1304), 4096 x 14336 with the residual 688, 4096 x 4096 215, 5120 x 4096 275.
+#include "qmm2_fmt.h"
+
+namespace {
+
+constexpr int G16_K = 64;                  // k of a tile
+constexpr int G16_NS = 5;                  // ring slots: A of tile t in 2 t mod 5, B in 2 t + 1 mod 5
+constexpr int G16_SLOT = 256 * 128;        // 256 rows of 128 bytes
+constexpr int G16_LDS = G16_NS * G16_SLOT; // all 160 KB
+
+// lane l: 16 bytes from the scalar base plus the lane's offset to LDS dst + 16 l
+MX_DEV void g16_dma(const void* base, uint32_t off, uint32_t dst) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(dst) : "memory", "m0");
+}
+
+MX_DEV f32x4 g16_mfma(u32x4 a, u32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
+
+template <int EPI>
+__global__ __launch_bounds__(256, 1) void gemm16_kernel(const uint16_t* __restrict__ A, int lda, const uint16_t* __restrict__ B, int ldb,
+                                                        int M, int N, int K, int n_mt, void* __restrict__ Cv, int ldc) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int g = lane >> 4, col = lane & 15;
+    const int wm = wave >> 1, wn = wave & 1;
+
+    // consecutive logical ids run on one XCD, row tiles in bands (q2_tile_of)
+    const int nwg = gridDim.x, bid = blockIdx.x;
+    const int xcd = bid & 7, q8 = nwg >> 3, r8 = nwg & 7;
+    const int lid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (bid >> 3);
+    int mt, nt;
+    q2_tile_of(lid, n_mt, nwg / n_mt, mt, nt);
+    const int m_base = mt * 256, n_base = nt * 256;
+    const int nk = K / G16_K;
+
+    // DMA instruction i of a wave brings rows 64 wave + 8 i .. + 7: lane l chunk (l & 7) of row l >> 3, taken from the row's chunk
+    // (l & 7) ^ ((row >> 1) & 7), so that 16 rows of one chunk lie in 16 bank quads. Rows past M / N repeat the last.
+    uint32_t ao[8], bo[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int row = 64 * wave + 8 * i + (lane >> 3), c = (lane & 7) ^ (4 * (i & 1) + (lane >> 4));
+        ao[i] = (uint32_t)min(row, M - 1 - m_base) * (uint32_t)(2 * lda) + 16 * c;
+        bo[i] = (uint32_t)min(row, N - 1 - n_base) * (uint32_t)(2 * ldb) + 16 * c;
+    }
+    const char* ab = (const char*)(A + (size_t)m_base * lda);
+    const char* bb = (const char*)(B + (size_t)n_base * ldb);
+    const uint32_t wdst = (uint32_t)(uintptr_t)(MX_LDS char*)smem + wave * 8192;
+    // instruction i of tile t's A or B into ring slot s; past the end the last tile again, never read
+    auto dma_a = [&](int t, int s, int i) { g16_dma(ab + (size_t)min(t, nk - 1) * 128, ao[i], wdst + s * G16_SLOT + i * 1024); };
+    auto dma_b = [&](int t, int s, int i) { g16_dma(bb + (size_t)min(t, nk - 1) * 128, bo[i], wdst + s * G16_SLOT + i * 1024); };
+
+    f32x4 acc[8][8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+    // fragment reads: row's chunk 4 ks + g at (4 ks + g) ^ ((row >> 1) & 7)
+    const uint32_t fx = (uint32_t)((g ^ ((col >> 1) & 7)) << 4);
+    const uint32_t a_rd = (uint32_t)((wm * 128 + col) * 128), b_rd = (uint32_t)((wn * 128 + col) * 128);
+    u32x4 f[2][16];  // of the two k-steps: [8 of A, 8 of B]
+    auto rd = [&](int sa, int sb, int ks, int i) {
+        const char* p = smem + (i < 8 ? sa : sb) * G16_SLOT + (i < 8 ? a_rd : b_rd) + (i & 7) * 2048 + (fx ^ (ks * 64));
+        f[ks][i] = *(const u32x4*)p;
+    };
+    auto next = [](int s) { return s >= G16_NS - 2 ? s - (G16_NS - 2) : s + 2; };
+
+#pragma unroll
+    for (int i = 0; i < 8; ++i) dma_a(0, 0, i);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) dma_b(0, 1, i);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) dma_a(1, 2, i);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) dma_b(1, 3, i);
+    q2_wait_barrier<16>();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) rd(0, 1, 0, i);
+
+    int sa = 0, sb = 1, sf = 4;  // slots of tile t, the free one
+    // W8: where among 8 products this wave puts its loads, another place for each wave
+    auto mainloop = [&](auto w_c) {
+        constexpr int W8 = decltype(w_c)::value;
+        int sa = 0, sb = 1, sf = 4;  // slots of tile t's A and B, and the free one
+        for (int t = 0; t < nk; ++t) {
+            const int na = next(sa), nb = next(sb);
+            auto step = [&](auto ks_c, auto beside) {
+                constexpr int ks = decltype(ks_c)::value;
+#pragma unroll
+                for (int m = 0; m < 64; ++m) {
+                    const int i = m >> 3, j = m & 7;
+                    acc[i][j] = g16_mfma(f[ks][8 + j], f[ks][i], acc[i][j]);  // (C^T: a lane's four sums are columns)
+                    beside(m);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            };
+            step(std::integral_constant<int, 0>{}, [&](int m) {
+                if (m < 48 && m % 3 == 0) rd(sa, sb, 1, m / 3);
+                if (m % 8 == W8) dma_a(t + 2, sf, m >> 3);
+            });
+            // A and B of tile t + 1 have landed (A of t + 2 may be on its way), and every wave holds what it needs of tile t: B of
+            // t + 2 follows into A's slot, A of t + 3 into B's
+            asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            step(std::integral_constant<int, 1>{}, [&](int m) {
+                if (m < 48 && m % 3 == 0) rd(na, nb, 0, m / 3);
+                if (m % 8 == W8) dma_b(t + 2, sa, m >> 3);
+            });
+            sf = sb;
+            sa = na;
+            sb = nb;
+        }
+    };
+    if (wave == 0) mainloop(std::integral_constant<int, 1>{});
+    else if (wave == 1) mainloop(std::integral_constant<int, 3>{});
+    else if (wave == 2) mainloop(std::integral_constant<int, 5>{});
+    else mainloop(std::integral_constant<int, 7>{});
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+
+    // ---- epilogue: lane holds columns nb + 4 g .. + 3 of row mb + col; the residual's rows a block ahead of their stores ----
+    int el = lane;
+    asm volatile("" : "+v"(el));  // (no address of it computed ahead of the loop, whose registers are all taken)
+    const int eg = el >> 4, m0 = m_base + wm * 128 + (el & 15), n0 = n_base + wn * 128 + 4 * eg;
+    if constexpr (EPI == E16_SWIGLU || EPI == E16_GEGLU) {
+        // B rows interleaved in 16-row groups: an even column tile is the gate, the next one the up of the same features
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (m0 + 16 * i < M)
+#pragma unroll
+                for (int j = 0; j < 8; j += 2) {
+                    if (n0 + 16 * j >= N) break;
+                    float v[4];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[r] = glu_gate_f<EPI>(acc[i][j][r]) * acc[i][j + 1][r];
+                    *(u32x2*)((uint16_t*)Cv + (size_t)(m0 + 16 * i) * ldc + ((n0 + 16 * j - 4 * eg) >> 1) + 4 * eg) =
+                        (u32x2){pack_act2<true>(v[0], v[1]), pack_act2<true>(v[2], v[3])};
+                }
+    } else if constexpr (EPI == E16_ACT) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (m0 + 16 * i < M)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    if (n0 + 16 * j >= N) break;
+                    *(u32x2*)((uint16_t*)Cv + (size_t)(m0 + 16 * i) * ldc + n0 + 16 * j) =
+                        (u32x2){pack_act2<true>(acc[i][j][0], acc[i][j][1]), pack_act2<true>(acc[i][j][2], acc[i][j][3])};
+                }
+    } else {
+        f32x4 old[2][8];
+        auto load = [&](int i) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)  // (past M / N: the last ones)
+                old[i & 1][j] = *(const f32x4*)((const float*)Cv + (size_t)min(m0 + 16 * i, M - 1) * ldc + min(n0 + 16 * j, N - 4));
+        };
+        if constexpr (EPI == E16_ADD_F32) load(0);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            if constexpr (EPI == E16_ADD_F32) {
+                if (i < 7) load(i + 1);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) acc[i][j] += old[i & 1][j];
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(acc[i][j]));  // (stored from there: from where they are, the loop spills)
+            }
+            if (m0 + 16 * i < M)
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if (n0 + 16 * j < N) *(f32x4*)((float*)Cv + (size_t)(m0 + 16 * i) * ldc + n0 + 16 * j) = acc[i][j];
+        }
+    }
+}
+
+template <int EPI>
+int launch_gemm16(const uint16_t* A, int lda, const uint16_t* B, int ldb, int M, int N, int K, void* C, int ldc, hipStream_t st) {
+    const int n_mt = (M + 255) / 256;
+    const long nwg = (long)n_mt * ((N + 255) / 256);
+    if (nwg > 0x7fffffff) return (int)hipErrorInvalidValue;
+    static bool attr_set = false;
+    if (!attr_set) {
+        (void)hipFuncSetAttribute((const void*)gemm16_kernel<EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, G16_LDS);
+        attr_set = true;
+    }
+    gemm16_kernel<EPI><<<dim3((unsigned)nwg), 256, G16_LDS, st>>>(A, lda, B, ldb, M, N, K, n_mt, C, ldc);
+    MXK_CHECK_LAUNCH();
+}
+
+// out[32 g + col][256 sb + ..] = the f16 weights of column group g's super-block sb as the GEMMs decode them (Q2B), a wave each;
+// the fragment of k-step s of tile jq is 16 bytes a lane at k 64 jq + 16 s + 8 h. Bound by its stores (2 of 2.6 bytes a weight).
+template <int QT>
+__global__ __launch_bounds__(256) void t32_expand_kernel(const uint8_t* __restrict__ W, int units, int nsb, uint16_t* __restrict__ out) {
+    using F = Q2F<QT>;
+    const int unit = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, h = lane >> 5, col = lane & 31;
+    if (unit >= units) return;
+    const int g = unit / nsb, sb = unit - g * nsb;
+    const char* u = (const char*)W + (size_t)unit * F::UNIT;
+    uint16_t* o = out + ((size_t)g * 32 + col) * ((size_t)nsb * 256) + sb * 256 + 8 * h;
+    Q2B<QT> b[4];
+    if constexpr (QT == MXQ_Q5_K) b[0].load_hdr(u, u + F::QH, col, h);  // (a header in two places)
+    else b[0].load_hdr(u, col, h);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        if (q > 0) b[q] = b[0];
+        b[q].load_q(u + F::qoff(q), col, h);
+    }
+    auto tile = [&](auto q_c) {
+        constexpr int Q = decltype(q_c)::value;
+        b[Q].template prep<Q>();
+        *(f16x8*)(o + 64 * Q) = b[Q].template frag<Q, 0>();
+        *(f16x8*)(o + 64 * Q + 16) = b[Q].template frag<Q, 1>();
+        *(f16x8*)(o + 64 * Q + 32) = b[Q].template frag<Q, 2>();
+        *(f16x8*)(o + 64 * Q + 48) = b[Q].template frag<Q, 3>();
+    };
+    tile(std::integral_constant<int, 0>{});
+    tile(std::integral_constant<int, 1>{});
+    tile(std::integral_constant<int, 2>{});
+    tile(std::integral_constant<int, 3>{});
+}
+
+}  // namespace
+
+// t32 weights [N, K] (N % 32 == 0, K % 256 == 0) -> f16 [N, K]
+extern "C" int mxk_t32_expand(int qtype, const uint8_t* W, int N, int K, uint16_t* out, hipStream_t st) {
+    if (N <= 0 || K <= 0) return 0;
+    if (N % 32 || K % 256 || ((uintptr_t)W & 15) || ((uintptr_t)out & 15)) return (int)hipErrorInvalidValue;
+    const long units = (long)(N / 32) * (K / 256);
+    if (units > 0x7ffffffc) return (int)hipErrorInvalidValue;
+#define T32X(QT_) \
+    case QT_: t32_expand_kernel<QT_><<<(unsigned)((units + 3) / 4), 256, 0, st>>>(W, (int)units, K / 256, out); break;
+    switch (qtype) {
+        T32X(MXQ_Q4_K) T32X(MXQ_Q5_K) T32X(MXQ_Q6_K) T32X(MXQ_Q3_K) T32X(MXQ_Q2_K) T32X(MXQ_Q8_0) T32X(MXQ_MX4F) T32X(MXQ_MX5F)
+        default: return (int)hipErrorInvalidValue;
+    }
+#undef T32X
+    MXK_CHECK_LAUNCH();
+}
+
+// A f16 [M, K], B f16 [N, K], rows 16-byte aligned, K % 64 == 0, N % 32 == 0; C rows of 16-byte (16-bit outputs: 8-byte) aligned
+// pieces. epi as mxk_qmm2 (no split).
+extern "C" int mxk_gemm16(int epi, const uint16_t* A, int lda, const uint16_t* B, int ldb, int M, int N, int K, void* C, int ldc,
+                          hipStream_t st) {
+    if (M <= 0 || N <= 0) return 0;
+    if (K <= 0 || K % G16_K || N % 32 || (lda & 7) || (ldb & 7) || ((uintptr_t)A & 15) || ((uintptr_t)B & 15) || lda < K || ldb < K ||
+        lda > (1 << 22) || ldb > (1 << 22) || ((uintptr_t)C & 15) || (ldc & 3))  // (256 rows of 2^23 bytes: the 32-bit lane offsets)
+        return (int)hipErrorInvalidValue;
+    switch (epi) {
+        case E16_F32: return launch_gemm16<E16_F32>(A, lda, B, ldb, M, N, K, C, ldc, st);
+        case E16_ACT: return launch_gemm16<E16_ACT>(A, lda, B, ldb, M, N, K, C, ldc, st);
+        case E16_ADD_F32: return launch_gemm16<E16_ADD_F32>(A, lda, B, ldb, M, N, K, C, ldc, st);
+        case E16_SWIGLU: return launch_gemm16<E16_SWIGLU>(A, lda, B, ldb, M, N, K, C, ldc, st);
+        case E16_GEGLU: return launch_gemm16<E16_GEGLU>(A, lda, B, ldb, M, N, K, C, ldc, st);
+    }
+    return (int)hipErrorInvalidValue;
+}

@@ -326,7 +326,7 @@ def row_chunks(M: int, chunk: int | None = None) -> list[tuple[int, int]]:
 def run_plan(plan: tuple, W: QWeight, x: torch.Tensor, epi: int, out: torch.Tensor, out_zeroed: bool,
              fuse: "NormFuse | None" = None):
     """Launch one GEMM plan (ops/autotune.py): ("q3", wm, splits) | ("q2", wm, ks, wn, splits) |
-    ("qr", wm, gw, kw, splits) | ("rows", chunk)."""
+    ("qr", wm, gw, kw, splits) | ("rows", chunk) | ("x16", columns, plan)."""
     M = x.shape[0]
     kind = plan[0]
     if fuse is not None and kind != "q2":
@@ -335,6 +335,8 @@ def run_plan(plan: tuple, W: QWeight, x: torch.Tensor, epi: int, out: torch.Tens
         for r0, r1 in row_chunks(M, plan[1]):
             _qmatmul_t32(W, x[r0:r1], epi, out[r0:r1], None, None, r1 - r0, out_zeroed)
         return out
+    if kind == "x16":
+        return _run_x16(plan, W, x, epi, out, out_zeroed)
     splits = plan[-1]
     e = EPI_ADD_F32 if (epi == EPI_F32 and splits > 1) else epi
     if e in (EPI_BF16, *GLU_EPIS):
@@ -369,6 +371,31 @@ def run_plan(plan: tuple, W: QWeight, x: torch.Tensor, epi: int, out: torch.Tens
     return out
 
 
+def _run_x16(plan: tuple, W: QWeight, x: torch.Tensor, epi: int, out: torch.Tensor, out_zeroed: bool):
+    """("x16", columns, plan): gemm16.hip on the weight's rows expanded to f16, `columns` of them at a time; `plan` where what
+    the kernel reads or writes is not aligned for it or the scratch cannot be had."""
+    M, glu = x.shape[0], epi in GLU_EPIS
+    if epi in (EPI_BF16, *GLU_EPIS) and out.dtype != x.dtype:
+        raise ValueError(f"qmatmul: {out.dtype} output with {x.dtype} activations")
+    ok = x.stride(0) % 8 == 0 and W.K <= x.stride(0) <= 1 << 22 and out.stride(0) % 4 == 0 and not (x.data_ptr() | out.data_ptr()) & 15
+    cols = min(plan[1], W.N)
+    try:
+        part = torch.empty(cols, W.K, dtype=torch.float16, device=x.device) if ok else None
+    except torch.cuda.OutOfMemoryError:
+        part = None
+    if part is None:
+        return run_plan(plan[2], W, x, epi, out, out_zeroed)
+    N.ensure_act(x.dtype)
+    st = N.stream_ptr()
+    row = W.data.numel() * W.data.element_size() // W.N  # bytes of a column of the product (whole 32-column units)
+    for n0 in range(0, W.N, cols):
+        n = min(cols, W.N - n0)
+        N.kcall("mxk_t32_expand", int(W.qtype), W.data.data_ptr() + n0 * row, n, W.K, part.data_ptr(), st)
+        N.kcall("mxk_gemm16", epi, x.data_ptr(), x.stride(0), part.data_ptr(), W.K, M, n, W.K,
+                out.data_ptr() + (n0 // 2 if glu else n0) * out.element_size(), out.stride(0), st)
+    return out
+
+
 def _t32_plan(W: QWeight, M: int, epi: int, out_zeroed: bool, dtype=torch.float16):
     """The plan _qmatmul_t32 runs for an M-row f16 GEMM on t32 weights, or None where it takes the dense copy."""
     can_split = epi == EPI_ADD_F32 or (epi == EPI_F32 and out_zeroed)
@@ -381,6 +408,8 @@ def _t32_plan(W: QWeight, M: int, epi: int, out_zeroed: bool, dtype=torch.float1
             plan = ("rows", ROW_CHUNK)
         else:
             plan = _gemm_pick(M, W.N, W.K, int(W.qtype), can_split)
+            if M >= X16_MIN_M and not forced and dtype == torch.float16:
+                plan = _expanded_plan(M, W.N, W.K, int(W.qtype), can_split, epi in GLU_EPIS) or plan
     return plan
 
 
@@ -623,8 +652,8 @@ _STAGE_BYTES = {int(QType.Q4_K): (1024, 512), int(QType.Q5_K): (1024, 1536), int
 
 
 @functools.lru_cache(maxsize=4096)
-def _large_plan(M: int, N_: int, K: int, qtype: int, can_split: bool):
-    """qmm2 plan of a GEMM of more than LARGE_M rows: the least of
+def _large_best(M: int, N_: int, K: int, qtype: int, can_split: bool):
+    """(estimate, plan): the qmm2 plan of a GEMM of more than LARGE_M rows: the least of
         6.6 + rounds * tile * K / splits * c  (+ 2.4e-6 * M * N * splits where partial sums meet in atomics)   us
     over the tiles whose ring fits the LDS for the format, rounds = workgroups / 256 with a last round that is r full
     counted as 0.6 + 0.4 r (a half-empty chip clocks and feeds its tiles faster). The constants are a fit to 13 shapes
@@ -644,7 +673,7 @@ def _large_plan(M: int, N_: int, K: int, qtype: int, can_split: bool):
         return t + 2.4e-6 * M * N_ * s if s > 1 else t
     square = next(t for t in _LARGE_TILES if t[:3] == (4, 2, 1))
     splits = 1 if N_ < 16384 and K < 8192 else _split_for(-(-M // 128) * -(-N_ // 128), K, can_split)
-    best = (0.93 * cost(*square, splits), ("q2", 4, 2, 1, splits))
+    best = first = (0.93 * cost(*square, splits), ("q2", 4, 2, 1, splits))
     for wm, ks, wn, c in _LARGE_TILES:
         bm, ng = 32 * wm * wn, 8 if ks == 17 else 4
         if 4 * (bm * 128 + ng * qb) + 2 * ng * hb > 160 * 1024:
@@ -655,7 +684,32 @@ def _large_plan(M: int, N_: int, K: int, qtype: int, can_split: bool):
             t = cost(wm, ks, wn, c, s)
             if t < best[0]:
                 best = (t, ("q2", wm, ks, wn, s))
-    return best[1]
+    return (best[0] / 0.93, best[1]) if best is first else best
+
+
+def _large_plan(M: int, N_: int, K: int, qtype: int, can_split: bool):
+    return _large_best(M, N_, K, qtype, can_split)[1]
+
+
+X16_MIN_M = 1025  # (steps of up to 1024 rows are captured: their graphs would keep the f16 scratch for good)
+X16_SCRATCH = 1 << 28  # bytes of f16 weights expanded at a time
+
+
+@functools.lru_cache(maxsize=4096)
+def _expanded_plan(M: int, N_: int, K: int, qtype: int, can_split: bool, glu: bool):
+    """("x16", columns, qmm2 plan) where expanding the weights to f16 and gemm16.hip are estimated below that plan, else None.
+    Expansion: 5 us + 0.62 per 10^6 weights; products: 6 us + 1.45 a 64-wide k-tile of each round of 256 x 256 tiles (the last one
+    counted as in _large_best) + 12 a round to fill and drain (gated: 5, it writes a quarter). _large_best is 5 % low against
+    these measurements, 12 % and more for gated products. Of 77 products (11 shapes 1024 x 4096 .. 28672 x 4096 at 1024 .. 8191 rows)
+    none picked was slower than the qmm2 plan; what it gives: us, gate|up 28672 x 4096 at 1536 / 2048 / 4096 / 8191 rows 392 -> 364,
+    477 -> 437, 943 -> 755, 1828 -> 1435; 4096 x 14336 Q4_K at 4096 / 8191 452 -> 376, 879 -> 719, Q6_K 485 -> 382, 922 -> 729; 4096 x
+    4096 142 -> 122, 271 -> 231; 6144 x 4096 at 8191 396 -> 324; 16384 x 2048 gated at 2048 / 8191 160 -> 144, 570 -> 449."""
+    t, plan = _large_best(M, N_, K, qtype, can_split)
+    full, rem = divmod(-(-M // 256) * -(-N_ // 256), CU_COUNT)
+    rounds = full + (0.6 + 0.4 * rem / CU_COUNT if rem else 0.0)
+    if 11.0 + rounds * (1.45 * K / 64 + (5.0 if glu else 12.0)) + 0.62e-6 * N_ * K < t * (1.12 if glu else 1.05):
+        return ("x16", max(256, X16_SCRATCH // (K * 512) * 256), plan)
+    return None
 
 
 def _gemm_pick(M: int, N_: int, K: int, qtype: int, can_split: bool):

@@ -102,3 +102,43 @@ def test_every_tile_in_bands(qt, tile):
         y = want.view(M, -1, 2, 16)
         g = (torch.nn.functional.silu(y[:, :, 0]) * y[:, :, 1]).reshape(M, -1)
         assert float((act.cpu().double() - g).norm() / g.norm()) < 4 * 2 ** -10
+
+
+def test_expanded_plans():
+    """Weights are expanded where rows are many and the tiles fill the chip; the scratch is bounded and whole column tiles wide."""
+    pick = lambda m, n, k, glu=False: L._expanded_plan(m, n, k, int(QType.Q4_K), not glu, glu)  # noqa: E731
+    assert pick(8191, 28672, 4096, True)[0] == pick(8191, 4096, 14336)[0] == "x16" and pick(2048, 4096, 14336) is None
+    assert pick(8191, 1024, 4096) is None and pick(1100, 1024, 4096) is None
+    kind, cols, plan = pick(8191, 57344, 8192, True)
+    assert cols % 256 == 0 and 256 <= cols and cols * 8192 * 2 <= L.X16_SCRATCH and plan == L._large_plan(8191, 57344, 8192, int(QType.Q4_K), False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("qt", [*QTYPES, QType.Q4_0, QType.Q5_0, QType.Q5_1])
+def test_expanded_products(qt):
+    """gemm16.hip on expanded weights: part-empty tiles of rows and columns, three pieces of columns, every epilogue; and the qmm2 plan
+    for rows that it cannot read as they lie."""
+    n, k = 288, 1536
+    W, dense = _weight(qt, n, k)
+    for M, cols in ((1, 512), (255, 256), (257, 256), (600, 32)):
+        plan = ("x16", cols, ("q2", 4, 2, 1, 1))
+        wide = (torch.randn(M, k + 8, generator=torch.Generator().manual_seed(M)) * 0.5).half()
+        x, xd = wide[:, :k], wide[:, :k].cuda()
+        want = x.double() @ dense.double().t()
+        base = torch.randn(M, n, generator=torch.Generator().manual_seed(1))
+        for rows in (xd.contiguous(), wide.cuda()[:, :k]):
+            out = torch.full((M, n), 7.0, device="cuda")
+            L.run_plan(plan, W, rows, L.EPI_F32, out, False)
+            assert float((out.cpu().double() - want).norm() / want.norm()) < 2 ** -10  # weights rounded to f16 once (2^-11)
+        out = base.cuda()
+        L.run_plan(plan, W, xd, L.EPI_ADD_F32, out, False)
+        assert float((out.cpu().double() - base - want).norm() / want.norm()) < 2 ** -10
+        o16 = torch.zeros(M, n, device="cuda", dtype=torch.float16)
+        L.run_plan(plan, W, xd, L.EPI_BF16, o16, False)
+        assert float((o16.cpu().double() - want).norm() / want.norm()) < 2 * 2 ** -10
+        y = want.view(M, -1, 2, 16)
+        for epi, act in ((L.EPI_SWIGLU, torch.nn.functional.silu), (L.EPI_GEGLU, lambda z: torch.nn.functional.gelu(z, approximate="tanh"))):
+            glu = torch.zeros(M, n // 2, device="cuda", dtype=torch.float16)
+            L.run_plan(plan, W, xd, epi, glu, False)
+            g = (act(y[:, :, 0]) * y[:, :, 1]).reshape(M, -1)
+            assert float((glu.cpu().double() - g).norm() / g.norm()) < 4 * 2 ** -10
