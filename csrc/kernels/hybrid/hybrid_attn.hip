@@ -351,13 +351,26 @@ MX_DEV bf16x8 v_fragment(const char* v_lds, int r0, int nt, int col) {
 // B holds column col, k = 8g .. 8g + 7; the result holds rows 4g .. 4g + 3 of column col.
 // P2: every softmax weight enters the value product as two bf16 numbers (its rounding, and the rounding of what that
 // lost) in two products that share the value fragment, so the weights count to 16 bits of mantissa.
+// The chunks of a step are one launch, the longest first: a launch ends with the few workgroups whose rows see the most keys
+// (chunks of 1111, 578 and 301 rows one after another 86 + 49 + 25 us, 123 us together).
+constexpr int ATTN_SEQS = 16;
+struct AttnSeqs {  // chunk i: workgroups first[i] .. first[i + 1], n rows from row on at positions p0 .., pages in row bt of the tables
+    int count, first[ATTN_SEQS + 1], bt[ATTN_SEQS], p0[ATTN_SEQS], n[ATTN_SEQS], row[ATTN_SEQS];
+};
 template <int DK, int DV, bool O16, bool P2>
 __global__ __launch_bounds__(256) void attn_chunk_mfma_kernel(const bf16_t* __restrict__ q, int ldq,
                                                               const bf16_t* __restrict__ kc,
                                                               const bf16_t* __restrict__ vc, int bs,
-                                                              const int* __restrict__ table, int p0, int n, void* out,
+                                                              const int* __restrict__ table, int bt_stride, AttnSeqs sq, void* out,
                                                               int ldo, int H, int G, int GW, float scale, int chunk,
                                                               int window, int sink, float out_scale, AttnExtra ex) {
+    int s = 0;
+    while (s + 1 < sq.count && sq.first[s + 1] <= (int)blockIdx.x) ++s;
+    const int p0 = sq.p0[s], n = sq.n[s], last = sq.first[s + 1] - 1;
+    table += (size_t)sq.bt[s] * bt_stride;
+    q += (size_t)sq.row[s] * ldq;
+    out = O16 ? (void*)((bf16_t*)out + (size_t)sq.row[s] * ldo) : (void*)((float*)out + (size_t)sq.row[s] * ldo);
+    if (ex.gate) ex.gate += (size_t)sq.row[s] * ex.ldg;
     constexpr int KT = 64;
     constexpr int KSTR = (DK + 8) * 2;  // bytes per key row in LDS (padded)
     constexpr int VSTR = (DV + 8) * 2;  // bytes per value row in LDS (padded)
@@ -372,7 +385,7 @@ __global__ __launch_bounds__(256) void attn_chunk_mfma_kernel(const bf16_t* __re
     const int hq = blockIdx.y * GW + (wave % GW);
     const int kvh = (blockIdx.y * GW) / (H / G);
     // the chunk's last rows see the most keys: their workgroups are scheduled first
-    const int q0 = (gridDim.x - 1 - blockIdx.x) * RT * 16;  // first query row of the workgroup
+    const int q0 = (last - (int)blockIdx.x) * RT * 16;  // first query row of the workgroup
     const int row_q0 = q0 + (wave / GW) * 16;     // first query row of this wave
     const int a_pos = p0 + q0;                    // position of the workgroup's first row
     const int kv_end = p0 + min(n, q0 + RT * 16);  // one past the last visible key
@@ -964,31 +977,56 @@ extern "C" int mxh_masked_softmax(const float* sc, void* pw, int p16, long rows,
     return (int)hipGetLastError();
 }
 
-// A prompt chunk of n rows of one sequence (q and out point at its first row) at positions p0 .., bf16 pools.
+// Prompt chunks of sequences, bf16 pools; seqs [count][4] (host): row of the tables, first position, rows, first row of q, out and gate.
 // Returns hipErrorInvalidValue for head sizes without an instantiation: the caller asks mxh_attention_mfma_ok first.
 extern "C" int mxh_attention_mfma_ok(int dk, int dv) {
     return ((dk == 64 || dk == 128) && (dv == 64 || dv == 128)) || (dk == 96 && dv == 96);
 }
 
 extern "C" int mxh_attention_mfma(const void* q, int ldq, const void* kc, const void* vc, int bs, const int* table,
-                                  int p0, int n, void* out, int ldo, int o16, int H, int G, int dk, int dv,
+                                  int bt_stride, const int* seqs, int count, void* out, int ldo, int o16, int H, int G, int dk, int dv,
                                   float scale, int chunk, int window, int sink, float out_scale, const float* sink_v,
                                   const float* bias, int nb, const float* gate, int ldg, int gv, int p2,
                                   int keep, int gw, float softcap, hipStream_t st) {
-    if (n <= 0) return 0;
+    if (count <= 0) return 0;
     MXH_CHECK((!bias || nb > 0) && (!gate || ldg >= H * gw) && (!sink_v || sink) && gv > 0 && G % gv == 0 && keep >= 0);
     MXH_CHECK((gw == 1 || gw == dv) && softcap >= 0.f);
     const AttnExtra ex = {sink_v, bias, nb, gate, ldg, gw, softcap, gv, keep};
-    MXH_CHECK(q && kc && vc && table && out && bs > 0 && p0 >= 0 && H > 0 && G > 0 && H % G == 0);
+    MXH_CHECK(q && kc && vc && table && out && bs > 0 && seqs && bt_stride >= 0 && H > 0 && G > 0 && H % G == 0);
     MXH_CHECK(mxh_attention_mfma_ok(dk, dv) && ldq >= H * dk && ldq % 8 == 0 && ldo >= H * dv && chunk >= 0 && window >= 0);
     const int rep = H / G;
     const int GW = rep % 4 == 0 ? 4 : rep % 2 == 0 ? 2 : 1;
     const int RT = 4 / GW;
     MXH_CHECK(H / GW <= 65535);
-    const dim3 grid((n + RT * 16 - 1) / (RT * 16), H / GW);
+    for (int i = 0; i < count; ++i) MXH_CHECK(seqs[4 * i] >= 0 && seqs[4 * i + 1] >= 0 && seqs[4 * i + 2] >= 0 && seqs[4 * i + 3] >= 0);
+    for (int i0 = 0; i0 < count; i0 += ATTN_SEQS) {
+        const int some = min(count - i0, ATTN_SEQS);
+        int order[ATTN_SEQS];  // by their last key, the longest first
+        for (int i = 0; i < some; ++i) {
+            auto end = [&](int k) { return (long)seqs[4 * k + 1] + seqs[4 * k + 2]; };
+            int j = i;
+            for (; j > 0 && end(order[j - 1]) < end(i0 + i); --j) order[j] = order[j - 1];
+            order[j] = i0 + i;
+        }
+        AttnSeqs sq = {};
+        long blocks = 0;
+        for (int i = 0; i < some; ++i) {
+            const int* c = seqs + 4 * order[i];
+            if (c[2] == 0) continue;
+            const int k = sq.count++;
+            sq.bt[k] = c[0];
+            sq.p0[k] = c[1];
+            sq.n[k] = c[2];
+            sq.row[k] = c[3];
+            blocks += (c[2] + RT * 16 - 1) / (RT * 16);
+            MXH_CHECK(blocks <= 0x7fffffff);
+            sq.first[k + 1] = (int)blocks;
+        }
+        if (blocks == 0) continue;
+        const dim3 grid((unsigned)blocks, H / GW);
 #define GO3(K_, V_, O_, P_)                                                                                       \
     attn_chunk_mfma_kernel<K_, V_, O_, P_><<<grid, 256, 0, st>>>((const bf16_t*)q, ldq, (const bf16_t*)kc,             \
-                                                                 (const bf16_t*)vc, bs, table, p0, n, out, ldo, H, G, \
+                                                                 (const bf16_t*)vc, bs, table, bt_stride, sq, out, ldo, H, G, \
                                                                  GW, scale, chunk, window, sink, out_scale, ex)
 #define GO(K_, V_)                                 \
     do {                                           \
@@ -997,11 +1035,12 @@ extern "C" int mxh_attention_mfma(const void* q, int ldq, const void* kc, const 
         else if (p2) GO3(K_, V_, false, true);     \
         else GO3(K_, V_, false, false);            \
     } while (0)
-    if (dk == 64 && dv == 64) GO(64, 64);
-    else if (dk == 64 && dv == 128) GO(64, 128);
-    else if (dk == 128 && dv == 64) GO(128, 64);
-    else if (dk == 96) GO(96, 96);
-    else GO(128, 128);
+        if (dk == 64 && dv == 64) GO(64, 64);
+        else if (dk == 64 && dv == 128) GO(64, 128);
+        else if (dk == 128 && dv == 64) GO(128, 64);
+        else if (dk == 96) GO(96, 96);
+        else GO(128, 128);
+    }
 #undef GO
 #undef GO3
     return (int)hipGetLastError();

@@ -182,10 +182,10 @@ HYBRID_SIGS = {
     # (value heads, kept first tokens, gates per head and score cap before the stream)
     "mxh_attention": [P, I, I, P, P, I, P, I, P, P, I, I, I, P, I, I, I, I, I, I, F, I, I, I, F, I, I, I, P, P, P, P, I,
                       P, I, I, I, I, F, P],
-    # q, ldq, kc, vc, bs, table, p0, n, out, ldo, o16, H, G, dk, dv, scale, chunk, window, sink, out_scale, sink_v,
-    # bias, bias_rows, gate, ldg, stream
+    # q, ldq, kc, vc, bs, tables, stride, chunks [count][4] on the host, count, out, ldo, o16, H, G, dk, dv, scale, chunk, window, sink,
+    # out_scale, sink_v, bias, bias_rows, gate, ldg, stream
     # (value heads, the two-part weights flag, kept first tokens, gates per head and score cap before the stream)
-    "mxh_attention_mfma": [P, I, P, P, I, P, I, I, P, I, I, I, I, I, I, F, I, I, I, F, P, P, I, P, I, I, I, I, I,
+    "mxh_attention_mfma": [P, I, P, P, I, P, I, P, I, P, I, I, I, I, I, I, F, I, I, I, F, P, P, I, P, I, I, I, I, I,
                            F, P],
     "mxh_attention_mfma_ok": [I, I],
     # q, ldq, kc, vc, bs, bt, bt_stride, ctx, n_seqs, out, ldo, o16, H, G, dk, dv, scale, chunk, window, sink, out_scale,

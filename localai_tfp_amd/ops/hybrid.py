@@ -47,6 +47,7 @@ states and the residual are fp32 in both; 16-bit tensors appear only as GEMM ope
 """
 from __future__ import annotations
 
+import ctypes
 import math
 
 import torch
@@ -652,27 +653,28 @@ def masked_attention(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, rag: R
         if lens is None or max(lens) < big or (not mfma and 0 < chunk < GEMM_MIN_ROWS):
             rows_kernel(0, T - nd)  # (mask chunks shorter than a block of rows: few visible keys, the row kernel's case)
             return out
-        r, run0 = 0, None  # run0: first row of a run of consecutive short chunks
+        r, run0, seqs = 0, None, []  # run0: first row of a run of consecutive short chunks
         for k, n in enumerate(lens):
             if n >= big:
                 if run0 is not None:
                     rows_kernel(run0, r - run0)
                     run0 = None
-                qk, ok = q[nd + r:nd + r + n], out[nd + r:nd + r + n]
-                gk = gate[nd + r:nd + r + n] if gate is not None else None
                 if mfma:
-                    N.kcall("mxh_attention_mfma", qk.data_ptr(), qk.stride(0), kc.data_ptr(), vc.data_ptr(), bs,
-                            rag.pf_bt[k].data_ptr(), rag.pf_ctx_host[k] - n, n, ok.data_ptr(), ok.stride(0), _is16(out),
-                            H, G, dk, dv, float(scale), int(chunk), int(window), int(sink), float(out_scale), *extra,
-                            N.ptr(gk), ldg, Gv, int(p32), int(keep), gw, cap, st)
+                    seqs += (k, rag.pf_ctx_host[k] - n, n, nd + r)
                 else:
-                    _attn_gemm_chunk(qk, kc, vc, rag.pf_bt[k], rag.pf_ctx_host[k] - n, n, H, G, dk, dv, scale, chunk,
-                                     window, sink, ok, out_scale, sink_v, bias, gk, Gv, p32, keep, softcap)
+                    gk = gate[nd + r:nd + r + n] if gate is not None else None
+                    _attn_gemm_chunk(q[nd + r:nd + r + n], kc, vc, rag.pf_bt[k], rag.pf_ctx_host[k] - n, n, H, G, dk, dv, scale, chunk,
+                                     window, sink, out[nd + r:nd + r + n], out_scale, sink_v, bias, gk, Gv, p32, keep, softcap)
             elif n and run0 is None:
                 run0 = r
             r += n
         if run0 is not None:
             rows_kernel(run0, r - run0)
+        if seqs:
+            N.kcall("mxh_attention_mfma", q.data_ptr(), q.stride(0), kc.data_ptr(), vc.data_ptr(), bs, rag.pf_bt.data_ptr(),
+                    rag.pf_bt.stride(0), (ctypes.c_int * len(seqs))(*seqs), len(seqs) // 4, out.data_ptr(), out.stride(0), _is16(out), H, G,
+                    dk, dv, float(scale), int(chunk), int(window), int(sink), float(out_scale), *extra, N.ptr(gate), ldg, Gv, int(p32),
+                    int(keep), gw, cap, st)
     return out
 
 

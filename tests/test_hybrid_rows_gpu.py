@@ -133,3 +133,33 @@ def test_glu_of_many_elements(act):
                 got[dev] = out.cpu().float()
             tol = 2e-5 if dt == torch.float32 else 2 ** -7
             assert ((got["cuda"] - got["cpu"]).abs() <= tol * got["cpu"].abs().clamp_min(1)).all()
+
+
+@pytest.mark.parametrize("chunk,window", [(0, 0), (128, 0), (0, 40)])
+def test_chunks_of_many_sequences(chunk, window):
+    """The chunks of a step are launched sixteen at a time, the longest first: eighteen sequences (with short ones between, which run on
+    the row kernel) behind cached tokens, each as it is alone on the CPU. bf16 weights and outputs: 2^-8 of numbers of order 1."""
+    H, G, D, bs = 4, 2, 64, 8
+    lens = [16, 70, 3, 129, 64, 33, 17, 200, 16, 48, 1, 90, 20, 31, 66, 16, 130, 25, 80, 40]
+    pre = [5 * i % 37 for i in range(len(lens))]
+    g, T = torch.Generator().manual_seed(3), sum(lens)
+    need = [-(-(p + n) // bs) for p, n in zip(pre, lens)]
+    order = torch.randperm(sum(need), generator=g).tolist()
+    tables, at = torch.zeros(len(lens), max(need), dtype=torch.int32), 0
+    for i, n in enumerate(need):
+        tables[i, :n] = torch.tensor(order[at:at + n], dtype=torch.int32)
+        at += n
+    q = torch.randn(T, H * D, generator=g).bfloat16()
+    kc, vc = (torch.randn(sum(need), bs, G * D, generator=g).bfloat16() for _ in range(2))
+    cu = [sum(lens[:i]) for i in range(len(lens) + 1)]
+    i32 = lambda x, dev: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    got = {}
+    for dev in ("cpu", "cuda"):
+        ctx = [p + n for p, n in zip(pre, lens)]
+        rag = HY.Ragged(types.SimpleNamespace(T=T, n_decode=0, positions=i32([0] * T, dev), seq_state=None, slots=None, pf_cu_q=i32(cu, dev),
+                                              pf_q_lens_host=lens, pf_ctx_lens_host=ctx, pf_block_tables=tables.to(dev), pf_ctx_lens=i32(ctx, dev),
+                                              dec_block_tables=None, dec_seq_lens=None, dec_max_len=0))
+        out = torch.zeros(T, H * D, device=dev, dtype=torch.bfloat16)
+        HY.masked_attention(q.to(dev), kc.to(dev), vc.to(dev), rag, H, G, D, D, D ** -0.5, out, chunk=chunk, window=window)
+        got[dev] = out.float().cpu()
+    assert (got["cuda"] - got["cpu"]).abs().max() <= 2 ** -6 and (got["cuda"] - got["cpu"]).norm() <= 2 ** -8 * got["cpu"].norm()
