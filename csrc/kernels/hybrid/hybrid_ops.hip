@@ -548,7 +548,8 @@ __global__ __launch_bounds__(NT) void glu_kernel(const float* a, int lda, const 
                                                  const float* bb, const float* scale, int lds, int group,
                                                  int scale_sigmoid, void* out, int ldo, int F, int act, float limit,
                                                  float alpha) {
-    const int f = (blockIdx.y * NT + threadIdx.x) * V, t = blockIdx.x;
+    const int chunks = (F + NT * V - 1) / (NT * V), t = blockIdx.x / chunks;  // neighbouring workgroups share a row
+    const int f = ((blockIdx.x - t * chunks) * NT + threadIdx.x) * V;
     if (f >= F) return;
     auto put = [&](const float* v) {
         if constexpr (V == 4 && B16)
@@ -580,13 +581,15 @@ __global__ __launch_bounds__(NT) void glu_kernel(const float* a, int lda, const 
             v[0] = *p;
         }
     };
+    float xb[V], yb[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) y[e] = xb[e] = yb[e] = 0.f;
     get(a + (long)t * lda + f, x);
-#pragma unroll
-    for (int e = 0; e < V; ++e) y[e] = 0.f;
     if (b) get(b + (long)t * ldb + f, y);
+    if (ba) get(ba + f, xb);
+    if (bb) get(bb + f, yb);
 #pragma unroll
-    for (int e = 0; e < V; ++e)
-        r[e] = glu_one(x[e] + (ba ? ba[f + e] : 0.f), y[e] + (bb ? bb[f + e] : 0.f), fac, act, limit, alpha);
+    for (int e = 0; e < V; ++e) r[e] = glu_one(x[e] + xb[e], y[e] + yb[e], fac, act, limit, alpha);
     put(r);
 }
 
@@ -843,9 +846,10 @@ extern "C" int mxh_glu(const float* a, int lda, const float* b, int ldb, const f
     MXH_CHECK(act == 2 || act == 4 ? !b : (b && ldb >= F));  // the squared ReLU and the plain gelu have one operand
     MXH_CHECK(!scale || (F % group == 0 && lds >= F / group));
     const bool four = (long)T * F >= 1 << 20 && F % 4 == 0 && group % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0 && ldo % 4 == 0 &&
-                      ((uintptr_t)a | (uintptr_t)b | (uintptr_t)out) % 16 == 0;
+                      ((uintptr_t)a | (uintptr_t)b | (uintptr_t)ba | (uintptr_t)bb | (uintptr_t)out) % 16 == 0;
+    MXH_CHECK((long)T * ((F + NT - 1) / NT) <= 0x7fffffff);
 #define GO(B, V)                                                                                                      \
-    glu_kernel<B, V><<<dim3(T, (F + NT * V - 1) / (NT * V)), NT, 0, st>>>(a, lda, b, ldb, ba, bb, scale, lds, group, \
+    glu_kernel<B, V><<<(unsigned)((long)T * ((F + NT * V - 1) / (NT * V))), NT, 0, st>>>(a, lda, b, ldb, ba, bb, scale, lds, group, \
                                                                          scale_sigmoid, out, ldo, F, act, limit, alpha)
     if (o16 && four) GO(true, 4);
     else if (o16) GO(true, 1);
