@@ -217,12 +217,16 @@ __global__ __launch_bounds__(1024) void scale_add_norm_kernel(const float* y, in
     }
 }
 
-// grid (T, H + G + Gv), one wave per (token, head): query heads, then key heads, then the Gv value heads. Element
-// e < rot_dims of a query / key head turns with its neighbour e ^ 1 by angle pos * base^(-(e / 2) * 2 / rot_dims); with
-// `half` the pairs are (i, i + rot_dims / 2) instead and pair i turns by pos * base^(-i * 2 / rot_dims). Given `freqs`
+// grid (T, groups of HPW heads), one wave a group: query heads, then key heads, then (groups of their own) the Gv value heads.
+// Many rows take eight heads a wave, which share the angles' sines and cosines, and ask for all their numbers before the first is
+// waited for (1990 rows of 40 + 8 heads of 128, 73 MB: 52 us with one head a wave and its numbers one by one, 28 so). Below 32768 heads
+// a group of eight would leave the chip under four waves a SIMD: one head a wave; heads of more than 128 numbers have no registers
+// for eight. Element e < rot_dims of a query / key head turns with its neighbour e ^ 1 by angle
+// pos * base^(-(e / 2) * 2 / rot_dims); with `half` the pairs are (i, i + rot_dims / 2) instead and pair i turns by pos * base^(-i * 2 / rot_dims). Given `freqs`
 // (one per pair) pair i turns by pos * freqs[i]; sine and cosine are multiplied by mag. qb, kb, vb: projection biases.
 constexpr int HEAD_E = 8;  // elements per lane: heads of up to 512 numbers
-template <bool Q16, bool C16>
+// E: elements per lane of this instance (2: heads of up to 128), HPW: heads of a wave
+template <bool Q16, bool C16, int E, int HPW>
 __global__ __launch_bounds__(64) void rope_norm_append_kernel(const float* qi, const float* ki, const float* vi,
                                                               int ldq, int ldk, int ldv, const int* positions, int H,
                                                               int G, int dk, int dv, int rot, float neg_log_base,
@@ -231,65 +235,95 @@ __global__ __launch_bounds__(64) void rope_norm_append_kernel(const float* qi, c
                                                               const float* kw, float temp_coef, int temp_every,
                                                               int half, int Gv, const float* freqs, float mag,
                                                               const float* qb, const float* kb, const float* vb) {
-    const int t = blockIdx.x, u = blockIdx.y, lane = threadIdx.x;
-    if (u >= H + G) {  // value head: plain copy into the pool
+    const int t = blockIdx.x, lane = threadIdx.x, rotated = (H + G + HPW - 1) / HPW;
+    if ((int)blockIdx.y >= rotated) {  // value heads: plain copies into the pool
         const int sl = slots[t];
         if (sl < 0) return;
-        const int g = u - H - G;
-        const float* src = vi + (long)t * ldv + (long)g * dv;
-        const long dst = ((long)sl * Gv + g) * dv;
-        for (int e = lane; e < dv; e += 64) st_elem<C16>(vc, dst + e, src[e] + (vb ? vb[g * dv + e] : 0.f));
+        const int g0 = (blockIdx.y - rotated) * HPW;
+        for (int g = g0; g < min(g0 + HPW, Gv); ++g) {
+            const float* src = vi + (long)t * ldv + (long)g * dv;
+            const long dst = ((long)sl * Gv + g) * dv;
+            for (int e = lane; e < dv; e += 64) st_elem<C16>(vc, dst + e, src[e] + (vb ? vb[g * dv + e] : 0.f));
+        }
         return;
     }
-    const bool isq = u < H;
-    const int hd = isq ? u : u - H;
-    int sl = 0;
-    if (!isq) {
-        sl = slots[t];
-        if (sl < 0) return;
-    }
-    const float* src = isq ? qi + (long)t * ldq + (long)hd * dk : ki + (long)t * ldk + (long)hd * dk;
-    const float* hb = isq ? qb : kb;
-    if (hb) hb += (long)hd * dk;
+    const int u0 = blockIdx.y * HPW, u1 = min(u0 + HPW, H + G), n2 = rot >> 1;
+    const int sl = u1 > H ? slots[t] : 0;
     const float pos = (float)positions[t];
-    float val[HEAD_E];
-    float ss = 0.f;
+    auto own = [&](int k) { return min(lane + k * 64, dk - 1); };  // (numbers past the head: its last one, worth nothing)
+    int mate[E];
+    bool second[E];  // the pair's second member turns as v cos + u sin
 #pragma unroll
-    for (int k = 0; k < HEAD_E; ++k) {
-        const int e = lane + k * 64;
-        float v = 0.f;
-        if (e < dk) {
-            v = src[e] + (hb ? hb[e] : 0.f);
-            if (e < rot) {
-                const int n2 = rot >> 1;
-                const bool second = half ? e >= n2 : (e & 1);  // the pair's second member turns as v cos + u sin
-                const int mate = half ? (second ? e - n2 : e + n2) : (e ^ 1);
-                const int pi = half ? (second ? e - n2 : e) : (e >> 1);
-                const float other = src[mate] + (hb ? hb[mate] : 0.f);
-                const float f = freqs ? freqs[pi] : expf((float)pi * (2.f / (float)rot) * neg_log_base);
-                float s, c;
-                sincosf(pos * f, &s, &c);
-                s *= mag;
-                c *= mag;
-                v = second ? v * c + other * s : v * c - other * s;
+    for (int k = 0; k < E; ++k) {
+        const int e = own(k);
+        second[k] = half ? e >= n2 : (e & 1);
+        mate[k] = e < rot ? half ? (second[k] ? e - n2 : e + n2) : (e ^ 1) : e;
+    }
+    // every head's numbers are asked for before the first is waited for
+    float val[HPW][E], other[HPW][E];
+#pragma unroll
+    for (int i = 0; i < HPW; ++i) {
+        const int u = min(u0 + i, u1 - 1), hd = u < H ? u : u - H;
+        const float* src = u < H ? qi + (long)t * ldq + (long)hd * dk : ki + (long)t * ldk + (long)hd * dk;
+#pragma unroll
+        for (int k = 0; k < E; ++k) {
+            val[i][k] = src[own(k)];
+            other[i][k] = src[mate[k]];
+        }
+        const float* hb = u < H ? qb : kb;
+        if (hb) {
+            hb += (long)hd * dk;
+#pragma unroll
+            for (int k = 0; k < E; ++k) {
+                val[i][k] += hb[own(k)];
+                other[i][k] += hb[mate[k]];
             }
         }
-        val[k] = v;
-        ss += v * v;
     }
-    float sc = 1.f;
-    if (norm) sc = 1.f / sqrtf(wave_sum(ss) / (float)dk + eps);
-    // the head norm's weight (shared by the heads) and, for queries, the temperature of the position
-    const float* hw = isq ? qw : kw;
-    if (isq && temp_coef != 0.f) sc *= 1.f + temp_coef * logf((float)((positions[t] + 1) / temp_every + 1));
-    const long dst = isq ? (long)t * ldqo + (long)hd * dk : ((long)sl * G + hd) * dk;
+    float sn[E], cs[E];
 #pragma unroll
-    for (int k = 0; k < HEAD_E; ++k) {
+    for (int k = 0; k < E; ++k) {
         const int e = lane + k * 64;
-        if (e < dk) {
-            const float v = hw ? val[k] * sc * hw[e] : val[k] * sc;
-            if (isq) st_elem<Q16>(qo, dst + e, v);
-            else st_elem<C16>(kc, dst + e, v);
+        sn[k] = 0.f;
+        cs[k] = 1.f;
+        if (e < rot) {
+            const int pi = half ? (second[k] ? e - n2 : e) : (e >> 1);
+            const float f = freqs ? freqs[pi] : expf((float)pi * (2.f / (float)rot) * neg_log_base);
+            float s, c;
+            sincosf(pos * f, &s, &c);
+            sn[k] = s * mag;
+            cs[k] = c * mag;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < HPW; ++i) {
+        const int u = u0 + i;
+        const bool isq = u < H;
+        if (u >= u1 || (!isq && sl < 0)) break;
+        float ss = 0.f;
+#pragma unroll
+        for (int k = 0; k < E; ++k) {
+            const int e = lane + k * 64;
+            float v = val[i][k];
+            if (e < rot) v = second[k] ? v * cs[k] + other[i][k] * sn[k] : v * cs[k] - other[i][k] * sn[k];
+            if (e >= dk) v = 0.f;
+            val[i][k] = v;
+            ss += v * v;
+        }
+        float sc = 1.f;
+        if (norm) sc = 1.f / sqrtf(wave_sum(ss) / (float)dk + eps);
+        // the head norm's weight (shared by the heads) and, for queries, the temperature of the position
+        const float* hw = isq ? qw : kw;
+        if (isq && temp_coef != 0.f) sc *= 1.f + temp_coef * logf((float)((positions[t] + 1) / temp_every + 1));
+        const long dst = isq ? (long)t * ldqo + (long)u * dk : ((long)sl * G + u - H) * dk;
+#pragma unroll
+        for (int k = 0; k < E; ++k) {
+            const int e = lane + k * 64;
+            if (e < dk) {
+                const float v = hw ? val[i][k] * sc * hw[e] : val[i][k] * sc;
+                if (isq) st_elem<Q16>(qo, dst + e, v);
+                else st_elem<C16>(kc, dst + e, v);
+            }
         }
     }
 }
@@ -748,17 +782,23 @@ extern "C" int mxh_rope_norm_append(const float* qi, const float* ki, const floa
     MXH_CHECK(H > 0 && G >= 0 && Gv >= 0 && (G > 0) == (Gv > 0) && dk > 0 && dv > 0 && dk <= 64 * HEAD_E && rot >= 0 &&
               rot <= dk && rot % 2 == 0);
     MXH_CHECK(ldq >= H * dk && ldk >= G * dk && ldv >= Gv * dv && ldqo >= H * dk && base > 0.f && H + G + Gv <= 65535);
-    const dim3 grid(T, H + G + Gv);
     const float nlb = -logf(base);
-#define GO(Q, C)                                                                                                   \
-    rope_norm_append_kernel<Q, C><<<grid, 64, 0, st>>>(qi, ki, vi, ldq, ldk, ldv, positions, H, G, dk, dv, rot, nlb, \
-                                                       norm, eps, qo, ldqo, kc, vc, slots, qw, kw, temp_coef, temp_every, \
-                                                       half, Gv, freqs, mag, qb, kb, vb)
+#define GO3(Q, C, E, P)                                                                                                          \
+    rope_norm_append_kernel<Q, C, E, P><<<dim3(T, (H + G + P - 1) / P + (Gv + P - 1) / P), 64, 0, st>>>(                       \
+        qi, ki, vi, ldq, ldk, ldv, positions, H, G, dk, dv, rot, nlb, norm, eps, qo, ldqo, kc, vc, slots, qw, kw, temp_coef, temp_every, \
+        half, Gv, freqs, mag, qb, kb, vb)
+#define GO(Q, C)                                                          \
+    do {                                                                  \
+        if (dk > 128) GO3(Q, C, HEAD_E, 1);                               \
+        else if ((long)T * (H + G + Gv) >= 32768) GO3(Q, C, 2, 8);        \
+        else GO3(Q, C, 2, 1);                                             \
+    } while (0)
     if (q16 && c16) GO(true, true);
     else if (q16) GO(true, false);
     else if (c16) GO(false, true);
     else GO(false, false);
 #undef GO
+#undef GO3
     return (int)hipGetLastError();
 }
 

@@ -135,6 +135,26 @@ def test_glu_of_many_elements(act):
             assert ((got["cuda"] - got["cpu"]).abs() <= tol * got["cpu"].abs().clamp_min(1)).all()
 
 
+@pytest.mark.parametrize("H,G,Gv,dk,dv,rot,half", [(18, 3, 3, 64, 40, 64, False), (9, 8, 7, 100, 64, 36, True), (24, 0, 0, 32, 32, 0, False)])
+def test_rotary_rows_of_many_heads(H, G, Gv, dk, dv, rot, half):
+    """Steps of 32768 heads and more take eight heads a wave: head counts that leave a group part empty or mix queries with keys, partial
+    rotation, rows without a slot. fp32 angles of positions below 3000 differ from fp32 of another order by 3000 * 2^-23 = 4e-4."""
+    T, g = 1367, torch.Generator().manual_seed(H)
+    q, k, v = torch.randn(T, H * dk, generator=g), torch.randn(T, max(G, 1) * dk, generator=g), torch.randn(T, max(Gv, 1) * dv, generator=g)
+    pos = torch.randint(0, 3000, (T,), generator=g, dtype=torch.int32)
+    slots = torch.randperm(T + 8, generator=g)[:T].to(torch.int32)
+    slots[::7] = -1
+    got = {}
+    for dev in ("cpu", "cuda"):
+        qo = torch.zeros(T, H * dk, device=dev)
+        kc, vc = torch.zeros(T + 8, 1, max(G, 1) * dk, device=dev), torch.zeros(T + 8, 1, max(Gv, 1) * dv, device=dev)
+        HY.rope_norm_append(q.to(dev), k.to(dev) if G else None, v.to(dev) if G else None, pos.to(dev), H, G, dk, dv, rot, 1e4, True, 1e-6, qo,
+                            kc if G else None, vc if G else None, slots.to(dev), half=half, v_heads=Gv, q_temp=(0.1, 100))
+        got[dev] = [t.cpu() for t in (qo, kc, vc)]
+    for a, b in zip(got["cuda"], got["cpu"]):
+        assert (a - b).abs().max() <= 1e-3 * max(1.0, float(b.abs().max()))
+
+
 @pytest.mark.parametrize("chunk,window", [(0, 0), (128, 0), (0, 40)])
 def test_chunks_of_many_sequences(chunk, window):
     """The chunks of a step are launched sixteen at a time, the longest first: eighteen sequences (with short ones between, which run on
