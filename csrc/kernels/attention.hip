@@ -335,6 +335,12 @@ MX_DEV int v_lds_off(int p, int nt) {
 // caches widened load by load: bf16 B=128 ctx 65-1021 53.1 -> 49.2 us at 512-key partitions (44.9 at 1024: 4.1 TB/s), B=9 ctx
 // 3001-24001 95 -> 85; q8_0 B=9 155 -> 64 us (3.2 TB/s), fp8 147 -> 59, q4_0 151 -> 60 (1.8 TB/s, bound by the widening's
 // vector work). Three waves per SIMD instead of two gave the quantised caches 73 -> 64 of that.
+// A key's pool row is worked out once, by one lane, and passed to the lanes that load its numbers (a division by the page size for
+// each of a lane's ten loads was half of a bf16 tile's vector instructions), masks and score caps stand in branches of their own:
+// 480 -> 250 vector instructions a bf16 tile, 700 -> 600 in q8_0 (320 of them the widening), 570 -> 370 in fp8. With the merge launch:
+// 128 rows of 65-1021 keys in one partition 43.1 -> 41.8 us (bf16), 31.6 -> 30.2 (q8_0), 27.1 -> 25.3 (fp8); 9 rows of 3001-24001 in
+// partitions of 256 q8_0 63.8 -> 62.4, fp8 57.4 -> 55.9, 32 rows of 97-4003 fp8 29.9 -> 28.6, bf16 39.6 -> 40.0 (the first tile's
+// rows take one hop more).
 // Occupancy, not register double buffering, hides HBM latency: 8 KB of LDS per wave lets 4
 // workgroups (16 waves) share a CU, each with one tile's 16 KB of K/V loads in flight.
 template <int D>
@@ -498,41 +504,36 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
     // issue order (LDS-DMA completions are not ordered against plain loads).
     constexpr bool PF = DPF && !KV8 && !TS && NW <= 8;  // (16-wave form: 128 VGPRs, no room for a second K tile)
     constexpr int NK = 2 * (D / 32);
-    auto load_k = [&](int kt, bf16x8(&kf_)[2][D / 32]) {
+    // lane l holds the pool row of the tile's key l % 32 (past the end: the last key's, P = 0 there); the lanes that load a key's
+    // numbers fetch its row from that lane: one division by the page size a tile
+    auto rows_of = [&](int kt) {
+        const unsigned key = min(kt + (lane & 31), p1 - 1), bi = key / (unsigned)bs;
+        return ((unsigned)sbt[bi - blk0] * Hkv + kvh) * bs + (key - bi * bs);
+    };
+    auto row_at = [&](unsigned rows, int key) { return (size_t)(unsigned)__builtin_amdgcn_ds_bpermute(4 * key, (int)rows); };
+    auto load_k = [&](unsigned rows, bf16x8(&kf_)[2][D / 32]) {
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            const int key = kt + 16 * t + col;
-            const bool ok = key < p1;
-            const int kk = (PF || ok) ? (ok ? key : kt) : 0;
-            const size_t eo = (PF || ok) ? (((size_t)sbt[kk / bs - blk0] * Hkv + kvh) * bs + kk % bs) * D : 0;
+            const char* r = kc + (row_at(rows, 16 * t + col) * D + 8 * g) * ES;
 #pragma unroll
-            for (int ks = 0; ks < D / 32; ++ks) {
-                if constexpr (PF) {
-                    const bf16x8 w = *(const bf16x8*)(kc + (eo + 32 * ks + 8 * g) * ES);
-                    kf_[t][ks] = ok ? w : (bf16x8){};
-                } else {
-                    kf_[t][ks] = ok ? *(const bf16x8*)(kc + (eo + 32 * ks + 8 * g) * ES) : (bf16x8){};
-                }
-            }
+            for (int ks = 0; ks < D / 32; ++ks) kf_[t][ks] = *(const bf16x8*)(r + 32 * ks * ES);
         }
     };
     // 8-bit and block-quantised caches: a tile's bytes wait in registers (keys past the end: the last one again, P = 0)
     [[maybe_unused]] DecRaw<KVF, D> raw;
-    auto load_raw = [&](int kt) {
-        auto row_of = [&](int key) {
-            const int kk = min(key, p1 - 1), bi = kk / bs;
-            return ((size_t)sbt[bi - blk0] * Hkv + kvh) * bs + (kk - bi * bs);
-        };
+    auto load_raw = [&](unsigned rows) {
 #pragma unroll
-        for (int t = 0; t < 2; ++t) raw.load_k(t, kc, row_of(kt + 16 * t + col), g);
-        raw.load_v(vc, row_of(kt + (lane >> 1)), lane & 1);
+        for (int t = 0; t < 2; ++t) raw.load_k(t, kc, row_at(rows, 16 * t + col), g);
+        raw.load_v(vc, row_at(rows, lane >> 1), lane & 1);
     };
+    unsigned rows = 0;  // of the tile whose loads come next
+    if (p_start + wave * KT < p1) rows = rows_of(p_start + wave * KT);
     if constexpr (KV8) {
-        if (p_start + wave * KT < p1) load_raw(p_start + wave * KT);
+        if (p_start + wave * KT < p1) load_raw(rows);
     }
     [[maybe_unused]] bf16x8 knext[2][D / 32];
     if constexpr (PF) {
-        if (p_start + wave * KT < p1) load_k(p_start + wave * KT, knext);
+        if (p_start + wave * KT < p1) load_k(rows, knext);
     }
     for (int kt0 = p_start + wave * KT; kt0 < p1; kt0 += NW * KT) {
         // ---- the tile's K fragments (PF: requested during the previous tile) and V chunk loads ----
@@ -548,7 +549,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
                 for (int ks = 0; ks < D / 32; ++ks) kf[t][ks] = raw.k(t, ks, g);
         } else {
-            load_k(kt0, kf);
+            load_k(rows, kf);
         }
         // V: bf16 caches go HBM -> LDS by DMA (global_load_lds, no VGPR staging): instruction j fills
         // bytes [1024 j, 1024 j + 1024) of the slice linearly by lane, so each lane fetches the chunk
@@ -560,7 +561,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
                 const int p = lane >> 1, c = (lane & 1) * (D / 16) + j;
                 *(uint4*)(v_lds + v_lds_off<D>(p, c >> 1) + 16 * (c & 1)) = raw.v(j);
             }
-            if (kt0 + NW * KT < p1) load_raw(kt0 + NW * KT);
+            if (kt0 + NW * KT < p1) load_raw(rows_of(kt0 + NW * KT));
         }
 #pragma unroll
         for (int j = 0; j < (KV8 ? 0 : NVC); ++j) {
@@ -570,16 +571,13 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
                 p = id / (D / 8);
                 c = id % (D / 8);
             } else {
-                const int X = 1024 * j + 16 * lane;  // slot in the V image
-                p = X / (D * 2);
-                const int o = X % (D * 2);
-                int sv;
-                if constexpr (D == 128) sv = (p & 3) | (((p >> 3) & 1) << 2);
-                else sv = ((p >> 1) & 1) | (((p >> 3) & 1) << 1);
-                c = 2 * ((o >> 5) ^ sv) + ((o >> 4) & 1);
+                // slot 1024 j + 16 lane of the V image
+                constexpr int CPR = D / 8;  // chunks a row
+                const int sv = D == 128 ? (lane / CPR) & 3 : (lane / CPR) >> 1 & 1;
+                p = 512 / D * j + lane / CPR;
+                c = (2 * ((lane % CPR >> 1) ^ sv) + (lane & 1)) ^ (D == 128 ? (j >> 1 & 1) * 8 : (j & 1) * 4);
             }
-            const int key = kt0 + p < p1 ? kt0 + p : kt0;  // past the end: a valid row (P = 0 there)
-            const size_t eo = (((size_t)sbt[key / bs - blk0] * Hkv + kvh) * bs + key % bs) * D + c * 8;
+            const size_t eo = row_at(rows, p) * D + c * 8;
             if constexpr (PF) {
                 vv[j] = *(const uint4*)(vc + eo * ES);  // rows past the end: a valid row, P = 0 there
             } else {
@@ -589,11 +587,13 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
         [[maybe_unused]] const bool more = kt0 + NW * KT < p1;  // wave-uniform
         if constexpr (PF) {
             __builtin_amdgcn_sched_barrier(0);
-            if (more) load_k(kt0 + NW * KT, knext);
+            if (more) load_k(rows = rows_of(kt0 + NW * KT), knext);
             __builtin_amdgcn_sched_barrier(0);
             // this tile's K (issued before its V DMAs and the next tile's K) has landed
             if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NVC + NK) : "memory");
             else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NVC) : "memory");
+        } else if constexpr (!KV8) {
+            if (more) rows = rows_of(kt0 + NW * KT);
         }
         // ---- S^T = K Q^T: 2 x 16 keys x 16 head columns; a lane holds keys 16 t + 4 g + i of head `col` ----
         f32x4 sacc[2];
@@ -616,19 +616,29 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
         }
         // ---- online softmax over the tile: the head's maximum over its four lanes, everything else lane-local ----
         float mx = -INFINITY;
+        if (softcap > 0.f) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sacc[t][i] = sc_l2 * tanhf(sacc[t][i] * qs * sc_inv);
+        } else {
+#pragma unroll
+            for (int t = 0; t < 2; ++t) sacc[t] *= qs;
+        }
+        if (kt0 + KT > p1) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (kt0 + 16 * t + 4 * g + i >= p1) sacc[t][i] = -INFINITY;
+        }
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float v = sacc[t][i] * qs;
-                if (softcap > 0.f) v = sc_l2 * tanhf(v * sc_inv);
-                if (kt0 + 16 * t + 4 * g + i >= p1) v = -INFINITY;
-                sacc[t][i] = v;
-                mx = fmaxf(mx, v);
-            }
+            for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sacc[t][i]);
         const float mn = fmaxf(mrow, quarters_max(mx));
         if (__any(mn > mrow)) {
-            const float alpha = mn == -INFINITY ? 1.f : exp2f(mrow - mn);
+            const float alpha = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(mrow - mn);
             lrow *= alpha;
 #pragma unroll
             for (int nt = 0; nt < D / 16; ++nt)
@@ -642,7 +652,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
             float pv[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                pv[i] = mn == -INFINITY ? 0.f : exp2f(sacc[t][i] - mn);
+                pv[i] = mn == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(sacc[t][i] - mn);
                 lrow += pv[i];
             }
             pw[2 * t] = pack_bf16x2(pv[0], pv[1]);

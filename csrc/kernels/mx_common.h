@@ -189,14 +189,13 @@ MX_DEV void kv_unpack8(const V& w, float (&f)[8]) {
         }
     }
 }
-// 8 fp8 -> 8 bf16 (exact: e4m3 values are representable in bf16)
+// 8 fp8 -> 8 bf16 (exact: e4m3 values are representable in bf16): one conversion a pair, where conversion to floats and their
+// upper halves took three instructions
 MX_DEV uint4 fp8x8_to_bf16x8(uint2 w) {
-    float f[8];
-    kv_unpack8<true>(u32x2{w.x, w.y}, f);
-    uint32_t o[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) o[j] = (__float_as_uint(f[2 * j]) >> 16) | (__float_as_uint(f[2 * j + 1]) & 0xFFFF0000u);
-    return make_uint4(o[0], o[1], o[2], o[3]);
+    const auto two = [](uint32_t x, auto hi) {
+        return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(x, 1.f, decltype(hi)::value));
+    };
+    return make_uint4(two(w.x, std::false_type()), two(w.x, std::true_type()), two(w.y, std::false_type()), two(w.y, std::true_type()));
 }
 
 // gate activation of the fused gated-FFN epilogues: EPI 3 = SwiGLU (silu), EPI 4 = GeGLU (gelu tanh)
