@@ -1,6 +1,7 @@
 // kvq.hip — quantise staged K / V rows into a block-quantised paged KV cache (kvq.h layout).
 //
-// The RoPE / KV-append writers (rope_kv.hip, the batch-1 qmv1 epilogue) write a quantised cache's new rows as bf16
+// The RoPE / KV-append writers (rope_kv.hip but for q8_0 rows of wholly rotated heads, which it quantises itself; the batch-1 qmv1
+// epilogue) write a quantised cache's new rows as bf16
 // into a per-step staging buffer [T, Hkv, D] (identity slots, block size 1); this kernel then quantises each 32-element
 // block with llama.cpp's reference quantisers (quantize_row_q8_0/q4_0/q4_1/q5_0/q5_1_ref; iq4_nl as ggml-cuda's
 // cpy_blck_f32_iq4_nl: nearest codebook entry at d = vmax / -127, then the weighted least-squares refit of d) and

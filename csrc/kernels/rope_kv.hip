@@ -1,4 +1,4 @@
-// rope_kv.hip — fused bias + RoPE + paged KV-cache append (K8 + K10 of SURVEY §2.6).
+// rope_kv.hip — fused bias + RoPE + paged KV-cache append.
 //
 // Consumes the fp32 QKV projection of T tokens ([T, (Hq + 2*Hkv) * D], written by the qgemm/qgemv
 // F32 epilogue), applies the optional QKV bias (Qwen2), rotates Q and K, writes Q as bf16 for the
@@ -11,7 +11,7 @@
 // QKN (Qwen3): per-head RMSNorm of every q and k head (weights qn / kn over head_dim) applied
 // after the bias and before the rotation — one wave per head computes the head's rms into LDS,
 // so the normalisation costs one extra read of the row instead of a separate kernel.
-#include "mx_common.h"
+#include "kvq.h"
 
 // Grid (T, NG): workgroup (t, g) handles heads [g*HPG, (g+1)*HPG) of the Hq+Hkv rotated heads and
 // its share of the Hkv V heads, so short decode batches still spread over the CUs. ZERO: after
@@ -115,7 +115,10 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(float* __restrict__ qkv, c
 // divisions. QKN (Qwen3 / Gemma-3 per-head RMSNorm of q and k before the rotation): a head's UPH threads are
 // consecutive lanes of one wave, so its sum of squares is a UPH-lane shuffle reduction of the values already in
 // registers (no LDS pass, no second read of the row).
-template <int D, bool NEOX, bool HAS_BIAS, bool ZERO, bool KV8, bool QKN = false>
+// KVF_Q8_0: eight consecutive lanes hold a block of 32, rounded to bf16 as the staged rows of the other block formats are, and store its
+// codes themselves: the rows' trip through a staging buffer was a second launch a layer (and one for its slots), 584 -> 559 us for a
+// four-layer step of 9 rows.
+template <int D, bool NEOX, bool HAS_BIAS, bool ZERO, int KVF, bool QKN = false>
 __global__ __launch_bounds__(256) void rope_kv4_kernel(float* __restrict__ qkv, const float* __restrict__ bias,
                                                        const int* __restrict__ pos, const int* __restrict__ slots,
                                                        const float* __restrict__ inv_freq, float attn_factor, int Hq,
@@ -162,19 +165,33 @@ __global__ __launch_bounds__(256) void rope_kv4_kernel(float* __restrict__ qkv, 
     __syncthreads();
     const int slot = slots[t];
     const int blk = slot >= 0 ? slot / block_size : 0, off = slot >= 0 ? slot % block_size : 0;
+    auto put = [&](void* pool, int kh, int d, float4 y) {
+        const size_t r = ((size_t)blk * Hkv + kh) * block_size + off;
+        if constexpr (KVF == KVF_Q8_0) {
+            using Q = KVQ<KVF_Q8_0, D>;
+            uint8_t* q = (uint8_t*)pool + r * Q::ROWB;
+            const float x[4] = {bf16_to_f32(f32_to_bf16(y.x)), bf16_to_f32(f32_to_bf16(y.y)), bf16_to_f32(f32_to_bf16(y.z)),
+                                bf16_to_f32(f32_to_bf16(y.w))};
+            const float dd = group_max<8>(fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])))) / 127.f;
+            const float inv = dd ? 1.f / dd : 0.f;
+            uint32_t w = 0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) w |= ((uint32_t)(int)roundf(x[i] * inv) & 0xFF) << (8 * i);
+            *(uint32_t*)(q + d) = w;
+            if (d % 32 == 0) *(_Float16*)(q + Q::CB + d / 16) = (_Float16)dd;
+        } else if constexpr (KVF == KVF_FP8) {
+            uint8_t* q = (uint8_t*)pool + r * D + d;
+            q[0] = f32_to_fp8(y.x); q[1] = f32_to_fp8(y.y); q[2] = f32_to_fp8(y.z); q[3] = f32_to_fp8(y.w);
+        } else {
+            *(uint2*)((bf16_t*)pool + r * D + d) = make_uint2(pack_bf16x2(y.x, y.y), pack_bf16x2(y.z, y.w));
+        }
+    };
     auto st4 = [&](int h, int d, float4 y) {
         if (h < Hq) {
             uint2 o = {pack_bf16x2(y.x, y.y), pack_bf16x2(y.z, y.w)};
             *(uint2*)(qo + ((size_t)t * Hq + h) * D + d) = o;
         } else if (slot >= 0) {
-            const size_t e = (((size_t)blk * Hkv + (h - Hq)) * block_size + off) * D + d;
-            if constexpr (KV8) {
-                ((uint8_t*)kc)[e] = f32_to_fp8(y.x); ((uint8_t*)kc)[e + 1] = f32_to_fp8(y.y);
-                ((uint8_t*)kc)[e + 2] = f32_to_fp8(y.z); ((uint8_t*)kc)[e + 3] = f32_to_fp8(y.w);
-            } else {
-                uint2 o = {pack_bf16x2(y.x, y.y), pack_bf16x2(y.z, y.w)};
-                *(uint2*)((bf16_t*)kc + e) = o;
-            }
+            put(kc, h - Hq, d, y);
         }
     };
     const float4 z4 = {0.f, 0.f, 0.f, 0.f};
@@ -232,14 +249,7 @@ __global__ __launch_bounds__(256) void rope_kv4_kernel(float* __restrict__ qkv, 
                 const float4 b = *(const float4*)(bias + (Hq + Hkv) * D + kh * D + d);
                 v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w;
             }
-            const size_t e = (((size_t)blk * Hkv + kh) * block_size + off) * D + d;
-            if constexpr (KV8) {
-                ((uint8_t*)vc)[e] = f32_to_fp8(v.x); ((uint8_t*)vc)[e + 1] = f32_to_fp8(v.y);
-                ((uint8_t*)vc)[e + 2] = f32_to_fp8(v.z); ((uint8_t*)vc)[e + 3] = f32_to_fp8(v.w);
-            } else {
-                uint2 o = {pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w)};
-                *(uint2*)((bf16_t*)vc + e) = o;
-            }
+            put(vc, kh, d, v);
         }
         if constexpr (ZERO) *(float4*)(vr + kh * D + d) = z4;
     }
@@ -248,9 +258,9 @@ __global__ __launch_bounds__(256) void rope_kv4_kernel(float* __restrict__ qkv, 
 extern "C" int mxk_rope_kv(float* qkv, const float* bias, const int* pos, const int* slots,
                            const float* inv_freq, float attn_factor, int T, int Hq, int Hkv, int D, int rot_dim,
                            int neox, bf16_t* qo, void* kc, void* vc, int block_size, const float* qn,
-                           const float* kn, float eps, int zero_after, int kv_fp8, hipStream_t st) {
+                           const float* kn, float eps, int zero_after, int kvf, hipStream_t st) {
     if (T <= 0) return 0;
-    if (rot_dim > 512 || (rot_dim & 1) || D & 1) return (int)hipErrorInvalidValue;
+    if (rot_dim > 512 || (rot_dim & 1) || D & 1 || kvf < 0 || kvf > KVF_Q8_0) return (int)hipErrorInvalidValue;
     const bool qkn = qn != nullptr && kn != nullptr;
     if (qkn && Hq + Hkv > 256) return (int)hipErrorInvalidValue;
     // enough workgroups for the 256 CUs even at small decode batches, >= 1 head per group
@@ -267,19 +277,26 @@ extern "C" int mxk_rope_kv(float* qkv, const float* bias, const int* pos, const 
         else rope_kv4_kernel<D_, N_, B_, Z_, K8_><<<grid, 256, 0, st>>>(qkv, bias, pos, slots, inv_freq, attn_factor,    \
                                                                         Hq, Hkv, qo, kc, vc, block_size);                \
     } while (0)
-#define RK4Z(D_, N_, B_) { if (zero_after) { if (kv_fp8) RK4(D_, N_, B_, true, true); else RK4(D_, N_, B_, true, false); } \
-                           else { if (kv_fp8) RK4(D_, N_, B_, false, true); else RK4(D_, N_, B_, false, false); } }
+#define RK4F(D_, N_, B_, Z_)                              \
+    {                                                     \
+        if (kvf == KVF_Q8_0) RK4(D_, N_, B_, Z_, KVF_Q8_0); \
+        else if (kvf) RK4(D_, N_, B_, Z_, KVF_FP8);       \
+        else RK4(D_, N_, B_, Z_, KVF_BF16);               \
+    }
+#define RK4Z(D_, N_, B_) { if (zero_after) RK4F(D_, N_, B_, true) else RK4F(D_, N_, B_, false) }
 #define RK4B(D_, N_) { if (bias) RK4Z(D_, N_, true) else RK4Z(D_, N_, false) }
         if (D == 128) { if (neox) RK4B(128, true) else RK4B(128, false) }
         else { if (neox) RK4B(64, true) else RK4B(64, false) }
 #undef RK4B
 #undef RK4Z
+#undef RK4F
 #undef RK4
         MXK_CHECK_LAUNCH();
     }
 #define RKZ(N_, B_, Q_, K8_) { if (zero_after) rope_kv_kernel<N_, B_, Q_, true, K8_><<<grid, 256, 0, st>>>(qkv, bias, pos, slots, inv_freq, attn_factor, Hq, Hkv, D, rot_dim, qo, kc, vc, block_size, qn, kn, eps); \
     else rope_kv_kernel<N_, B_, Q_, false, K8_><<<grid, 256, 0, st>>>(qkv, bias, pos, slots, inv_freq, attn_factor, Hq, Hkv, D, rot_dim, qo, kc, vc, block_size, qn, kn, eps); }
-#define RK(N_, B_, Q_) { if (kv_fp8) RKZ(N_, B_, Q_, true) else RKZ(N_, B_, Q_, false) }
+    if (kvf > KVF_FP8) return (int)hipErrorInvalidValue;
+#define RK(N_, B_, Q_) { if (kvf) RKZ(N_, B_, Q_, true) else RKZ(N_, B_, Q_, false) }
 #define RKQ(N_, B_) { if (qkn) RK(N_, B_, true) else RK(N_, B_, false) }
     if (neox) { if (bias) RKQ(true, true) else RKQ(true, false) }
     else { if (bias) RKQ(false, true) else RKQ(false, false) }

@@ -291,7 +291,9 @@ def rope_kv(qkv: torch.Tensor, bias: torch.Tensor | None, positions: torch.Tenso
                 v_cache[blk, :, off, :] = _to_cache(v[t], v_cache.dtype)
         return
     kvf = kv_format(k_cache)
-    if kvf >= 2:
+    norms = tuple(qk_norm[:2]) if qk_norm else ()
+    whole = rot_dim == D and D in (64, 128) and all(t is None or t.data_ptr() % 16 == 0 for t in (qkv, bias, *norms))
+    if kvf >= 2 and not (kvf == KVF_Q8_0 and whole):  # (q8_0 rows of wholly rotated heads: quantised by the rotation itself)
         # block-quantised cache: the rotated K and V rows go to a bf16 staging buffer [T, Hkv, D] (identity slots,
         # block size 1), then kvq.hip quantises them into their paged slots (one extra launch per layer)
         ks = torch.empty(T, Hkv, D, dtype=torch.bfloat16, device=qkv.device)
@@ -309,17 +311,13 @@ def rope_kv(qkv: torch.Tensor, bias: torch.Tensor | None, positions: torch.Tenso
             float(attn_factor), T, Hq, Hkv, D, rot_dim, int(neox), q_out.data_ptr(), k_cache.data_ptr(),
             v_cache.data_ptr(), block_size, N.ptr(qk_norm[0]) if qk_norm else None,
             N.ptr(qk_norm[1]) if qk_norm else None, float(qk_norm[2]) if qk_norm else 0.0, int(zero_after),
-            int(is_fp8(k_cache)), N.stream_ptr())
+            kvf, N.stream_ptr())
 
 
-from .kvq import kv_format  # noqa: E402  (0 bf16, 1 fp8, 2.. llama.cpp block formats)
+from .kvq import KVF_Q8_0, kv_format  # noqa: E402  (0 bf16, 1 fp8, 2.. llama.cpp block formats)
 
 FP8_KV = torch.float8_e4m3fn  # OCP e4m3: the gfx950 hardware conversion format
 FP8_MAX = 448.0
-
-
-def is_fp8(t: torch.Tensor) -> bool:
-    return t.dtype == FP8_KV
 
 
 def _to_cache(x: torch.Tensor, dtype) -> torch.Tensor:

@@ -132,3 +132,36 @@ def test_engine_gpu_quantised_cache(fmt):
                          max_tokens=16) for i in range(3)]
     assert all(len(o.token_ids) == 16 for o in outs)
     assert eng.kv.k.dtype == torch.uint8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,neox,bias,norm", [(128, False, False, False), (128, True, True, True), (64, False, True, True), (64, True, False, False)])
+@pytest.mark.parametrize("T,Hq,Hkv", [(1, 4, 1), (9, 6, 3), (700, 5, 5)])
+def test_rotation_quantises_q8_0_rows(D, neox, bias, norm, T, Hq, Hkv):
+    """Rotation into a q8_0 cache against rotation into bf16 rows that are then quantised: the same rounding to bf16 and the same codes
+    (a product and sum that the two fuse differently may move a code by one), rows without a slot left alone."""
+    from localai_tfp_amd import _native as N
+    from localai_tfp_amd.ops import core as K
+    f, bs, g = KQ.FORMATS["q8_0"], 16, torch.Generator().manual_seed(T + D)
+    qkv = torch.randn(T, (Hq + 2 * Hkv) * D, generator=g)
+    qkv[0, (Hq + Hkv) * D:(Hq + Hkv) * D + 32] = 0.0  # a block of zeros
+    b = torch.randn((Hq + 2 * Hkv) * D, generator=g).cuda() if bias else None
+    qk = (torch.rand(D, generator=g).cuda() + 0.5, torch.rand(D, generator=g).cuda() + 0.5, 1e-6) if norm else None
+    pos, nb = torch.randint(0, 5000, (T,), generator=g, dtype=torch.int32).cuda(), -(-T // bs) + 1
+    slots = torch.randperm(nb * bs, generator=g)[:T].to(torch.int32)
+    slots[T // 2:T // 2 + T // 8] = -1
+    slots = slots.cuda()
+    inv = (10000.0 ** (-torch.arange(0, D, 2).double() / D)).float().cuda()
+    q = [torch.zeros(T, Hq, D, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    kc, vc, kr, vr = (torch.full((nb, Hkv, bs, KQ.row_bytes(f, D)), 77, dtype=torch.uint8, device="cuda") for _ in range(4))
+    ks, vs = (torch.zeros(T, Hkv, D, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    x = qkv.cuda()
+    K.rope_kv(x, b, pos, slots, inv, 1.0, Hq, Hkv, D, D, neox, q[0], KQ.tag(kc, f), KQ.tag(vc, f), bs, qk_norm=qk, zero_after=True)
+    assert not x.any()
+    K.rope_kv(qkv.cuda(), b, pos, torch.arange(T, dtype=torch.int32, device="cuda"), inv, 1.0, Hq, Hkv, D, D, neox, q[1], ks, vs, 1, qk_norm=qk)
+    N.kcall("mxk_kvq_append", f, ks.data_ptr(), vs.data_ptr(), slots.data_ptr(), T, Hkv, D, bs, kr.data_ptr(), vr.data_ptr(), N.stream_ptr())
+    assert torch.equal(q[0], q[1])
+    for got, want in ((kc, kr), (vc, vr)):
+        codes = (got[..., :D].view(torch.int8).int() - want[..., :D].view(torch.int8).int()).abs()
+        scales = (got[..., D:].contiguous().view(torch.float16).float() - want[..., D:].contiguous().view(torch.float16).float()).abs()
+        assert codes.max() <= 1 and (codes > 0).float().mean() < 0.01 and (scales <= 2 ** -8 * want[..., D:].contiguous().view(torch.float16).float().abs()).all()
