@@ -477,11 +477,10 @@ struct QRope {
 // (ticket `skc[g]`) runs the epilogue on the total, then re-zeroes its workspace columns and ticket (graph replays
 // start clean). Lets the narrow batch-1 projections (qkv parts of 1024-6144 columns: 32-192 column groups) use
 // every CU. SRC_NORM then reads the whole row once more for the norm's sum of squares.
-template <int QT, int EPI, bool F16, int SRC, int NU = 2>
-__global__ __launch_bounds__(64 * QMV_WAVES) void qmv1_kernel(const uint8_t* __restrict__ W, int N, int K,
-                                                              void* __restrict__ Cv, const void* __restrict__ xsrc,
-                                                              const float* __restrict__ nw, float eps, QRope rp,
-                                                              float* __restrict__ skw, unsigned* __restrict__ skc) {
+template <int QT, int EPI, bool F16, int SRC, int NU>
+__device__ __forceinline__ void qmv1_columns(int g, const uint8_t* __restrict__ W, int K, void* __restrict__ Cv,
+                                             const void* __restrict__ xsrc, const float* __restrict__ nw, float eps, const QRope& rp,
+                                             float* __restrict__ skw, unsigned* __restrict__ skc) {
     using U = TUnit<QT>;
     constexpr int NT = 64 * QMV_WAVES;
     constexpr int NP = NU / 2;  // activation passes of 8 elements per thread
@@ -492,7 +491,6 @@ __global__ __launch_bounds__(64 * QMV_WAVES) void qmv1_kernel(const uint8_t* __r
     extern __shared__ __attribute__((aligned(16))) char qmv1_smem[];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int r = lane & 31, h = lane >> 5;
-    const int g = blockIdx.x;
     const int nunit = K / U::ELEMS;  // SRC_NORM: K == 4096 NU (checked by the launcher)
     const int per = (nunit + gridDim.y - 1) / gridDim.y;
     const int u0 = blockIdx.y * per, u1 = min(nunit, u0 + per);
@@ -653,6 +651,27 @@ __global__ __launch_bounds__(64 * QMV_WAVES) void qmv1_kernel(const uint8_t* __r
         else if (gridDim.y > 1) atomicAdd(((float*)Cv) + n, v);
         else ((float*)Cv)[n] += v;
     }
+}
+
+template <int QT, int EPI, bool F16, int SRC, int NU = 2>
+__global__ __launch_bounds__(64 * QMV_WAVES) void qmv1_kernel(const uint8_t* __restrict__ W, int N, int K,
+                                                              void* __restrict__ Cv, const void* __restrict__ xsrc,
+                                                              const float* __restrict__ nw, float eps, QRope rp,
+                                                              float* __restrict__ skw, unsigned* __restrict__ skc) {
+    qmv1_columns<QT, EPI, F16, SRC, NU>(blockIdx.x, W, K, Cv, xsrc, nw, eps, rp, skw, skc);
+}
+
+// The two parts of a q|k|v projection that mixes formats (q|k in one, v in a wider one) in one launch: the parts' 160 + 32 column
+// groups of 4096 x (5120 + 1024) leave the chip idle one after the other (7.6 + 7.6 us, the latency of a workgroup each) and fit
+// it together (8.6 us). The first `groups` workgroups are part a's.
+template <int QTA, int QTB, int NU>
+__global__ __launch_bounds__(64 * QMV_WAVES) void qmv1_rope_pair_kernel(const uint8_t* __restrict__ wa, const uint8_t* __restrict__ wb,
+                                                                        int groups, int K, const float* __restrict__ x,
+                                                                        const float* __restrict__ nw, float eps, QRope ra, QRope rb) {
+    if ((int)blockIdx.x < groups)
+        qmv1_columns<QTA, EPI_ROPEKV, true, SRC_NORM, NU>(blockIdx.x, wa, K, nullptr, x, nw, eps, ra, nullptr, nullptr);
+    else
+        qmv1_columns<QTB, EPI_ROPEKV, true, SRC_NORM, NU>(blockIdx.x - groups, wb, K, nullptr, x, nw, eps, rb, nullptr, nullptr);
 }
 
 // ---- dequantise whole rows (output features) of a t32 weight: embedding gather / debugging ----
@@ -902,6 +921,30 @@ extern "C" int mxk_qmv1_rope(int qtype, const float* x, const float* nw, float e
     }
 #undef QR1
     MXK_CHECK_LAUNCH();
+}
+
+// As mxk_qmv1_rope, unsplit, for two parts of different formats that follow each other in the q|k|v row (columns 0 .. na + nb): the
+// mixes of the K_M files, whose v (or k and v) is kept wider. Other pairs: hipErrorInvalidValue (mxk_qmv1_rope takes a part at a time).
+extern "C" int mxk_qmv1_rope_pair(int qa, int qb, const float* x, const float* nw, float eps, const uint8_t* wa, int na,
+                                  const uint8_t* wb, int nb, int K, const int* pos, const int* slots, const float* inv_freq,
+                                  const float* bias, float attn_factor, int Hq, int Hkv, int D, bf16_t* qo, bf16_t* kc, bf16_t* vc,
+                                  int block_size, hipStream_t st) {
+    if ((K != 4096 && K != 8192) || na <= 0 || nb <= 0 || na % 32 || nb % 32 || (D != 64 && D != 128) || ((uintptr_t)x & 15))
+        return (int)hipErrorInvalidValue;
+    const QRope ra{pos, slots, inv_freq, bias, attn_factor, Hq, Hkv, D, 0, block_size, qo, kc, vc};
+    const QRope rb{pos, slots, inv_freq, bias ? bias + na : nullptr, attn_factor, Hq, Hkv, D, na, block_size, qo, kc, vc};
+    const size_t lds = (size_t)K + K / 32 * sizeof(float2);
+#define QRP(A_, B_)                                                                                                              \
+    if (qa == A_ && qb == B_) {                                                                                                  \
+        if (K == 8192) qmv1_rope_pair_kernel<A_, B_, 4><<<(na + nb) / 32, 64 * QMV_WAVES, lds, st>>>(wa, wb, na / 32, K, x, nw, eps, ra, rb); \
+        else qmv1_rope_pair_kernel<A_, B_, 2><<<(na + nb) / 32, 64 * QMV_WAVES, lds, st>>>(wa, wb, na / 32, K, x, nw, eps, ra, rb);           \
+        MXK_CHECK_LAUNCH();                                                                                                      \
+    }
+    QRP(MXQ_Q4_K, MXQ_Q6_K)
+    QRP(MXQ_Q5_K, MXQ_Q6_K)
+    QRP(MXQ_Q3_K, MXQ_Q5_K)
+#undef QRP
+    return (int)hipErrorInvalidValue;
 }
 
 extern "C" int mxk_qmv1_enable(int on) {

@@ -37,7 +37,7 @@ from ..ops import core as K
 from ..ops import quant as Q
 from ..ops.linear import (ACT_DTYPE, EPI_ADD_F32, EPI_BF16, EPI_F32, EPI_GEGLU, EPI_SWIGLU, QWeight, concat_rows,
                           _fp32_out_ok, dense_min_m, interleave_gate_up, glu_interleaved, qmatmul, qmv_fusable, qmv_rope_ok,
-                          qmv_fused, qmv_rope_fused, NormFuse, norm_fusable)
+                          qmv_fused, qmv_rope_fused, qmv_rope_pair_fused, NormFuse, norm_fusable)
 from ..ops import linear as _LIN
 from ..ops import autotune as _AT
 from ..ops.moe import MoEWeights, moe_ffn
@@ -684,7 +684,8 @@ class LlamaModel:
                 for w in L.qkv_parts:
                     rope_fused = rope_fused and qmv_rope_ok(w, h, q, kc, vc, D, o2)
                     o2 += w.N
-            if rope_fused:
+            if rope_fused and not qmv_rope_pair_fused(L.qkv_parts, h, L.attn_norm, eps, fb.positions, fb.slots, inv_freq, L.bqkv, attn_factor,
+                                                      Hq, Hkv, D, q.view(T, Hq, D), kc, vc, kv.block_size):
                 o2 = 0
                 for w in L.qkv_parts:
                     b = L.bqkv[o2:o2 + w.N] if L.bqkv is not None else None

@@ -573,6 +573,26 @@ def qmv_rope_fused(W: QWeight, x: torch.Tensor, norm: torch.Tensor, eps: float, 
     return True
 
 
+# q|k|v parts whose formats mxk_qmv1_rope_pair is built for (the K_M mixes)
+QMV_ROPE_PAIRS = {(int(QType.Q4_K), int(QType.Q6_K)), (int(QType.Q5_K), int(QType.Q6_K)), (int(QType.Q3_K), int(QType.Q5_K))}
+
+
+def qmv_rope_pair_fused(parts, x: torch.Tensor, norm: torch.Tensor, eps: float, positions, slots, inv_freq: torch.Tensor, bias,
+                        attn_factor: float, Hq: int, Hkv: int, D: int, q_out: torch.Tensor, k_cache: torch.Tensor,
+                        v_cache: torch.Tensor, block_size: int) -> bool:
+    """qmv_rope_fused of a q|k|v projection in two parts of different formats, one launch. False: not applicable, nothing launched."""
+    if len(parts) != 2 or QMV_ROPE_SPLIT or not all(
+            qmv_rope_ok(w, x, q_out, k_cache, v_cache, D, o) for w, o in zip(parts, (0, parts[0].N))):
+        return False
+    a, b = parts
+    if (int(a.qtype), int(b.qtype)) not in QMV_ROPE_PAIRS or a.K != b.K:
+        return False
+    N.kcall("mxk_qmv1_rope_pair", int(a.qtype), int(b.qtype), x.data_ptr(), norm.data_ptr(), float(eps), a.data.data_ptr(), a.N,
+            b.data.data_ptr(), b.N, a.K, positions.data_ptr(), slots.data_ptr(), inv_freq.data_ptr(), N.ptr(bias), float(attn_factor),
+            Hq, Hkv, D, q_out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), block_size, N.stream_ptr())
+    return True
+
+
 def dense_min_m(dtype, epi: int = EPI_ADD_F32, can_split: bool = True) -> int:
     """Smallest M routed to the dense weight cache (hipBLASLt). From tools/bench_qgemm.py +
     tools/tune_qgemm16.py on MI355X (Llama-3-8B shapes): the bf16 dequant-MFMA kernel loses to the

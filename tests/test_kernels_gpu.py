@@ -1065,3 +1065,40 @@ def test_qmv_rope_fused(qt, bias, k, split, monkeypatch):
     touched = torch.zeros(nb, bs, dtype=torch.bool)
     touched[3, 5] = True
     assert float(kc.float().abs().sum(dim=(1, 3)).cpu()[~touched].sum()) == 0.0
+
+
+@pytest.mark.parametrize("qa,qb", [(QType.Q4_K, QType.Q6_K), (QType.Q5_K, QType.Q6_K), (QType.Q3_K, QType.Q5_K), (QType.Q6_K, QType.Q4_K)])
+@pytest.mark.parametrize("k,D,Hq,Hkv,cut", [(4096, 128, 8, 2, 10), (8192, 64, 3, 1, 3), (4096, 64, 1, 1, 2)])
+def test_qmv_rope_pair(qa, qb, k, D, Hq, Hkv, cut):
+    """Two parts of a q|k|v projection in one launch write what a launch each writes, bit for bit; other pairs launch nothing. Odd head
+    counts, v alone or k and v in the second part, a row without a slot."""
+    from localai_tfp_amd.ops.linear import qmv_rope_fused, qmv_rope_pair_fused
+    bs, n, cut = 16, (Hq + 2 * Hkv) * D, cut * D
+    parts = []
+    for qt, rows in ((qa, cut), (qb, n - cut)):
+        W = QWeight.from_ggml(make_w(qt, rows, k, seed=rows)[0], qt, rows, k, DEV, t32=True)
+        assert W.to_t32()
+        parts.append(W)
+    g = torch.Generator().manual_seed(7)
+    h, nw = torch.randn(1, k, generator=g).to(DEV) * 2, (torch.rand(k, generator=g) + 0.5).to(DEV)
+    inv_freq = (1.0 / (500000.0 ** (torch.arange(0, D, 2).float() / D))).to(DEV)
+    pos = torch.tensor([37], dtype=torch.int32, device=DEV)
+    for bias in (None, torch.randn(n, generator=g).to(DEV)):
+        for slot in (3 * bs + 5, -1):
+            slots = torch.tensor([slot], dtype=torch.int32, device=DEV)
+            got = []
+            for pair in (True, False):
+                q, kc, vc = torch.zeros(1, Hq, D, dtype=torch.bfloat16, device=DEV), *torch.zeros(2, 8, Hkv, bs, D, dtype=torch.bfloat16, device=DEV)
+                rest = (pos, slots, inv_freq)
+                if pair:
+                    ok = qmv_rope_pair_fused(parts, h, nw, 1e-5, *rest, bias, 1.0, Hq, Hkv, D, q, kc, vc, bs)
+                    assert ok == ((qa, qb) != (QType.Q6_K, QType.Q4_K))
+                    if not ok:
+                        assert not q.any() and not kc.any() and not vc.any()
+                        return
+                else:
+                    for W, off in zip(parts, (0, cut)):
+                        assert qmv_rope_fused(W, h, nw, 1e-5, off, *rest, bias[off:off + W.N] if bias is not None else None, 1.0, Hq, Hkv, D,
+                                              q, kc, vc, bs)
+                got.append((q, kc, vc))
+            assert all(torch.equal(a, b) for a, b in zip(*got)) and got[0][0].any() and got[0][2].any() == (slot >= 0)
