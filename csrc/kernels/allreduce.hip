@@ -13,7 +13,9 @@
 //    replays correctly with ONE launch per all-reduce; epoch >= 1, the buffers are zeroed at allocation;
 //  * two parity halves: a rank can only start call e+2 (writing parity e%2 again) after it received
 //    every peer's call-e+1 data, which each peer pushes only after finishing its call-e reads;
-//  * spins are bounded: a peer that never arrives sets *err and the kernel exits (the host raises).
+//  * waits are bounded by time (the constant-rate clock): a peer that never arrives sets *err and the kernel exits (the host
+//    raises); later calls find *err set and wait no more. The bound is not a count of polls: a count lasts as long as its
+//    loads do, and a peer whose host is late by less than that, or whose process is not scheduled on a shared GPU, is not dead.
 // Grid: <= 128 workgroups (all resident, so no cross-rank scheduling dependency), grid-stride granules.
 #include "mx_common.h"
 
@@ -29,7 +31,7 @@ template <bool F16, bool RES>
 __global__ __launch_bounds__(256) void allreduce_1shot_kernel(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
                                                               int ng, int rank, int world, MxArPeers peers,
                                                               long slot_granules, uint32_t* epoch_ctr,
-                                                              int* err, float2* __restrict__ res) {
+                                                              int* err, long long wait_ticks, float2* __restrict__ res) {
     const uint32_t epoch = __hip_atomic_load(epoch_ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
     const long par = epoch & 1u;
     const int stride = gridDim.x * blockDim.x;
@@ -44,14 +46,17 @@ __global__ __launch_bounds__(256) void allreduce_1shot_kernel(const uint32_t* __
     // phase 2: gather every rank's granule i from the local receive buffer, sum in fp32
     unsigned long long* local = peers.recv[rank];
     bool dead = false;
+    long long since = -1;  // when this thread first found a granule missing
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < ng && !dead; i += stride) {
         float a = 0.f, b = 0.f;
         for (int p = 0; p < world; ++p) {
             unsigned long long* src = local + (par * world + p) * slot_granules + i;
             unsigned long long g = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            unsigned spins = 0;
-            while ((uint32_t)(g >> 32) != epoch) {
-                if (++spins > (1u << 22)) {  // ~seconds: a dead peer, not a slow one
+            for (unsigned polls = 0; (uint32_t)(g >> 32) != epoch; ++polls) {
+                const long long now = wall_clock64();
+                if (since < 0) since = now;
+                if (now - since > wait_ticks ||
+                    (polls % 64 == 0 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
                     __hip_atomic_fetch_max(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     dead = true;
                     break;
@@ -106,15 +111,20 @@ extern "C" int mxk_ar_ipc_open(const void* handle /* 64 B */, void** ptr) {
 }
 extern "C" int mxk_ar_ipc_close(void* ptr) { return (int)hipIpcCloseMemHandle(ptr); }
 extern "C" int mxk_ar_handle_size() { return (int)sizeof(hipIpcMemHandle_t); }
+// ticks of the clock the waits are bounded by in a millisecond; 0: not known
+extern "C" int mxk_ar_clock_khz(int device) {
+    int khz = 0;
+    return hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) == hipSuccess ? khz : 0;
+}
 
 // in/out: n 16-bit elements (n even, 4-B aligned; out may alias in); peers: world receive-buffer pointers
 // (host array; [rank] = this rank's own buffer); slot_granules >= n / 2; epoch_ctr: 2 device words {epoch,
-// ticket}, zeroed once; err: device word.
+// ticket}, zeroed once; err: device word; wait_ticks: how long a thread waits for its peers, in ticks of mxk_ar_clock_khz.
 extern "C" int mxk_allreduce_1shot(const uint16_t* in, uint16_t* out, int n, int rank, int world,
                                    unsigned long long* const* peers, long slot_granules, uint32_t* epoch_ctr,
-                                   int* err, hipStream_t st) {
+                                   int* err, long long wait_ticks, hipStream_t st) {
     if (n <= 0) return 0;
-    if ((n & 1) || world < 1 || world > MX_AR_MAX_WORLD || rank < 0 || rank >= world || (long)(n / 2) > slot_granules ||
+    if (wait_ticks <= 0 || (n & 1) || world < 1 || world > MX_AR_MAX_WORLD || rank < 0 || rank >= world || (long)(n / 2) > slot_granules ||
         ((uintptr_t)in & 3) || ((uintptr_t)out & 3))
         return (int)hipErrorInvalidValue;
     MxArPeers pp{};
@@ -123,16 +133,16 @@ extern "C" int mxk_allreduce_1shot(const uint16_t* in, uint16_t* out, int n, int
     int blocks = (ng + 255) / 256;
     if (blocks > 128) blocks = 128;
     MX_ACT_DISPATCH((allreduce_1shot_kernel<F16, false><<<blocks, 256, 0, st>>>(
-        (const uint32_t*)in, (uint32_t*)out, ng, rank, world, pp, slot_granules, epoch_ctr, err, nullptr)));
+        (const uint32_t*)in, (uint32_t*)out, ng, rank, world, pp, slot_granules, epoch_ctr, err, wait_ticks, nullptr)));
     MXK_CHECK_LAUNCH();
 }
 
 // same, but res (fp32, n elements, 8-B aligned) += the sum; `in` is not overwritten.
 extern "C" int mxk_allreduce_1shot_add(const uint16_t* in, float* res, int n, int rank, int world,
                                        unsigned long long* const* peers, long slot_granules, uint32_t* epoch_ctr,
-                                       int* err, hipStream_t st) {
+                                       int* err, long long wait_ticks, hipStream_t st) {
     if (n <= 0) return 0;
-    if ((n & 1) || world < 1 || world > MX_AR_MAX_WORLD || rank < 0 || rank >= world || (long)(n / 2) > slot_granules ||
+    if (wait_ticks <= 0 || (n & 1) || world < 1 || world > MX_AR_MAX_WORLD || rank < 0 || rank >= world || (long)(n / 2) > slot_granules ||
         ((uintptr_t)in & 3) || ((uintptr_t)res & 7))
         return (int)hipErrorInvalidValue;
     MxArPeers pp{};
@@ -141,6 +151,6 @@ extern "C" int mxk_allreduce_1shot_add(const uint16_t* in, float* res, int n, in
     int blocks = (ng + 255) / 256;
     if (blocks > 128) blocks = 128;
     MX_ACT_DISPATCH((allreduce_1shot_kernel<F16, true><<<blocks, 256, 0, st>>>(
-        (const uint32_t*)in, nullptr, ng, rank, world, pp, slot_granules, epoch_ctr, err, (float2*)res)));
+        (const uint32_t*)in, nullptr, ng, rank, world, pp, slot_granules, epoch_ctr, err, wait_ticks, (float2*)res)));
     MXK_CHECK_LAUNCH();
 }

@@ -9,7 +9,7 @@ different GPUs of one node (xGMI) and for several processes sharing one GPU (the
     ar = OneShotAllReduce(group, device, max_bytes=1 << 20)
     ar(t)          # in place, t: 16-bit CUDA tensor; falls back to dist.all_reduce when too large
     ar.snapshot()  # after a step's launches: async copy of the error flag into a pinned ring + an event
-    ar.check()     # raises if a completed snapshot saw a peer that never arrived (bounded spin in the kernel);
+    ar.check()     # raises if a completed snapshot saw a peer that never arrived within timeout_s;
                    # never blocks on queued work (block=True waits for every snapshot: shutdown / tests)
 """
 from __future__ import annotations
@@ -29,10 +29,11 @@ _SIGS = {
     "mxk_ar_ipc_open": [C.c_void_p, C.POINTER(C.c_void_p)],
     "mxk_ar_ipc_close": [C.c_void_p],
     "mxk_ar_handle_size": [],
+    "mxk_ar_clock_khz": [C.c_int],
     "mxk_allreduce_1shot": [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_void_p), C.c_long,
-                            C.c_void_p, C.c_void_p, C.c_void_p],
+                            C.c_void_p, C.c_void_p, C.c_longlong, C.c_void_p],
     "mxk_allreduce_1shot_add": [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_void_p), C.c_long,
-                                C.c_void_p, C.c_void_p, C.c_void_p],
+                                C.c_void_p, C.c_void_p, C.c_longlong, C.c_void_p],
 }
 
 
@@ -53,8 +54,10 @@ def _ok(rc, what):
 class OneShotAllReduce:
     MAX_WORLD = 8
 
-    def __init__(self, group, device, max_bytes: int = 1 << 20, rank: int | None = None, world: int | None = None):
-        """group None with world 1: a single-rank instance (no process group, no handle exchange) — the same
+    def __init__(self, group, device, max_bytes: int = 1 << 20, rank: int | None = None, world: int | None = None, timeout_s: float = 20.0):
+        """timeout_s: how long a call waits on the device for its peers before it gives up (check() raises then, and no later
+        call waits): longer than a peer's host is ever late by (garbage collection, a graph captured or a kernel tuned first).
+        group None with world 1: a single-rank instance (no process group, no handle exchange) — the same
         kernel over its own slot only, which the one-GPU tensor-parallel rehearsal runs where the real group's
         all-reduce + residual add would be (bench.py --tp-rehearsal)."""
         import torch.distributed as dist
@@ -70,6 +73,10 @@ class OneShotAllReduce:
         lib = _lib()
         self.lib = lib
         with torch.cuda.device(self.device):
+            khz = lib.mxk_ar_clock_khz(torch.cuda.current_device())
+            if khz <= 0:
+                raise N.NativeError("one-shot all-reduce: the device's clock rate is not known")
+            self.wait_ticks = max(1, int(timeout_s * 1e3 * khz))
             self.buf = C.c_void_p()
             _ok(lib.mxk_ar_alloc(2 * self.world * self.slot * 8, C.byref(self.buf)), "mxk_ar_alloc")
             self.ptrs = (C.c_void_p * self.world)()
@@ -115,7 +122,7 @@ class OneShotAllReduce:
             return out
         N.ensure_act(t.dtype)
         _ok(self.lib.mxk_allreduce_1shot(t.data_ptr(), out.data_ptr(), n, self.rank, self.world, self.ptrs,
-                                         self.slot, self.epoch.data_ptr(), self.err.data_ptr(),
+                                         self.slot, self.epoch.data_ptr(), self.err.data_ptr(), self.wait_ticks,
                                          N.stream_ptr(self.device)), "mxk_allreduce_1shot")
         return out
 
@@ -132,7 +139,7 @@ class OneShotAllReduce:
             return res
         N.ensure_act(t.dtype)
         _ok(self.lib.mxk_allreduce_1shot_add(t.data_ptr(), res.data_ptr(), t.numel(), self.rank, self.world, self.ptrs,
-                                             self.slot, self.epoch.data_ptr(), self.err.data_ptr(),
+                                             self.slot, self.epoch.data_ptr(), self.err.data_ptr(), self.wait_ticks,
                                              N.stream_ptr(self.device)), "mxk_allreduce_1shot_add")
         return res
 

@@ -10,6 +10,7 @@ import torch.distributed as dist  # noqa: E402
 
 def main():
     rank, world = int(os.environ["RANK"]), int(os.environ["WORLD_SIZE"])
+    torch.set_num_threads(max(1, 8 // world))  # (all ranks on one host: their thread pools would wait for each other's cores)
     dist.init_process_group("gloo", rank=rank, world_size=world)
     ndev = torch.cuda.device_count()
     dev = torch.device("cuda", rank % ndev)
@@ -24,6 +25,8 @@ def main():
         parts = [torch.randn(n, generator=torch.Generator().manual_seed(1000 * it + r)) for r in range(world)]
         ref = sum(p.to(dt).float() for p in parts)
         t = x.to(dev, dt)
+        torch.cuda.synchronize()
+        dist.barrier()  # (hosts come out of the draws and the reference apart; none starts its wait before all are here)
         ar(t)
         torch.cuda.synchronize()
         ar.check(block=True)
@@ -36,7 +39,10 @@ def main():
         parts = [torch.randn(n, generator=torch.Generator().manual_seed(77 + r)) for r in range(world)]
         ref = sum(p.half().float() for p in parts) + 1.5
         res = torch.full((n,), 1.5, device=dev)
-        ar.add_into(parts[rank].to(dev, torch.float16), res)
+        mine = parts[rank].to(dev, torch.float16)
+        torch.cuda.synchronize()
+        dist.barrier()
+        ar.add_into(mine, res)
         torch.cuda.synchronize()
         ar.check(block=True)
         err = (res.cpu() - ref).abs().max().item()
@@ -46,6 +52,8 @@ def main():
     t = torch.zeros(8192, device=dev, dtype=torch.float16)
     s = torch.cuda.Stream(dev)
     s.wait_stream(torch.cuda.current_stream(dev))
+    torch.cuda.synchronize()
+    dist.barrier()
     with torch.cuda.stream(s):
         t.fill_(rank + 1)
         ar(t)
@@ -57,6 +65,7 @@ def main():
         t.fill_(rank + 1)
         ar(t)
     for _ in range(5):
+        dist.barrier()
         graph.replay()
         torch.cuda.synchronize()
         ar.check(block=True)
@@ -65,6 +74,7 @@ def main():
     # check() never blocks on queued work: a long kernel queued after the snapshot leaves it pending,
     # and the host call returns at once (the overlap pipeline calls it between two launched steps)
     import time
+    dist.barrier()
     ar(t)
     ar.snapshot()
     torch.cuda._sleep(int(1e9))  # ~0.4-0.5 s of device time queued behind the snapshot

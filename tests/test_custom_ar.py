@@ -81,3 +81,32 @@ def test_one_shot_allreduce_single_rank_graph():
     assert torch.allclose(res, 50 * t.float(), atol=1e-3)
     assert int(ar.epoch[0]) == e0 + 51  # the warm-up call + 50 replays (capture launches nothing)
     assert int(ar.epoch[1]) == 0
+
+
+@pytest.mark.gpu
+def test_missing_peer_is_given_up_by_time():
+    """A peer that never delivers ends the wait after timeout_s of the clock, whatever a poll costs; calls after that wait no more.
+    Rank 0 of two whose second rank exists only as a buffer."""
+    import ctypes
+    import torch
+    from localai_tfp_amd.parallel.custom_ar import OneShotAllReduce
+    peer = OneShotAllReduce(None, "cuda", 1 << 20, world=1)
+    t = torch.ones(8192, device="cuda", dtype=torch.float16)
+    for timeout in (0.1, 0.4):
+        ar = OneShotAllReduce(None, "cuda", 1 << 20, world=1, timeout_s=timeout)
+        ar.slot //= 2  # (two slots in the room of one)
+        ar.ptrs, ar.world = (ctypes.c_void_p * 2)(ar.buf, peer.buf), 2
+        torch.cuda.synchronize()
+        ms = []
+        for _ in range(3):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            ar(t)
+            e1.record()
+            torch.cuda.synchronize()
+            ms.append(e0.elapsed_time(e1))
+        print(f"given up after {ms[0]:.1f} ms of {1e3 * timeout:.0f}, then {ms[1]:.3f}, {ms[2]:.3f} ms", flush=True)
+        assert 990 * timeout <= ms[0] <= 1000 * timeout + 50 and max(ms[1:]) < 50
+        with pytest.raises(RuntimeError, match="never delivered"):
+            ar.check(block=True)
+        ar.world, ar.ptrs = 1, (ctypes.c_void_p * 1)(ar.buf)
