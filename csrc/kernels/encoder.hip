@@ -21,7 +21,7 @@ __host__ constexpr int enc_parts(int K) { return K >= 2048 ? 4 : 1; }
 
 // A row is held by a wave: lane has the 8-element chunks lane + 64 j. Chunks past H are loaded from the row's last one and count
 // as zero: loads behind a branch are waited for inside it, one after another (LayerNorm of 19 rows after four parts of a product
-// 6.6 -> 4.6 us, the gains and offsets asked for ahead of the sums).
+// 6.6 -> 4.6 us, the gains and offsets asked for ahead of the sums). So a lane is given no more chunks than the row has (ENC_NC).
 MX_DEV int enc_chunk(int j, int H, int lane) { return min(8 * (lane + 64 * j), H - 8); }
 MX_DEV bool enc_has(int j, int H, int lane) { return 8 * (lane + 64 * j) < H; }
 
@@ -116,12 +116,20 @@ __global__ __launch_bounds__(64 * EW) void enc_embed_kernel(const int* __restric
                                                             float eps, uint16_t* __restrict__ x) {
     const int row = blockIdx.x * EW + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (row >= rows) return;
+    // gains ahead of the tables' rows where there are registers for both: a wide row's three tables and gains leave a SIMD a wave or
+    // two (6428 rows of 2048 36.5 us, 17.4 with the gains after them), a narrow one is bound by its rows in flight (512: 5.6 / 5.4)
+    constexpr bool AHEAD = NC == 2 || NC == 3;
     LnGain<NC> gb;
-    gb.load(g, b, H, lane);
     float v[NC][8] = {};
-    add_f32<NC>(v, tok + (size_t)ids[row] * H, H, lane);
-    add_f32<NC>(v, pos + (size_t)ids[rows + row] * H, H, lane);
-    if (typ) add_f32<NC>(v, typ + (size_t)ids[2 * rows + row] * H, H, lane);
+    const int ti = ids[row], pi = ids[rows + row], yi = typ ? ids[2 * rows + row] : 0;
+    if constexpr (AHEAD) gb.load(g, b, H, lane);
+    add_f32<NC>(v, tok + (size_t)ti * H, H, lane);
+    add_f32<NC>(v, pos + (size_t)pi * H, H, lane);
+    if (typ) add_f32<NC>(v, typ + (size_t)yi * H, H, lane);
+    if constexpr (!AHEAD) {
+        __builtin_amdgcn_sched_barrier(0);
+        gb.load(g, b, H, lane);
+    }
     ln_row<NC, F16>(v, H, gb, eps, x + (size_t)row * H, lane);
 }
 
@@ -316,11 +324,17 @@ int enc_gemm(const uint16_t* x, const uint16_t* W, const uint16_t* bias, void* y
     return (int)hipGetLastError();
 }
 
-// chunks of a row per lane: H <= 512 NC
-#define ENC_NC(H, ...)                                \
-    do {                                              \
-        if ((H) <= 1024) { constexpr int NC = 2; __VA_ARGS__; } \
-        else { constexpr int NC = 8; __VA_ARGS__; }   \
+// Chunks a lane holds, no more than the row has: those past its end are loaded all the same. With 2 and 8 alone, x = LN(a + x) of
+// 6428 rows took, us, 256 / 512 / 1536 / 2048 wide: 5.6 / 6.0 / 17.0 / 18.9, now 4.1 / 4.5 / 10.1 / 14.7; 19 rows 2.7 / 2.7 / 4.2 /
+// 4.2, now 2.3 / 2.3 / 2.9 / 3.2. The sum of the embeddings, 6428 rows: 7.1 / 7.4 / 33.3 / 36.5, now 5.0 / 5.4 / 13.1 / 17.4.
+#define ENC_NC(H, ...)                                          \
+    do {                                                        \
+        if ((H) <= 512) { constexpr int NC = 1; __VA_ARGS__; }  \
+        else if ((H) <= 1024) { constexpr int NC = 2; __VA_ARGS__; } \
+        else if ((H) <= 1536) { constexpr int NC = 3; __VA_ARGS__; } \
+        else if ((H) <= 2048) { constexpr int NC = 4; __VA_ARGS__; } \
+        else if ((H) <= 3072) { constexpr int NC = 6; __VA_ARGS__; } \
+        else { constexpr int NC = 8; __VA_ARGS__; }             \
     } while (0)
 
 int enc_add_ln(const uint16_t* a, uint16_t* x, int rows, const float* g, const float* b, int H, float eps, hipStream_t st) {

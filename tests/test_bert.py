@@ -161,6 +161,51 @@ def test_packed_rows_match_fp32(hidden, heads, ffn, pooling, monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("H", [8, 256, 504, 512, 520, 1024, 1032, 1536, 1544, 2048, 2056, 3072, 3080, 4096])
+def test_row_kernels_at_the_edges_of_their_widths(H, dtype):
+    """Sum of embeddings and x = LN(a + x), rows that fill a lane's chunks, leave lanes without one and start the next chunk, against
+    float64: the output is rounded to 16 bits (half a unit, relative 2^-11 / 2^-8), sums of 4096 fp32 numbers of order 1 are within
+    1e-5 of their length. Rows behind the last are left alone."""
+    from localai_tfp_amd import _native as N
+    g = torch.Generator().manual_seed(H)
+    gain, off = torch.randn(H, generator=g), torch.randn(H, generator=g)
+    tok, pos, typ = (torch.randn(n, H, generator=g) for n in (50, 20, 2))
+    unit = 2 ** -11 if dtype == torch.float16 else 2 ** -8
+    N.ensure_act(dtype)
+    for rows in (1, 6):
+        ids = torch.stack([torch.randint(0, n, (rows,), generator=g) for n in (50, 20, 2)])
+        a, x = torch.randn(rows, H, generator=g).to(dtype), torch.randn(rows, H, generator=g).to(dtype)
+        for b, t in ((off, typ), (None, None)):
+            e = tok[ids[0]].double() + pos[ids[1]].double() + (t[ids[2]].double() if t is not None else 0)
+            d = [v.cuda() if v is not None else None for v in (tok, pos, t, gain, b)]
+            i32, y, z = ids.int().cuda(), torch.full((rows + 1, H), 7.0, dtype=dtype, device="cuda"), torch.full((rows + 1, H), 7.0, dtype=dtype, device="cuda")
+            N.kcall("mxk_enc_embed", i32.data_ptr(), rows, *(N.ptr(v) for v in d), H, 1e-6, y.data_ptr(), N.stream_ptr())
+            z[:rows] = x.cuda()
+            ad = a.cuda()
+            N.kcall("mxk_enc_add_ln", ad.data_ptr(), z.data_ptr(), rows, d[3].data_ptr(), N.ptr(d[4]), H, 1e-6, N.stream_ptr())
+            for got, v in ((y, e), (z, a.double() + x.double())):
+                want = (v - v.mean(1, keepdim=True)) * torch.rsqrt(v.var(1, unbiased=False, keepdim=True) + 1e-6) * gain.double()
+                want = want + (b.double() if b is not None else 0)
+                assert ((got[:rows].cpu().double() - want).abs() <= unit * want.abs() + 1e-4).all() and (got[rows:] == 7.0).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hidden", [1536, 2560])
+def test_wide_one_call_layers(hidden, monkeypatch):
+    """Rows of three and of five chunks a lane through the one-call layers (sums of one and of four parts of K): bounds as above."""
+    cfg = BM.BertConfig(vocab=400, hidden=hidden, n_layers=1, n_heads=hidden // 64, ffn=2048, max_pos=64, name="t")
+    get = BM.synthetic_bert(cfg, 5)
+    g, c = BM.BertModel.load(cfg, get, "cuda:0"), BM.BertModel.load(cfg, get, "cpu")
+    monkeypatch.setattr(BM, "small_rows", lambda H, F: 4096)
+    ids = [list(range(10, 10 + n)) for n in (17, 3)]
+    hid, n = g.encode(ids)
+    want, _ = c.encode(ids)
+    for i, k in enumerate(n.tolist()):
+        assert (hid[i, :k].cpu() - want[i, :k]).abs().max() < 5e-2
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("pooling", ["mean", "cls", "last"])
 def test_empty_texts_match_the_padded_batch(pooling):
     """An empty text has a row too: nothing for the mean, its first row, or the batch's last position."""
