@@ -135,6 +135,22 @@ def test_glu_of_many_elements(act):
             assert ((got["cuda"] - got["cpu"]).abs() <= tol * got["cpu"].abs().clamp_min(1)).all()
 
 
+@pytest.mark.parametrize("F", [257, 1028])
+def test_glu_of_more_workgroups_than_a_grid_dimension(F):
+    """Rows x chunks of a row beyond the 2^24 - 1 workgroups of 256 threads that a grid dimension holds, with one element a thread (odd
+    widths) and with four: rows at both ends and where a second launch begins."""
+    T = (1 << 23) + 5
+    a, out = torch.full((T, F), 1.5, device="cuda"), torch.zeros(T, F, device="cuda", dtype=torch.bfloat16)
+    at = torch.tensor([0, 1, (1 << 23) - 2, (1 << 23) - 1, 1 << 23, (1 << 23) + 1, T - 2, T - 1], device="cuda")
+    x = torch.randn(len(at), F, generator=torch.Generator().manual_seed(F))
+    a[at] = x.cuda()
+    HY.glu(a, None, None, None, out, act="relu2")
+    want = torch.relu(x).pow(2).bfloat16()
+    assert torch.equal(out[at].cpu(), want) and bool((out[5:(1 << 23) - 5:4099] == 2.25).all())
+    del a, out
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("H,G,Gv,dk,dv,rot,half", [(18, 3, 3, 64, 40, 64, False), (9, 8, 7, 100, 64, 36, True), (24, 0, 0, 32, 32, 0, False)])
 def test_rotary_rows_of_many_heads(H, G, Gv, dk, dv, rot, half):
     """Steps of 32768 heads and more take eight heads a wave: head counts that leave a group part empty or mix queries with keys, partial
