@@ -576,17 +576,18 @@ MX_DEV float glu_one(float x, float y, float fac, int act, float limit, float al
 }
 // V elements a thread: 4 where every row, factor group and operand allows 16-byte reads and there are a million of them, else 1.
 // Many are bound by their bytes: 1990 rows of 14336 (285 MB) took 113 us with one element a thread, 84 with four; few by the chain
-// of one thread: 128 x 2048 2.9 us with one, 3.4 with four; 128 x 14336 5.5 / 4.6. With four elements neighbouring workgroups share a
-// row (1990 rows of 14336 with biases 82 us the other way, 56 so; 301 17.2 / 11.6), with one they have a row each (64 rows of 14336
-// 4.4 us sharing a row, 4.1 so; 1990 of 384 4.4 / 4.1).
+// of one thread: 128 x 2048 2.9 us with one, 3.4 with four; 128 x 14336 5.5 / 4.6. SHARE: neighbouring workgroups share a row, else they
+// have a row each. Shared with four elements (1990 rows of 14336 with biases 82 us the other way, 56 so; 301 17.2 / 11.6) and with one
+// from eight million numbers on (biases off 16 bytes, 1990 rows 89.5 / 84.1; 301 rows 11.6 / 12.4, 1990 of 2048 10.9 / 11.7, 64 of 14336
+// 4.1 / 4.4, 1990 of 384 4.1 / 4.4).
 constexpr int GLU_BLOCKS = (1 << 24) - 1;  // of 256 threads: a grid dimension holds less than 2^32 threads
-template <bool B16, int V>
+template <bool B16, int V, bool SHARE>
 __global__ __launch_bounds__(NT) void glu_kernel(const float* a, int lda, const float* b, int ldb, const float* ba,
                                                  const float* bb, const float* scale, int lds, int group,
                                                  int scale_sigmoid, void* out, int ldo, int F, int act, float limit,
                                                  float alpha) {
-    const int chunks = V == 4 ? (F + NT * V - 1) / (NT * V) : 1, t = blockIdx.x / chunks;
-    const int f = ((V == 4 ? blockIdx.x - t * chunks : blockIdx.y) * NT + threadIdx.x) * V;
+    const int chunks = SHARE ? (F + NT * V - 1) / (NT * V) : 1, t = blockIdx.x / chunks;
+    const int f = ((SHARE ? blockIdx.x - t * chunks : blockIdx.y) * NT + threadIdx.x) * V;
     if (f >= F) return;
     auto put = [&](const float* v) {
         if constexpr (V == 4 && B16)
@@ -890,19 +891,22 @@ extern "C" int mxh_glu(const float* a, int lda, const float* b, int ldb, const f
     MXH_CHECK(!scale || (F % group == 0 && lds >= F / group));
     const bool four = (long)T * F >= 1 << 20 && F % 4 == 0 && group % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0 && ldo % 4 == 0 &&
                       ((uintptr_t)a | (uintptr_t)b | (uintptr_t)ba | (uintptr_t)bb | (uintptr_t)out) % 16 == 0;
+    const bool share = four || (long)T * F >= 1 << 23;
     const int chunks = (F + NT * (four ? 4 : 1) - 1) / (NT * (four ? 4 : 1));
-    const int rows = four ? min(T, GLU_BLOCKS / chunks) : T;
+    const int rows = share ? min(T, GLU_BLOCKS / chunks) : T;
     for (long t0 = 0; t0 < T; t0 += rows) {
         const int n = (int)min((long)rows, T - t0);
         const float *at = a + t0 * lda, *bt = b ? b + t0 * ldb : nullptr, *ft = scale ? scale + t0 * lds : nullptr;
         void* ot = (char*)out + t0 * ldo * (o16 ? 2 : 4);
-        const dim3 grid = four ? dim3((unsigned)n * chunks) : dim3(n, chunks);
-#define GO(B, V)                                                                                                                 \
-    glu_kernel<B, V><<<grid, NT, 0, st>>>(at, lda, bt, ldb, ba, bb, ft, lds, group, scale_sigmoid, ot, ldo, F, act, limit, alpha)
-        if (o16 && four) GO(true, 4);
-        else if (o16) GO(true, 1);
-        else if (four) GO(false, 4);
-        else GO(false, 1);
+        const dim3 grid = share ? dim3((unsigned)n * chunks) : dim3(n, chunks);
+#define GO(B, V, S)                                                                                                              \
+    glu_kernel<B, V, S><<<grid, NT, 0, st>>>(at, lda, bt, ldb, ba, bb, ft, lds, group, scale_sigmoid, ot, ldo, F, act, limit, alpha)
+        if (o16 && four) GO(true, 4, true);
+        else if (o16 && share) GO(true, 1, true);
+        else if (o16) GO(true, 1, false);
+        else if (four) GO(false, 4, true);
+        else if (share) GO(false, 1, true);
+        else GO(false, 1, false);
     }
 #undef GO
     return (int)hipGetLastError();

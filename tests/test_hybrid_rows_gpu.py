@@ -135,6 +135,22 @@ def test_glu_of_many_elements(act):
             assert ((got["cuda"] - got["cpu"]).abs() <= tol * got["cpu"].abs().clamp_min(1)).all()
 
 
+@pytest.mark.parametrize("off", [0, 1])
+def test_glu_biases_of_any_alignment(off):
+    """Four elements a thread with biases that start on 16 bytes or not; the bound of test_glu_widths."""
+    g = torch.Generator().manual_seed(off)
+    T, F = 300, 4096
+    a, b, bias = torch.randn(T, F, generator=g), torch.randn(T, F, generator=g), torch.randn(2 * F + 8, generator=g)
+    for dt in (torch.float32, torch.bfloat16):
+        got = {}
+        for dev in ("cpu", "cuda"):
+            out, d = torch.empty(T, F, dtype=dt, device=dev), bias.to(dev)
+            HY.glu(a.to(dev), b.to(dev), d[off:off + F], d[F + 4 + off:2 * F + 4 + off], out)
+            got[dev] = out.cpu().float()
+        tol = 2e-5 if dt == torch.float32 else 2 ** -7
+        assert ((got["cuda"] - got["cpu"]).abs() <= tol * got["cpu"].abs().clamp_min(1)).all()
+
+
 @pytest.mark.parametrize("F", [257, 1028])
 def test_glu_of_more_workgroups_than_a_grid_dimension(F):
     """Rows x chunks of a row beyond the 2^24 - 1 workgroups of 256 threads that a grid dimension holds, with one element a thread (odd
