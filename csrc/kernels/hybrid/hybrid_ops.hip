@@ -225,7 +225,9 @@ __global__ __launch_bounds__(1024) void scale_add_norm_kernel(const float* y, in
 // pos * base^(-(e / 2) * 2 / rot_dims); with `half` the pairs are (i, i + rot_dims / 2) instead and pair i turns by pos * base^(-i * 2 / rot_dims). Given `freqs`
 // (one per pair) pair i turns by pos * freqs[i]; sine and cosine are multiplied by mag. qb, kb, vb: projection biases.
 constexpr int HEAD_E = 8;  // elements per lane: heads of up to 512 numbers
-// E: elements per lane of this instance (2: heads of up to 128), HPW: heads of a wave
+// E: elements per lane of this instance, no more than a head needs, since all are loaded (2 per head of 64 or 128, 3, 4, 6, 8: with 8
+// beyond 128 numbers 128 rows of 16 + 2 heads of 192 took 4.2 us, 301 5.9, now 3.7 and 5.1; 1990 of 16 + 4 heads of 256 33 / 31),
+// HPW: heads of a wave
 template <bool Q16, bool C16, int E, int HPW>
 __global__ __launch_bounds__(64) void rope_norm_append_kernel(const float* qi, const float* ki, const float* vi,
                                                               int ldq, int ldk, int ldv, const int* positions, int H,
@@ -793,9 +795,12 @@ extern "C" int mxh_rope_norm_append(const float* qi, const float* ki, const floa
         half, Gv, freqs, mag, qb, kb, vb)
 #define GO(Q, C)                                                          \
     do {                                                                  \
-        if (dk > 128) GO3(Q, C, HEAD_E, 1);                               \
-        else if ((long)T * (H + G + Gv) >= 32768) GO3(Q, C, 2, 8);        \
-        else GO3(Q, C, 2, 1);                                             \
+        if (dk <= 128 && (long)T * (H + G + Gv) >= 32768) GO3(Q, C, 2, 8); \
+        else if (dk <= 128) GO3(Q, C, 2, 1);                              \
+        else if (dk <= 192) GO3(Q, C, 3, 1);                              \
+        else if (dk <= 256) GO3(Q, C, 4, 1);                              \
+        else if (dk <= 384) GO3(Q, C, 6, 1);                              \
+        else GO3(Q, C, HEAD_E, 1);                                        \
     } while (0)
     if (q16 && c16) GO(true, true);
     else if (q16) GO(true, false);

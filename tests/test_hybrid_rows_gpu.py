@@ -187,6 +187,27 @@ def test_rotary_rows_of_many_heads(H, G, Gv, dk, dv, rot, half):
         assert (a - b).abs().max() <= 1e-3 * max(1.0, float(b.abs().max()))
 
 
+@pytest.mark.parametrize("dk", [130, 191, 192, 194, 256, 258, 383, 384, 386, 512])
+def test_rotary_rows_of_wide_heads(dk):
+    """Heads at the edges of three, four, six and eight numbers a lane: pairs of neighbours and of halves, whole and partial rotation,
+    biases, rows without a slot; the bound of test_rotary_rows_of_many_heads."""
+    T, H, G, g = 9, 3, 2, torch.Generator().manual_seed(dk)
+    q, k, v = torch.randn(T, H * dk + 4, generator=g), torch.randn(T, G * dk, generator=g), torch.randn(T, G * dk, generator=g)
+    bias, w = torch.randn((H + 2 * G) * dk, generator=g), torch.rand(2, dk, generator=g) + 0.5
+    pos, slots = torch.randint(0, 3000, (T,), generator=g, dtype=torch.int32), torch.randperm(T + 3, generator=g)[:T].to(torch.int32)
+    slots[3] = -1
+    for rot, half, dt in ((dk // 2 * 2, False, torch.float32), (dk // 2 * 2, True, torch.bfloat16), (64, True, torch.float32), (0, False, torch.float32)):
+        got = {}
+        for dev in ("cpu", "cuda"):
+            b, hw = bias.to(dev), w.to(dev)
+            qo, kc, vc = torch.zeros(T, H * dk, device=dev, dtype=dt), torch.zeros(T + 3, 1, G * dk, device=dev, dtype=dt), torch.zeros(T + 3, 1, G * dk, device=dev, dtype=dt)
+            HY.rope_norm_append(q.to(dev)[:, 4:], k.to(dev), v.to(dev), pos.to(dev), H, G, dk, dk, rot, 1e4, True, 1e-6, qo, kc, vc, slots.to(dev), q_weight=hw[0],
+                                k_weight=hw[1], half=half, q_bias=b[:H * dk], k_bias=b[H * dk:(H + G) * dk], v_bias=b[(H + G) * dk:])
+            got[dev] = [t.cpu().float() for t in (qo, kc, vc)]
+        for a, b in zip(got["cuda"], got["cpu"]):
+            assert (a - b).abs().max() <= (1e-3 if dt == torch.float32 else 2 ** -7) * max(1.0, float(b.abs().max()))
+
+
 @pytest.mark.parametrize("chunk,window", [(0, 0), (128, 0), (0, 40)])
 def test_chunks_of_many_sequences(chunk, window):
     """The chunks of a step are launched sixteen at a time, the longest first: eighteen sequences (with short ones between, which run on
