@@ -337,10 +337,15 @@ MX_DEV int v_lds_off(int p, int nt) {
 // vector work). Three waves per SIMD instead of two gave the quantised caches 73 -> 64 of that.
 // A key's pool row is worked out once, by one lane, and passed to the lanes that load its numbers (a division by the page size for
 // each of a lane's ten loads was half of a bf16 tile's vector instructions), masks and score caps stand in branches of their own:
-// 480 -> 250 vector instructions a bf16 tile, 700 -> 600 in q8_0 (320 of them the widening), 570 -> 370 in fp8. With the merge launch:
-// 128 rows of 65-1021 keys in one partition 43.1 -> 41.8 us (bf16), 31.6 -> 30.2 (q8_0), 27.1 -> 25.3 (fp8); 9 rows of 3001-24001 in
-// partitions of 256 q8_0 63.8 -> 62.4, fp8 57.4 -> 55.9, 32 rows of 97-4003 fp8 29.9 -> 28.6, bf16 39.6 -> 40.0 (the first tile's
-// rows take one hop more).
+// 700 -> 600 vector instructions a tile in q8_0 (320 of them the widening), 570 -> 370 in fp8. With the merge launch, us: 128 rows of
+// 65-1021 keys in one partition q8_0 30.0 -> 28.6, fp8 25.5 -> 23.1; 9 rows of 3001-24001 in partitions of 256 63.0 -> 61.9, 58.5 ->
+// 56.7; 32 rows of 97-4003 30.0 -> 28.8, 29.1 -> 27.3. bf16 of head dim 64 the same way 22.2 -> 20.9.
+// bf16 of head dim 128, four waves, keeps mask and cap in one pass, which measures faster (why, no counter shows; fewer instructions
+// between a tile's loads are no gain there: with all ten rows fetched ahead of the first load 32 rows of 97-4003 took 45.4). Before /
+// with branches / so, us: 32 rows of 97-4003 39.3 / 39.7 / 39.2; 20 rows of 2000-6000 in partitions of 128 72.3 / 75.7 / 73.2; 12 rows
+// of 30-200 9.4 / 9.1 / 9.0; 128 rows of 65-1021 in one 44.5 / 42.9 / 42.9. What is left of the loss is 1 % for long contexts in many
+// partitions, 2 % for 32 x 1000 in four, 3 % for 48 x 100-500 in two; rows worked out by each lane again give it back, at 4 to 8 % for
+// short contexts (32 rows of 30-400 13.0 / 14.1), and the host does not know which they are.
 // Occupancy, not register double buffering, hides HBM latency: 8 KB of LDS per wave lets 4
 // workgroups (16 waves) share a CU, each with one tile's 16 KB of K/V loads in flight.
 template <int D>
@@ -498,7 +503,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
     const char* vc = (const char*)vcv;
 
     // PF (bf16 caches): the next tile's K fragments are requested while this tile computes. Every K load is then
-    // issued unconditionally (keys past the end read a valid row and are zeroed after the load), and V comes
+    // issued unconditionally (keys past the end repeat the last key's row, the mask alone makes their weights 0), and V comes
     // through registers (plain loads, stored to the LDS image after QK^T) instead of LDS-DMA: the explicit vmcnt
     // waits below count exactly NK K loads and NVC V loads per tile, which holds only for loads that complete in
     // issue order (LDS-DMA completions are not ordered against plain loads).
@@ -616,26 +621,40 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
         }
         // ---- online softmax over the tile: the head's maximum over its four lanes, everything else lane-local ----
         float mx = -INFINITY;
-        if (softcap > 0.f) {
+        // the mask and the cap: in one pass over the scores, or in branches of their own that most tiles skip (see above)
+        if constexpr (!KV8 && D == 128 && NW == 4) {
 #pragma unroll
             for (int t = 0; t < 2; ++t)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) sacc[t][i] = sc_l2 * tanhf(sacc[t][i] * qs * sc_inv);
+                for (int i = 0; i < 4; ++i) {
+                    float v = sacc[t][i] * qs;
+                    if (softcap > 0.f) v = sc_l2 * tanhf(v * sc_inv);
+                    if (kt0 + 16 * t + 4 * g + i >= p1) v = -INFINITY;
+                    sacc[t][i] = v;
+                    mx = fmaxf(mx, v);
+                }
         } else {
+            if (softcap > 0.f) {
 #pragma unroll
-            for (int t = 0; t < 2; ++t) sacc[t] *= qs;
-        }
-        if (kt0 + KT > p1) {
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) sacc[t][i] = sc_l2 * tanhf(sacc[t][i] * qs * sc_inv);
+            } else {
+#pragma unroll
+                for (int t = 0; t < 2; ++t) sacc[t] *= qs;
+            }
+            if (kt0 + KT > p1) {
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (kt0 + 16 * t + 4 * g + i >= p1) sacc[t][i] = -INFINITY;
+            }
 #pragma unroll
             for (int t = 0; t < 2; ++t)
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (kt0 + 16 * t + 4 * g + i >= p1) sacc[t][i] = -INFINITY;
+                for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sacc[t][i]);
         }
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sacc[t][i]);
         const float mn = fmaxf(mrow, quarters_max(mx));
         if (__any(mn > mrow)) {
             const float alpha = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(mrow - mn);

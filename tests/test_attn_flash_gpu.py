@@ -180,3 +180,31 @@ def test_decode_partitions_that_start_inside_a_page(bs, part, fmt, impl):
         got = out.cpu().float()
         # as for prompts: probabilities and outputs are rounded to 16 bits once each
         assert float((got - want[rows]).norm() / want[rows].norm()) < 4 * 2 ** -9
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", ["bf16", "fp8", "q8_0"])
+@pytest.mark.parametrize("Hq,Hkv,D", [(8, 2, 128), (8, 1, 64)])
+@pytest.mark.parametrize("window,softcap", [(0, 0.0), (0, 4.0), (50, 0.0)])
+def test_decode_reads_nothing_behind_a_context(fmt, Hq, Hkv, D, window, softcap):
+    """Slots of the pool that no context holds are not numbers, those of the last page behind it among them: the last tile's mask, with
+    and without a cap, in every form (few rows take more waves a workgroup)."""
+    pre = [0, 1, 30, 31, 32, 95, 127, 128, 200, 511, 700]
+    q, kc, vc, bt, _, ctx = _case(Hq, Hkv, D, [1] * len(pre), pre, fmt=fmt)
+    want = torch.stack([K._attn_ref_one(q[i:i + 1], kc, vc, bt[i], int(c), int(c) - 1, D ** -0.5, 16, window, softcap)[0] for i, c in enumerate(ctx)])
+    free = torch.ones(kc.shape[0], 16, dtype=torch.bool)
+    for i, c in enumerate(ctx.tolist()):
+        at = torch.arange(c)
+        free[bt[i].long()[at // 16], at % 16] = False
+    assert free.any()
+    for c in (kc, vc):
+        rows = c.view(torch.uint8 if c.element_size() == 1 else torch.int16).permute(0, 2, 1, 3)
+        rows[free] = -1 if c.element_size() == 2 else 255  # bf16, fp8 and f16 scales of all ones are not numbers
+    kd, vd = kc.cuda(), vc.cuda()
+    if hasattr(kc, "kvf"):
+        kd.kvf, vd.kvf = kc.kvf, vc.kvf
+    for rows, part in ((slice(None), 128), (slice(None), 256), (slice(None), 1024), (slice(5, 11), 512), (slice(5, 11), 256)):
+        out = torch.full((len(ctx[rows]), Hq, D), float("nan"), dtype=torch.float16, device="cuda")
+        K.attn_decode(q[rows].cuda(), kd, vd, bt[rows].contiguous().cuda(), ctx[rows].cuda(), D ** -0.5, out, part_size=part, window=window, softcap=softcap)
+        # as for prompts: probabilities and outputs are rounded to 16 bits once each
+        assert float((out.cpu().float() - want[rows]).norm() / want[rows].norm()) < 4 * 2 ** -9, part
