@@ -732,6 +732,41 @@ def _expanded_plan(M: int, N_: int, K: int, qtype: int, can_split: bool, glu: bo
     return None
 
 
+def _few_rows_pick_qmmr(M: int, N_: int, K: int, qtype: int, can_split: bool) -> bool:
+    """Whether an untuned product of up to 32 rows runs qmmr.hip rather than the 64-row qmm2 tile. qmmr decodes in registers at four
+    waves a SIMD and is bound by that; qmm2's tiles wait for their LDS ring. So qmmr wins where a launch is short or its workgroups
+    make one round, and loses with the formats that decode slowest (Q6_K and five-bit MX5F) and where K splits fill the chip for qmm2.
+    qmm2 / qmmr, us, 9 or 16 rows, weights in no cache, eight formats x 43 shapes:
+      one round of 128-column workgroups (N 16384 .. 32768): 28672 x 4096 gated Q4_K 28 / 20, Q8_0 32 / 25, Q6_K 31 / 28, MX5F 30 / 31;
+        20480 x 4096 into the residual (qmm2 splits K) Q6_K 25 / 28, MX5F 25 / 31, others even or better;
+      more rounds: 57344 x 8192 Q4_K 90 / 73, Q8_0 102 / 93, Q6_K 96 / 103, MX5F 94 / 116; 128256 x 4096 Q4_K 92 / 84, Q8_0 115 / 102, Q3_K 91 / 93,
+        Q6_K 106 / 113; 37888 x 3584 (1.2 rounds) Q8_0 38 / 41, Q4_K 39 / 33; 151936 x 1536 Q3_K 47 / 54, Q4_K 46.5 / 47.3, MX4F 49 / 47;
+      fewer columns, K not splittable: always qmmr (4096 x 4096 Q4_K 23 / 13, Q6_K 26 / 22);
+      K splittable: 4096 x 4096 Q4_K 8.0 / 6.4, Q6_K at 5 rows 7.9 / 8.1; 2560 x 9728 all formats; 6144 x 4096 at 5 rows Q3_K 9.7 / 10.2, Q6_K
+        10.3 / 12.8, at 16 Q3_K 10.2 / 10.1; 4096 x 14336 at 16 rows Q4_K 15.5 / 15.0, Q2_K 14.6 / 16.0, Q6_K 17 / 21; 8192 x 28672 Q4_K 46 / 48, Q6_K
+        50 / 73, Q8_0 54 / 52."""
+    heavy, weights = qtype in (int(QType.Q6_K), int(QType.MX5F)), N_ * K
+    if N_ > 32768:
+        if heavy:
+            return False
+        if qtype == int(QType.MX4F):
+            return True
+        if qtype == int(QType.Q4_K):
+            return K >= 3072
+        return K >= 4096 and N_ >= 49152 and (N_ < 98304 or qtype == int(QType.Q8_0))
+    if N_ >= 16384:
+        if qtype == int(QType.MX5F):
+            return weights <= 1 << 24 and not can_split
+        return qtype != int(QType.Q6_K) or not can_split or N_ >= 24576
+    if not can_split or qtype == int(QType.Q8_0):
+        return True
+    if heavy:
+        return weights <= 15_000_000 and N_ <= 5120
+    if weights <= 25_000_000 and (N_ <= 12288 or M >= 16):
+        return True
+    return M >= 16 and weights <= (1 << 25 if qtype == int(QType.Q2_K) else 60_000_000)
+
+
 def _gemm_pick(M: int, N_: int, K: int, qtype: int, can_split: bool):
     """Untuned fallback plan (run_plan) for a t32 GEMM — shapes the load-time
     autotuner (ops/autotune.py) did not time. The rule follows the tuned Llama-3-8B table
@@ -745,7 +780,7 @@ def _gemm_pick(M: int, N_: int, K: int, qtype: int, can_split: bool):
         return _large_plan(M, N_, K, qtype, can_split)
     nct = -(-N_ // 128)
     wide = N_ >= 16384
-    if M <= 32:  # qmmr from its table (qmmr.hip): 128 columns a workgroup where they fill the chip, else 64 and K splits
+    if M <= 32 and _few_rows_pick_qmmr(M, N_, K, qtype, can_split):  # 128 columns a workgroup where they fill the chip, else 64 and K splits
         return ("qr", 1, 4, 4, 1) if wide else ("qr", 1, 2, 4, _split_for(-(-N_ // 64), K, can_split))
     if M <= 64 or (not wide and K < 8192 and M <= 256):
         return ("q2", 2, 2, 1, _split_for(-(-M // 64) * nct, K, can_split))

@@ -142,3 +142,20 @@ def test_expanded_products(qt):
             L.run_plan(plan, W, xd, epi, glu, False)
             g = (act(y[:, :, 0]) * y[:, :, 1]).reshape(M, -1)
             assert float((glu.cpu().double() - g).norm() / g.norm()) < 4 * 2 ** -10
+
+
+def test_few_rows_by_format():
+    """Untuned products of up to 32 rows: the formats that decode slowest leave the register kernel where qmm2's K splits fill the chip
+    or its workgroups make a second round; what measured faster there stays."""
+    kind = lambda m, n, k, qt, split=False: L._gemm_pick(m, n, k, int(qt), split)[0]  # noqa: E731
+    for m in (5, 9, 16, 32):
+        for qt in (QType.Q6_K, QType.MX5F):
+            assert kind(m, 4096, 14336, qt, True) == kind(m, 6144, 4096, qt, True) == kind(m, 8192, 28672, qt, True) == "q2"
+            assert kind(m, 57344, 8192, qt) == kind(m, 128256, 4096, qt, True) == "q2"
+            assert kind(m, 1024, 4096, qt, True) == kind(m, 2048, 2048, qt, True) == kind(m, 4096, 4096, qt) == "qr"
+        assert kind(m, 28672, 4096, QType.Q6_K) == "qr" and kind(m, 28672, 4096, QType.MX5F) == "q2"
+        for qt in (QType.Q4_K, QType.MX4F, QType.Q8_0):
+            assert kind(m, 28672, 4096, qt) == kind(m, 57344, 8192, qt) == kind(m, 4096, 4096, qt, True) == "qr"
+        assert kind(m, 8192, 28672, QType.Q8_0, True) == "qr" and kind(m, 8192, 28672, QType.Q4_K, True) == "q2"
+        assert kind(m, 4096, 14336, QType.Q2_K, True) == "q2" and kind(m, 151936, 1536, QType.Q3_K, True) == "q2"
+    assert kind(9, 4096, 14336, QType.Q4_K, True) == "q2" and kind(16, 4096, 14336, QType.Q4_K, True) == "qr"
