@@ -718,17 +718,22 @@ X16_SCRATCH = 1 << 28  # bytes of f16 weights expanded at a time
 @functools.lru_cache(maxsize=4096)
 def _expanded_plan(M: int, N_: int, K: int, qtype: int, can_split: bool, glu: bool):
     """("x16", columns, qmm2 plan) where expanding the weights to f16 and gemm16.hip are estimated below that plan, else None.
-    Expansion: 5 us + 0.62 per 10^6 weights; products: 6 us + 1.45 a 64-wide k-tile of each round of 256 x 256 tiles (the last one
-    counted as in _large_best) + 12 a round to fill and drain (gated: 5, it writes a quarter). _large_best is 5 % low against
-    these measurements, 12 % and more for gated products. Of 77 products (11 shapes 1024 x 4096 .. 28672 x 4096 at 1024 .. 8191 rows)
-    none picked was slower than the qmm2 plan; what it gives: us, gate|up 28672 x 4096 at 1536 / 2048 / 4096 / 8191 rows 392 -> 364,
-    477 -> 437, 943 -> 755, 1828 -> 1435; 4096 x 14336 Q4_K at 4096 / 8191 452 -> 376, 879 -> 719, Q6_K 485 -> 382, 922 -> 729; 4096 x
-    4096 142 -> 122, 271 -> 231; 6144 x 4096 at 8191 396 -> 324; 16384 x 2048 gated at 2048 / 8191 160 -> 144, 570 -> 449."""
+    Weights: 0.62 us per 10^6. Each piece of columns that the scratch holds, a launch of its own: 11 us, 1.45 a 64-wide k-tile of each
+    round of 256 x 256 tiles (the last one counted as in _large_best) and 12 a round to fill and drain (gated: 5, it writes a quarter).
+    _large_best is 5 % low against these measurements, 12 % for gated products; MX4F, which decodes fastest, 3 and 10 %.
+    Measured, qmm2 / x16 us, eight formats x 14 shapes (2048 x 2048 .. 57344 x 8192, 8192 x 28672) x 12 row counts 1025 .. 8191: 481 picks,
+    none more than 1.5 % slower. gate|up 28672 x 4096 Q4_K at 1536 / 2048 / 4096 / 8191 rows 375 / 358, 485 / 455, 964 / 776, 1860 / 1495,
+    Q8_0 at 8191 2054 / 1507; 4096 x 14336 Q4_K at 4096 / 8191 468 / 389, 921 / 741, Q6_K 501 / 392, 943 / 737; 4096 x 4096 148 / 129, 280 /
+    238. Weights in two pieces leave half a round each: 8192 x 28672 Q4_K at 2048 rows 904 / 1155, at 4096 1791 / 1911, at 8191 3591 / 3259;
+    57344 x 8192 at 2304 2021 / 2162, at 4096 3603 / 2992."""
     t, plan = _large_best(M, N_, K, qtype, can_split)
-    full, rem = divmod(-(-M // 256) * -(-N_ // 256), CU_COUNT)
-    rounds = full + (0.6 + 0.4 * rem / CU_COUNT if rem else 0.0)
-    if 11.0 + rounds * (1.45 * K / 64 + (5.0 if glu else 12.0)) + 0.62e-6 * N_ * K < t * (1.12 if glu else 1.05):
-        return ("x16", max(256, X16_SCRATCH // (K * 512) * 256), plan)
+    cols = max(256, X16_SCRATCH // (K * 512) * 256)
+    us = 0.62e-6 * N_ * K
+    for n0 in range(0, N_, cols):
+        full, rem = divmod(-(-M // 256) * -(-min(cols, N_ - n0) // 256), CU_COUNT)
+        us += 11.0 + (full + (0.6 + 0.4 * rem / CU_COUNT if rem else 0.0)) * (1.45 * K / 64 + (5.0 if glu else 12.0))
+    if us < t * (1.12 if glu else 1.05) * (0.98 if qtype == int(QType.MX4F) else 1.0):
+        return ("x16", cols, plan)
     return None
 
 

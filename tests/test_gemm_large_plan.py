@@ -113,6 +113,15 @@ def test_expanded_plans():
     assert cols % 256 == 0 and 256 <= cols and cols * 8192 * 2 <= L.X16_SCRATCH and plan == L._large_plan(8191, 57344, 8192, int(QType.Q4_K), False)
 
 
+def test_expanded_plans_count_rounds_by_piece():
+    """Weights of more than the scratch are multiplied piece by piece: where a piece leaves half the chip idle, the quantised plan."""
+    pick = lambda m, n, k, glu, qt: L._expanded_plan(m, n, k, int(qt), not glu, glu)  # noqa: E731
+    for qt in (QType.Q4_K, QType.Q3_K, QType.Q2_K, QType.Q5_K, QType.Q8_0, QType.MX4F):
+        assert pick(1800, 8192, 28672, False, qt) is None and pick(2048, 8192, 28672, False, qt) is None
+        assert pick(8191, 8192, 28672, False, qt)[0] == pick(4096, 57344, 8192, True, qt)[0] == pick(8191, 28672, 4096, True, qt)[0] == "x16"
+    assert pick(2304, 57344, 8192, True, QType.Q4_K) is None and pick(4096, 8192, 28672, False, QType.Q4_K) is None
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("qt", [*QTYPES, QType.Q4_0, QType.Q5_0, QType.Q5_1])
 def test_expanded_products(qt):
