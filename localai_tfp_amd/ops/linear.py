@@ -373,11 +373,13 @@ def run_plan(plan: tuple, W: QWeight, x: torch.Tensor, epi: int, out: torch.Tens
 
 def _run_x16(plan: tuple, W: QWeight, x: torch.Tensor, epi: int, out: torch.Tensor, out_zeroed: bool):
     """("x16", columns, plan): gemm16.hip on the weight's rows expanded to f16, `columns` of them at a time; `plan` where what
-    the kernel reads or writes is not aligned for it or the scratch cannot be had."""
+    the kernel reads or writes is not aligned for it or the scratch cannot be had, and in a step that is being captured: its graph would
+    keep the scratch for good."""
     M, glu = x.shape[0], epi in GLU_EPIS
     if epi in (EPI_BF16, *GLU_EPIS) and out.dtype != x.dtype:
         raise ValueError(f"qmatmul: {out.dtype} output with {x.dtype} activations")
     ok = x.stride(0) % 8 == 0 and W.K <= x.stride(0) <= 1 << 22 and out.stride(0) % 4 == 0 and not (x.data_ptr() | out.data_ptr()) & 15
+    ok = ok and not torch.cuda.is_current_stream_capturing()
     cols = min(plan[1], W.N)
     try:
         part = torch.empty(cols, W.K, dtype=torch.float16, device=x.device) if ok else None
@@ -711,7 +713,7 @@ def _large_plan(M: int, N_: int, K: int, qtype: int, can_split: bool):
     return _large_best(M, N_, K, qtype, can_split)[1]
 
 
-X16_MIN_M = 1025  # (steps of up to 1024 rows are captured: their graphs would keep the f16 scratch for good)
+X16_MIN_M = 1025  # (the estimates below are fitted from 1024 rows on)
 X16_SCRATCH = 1 << 28  # bytes of f16 weights expanded at a time
 
 

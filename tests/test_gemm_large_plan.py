@@ -168,3 +168,36 @@ def test_few_rows_by_format():
         assert kind(m, 8192, 28672, QType.Q8_0, True) == "qr" and kind(m, 8192, 28672, QType.Q4_K, True) == "q2"
         assert kind(m, 4096, 14336, QType.Q2_K, True) == "q2" and kind(m, 151936, 1536, QType.Q3_K, True) == "q2"
     assert kind(9, 4096, 14336, QType.Q4_K, True) == "q2" and kind(16, 4096, 14336, QType.Q4_K, True) == "qr"
+
+
+def _launches(monkeypatch):
+    """Names of the kernel entries called from here on."""
+    names, call = [], L.N.kcall
+    monkeypatch.setattr(L.N, "kcall", lambda name, *a: (names.append(name), call(name, *a))[1])
+    return names
+
+
+@pytest.mark.gpu
+def test_expansion_is_not_captured(monkeypatch):
+    """A captured step of more than 1024 rows (256 decode rows beside a chunk of 1024) runs the quantised plan and its graph keeps no
+    scratch; replays give what the eager call of that plan gives."""
+    qt, n, k, M = QType.Q4_K, 288, 1536, 1280  # (the size that the weights of this file are kept in)
+    W, _ = _weight(qt, n, k)
+    x = (torch.randn(M, k, generator=torch.Generator().manual_seed(3)) * 0.5).half().cuda()
+    out, want, plan = torch.zeros(M, n, device="cuda"), torch.zeros(M, n, device="cuda"), ("x16", 512, ("q2", 4, 2, 1, 1))
+    names = _launches(monkeypatch)
+    L.run_plan(plan, W, x, L.EPI_F32, want, False)
+    assert names == ["mxk_t32_expand", "mxk_gemm16"]
+    L.run_plan(plan[2], W, x, L.EPI_F32, want, False)
+    names.clear()
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        L.run_plan(plan, W, x, L.EPI_F32, out, False)
+    assert names == ["mxk_qmm2"]
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
