@@ -65,7 +65,7 @@ def candidates(M: int, N: int, K: int, qtype: int, can_split: bool) -> list[tupl
                 continue
             for s in sp:
                 out.append(("q3", wm, s))
-    if M <= L.QMMR_MAX_M:
+    if M <= L.QMMR_MAX_M and not (L.NORM_FUSE or L.ROPE_FUSE):  # (qmmr has no fused instances)
         for wm, gw, kw in L.QMMR_CONFIGS:
             if 32 * wm <= max(32, M):
                 for s in sp:
@@ -203,7 +203,7 @@ def tune_gemms(specs, buckets=BUCKETS) -> float:
         if key in seen:
             continue
         seen.add(key)
-        ck = ",".join(map(str, key)) + "|" + ",".join(map(str, buckets))
+        ck = ",".join(map(str, key)) + "|" + ",".join(map(str, buckets)) + ("|fused" if L.NORM_FUSE or L.ROPE_FUSE else "")
         if ck in cache:
             TUNED[key] = [(b, tuple(p)) for b, p in cache[ck]]
             continue

@@ -410,7 +410,7 @@ def _t32_plan(W: QWeight, M: int, epi: int, out_zeroed: bool, dtype=torch.float1
             plan = ("rows", ROW_CHUNK)
         else:
             plan = _gemm_pick(M, W.N, W.K, int(W.qtype), can_split)
-            if M >= X16_MIN_M and not forced and dtype == torch.float16:
+            if M >= X16_MIN_M and not forced and not (NORM_FUSE or ROPE_FUSE) and dtype == torch.float16:
                 plan = _expanded_plan(M, W.N, W.K, int(W.qtype), can_split, epi in GLU_EPIS) or plan
     return plan
 
@@ -432,6 +432,7 @@ class NormFuse:
         self.rope = rope
 
 
+# (only qmm2 has the fused instances: with either switch products take neither qmmr nor expanded weights)
 NORM_FUSE = os.environ.get("MX_NORM_FUSE", "0") != "0"
 ROPE_FUSE = os.environ.get("MX_ROPE_FUSE", "0") != "0"
 _NORM_FUSE_QT = None
@@ -787,7 +788,7 @@ def _gemm_pick(M: int, N_: int, K: int, qtype: int, can_split: bool):
         return _large_plan(M, N_, K, qtype, can_split)
     nct = -(-N_ // 128)
     wide = N_ >= 16384
-    if M <= 32 and _few_rows_pick_qmmr(M, N_, K, qtype, can_split):  # 128 columns a workgroup where they fill the chip, else 64 and K splits
+    if M <= 32 and not (NORM_FUSE or ROPE_FUSE) and _few_rows_pick_qmmr(M, N_, K, qtype, can_split):  # 128 columns a workgroup where they fill the chip, else 64 and K splits
         return ("qr", 1, 4, 4, 1) if wide else ("qr", 1, 2, 4, _split_for(-(-N_ // 64), K, can_split))
     if M <= 64 or (not wide and K < 8192 and M <= 256):
         return ("q2", 2, 2, 1, _split_for(-(-M // 64) * nct, K, can_split))

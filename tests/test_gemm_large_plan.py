@@ -122,6 +122,19 @@ def test_expanded_plans_count_rounds_by_piece():
     assert pick(2304, 57344, 8192, True, QType.Q4_K) is None and pick(4096, 8192, 28672, False, QType.Q4_K) is None
 
 
+@pytest.mark.parametrize("switch", ["NORM_FUSE", "ROPE_FUSE"])
+def test_fused_epilogues_keep_their_kernel(switch, monkeypatch):
+    """The RMSNorm and rotation epilogues exist in qmm2 alone: with their switches few and many rows run it, tuned or not."""
+    import types
+    from localai_tfp_amd.ops import autotune as AT
+    W = types.SimpleNamespace(N=4096, K=4096, qtype=int(QType.Q4_K), bf16_cache=None)
+    plans = lambda: {L._t32_plan(W, m, L.EPI_ADD_F32, False)[0] for m in (5, 32, 128, 8191)}  # noqa: E731
+    kinds = lambda: {p[0] for p in AT.candidates(32, 4096, 4096, int(QType.Q4_K), True)}  # noqa: E731
+    assert plans() == {"qr", "q2", "x16"} and "qr" in kinds()
+    monkeypatch.setattr(L, switch, True)
+    assert plans() == {"q2"} and kinds() == {"q2", "q3"}
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("qt", [*QTYPES, QType.Q4_0, QType.Q5_0, QType.Q5_1])
 def test_expanded_products(qt):
