@@ -98,7 +98,8 @@ __global__ __launch_bounds__(256) void allreduce_1shot_kernel(const uint32_t* __
 extern "C" int mxk_ar_alloc(size_t bytes, void** ptr) {
     hipError_t e = hipExtMallocWithFlags(ptr, bytes, hipDeviceMallocUncached);
     if (e != hipSuccess) return (int)e;
-    return (int)hipMemset(*ptr, 0, bytes);
+    if ((e = hipMemset(*ptr, 0, bytes)) != hipSuccess) return (int)e;
+    return (int)hipDeviceSynchronize();  // (the fill need not be over when hipMemset returns, and peers push as soon as they know the buffer)
 }
 extern "C" int mxk_ar_free(void* ptr) { return (int)hipFree(ptr); }
 extern "C" int mxk_ar_ipc_handle(void* ptr, void* out /* 64 B */) {
