@@ -95,13 +95,17 @@ __global__ __launch_bounds__(256) void allreduce_1shot_kernel(const uint32_t* __
 
 // ---- host side ----------------------------------------------------------------------------------
 // Receive buffer: 2 parities x world slots x slot_granules 8-byte granules, uncached device memory.
-extern "C" int mxk_ar_alloc(size_t bytes, void** ptr) {
-    hipError_t e = hipExtMallocWithFlags(ptr, bytes, hipDeviceMallocUncached);
+extern "C" int mxk_ar_clear(void* ptr, size_t bytes) {
+    hipError_t e = hipDeviceSynchronize();  // (calls of the instance that had it before)
+    if (e == hipSuccess) e = hipMemset(ptr, 0, bytes);
     if (e != hipSuccess) return (int)e;
-    if ((e = hipMemset(*ptr, 0, bytes)) != hipSuccess) return (int)e;
     return (int)hipDeviceSynchronize();  // (the fill need not be over when hipMemset returns, and peers push as soon as they know the buffer)
 }
-extern "C" int mxk_ar_free(void* ptr) { return (int)hipFree(ptr); }
+// Not to be freed before the process ends: memory handed out after such a free has held wrong values.
+extern "C" int mxk_ar_alloc(size_t bytes, void** ptr) {
+    const hipError_t e = hipExtMallocWithFlags(ptr, bytes, hipDeviceMallocUncached);
+    return e != hipSuccess ? (int)e : mxk_ar_clear(*ptr, bytes);
+}
 extern "C" int mxk_ar_ipc_handle(void* ptr, void* out /* 64 B */) {
     return (int)hipIpcGetMemHandle((hipIpcMemHandle_t*)out, ptr);
 }

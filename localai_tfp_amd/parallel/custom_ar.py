@@ -24,7 +24,7 @@ from .. import _native as N
 
 _SIGS = {
     "mxk_ar_alloc": [C.c_size_t, C.POINTER(C.c_void_p)],
-    "mxk_ar_free": [C.c_void_p],
+    "mxk_ar_clear": [C.c_void_p, C.c_size_t],
     "mxk_ar_ipc_handle": [C.c_void_p, C.c_void_p],
     "mxk_ar_ipc_open": [C.c_void_p, C.POINTER(C.c_void_p)],
     "mxk_ar_ipc_close": [C.c_void_p],
@@ -77,8 +77,7 @@ class OneShotAllReduce:
             if khz <= 0:
                 raise N.NativeError("one-shot all-reduce: the device's clock rate is not known")
             self.wait_ticks = max(1, int(timeout_s * 1e3 * khz))
-            self.buf = C.c_void_p()
-            _ok(lib.mxk_ar_alloc(2 * self.world * self.slot * 8, C.byref(self.buf)), "mxk_ar_alloc")
+            self.buf = self._buffer(2 * self.world * self.slot * 8)
             self.ptrs = (C.c_void_p * self.world)()
             self._opened = []
             if not solo:
@@ -108,6 +107,21 @@ class OneShotAllReduce:
         self._snap_i = 0
         if not solo:
             dist.barrier(group=group)
+
+    # uncached buffers of closed instances by (device, bytes): never freed (allreduce.hip mxk_ar_alloc), the next instance takes them
+    _spare: dict = {}
+
+    def _buffer(self, nbytes: int):
+        self._key = (torch.cuda.current_device(), nbytes)
+        spare = self._spare.setdefault(self._key, [])
+        try:
+            buf = spare.pop()
+        except IndexError:
+            buf = C.c_void_p()
+            _ok(self.lib.mxk_ar_alloc(nbytes, C.byref(buf)), "mxk_ar_alloc")
+        else:
+            _ok(self.lib.mxk_ar_clear(buf, nbytes), "mxk_ar_clear")
+        return buf
 
     def __call__(self, t: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
         out = t if out is None else out
@@ -187,7 +201,7 @@ class OneShotAllReduce:
             self.lib.mxk_ar_ipc_close(p)
         self._opened = []
         if self.buf:
-            self.lib.mxk_ar_free(self.buf)
+            self._spare[self._key].append(self.buf)
             self.buf = C.c_void_p()
 
     def __del__(self):

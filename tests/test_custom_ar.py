@@ -110,3 +110,25 @@ def test_missing_peer_is_given_up_by_time():
         with pytest.raises(RuntimeError, match="never delivered"):
             ar.check(block=True)
         ar.world, ar.ptrs = 1, (ctypes.c_void_p * 1)(ar.buf)
+
+
+@pytest.mark.gpu
+def test_closed_buffers_are_kept_for_the_next_instance():
+    """Uncached memory that kernels have read is not freed: a closed instance's buffer goes to the next of its size, zeroed, and to no
+    other; epochs that the two share do not read what the first left."""
+    import torch
+    from localai_tfp_amd.parallel.custom_ar import OneShotAllReduce
+    t = torch.randn(4096, device="cuda").half()
+    ptrs = []
+    for nbytes in (40960, 40960, 81920):
+        ar = OneShotAllReduce(None, "cuda", nbytes, world=1)
+        ptrs.append(ar.buf.value)
+        out = torch.zeros_like(t)
+        ar(t, out)
+        torch.cuda.synchronize()
+        assert torch.equal(out, t)
+        ar.check(block=True)
+        ar.close()
+        assert not ar.buf
+        t = t + 1
+    assert ptrs[0] == ptrs[1] != ptrs[2] and not hasattr(ar.lib, "mxk_ar_free")
