@@ -96,7 +96,6 @@ __global__ __launch_bounds__(256, 1) void gemm16_kernel(const uint16_t* __restri
 #pragma unroll
     for (int i = 0; i < 16; ++i) rd(0, 1, 0, i);
 
-    int sa = 0, sb = 1, sf = 4;  // slots of tile t, the free one
     // W8: where among 8 products this wave puts its loads, another place for each wave
     auto mainloop = [&](auto w_c) {
         constexpr int W8 = decltype(w_c)::value;
@@ -147,11 +146,11 @@ __global__ __launch_bounds__(256, 1) void gemm16_kernel(const uint16_t* __restri
 #pragma unroll
                 for (int j = 0; j < 8; j += 2) {
                     if (n0 + 16 * j >= N) break;
-                    float v[4];
+                    uint32_t w[4];  // (each rounded once, product and conversion together, as in qmm2; a packed conversion rounds the product first)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) v[r] = glu_gate_f<EPI>(acc[i][j][r]) * acc[i][j + 1][r];
+                    for (int r = 0; r < 4; ++r) w[r] = f32_to_act<true>(glu_gate_f<EPI>(acc[i][j][r]) * acc[i][j + 1][r]);
                     *(u32x2*)((uint16_t*)Cv + (size_t)(m0 + 16 * i) * ldc + ((n0 + 16 * j - 4 * eg) >> 1) + 4 * eg) =
-                        (u32x2){pack_act2<true>(v[0], v[1]), pack_act2<true>(v[2], v[3])};
+                        (u32x2){w[0] | w[1] << 16, w[2] | w[3] << 16};
                 }
     } else if constexpr (EPI == E16_ACT) {
 #pragma unroll

@@ -214,3 +214,26 @@ def test_expansion_is_not_captured(monkeypatch):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("qt", [*QTYPES, QType.Q4_0, QType.Q5_0, QType.Q5_1])
+def test_expanded_products_equal_the_wide_tiles(qt, monkeypatch):
+    """gemm16.hip adds a sum's products in the order of qmm2's wide tiles (one wave through K) and rounds outputs where they do: every
+    epilogue bit for bit. Five row tiles (a band of four and its rest) and three column tiles in one launch."""
+    n, k, M = 768, 1536, 1100
+    raw = Q.random_quantized(__import__("numpy").random.default_rng(5), int(qt), n, k).reshape(n, -1)
+    W = L.QWeight.from_ggml(raw, int(qt), n, k, "cuda", t32=True)
+    assert W.to_t32()
+    x = (torch.randn(M, k, generator=torch.Generator().manual_seed(1)) * 0.5).half().cuda()
+    base = torch.randn(M, n, generator=torch.Generator().manual_seed(2)).cuda()
+    for epi in (L.EPI_F32, L.EPI_ADD_F32, L.EPI_BF16, L.EPI_SWIGLU, L.EPI_GEGLU):
+        got = []
+        for plan in (("q2", 4, 17, 1, 1), ("x16", n, None)):
+            out = base.clone() if epi in (L.EPI_F32, L.EPI_ADD_F32) else torch.zeros(M, n // 2 if epi in L.GLU_EPIS else n, device="cuda", dtype=torch.float16)
+            names = _launches(monkeypatch)
+            L.run_plan(plan, W, x, epi, out, False)
+            monkeypatch.undo()
+            assert names == (["mxk_t32_expand", "mxk_gemm16"] if plan[0] == "x16" else ["mxk_qmm2"])
+            got.append(out)
+        assert torch.equal(*got), (epi, int((got[0] != got[1]).sum()))
