@@ -307,7 +307,8 @@ __global__ __launch_bounds__(64) void rope_norm_append_kernel(const float* qi, c
         for (int k = 0; k < E; ++k) {
             const int e = lane + k * 64;
             float v = val[i][k];
-            if (e < rot) v = second[k] ? v * cs[k] + other[i][k] * sn[k] : v * cs[k] - other[i][k] * sn[k];
+            // (the mate's product is rounded, the other one is not: written out, since which one is left to the compiler differs by instance)
+            if (e < rot) v = fmaf(v, cs[k], second[k] ? other[i][k] * sn[k] : -(other[i][k] * sn[k]));
             if (e >= dk) v = 0.f;
             val[i][k] = v;
             ss += v * v;

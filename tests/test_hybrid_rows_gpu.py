@@ -208,6 +208,26 @@ def test_rotary_rows_of_wide_heads(dk):
             assert (a - b).abs().max() <= (1e-3 if dt == torch.float32 else 2 ** -7) * max(1.0, float(b.abs().max()))
 
 
+@pytest.mark.parametrize("T,H,dk", [(33, 8, 64), (33, 8, 128), (1300, 32, 128), (33, 4, 192), (33, 4, 512)])
+def test_rotations_round_the_same_in_every_instance(T, H, dk):
+    """x' = x c -+ round(y s) with one rounding of the sum, however many heads share a wave: c and s are read off unit vectors, the rest is
+    float64 (the products of fp32 numbers are exact there; its own rounding can tip one fp32 rounding in 2^28)."""
+    g = torch.Generator().manual_seed(dk + T)
+    pos, slots = torch.randint(0, 3000, (T,), generator=g, dtype=torch.int32).cuda(), torch.zeros(T, dtype=torch.int32, device="cuda")
+
+    def turn(x):
+        out = torch.zeros(T, H * dk, device="cuda")
+        HY.rope_norm_append(x.cuda(), None, None, pos, H, 0, dk, dk, dk, 1e4, False, 1e-6, out, None, None, slots)
+        return out.cpu().view(T, H, dk // 2, 2)
+    unit, x = torch.zeros(T, H * dk), torch.randn(T, H * dk, generator=g)
+    unit[:, ::2] = 1.0
+    cs = turn(unit).double()
+    c, s = cs[..., 0], cs[..., 1]
+    a, b = x.view(T, H, dk // 2, 2).double().unbind(-1)
+    want = torch.stack([a * c - (b * s).float().double(), b * c + (a * s).float().double()], -1).float()
+    assert (turn(x) != want).float().mean() < 1e-6
+
+
 @pytest.mark.parametrize("chunk,window", [(0, 0), (128, 0), (0, 40)])
 def test_chunks_of_many_sequences(chunk, window):
     """The chunks of a step are launched sixteen at a time, the longest first: eighteen sequences (with short ones between, which run on
