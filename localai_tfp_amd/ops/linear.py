@@ -372,9 +372,9 @@ def run_plan(plan: tuple, W: QWeight, x: torch.Tensor, epi: int, out: torch.Tens
 
 
 def _run_x16(plan: tuple, W: QWeight, x: torch.Tensor, epi: int, out: torch.Tensor, out_zeroed: bool):
-    """("x16", columns, plan): gemm16.hip on the weight's rows expanded to f16, `columns` of them at a time; `plan` where what
-    the kernel reads or writes is not aligned for it or the scratch cannot be had, and in a step that is being captured: its graph would
-    keep the scratch for good."""
+    """("x16", columns, plan): gemm16.hip on the weight's rows expanded to f16, `columns` of them at a time; `plan` where the output is not
+    aligned for its 16-byte stores, rows of x overlap or lie more than 8 MB apart, or the scratch cannot be had, and in a step that is
+    being captured: its graph would keep the scratch for good. (Rows of x off 16 bytes are refused by both.)"""
     M, glu = x.shape[0], epi in GLU_EPIS
     if epi in (EPI_BF16, *GLU_EPIS) and out.dtype != x.dtype:
         raise ValueError(f"qmatmul: {out.dtype} output with {x.dtype} activations")

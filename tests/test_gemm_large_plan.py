@@ -138,8 +138,8 @@ def test_fused_epilogues_keep_their_kernel(switch, monkeypatch):
 @pytest.mark.gpu
 @pytest.mark.parametrize("qt", [*QTYPES, QType.Q4_0, QType.Q5_0, QType.Q5_1])
 def test_expanded_products(qt):
-    """gemm16.hip on expanded weights: part-empty tiles of rows and columns, three pieces of columns, every epilogue; and the qmm2 plan
-    for rows that it cannot read as they lie."""
+    """gemm16.hip on expanded weights: part-empty tiles of rows and columns, three pieces of columns, every epilogue, rows that lie
+    together and apart."""
     n, k = 288, 1536
     W, dense = _weight(qt, n, k)
     for M, cols in ((1, 512), (255, 256), (257, 256), (600, 32)):
@@ -237,3 +237,36 @@ def test_expanded_products_equal_the_wide_tiles(qt, monkeypatch):
             assert names == (["mxk_t32_expand", "mxk_gemm16"] if plan[0] == "x16" else ["mxk_qmm2"])
             got.append(out)
         assert torch.equal(*got), (epi, int((got[0] != got[1]).sum()))
+
+
+@pytest.mark.gpu
+def test_expansion_gives_way_to_the_quantised_plan(monkeypatch):
+    """Outputs off 16 bytes or with rows off four numbers, rows that repeat, and no memory for the scratch run the qmm2 plan, with its
+    results; activations off 16 bytes are refused, as qmm2 refuses them."""
+    n, k, M = 288, 1536, 70
+    W, dense = _weight(QType.Q4_K, n, k)
+    x = (torch.randn(M, k, generator=torch.Generator().manual_seed(1)) * 0.5).half()
+    want, plan = x.double() @ dense.double().t(), ("x16", 512, ("q2", 4, 2, 1, 1))
+
+    def run(rows, epi, out, kernel, ref=want):
+        names = _launches(monkeypatch)
+        L.run_plan(plan, W, rows, epi, out, False)
+        monkeypatch.undo()
+        assert names[-1] == kernel and float((out.cpu().double() - ref).norm() / ref.norm()) < 2 * 2 ** -10
+    for epi, dt in ((L.EPI_F32, torch.float32), (L.EPI_BF16, torch.float16)):
+        for left, width, kernel in ((0, n, "mxk_gemm16"), (1, n + 3, "mxk_qmm2"), (0, n + 2, "mxk_qmm2"), (8, n + 8, "mxk_gemm16")):
+            run(x.cuda(), epi, torch.zeros(M, width, device="cuda", dtype=dt)[:, left:left + n], kernel)
+    run(x[:1].cuda().expand(M, k), L.EPI_F32, torch.zeros(M, n, device="cuda"), "mxk_qmm2", want[:1].expand(M, n))
+    out, xd, empty = torch.zeros(M, n, device="cuda"), x.cuda(), torch.empty
+
+    def full(*a, **kw):
+        raise torch.cuda.OutOfMemoryError("none left")
+    monkeypatch.setattr(torch, "empty", full)
+    names = _launches(monkeypatch)
+    L.run_plan(plan, W, xd, L.EPI_F32, out, False)
+    monkeypatch.undo()
+    assert torch.empty is empty and names == ["mxk_qmm2"] and float((out.cpu().double() - want).norm() / want.norm()) < 2 ** -10
+    off = torch.zeros(M, k + 8, device="cuda", dtype=torch.float16)[:, 1:k + 1]
+    for p in (plan, plan[2]):
+        with pytest.raises(L.N.NativeError):
+            L.run_plan(p, W, off, L.EPI_F32, out, False)
