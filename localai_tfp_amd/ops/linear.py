@@ -740,20 +740,29 @@ def _expanded_plan(M: int, N_: int, K: int, qtype: int, can_split: bool, glu: bo
     return None
 
 
+# super-blocks of a qmmr workgroup up to which it is the faster one, at 5 to 15 and 16 to 32 rows
+_QMMR_DEEP = {int(QType.Q4_K): (16, 16), int(QType.Q8_0): (64, 64), int(QType.Q3_K): (6, 16), int(QType.Q5_K): (6, 16),
+              int(QType.MX4F): (6, 16), int(QType.Q2_K): (6, 8), int(QType.Q6_K): (3, 5), int(QType.MX5F): (3, 5)}
+
+
 def _few_rows_pick_qmmr(M: int, N_: int, K: int, qtype: int, can_split: bool) -> bool:
     """Whether an untuned product of up to 32 rows runs qmmr.hip rather than the 64-row qmm2 tile. qmmr decodes in registers at four
-    waves a SIMD and is bound by that; qmm2's tiles wait for their LDS ring. So qmmr wins where a launch is short or its workgroups
-    make one round, and loses with the formats that decode slowest (Q6_K and five-bit MX5F) and where K splits fill the chip for qmm2.
-    qmm2 / qmmr, us, 9 or 16 rows, weights in no cache, eight formats x 43 shapes:
+    waves a SIMD and is bound by that, one workgroup after another through the super-blocks of its split (`deep`); qmm2's tiles wait for
+    their LDS ring, with more workgroups through fewer super-blocks where K can be split. So qmmr wins where it goes through few, where
+    qmm2's splits leave the chip idle and where K is not split, the formats that decode slowest (Q6_K and five-bit MX5F) for fewer, and
+    more rows cost it less. Of 3024 measurements (eight formats, 68 shapes, 5 to 32 rows, weights in no cache) the rule leaves 9 more than
+    1.5 % slower than the other kernel (4 % at most) and 32 more than 2.5 % (6 %; Q8_0 below). qmm2 / qmmr, us, 9 or 16 rows:
       one round of 128-column workgroups (N 16384 .. 32768): 28672 x 4096 gated Q4_K 28 / 20, Q8_0 32 / 25, Q6_K 31 / 28, MX5F 30 / 31;
         20480 x 4096 into the residual (qmm2 splits K) Q6_K 25 / 28, MX5F 25 / 31, others even or better;
       more rounds: 57344 x 8192 Q4_K 90 / 73, Q8_0 102 / 93, Q6_K 96 / 103, MX5F 94 / 116; 128256 x 4096 Q4_K 92 / 84, Q8_0 115 / 102, Q3_K 91 / 93,
-        Q6_K 106 / 113; 37888 x 3584 (1.2 rounds) Q8_0 38 / 41, Q4_K 39 / 33; 151936 x 1536 Q3_K 47 / 54, Q4_K 46.5 / 47.3, MX4F 49 / 47;
+        Q6_K 106 / 113; 37888 x 3584 (1.2 rounds) Q8_0 38 / 41, Q4_K 39 / 33; 151936 x 1536 Q3_K 47 / 54, Q4_K 46.5 / 47.3 (Q8_0 there and
+        at 128256 columns 57-67 / 58 and 105-117 / 102-107 from card to card);
       fewer columns, K not splittable: always qmmr (4096 x 4096 Q4_K 23 / 13, Q6_K 26 / 22);
-      K splittable: 4096 x 4096 Q4_K 8.0 / 6.4, Q6_K at 5 rows 7.9 / 8.1; 2560 x 9728 all formats; 6144 x 4096 at 5 rows Q3_K 9.7 / 10.2, Q6_K
-        10.3 / 12.8, at 16 Q3_K 10.2 / 10.1; 4096 x 14336 at 16 rows Q4_K 15.5 / 15.0, Q2_K 14.6 / 16.0, Q6_K 17 / 21; 8192 x 28672 Q4_K 46 / 48, Q6_K
-        50 / 73, Q8_0 54 / 52."""
-    heavy, weights = qtype in (int(QType.Q6_K), int(QType.MX5F)), N_ * K
+      K splittable, super-blocks a workgroup: 3584 x 3584 (4, qmm2 on 112 units) Q6_K 9.4 / 7.5; 4096 x 4096 (4) Q4_K 8.0 / 6.4, Q6_K at 5 rows
+        7.9 / 8.1, at 16 8.7 / 8.1; 6144 x 4096 (8) Q4_K even, Q3_K 9.7 / 10.1, at 20 10.4 / 10.1, Q6_K 10.3 / 12.8; 4096 x 14336 (14) Q4_K at 20
+        16.0 / 14.9, Q2_K 14.6 / 16.0, Q6_K 17 / 21; 3072 x 24576 (24) Q3_K 22 / 23, Q6_K 23 / 33; 8192 x 28672 (56) Q4_K 46 / 48, Q6_K 50 / 73, Q8_0
+        54 / 52."""
+    heavy = qtype in (int(QType.Q6_K), int(QType.MX5F))
     if N_ > 32768:
         if heavy:
             return False
@@ -761,18 +770,26 @@ def _few_rows_pick_qmmr(M: int, N_: int, K: int, qtype: int, can_split: bool) ->
             return True
         if qtype == int(QType.Q4_K):
             return K >= 3072
-        return K >= 4096 and N_ >= 49152 and (N_ < 98304 or qtype == int(QType.Q8_0))
+        return K >= 4096 and N_ >= 49152 and (N_ < 98304 or qtype == int(QType.Q8_0) and M <= 16)
     if N_ >= 16384:
         if qtype == int(QType.MX5F):
-            return weights <= 1 << 24 and not can_split
+            return N_ * K <= 1 << 24 and not can_split
         return qtype != int(QType.Q6_K) or not can_split or N_ >= 24576
-    if not can_split or qtype == int(QType.Q8_0):
+    if not can_split:
         return True
-    if heavy:
-        return weights <= 15_000_000 and N_ <= 5120
-    if weights <= 25_000_000 and (N_ <= 12288 or M >= 16):
+    tiles = -(-N_ // 128)
+    if tiles * _split_for(tiles, K, True) <= 128:
         return True
-    return M >= 16 and weights <= (1 << 25 if qtype == int(QType.Q2_K) else 60_000_000)
+    groups = -(-N_ // 64)
+    splits = _split_for(groups, K, True)
+    deep = -(-(K // 256) // splits)
+    if splits == 1 and qtype not in (int(QType.Q4_K), int(QType.Q8_0)):
+        return deep <= 4 and M >= (24 if heavy else 12) or deep <= 8 and M >= 20 and not heavy
+    if groups * splits > CU_COUNT and not heavy and qtype != int(QType.Q2_K):
+        return deep <= 16
+    if qtype == int(QType.Q6_K) and (deep <= 5 and groups * splits > CU_COUNT or deep <= 6 and M >= 24):
+        return True
+    return deep <= _QMMR_DEEP[qtype][M >= 16]
 
 
 def _gemm_pick(M: int, N_: int, K: int, qtype: int, can_split: bool):

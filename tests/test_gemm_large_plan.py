@@ -180,7 +180,9 @@ def test_few_rows_by_format():
             assert kind(m, 28672, 4096, qt) == kind(m, 57344, 8192, qt) == kind(m, 4096, 4096, qt, True) == "qr"
         assert kind(m, 8192, 28672, QType.Q8_0, True) == "qr" and kind(m, 8192, 28672, QType.Q4_K, True) == "q2"
         assert kind(m, 4096, 14336, QType.Q2_K, True) == "q2" and kind(m, 151936, 1536, QType.Q3_K, True) == "q2"
-    assert kind(9, 4096, 14336, QType.Q4_K, True) == "q2" and kind(16, 4096, 14336, QType.Q4_K, True) == "qr"
+    assert kind(9, 6144, 4096, QType.Q3_K, True) == "q2" and kind(16, 6144, 4096, QType.Q3_K, True) == kind(9, 4096, 14336, QType.Q4_K, True) == "qr"
+    assert kind(5, 3584, 3584, QType.Q6_K, True) == kind(16, 4096, 4096, QType.Q6_K, True) == "qr" and kind(5, 4096, 4096, QType.Q6_K, True) == "q2"
+    assert kind(5, 14336, 1024, QType.MX4F, True) == "q2" and kind(12, 14336, 1024, QType.MX4F, True) == "qr"
 
 
 def _launches(monkeypatch):
