@@ -1,0 +1,136 @@
+// dense16_impl.h — products of a 16-bit matrix's rows with 16-bit weights: the kernel of dense16.hip (what it is for and its times stand
+// there) over g16_tile's tiles. Tiles whose K is split over workgroups leave their sums in `part`; dense16_sum_kernel adds them in order.
+#pragma once
+#include "gemm16_impl.h"
+
+namespace {
+
+enum { D16_F32 = 0, D16_ADD = 1, D16_GLU = 4, D16_PART = 5 };
+
+struct D16Args {
+    const uint16_t *A, *B;
+    int lda, ldb, M, N, nk;  // N: columns of C; nk 64-wide k-tiles
+    int n_mt, n_nt;          // tiles of C
+    int full, parts;         // tiles from `full` on are summed in `parts` parts of K
+    float* part;             // [tile - full][part][TM][TN]
+    const float* bias;       // of C's columns, or null
+    float* C;
+    int ldc;
+    // gated columns (D16_GLU): G[m, f] = silu(A · B[gate0 + f] + gate_b[f]) (A · B[up0 + f] + up_b[f]) in 16 bits, beside C
+    int g_nt, F, gate0, up0;
+    const float *gate_b, *up_b;
+    uint16_t* G;
+    int ldg;
+};
+
+MX_DEV float d16_silu(float x) { return x / (1.f + expf(-x)); }
+
+template <int EPI, bool F16, int MI, int NJ>
+__global__ __launch_bounds__(256, 1) void dense16_kernel(D16Args a) {
+    using T = G16T<MI, NJ>;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int bid = blockIdx.x;
+    int tile = g16_lid(bid, gridDim.x), p = 0, np = 1;
+    if constexpr (EPI == D16_PART) {
+        np = a.parts;
+        p = tile % np;
+        tile = a.full + tile / np;
+    }
+    const int gt = EPI == D16_GLU || EPI == D16_PART ? a.n_mt * a.g_nt : 0;
+    const bool glu = EPI == D16_GLU && tile < gt;
+    int mt, nt;
+    q2_tile_of(glu ? tile : tile - gt, a.n_mt, glu ? a.g_nt : a.n_nt, mt, nt);
+    const int m_base = mt * T::TM, n_base = nt * T::TN;
+    const int k0 = (int)((long)a.nk * p / np), k1 = (int)((long)a.nk * (p + 1) / np);
+    const char* ab = (const char*)(a.A + (size_t)m_base * a.lda) + (size_t)k0 * 128;
+    const char* bb = (const char*)(a.B + (glu ? (size_t)0 : (size_t)n_base * a.ldb)) + (size_t)k0 * 128;
+    f32x4 acc[MI][NJ];
+    // up to 64 rows workgroups start at different k-tiles: in step, all of them read the same few channels of memory (40992 x 4096, 33 rows 74.4
+    // -> 67.3 us, 64 rows 78 -> 72.8; more rows lose, since row tiles of the same columns then meet in no cache: 1990 rows 572 -> 600)
+    constexpr bool ROT = MI <= 2 && EPI != D16_PART;
+    g16_tile<F16, MI, NJ, ROT>(
+        smem, ab, bb, k1 - k0, [&](int r) { return (uint32_t)min(r, a.M - 1 - m_base) * (uint32_t)(2 * a.lda); },
+        [&](int r) {
+            // gated: rows in 16-row groups, an even one gates and the next one the ups of the same features
+            if (EPI == D16_GLU && glu) {
+                const int f = min(nt * (T::TN / 2) + (r >> 5) * 16 + (r & 15), a.F - 1);
+                return (uint32_t)((r & 16 ? a.up0 : a.gate0) + f) * (uint32_t)(2 * a.ldb);
+            }
+            return (uint32_t)min(r, a.N - 1 - n_base) * (uint32_t)(2 * a.ldb);
+        },
+        acc, ROT ? (int)(bid * 17u % (unsigned)(k1 - k0)) : 0);
+
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int el = threadIdx.x & 63;
+    asm volatile("" : "+v"(el));  // (no address of it computed ahead of the loop, whose registers are all taken)
+    const int eg = el >> 4, wm = wave >> 1, wn = wave & 1;
+    const int m0 = m_base + wm * (16 * MI) + (el & 15), n0 = n_base + wn * (16 * NJ) + 4 * eg;
+    if constexpr (EPI == D16_GLU && NJ % 2 == 0) {
+        if (glu) {
+            const int f0 = nt * (T::TN / 2) + wn * (8 * NJ) + 4 * eg;
+#pragma unroll
+            for (int j = 0; j < NJ / 2; ++j) {
+                const int f = f0 + 16 * j, fc = min(f, a.F - 4);
+                const f32x4 gb = a.gate_b ? *(const f32x4*)(a.gate_b + fc) : (f32x4){0.f, 0.f, 0.f, 0.f};
+                const f32x4 ub = a.up_b ? *(const f32x4*)(a.up_b + fc) : (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int i = 0; i < MI; ++i) {
+                    float v[4];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[r] = d16_silu(acc[i][2 * j][r] + gb[r]) * (acc[i][2 * j + 1][r] + ub[r]);
+                    if (m0 + 16 * i < a.M && f < a.F)
+                        *(u32x2*)(a.G + (size_t)(m0 + 16 * i) * a.ldg + f) = (u32x2){pack_act2<F16>(v[0], v[1]), pack_act2<F16>(v[2], v[3])};
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            return;
+        }
+    }
+    // fp32 rows, or a part's sums
+    float* C = a.C;
+    int ldc = a.ldc;
+    if constexpr (EPI == D16_PART) {
+        C = a.part + ((size_t)(tile - a.full) * np + p) * (T::TM * T::TN) - ((size_t)m_base * T::TN + n_base);
+        ldc = T::TN;
+    }
+    f32x4 b[NJ], old[2][NJ];
+    if constexpr (EPI != D16_PART)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+            b[j] = a.bias ? *(const f32x4*)(a.bias + min(n0 + 16 * j, a.N - 4)) : (f32x4){0.f, 0.f, 0.f, 0.f};
+    auto load = [&](int i) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)  // (past M / N: the last ones)
+            old[i & 1][j] = *(const f32x4*)(C + (size_t)min(m0 + 16 * i, a.M - 1) * ldc + min(n0 + 16 * j, a.N - 4));
+    };
+    if constexpr (EPI == D16_ADD) load(0);
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+        if constexpr (EPI == D16_ADD)
+            if (i < MI - 1) load(i + 1);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            f32x4 v = acc[i][j];
+            asm volatile("" : "+v"(v));  // (stored from there: from where they are, the loop spills)
+            if constexpr (EPI != D16_PART) v += b[j];
+            if constexpr (EPI == D16_ADD) v += old[i & 1][j];
+            if (m0 + 16 * i < a.M && n0 + 16 * j < a.N) *(f32x4*)(C + (size_t)(m0 + 16 * i) * ldc + n0 + 16 * j) = v;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+#define D16_TILES(GO) GO(8, 8) GO(7, 8) GO(6, 8) GO(5, 8) GO(8, 6) GO(6, 6) GO(8, 4) GO(5, 4) GO(4, 4) GO(2, 8) GO(2, 4)
+
+template <int EPI, bool F16, int MI, int NJ>
+void dense16_launch(const D16Args& a, unsigned n, hipStream_t st) {
+    using T = G16T<MI, NJ>;
+    static const hipError_t attr = hipFuncSetAttribute((const void*)dense16_kernel<EPI, F16, MI, NJ>, hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS);
+    (void)attr;
+    dense16_kernel<EPI, F16, MI, NJ><<<dim3(n), 256, T::LDS, st>>>(a);
+}
+
+}  // namespace
+
+// n workgroups of the gated kernel (dense16_glu.hip); tile 16 MI + NJ
+void mx_dense16_glu(const void* args, int tile, unsigned n, hipStream_t st);

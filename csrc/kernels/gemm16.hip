@@ -17,122 +17,27 @@
 //     16 rows ahead (read just before each store the epilogue of 4096 columns took 110 us of 310, now 15).
 // Measured at 8191 rows, us, expansion apart: gate|up 28672 x 4096 with SwiGLU 1370 (1.40 PFLOP/s; the library's product without it
 // 1304), 4096 x 14336 with the residual 688, 4096 x 4096 215, 5120 x 4096 275.
-#include "qmm2_fmt.h"
+#include "gemm16_impl.h"
 
 namespace {
-
-constexpr int G16_K = 64;                  // k of a tile
-constexpr int G16_NS = 5;                  // ring slots: A of tile t in 2 t mod 5, B in 2 t + 1 mod 5
-constexpr int G16_SLOT = 256 * 128;        // 256 rows of 128 bytes
-constexpr int G16_LDS = G16_NS * G16_SLOT; // all 160 KB
-
-// lane l: 16 bytes from the scalar base plus the lane's offset to LDS dst + 16 l
-MX_DEV void g16_dma(const void* base, uint32_t off, uint32_t dst) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(dst) : "memory", "m0");
-}
-
-MX_DEV f32x4 g16_mfma(u32x4 a, u32x4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-}
 
 template <int EPI>
 __global__ __launch_bounds__(256, 1) void gemm16_kernel(const uint16_t* __restrict__ A, int lda, const uint16_t* __restrict__ B, int ldb,
                                                         int M, int N, int K, int n_mt, void* __restrict__ Cv, int ldc) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int g = lane >> 4, col = lane & 15;
     const int wm = wave >> 1, wn = wave & 1;
 
     // consecutive logical ids run on one XCD, row tiles in bands (q2_tile_of)
-    const int nwg = gridDim.x, bid = blockIdx.x;
-    const int xcd = bid & 7, q8 = nwg >> 3, r8 = nwg & 7;
-    const int lid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (bid >> 3);
+    const int nwg = gridDim.x, lid = g16_lid(blockIdx.x, nwg);
     int mt, nt;
     q2_tile_of(lid, n_mt, nwg / n_mt, mt, nt);
     const int m_base = mt * 256, n_base = nt * 256;
-    const int nk = K / G16_K;
-
-    // DMA instruction i of a wave brings rows 64 wave + 8 i .. + 7: lane l chunk (l & 7) of row l >> 3, taken from the row's chunk
-    // (l & 7) ^ ((row >> 1) & 7), so that 16 rows of one chunk lie in 16 bank quads. Rows past M / N repeat the last.
-    uint32_t ao[8], bo[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int row = 64 * wave + 8 * i + (lane >> 3), c = (lane & 7) ^ (4 * (i & 1) + (lane >> 4));
-        ao[i] = (uint32_t)min(row, M - 1 - m_base) * (uint32_t)(2 * lda) + 16 * c;
-        bo[i] = (uint32_t)min(row, N - 1 - n_base) * (uint32_t)(2 * ldb) + 16 * c;
-    }
-    const char* ab = (const char*)(A + (size_t)m_base * lda);
-    const char* bb = (const char*)(B + (size_t)n_base * ldb);
-    const uint32_t wdst = (uint32_t)(uintptr_t)(MX_LDS char*)smem + wave * 8192;
-    // instruction i of tile t's A or B into ring slot s; past the end the last tile again, never read
-    auto dma_a = [&](int t, int s, int i) { g16_dma(ab + (size_t)min(t, nk - 1) * 128, ao[i], wdst + s * G16_SLOT + i * 1024); };
-    auto dma_b = [&](int t, int s, int i) { g16_dma(bb + (size_t)min(t, nk - 1) * 128, bo[i], wdst + s * G16_SLOT + i * 1024); };
-
     f32x4 acc[8][8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
-    // fragment reads: row's chunk 4 ks + g at (4 ks + g) ^ ((row >> 1) & 7)
-    const uint32_t fx = (uint32_t)((g ^ ((col >> 1) & 7)) << 4);
-    const uint32_t a_rd = (uint32_t)((wm * 128 + col) * 128), b_rd = (uint32_t)((wn * 128 + col) * 128);
-    u32x4 f[2][16];  // of the two k-steps: [8 of A, 8 of B]
-    auto rd = [&](int sa, int sb, int ks, int i) {
-        const char* p = smem + (i < 8 ? sa : sb) * G16_SLOT + (i < 8 ? a_rd : b_rd) + (i & 7) * 2048 + (fx ^ (ks * 64));
-        f[ks][i] = *(const u32x4*)p;
-    };
-    auto next = [](int s) { return s >= G16_NS - 2 ? s - (G16_NS - 2) : s + 2; };
-
-#pragma unroll
-    for (int i = 0; i < 8; ++i) dma_a(0, 0, i);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) dma_b(0, 1, i);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) dma_a(1, 2, i);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) dma_b(1, 3, i);
-    q2_wait_barrier<16>();
-#pragma unroll
-    for (int i = 0; i < 16; ++i) rd(0, 1, 0, i);
-
-    // W8: where among 8 products this wave puts its loads, another place for each wave
-    auto mainloop = [&](auto w_c) {
-        constexpr int W8 = decltype(w_c)::value;
-        int sa = 0, sb = 1, sf = 4;  // slots of tile t's A and B, and the free one
-        for (int t = 0; t < nk; ++t) {
-            const int na = next(sa), nb = next(sb);
-            auto step = [&](auto ks_c, auto beside) {
-                constexpr int ks = decltype(ks_c)::value;
-#pragma unroll
-                for (int m = 0; m < 64; ++m) {
-                    const int i = m >> 3, j = m & 7;
-                    acc[i][j] = g16_mfma(f[ks][8 + j], f[ks][i], acc[i][j]);  // (C^T: a lane's four sums are columns)
-                    beside(m);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            };
-            step(std::integral_constant<int, 0>{}, [&](int m) {
-                if (m < 48 && m % 3 == 0) rd(sa, sb, 1, m / 3);
-                if (m % 8 == W8) dma_a(t + 2, sf, m >> 3);
-            });
-            // A and B of tile t + 1 have landed (A of t + 2 may be on its way), and every wave holds what it needs of tile t: B of
-            // t + 2 follows into A's slot, A of t + 3 into B's
-            asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            step(std::integral_constant<int, 1>{}, [&](int m) {
-                if (m < 48 && m % 3 == 0) rd(na, nb, 0, m / 3);
-                if (m % 8 == W8) dma_b(t + 2, sa, m >> 3);
-            });
-            sf = sb;
-            sa = na;
-            sb = nb;
-        }
-    };
-    if (wave == 0) mainloop(std::integral_constant<int, 1>{});
-    else if (wave == 1) mainloop(std::integral_constant<int, 3>{});
-    else if (wave == 2) mainloop(std::integral_constant<int, 5>{});
-    else mainloop(std::integral_constant<int, 7>{});
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    g16_tile<true, 8, 8>(
+        smem, (const char*)(A + (size_t)m_base * lda), (const char*)(B + (size_t)n_base * ldb), K / G16_K,
+        [&](int r) { return (uint32_t)min(r, M - 1 - m_base) * (uint32_t)(2 * lda); },
+        [&](int r) { return (uint32_t)min(r, N - 1 - n_base) * (uint32_t)(2 * ldb); }, acc);
 
     // ---- epilogue: lane holds columns nb + 4 g .. + 3 of row mb + col; the residual's rows a block ahead of their stores ----
     int el = lane;
@@ -176,14 +81,15 @@ __global__ __launch_bounds__(256, 1) void gemm16_kernel(const uint16_t* __restri
                 if (i < 7) load(i + 1);
 #pragma unroll
                 for (int j = 0; j < 8; ++j) acc[i][j] += old[i & 1][j];
-            } else {
-#pragma unroll
-                for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(acc[i][j]));  // (stored from there: from where they are, the loop spills)
             }
             if (m0 + 16 * i < M)
 #pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    if (n0 + 16 * j < N) *(f32x4*)((float*)Cv + (size_t)(m0 + 16 * i) * ldc + n0 + 16 * j) = acc[i][j];
+                for (int j = 0; j < 8; ++j) {
+                    f32x4 v = acc[i][j];
+                    asm volatile("" : "+v"(v));  // (stored from there: from where they are, the loop spills)
+                    if (n0 + 16 * j < N) *(f32x4*)((float*)Cv + (size_t)(m0 + 16 * i) * ldc + n0 + 16 * j) = v;
+                }
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
 }
@@ -195,10 +101,10 @@ int launch_gemm16(const uint16_t* A, int lda, const uint16_t* B, int ldb, int M,
     if (nwg > 0x7fffffff) return (int)hipErrorInvalidValue;
     static bool attr_set = false;
     if (!attr_set) {
-        (void)hipFuncSetAttribute((const void*)gemm16_kernel<EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, G16_LDS);
+        (void)hipFuncSetAttribute((const void*)gemm16_kernel<EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, G16T<8, 8>::LDS);
         attr_set = true;
     }
-    gemm16_kernel<EPI><<<dim3((unsigned)nwg), 256, G16_LDS, st>>>(A, lda, B, ldb, M, N, K, n_mt, C, ldc);
+    gemm16_kernel<EPI><<<dim3((unsigned)nwg), 256, G16T<8, 8>::LDS, st>>>(A, lda, B, ldb, M, N, K, n_mt, C, ldc);
     MXK_CHECK_LAUNCH();
 }
 

@@ -45,6 +45,7 @@ KERNEL_SIGS = {
     "mxk_qmmr": [I, I, I, I, I, P, I, P, I, I, I, I, P, I, P],
     "mxk_t32_expand": [I, P, I, I, P, P],
     "mxk_gemm16": [I, P, I, P, I, I, I, I, P, I, P],
+    "mxk_dense16": [I, I, P, I, P, I, I, I, I, P, P, I, I, I, P, I, I, I, P, P, P, I, P],
     "mxk_sample_trace": [I, P],
     "mxk_qmv1_enable": [I],
     "mxk_qmv1_rope": [I, P, P, F, P, I, I, I, P, P, P, P, F, I, I, I, P, P, P, I, I, P, P, P],

@@ -24,11 +24,11 @@ the embedding output is added to the residual before each pass but the first.
 How a layer maps onto launches (T rows of a ragged engine step):
 
     norm                      -> hin (GEMM operand)                                   hybrid_ops.hip
-    y = hin W_in^T            every projection that reads h, stacked into ONE GEMM    hipBLASLt, fp32 out
+    y = hin W_in^T            every projection that reads h, stacked into ONE GEMM    dense16.hip / hipBLASLt, fp32 out
     left:  rope + head norm + paged append; masked attention -> cat[:, left]          hybrid_ops / hybrid_attn.hip
     right: conv + SiLU (q|k|v stacked); unit norms; decay / beta; scan; head norm * silu(g) -> cat[:, right]
     mamba2: conv + SiLU over x|B|C; decay / dt; scan (+ D x); silu(z) gate + group norm -> cat[:, mixer]
-    ff:    glu -> cat[:, ff] (dense: biases; moe: router -> dense [T, E] routing weights, every expert's gate/up
+    ff:    glu -> cat[:, ff] (dense: biases, on the GPU mostly in the input GEMM's epilogue; moe: router -> dense [T, E] routing weights, every expert's gate/up
            evaluated from the stacked GEMM and its activation scaled by its routing weight, 0 when not chosen;
            shared expert scaled by its sigmoid gate)
     x += cat W_out^T (+ bias) every output projection (left o, right o, down, shared down, all experts' down
@@ -117,6 +117,12 @@ class VugotarLayerCfg:
     type: str  # parallel | mamba2
     mixer: ParallelCfg | Mamba2Cfg
     mlp: MlpCfg | None
+
+    @property
+    def mixer_out(self) -> int:
+        """Columns of the output GEMM's operand that the mixer fills; the feed-forward's follow."""
+        m = self.mixer
+        return m.inner if self.type == "mamba2" else m.left.heads * m.left.vdim + m.right.heads * m.right.vdim
 
 
 def _need(cond: bool, what: str):
@@ -501,18 +507,23 @@ class VugotarModel:
                 HY.embed_rows(self.embed, fb.tokens, x, accumulate=True)
             HY.offset_rmsnorm(x, W.norm, eps, out32=None if b16 else hin, out16=hin if b16 else None)
             y = ws.y[:T * W.n_in].view(T, W.n_in)
-            W.w_in.into(hin, y)
             cat = ws.cat[:T * W.k_out].view(T, W.k_out)
-            c = W.cols
+            c, f = W.cols, L.mlp
+            glu = False  # the gated unit is done by the input GEMM
+            if f is not None and f.kind == "dense":
+                k0 = L.mixer_out
+                glu = W.w_in.gated(hin, y[:, :c["gate"]], c["gate"], c["up"], W.gate_b, W.up_b, cat[:, k0:k0 + f.ff])
+            if not glu:
+                W.w_in.into(hin, y)
             if L.type == "parallel":
                 k0 = self._left(L.mixer, y, c, fb, rag, kv, ws, cat, eps)
                 k0 = self._right(L.mixer, W, y, c, rag, state, tails, ws, cat, k0, eps)
             else:
                 k0 = self._mamba2(L.mixer, W, y, c, rag, state, tails, ws, cat, eps)
-            f = L.mlp
             if f is not None and f.kind == "dense":
-                HY.glu(y[:, c["gate"]:c["gate"] + f.ff], y[:, c["up"]:c["up"] + f.ff], W.gate_b, W.up_b,
-                       cat[:, k0:k0 + f.ff])
+                if not glu:
+                    HY.glu(y[:, c["gate"]:c["gate"] + f.ff], y[:, c["up"]:c["up"] + f.ff], W.gate_b, W.up_b,
+                           cat[:, k0:k0 + f.ff])
             elif f is not None:
                 if f.shared_ff:
                     Fs = f.shared_ff

@@ -1,15 +1,18 @@
 """Dense 16-bit layers for the non-LLM model families (BERT, Whisper, CLIP/T5 text encoders, UNet /
-MMDiT, VAE, TTS): plain library GEMMs on hipBLASLt (few rows by matrices it is slow on: lin16.hip) with the bias folded into
-the GEMM, fp32 accumulation into the residual stream, and the library's act16 activations.
+MMDiT, VAE, TTS): plain library GEMMs on hipBLASLt (bf16 products of long K or many columns: dense16.hip; few rows by other
+matrices the library is slow on: lin16.hip) with the bias folded into the GEMM, fp32 accumulation into the residual stream, and the
+library's act16 activations.
 
 On CPU everything runs in fp32 (the numerics oracle for the tests)."""
 from __future__ import annotations
+
+import functools
 
 import numpy as np
 import torch
 import torch.nn.functional as F
 
-from .linear import ACT_DTYPE, _fp32_out_ok
+from .linear import ACT_DTYPE, CU_COUNT, _fp32_out_ok
 
 
 def model_dtype(device) -> torch.dtype:
@@ -59,6 +62,130 @@ def _few_rows(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, acc: bool) ->
     part = torch.empty(parts, M, N_, dtype=torch.float32, device=x.device) if parts > 1 else None
     N.kcall("mxk_lin16", x.data_ptr(), ldx, w.data_ptr(), out.data_ptr(), out.stride(0), N.ptr(part), parts, M, N_, K,
             int(x.dtype == torch.float16), int(acc), N.stream_ptr())
+    return True
+
+
+# dense16.hip's tiles (16-row units, 16-column units of a wave): us a 64-wide k-tile and a round of workgroups, us to fill and drain a
+# round, share of a round that its first workgroup takes, us and us a MB for the sum of parts, us for parts behind whole tiles. Fitted to
+# 6300 measurements (26 shapes 1024 x 2048 .. 151936 x 1536, 1 to 4000 rows, weights in no cache): the pick is 1.5 % slower than the best
+# of them on average.
+_D16_COST = {(8, 8): (1.352, 16.3, 0.68, 1.0, 0.075, 3.7), (7, 8): (1.245, 14.4, 0.69, 1.1, 0.087, 2.6), (6, 8): (1.18, 11.2, 0.68, 2.8, 0.095, 0.0),
+             (5, 8): (1.11, 8.4, 0.66, 3.5, 0.116, 0.0), (8, 6): (1.083, 12.8, 0.69, 1.0, 0.097, 0.0), (6, 6): (0.977, 8.7, 0.65, 2.6, 0.118, 0.0),
+             (8, 4): (0.872, 8.1, 0.65, 3.4, 0.106, 0.0), (5, 4): (0.578, 7.2, 0.62, 2.1, 0.184, 0.0), (4, 4): (0.527, 6.0, 0.62, 1.9, 0.247, 0.0),
+             (2, 4): (0.5, 3.4, 0.48, 2.8, 0.246, 0.9)}
+
+
+@functools.lru_cache(maxsize=4096)
+def dense16_plan(M: int, N_: int, K: int, Fn: int = 0):
+    """(16-row units, 16-column units, whole tiles, parts of K of the others) of dense16.hip's tiles for M rows by N_ columns and Fn gated
+    ones. Parts of K keep every compute unit at work where tiles leave some idle; only plain columns can have them. One round of parts
+    at most, so their sums take at most 64 MB.
+
+    Up to 64 rows the weights' bytes bound the product: 64-row tiles, 256 columns wide where 128 make more than one round of workgroups
+    and these do not (us, 128 / 256 wide: 28672 x 4096 45 / 54, 40992 x 4096 74 / 64, 50304 x 2048 41 / 39.5, 128256 x 4096 177 / 194); by long K
+    in up to 8 parts (4096 x 20480 at 33 rows 1 / 4 / 8 parts 120 / 46 / 38)."""
+    nk = K // 64
+
+    def tiles(mi, nj):
+        return -(-M // (32 * mi)), -(-N_ // (32 * nj)), -(-2 * Fn // (32 * nj))
+    if M <= 64:
+        _, n, g = tiles(2, 4)
+        if not Fn and K >= 2 * N_:
+            return 2, 4, 0, max(1, min(8, CU_COUNT // n, nk))
+        wide = sum(tiles(2, 8)[1:])
+        return (2, 8, wide, 1) if n + g > CU_COUNT >= wide else (2, 4, n + g, 1)
+    floor = (2 * K * (N_ + 2 * Fn + M) + 4 * M * N_ + 2 * M * Fn) / 5.6e6 + 4  # us: every byte once
+    best = None
+    for (mi, nj), (a, fill, first, e1, e2, e3) in _D16_COST.items():
+        m, n, g = tiles(mi, nj)
+        t = m * (n + g)
+        for parts in (1, 2, 3, 4, 6, 8):
+            whole = t if parts == 1 else t // CU_COUNT * CU_COUNT
+            rest = t - whole
+            if parts > 1 and (not rest or rest > m * n or parts > nk or rest * parts > CU_COUNT):
+                continue
+
+            def rounds(w):
+                full, rem = divmod(w, CU_COUNT)
+                return full + (first + (1 - first) * rem / CU_COUNT if rem else 0.0)
+            us = rounds(whole) * nk * a + -(-whole // CU_COUNT) * fill
+            if rest:
+                us += rounds(rest * parts) * -(-nk // parts) * a + fill + e1 + (e3 if whole else 0.0) + e2 * rest * parts * min(M, 32 * mi) * 32 * nj * 8e-6
+            us = (us ** 4 + floor ** 4) ** 0.25
+            if best is None or us < best[0]:
+                best = us, (mi, nj, whole, parts)
+    return best[1]
+
+
+def takes_dense16(M: int, N_: int, K: int) -> bool:
+    """Whether x w^T (bf16, fp32 out) runs dense16.hip. Measured beside the library's products in a graph, weights in no cache, us
+    (library / here): long K, whose columns leave compute units idle or to products the library splits badly, 4096 x 20480 at 4 / 64 / 240 /
+    944 / 1768 rows 56 / 35, 127 / 39, 225 / 58, 233 / 146, 381 / 241 (2351 and 3069 rows 333 / 336, 370 / 372), 5120 x 13824 at 64 / 101 / 693 / 3289
+    47 / 34, 63 / 38, 123 / 96, 681 / 344 (up to 16 rows even), 2048 x 10240 at 64 / 512 / 2123 23 / 18, 49 / 37, 102 / 88 (8 rows 12.5 / 14), 1536 x 9216
+    at 121 / 891 20 / 17, 43 / 36 (75 rows 15.4 / 16.4). Many columns by up to 64 rows: 28672 x 4096 at 5 / 33 rows 60 / 45, 50 / 46, 32000 60 / 53, 65536
+    119 / 101, 123 / 103, 128256 187 / 181, 208 / 191, 50304 x 2048 48 / 40, 50 / 42, 151936 x 1536 161 / 89, 112 / 105; by up to 16 rows also 24576 x
+    3072 49 / 30 (33 rows 32.2 / 32.3) and 25000 x 5120 69 / 47 (33 rows 50 / 52). The rest is the library's: 2048 x 2048 .. 4096 x 4096 are 5 to
+    20 % slower here, 8192 x 8192 0.84 to 1.17, wide matrices by 65 to 300 rows 0.8 to 1.0, by more rows 0.9 to 1.5 as its choice falls."""
+    if K % 64 or N_ % 4 or M <= 0 or K < 64:
+        return False
+    if K >= 2 * N_:
+        return M >= (1 if K > 16384 else 64) and N_ * K >= 1 << 24 or M >= 96 and N_ * K >= 12 << 20
+    if N_ >= 24576 and M <= 64:
+        return K <= 2048 or K <= 4096 and N_ >= 28672 or K <= 5120 and M <= 16
+    return False
+
+
+def takes_gated16(M: int, N_: int, K: int, Fn: int) -> bool:
+    """Whether a projection's N_ plain columns and its gated unit of Fn features run as one launch of dense16.hip. us, the library's product
+    and the gating kernel / here: 12320 + 2 x 14336 columns x 4096 at 1 / 33 / 112 / 322 / 703 / 2062 rows 76 / 64, 78 / 67, 92 / 88, 214 / 143, 334 / 227,
+    733 / 641, 6176 + 2 x 8192 x 2048 at 5 / 33 / 310 / 1693 / 3557 38 / 22, 29 / 23, 50 / 47, 197 / 158, 407 / 307 (184 rows 41 / 42), 9000 + 2 x 20000 x
+    6144 134 / 111, 145 / 110, 194 / 165 (239 rows); 3000 + 2 x 5632 x 2048 even up to 64 rows (20 / 20 and 20.6 / 21.5), 465 rows 52 / 40."""
+    return M > 0 and K % 64 == 0 and K >= 512 and N_ > 0 and N_ % 4 == 0 and Fn % 4 == 0 and Fn > 0 and (N_ + 2 * Fn) * K >= (1 << 22 if M > 64 else 1 << 25)
+
+
+def _dense16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, acc: bool, bias, gated=None) -> bool:
+    """out (fp32) (+)= x w^T + bias by dense16.hip; gated = (first gate row of w, first up row, features, gate bias, up bias, 16-bit out): out
+    takes the first out.shape[1] rows' products alone. False: nothing done; as for _few_rows, operands that the kernel cannot read as they
+    lie and graphs that need a gradient are the library's business."""
+    if not (x.is_cuda and x.dim() == 2 and out.dim() == 2 and x.dtype == w.dtype == torch.bfloat16):
+        return False
+    M, K = x.shape
+    N_ = out.shape[1]
+    if not (takes_gated16(M, N_, K, gated[2]) if gated else takes_dense16(M, N_, K)):
+        return False
+    if w.device != x.device or out.device != x.device or x.device.index != torch.cuda.current_device() or w.shape[1] != K \
+            or (w.shape[0] < N_ if gated else w.shape[0] != N_) \
+            or (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or out.requires_grad)):
+        return False
+    ldx, ldo = (x.stride(0), out.stride(0)) if M > 1 else (K, N_)
+    if x.stride(1) != 1 or not K <= ldx <= 1 << 22 or ldx % 8 or x.data_ptr() % 16 or not w.is_contiguous() or w.data_ptr() % 16 or K > 1 << 22 \
+            or out.dtype != torch.float32 or out.shape[0] != M or out.stride(1) != 1 or ldo < N_ or ldo % 4 or out.data_ptr() % 16:
+        return False
+    g = (0, 0, 0, None, None, None, 0)
+    if gated:
+        gate, up, Fn, gate_b, up_b, gout = gated
+        ldg = gout.stride(0) if M > 1 else Fn
+        if gout.dtype != x.dtype or gout.device != x.device or tuple(gout.shape) != (M, Fn) or gout.stride(1) != 1 or ldg < Fn or ldg % 4 \
+                or gout.data_ptr() % 8 or gate < N_ or up < gate + Fn or up + Fn > w.shape[0] or w.numel() * 2 >= 1 << 32 \
+                or any(b is not None and (b.dtype != torch.float32 or b.numel() != Fn or not b.is_contiguous() or b.data_ptr() % 16 or b.device != x.device)
+                       for b in (gate_b, up_b)):
+            return False
+    if bias is not None and (bias.dtype != torch.float32 or bias.numel() != N_ or not bias.is_contiguous() or bias.data_ptr() % 16 or bias.device != x.device):
+        return False
+    from .. import _native as N
+    mi, nj, whole, parts = dense16_plan(M, N_, K, gated[2] if gated else 0)
+    part = None
+    if parts > 1:
+        m, cols = -(-M // (32 * mi)), 32 * nj
+        t = m * (-(-N_ // cols) + (-(-2 * gated[2] // cols) if gated else 0))
+        try:
+            part = torch.empty((t - whole) * parts * 32 * mi * cols, dtype=torch.float32, device=x.device)
+        except torch.cuda.OutOfMemoryError:
+            whole, parts = t, 1  # (whole tiles need no room)
+    if gated:
+        g = (Fn, gate, up, N.ptr(gate_b), N.ptr(up_b), gout.data_ptr(), ldg)
+    N.kcall("mxk_dense16", 4 if gated else int(acc), 16 * mi + nj, x.data_ptr(), ldx, w.data_ptr(), K, M, N_, K, N.ptr(bias), out.data_ptr(), ldo,
+            whole, parts, N.ptr(part), *g, N.stream_ptr())
     return True
 
 
@@ -112,7 +239,7 @@ class Dense:
             else:
                 torch.mm(x, self.wt, out=out)
             return out
-        if self.b32 is None and _few_rows(x, self.w, out, False):
+        if _dense16(x, self.w, out, False, self.b32) or self.b32 is None and _few_rows(x, self.w, out, False):
             return out
         if _fp32_out_ok(x.dtype):
             if self.b32 is not None:
@@ -124,12 +251,19 @@ class Dense:
         out.copy_(self(x))
         return out
 
+    def gated(self, x: torch.Tensor, out: torch.Tensor, gate: int, up: int, gate_b, up_b, gout: torch.Tensor) -> bool:
+        """out (fp32 [T, n]) = x times the first n rows of W and gout (16-bit [T, F]) = silu(x W[gate:gate + F]^T + gate_b) (x W[up:up + F]^T +
+        up_b) in one launch, without the gated unit's operands in memory; False where that is not done (nothing is written)."""
+        return self.b32 is None and _dense16(x, self.w, out, False, None, (gate, up, gout.shape[1], gate_b, up_b, gout))
+
     def acc(self, x: torch.Tensor, acc: torch.Tensor) -> torch.Tensor:
         """acc (fp32) += x W^T + b — the residual add fused as GEMM beta = 1."""
         if x.dtype == torch.float32 and acc.is_contiguous():
             if self.b32 is not None:
                 acc.add_(self.b32)
             torch.addmm(acc, x, self.wt, out=acc)
+            return acc
+        if acc.is_contiguous() and _dense16(x, self.w, acc, True, self.b32):
             return acc
         if x.dtype != torch.float32 and _fp32_out_ok(x.dtype) and acc.is_contiguous():
             if self.b32 is not None:
