@@ -1,18 +1,17 @@
 // dense16_impl.h — products of a 16-bit matrix's rows with 16-bit weights: the kernel of dense16.hip (what it is for and its times stand
 // there) over g16_tile's tiles. Tiles whose K is split over workgroups leave their sums in `part`; dense16_sum_kernel adds them in order.
 #pragma once
+#include "dense16.h"
 #include "gemm16_impl.h"
 
 namespace {
-
-enum { D16_F32 = 0, D16_ADD = 1, D16_GLU = 4, D16_PART = 5 };
 
 struct D16Args {
     const uint16_t *A, *B;
     int lda, ldb, M, N, nk;  // N: columns of C; nk 64-wide k-tiles
     int n_mt, n_nt;          // tiles of C
     int full, parts;         // tiles from `full` on are summed in `parts` parts of K
-    float* part;             // [tile - full][part][TM][TN]
+    float* part;             // [tile - full][part][TM][TN], or with part_rows [part][M][N]
     const float* bias;       // of C's columns, or null
     float* C;
     int ldc;
@@ -21,6 +20,10 @@ struct D16Args {
     const float *gate_b, *up_b;
     uint16_t* G;
     int ldg;
+    // 16-bit outputs (D16_ACT, D16_GELU: gelu of the sum, erf form) instead of C, with a 16-bit bias or null
+    uint16_t* Y;
+    const uint16_t* bias16;
+    int part_rows;
 };
 
 MX_DEV float d16_silu(float x) { return x / (1.f + expf(-x)); }
@@ -56,6 +59,8 @@ __global__ __launch_bounds__(256, 1) void dense16_kernel(D16Args a) {
                 const int f = min(nt * (T::TN / 2) + (r >> 5) * 16 + (r & 15), a.F - 1);
                 return (uint32_t)((r & 16 ? a.up0 : a.gate0) + f) * (uint32_t)(2 * a.ldb);
             }
+            // 16-bit outputs: neighbouring 16-column tiles share 32 columns so that a lane ends with eight in a row
+            if (EPI == D16_ACT || EPI == D16_GELU) r = (r & ~31) + ((r & 12) << 1) + ((r >> 2) & 4) + (r & 3);
             return (uint32_t)min(r, a.N - 1 - n_base) * (uint32_t)(2 * a.ldb);
         },
         acc, ROT ? (int)(bid * 17u % (unsigned)(k1 - k0)) : 0);
@@ -86,12 +91,38 @@ __global__ __launch_bounds__(256, 1) void dense16_kernel(D16Args a) {
             return;
         }
     }
+    if constexpr (EPI == D16_ACT || EPI == D16_GELU) {
+        const int n1 = n_base + wn * (16 * NJ) + 8 * eg;  // a lane's eight columns of a pair of 16-column tiles
+        u32x4 b[NJ / 2];
+#pragma unroll
+        for (int q = 0; q < NJ / 2; ++q) b[q] = a.bias16 ? *(const u32x4*)(a.bias16 + min(n1 + 32 * q, a.N - 8)) : (u32x4){0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+#pragma unroll
+            for (int q = 0; q < NJ / 2; ++q) {
+                float v[8];
+                u32x4 w;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) unpack_act2<F16>(b[q][e], v[2 * e], v[2 * e + 1]);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    v[e] += acc[i][2 * q + (e >> 2)][e & 3];
+                    if constexpr (EPI == D16_GELU) v[e] = gelu_erf_f(v[e]);
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) w[e] = pack_act2<F16>(v[2 * e], v[2 * e + 1]);
+                if (m0 + 16 * i < a.M && n1 + 32 * q < a.N) *(u32x4*)(a.Y + (size_t)(m0 + 16 * i) * a.ldc + n1 + 32 * q) = w;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        return;
+    }
     // fp32 rows, or a part's sums
     float* C = a.C;
     int ldc = a.ldc;
     if constexpr (EPI == D16_PART) {
-        C = a.part + ((size_t)(tile - a.full) * np + p) * (T::TM * T::TN) - ((size_t)m_base * T::TN + n_base);
-        ldc = T::TN;
+        C = a.part_rows ? a.part + (size_t)p * a.M * a.N : a.part + ((size_t)(tile - a.full) * np + p) * (T::TM * T::TN) - ((size_t)m_base * T::TN + n_base);
+        ldc = a.part_rows ? a.N : T::TN;
     }
     f32x4 b[NJ], old[2][NJ];
     if constexpr (EPI != D16_PART)

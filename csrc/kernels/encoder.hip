@@ -8,6 +8,7 @@
 // Measured on BERT-base, against padded rows with fp32 copies around each LayerNorm and a library call per operation: one
 // text of 19 tokens 2019 -> 483 us (87 launches of 4-6 us), 48 texts of 23-401 tokens (6428 rows of 19248 padded) 7147 ->
 // 2278: LayerNorm + casts 74 -> 8.3 us (30 MB: 3.6 TB/s), GELU 40 -> 16 (79 MB: 4.9 TB/s).
+#include "dense16.h"
 #include "mx_common.h"
 
 #include <type_traits>
@@ -382,6 +383,20 @@ extern "C" int mxk_enc_pool(const uint16_t* x, const int* cu, const int* klen, i
     MXK_CHECK_LAUNCH();
 }
 
+// x = LN(sum of np parts + bias + x)
+int enc_parts_ln(int np, const float* parts, const uint16_t* bias, uint16_t* x, int rows, const float* g, const float* b, int H, float eps, hipStream_t st) {
+    auto go = [&](auto kern) {
+        kern<<<(rows + EW - 1) / EW, 64 * EW, 0, st>>>(parts, bias, x, rows, g, b, H, eps);
+        return (int)hipGetLastError();
+    };
+    int rc = (int)hipErrorInvalidValue;
+#define NP_(N_) \
+    if (np == N_) MX_ACT_DISPATCH(ENC_NC(H, rc = go(enc_parts_ln_kernel<NC, N_, F16>)));
+    NP_(1) NP_(2) NP_(3) NP_(4) NP_(8)
+#undef NP_
+    return rc;
+}
+
 // w: 12 device pointers a layer: qkv W, b, output W, b, norm g, b (fp32), up W, b, down W, b, norm g, b (fp32); biases may be
 // null. x [rows][H] in and out; qkv [rows][3 H], attn [rows][H], up [rows][F] and parts [4][rows][H] fp32 are scratch.
 extern "C" int mxk_enc_layers(const void* const* w, int n_layers, uint16_t* x, int rows, int B, int Smax, const int* cu,
@@ -393,13 +408,7 @@ extern "C" int mxk_enc_layers(const void* const* w, int n_layers, uint16_t* x, i
     for (int l = 0; l < n_layers; ++l, w += 12) {
         auto at = [&](int i) { return (const uint16_t*)w[i]; };
         auto ln = [&](int K, int i, int j) {  // x = LN(parts of a product over K + bias i + x) with norm j
-            auto go = [&](auto kern) {
-                kern<<<(rows + EW - 1) / EW, 64 * EW, 0, st>>>(parts, at(i), x, rows, (const float*)w[j], (const float*)w[j + 1], H, eps);
-                return (int)hipGetLastError();
-            };
-            int rc = 0;
-            MX_ACT_DISPATCH(ENC_NC(H, rc = enc_parts(K) == 1 ? go(enc_parts_ln_kernel<NC, 1, F16>) : go(enc_parts_ln_kernel<NC, 4, F16>)));
-            return rc;
+            return enc_parts_ln(enc_parts(K), parts, at(i), x, rows, (const float*)w[j], (const float*)w[j + 1], H, eps, st);
         };
         int rc = 0;
         MX_ACT_DISPATCH((rc = enc_gemm<F16, ENC_ACT>(x, at(0), at(1), qkv, rows, 3 * H, H, st)));
@@ -410,6 +419,35 @@ extern "C" int mxk_enc_layers(const void* const* w, int n_layers, uint16_t* x, i
         if (!rc) MX_ACT_DISPATCH((rc = enc_gemm<F16, ENC_GELU>(x, at(6), at(7), up, rows, F, H, st)));
         if (!rc) MX_ACT_DISPATCH((rc = enc_gemm<F16, ENC_PART>(up, at(8), nullptr, parts, rows, H, F, st)));
         if (!rc) rc = ln(F, 9, 10);
+        if (rc) return rc;
+    }
+    return 0;
+}
+
+// The same layers by dense16.hip's tiles. plan: tile of the qkv product; tile and parts of K of the output product; tile of the up product; tile and
+// parts of the down product (parts 1, 2, 3, 4 or 8; with 1 the product is stored in 16 bits with its bias, as `up`'s input is). H and F multiples
+// of 64; parts [most parts][rows][H] where there are any.
+extern "C" int mxk_enc_layers_tiled(const void* const* w, int n_layers, uint16_t* x, int rows, int B, int Smax, const int* cu, const int* klen, int H,
+                                    int heads, int F, float scale, float eps, uint16_t* qkv, uint16_t* attn, float* parts, uint16_t* up,
+                                    const int* plan, hipStream_t st) {
+    if (rows <= 0 || n_layers <= 0) return 0;
+    if (!enc_width_ok(H) || H % 64 || F <= 0 || F % 64 || heads <= 0 || H % heads) return (int)hipErrorInvalidValue;
+    for (int l = 0; l < n_layers; ++l, w += 12) {
+        auto at = [&](int i) { return (const uint16_t*)w[i]; };
+        auto add_ln = [&](const uint16_t* a, int K, int tile, int np, int i) {  // x = LN(a W^T + bias + x): weights i, bias i + 1, norm i + 2
+            const float *g = (const float*)w[i + 2], *b = (const float*)w[i + 3];
+            if (np == 1) {  // (the q|k|v rows are read by now)
+                const int rc = mx_dense16_enc(D16_ACT, tile, a, K, at(i), rows, H, K, at(i + 1), qkv, H, 1, nullptr, st);
+                return rc ? rc : enc_add_ln(qkv, x, rows, g, b, H, eps, st);
+            }
+            const int rc = mx_dense16_enc(D16_PART, tile, a, K, at(i), rows, H, K, nullptr, nullptr, 0, np, parts, st);
+            return rc ? rc : enc_parts_ln(np, parts, at(i + 1), x, rows, g, b, H, eps, st);
+        };
+        int rc = mx_dense16_enc(D16_ACT, plan[0], x, H, at(0), rows, 3 * H, H, at(1), qkv, 3 * H, 1, nullptr, st);
+        if (!rc) rc = mxk_attn_dense_ragged(qkv, 3 * H, qkv + H, 3 * H, qkv + 2 * H, 3 * H, attn, H, B, Smax, heads, H / heads, cu, klen, scale, st);
+        if (!rc) rc = add_ln(attn, H, plan[1], plan[2], 2);
+        if (!rc) rc = mx_dense16_enc(D16_GELU, plan[3], x, H, at(6), rows, F, H, at(7), up, F, 1, nullptr, st);
+        if (!rc) rc = add_ln(up, F, plan[4], plan[5], 8);
         if (rc) return rc;
     }
     return 0;

@@ -7,8 +7,8 @@ backend/python/rerankers/backend.py:72-91).
 
 MI355X path: 16-bit activations (the library's act16 format) in packed rows, no padding (encoder.hip): embeddings, LayerNorms
 with the fp32 residual sum, GELU and pooling in one pass each, attention on the fused MFMA flash kernel (attention_dense.hip);
-few rows run whole layers from one native call with their own GEMMs, many multiply on hipBLASLt with fused bias. Shapes
-encoder.hip does not take run padded, the LayerNorms on norm.hip. Weights load from GGUF (llama.cpp `bert` /
+all layers run from one native call, few rows on 16-column GEMMs (encoder.hip), more on tiles with bias and GELU in their epilogues
+(dense16_enc.hip); feed-forwards that are not whole 64s wide multiply on hipBLASLt. Shapes encoder.hip does not take run padded, the LayerNorms on norm.hip. Weights load from GGUF (llama.cpp `bert` /
 `nomic-bert` / `jina-bert-v2` tensor names, any ggml type -> dequantised to 16-bit) or are
 random-initialised for `synthetic:bert-*`.
 """
@@ -24,15 +24,21 @@ import torch.nn.functional as F
 
 from .. import _native as N
 from ..ops import core as K
+from ..ops.dense import encoder_plan
 from ..ops.linear import ACT_DTYPE
 
-# packed rows up to which encoder.hip runs the layers in one call; above, the library multiplies
-ENC_SMALL_ROWS = 448
+# packed rows up to which encoder.hip's 16-column GEMMs run the layers. Whole embed calls, us, these / tiles (dense16_enc.hip): 768 x 3072, 12 layers, 19 / 64 /
+# 65 / 128 / 448 rows 436 / 519, 515 / 551, 587 / 563, 633 / 568, 1092 / 608; 1024 x 4096, 8 layers, 64 / 65 397 / 425, 455 / 422; 1536 x 6144 33 / 48 / 65 408 / 426,
+# 457 / 449, 529 / 412. Beyond, the library's GEMMs issued from Python and a pass for GELU before / tiles: 384 x 1536 600 / 3000 rows 1360 / 508, 1393 / 732; 768 x 3072
+# 600 / 1700 / 6428 / 12000 rows 1378 / 640, 1392 / 1036, 2450 / 2191, 4233 / 3602; 1024 x 4096 1000 / 6428 927 / 617, 2288 / 2232; 2048 x 8192, 4 layers, 100 /
+# 1700 / 12000 492 / 352, 1043 / 924, 5407 / 4938 (6428 rows 2769 / 2837).
+ENC_FEW_ROWS = 64
+ENC_SMALL_ROWS = 448  # where tiles do not take the widths
 
 
 def small_rows(hidden: int, ffn: int) -> int:
-    """Packed rows up to which the layers run in one call (encoder.hip's own GEMMs read a layer's weights once per 64 rows, so
-    rows x weights decide; beyond 64 M weights a layer the library's tiles win at any row count).
+    """Packed rows up to which the layers run on encoder.hip's 16-column GEMMs rather than the library's (they read a layer's weights once
+    per 64 rows, so rows x weights decide; beyond 64 M weights a layer the library's tiles win at any row count).
 
     Whole embed calls, us, one call / library GEMMs issued from Python (110 us a layer at least): 384 x 1536, 12 layers, 448 rows
     679 / 1433; 768 x 3072, 12 layers, 64 rows 657 / 1374, 384 1161 / 1363, 512 1275 / 1356, 640 1488 / 1354; 1024 x 4096, 24
@@ -218,6 +224,14 @@ class BertModel:
         st = N.stream_ptr()
         N.kcall("mxk_enc_embed", img.data_ptr(), R, *ptrs[:5], H, float(cfg.eps), x.data_ptr(), st)
         scale = 1.0 / math.sqrt(H // cfg.n_heads)
+        if H % 64 == 0 and Fd % 64 == 0 and (R > ENC_FEW_ROWS or R > small_rows(H, Fd)):
+            plan = encoder_plan(R, H, Fd)
+            most = max(plan[2], plan[5])
+            parts = torch.empty(most, R, H, dtype=torch.float32, device=dev) if most > 1 else None
+            qkv, up = (torch.empty(R, n, dtype=self.dtype, device=dev) for n in (3 * H, Fd))
+            N.kcall("mxk_enc_layers_tiled", (ctypes.c_void_p * (12 * cfg.n_layers))(*ptrs[5:]), cfg.n_layers, x.data_ptr(), R, B, S, cu_d.data_ptr(), len_d.data_ptr(), H,
+                    cfg.n_heads, Fd, scale, float(cfg.eps), qkv.data_ptr(), attn.data_ptr(), N.ptr(parts), up.data_ptr(), (ctypes.c_int * 6)(*plan), st)
+            return x, cu_d, len_d
         if R <= small_rows(H, Fd):
             parts = torch.empty(4, R, H, dtype=torch.float32, device=dev)  # fp32 sums of up to four parts of K
             qkv, up = (torch.empty(R, n, dtype=self.dtype, device=dev) for n in (3 * H, Fd))

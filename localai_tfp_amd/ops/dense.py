@@ -117,6 +117,49 @@ def dense16_plan(M: int, N_: int, K: int, Fn: int = 0):
     return best[1]
 
 
+# the same tiles with 16-bit outputs of 12 to 64 k-tiles (encoders; weights in the last-level cache): us a k-tile and a round, us to fill and
+# store a round, share of a round that its first workgroup takes; plain, with GELU, and fp32 parts of K. Fitted to 2800 measurements (384 x 384
+# .. 4096 x 1024, 64 to 24000 rows): picks are 0.1 % slower than the best of them on average, parts 0.7 %.
+_D16_ENC_COST = (
+    {(8, 8): (1.27, 8.49, 0.73), (7, 8): (1.12, 7.74, 0.74), (6, 8): (0.967, 6.9, 0.74), (5, 8): (0.851, 5.91, 0.74), (8, 6): (0.971, 6.65, 0.73),
+     (6, 6): (0.785, 5.38, 0.73), (8, 4): (0.728, 4.65, 0.72), (5, 4): (0.476, 3.63, 0.75), (4, 4): (0.409, 3.25, 0.75), (2, 8): (0.614, 2.79, 0.67),
+     (2, 4): (0.369, 1.66, 0.69)},
+    {(8, 8): (1.11, 19.6, 0.82), (7, 8): (0.955, 17.1, 0.82), (6, 8): (0.823, 15.3, 0.81), (5, 8): (0.742, 12.9, 0.81), (8, 6): (0.825, 15.0, 0.82),
+     (6, 6): (0.642, 11.9, 0.81), (8, 4): (0.607, 10.3, 0.82), (5, 4): (0.425, 7.18, 0.8), (4, 4): (0.36, 6.04, 0.83), (2, 8): (0.599, 5.53, 0.76),
+     (2, 4): (0.281, 3.76, 0.83)},
+    {(8, 8): (1.41, 13.7, 0.64), (7, 8): (1.23, 12.4, 0.67), (6, 8): (1.03, 11.0, 0.7), (5, 8): (0.899, 9.64, 0.69), (8, 6): (1.1, 11.0, 0.63),
+     (6, 6): (0.839, 8.76, 0.66), (8, 4): (0.877, 8.06, 0.57), (5, 4): (0.571, 6.02, 0.62), (4, 4): (0.529, 5.21, 0.58), (2, 8): (0.573, 5.21, 0.67),
+     (2, 4): (0.322, 3.38, 0.69)})
+
+
+def _enc_tile(M: int, N_: int, K: int, kind: int, parts: int = 1):
+    """(estimated us, 16 * row units + column units) of the best tile."""
+    best = None
+    for (mi, nj), (a, fill, first) in _D16_ENC_COST[kind].items():
+        full, rem = divmod(-(-M // (32 * mi)) * -(-N_ // (32 * nj)) * parts, CU_COUNT)
+        us = (full + (first + (1 - first) * rem / CU_COUNT if rem else 0.0)) * (-(-K // 64 // parts) * a + fill)
+        if best is None or us < best[0]:
+            best = us, 16 * mi + nj
+    return best
+
+
+@functools.lru_cache(maxsize=1024)
+def encoder_plan(M: int, H: int, Fn: int) -> tuple:
+    """Tiles (and parts of K) of an encoder layer's q|k|v, output, up and down products for M rows, as encoder.hip takes them. Parts that the
+    LayerNorm adds up cost it 4 bytes a number each, the 16-bit sums of an undivided product 2."""
+    def narrow(K):
+        best = None
+        for parts in (1, 2, 3, 4, 8):
+            if parts > K // 64 or parts > 1 and M * H * parts > 1 << 25:
+                break
+            us, tile = _enc_tile(M, H, K, 2 if parts > 1 else 0, parts)
+            us += M * H * (4 * parts if parts > 1 else 2) / 4e6
+            if best is None or us < best[0]:
+                best = us, (tile, parts)
+        return best[1]
+    return (_enc_tile(M, 3 * H, H, 0)[1], *narrow(H), _enc_tile(M, Fn, H, 1)[1], *narrow(Fn))
+
+
 def takes_dense16(M: int, N_: int, K: int) -> bool:
     """Whether x w^T (bf16, fp32 out) runs dense16.hip. Measured beside the library's products in a graph, weights in no cache, us
     (library / here): long K, whose columns leave compute units idle or to products the library splits badly, 4096 x 20480 at 4 / 64 / 240 /

@@ -215,3 +215,55 @@ def test_empty_texts_match_the_padded_batch(pooling):
     ids = [[5, 6, 7, 8, 9], [], [11, 12], []]
     assert g._packed_weights(ids) is not None
     assert (g.embed(ids).cpu() - c.embed(ids)).abs().max() < 5e-3  # (the bound of test_packed_rows_match_fp32)
+
+
+def test_encoder_plans_are_within_what_the_kernels_take():
+    from localai_tfp_amd.ops import dense as D
+    tiles = {16 * a + b for a, b in D._D16_ENC_COST[0]}
+    for rows in (1, 65, 449, 1000, 6428, 100000):
+        for H, F in ((64, 64), (128, 512), (768, 3072), (1024, 2816), (4096, 16384)):
+            q, o, po, u, d, pd = D.encoder_plan(rows, H, F)
+            assert {q, o, u, d} <= tiles and po in (1, 2, 3, 4, 8) and pd in (1, 2, 3, 4, 8) and po <= H // 64 and pd <= F // 64
+            assert max(po, pd) == 1 or rows * H * max(po, pd) <= 1 << 25
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", [136, 120, 104, 88, 134, 102, 132, 84, 68, 40, 36])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_tiled_layers_match_fp32(tile, dtype, monkeypatch):
+    """Every tile in every product of a layer, undivided and in each number of parts, one row, part-empty tiles and some of each: the bound
+    of test_packed_rows_match_fp32 (bf16: eight times, its rounding)."""
+    cfg = BM.BertConfig(vocab=400, hidden=192, n_layers=2, n_heads=3, ffn=576, max_pos=300, name="t")
+    get = BM.synthetic_bert(cfg, 5)
+    monkeypatch.setattr(BM, "ACT_DTYPE", dtype)
+    g, c = BM.BertModel.load(cfg, get, "cuda:0"), BM.BertModel.load(cfg, get, "cpu")
+    monkeypatch.setattr(BM, "ENC_FEW_ROWS", 0)
+    used = []
+    real = BM.N.kcall
+    monkeypatch.setattr(BM.N, "kcall", lambda name, *a: (used.append(name), real(name, *a))[1])
+    for lens, po, pd in (([1], 1, 1), ([33, 200, 24], 3, 8), ([258, 3], 2, 4), ([63], 1, 3)):
+        monkeypatch.setattr(BM, "encoder_plan", lambda R, H, F: (tile, tile, po, tile, tile, pd))
+        ids = [list(range(10, 10 + n)) for n in lens]
+        got, want = g.embed(ids).cpu(), c.embed(ids)
+        assert "mxk_enc_layers_tiled" in used and (got - want).abs().max() < (5e-3 if dtype == torch.float16 else 4e-2), (lens, po, pd)
+
+
+@pytest.mark.gpu
+def test_gelu_rounds_like_64_bits():
+    """Every finite f16: within a unit of the last place, and the nearest f16 for all but one in a thousand (fp32 arithmetic near the
+    middle of two). Infinities and NaN as 0.5 x (1 + erf(x / sqrt 2)) has them."""
+    from localai_tfp_amd import _native as N
+    N.ensure_act(torch.float16)
+    x = torch.arange(1 << 16, dtype=torch.int32).to(torch.int16).view(torch.float16)
+    y = x.cuda()
+    N.kcall("mxk_enc_gelu", y.data_ptr(), y.numel(), N.stream_ptr())
+    y, d = y.cpu(), x.double()
+    want = 0.5 * d * torch.special.erfc(-d * 2 ** -0.5)
+    ok = torch.isfinite(x)
+    near = want.to(torch.float16)
+    # (neighbours in order: sign and magnitude bits as one whole number)
+    step = (y.view(torch.int16).int() & 0x7FFF) - (near.view(torch.int16).int() & 0x7FFF)
+    assert (step[ok].abs() <= 1).all() and (step[ok] != 0).float().mean() < 1e-3
+    assert (y[ok & (want.abs() > 1e-7)].sign() == near[ok & (want.abs() > 1e-7)].sign()).all()
+    inf = float("inf")
+    assert y[x == inf].item() == inf and torch.isnan(y[x == -inf]).all() and torch.isnan(y[torch.isnan(x)]).all()
