@@ -66,8 +66,8 @@ extern "C" int mxk_dense16(int epi, int tile, const uint16_t* A, int lda, const 
     if ((epi != D16_F32 && epi != D16_ADD && epi != D16_GLU) || K <= 0 || K % G16_K || N % 4 || (lda & 7) || (ldb & 7) || lda < K || ldb < K ||
         lda > (1 << 22) || ldb > (1 << 22) || (ldc & 3) || ldc < N || (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C | (uintptr_t)bias | (uintptr_t)part) & 15))
         return (int)hipErrorInvalidValue;  // (256 rows of 2^23 bytes: the 32-bit lane offsets)
-    if (epi == D16_GLU && (F <= 0 || F % 4 || gate0 < N || up0 < gate0 + F || ((long)up0 + F) * ldb * 2 > 0xffffffffl || !G || (ldg & 3) || ldg < F ||
-                           ((uintptr_t)G & 7) || (((uintptr_t)gate_b | (uintptr_t)up_b) & 15) || bias))
+    if (epi == D16_GLU && (F <= 0 || F % 8 || gate0 < N || up0 < gate0 + F || ((long)up0 + F) * ldb * 2 > 0xffffffffl || !G || (ldg & 7) || ldg < F ||
+                           ((uintptr_t)G & 15) || (((uintptr_t)gate_b | (uintptr_t)up_b) & 15) || bias))
         return (int)hipErrorInvalidValue;
     int TM = 0, TN = 0;
 #define GO(M_, N_) \

@@ -54,10 +54,11 @@ __global__ __launch_bounds__(256, 1) void dense16_kernel(D16Args a) {
     g16_tile<F16, MI, NJ, ROT>(
         smem, ab, bb, k1 - k0, [&](int r) { return (uint32_t)min(r, a.M - 1 - m_base) * (uint32_t)(2 * a.lda); },
         [&](int r) {
-            // gated: rows in 16-row groups, an even one gates and the next one the ups of the same features
+            // gated: rows in 16-row groups, an even one gates and the next one the ups of the same features; two such pairs share 32 features
+            // so that a lane ends with eight in a row
             if (EPI == D16_GLU && glu) {
-                const int f = min(nt * (T::TN / 2) + (r >> 5) * 16 + (r & 15), a.F - 1);
-                return (uint32_t)((r & 16 ? a.up0 : a.gate0) + f) * (uint32_t)(2 * a.ldb);
+                const int f = NJ % 4 ? (r >> 5) * 16 + (r & 15) : (r >> 6) * 32 + ((r & 12) << 1) + ((r >> 3) & 4) + (r & 3);
+                return (uint32_t)((r & 16 ? a.up0 : a.gate0) + min(nt * (T::TN / 2) + f, a.F - 1)) * (uint32_t)(2 * a.ldb);
             }
             // 16-bit outputs: neighbouring 16-column tiles share 32 columns so that a lane ends with eight in a row
             if (EPI == D16_ACT || EPI == D16_GELU) r = (r & ~31) + ((r & 12) << 1) + ((r >> 2) & 4) + (r & 3);
@@ -70,21 +71,37 @@ __global__ __launch_bounds__(256, 1) void dense16_kernel(D16Args a) {
     asm volatile("" : "+v"(el));  // (no address of it computed ahead of the loop, whose registers are all taken)
     const int eg = el >> 4, wm = wave >> 1, wn = wave & 1;
     const int m0 = m_base + wm * (16 * MI) + (el & 15), n0 = n_base + wn * (16 * NJ) + 4 * eg;
-    if constexpr (EPI == D16_GLU && NJ % 2 == 0) {
+    if constexpr (EPI == D16_GLU) {
         if (glu) {
-            const int f0 = nt * (T::TN / 2) + wn * (8 * NJ) + 4 * eg;
+            constexpr int FL = NJ % 4 ? 4 : 8, NQ = NJ * 2 / FL;  // features of a lane's piece, pieces
+            static_assert(NJ % 2 == 0, "gates and ups in pairs of tiles");
+            const int f0 = nt * (T::TN / 2) + wn * (8 * NJ) + FL * eg;
 #pragma unroll
-            for (int j = 0; j < NJ / 2; ++j) {
-                const int f = f0 + 16 * j, fc = min(f, a.F - 4);
-                const f32x4 gb = a.gate_b ? *(const f32x4*)(a.gate_b + fc) : (f32x4){0.f, 0.f, 0.f, 0.f};
-                const f32x4 ub = a.up_b ? *(const f32x4*)(a.up_b + fc) : (f32x4){0.f, 0.f, 0.f, 0.f};
+            for (int q = 0; q < NQ; ++q) {
+                const int f = f0 + 4 * FL * q;
+                float gb[FL], ub[FL];
+#pragma unroll
+                for (int e = 0; e < FL; e += 4) {
+                    const int fc = min(f + e, a.F - 4);
+                    *(f32x4*)(gb + e) = a.gate_b ? *(const f32x4*)(a.gate_b + fc) : (f32x4){0.f, 0.f, 0.f, 0.f};
+                    *(f32x4*)(ub + e) = a.up_b ? *(const f32x4*)(a.up_b + fc) : (f32x4){0.f, 0.f, 0.f, 0.f};
+                }
 #pragma unroll
                 for (int i = 0; i < MI; ++i) {
-                    float v[4];
+                    uint32_t w[FL / 2];
+                    float v[FL];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) v[r] = d16_silu(acc[i][2 * j][r] + gb[r]) * (acc[i][2 * j + 1][r] + ub[r]);
-                    if (m0 + 16 * i < a.M && f < a.F)
-                        *(u32x2*)(a.G + (size_t)(m0 + 16 * i) * a.ldg + f) = (u32x2){pack_act2<F16>(v[0], v[1]), pack_act2<F16>(v[2], v[3])};
+                    for (int e = 0; e < FL; ++e) {
+                        const int j = q * (FL / 2) + (e >> 2) * 2;
+                        v[e] = d16_silu(acc[i][j][e & 3] + gb[e]) * (acc[i][j + 1][e & 3] + ub[e]);
+                    }
+#pragma unroll
+                    for (int e = 0; e < FL; e += 2) w[e / 2] = pack_act2<F16>(v[e], v[e + 1]);
+                    uint16_t* g = a.G + (size_t)(m0 + 16 * i) * a.ldg + f;
+                    if (m0 + 16 * i < a.M && f < a.F) {
+                        if constexpr (FL == 8) *(u32x4*)g = (u32x4){w[0], w[1], w[2], w[3]};
+                        else *(u32x2*)g = (u32x2){w[0], w[1]};
+                    }
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }

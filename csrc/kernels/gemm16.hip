@@ -37,35 +37,60 @@ __global__ __launch_bounds__(256, 1) void gemm16_kernel(const uint16_t* __restri
     g16_tile<true, 8, 8>(
         smem, (const char*)(A + (size_t)m_base * lda), (const char*)(B + (size_t)n_base * ldb), K / G16_K,
         [&](int r) { return (uint32_t)min(r, M - 1 - m_base) * (uint32_t)(2 * lda); },
-        [&](int r) { return (uint32_t)min(r, N - 1 - n_base) * (uint32_t)(2 * ldb); }, acc);
+        [&](int r) {
+            // 16-bit outputs: neighbouring 16-column tiles (gated: pairs of a gate's and an up's) share 32 columns, so that a lane ends
+            // with eight in a row; B's rows lie interleaved in 16-row groups, a gate's and the up's of the same features
+            if constexpr (EPI == E16_ACT) r = (r & ~31) + ((r & 12) << 1) + ((r >> 2) & 4) + (r & 3);
+            if constexpr (EPI == E16_SWIGLU || EPI == E16_GEGLU) {
+                const int f = ((r & 12) << 1) + ((r >> 3) & 4) + (r & 3);
+                r = (r & ~63) + ((f & 16) << 1) + (r & 16) + (f & 15);
+            }
+            return (uint32_t)min(r, N - 1 - n_base) * (uint32_t)(2 * ldb);
+        },
+        acc);
 
     // ---- epilogue: lane holds columns nb + 4 g .. + 3 of row mb + col; the residual's rows a block ahead of their stores ----
     int el = lane;
     asm volatile("" : "+v"(el));  // (no address of it computed ahead of the loop, whose registers are all taken)
     const int eg = el >> 4, m0 = m_base + wm * 128 + (el & 15), n0 = n_base + wn * 128 + 4 * eg;
+    auto put = [&](uint16_t* p, const uint32_t (&w)[4]) {
+        if (ldc & 7) {  // (rows 8 bytes apart from 16)
+            *(u32x2*)p = (u32x2){w[0], w[1]};
+            *(u32x2*)(p + 4) = (u32x2){w[2], w[3]};
+        } else {
+            *(u32x4*)p = (u32x4){w[0], w[1], w[2], w[3]};
+        }
+    };
     if constexpr (EPI == E16_SWIGLU || EPI == E16_GEGLU) {
-        // B rows interleaved in 16-row groups: an even column tile is the gate, the next one the up of the same features
+        const int f0 = (n_base >> 1) + wn * 64 + 8 * eg;
 #pragma unroll
         for (int i = 0; i < 8; ++i)
             if (m0 + 16 * i < M)
 #pragma unroll
-                for (int j = 0; j < 8; j += 2) {
-                    if (n0 + 16 * j >= N) break;
-                    uint32_t w[4];  // (each rounded once, product and conversion together, as in qmm2; a packed conversion rounds the product first)
+                for (int q = 0; q < 2; ++q) {
+                    if (f0 + 32 * q >= N >> 1) break;
+                    uint32_t v[8], w[4];  // (each rounded once, product and conversion together, as in qmm2; a packed conversion rounds the product first)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) w[r] = f32_to_act<true>(glu_gate_f<EPI>(acc[i][j][r]) * acc[i][j + 1][r]);
-                    *(u32x2*)((uint16_t*)Cv + (size_t)(m0 + 16 * i) * ldc + ((n0 + 16 * j - 4 * eg) >> 1) + 4 * eg) =
-                        (u32x2){w[0] | w[1] << 16, w[2] | w[3] << 16};
+                    for (int e = 0; e < 8; ++e) {
+                        const int j = 4 * q + (e >> 2) * 2;
+                        v[e] = f32_to_act<true>(glu_gate_f<EPI>(acc[i][j][e & 3]) * acc[i][j + 1][e & 3]);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) w[e] = v[2 * e] | v[2 * e + 1] << 16;
+                    put((uint16_t*)Cv + (size_t)(m0 + 16 * i) * ldc + f0 + 32 * q, w);
                 }
     } else if constexpr (EPI == E16_ACT) {
+        const int n1 = n_base + wn * 128 + 8 * eg;
 #pragma unroll
         for (int i = 0; i < 8; ++i)
             if (m0 + 16 * i < M)
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    if (n0 + 16 * j >= N) break;
-                    *(u32x2*)((uint16_t*)Cv + (size_t)(m0 + 16 * i) * ldc + n0 + 16 * j) =
-                        (u32x2){pack_act2<true>(acc[i][j][0], acc[i][j][1]), pack_act2<true>(acc[i][j][2], acc[i][j][3])};
+                for (int q = 0; q < 4; ++q) {
+                    if (n1 + 32 * q >= N) break;
+                    uint32_t w[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) w[e] = pack_act2<true>(acc[i][2 * q + (e >> 1)][2 * (e & 1)], acc[i][2 * q + (e >> 1)][2 * (e & 1) + 1]);
+                    put((uint16_t*)Cv + (size_t)(m0 + 16 * i) * ldc + n1 + 32 * q, w);
                 }
     } else {
         f32x4 old[2][8];

@@ -183,7 +183,7 @@ def takes_gated16(M: int, N_: int, K: int, Fn: int) -> bool:
     and the gating kernel / here: 12320 + 2 x 14336 columns x 4096 at 1 / 33 / 112 / 322 / 703 / 2062 rows 76 / 64, 78 / 67, 92 / 88, 214 / 143, 334 / 227,
     733 / 641, 6176 + 2 x 8192 x 2048 at 5 / 33 / 310 / 1693 / 3557 38 / 22, 29 / 23, 50 / 47, 197 / 158, 407 / 307 (184 rows 41 / 42), 9000 + 2 x 20000 x
     6144 134 / 111, 145 / 110, 194 / 165 (239 rows); 3000 + 2 x 5632 x 2048 even up to 64 rows (20 / 20 and 20.6 / 21.5), 465 rows 52 / 40."""
-    return M > 0 and K % 64 == 0 and K >= 512 and N_ > 0 and N_ % 4 == 0 and Fn % 4 == 0 and Fn > 0 and (N_ + 2 * Fn) * K >= (1 << 22 if M > 64 else 1 << 25)
+    return M > 0 and K % 64 == 0 and K >= 512 and N_ > 0 and N_ % 4 == 0 and Fn % 8 == 0 and Fn > 0 and (N_ + 2 * Fn) * K >= (1 << 22 if M > 64 else 1 << 25)
 
 
 def _dense16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, acc: bool, bias, gated=None) -> bool:
@@ -208,8 +208,8 @@ def _dense16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, acc: bool, bia
     if gated:
         gate, up, Fn, gate_b, up_b, gout = gated
         ldg = gout.stride(0) if M > 1 else Fn
-        if gout.dtype != x.dtype or gout.device != x.device or tuple(gout.shape) != (M, Fn) or gout.stride(1) != 1 or ldg < Fn or ldg % 4 \
-                or gout.data_ptr() % 8 or gate < N_ or up < gate + Fn or up + Fn > w.shape[0] or w.numel() * 2 >= 1 << 32 \
+        if gout.dtype != x.dtype or gout.device != x.device or tuple(gout.shape) != (M, Fn) or gout.stride(1) != 1 or ldg < Fn or ldg % 8 \
+                or gout.data_ptr() % 16 or gate < N_ or up < gate + Fn or up + Fn > w.shape[0] or w.numel() * 2 >= 1 << 32 \
                 or any(b is not None and (b.dtype != torch.float32 or b.numel() != Fn or not b.is_contiguous() or b.data_ptr() % 16 or b.device != x.device)
                        for b in (gate_b, up_b)):
             return False

@@ -72,19 +72,19 @@ def test_gated_columns_match_64_bits(tile):
     rounding (2^-20) and bf16's (2^-8 of the result)."""
     tm, tn = 32 * tile[0], 32 * tile[1]
     gen = torch.Generator().manual_seed(tm * tn)
-    for M, n, F, K, whole, parts in ((tm + 1, 36, tn // 2 + 4, 576, 0, 1), (tm - 1, tn + 4, 12, 320, 1, 2), (3, 4, tn, 64, 0, 1)):
+    for M, n, F, K, whole, parts in ((tm + 1, 36, tn // 2 + 8, 576, 0, 1), (tm - 1, tn + 4, 24, 320, 1, 2), (3, 4, tn, 64, 0, 1)):
         x, w = torch.randn(M, K, generator=gen).bfloat16().cuda(), (torch.randn(n + 8 + 2 * F + 4, K, generator=gen) * K ** -0.5).bfloat16().cuda()
-        gb, y, G = torch.randn(F, generator=gen).cuda(), torch.zeros(M, n, device="cuda"), torch.zeros(M, F + 8, device="cuda").bfloat16()
+        gb, y, G = torch.randn(F, generator=gen).cuda(), torch.zeros(M, n, device="cuda"), torch.zeros(M, F + 16, device="cuda").bfloat16()
         gate, up = n + 8, n + 8 + F + 4
-        _run(4, tile, x, w, y, whole and -(-2 * F // tn) + whole, parts, None, (F, gate, up, gb, None, G[:, 4:F + 4]))
+        _run(4, tile, x, w, y, whole and -(-2 * F // tn) + whole, parts, None, (F, gate, up, gb, None, G[:, 8:F + 8]))
         xd, wd, d = x.double(), w.double(), (K + 1) * 2 ** -24
         assert ((y.double() - xd @ wd[:n].t()).abs() <= d * (xd.abs() @ wd[:n].abs().t())).all()
         g, u = xd @ wd[gate:gate + F].t() + gb.double(), xd @ wd[up:up + F].t()
         dg, du = d * (xd.abs() @ wd[gate:gate + F].abs().t() + gb.abs()), d * (xd.abs() @ wd[up:up + F].abs().t())
         want = torch.nn.functional.silu(g) * u
         tol = 1.1 * dg * u.abs() + du * g.abs() + dg * du + (2 ** -8 + 2 ** -20) * want.abs() + 1e-30
-        assert ((G[:, 4:F + 4].double() - want).abs() <= tol).all(), (tile, M, n, F, K)
-        assert not G[:, :4].any() and not G[:, F + 4:].any()
+        assert ((G[:, 8:F + 8].double() - want).abs() <= tol).all(), (tile, M, n, F, K)
+        assert not G[:, :8].any() and not G[:, F + 8:].any()
 
 
 @pytest.mark.gpu
