@@ -13,9 +13,12 @@
 // 128: 128 blocks; a step is 32 vector operations a lane and a chain of two sums): the read S^T k uses the undecayed state
 // (its decay is multiplied in after the sum), a step's LDS reads are asked for a step ahead, and output sums over a column's
 // lanes are made for 8 or 16 steps together, transposed on the way (3 operations a step instead of a chain of 4 and a store).
-// Prompts of 301 / 578 / 1111 rows: delta rule 576 -> 250 us, 64 heads of 64 x 128 without it 554 -> 227 (0.2 us a step;
-// most of the gain is that a round's loads no longer wait for each other). Decode rows and short chunks (ONE) stage one token and
-// sum at once: 33 rows 18.0 -> 12.6 and 30.3 -> 22.2 us (6.2 TB/s of states read and written).
+// Prompts of 301 / 578 / 1111 rows: delta rule 576 -> 250 us, 64 heads of 64 x 128 without it 554 -> 227 (most of the gain is that a
+// round's loads no longer wait for each other); with whole rounds free of tests between their steps and the staged numbers' scales and
+// masks worked out once (a step 36 instructions for some 65, the delta rule's 58 for 90) 262 -> 217 and 247 -> 201, one of 2900 rows
+// 644 -> 512 and 533 -> 390. Steps read two or more ahead change nothing: one wave a SIMD issues a vector instruction every 9 cycles.
+// Decode rows and short chunks (ONE) stage one token and sum at once: 33 rows 18.0 -> 12.6 and 30.3 -> 22.2 us (6.2 TB/s of states read
+// and written).
 // CHD (gated linear attention): the decay is one number per head and state row, a_t[n], staged beside k_t and q_t:
 // S[n][p] <- a_t[n] S[n][p] + k_t[n] u[p]; with DELTA as well, the delta rule's read follows that per-row decay. A
 // missing write strength means 1, one given as pre-activations (coef_sigmoid, row stride ldc) passes a sigmoid when
@@ -24,6 +27,8 @@
 // nout: the state has one more column per head (P + 1 of them) whose value is 1 at every token, so it holds
 // n <- a_t n + c_t k_t; its product n^T q_t goes to nout [rows, H] (the normaliser of a matrix memory).
 #include "../mx_common.h"
+
+#include <type_traits>
 
 namespace {
 
@@ -93,14 +98,14 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk
     auto at = [&](int j) { return (j >> 2) * (4 * LPC) + part * 4 + (j & 3); };  // which number of the column S[j] is
     float S[NPL];
     if (whole) {
-        const float4* s4 = (const float4*)sp + part;
+        const f32x4* s4 = (const f32x4*)sp + part;
 #pragma unroll
         for (int j = 0; j < NPL / 4; ++j) {
-            const float4 x = s4[j * LPC];
-            S[4 * j] = x.x;
-            S[4 * j + 1] = x.y;
-            S[4 * j + 2] = x.z;
-            S[4 * j + 3] = x.w;
+            const f32x4 x = s4[j * LPC];  // (as a vector: as four numbers the compiler joins them with the other branch's single loads)
+            S[4 * j] = x[0];
+            S[4 * j + 1] = x[1];
+            S[4 * j + 2] = x[2];
+            S[4 * j + 3] = x[3];
         }
     } else {
 #pragma unroll
@@ -150,16 +155,30 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk
             st_ac = *src;
         }
     };
+    // which vector and number of it, and which column, a thread stages: the same in every group where groups are whole tokens
+    constexpr int KC = NT % (NW * NP) ? KQ_PT : 1, VC = NT % COLS ? V_PT : 1;
+    float st_mul[KC];
+    bool st_on[KC];
+    int st_col[VC];
+#pragma unroll
+    for (int i = 0; i < KC; ++i) {
+        const int idx = threadIdx.x + i * NT;
+        st_mul[i] = (idx / NP) % NW == 1 ? q_scale : 1.f;
+        st_on[i] = idx % NP < N;
+    }
+#pragma unroll
+    for (int i = 0; i < VC; ++i) st_col[i] = blockIdx.x * COLS + (threadIdx.x + i * NT) % COLS;
     auto publish = [&](int b) {
 #pragma unroll
         for (int i = 0; i < KQ_PT; ++i) {
             const int idx = threadIdx.x + i * NT;
             if (ONE && idx >= TB * NW * NP) continue;
-            (&kq[b][0][0][0])[idx] = idx % NP < N ? ((idx / NP) % NW == 1 ? st_kq[i] * q_scale : st_kq[i]) : 0.f;
+            if constexpr (ONE) (&kq[b][0][0][0])[idx] = idx % NP < N ? ((idx / NP) % NW == 1 ? st_kq[i] * q_scale : st_kq[i]) : 0.f;
+            else (&kq[b][0][0][0])[idx] = st_on[i % KC] ? st_kq[i] * st_mul[i % KC] : 0.f;
         }
 #pragma unroll
         for (int i = 0; i < V_PT; ++i)
-            if (threadIdx.x + i * NT < TB * COLS) (&vs[b][0][0])[threadIdx.x + i * NT] = st_v[i];
+            if (threadIdx.x + i * NT < TB * COLS) (&vs[b][0][0])[threadIdx.x + i * NT] = ONE || st_col[i % VC] < P ? st_v[i] : st_col[i % VC] < PT ? 1.f : 0.f;
         if (threadIdx.x < 2 * TB) {
             float x = st_ac;
             if (threadIdx.x & 1) x = !coef ? 1.f : coef_sigmoid ? 1.f / (1.f + expf(-x)) : x;
@@ -198,40 +217,47 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk
                 if constexpr (CHD) *(float4*)(x.d + j) = *(const float4*)&kq[b][tt][NW - 1][j * LPC + part * 4];
             }
         };
-        read(0, tok[0]);
+        // whole rounds without a test between steps: those cost nine register moves a step beside the branch
+        auto steps = [&](auto whole_c) {
+            constexpr bool ALL = decltype(whole_c)::value;
+            read(0, tok[0]);
 #pragma unroll
-        for (int tt = 0; tt < TB; ++tt) {
-            os[tt] = 0.f;
-            if (tt + 1 < TB && tt + 1 < nt) read(tt + 1, tok[(tt + 1) & 1]);
-            __builtin_amdgcn_sched_barrier(0);
-            if (tt >= nt) continue;
-            const Tok& x = tok[tt & 1];
-            const float a = x.a, cf = x.cf, vv = col < P ? x.v : live ? 1.f : 0.f;
-            const float *kb = x.k, *qb = x.q, *ab = x.d;
-            float u;
-            if constexpr (DELTA) {
-                if constexpr (CHD) {
+            for (int tt = 0; tt < TB; ++tt) {
+                os[tt] = 0.f;
+                if (tt + 1 < TB && (ALL || tt + 1 < nt)) read(tt + 1, tok[(tt + 1) & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+                if (!ALL && tt >= nt) continue;
+                const Tok& x = tok[tt & 1];
+                const float a = x.a, cf = x.cf, vv = !ONE || col < P ? x.v : live ? 1.f : 0.f;
+                const float *kb = x.k, *qb = x.q, *ab = x.d;
+                float u;
+                if constexpr (DELTA) {
+                    if constexpr (CHD) {
 #pragma unroll
-                    for (int j = 0; j < NPL; ++j) S[j] *= ab[j];
+                        for (int j = 0; j < NPL; ++j) S[j] *= ab[j];
+                    }
+                    float d[4] = {0.f, 0.f, 0.f, 0.f};  // four chains of dependent adds
+#pragma unroll
+                    for (int j = 0; j < NPL; ++j) d[j & 3] += S[j] * kb[j];
+                    const float dk = lanes_sum<LPC>((d[0] + d[1]) + (d[2] + d[3]));
+                    u = cf * (CHD ? vv - dk : vv - a * dk);  // (one decay for all rows: taken out of the sum)
+                } else {
+                    u = cf * vv;
                 }
-                float d[4] = {0.f, 0.f, 0.f, 0.f};  // four chains of dependent adds
+                float o[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int j = 0; j < NPL; ++j) d[j & 3] += S[j] * kb[j];
-                const float dk = lanes_sum<LPC>((d[0] + d[1]) + (d[2] + d[3]));
-                u = cf * (CHD ? vv - dk : vv - a * dk);  // (one decay for all rows: taken out of the sum)
-            } else {
-                u = cf * vv;
+                for (int j = 0; j < NPL; ++j) {
+                    if constexpr (!(DELTA && CHD)) S[j] *= CHD ? ab[CHD ? j : 0] : a;
+                    S[j] += kb[j] * u;
+                    o[j & 3] += S[j] * qb[j];
+                }
+                os[tt] = (o[0] + o[1]) + (o[2] + o[3]);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            float o[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int j = 0; j < NPL; ++j) {
-                if constexpr (!(DELTA && CHD)) S[j] *= CHD ? ab[CHD ? j : 0] : a;
-                S[j] += kb[j] * u;
-                o[j & 3] += S[j] * qb[j];
-            }
-            os[tt] = (o[0] + o[1]) + (o[2] + o[3]);
-            __builtin_amdgcn_sched_barrier(0);
-        }
+        };
+        if constexpr (ONE) steps(std::true_type{});
+        else if (nt == TB) steps(std::true_type{});
+        else steps(std::false_type{});
         auto put = [&](int tt, float o) {
             if (tt >= nt || !live) return;
             const long row = row0 + c * TB + tt;
