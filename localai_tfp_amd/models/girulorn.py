@@ -283,7 +283,7 @@ class GirulornWorkspace:
         self.hs = torch.empty((S, C), **m16)
         self.logits = torch.empty((S, cfg.vocab), **f32)
         att = [L.mixer for L in cfg.layers if L.type == "attention"]
-        rows = HY.DECODE_WAVES + max_seqs * max([a.heads for a in att] or [1])
+        rows = max([HY.partition_rows(max_seqs, a.heads, a.heads // a.kv_heads) for a in att] or [1])
         self.part_ml = torch.empty((rows, 2), **f32)
         self.part_o = torch.empty((rows, max([a.vdim for a in att] or [1])), **f32)
 

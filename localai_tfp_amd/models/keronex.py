@@ -365,7 +365,7 @@ class KeronexWorkspace:
         self.hs = torch.empty((R, C), **m16)
         self.logits = torch.empty((R, cfg.vocab), **f32)
         att = [L.mixer for L in cfg.layers if L.type == "attention"]
-        rows = HY.DECODE_WAVES + max_seqs * max([2 * a.heads for a in att] or [1])
+        rows = max([HY.partition_rows(max_seqs, 2 * a.heads, a.heads // a.kv_heads) for a in att] or [1])
         self.part_ml = torch.empty((rows, 2), **f32)
         self.part_o = torch.empty((rows, max([a.vdim for a in att] or [1])), **f32)
 

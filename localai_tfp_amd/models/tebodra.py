@@ -311,7 +311,7 @@ class TebodraWorkspace:
         self.cat = torch.zeros((T * k_cat,), **m16)  # zero: padded columns are read, never written
         self.hs = torch.empty((R, C), **m16)
         self.logits = torch.empty((R, cfg.vocab), **f32)
-        rows = HY.DECODE_WAVES + max_seqs * max([a.heads for a in att] or [1])
+        rows = max([HY.partition_rows(max_seqs, a.heads, a.heads // a.kv_heads) for a in att] or [1])
         self.part_ml = torch.empty((rows, 2), **f32)
         self.part_o = torch.empty((rows, max([a.vdim for a in att] or [1])), **f32)
 

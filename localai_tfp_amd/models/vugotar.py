@@ -330,9 +330,9 @@ class VugotarWorkspace:
         self.hs = torch.empty((S, C), **m16)
         self.logits = torch.empty((S, cfg.vocab), **f32)
         # partial results of decode rows whose visible keys are split into partitions
-        h_att = max([L.mixer.left.heads for L in cfg.layers if L.type == "parallel"] or [1])
-        v_att = max([L.mixer.left.vdim for L in cfg.layers if L.type == "parallel"] or [1])
-        rows = HY.DECODE_WAVES + max_seqs * h_att  # few sequences take many partitions each, many take few
+        att = [L.mixer.left for L in cfg.layers if L.type == "parallel"]
+        v_att = max([a.vdim for a in att] or [1])
+        rows = max([HY.partition_rows(max_seqs, a.heads, a.heads // a.kv_heads) for a in att] or [1])
         self.part_ml = torch.empty((rows, 2), **f32)
         self.part_o = torch.empty((rows, v_att), **f32)
 

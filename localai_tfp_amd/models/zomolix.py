@@ -345,7 +345,7 @@ class ZomolixWorkspace:
         # partial results of decode rows whose visible keys are split into partitions (one layer at a time)
         rows = 1
         if att:
-            rows = HY.DECODE_WAVES + max_seqs * max(a.heads for a in att)
+            rows = max(HY.partition_rows(max_seqs, a.heads, a.heads // a.kv_heads) for a in att)
         if lat:
             rows = max(rows, max(m.heads for m in lat) * max(max_seqs * max_parts, 256))
         self.part_ml = torch.empty((rows, 2), **f32)

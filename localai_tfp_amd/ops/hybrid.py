@@ -476,12 +476,26 @@ GEMM_MAX_SCORES = 1 << 26  # fp32 scores of one sub-problem of that route
 DECODE_WAVES = 4096  # decode rows: waves to aim for when splitting contexts into key partitions
 
 
-def decode_part_len(n_dec: int, heads: int, visible: int) -> int:
+def decode_part_len(n_dec: int, heads: int, visible: int, waves: int | None = None) -> int:
     """Keys per partition of the decode rows: one wave walks a (row, head, partition), so few sequences with long
     visible ranges are split finely (down to one 64-key tile) and large batches coarsely."""
-    want = max(1, DECODE_WAVES // max(1, n_dec * heads))
+    want = max(1, (DECODE_WAVES if waves is None else waves) // max(1, n_dec * heads))
     per = -(-max(1, visible) // want)
     return max(64, -(-per // 64) * 64)
+
+
+def decode_waves_mfma() -> int:
+    """Waves to aim for on the matrix-core route, whose wave serves all query heads of a key / value head: 32 a compute unit, since a wave
+    waits 3 us for each tile of 32 keys. us with 8 / 16 / 32 / 64 a unit (kernel and merge, H 32, G 8, heads of 128): 33 rows of contexts
+    101-4001 under chunks of 2048 72.8 (3 a unit) / 42.9 / 30.9 / 35.2, plain 256 / 122 (7 partitions) / 54 / 55, 64 rows of 65-1021 62 / 40 / 39 / 39, of 1000-8000 452 / 292 /
+    237 / 244, 9 rows of 64-2000 25.9 / 21.8 / 18.8 / 18.8; G 16, heads of 64: 33 rows 215 / 156 / 58 / 42; G 2: 33 rows 58 / 39 / 25 / 25."""
+    return 2 * DECODE_WAVES
+
+
+def partition_rows(max_seqs: int, heads: int, group: int) -> int:
+    """Rows of the decode partitions' workspace (part_ml, part_o) for `heads` query heads, `group` of them on a key / value head: what the
+    partition lengths above come to, at most 64 partitions a row."""
+    return max(DECODE_WAVES + max_seqs * heads, min(64 * max_seqs * heads, decode_waves_mfma() * min(group, 16)))
 
 
 def _visible_blocks(p0: int, n: int, chunk: int, window: int, heads: int):
@@ -622,7 +636,7 @@ def masked_attention(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, rag: R
         dec_mfma = mfma_ok and H // G <= 16  # a wave's 16 rows are the query heads of one key / value head
         parts, plen = 1, 0
         if workspace is not None:
-            plen = decode_part_len(nd, G * 4 if dec_mfma else H, vis)
+            plen = decode_part_len(nd, G, vis, decode_waves_mfma()) if dec_mfma else decode_part_len(nd, H, vis)
             parts = -(-vis // plen)
             room = min(64, workspace[0].shape[0] // (nd * H))  # the merge holds one partition per lane
             if parts > room:
