@@ -9,7 +9,13 @@
 // but K and V.
 //
 // Tiles of 64 keys are double-buffered: a tile's 16-byte chunks are requested one tile ahead, wait in registers (where
-// fp8 and block formats are widened to bf16) and are stored to the other buffer, one barrier per tile.
+// fp8 and block formats are widened to bf16) and are stored to the other buffer, one barrier per tile. The next tile is stored, and
+// the one after it requested, a piece beside each pair of the scores' products, while the matrix unit is busy: as a stretch of its
+// own before or after the tile it took a seventh of the time (8191 rows 576 -> 548 us, 2000 57 -> 55).
+// A wave requests 4 (head dim 128) or 8 rows with one instruction, which lie in one page where its size is a multiple of that: each
+// lane looks up one such group's row, for 16 tiles or more at once, and the address is a readlane away. (A division, a load of the
+// block table and 64-bit products for each 16 bytes were 100 of an fp8 tile's 400 vector instructions: 416 rows behind 12000 keys
+// 128 -> 120 us with 4 waves.)
 //
 // A short chunk behind a long context has too few workgroups (7 x 8 for 416 rows of a 32 / 8-head model), so the key
 // range is split over grid.z: parts of MIN_TILES tiles or more, the last one of what is left (17 tiles: 16 + 1), write (m, l, O)
@@ -17,10 +23,11 @@
 // finished by that part.
 //
 // Measured, 32 / 8 heads of 128, against the 16-row kernel this replaced (which read each K / V fragment for one 16x16x32
-// product and moved P through LDS): an 8191-token prompt 2400 -> 600 us (917 TFLOP/s), 2048 233 -> 65, 333 18.5 -> 14.0;
-// 416 rows behind 12000 keys 498 -> 140 us in bf16, 788 -> 140 in fp8. Heads of 64, 8191 rows: 1253 -> 360 us. Bound by
-// the vector unit beside the matrix unit (32 exponentials and ~100 other vector operations a lane and tile against 32
-// products); short prompts by the chain of one tile (~1.3 us) times their tiles.
+// product and moved P through LDS): an 8191-token prompt 2400 -> 560 us (980 TFLOP/s), 2048 233 -> 58, 333 18.5 -> 14.0;
+// 416 rows behind 12000 keys 498 -> 110 us in bf16, 788 -> 110 in fp8. Heads of 64, 8191 rows: 1253 -> 360 us. Bound by
+// the vector unit beside the matrix unit (32 exponentials and ~170 other vector operations a lane and tile against 32
+// products: counters show each busy for 40 % of the time and little of both at once); short prompts by the chain of one tile
+// (~1.3 us) times their tiles.
 #include <type_traits>
 
 #include "attn_tile.h"
@@ -61,6 +68,17 @@ MX_DEV typename FRaw<KVF>::T f_load(const void* base, size_t eo) {
     else if constexpr (KVF == KVF_FP8) return *(const uint2*)((const uint8_t*)base + eo);
     else return *(const uint4*)((const bf16_t*)base + eo);
 }
+template <int KVF, int D>
+constexpr uint32_t f_row_bytes() {  // of the cache
+    if constexpr (KVF >= KVF_Q8_0) return KVQ<KVF, D>::ROWB;
+    else return D * (KVF == KVF_FP8 ? 1 : 2);
+}
+template <int KVF, int D>
+MX_DEV typename FRaw<KVF>::T f_load_row(const uint8_t* base, uint32_t v, uint32_t e) {  // row v, elements e .. e + 7
+    const uint32_t r = v * f_row_bytes<KVF, D>();
+    if constexpr (KVF >= KVF_Q8_0) return kvq_load_row<KVF, D>(base, r, e);
+    else return *(const typename FRaw<KVF>::T*)(base + (r + e * (KVF == KVF_FP8 ? 1 : 2)));
+}
 template <int KVF>
 MX_DEV uint4 f_widen(const typename FRaw<KVF>::T& w) {
     if constexpr (KVF >= KVF_Q8_0) return kvq_to_bf16x8<KVF>(w);
@@ -68,8 +86,10 @@ MX_DEV uint4 f_widen(const typename FRaw<KVF>::T& w) {
     else return w;
 }
 
-// GEN: sliding window, soft cap, or a scale that is not positive; without it the scale is one FMA with the maximum
-template <int D, int NW, int KVF, bool GEN>
+// GEN: sliding window, soft cap, or a scale that is not positive; without it the scale is one FMA with the maximum.
+// UNI: the rows that a wave requests with one instruction (4 of head dim 128, 8 of 64, beginning at a multiple of that) lie in
+// one page: their address is scalar but for the lane's place in them.
+template <int D, int NW, int KVF, bool GEN, bool UNI>
 __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_flash_kernel(const bf16_t* __restrict__ q, const void* __restrict__ kc,
                                                              const void* __restrict__ vc, const int* __restrict__ block_tables,
                                                              int bt_stride, const int* __restrict__ cu_q,
@@ -148,12 +168,23 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_flash_kernel(co
     const int wq0 = pos_off + min(q0 + wave * 32 / G, qlen - 1);
     const int wq1 = pos_off + min(q0 + min(RQ - 1, (wave * 32 + 31) / G), qlen - 1);
 
-    // A tile's chunks: block ids one tile before their rows, rows one tile before they are stored. Rows past the last
-    // key repeat it: no column sees them.
+    // A tile's chunks: rows one tile before they are stored. Rows past the last key repeat it: no column sees them.
     typename FRaw<KVF>::T kr[NCH], vr[NCH];
+    constexpr int RPW = 512 / D;                 // rows that a wave requests at a time
+    // UNI: a lane looks up one chunk of the wave's, lane = tile * NCH + chunk of GT tiles, and the next GT tiles' block id
+    constexpr int GT = 64 / NCH;
+    uint32_t place = 0;                          // its first row / RPW
+    int next = 0;
+    // else, for each of the thread's chunks, the block id and the row in it, one tile before the rows
     int blk[NCH], off[NCH];
     const size_t page = (size_t)Hkv * bs * D;
+    auto first_key = [&](int t, int j) {         // of the wave's chunk j of tile t; past the end: the last key's rows
+        return min(kt_begin + t * FT + j * (NT * 8 / D) + wave * RPW, (kv_end - 1) & -RPW);
+    };
+    auto page_of = [&](int key) { return bs_sh >= 0 ? key >> bs_sh : key / bs; };
+    auto lane_key = [&](int t) { return first_key(t + lane / NCH, lane % NCH); };
     auto find_rows = [&](int t) {
+        if constexpr (UNI) return;
 #pragma unroll
         for (int j = 0; j < NCH; ++j) off[j] = min(kt_begin + t * FT + (int)(threadIdx.x + j * NT) / (D / 8), kv_end - 1);
         int bi[NCH];
@@ -170,33 +201,55 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_flash_kernel(co
             off[j] -= bi[j] * bs;
         }
     };
-    auto load_rows = [&]() {
-#pragma unroll
-        for (int j = 0; j < NCH; ++j) {
+    auto look_up = [&](int t) {                  // before tile t's rows, tiles in turn from t0
+        if constexpr (UNI) {
+            if ((t - t0) % GT) return;
+            const int key = lane_key(t), bi = page_of(key);
+            place = (uint32_t)(next * Hkv + kvh) * (uint32_t)(bs / RPW) + (uint32_t)((key - bi * bs) / RPW);
+            next = bt[page_of(lane_key(t + GT))];
+        } else {
+            find_rows(t);
+        }
+    };
+    auto load_chunk = [&](int t, int j) {
+        if constexpr (UNI) {
+            const size_t at = (size_t)(uint32_t)__builtin_amdgcn_readlane(place, (t - t0) % GT * NCH + j) * (RPW * f_row_bytes<KVF, D>());
+            const uint32_t v = min(lane / (D / 8), kv_end - 1 - first_key(t, j)), e = lane % (D / 8) * 8;
+            kr[j] = f_load_row<KVF, D>((const uint8_t*)kc + at, v, e);
+            vr[j] = f_load_row<KVF, D>((const uint8_t*)vc + at, v, e);
+        } else {
             const size_t eo = blk[j] * page + (size_t)((kvh * bs + off[j]) * D + (int)(threadIdx.x + j * NT) % (D / 8) * 8);
             kr[j] = f_load<KVF, D>(kc, eo);
             vr[j] = f_load<KVF, D>(vc, eo);
         }
     };
-    auto store_rows = [&](int buf) {
-        char* kb = smem + buf * (2 * IMG);
-#pragma unroll
-        for (int j = 0; j < NCH; ++j) {
-            const int id = threadIdx.x + j * NT;
-            const int p = id / (D / 8), c = id % (D / 8);
-            *(uint4*)(kb + at_k_off<D>(p, c)) = f_widen<KVF>(kr[j]);
-            *(uint4*)(kb + IMG + at_v_off<D>(p, c >> 1) + 16 * (c & 1)) = f_widen<KVF>(vr[j]);
-        }
+    auto store_k = [&](int buf, int j) {
+        const int id = threadIdx.x + j * NT;
+        *(uint4*)(smem + buf * (2 * IMG) + at_k_off<D>(id / (D / 8), id % (D / 8))) = f_widen<KVF>(kr[j]);
     };
-    constexpr int KB = NW == 8 ? D / 32 : D / 64;  // K fragments read together (a thread of 4 waves holds twice as much staged)
+    auto store_v = [&](int buf, int j) {
+        const int id = threadIdx.x + j * NT, p = id / (D / 8), c = id % (D / 8);
+        *(uint4*)(smem + buf * (2 * IMG) + IMG + at_v_off<D>(p, c >> 1) + 16 * (c & 1)) = f_widen<KVF>(vr[j]);
+    };
+    constexpr int KB = UNI || NW == 8 || D == 64 ? D / 64 : 1;  // k-steps whose K fragments are read together
     int vo[D / 32];
     at_v_lane<D>(lane, vo);
+    // tile t + 1 from the registers to the other buffer, tile t + 2's rows requested: a piece beside each pair of products
+    auto piece = [&](int t, int i) {
+        if (i >= 2 * NCH) return;
+        if (i % 2 == 0) store_k((t + 1) & 1, i / 2);
+        else {
+            store_v((t + 1) & 1, i / 2);
+            load_chunk(min(t + 2, t1 - 1), i / 2);
+        }
+    };
     auto work = [&](int t) {
         const char* kb = smem + (t & 1) * (2 * IMG);
         const char* vb = kb + IMG;
         const int kt0 = kt_begin + t * FT;
         f32x16 sc[2];
-        at_scores<D, false, KB>(kb, h, col, qf, sc);
+        at_scores<D, false, KB>(kb, h, col, qf, sc, [&](int ks) { piece(t, ks); });
+        if (kt0 > wq1) return;  // (uniform per wave) tiles past the wave's last query carry nothing
         u32x4 vf[4][D / 32];
         __builtin_amdgcn_sched_barrier(0);
         at_read_v<D>(vb, vo, 0, vf);
@@ -224,26 +277,23 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_flash_kernel(co
     };
 
     if (t0 < t1) {
-        find_rows(t0);
-        load_rows();
-        find_rows(min(t0 + 1, t1 - 1));
-        store_rows(t0 & 1);
-        load_rows();
-        find_rows(min(t0 + 2, t1 - 1));
+        if constexpr (UNI) next = bt[page_of(lane_key(t0))];
+        look_up(t0);
+#pragma unroll
+        for (int j = 0; j < NCH; ++j) load_chunk(t0, j);
+#pragma unroll
+        for (int j = 0; j < NCH; ++j) {
+            store_k(t0 & 1, j);
+            store_v(t0 & 1, j);
+        }
+        if (t0 + 1 < t1) look_up(t0 + 1);
+#pragma unroll
+        for (int j = 0; j < NCH; ++j) load_chunk(min(t0 + 1, t1 - 1), j);
         __syncthreads();
         for (int t = t0; t < t1; ++t) {
-            // the other buffer was last read while tile t - 1 was worked on, before the barrier that ended that round;
-            // half of the waves store first and half work first, so that one's matrix products run beside the other's loads
-            auto stage = [&]() {
-                if (t + 1 >= t1) return;
-                store_rows((t + 1) & 1);
-                load_rows();  // (past the end: the last tile's rows once more, not stored)
-                find_rows(min(t + 3, t1 - 1));
-            };
-            const bool first = wave < NW / 2;
-            if (first) stage();
-            if (kt_begin + t * FT <= wq1) work(t);  // (uniform per wave) tiles past the wave's last query carry nothing
-            if (!first) stage();
+            // the other buffer was last read while tile t - 1 was worked on, before the barrier that ended that round
+            if (t + 2 < t1) look_up(t + 2);
+            work(t);
             __syncthreads();
         }
     }
@@ -326,17 +376,22 @@ int launch_flash(const bf16_t* q, const void* kc, const void* vc, const int* bt,
     constexpr int LDS = 4 * FT * D * 2;
     const int sh = (bs & (bs - 1)) ? -1 : __builtin_ctz(bs);
     const bool gen = window > 0 || softcap > 0.f || !(scale > 0.f);
-#define FL(GEN_)                                                                                                             \
+#define FL(GEN_, UNI_)                                                                                                       \
     do {                                                                                                                     \
-        static const hipError_t once = hipFuncSetAttribute((const void*)attn_flash_kernel<D, NW, KVF, GEN_>,            \
+        static const hipError_t once = hipFuncSetAttribute((const void*)attn_flash_kernel<D, NW, KVF, GEN_, UNI_>,            \
                                                            hipFuncAttributeMaxDynamicSharedMemorySize, LDS);                 \
         if (once != hipSuccess) return (int)once;                                                                            \
-        attn_flash_kernel<D, NW, KVF, GEN_><<<grid, 64 * NW, LDS, st>>>(q, kc, vc, bt, bt_stride, cu_q, ctx_lens, n_seqs, \
+        attn_flash_kernel<D, NW, KVF, GEN_, UNI_><<<grid, 64 * NW, LDS, st>>>(q, kc, vc, bt, bt_stride, cu_q, ctx_lens, n_seqs, \
                                                                              T, Hq, Hkv, G, bs, sh, scale, window, softcap,  \
                                                                              out, g_mx_act_f16, part_o, part_ml);                          \
     } while (0)
-    if (gen) FL(true);
-    else FL(false);
+    if (bs % (512 / D) == 0) {
+        if (gen) FL(true, true);
+        else FL(false, true);
+    } else {
+        if (gen) FL(true, false);
+        else FL(false, false);
+    }
     if (n_parts > 1)
         attn_flash_merge_kernel<D><<<(unsigned)(((long)T * Hq * (D / 8) + 255) / 256), 256, 0, st>>>(part_o, part_ml, n_parts, cu_q,
                                                                                                n_seqs, T, Hq, out, g_mx_act_f16);

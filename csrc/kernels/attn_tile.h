@@ -4,6 +4,8 @@
 // probabilities are then the B operand of O^T = V^T P^T as they lie, both operands' k slot (h, e) being key 8 (e / 4) + 4 h + e % 4
 // of the 16.
 #pragma once
+#include <type_traits>
+
 #include "mx_common.h"
 
 namespace {
@@ -44,9 +46,13 @@ MX_DEV f32x16 at_mfma(u32x4 a, u32x4 b, f32x16 c) {
 // A tile in three steps; sc[u][j] is key 32 u + 8 (j / 4) + 4 h + j % 4 of the lane's column. The fences keep the fragment reads ahead
 // of what they wait behind: K's before the first product, V's first before the softmax, its others one k-step ahead of their
 // products (left alone, the scheduler puts every read next to its use).
-// 1. sc = K Q^T; qf: Q^T as B operand (lane = column, dims 16 ks + 8 h). KB: k-steps whose K fragments are read together
-template <int D, bool F16, int KB>
-MX_DEV void at_scores(const char* kb, int h, int col, const u32x4 (&qf)[D / 16], f32x16 (&sc)[2]) {
+// 1. sc = K Q^T; qf: Q^T as B operand (lane = column, dims 16 ks + 8 h). KB: k-steps whose K fragments are read together;
+// mid(ks): other work of the wave, issued while k-step ks's two products run (each holds the matrix unit for 32 cycles)
+struct AtNone {
+    MX_DEV void operator()(int) const {}
+};
+template <int D, bool F16, int KB, class Mid = AtNone>
+MX_DEV void at_scores(const char* kb, int h, int col, const u32x4 (&qf)[D / 16], f32x16 (&sc)[2], Mid mid = {}) {
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -65,9 +71,15 @@ MX_DEV void at_scores(const char* kb, int h, int col, const u32x4 (&qf)[D / 16],
         if (k0 + KB < D / 16) read_k(k0 + KB);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int ks = k0; ks < k0 + KB; ++ks)
+        for (int ks = k0; ks < k0 + KB; ++ks) {
 #pragma unroll
             for (int u = 0; u < 2; ++u) sc[u] = at_mfma<F16>(kf[ks][u], qf[ks], sc[u]);
+            if constexpr (!std::is_same<Mid, AtNone>::value) {
+                __builtin_amdgcn_sched_barrier(0);
+                mid(ks);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
     }
 }
 // Where in a V image this lane's reads of V^T's fragments begin: row 4 h + (lane % 16) / 4, dims 32 mt on. The rows of a k-step and its

@@ -35,21 +35,24 @@ struct KVQRaw {
     uint32_t hb;  // high-bit byte (q5_*)
 };
 
+// elements e .. e + 7 (e % 8 == 0) of the row of ROWB bytes at base + r (32-bit offsets: a base that all lanes share stays scalar)
+template <int KVF, int D>
+MX_DEV KVQRaw kvq_load_row(const uint8_t* base, uint32_t r, uint32_t e) {
+    using Q = KVQ<KVF, D>;
+    KVQRaw o;
+    if constexpr (Q::Q8) o.c = *(const uint2*)(base + (r + e));
+    else o.c = make_uint2(*(const uint32_t*)(base + (r + e / 2)), 0u);
+    if constexpr (Q::HB) o.hb = base[r + Q::CB + e / 8];
+    else o.hb = 0;
+    if constexpr (Q::MIN) o.s = *(const uint32_t*)(base + (r + Q::CB + Q::HBB + (e / 32) * 4));
+    else o.s = *(const uint16_t*)(base + (r + Q::CB + Q::HBB + (e / 32) * 2));
+    return o;
+}
+
 // 8 elements starting at element offset eo (= row * D + e, e % 8 == 0) of a cache laid out as rows of ROWB bytes
 template <int KVF, int D>
 MX_DEV KVQRaw kvq_load(const void* base, size_t eo) {
-    using Q = KVQ<KVF, D>;
-    const size_t row = eo / D;
-    const int e = (int)(eo % D);
-    const uint8_t* r = (const uint8_t*)base + row * Q::ROWB;
-    KVQRaw o;
-    if constexpr (Q::Q8) o.c = *(const uint2*)(r + e);
-    else o.c = make_uint2(*(const uint32_t*)(r + e / 2), 0u);
-    if constexpr (Q::HB) o.hb = r[Q::CB + e / 8];
-    else o.hb = 0;
-    if constexpr (Q::MIN) o.s = *(const uint32_t*)(r + Q::CB + Q::HBB + (e / 32) * 4);
-    else o.s = *(const uint16_t*)(r + Q::CB + Q::HBB + (e / 32) * 2);
-    return o;
+    return kvq_load_row<KVF, D>((const uint8_t*)base + eo / D * KVQ<KVF, D>::ROWB, 0u, (uint32_t)(eo % D));
 }
 
 template <int KVF>

@@ -132,6 +132,33 @@ def test_windows_caps_and_scales(window, softcap, scale, monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("D,waves", [(128, 4), (128, 8), (64, 4), (64, 8)])
+@pytest.mark.parametrize("bs", [4, 6, 8, 10, 24, 256, 5000])
+@pytest.mark.parametrize("rise", [0.0, 40.0])
+def test_pages_and_rising_scores(bs, D, waves, rise, monkeypatch):
+    """Pages that hold the groups of rows a wave requests (4 of head dim 128, 8 of 64) and pages that cut them, over more tiles than one
+    look-up covers (16, 32 or 64); slots behind the contexts are not numbers. rise: log2 by which the scores grow over a context, so
+    that every tile finds a new maximum."""
+    q, kc, vc, bt, cu, ctx = _case(8, 2, D, [70, 33], [4130, 61], bs=bs, seed=bs)
+    free = torch.ones(kc.shape[0], bs, dtype=torch.bool)
+    q[..., 0] = 1.0
+    for i, c in enumerate(ctx.tolist()):
+        at = torch.arange(c)
+        b, r = bt[i].long()[at // bs], at % bs
+        free[b, r] = False
+        kc[b, :, r, 0] = (at[:, None] / c * rise * math.log(2) * D ** 0.5).to(torch.bfloat16)
+    for t in (kc, vc):
+        t.transpose(1, 2)[free] = float("nan")
+    want = torch.cat([K._attn_ref_one(q[int(cu[i]):int(cu[i + 1])], kc, vc, bt[i], int(c), int(c) - int(cu[i + 1] - cu[i]), D ** -0.5, bs)
+                      for i, c in enumerate(ctx)])
+    monkeypatch.setattr(K, "flash_plan", lambda *a, **k: (waves, 2))
+    out = torch.full(q.shape, float("nan"), dtype=torch.float16, device="cuda")
+    K.attn_prefill(q.cuda(), kc.cuda(), vc.cuda(), bt.cuda(), cu.cuda(), ctx.cuda(), D ** -0.5, out, [70, 33], ctx.tolist())
+    # probabilities and outputs are rounded to 16 bits once each
+    assert float((out.cpu().float() - want).norm() / want.norm()) < 4 * 2 ** -9
+
+
+@pytest.mark.gpu
 def test_infinite_scores_behave_like_the_reference():
     """A key of infinite score makes its row NaN, and no other row."""
     q, kc, vc, bt, cu, ctx = _case(4, 1, 128, [80], [0])
