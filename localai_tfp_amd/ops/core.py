@@ -450,6 +450,10 @@ def flash_plan(T: int, n_seqs: int, Hq: int, Hkv: int, D: int, block_size: int, 
     A grid of fewer than two workgroups per compute unit is split over its keys where the context is long: 416 rows behind
     12000 keys 275 -> 140 us, 289 behind 2000 58 -> 41; the merge launch costs 1.5-2 us where it has nothing to merge, so
     contexts that are known to be short (else what the block tables can hold) do not ask for it.
+    One sequence's chunk behind a context known to be 64 key tiles or more and four times its rows goes to 8 waves in as many
+    parts as still run at once: half the staging per product (32 / 8 x 128, us with 4 / 8: 416 rows behind 12000 keys 119 / 110,
+    in fp8 136 / 114, behind 6000 73 / 68, 1000 behind 12000 238 / 215, 2048 457 / 433). Not chunks of fewer than two blocks (64
+    rows behind 30000 81 / 101), nor shorter contexts (289 behind 2000 41 / 50, whole prompts of 1500 42 / 48).
     Contexts of one key tile are the 16-row kernel's where its smaller workgroups wait less (us here / there, D 128): few of
     them 8.6 / 7.4 (33 rows), sequences that its row tiles hold whole 9.4 / 7.4 (64 x 1), 27 / 19 (200 x 1), 17.4 / 14.4 (100 x
     10), with a soft cap 9.4 / 7.5 (33 rows); not 11.7 / 17.3 (64 x 17), nor beyond what the chip holds at once with more than 4
@@ -469,6 +473,10 @@ def flash_plan(T: int, n_seqs: int, Hq: int, Hkv: int, D: int, block_size: int, 
     blocks = lambda waves: T // (32 * waves // G) + min(n_seqs, T)  # noqa: E731
     if D == 128 and T >= 4096 * n_seqs and T // (256 // G) * Hkv >= 2 * CU_COUNT:
         return (8, 1) if blocks(8) <= 65535 else None
+    rows8 = 256 // G
+    wide = -(-T // rows8) * Hkv
+    if n_seqs == 1 and ctx_lens_host and window <= 0 and longest >= max(4096, 4 * T) and T >= 2 * rows8 and wide <= CU_COUNT:
+        return 8, min(16, CU_COUNT // wide)
     base = blocks(4) * Hkv
     keys = min(longest, window + 32 * 4 // G) if window > 0 else longest
     parts = max(1, min(16, 2 * CU_COUNT // base)) if keys >= FLASH_SPLIT_KEYS else 1

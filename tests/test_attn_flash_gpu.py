@@ -158,6 +158,15 @@ def test_pages_and_rising_scores(bs, D, waves, rise, monkeypatch):
     assert float((out.cpu().float() - want).norm() / want.norm()) < 4 * 2 ** -9
 
 
+def test_plan_of_chunks_behind_long_contexts():
+    """8 waves for one sequence's chunk of two blocks or more where 64 key tiles and four times its rows are known to lie before it."""
+    p = lambda T, ctx, n=1, H=32, window=0: K.flash_plan(T, n, H, 8, 128, 16, 2048, window, ctx)  # noqa: E731
+    assert p(416, [12416]) == (8, 4) and p(128, [4096]) == (8, 16) and p(1024, [4096]) == (8, 2) and p(2048, [14048]) == (8, 1)
+    assert p(127, [4096])[0] == 4 and p(416, [4095])[0] == 4 and p(1025, [4096])[0] == 4 and p(2049, [14048])[0] == 4
+    assert p(416, None)[0] == 4 and p(416, [12416] * 2, 2)[0] == 4 and p(416, [12416], window=512)[0] == 4
+    assert p(64, [9000], H=64) == (8, 16) and p(63, [9000], H=64)[0] == 4
+
+
 @pytest.mark.gpu
 def test_infinite_scores_behave_like_the_reference():
     """A key of infinite score makes its row NaN, and no other row."""
