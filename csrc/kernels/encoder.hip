@@ -3,10 +3,11 @@
 // A layer is four GEMMs, attention (attention_dense.hip) and two LayerNorms. Batches of few rows are bound by launches
 // and by the time a workgroup waits for its first loads, large ones by the GEMMs and by the passes between them; so
 //   - few rows run whole layers from one call (mxk_enc_layers), with a GEMM that splits K over the waves of a workgroup
-//     and applies bias and GELU to its fp32 sums;
+//     and applies bias and GELU to its fp32 sums, and with what lies before a product done inside it where that is cheaper
+//     than a launch: attention of one text up to 64 rows, the norms up to 16;
 //   - above, the caller multiplies with the library and the passes between are one kernel each, over 16-bit rows.
 // Measured on BERT-base, against padded rows with fp32 copies around each LayerNorm and a library call per operation: one
-// text of 19 tokens 2019 -> 483 us (87 launches of 4-6 us), 48 texts of 23-401 tokens (6428 rows of 19248 padded) 7147 ->
+// text of 19 tokens 2019 -> 375 us (75 launches of 4-5 us; 8 tokens 275, 51 launches), 48 texts of 23-401 tokens (6428 rows of 19248 padded) 7147 ->
 // 2278: LayerNorm + casts 74 -> 8.3 us (30 MB: 3.6 TB/s), GELU 40 -> 16 (79 MB: 4.9 TB/s).
 #include "dense16.h"
 #include "mx_common.h"
@@ -41,6 +42,20 @@ struct LnGain {
     }
 };
 
+// Sum over the wave, in every lane, without LDS: with __shfl_xor's six permutations through LDS each of a row's two sums took 0.6 us.
+template <int CTRL>
+MX_DEV float dpp_add(float v) { return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true)); }
+MX_DEV float row_sum(float v) {
+    v = dpp_add<0xB1>(v);   // lanes 1 0 3 2 of a quad
+    v = dpp_add<0x4E>(v);   // 2 3 0 1
+    v = dpp_add<0x141>(v);  // mirrored in 8 lanes
+    v = dpp_add<0x140>(v);  // in 16
+    u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false));
+    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false));
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
 // LayerNorm of one row. Two passes over registers: the variance is a sum of squares about the mean.
 template <int NC, bool F16>
 MX_DEV void ln_row(float (&v)[NC][8], int H, const LnGain<NC>& gb, float eps, uint16_t* __restrict__ out, int lane) {
@@ -49,7 +64,7 @@ MX_DEV void ln_row(float (&v)[NC][8], int H, const LnGain<NC>& gb, float eps, ui
     for (int j = 0; j < NC; ++j)
 #pragma unroll
         for (int e = 0; e < 8; ++e) s += v[j][e];
-    const float mean = wave_sum(s) / H;
+    const float mean = row_sum(s) / H;
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
@@ -58,7 +73,7 @@ MX_DEV void ln_row(float (&v)[NC][8], int H, const LnGain<NC>& gb, float eps, ui
         for (int e = 0; e < 8; ++e) q += (v[j][e] - mean) * (v[j][e] - mean);
         ss += enc_has(j, H, lane) ? q : 0.f;
     }
-    const float rs = rsqrtf(wave_sum(ss) / H + eps);
+    const float rs = rsqrtf(row_sum(ss) / H + eps);
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
         float y[8];
@@ -149,12 +164,11 @@ __global__ __launch_bounds__(64 * EW) void enc_add_ln_kernel(const uint16_t* __r
     ln_row<NC, F16>(v, H, gb, eps, x + (size_t)row * H, lane);
 }
 
-// x = LN(sum of parts + bias + x); parts [NP][rows][H] fp32
+// y = LN(sum of parts + bias + x); parts [NP][rows][H] fp32; y may be x
 template <int NC, int NP, bool F16>
-__global__ __launch_bounds__(64 * EW) void enc_parts_ln_kernel(const float* __restrict__ parts,
-                                                               const uint16_t* __restrict__ bias, uint16_t* __restrict__ x, int rows,
-                                                               const float* __restrict__ g, const float* __restrict__ b, int H,
-                                                               float eps) {
+__global__ __launch_bounds__(64 * EW) void enc_parts_ln_kernel(const float* __restrict__ parts, const uint16_t* __restrict__ bias,
+                                                               const uint16_t* x, uint16_t* y, int rows, const float* __restrict__ g,
+                                                               const float* __restrict__ b, int H, float eps) {
     const int row = blockIdx.x * EW + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (row >= rows) return;
     LnGain<NC> gb;
@@ -164,7 +178,7 @@ __global__ __launch_bounds__(64 * EW) void enc_parts_ln_kernel(const float* __re
     for (int p = 0; p < NP; ++p) add_f32<NC>(v, parts + ((size_t)p * rows + row) * H, H, lane);
     if (bias) add_act<NC, F16>(v, bias, H, lane);
     add_act<NC, F16>(v, x + (size_t)row * H, H, lane);
-    ln_row<NC, F16>(v, H, gb, eps, x + (size_t)row * H, lane);
+    ln_row<NC, F16>(v, H, gb, eps, y + (size_t)row * H, lane);
 }
 
 // y = gelu(y) in place, 8 elements a thread
@@ -250,6 +264,24 @@ MX_DEV f32x4 enc_mfma(u32x4 a, u32x4 b, f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
+// element idx of a 16 MT x 16 tile whose 8 waves' sums are in red
+template <int MT, bool F16, int OUT>
+MX_DEV void enc_store(const float* red, int idx, const uint16_t* __restrict__ bias, void* __restrict__ y, int m0, int M, int N, int n0) {
+    const int n = idx & 15, r = idx >> 4, m = m0 + r;
+    if (m >= M) return;
+    const int e = (r >> 4) * 256 + (((r & 15) >> 2) * 16 + n) * 4 + (r & 3);
+    float v = 0.f;
+#pragma unroll
+    for (int w = 0; w < GW; ++w) v += red[w * MT * 256 + e];
+    if constexpr (OUT == ENC_PART) {
+        ((float*)y)[(size_t)m * N + n0 + n] = v;
+    } else {
+        if (bias) v += act_to_f32<F16>(bias[n0 + n]);
+        if constexpr (OUT == ENC_GELU) v = gelu_erf_f(v);
+        ((uint16_t*)y)[(size_t)m * N + n0 + n] = f32_to_act<F16>(v);
+    }
+}
+
 // y[M, N] = act(x[M, K] W[N, K]^T + bias), 16-bit in and out, fp32 sums; or, ENC_PART, the fp32 sums of gridDim.z parts of K
 // one after another, which the LayerNorm that follows adds up. A workgroup has 16 columns and 16 MT rows; its 8 waves take
 // every 8th 32-wide k-step and their sums meet in LDS. What bounds it is the wait for the first loads: a wave asks for U
@@ -296,21 +328,218 @@ __global__ __launch_bounds__(64 * GW) void enc_gemm_kernel(const uint16_t* __res
     for (int t = 0; t < MT; ++t)
         *(float4*)(red + ((wave * MT + t) * 64 + lane) * 4) = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
     __syncthreads();
-    for (int idx = threadIdx.x; idx < MT * 256; idx += 64 * GW) {
-        const int n = idx & 15, r = idx >> 4, m = m0 + r;
-        if (m >= M) continue;
-        const int e = (r >> 4) * 256 + (((r & 15) >> 2) * 16 + n) * 4 + (r & 3);
-        float v = 0.f;
+    if constexpr (OUT == ENC_PART) y = (float*)y + (size_t)blockIdx.z * M * N;
+    for (int idx = threadIdx.x; idx < MT * 256; idx += 64 * GW) enc_store<MT, F16, OUT>(red, idx, bias, y, m0, M, N, n0);
+}
+
+// ---- few rows: what comes before a product is done by each of its workgroups, on rows that stay in LDS ----
+// Every launch of a layer waits ~4 us for its first loads whatever it does, and the host issues one in as long: seven a layer become six
+// (one text up to 64 rows: attention inside the output product), five (several texts, up to 16 rows: both norms inside) or four. A
+// workgroup has all M rows and 16 columns of the weights, whose fragments (all NS k-steps of its wave) are asked for ahead of the rows.
+template <int MT, int NS, bool F16>
+struct EncTail {
+    u32x4 wf[NS];
+    int wave, lane, steps;
+    MX_DEV void load(const uint16_t* __restrict__ W, int n0, int K, int k0, int k1) {  // columns n0 .. n0 + 15, K's k0 .. k1
+        wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        lane = threadIdx.x & 63;
+        steps = (k1 - k0) / 32;
+        const uint16_t* wp = W + (size_t)(n0 + (lane & 15)) * K + k0 + 8 * (lane >> 4);
 #pragma unroll
-        for (int w = 0; w < GW; ++w) v += red[w * MT * 256 + e];
-        if constexpr (OUT == ENC_PART) {
-            ((float*)y)[((size_t)blockIdx.z * M + m) * N + n0 + n] = v;
-        } else {
-            if (bias) v += act_to_f32<F16>(bias[n0 + n]);
-            if constexpr (OUT == ENC_GELU) v = gelu_erf_f(v);
-            ((uint16_t*)y)[(size_t)m * N + n0 + n] = f32_to_act<F16>(v);
+        for (int u = 0; u < NS; ++u) wf[u] = *(const u32x4*)(wp + 32 * min(wave + GW * u, steps - 1));
+    }
+    // y[M, N] as enc_gemm_kernel's, from rows [16 MT][ld] in LDS that are complete behind a barrier; the sums take their place. ld: 8 more
+    // than the rows have, so that 16 rows' chunks lie in different banks
+    template <int OUT>
+    MX_DEV void store(char* smem, int ld, const uint16_t* __restrict__ bias, void* __restrict__ y, int M, int N, int n0) {
+        const uint16_t* rows = (const uint16_t*)smem + (lane & 15) * ld + 8 * (lane >> 4);
+        float* red = (float*)smem;
+        f32x4 acc[MT];
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < NS; ++u)
+            if (wave + GW * u < steps)
+#pragma unroll
+                for (int t = 0; t < MT; ++t) acc[t] = enc_mfma<F16>(*(const u32x4*)(rows + 16 * t * ld + 32 * (wave + GW * u)), wf[u], acc[t]);
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < MT; ++t) *(float4*)(red + ((wave * MT + t) * 64 + lane) * 4) = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
+        __syncthreads();
+        for (int idx = threadIdx.x; idx < MT * 256; idx += 64 * GW) enc_store<MT, F16, OUT>(red, idx, bias, y, 0, M, N, n0);
+    }
+};
+
+// y = act(LN(sum of parts + pbias + x) W^T + bias); the first workgroup stores the normalised rows, the next residual, to xn (not x). A wave
+// has RW rows. Bound by reading the parts into every compute unit: with 768 x 3072 weights and four parts 9.2 us at 16 rows, 13.3 at 19, where
+// norm and product are 4.1 + 4.7; whole calls, us, norms apart / inside, 12 layers: 8 rows 398 / 279, 16 rows 403 / 339, 17 rows 344 / 435.
+template <int RW, int NC, int NP, bool F16, int OUT>
+__global__ __launch_bounds__(64 * GW) void enc_ln_gemm_kernel(const float* __restrict__ parts, const uint16_t* __restrict__ pbias,
+                                                              const uint16_t* __restrict__ x, const float* __restrict__ g, const float* __restrict__ b,
+                                                              float eps, uint16_t* __restrict__ xn, const uint16_t* __restrict__ W,
+                                                              const uint16_t* __restrict__ bias, void* __restrict__ y, int M, int N, int K) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int n0 = blockIdx.x * 16, ld = K + 8;
+    EncTail<(RW + 1) / 2, 2 * NC, F16> tail;
+    tail.load(W, n0, K, 0, K);
+    const int lane = tail.lane;
+    LnGain<NC> gb;
+    gb.load(g, b, K, lane);
+    float v[RW][NC][8] = {};  // (rows past M: the last one's again, not stored)
+#pragma unroll
+    for (int i = 0; i < RW; ++i) {
+        const int row = min(tail.wave + GW * i, M - 1);
+#pragma unroll
+        for (int p = 0; p < NP; ++p) add_f32<NC>(v[i], parts + ((size_t)p * M + row) * K, K, lane);
+        if (pbias) add_act<NC, F16>(v[i], pbias, K, lane);
+        add_act<NC, F16>(v[i], x + (size_t)row * K, K, lane);
+    }
+#pragma unroll
+    for (int i = 0; i < RW; ++i) ln_row<NC, F16>(v[i], K, gb, eps, (uint16_t*)smem + (tail.wave + GW * i) * ld, lane);
+    __syncthreads();
+    if (blockIdx.x == 0)
+        for (int c = threadIdx.x; c < M * (K / 8); c += 64 * GW) {
+            const int r = c / (K / 8), e = (c - r * (K / 8)) * 8;
+            *(uint4*)(xn + (size_t)r * K + e) = *(const uint4*)((const uint16_t*)smem + r * ld + e);
+        }
+    tail.template store<OUT>(smem, ld, bias, y, M, N, n0);
+}
+
+// y = attention(qkv) W^T, fp32, of one text of M <= 16 MT rows that sees its first klen keys; heads of 64, gridDim.z parts of them, whose
+// products go to as many parts of y: every workgroup computes its heads anew for its 16 columns. A wave takes every 8th pair of a head
+// and 16 queries: S^T = K Q^T gives a lane its query's keys 16 t + 4 g + i, which are the next product's B operand with the k slots in
+// that order; V is gathered to match. Nothing but the heads' outputs goes through LDS. 12 heads, 19 rows: 4.3 us in four parts of the
+// heads (8.6 in one: three pairs a wave, one after another) where attention and product were 4.6 + 4.3.
+template <int MT, int NS, bool F16>
+__global__ __launch_bounds__(64 * GW) void enc_attn_gemm_kernel(const uint16_t* __restrict__ qkv, const int* __restrict__ klen, float scale, int heads,
+                                                                const uint16_t* __restrict__ W, float* __restrict__ y, int M, int H) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int h0 = heads * blockIdx.z / gridDim.z, h1 = heads * (blockIdx.z + 1) / gridDim.z;
+    const int n0 = blockIdx.x * 16, ld = (h1 - h0) * 64 + 8, qld = 3 * H;
+    EncTail<MT, NS, F16> tail;
+    tail.load(W, n0, H, 64 * h0, 64 * h1);
+    const int lane = tail.lane, col = lane & 15, g = lane >> 4;
+    const int live = min(klen[0], M), last = max(live, 1) - 1;
+    constexpr int KS = (MT + 1) / 2;  // 32-key steps
+    const float qs = scale * 1.4426950408889634f;
+    for (int u = tail.wave; u < (h1 - h0) * MT; u += GW) {
+        const int hd = u / MT * 64, q0 = u % MT * 16;
+        const uint16_t* base = qkv + 64 * h0 + hd;
+        u32x4 qf[2], kf[MT][2];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            qf[ks] = *(const u32x4*)(base + (size_t)min(q0 + col, M - 1) * qld + 32 * ks + 8 * g);
+#pragma unroll
+            for (int t = 0; t < MT; ++t) kf[t][ks] = *(const u32x4*)(base + H + (size_t)min(16 * t + col, last) * qld + 32 * ks + 8 * g);
+        }
+        uint16_t vv[4][8 * KS] = {};  // [16 dims][key]
+#pragma unroll
+        for (int e = 0; e < 4 * MT; ++e) {
+            const uint16_t* vp = base + 2 * H + (size_t)min(16 * (e >> 2) + 4 * g + (e & 3), last) * qld + col;
+#pragma unroll
+            for (int mt = 0; mt < 4; ++mt) vv[mt][e] = vp[16 * mt];
+        }
+        float p[8 * KS] = {}, m = -INFINITY, l = 0.f;
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            f32x4 sc = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) sc = enc_mfma<F16>(kf[t][ks], qf[ks], sc);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                p[4 * t + i] = 16 * t + 4 * g + i < live ? sc[i] * qs : -INFINITY;
+                m = fmaxf(m, p[4 * t + i]);
+            }
+        }
+        m = fmaxf(m, __shfl_xor(m, 16));
+        m = fmaxf(m, __shfl_xor(m, 32));
+        const float mu = m == -INFINITY ? 0.f : m;
+#pragma unroll
+        for (int e = 0; e < 4 * MT; ++e) {
+            p[e] = __builtin_amdgcn_exp2f(p[e] - mu);
+            l += p[e];
+        }
+        l += __shfl_xor(l, 16);
+        l += __shfl_xor(l, 32);
+        const float inv = l > 0.f ? 1.f / l : 0.f;
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) {
+            f32x4 o = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                uint32_t a[4], w[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int k = 8 * ks + 2 * e;
+                    a[e] = (uint32_t)vv[mt][k] | (uint32_t)vv[mt][k + 1] << 16;
+                    w[e] = pack_act2<F16>(p[k], p[k + 1]);
+                }
+                o = enc_mfma<F16>((u32x4){a[0], a[1], a[2], a[3]}, (u32x4){w[0], w[1], w[2], w[3]}, o);
+            }
+            *(uint2*)((uint16_t*)smem + (q0 + col) * ld + hd + 16 * mt + 4 * g) =
+                live > 0 ? make_uint2(pack_act2<F16>(o[0] * inv, o[1] * inv), pack_act2<F16>(o[2] * inv, o[3] * inv)) : make_uint2(0, 0);
         }
     }
+    __syncthreads();
+    tail.template store<ENC_PART>(smem, ld, nullptr, y + (size_t)blockIdx.z * M * H, M, H, n0);
+}
+
+template <int MT>
+constexpr size_t enc_fused_lds(int K) {
+    const size_t rows = (size_t)16 * MT * (K + 8) * 2, red = (size_t)GW * MT * 1024;
+    return rows > red ? rows : red;
+}
+constexpr int ENC_NORM_ROWS = 16, ENC_ATTN_ROWS = 64, ENC_FUSED_H = 1024;
+int enc_attn_parts(int M, int heads) { return heads < 2 ? 1 : heads < 4 || M <= 16 ? 2 : 4; }  // of the heads: a pair a wave or two
+
+template <bool F16, int OUT>
+int enc_ln_gemm(int np, const float* parts, const uint16_t* pbias, const uint16_t* x, const float* g, const float* b, float eps, uint16_t* xn,
+                const uint16_t* W, const uint16_t* bias, void* y, int M, int N, int K, hipStream_t st) {
+#define EL(RW_, NC_, NP_)                                                                                                              \
+    do {                                                                                                                               \
+        constexpr int MT = (RW_ + 1) / 2;                                                                                              \
+        static const hipError_t once = hipFuncSetAttribute((const void*)enc_ln_gemm_kernel<RW_, NC_, NP_, F16, OUT>,                   \
+                                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)enc_fused_lds<MT>(512 * NC_)); \
+        if (once != hipSuccess) return (int)once;                                                                                      \
+        enc_ln_gemm_kernel<RW_, NC_, NP_, F16, OUT><<<N / 16, 64 * GW, enc_fused_lds<MT>(K), st>>>(parts, pbias, x, g, b, eps, xn, W, bias, y, M, N, K); \
+        return (int)hipGetLastError();                                                                                                 \
+    } while (0)
+#define ELN(RW_)                             \
+    if (M <= GW * RW_) {                     \
+        if (K <= 512 && np == 1) EL(RW_, 1, 1); \
+        if (K <= 512 && np == 2) EL(RW_, 1, 2); \
+        if (K <= 512) EL(RW_, 1, 4);         \
+        if (np == 1) EL(RW_, 2, 1);          \
+        if (np == 2) EL(RW_, 2, 2);          \
+        EL(RW_, 2, 4);                       \
+    }
+    ELN(1) ELN(2)
+#undef ELN
+#undef EL
+    return (int)hipErrorInvalidValue;
+}
+
+template <bool F16>
+int enc_attn_gemm(const uint16_t* qkv, const int* klen, float scale, int heads, const uint16_t* W, float* y, int M, int H, hipStream_t st) {
+    const int parts = enc_attn_parts(M, heads), K = (heads + parts - 1) / parts * 64;  // (of the largest part)
+#define EA(MT_, NS_)                                                                                                                   \
+    do {                                                                                                                               \
+        static const hipError_t once = hipFuncSetAttribute((const void*)enc_attn_gemm_kernel<MT_, NS_, F16>,                           \
+                                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)enc_fused_lds<MT_>(256 * NS_)); \
+        if (once != hipSuccess) return (int)once;                                                                                      \
+        enc_attn_gemm_kernel<MT_, NS_, F16><<<dim3(H / 16, 1, parts), 64 * GW, enc_fused_lds<MT_>(K), st>>>(qkv, klen, scale, heads, W, y, M, H); \
+        return (int)hipGetLastError();                                                                                                 \
+    } while (0)
+#define EAM(MT_)                      \
+    if (M <= 16 * MT_) {              \
+        if (K <= 256) EA(MT_, 1);     \
+        if (K <= 512) EA(MT_, 2);     \
+        EA(MT_, 4);                   \
+    }
+    EAM(1) EAM(2) EAM(3) EAM(4)
+#undef EAM
+#undef EA
+    return (int)hipErrorInvalidValue;
 }
 
 template <bool F16, int OUT>
@@ -383,10 +612,10 @@ extern "C" int mxk_enc_pool(const uint16_t* x, const int* cu, const int* klen, i
     MXK_CHECK_LAUNCH();
 }
 
-// x = LN(sum of np parts + bias + x)
-int enc_parts_ln(int np, const float* parts, const uint16_t* bias, uint16_t* x, int rows, const float* g, const float* b, int H, float eps, hipStream_t st) {
+// y = LN(sum of np parts + bias + x); y may be x
+int enc_parts_ln(int np, const float* parts, const uint16_t* bias, const uint16_t* x, uint16_t* y, int rows, const float* g, const float* b, int H, float eps, hipStream_t st) {
     auto go = [&](auto kern) {
-        kern<<<(rows + EW - 1) / EW, 64 * EW, 0, st>>>(parts, bias, x, rows, g, b, H, eps);
+        kern<<<(rows + EW - 1) / EW, 64 * EW, 0, st>>>(parts, bias, x, y, rows, g, b, H, eps);
         return (int)hipGetLastError();
     };
     int rc = (int)hipErrorInvalidValue;
@@ -398,27 +627,41 @@ int enc_parts_ln(int np, const float* parts, const uint16_t* bias, uint16_t* x, 
 }
 
 // w: 12 device pointers a layer: qkv W, b, output W, b, norm g, b (fp32), up W, b, down W, b, norm g, b (fp32); biases may be
-// null. x [rows][H] in and out; qkv [rows][3 H], attn [rows][H], up [rows][F] and parts [4][rows][H] fp32 are scratch.
+// null. x [rows][H] in and out; qkv [rows][3 H], attn [rows][H], up [rows][F] and parts [5][rows][H] fp32 are scratch.
 extern "C" int mxk_enc_layers(const void* const* w, int n_layers, uint16_t* x, int rows, int B, int Smax, const int* cu,
                               const int* klen, int H, int heads, int F, float scale, float eps, uint16_t* qkv, uint16_t* attn,
                               float* parts, uint16_t* up, hipStream_t st) {
     if (rows <= 0 || n_layers <= 0) return 0;
     if (!enc_width_ok(H) || H % 32 || F % 32 || heads <= 0 || H % heads) return (int)hipErrorInvalidValue;
     static_assert(enc_parts(32) == 1 && enc_parts(1 << 20) == 4, "parts");
+    const int np = enc_parts(F);
+    const bool one = B == 1 && H / heads == 64 && rows <= ENC_ATTN_ROWS && H <= ENC_FUSED_H;
+    const bool norms = rows <= ENC_NORM_ROWS && H <= ENC_FUSED_H;
+    uint16_t* xm = norms ? (uint16_t*)(parts + (size_t)4 * rows * H) : x;  // the rows between a layer's halves: where none is read and written at once
     for (int l = 0; l < n_layers; ++l, w += 12) {
         auto at = [&](int i) { return (const uint16_t*)w[i]; };
-        auto ln = [&](int K, int i, int j) {  // x = LN(parts of a product over K + bias i + x) with norm j
-            return enc_parts_ln(enc_parts(K), parts, at(i), x, rows, (const float*)w[j], (const float*)w[j + 1], H, eps, st);
-        };
+        auto norm = [&](int i) { return (const float*)w[i]; };  // (of the layer before: - 12)
+        const int np1 = one ? enc_attn_parts(rows, heads) : enc_parts(H);
         int rc = 0;
-        MX_ACT_DISPATCH((rc = enc_gemm<F16, ENC_ACT>(x, at(0), at(1), qkv, rows, 3 * H, H, st)));
-        if (!rc) rc = mxk_attn_dense_ragged(qkv, 3 * H, qkv + H, 3 * H, qkv + 2 * H, 3 * H, attn, H, B, Smax, heads, H / heads, cu,
-                                            klen, scale, st);
-        if (!rc) MX_ACT_DISPATCH((rc = enc_gemm<F16, ENC_PART>(attn, at(2), nullptr, parts, rows, H, H, st)));
-        if (!rc) rc = ln(H, 3, 4);
-        if (!rc) MX_ACT_DISPATCH((rc = enc_gemm<F16, ENC_GELU>(x, at(6), at(7), up, rows, F, H, st)));
+        if (norms && l) {
+            MX_ACT_DISPATCH((rc = enc_ln_gemm<F16, ENC_ACT>(np, parts, at(-3), xm, norm(-2), norm(-1), eps, x, at(0), at(1), qkv, rows, 3 * H, H, st)));
+        } else {
+            MX_ACT_DISPATCH((rc = enc_gemm<F16, ENC_ACT>(x, at(0), at(1), qkv, rows, 3 * H, H, st)));
+        }
+        if (!rc && one) {
+            MX_ACT_DISPATCH((rc = enc_attn_gemm<F16>(qkv, klen, scale, heads, at(2), parts, rows, H, st)));
+        } else if (!rc) {
+            rc = mxk_attn_dense_ragged(qkv, 3 * H, qkv + H, 3 * H, qkv + 2 * H, 3 * H, attn, H, B, Smax, heads, H / heads, cu, klen, scale, st);
+            if (!rc) MX_ACT_DISPATCH((rc = enc_gemm<F16, ENC_PART>(attn, at(2), nullptr, parts, rows, H, H, st)));
+        }
+        if (!rc && norms) {
+            MX_ACT_DISPATCH((rc = enc_ln_gemm<F16, ENC_GELU>(np1, parts, at(3), x, norm(4), norm(5), eps, xm, at(6), at(7), up, rows, F, H, st)));
+        } else if (!rc) {
+            rc = enc_parts_ln(np1, parts, at(3), x, x, rows, norm(4), norm(5), H, eps, st);
+            if (!rc) MX_ACT_DISPATCH((rc = enc_gemm<F16, ENC_GELU>(x, at(6), at(7), up, rows, F, H, st)));
+        }
         if (!rc) MX_ACT_DISPATCH((rc = enc_gemm<F16, ENC_PART>(up, at(8), nullptr, parts, rows, H, F, st)));
-        if (!rc) rc = ln(F, 9, 10);
+        if (!rc && (!norms || l == n_layers - 1)) rc = enc_parts_ln(np, parts, at(9), xm, x, rows, norm(10), norm(11), H, eps, st);
         if (rc) return rc;
     }
     return 0;
@@ -441,7 +684,7 @@ extern "C" int mxk_enc_layers_tiled(const void* const* w, int n_layers, uint16_t
                 return rc ? rc : enc_add_ln(qkv, x, rows, g, b, H, eps, st);
             }
             const int rc = mx_dense16_enc(D16_PART, tile, a, K, at(i), rows, H, K, nullptr, nullptr, 0, np, parts, st);
-            return rc ? rc : enc_parts_ln(np, parts, at(i + 1), x, rows, g, b, H, eps, st);
+            return rc ? rc : enc_parts_ln(np, parts, at(i + 1), x, x, rows, g, b, H, eps, st);
         };
         int rc = mx_dense16_enc(D16_ACT, plan[0], x, H, at(0), rows, 3 * H, H, at(1), qkv, 3 * H, 1, nullptr, st);
         if (!rc) rc = mxk_attn_dense_ragged(qkv, 3 * H, qkv + H, 3 * H, qkv + 2 * H, 3 * H, attn, H, B, Smax, heads, H / heads, cu, klen, scale, st);

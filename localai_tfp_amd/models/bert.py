@@ -28,7 +28,7 @@ from ..ops.dense import encoder_plan
 from ..ops.linear import ACT_DTYPE
 
 # packed rows up to which encoder.hip's 16-column GEMMs run the layers. Whole embed calls, us, these / tiles (dense16_enc.hip): 768 x 3072, 12 layers, 19 / 64 /
-# 65 / 128 / 448 rows 436 / 519, 515 / 551, 587 / 563, 633 / 568, 1092 / 608; 1024 x 4096, 8 layers, 64 / 65 397 / 425, 455 / 422; 1536 x 6144 33 / 48 / 65 408 / 426,
+# 65 / 128 / 448 rows 371 / 519, 490 / 551, 587 / 563, 633 / 568, 1092 / 608; 1024 x 4096, 8 layers, 64 / 65 385 / 425, 455 / 422; 1536 x 6144 33 / 48 / 65 408 / 426,
 # 457 / 449, 529 / 412. Beyond, the library's GEMMs issued from Python and a pass for GELU before / tiles: 384 x 1536 600 / 3000 rows 1360 / 508, 1393 / 732; 768 x 3072
 # 600 / 1700 / 6428 / 12000 rows 1378 / 640, 1392 / 1036, 2450 / 2191, 4233 / 3602; 1024 x 4096 1000 / 6428 927 / 617, 2288 / 2232; 2048 x 8192, 4 layers, 100 /
 # 1700 / 12000 492 / 352, 1043 / 924, 5407 / 4938 (6428 rows 2769 / 2837).
@@ -233,7 +233,7 @@ class BertModel:
                     cfg.n_heads, Fd, scale, float(cfg.eps), qkv.data_ptr(), attn.data_ptr(), N.ptr(parts), up.data_ptr(), (ctypes.c_int * 6)(*plan), st)
             return x, cu_d, len_d
         if R <= small_rows(H, Fd):
-            parts = torch.empty(4, R, H, dtype=torch.float32, device=dev)  # fp32 sums of up to four parts of K
+            parts = torch.empty(5, R, H, dtype=torch.float32, device=dev)  # fp32 sums of up to four parts of K, and a norm's rows
             qkv, up = (torch.empty(R, n, dtype=self.dtype, device=dev) for n in (3 * H, Fd))
             N.kcall("mxk_enc_layers", (ctypes.c_void_p * (12 * cfg.n_layers))(*ptrs[5:]), cfg.n_layers, x.data_ptr(), R, B, S, cu_d.data_ptr(), len_d.data_ptr(), H,
                     cfg.n_heads, Fd, scale, float(cfg.eps), qkv.data_ptr(), attn.data_ptr(), parts.data_ptr(), up.data_ptr(), st)

@@ -206,6 +206,26 @@ def test_wide_one_call_layers(hidden, monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("hidden,heads,ffn", [(64, 1, 96), (512, 8, 2048), (576, 9, 2080), (1024, 16, 2048), (1024, 8, 160), (1088, 17, 96)])
+def test_few_rows_with_norms_and_attention_inside_the_products(hidden, heads, ffn, dtype, monkeypatch):
+    """Norms inside the products up to 16 rows, attention of one text up to 64: at the edges of the 16-row tiles and of the widths a lane
+    holds in one chunk or two, products in one part and in four, heads of 64 and of 128; 1088 columns beside them. The bound of test_packed_rows_match_fp32 (bf16:
+    eight times, its rounding)."""
+    cfg = BM.BertConfig(vocab=400, hidden=hidden, n_layers=3, n_heads=heads, ffn=ffn, max_pos=64, name="t")
+    get = BM.synthetic_bert(cfg, 5)
+    monkeypatch.setattr(BM, "ACT_DTYPE", dtype)
+    g, c = BM.BertModel.load(cfg, get, "cuda:0"), BM.BertModel.load(cfg, get, "cpu")
+    used = []
+    real = BM.N.kcall
+    monkeypatch.setattr(BM.N, "kcall", lambda name, *a: (used.append(name), real(name, *a))[1])
+    for lens in ([1], [0], [8], [9], [16], [17], [32], [33], [48], [49], [64], [3, 0, 12], [9, 8], [1] * 16):
+        ids = [list(range(10, 10 + n)) for n in lens]
+        got, want = g.embed(ids).cpu(), c.embed(ids)
+        assert "mxk_enc_layers" in used and (got - want).abs().max() < (5e-3 if dtype == torch.float16 else 4e-2), lens
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("pooling", ["mean", "cls", "last"])
 def test_empty_texts_match_the_padded_batch(pooling):
     """An empty text has a row too: nothing for the mean, its first row, or the batch's last position."""
