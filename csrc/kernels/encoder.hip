@@ -42,20 +42,6 @@ struct LnGain {
     }
 };
 
-// Sum over the wave, in every lane, without LDS: with __shfl_xor's six permutations through LDS each of a row's two sums took 0.6 us.
-template <int CTRL>
-MX_DEV float dpp_add(float v) { return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true)); }
-MX_DEV float row_sum(float v) {
-    v = dpp_add<0xB1>(v);   // lanes 1 0 3 2 of a quad
-    v = dpp_add<0x4E>(v);   // 2 3 0 1
-    v = dpp_add<0x141>(v);  // mirrored in 8 lanes
-    v = dpp_add<0x140>(v);  // in 16
-    u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false));
-    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-    r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false));
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
 // LayerNorm of one row. Two passes over registers: the variance is a sum of squares about the mean.
 template <int NC, bool F16>
 MX_DEV void ln_row(float (&v)[NC][8], int H, const LnGain<NC>& gb, float eps, uint16_t* __restrict__ out, int lane) {
@@ -64,7 +50,7 @@ MX_DEV void ln_row(float (&v)[NC][8], int H, const LnGain<NC>& gb, float eps, ui
     for (int j = 0; j < NC; ++j)
 #pragma unroll
         for (int e = 0; e < 8; ++e) s += v[j][e];
-    const float mean = row_sum(s) / H;
+    const float mean = wave_sum_all(s) / H;
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
@@ -73,7 +59,7 @@ MX_DEV void ln_row(float (&v)[NC][8], int H, const LnGain<NC>& gb, float eps, ui
         for (int e = 0; e < 8; ++e) q += (v[j][e] - mean) * (v[j][e] - mean);
         ss += enc_has(j, H, lane) ? q : 0.f;
     }
-    const float rs = rsqrtf(row_sum(ss) / H + eps);
+    const float rs = rsqrtf(wave_sum_all(ss) / H + eps);
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
         float y[8];

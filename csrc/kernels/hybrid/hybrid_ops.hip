@@ -30,7 +30,7 @@ MX_DEV float softplus_acc(float x) { return x > 30.f ? x : log1pf(expf(x)); }
 
 // sum over the threads of a block of blockDim.x = 64 * k threads (k <= 16), returned to every thread
 MX_DEV float block_sum_dyn(float v, float* red) {
-    v = wave_sum(v);
+    v = wave_sum_all(v);
     const int nw = blockDim.x >> 6;
     if (nw == 1) return v;
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;

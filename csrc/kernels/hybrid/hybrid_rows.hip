@@ -178,7 +178,7 @@ __global__ __launch_bounds__(1024) void row_rope_append_kernel(RowRope a, int bq
         if (cached) ss = load(0, true);
         else
             for (int base = 0; base < n_items; base += stride) ss += load(base, false);
-        ss = wave_sum(ss);
+        ss = wave_sum_all(ss);
         if ((tid & 63) == 0) red[tid >> 6] = ss;
     } else {
         load(part * stride, true);  // requested before the wait for the angles

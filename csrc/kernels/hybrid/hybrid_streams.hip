@@ -29,7 +29,7 @@ MX_DEV float ld_e(const void* p, long i) {
 
 // sum over the threads of a block of blockDim.x = 64 * k threads (k <= 16), returned to every thread
 MX_DEV float block_sum_any(float v, float* red) {
-    v = wave_sum(v);
+    v = wave_sum_all(v);
     const int nw = blockDim.x >> 6;
     __syncthreads();  // red may still be read from an earlier call
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;

@@ -345,7 +345,7 @@ __global__ __launch_bounds__(64 * QMV_WAVES) void qmv_kernel(const int8_t* __res
                     const float4 v = *(const float4*)(xr + c);
                     ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
                 }
-                ss = wave_sum(ss);
+                ss = wave_sum_all(ss);
                 if (lane == 0) nred[m][wave] = ss;
             }
             // 8 consecutive elements per lane, 4 lanes per 32-element q8 block (klen % 256 == 0, so the
@@ -546,7 +546,7 @@ __device__ __forceinline__ void qmv1_columns(int g, const uint8_t* __restrict__ 
                       v1.w * v1.w;
             }
         }
-        ss = wave_sum(ss);
+        ss = wave_sum_all(ss);
         if (lane == 0) nred[wave] = ss;
     }
 #pragma unroll
