@@ -117,15 +117,26 @@ template <int CTRL>
 MX_DEV float dpp_add(float v) {
     return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
 }
-MX_DEV float wave_sum_all(float v) {
-    v = dpp_add<0xB1>(v);   // lanes 1 0 3 2 of a quad
-    v = dpp_add<0x4E>(v);   // 2 3 0 1
-    v = dpp_add<0x141>(v);  // mirrored in 8 lanes
-    v = dpp_add<0x140>(v);  // in 16
-    u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false));
+MX_DEV float wave_sum_all(float v) {  // (wave_sum's pairs in wave_sum's order: the same bits)
+    u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false));
     v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false));
+    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    v = dpp_add<0x128>(v);  // rotated by 8 in 16 lanes
+    v = dpp_add<0x124>(v);  // by 4: the two halves of 8 are alike by now
+    v = dpp_add<0x4E>(v);   // lanes 2 3 0 1 of a quad
+    return dpp_add<0xB1>(v);  // 1 0 3 2
+}
+template <int CTRL>
+MX_DEV float dpp_max(float v) {
+    return fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true)));
+}
+MX_DEV float wave_max_all(float v) {  // all 64 lanes active
+    v = dpp_max<0x140>(dpp_max<0x141>(dpp_max<0x4E>(dpp_max<0xB1>(v))));
+    u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false));
+    v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
     r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false));
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 MX_DEV float wave_max(float v) {
 #pragma unroll

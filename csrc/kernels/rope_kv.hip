@@ -155,7 +155,11 @@ __global__ __launch_bounds__(256) void rope_kv4_kernel(float* __restrict__ qkv, 
         a0 = ld4(h * D + 4 * u);
         if constexpr (NEOX) b0 = ld4(h * D + 4 * u + HALF);
     }
-    const int p = pos[t];
+    const int vi = v_lo * (D / 4) + threadIdx.x;
+    float4 v0 = {0.f, 0.f, 0.f, 0.f};
+    if (vi < v_hi * (D / 4)) v0 = *(const float4*)(row + (Hq + Hkv) * D + 4 * vi);
+    const int p = pos[t], slot = slots[t];  // (behind the barrier the slot and the values were waits of their own)
+    const int blk = slot >= 0 ? slot / block_size : 0, off = slot >= 0 ? slot % block_size : 0;
     for (int i = threadIdx.x; i < HALF; i += 256) {
         float sv, cv;
         sincosf((float)p * inv_freq[i], &sv, &cv);
@@ -163,8 +167,6 @@ __global__ __launch_bounds__(256) void rope_kv4_kernel(float* __restrict__ qkv, 
         sn[i] = sv * attn_factor;
     }
     __syncthreads();
-    const int slot = slots[t];
-    const int blk = slot >= 0 ? slot / block_size : 0, off = slot >= 0 ? slot % block_size : 0;
     auto put = [&](void* pool, int kh, int d, float4 y) {
         const size_t r = ((size_t)blk * Hkv + kh) * block_size + off;
         if constexpr (KVF == KVF_Q8_0) {
@@ -241,10 +243,10 @@ __global__ __launch_bounds__(256) void rope_kv4_kernel(float* __restrict__ qkv, 
         }
     }
     float* vr = row + (Hq + Hkv) * D;
-    for (int idx = v_lo * (D / 4) + threadIdx.x; idx < v_hi * (D / 4); idx += 256) {
+    for (int idx = vi; idx < v_hi * (D / 4); idx += 256) {
         const int kh = idx / (D / 4), d = (idx % (D / 4)) * 4;
         if (slot >= 0) {
-            float4 v = *(const float4*)(vr + kh * D + d);
+            float4 v = idx == vi ? v0 : *(const float4*)(vr + kh * D + d);
             if (HAS_BIAS) {
                 const float4 b = *(const float4*)(bias + (Hq + Hkv) * D + kh * D + d);
                 v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w;

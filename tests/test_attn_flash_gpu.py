@@ -244,3 +244,17 @@ def test_decode_reads_nothing_behind_a_context(fmt, Hq, Hkv, D, window, softcap)
         K.attn_decode(q[rows].cuda(), kd, vd, bt[rows].contiguous().cuda(), ctx[rows].cuda(), D ** -0.5, out, part_size=part, window=window, softcap=softcap)
         # as for prompts: probabilities and outputs are rounded to 16 bits once each
         assert float((out.cpu().float() - want[rows]).norm() / want[rows].norm()) < 4 * 2 ** -9, part
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_decode_merges_any_number_of_partitions(D):
+    """One more, as many and fewer than a group of the merge's threads asks for ahead (four each of 16, 8 or 4 groups), and more than have
+    their weights in LDS."""
+    parts = [1, 2, 3, 15, 16, 17, 31, 32, 33, 63, 64, 65, 511, 512, 520]
+    q, kc, vc, bt, _, ctx = _case(4, 2, D, [1] * len(parts), [32 * n - 1 - n % 3 for n in parts])
+    want = torch.stack([K._attn_ref_one(q[i:i + 1], kc, vc, bt[i], int(c), int(c) - 1, D ** -0.5, 16)[0] for i, c in enumerate(ctx)])
+    out = torch.full(q.shape, float("nan"), dtype=torch.float16, device="cuda")
+    K.attn_decode(q.cuda(), kc.cuda(), vc.cuda(), bt.cuda(), ctx.cuda(), D ** -0.5, out, part_size=32)
+    # as for prompts: probabilities and outputs are rounded to 16 bits once each
+    assert float((out.cpu().float() - want).norm() / want.norm()) < 4 * 2 ** -9
