@@ -202,14 +202,11 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_flash_kernel(co
         }
     };
     auto look_up = [&](int t) {                  // before tile t's rows, tiles in turn from t0
-        if constexpr (UNI) {
-            if ((t - t0) % GT) return;
-            const int key = lane_key(t), bi = page_of(key);
-            place = (uint32_t)(next * Hkv + kvh) * (uint32_t)(bs / RPW) + (uint32_t)((key - bi * bs) / RPW);
-            next = bt[page_of(lane_key(t + GT))];
-        } else {
-            find_rows(t);
-        }
+        if constexpr (!UNI) return;
+        if ((t - t0) % GT) return;
+        const int key = lane_key(t), bi = page_of(key);
+        place = (uint32_t)(next * Hkv + kvh) * (uint32_t)(bs / RPW) + (uint32_t)((key - bi * bs) / RPW);
+        next = bt[page_of(lane_key(t + GT))];
     };
     auto load_chunk = [&](int t, int j) {
         if constexpr (UNI) {
@@ -279,8 +276,10 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_flash_kernel(co
     if (t0 < t1) {
         if constexpr (UNI) next = bt[page_of(lane_key(t0))];
         look_up(t0);
+        find_rows(t0);
 #pragma unroll
         for (int j = 0; j < NCH; ++j) load_chunk(t0, j);
+        find_rows(min(t0 + 1, t1 - 1));
 #pragma unroll
         for (int j = 0; j < NCH; ++j) {
             store_k(t0 & 1, j);
@@ -289,11 +288,13 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_flash_kernel(co
         if (t0 + 1 < t1) look_up(t0 + 1);
 #pragma unroll
         for (int j = 0; j < NCH; ++j) load_chunk(min(t0 + 1, t1 - 1), j);
+        find_rows(min(t0 + 2, t1 - 1));
         __syncthreads();
         for (int t = t0; t < t1; ++t) {
             // the other buffer was last read while tile t - 1 was worked on, before the barrier that ended that round
             if (t + 2 < t1) look_up(t + 2);
             work(t);
+            find_rows(min(t + 3, t1 - 1));
             __syncthreads();
         }
     }
