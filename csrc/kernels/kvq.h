@@ -13,9 +13,13 @@
 
 enum { KVF_BF16 = 0, KVF_FP8 = 1, KVF_Q8_0 = 2, KVF_Q4_0 = 3, KVF_Q4_1 = 4, KVF_Q5_0 = 5, KVF_Q5_1 = 6, KVF_IQ4_NL = 7 };
 
-__device__ __constant__ static const float kvq_iq4nl_values[16] = {-127.f, -104.f, -83.f, -65.f, -49.f, -35.f, -22.f,
-                                                                   -10.f,  1.f,    13.f,  25.f,  38.f,  53.f,  69.f,
-                                                                   89.f,   113.f};
+// The values of four iq4_nl codes, one a byte of x, as signed bytes: -127 -104 -83 -65 | -49 -35 -22 -10 | 1 13 25 38 | 53 69 89 113, picked
+// by byte permutations. (A table in memory was a load an element: attention of a 2000-token prompt over such a cache 92 us, 72 so.)
+MX_DEV uint32_t kvq_iq4nl4(uint32_t x) {
+    const uint32_t sel = x & 0x07070707u, y = x & 0x08080808u, up = (y << 5) - (y >> 3);  // up: 0xFF where the code is 8 or more
+    const uint32_t lo = __builtin_amdgcn_perm(0xF6EADDCFu, 0xBFAD9881u, sel), hi = __builtin_amdgcn_perm(0x71594535u, 0x26190D01u, sel);
+    return (hi & up) | (lo & ~up);
+}
 
 template <int KVF, int D>
 struct KVQ {
@@ -65,6 +69,10 @@ MX_DEV void kvq_dequant(const KVQRaw& w, float (&f)[8]) {
             const uint32_t word = i < 4 ? w.c.x : w.c.y;
             f[i] = d * (float)(int8_t)((word >> (8 * (i & 3))) & 0xFF);
         }
+    } else if constexpr (KVF == KVF_IQ4_NL) {
+        const uint32_t even = kvq_iq4nl4(w.c.x & 0x0F0F0F0Fu), odd = kvq_iq4nl4((w.c.x >> 4) & 0x0F0F0F0Fu);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) f[i] = d * (float)(int8_t)(((i & 1 ? odd : even) >> (8 * (i >> 1))) & 0xFF);
     } else {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -72,7 +80,6 @@ MX_DEV void kvq_dequant(const KVQRaw& w, float (&f)[8]) {
             if constexpr (KVF == KVF_Q5_0 || KVF == KVF_Q5_1) q |= (int)((w.hb >> i) & 1u) << 4;
             if constexpr (KVF == KVF_Q4_0) f[i] = d * (float)(q - 8);
             else if constexpr (KVF == KVF_Q5_0) f[i] = d * (float)(q - 16);
-            else if constexpr (KVF == KVF_IQ4_NL) f[i] = d * kvq_iq4nl_values[q];
             else f[i] = fmaf(d, (float)q, m);  // q4_1 / q5_1
         }
     }

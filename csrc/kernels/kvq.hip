@@ -10,6 +10,9 @@
 
 namespace {
 
+__device__ __constant__ const float kvq_iq4nl_values[16] = {-127.f, -104.f, -83.f, -65.f, -49.f, -35.f, -22.f, -10.f,
+                                                            1.f,    13.f,   25.f,  38.f,  53.f,  69.f,  89.f,  113.f};
+
 MX_DEV int iq4nl_best(float x) {
     const float* v = kvq_iq4nl_values;
     if (x <= v[0]) return 0;
