@@ -201,7 +201,8 @@ constexpr int DEC_RED_MAXP = 512;  // partitions whose merge weights fit the red
 // merge weights through LDS; then groups of D / 4 threads take every n-th partition, four dims a thread and four partitions in
 // flight, and their sums meet in LDS. A chain of memory latencies bounds it: 9 contexts of 3001-24001 in 256-key partitions 9.9 us
 // with one group of D threads, 5.7 with eight of 32; the first four partitions of a group are asked for ahead of the weights
-// (attention and merge of one context of 711 in 48-key partitions 8.65 -> 8.0 us, of 32 of 97-3879 in 128-key ones 48.6 -> 47.7).
+// (attention and merge of one context of 711 in 48-key partitions 8.65 -> 8.0 us, of 32 of 97-3879 in 128-key ones 48.9
+// -> 47.8, of 192 of 300-491 in 256-key ones, head dim 64, 37.6 -> 35.6).
 template <bool F16>
 __global__ __launch_bounds__(256) void attn_decode_reduce_kernel(const float2* __restrict__ part_ml,
                                                                   const float* __restrict__ part_o, int n_parts,
@@ -218,11 +219,13 @@ __global__ __launch_bounds__(256) void attn_decode_reduce_kernel(const float2* _
     const size_t pb = (size_t)bh * n_parts;
     const int nq = D / 4, groups = 256 / nq, grp = threadIdx.x / nq, d = threadIdx.x % nq * 4;  // (D 64, 128 or 256)
     auto at = [&](int p) { return *(const float4*)(part_o + (pb + p) * D + d); };
-    float4 o[4];
+    float2 ml0 = make_float2(-INFINITY, 0.f);
+    if (threadIdx.x < 64) ml0 = part_ml[pb + min((int)threadIdx.x, np - 1)];
+    float4 o[4] = {};
 #pragma unroll
-    for (int u = 0; u < 4; ++u) o[u] = at(min(grp + u * groups, np - 1));
+    for (int u = 0; u < 4; ++u)
+        if (grp + u * groups < np) o[u] = at(grp + u * groups);
     if (threadIdx.x < 64) {
-        const float2 ml0 = part_ml[pb + min((int)threadIdx.x, np - 1)];
         float m = ml0.x;
         for (int p = threadIdx.x + 64; p < np; p += 64) m = fmaxf(m, part_ml[pb + p].x);
         m = wave_max_all(m);
