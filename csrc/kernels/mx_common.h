@@ -112,7 +112,7 @@ MX_DEV float wave_sum(float v) {
     return v;
 }
 // The same with all 64 lanes active, without LDS: wave_sum is a chain of six permutations through it, 0.3 us longer, which a kernel
-// that waits for its sum does not hide (norms of rows one after another, two sums each: 1.5 us a row, 0.9 with this).
+// that waits for its sum does not hide (LayerNorm of 19 rows after four parts of a product, two sums: 5.0 -> 4.1 us in a profile).
 template <int CTRL>
 MX_DEV float dpp_add(float v) {
     return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
