@@ -41,7 +41,8 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* __restrict__ 
             v[i].w += __uint_as_float(r[i].y & 0xFFFF0000u);
             *(float4*)(xout + (size_t)row * ldx + (i * 256 + threadIdx.x) * 4) = v[i];
         }
-        ss += v[i].x * v[i].x + v[i].y * v[i].y + v[i].z * v[i].z + v[i].w * v[i].w;
+        // (which of the squares is rounded by itself is written out: left to the compiler it is another one for another width)
+        ss += fmaf(v[i].w, v[i].w, fmaf(v[i].z, v[i].z, fmaf(v[i].x, v[i].x, v[i].y * v[i].y)));
     }
     ss = block_sum<256>(ss, red);
     const float rs = rsqrtf(ss / (float)H + eps);

@@ -27,3 +27,19 @@ def test_each_width_in_whole_chunks(chunks, rows, res, dtype):
     b = want.view(rows, -1, 32)
     d = b.abs().amax(-1, keepdim=True) / 127
     assert ((q8[0].cpu().view(rows, -1, 32) * q8[1].cpu()[..., :1].double() - b).abs() <= d * 0.501 + 1e-6).all()  # half a step
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("narrow", [1024, 2048])
+def test_a_width_does_not_choose_the_rounding(narrow):
+    """Rows of 1024 n numbers and the same rows with zeros up to four times the width, eps a quarter: a quarter of the mean square, the
+    square root of it halved, both without rounding, so all outputs are doubled bit for bit."""
+    g = torch.Generator().manual_seed(narrow)
+    x, w = torch.randn(700, 4 * narrow, generator=g).cuda(), (torch.rand(4 * narrow, generator=g) + 0.5).cuda()
+    x[:, narrow:] = 0
+    out = [torch.empty(700, H, dtype=torch.float16, device="cuda") for H in (narrow, 4 * narrow)]
+    K.rmsnorm(x[:, :narrow].contiguous(), w[:narrow].contiguous(), 2.0 ** -16, out_bf16=out[0])
+    K.rmsnorm(x, w, 2.0 ** -18, out_bf16=out[1])
+    a, b = out[0].float(), out[1][:, :narrow].float()
+    normal = a.abs() >= 2.0 ** -14  # (smaller ones have fewer bits)
+    assert torch.equal(2 * a[normal], b[normal]) and normal.float().mean() > 0.99
