@@ -654,8 +654,8 @@ extern "C" int mxk_enc_layers(const void* const* w, int n_layers, uint16_t* x, i
 }
 
 // The same layers by dense16.hip's tiles. plan: tile of the qkv product; tile and parts of K of the output product; tile of the up product; tile and
-// parts of the down product (parts 1, 2, 3, 4 or 8; with 1 the product is stored in 16 bits with its bias, as `up`'s input is). H and F multiples
-// of 64; parts [most parts][rows][H] where there are any.
+// parts of the down product: 1, 2, 3, 4 or 8 parts of fp32 sums, or 0: stored in 16 bits with its bias. H and F multiples of 64; parts
+// [most parts][rows][H] where there are any.
 extern "C" int mxk_enc_layers_tiled(const void* const* w, int n_layers, uint16_t* x, int rows, int B, int Smax, const int* cu, const int* klen, int H,
                                     int heads, int F, float scale, float eps, uint16_t* qkv, uint16_t* attn, float* parts, uint16_t* up,
                                     const int* plan, hipStream_t st) {
@@ -665,7 +665,7 @@ extern "C" int mxk_enc_layers_tiled(const void* const* w, int n_layers, uint16_t
         auto at = [&](int i) { return (const uint16_t*)w[i]; };
         auto add_ln = [&](const uint16_t* a, int K, int tile, int np, int i) {  // x = LN(a W^T + bias + x): weights i, bias i + 1, norm i + 2
             const float *g = (const float*)w[i + 2], *b = (const float*)w[i + 3];
-            if (np == 1) {  // (the q|k|v rows are read by now)
+            if (np == 0) {  // (the q|k|v rows are read by now)
                 const int rc = mx_dense16_enc(D16_ACT, tile, a, K, at(i), rows, H, K, at(i + 1), qkv, H, 1, nullptr, st);
                 return rc ? rc : enc_add_ln(qkv, x, rows, g, b, H, eps, st);
             }

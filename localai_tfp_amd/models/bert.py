@@ -24,7 +24,7 @@ import torch.nn.functional as F
 
 from .. import _native as N
 from ..ops import core as K
-from ..ops.dense import encoder_plan
+from ..ops.dense import ENC_SMALL_ROWS, encoder_plan, small_rows  # noqa: F401
 from ..ops.linear import ACT_DTYPE
 
 # packed rows up to which encoder.hip's 16-column GEMMs run the layers. Whole embed calls, us, these / tiles (dense16_enc.hip): 768 x 3072, 12 layers, 19 / 64 /
@@ -33,20 +33,6 @@ from ..ops.linear import ACT_DTYPE
 # 600 / 1700 / 6428 / 12000 rows 1378 / 640, 1392 / 1036, 2450 / 2191, 4233 / 3602; 1024 x 4096 1000 / 6428 927 / 617, 2288 / 2232; 2048 x 8192, 4 layers, 100 /
 # 1700 / 12000 492 / 352, 1043 / 924, 5407 / 4938 (6428 rows 2769 / 2837).
 ENC_FEW_ROWS = 64
-ENC_SMALL_ROWS = 448  # where tiles do not take the widths
-
-
-def small_rows(hidden: int, ffn: int) -> int:
-    """Packed rows up to which the layers run on encoder.hip's 16-column GEMMs rather than the library's (they read a layer's weights once
-    per 64 rows, so rows x weights decide; beyond 64 M weights a layer the library's tiles win at any row count).
-
-    Whole embed calls, us, one call / library GEMMs issued from Python (110 us a layer at least): 384 x 1536, 12 layers, 448 rows
-    679 / 1433; 768 x 3072, 12 layers, 64 rows 657 / 1374, 384 1161 / 1363, 512 1275 / 1356, 640 1488 / 1354; 1024 x 4096, 24
-    layers, 64 rows 1428 / 2631, 256 2263 / 2605, 320 2857 / 2624; 1280 x 5120, 8 layers, 128 rows 828 / 910, 192 940 / 906; 1536 x
-    6144, 8 layers, 96 rows 813 / 958, 128 994 / 952; 2048 x 8192, 8 layers, 48 rows 899 / 963, 128 1388 / 947; 3072 x 12288, 4
-    layers, 16 rows 596 / 534, 256 2320 / 883."""
-    weights = 4 * hidden * hidden + 2 * hidden * ffn
-    return min(ENC_SMALL_ROWS, 3_200_000_000 // weights) if weights <= 64_000_000 else 0
 
 
 @dataclass
@@ -225,10 +211,11 @@ class BertModel:
         N.kcall("mxk_enc_embed", img.data_ptr(), R, *ptrs[:5], H, float(cfg.eps), x.data_ptr(), st)
         scale = 1.0 / math.sqrt(H // cfg.n_heads)
         if H % 64 == 0 and Fd % 64 == 0 and (R > ENC_FEW_ROWS or R > small_rows(H, Fd)):
-            plan = encoder_plan(R, H, Fd)
+            plan, keep = encoder_plan(R, H, Fd), R <= small_rows(H, Fd)
+            plan = [n if i not in (2, 5) or n > 1 or keep else 0 for i, n in enumerate(plan)]  # 0 parts: 16-bit sums
             most = max(plan[2], plan[5])
-            parts = torch.empty(most, R, H, dtype=torch.float32, device=dev) if most > 1 else None
             qkv, up = (torch.empty(R, n, dtype=self.dtype, device=dev) for n in (3 * H, Fd))
+            parts = torch.empty(most, R, H, dtype=torch.float32, device=dev) if most else None
             N.kcall("mxk_enc_layers_tiled", (ctypes.c_void_p * (12 * cfg.n_layers))(*ptrs[5:]), cfg.n_layers, x.data_ptr(), R, B, S, cu_d.data_ptr(), len_d.data_ptr(), H,
                     cfg.n_heads, Fd, scale, float(cfg.eps), qkv.data_ptr(), attn.data_ptr(), N.ptr(parts), up.data_ptr(), (ctypes.c_int * 6)(*plan), st)
             return x, cu_d, len_d

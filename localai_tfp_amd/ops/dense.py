@@ -143,17 +143,36 @@ def _enc_tile(M: int, N_: int, K: int, kind: int, parts: int = 1):
     return best
 
 
+ENC_SMALL_ROWS = 448  # where tiles do not take the widths
+
+
+def small_rows(hidden: int, ffn: int) -> int:
+    """Packed rows up to which the layers run on encoder.hip's 16-column GEMMs rather than the library's (they read a layer's weights once
+    per 64 rows, so rows x weights decide; beyond 64 M weights a layer the library's tiles win at any row count).
+
+    Whole embed calls, us, one call / library GEMMs issued from Python (110 us a layer at least): 384 x 1536, 12 layers, 448 rows
+    679 / 1433; 768 x 3072, 12 layers, 64 rows 657 / 1374, 384 1161 / 1363, 512 1275 / 1356, 640 1488 / 1354; 1024 x 4096, 24
+    layers, 64 rows 1428 / 2631, 256 2263 / 2605, 320 2857 / 2624; 1280 x 5120, 8 layers, 128 rows 828 / 910, 192 940 / 906; 1536 x
+    6144, 8 layers, 96 rows 813 / 958, 128 994 / 952; 2048 x 8192, 8 layers, 48 rows 899 / 963, 128 1388 / 947; 3072 x 12288, 4
+    layers, 16 rows 596 / 534, 256 2320 / 883."""
+    weights = 4 * hidden * hidden + 2 * hidden * ffn
+    return min(ENC_SMALL_ROWS, 3_200_000_000 // weights) if weights <= 64_000_000 else 0
+
+
 @functools.lru_cache(maxsize=1024)
 def encoder_plan(M: int, H: int, Fn: int) -> tuple:
     """Tiles (and parts of K) of an encoder layer's q|k|v, output, up and down products for M rows, as encoder.hip takes them. Parts that the
-    LayerNorm adds up cost it 4 bytes a number each, the 16-bit sums of an undivided product 2."""
+    LayerNorm adds up cost it 4 bytes a number each, an undivided product's sums 2 bytes where the library rounded them to 16 bits too; up to
+    `small_rows` they are one fp32 part, as the 16-column GEMMs had them."""
+    kind = 2 if M <= small_rows(H, Fn) else 0
+
     def narrow(K):
         best = None
         for parts in (1, 2, 3, 4, 8):
             if parts > K // 64 or parts > 1 and M * H * parts > 1 << 25:
                 break
-            us, tile = _enc_tile(M, H, K, 2 if parts > 1 else 0, parts)
-            us += M * H * (4 * parts if parts > 1 else 2) / 4e6
+            us, tile = _enc_tile(M, H, K, 2 if parts > 1 else kind, parts)
+            us += M * H * (4 * parts if parts > 1 or kind else 2) / 4e6
             if best is None or us < best[0]:
                 best = us, (tile, parts)
         return best[1]

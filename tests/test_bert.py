@@ -269,6 +269,26 @@ def test_tiled_layers_match_fp32(tile, dtype, monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("hidden,rows", [(64, 65), (128, 300), (384, 448), (512, 200), (640, 300), (768, 400), (832, 350)])
+def test_sums_stay_in_fp32_until_the_norm(hidden, rows):
+    """Biases of 1000, which the norms take away again: an f16 there has steps of 0.5, fp32 of 6e-5, beside rows of order 1. Up to small_rows
+    the bound of test_wide_one_call_layers holds all the same; the smallest widths have undivided products throughout."""
+    cfg = BM.BertConfig(vocab=400, hidden=hidden, n_layers=2, n_heads=hidden // 64, ffn=4 * hidden, max_pos=300, name="t")
+    src = BM.synthetic_bert(cfg, 5)
+
+    def get(name):
+        t = src(name)
+        return t + 1000 if t is not None and name in [f"blk.{i}.{b}.bias" for i in (0, 1) for b in ("attn_output", "ffn_down")] else t
+    g, c = BM.BertModel.load(cfg, get, "cuda:0"), BM.BertModel.load(cfg, get, "cpu")
+    assert rows <= BM.small_rows(hidden, 4 * hidden) and float(c.w["blk.0.ffn_down.bias"].float().mean()) > 900
+    ids = [list(range(10, 10 + n)) for n in (rows // 2, rows - rows // 2)]
+    hid, n = g.encode(ids)
+    want, _ = c.encode(ids)
+    for i, k in enumerate(n.tolist()):
+        assert (hid[i, :k].cpu() - want[i, :k]).abs().max() < 5e-2
+
+
+@pytest.mark.gpu
 def test_gelu_rounds_like_64_bits():
     """Every finite f16: within a unit of the last place, and the nearest f16 for all but one in a thousand (fp32 arithmetic near the
     middle of two). Infinities and NaN as 0.5 x (1 + erf(x / sqrt 2)) has them."""
