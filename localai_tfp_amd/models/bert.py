@@ -215,7 +215,11 @@ class BertModel:
             plan = [n if i not in (2, 5) or n > 1 or keep else 0 for i, n in enumerate(plan)]  # 0 parts: 16-bit sums
             most = max(plan[2], plan[5])
             qkv, up = (torch.empty(R, n, dtype=self.dtype, device=dev) for n in (3 * H, Fd))
-            parts = torch.empty(most, R, H, dtype=torch.float32, device=dev) if most else None
+            try:
+                parts = torch.empty(most, R, H, dtype=torch.float32, device=dev) if most else None
+            except torch.cuda.OutOfMemoryError:  # (up to 128 MB; undivided products need one part or none)
+                plan[2] = plan[5] = int(keep)
+                parts = torch.empty(R, H, dtype=torch.float32, device=dev) if keep else None
             N.kcall("mxk_enc_layers_tiled", (ctypes.c_void_p * (12 * cfg.n_layers))(*ptrs[5:]), cfg.n_layers, x.data_ptr(), R, B, S, cu_d.data_ptr(), len_d.data_ptr(), H,
                     cfg.n_heads, Fd, scale, float(cfg.eps), qkv.data_ptr(), attn.data_ptr(), N.ptr(parts), up.data_ptr(), (ctypes.c_int * 6)(*plan), st)
             return x, cu_d, len_d

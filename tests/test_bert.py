@@ -289,6 +289,30 @@ def test_sums_stay_in_fp32_until_the_norm(hidden, rows):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("small", [448, 0])
+def test_parts_that_do_not_fit_are_done_without(small, monkeypatch):
+    """No room for a product's parts (refused here from the host): undivided products, in one fp32 part up to small_rows, else with
+    16-bit sums. The bound of test_packed_rows_match_fp32."""
+    cfg = BM.BertConfig(vocab=400, hidden=192, n_layers=2, n_heads=3, ffn=576, max_pos=300, name="t")
+    get = BM.synthetic_bert(cfg, 5)
+    g, c = BM.BertModel.load(cfg, get, "cuda:0"), BM.BertModel.load(cfg, get, "cpu")
+    monkeypatch.setattr(BM, "small_rows", lambda H, F: small)
+    monkeypatch.setattr(BM, "encoder_plan", lambda R, H, F: (36, 68, 3, 36, 40, 8))
+    ids = [list(range(10, 10 + n)) for n in (200, 57)]
+    want, refused, real = c.embed(ids), [], torch.empty
+
+    def empty(*a, **k):
+        if k.get("dtype") == torch.float32 and len(a) == 3 and a[0] > 1:
+            refused.append(a)
+            raise torch.cuda.OutOfMemoryError("no room")
+        return real(*a, **k)
+    monkeypatch.setattr(torch, "empty", empty)
+    got = g.embed(ids)
+    monkeypatch.setattr(torch, "empty", real)
+    assert refused == [(8, 257, 192)] and (got.cpu() - want).abs().max() < 5e-3
+
+
+@pytest.mark.gpu
 def test_gelu_rounds_like_64_bits():
     """Every finite f16: within a unit of the last place, and the nearest f16 for all but one in a thousand (fp32 arithmetic near the
     middle of two). Infinities and NaN as 0.5 x (1 + erf(x / sqrt 2)) has them."""
