@@ -400,6 +400,43 @@ def test_prompt_portions_and_decoding(dev, dt, tol, shape):
     assert eng.bm.num_free == eng.bm.num_blocks - 1 and len(eng.state_slots.free) == 4
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("ff,cuts", [(2816, [75]), (16384, [40, 1, 33, 1])])
+def test_gated_units_in_the_input_product(ff, cuts, monkeypatch):
+    """Layers wide enough for the input product's gated columns (beyond 64 rows, and below by more weights): every call's columns against 64
+    bits, and the logits against the oracle and the same steps with the gated unit in a launch of its own. A column's fp32 sum of 1024
+    products is within 1024 x 2^-24 of their magnitudes; the unit's slopes are at most 1.1 and 1 times the other factor, and its result is
+    rounded to bf16, 2^-8 at most."""
+    from localai_tfp_amd.ops import dense as D
+    cfg, tensors, model = build("cuda", "bfloat16", seed=4, hidden=1024, vocab=97, pattern=("parallel", "mamba2"), mlps=("dense",), heads=4, kv_heads=2, dim=64,
+                                vdim=64, chunk=24, d_heads=4, d_kv_heads=2, d_dim=32, d_vdim=32, m_heads=4, m_vdim=32, m_state=32, m_groups=2, m_norm_groups=2, ff=ff)
+    t = toks(sum(cuts), cfg.vocab, 5)
+    want = oracle(cfg, tensors, t)
+    done, real = [], D.Dense.gated
+
+    def gated(self, x, out, gate, up, gate_b, up_b, gout):
+        ok = real(self, x, out, gate, up, gate_b, up_b, gout)
+        done.append(ok)
+        if ok:
+            F, xd, wd = gout.shape[1], x.double(), self.w.double()
+            y, mag = xd @ wd.t(), 1026 * 2 ** -24 * (xd.abs() @ wd.abs().t())
+            n = out.shape[1]
+            assert n == gate and up == gate + F and ((out.double() - y[:, :n]).abs() <= mag[:, :n]).all()
+            g, u = y[:, gate:gate + F] + gate_b.double(), y[:, up:up + F] + up_b.double()
+            dg, du = mag[:, gate:gate + F], mag[:, up:up + F]
+            h = g * torch.sigmoid(g) * u
+            assert ((gout.double() - h).abs() <= 1.1 * dg * u.abs() + du * g.abs() + dg * du + (2 ** -8 + 2 ** -20) * h.abs() + 1e-30).all()
+        return ok
+    monkeypatch.setattr(D.Dense, "gated", gated)
+    got = run_cuts(engine(model, 96), "a", t, cuts)
+    assert done == [True] * (2 * len(cuts))
+    monkeypatch.setattr(D, "takes_gated16", lambda *a: False)
+    apart = run_cuts(engine(model, 96), "b", t, cuts)
+    assert done[2 * len(cuts):] == [False] * (2 * len(cuts))
+    close(got, want, 3e-2, True)
+    close(got, apart, 3e-2, True)
+
+
 @pytest.mark.parametrize("dev,dt,tol", RUNS)
 def test_recurrent_layers_only(dev, dt, tol):
     """A model without any attention layer: the paged pool is empty, blocks are bookkeeping only (the engine sizes
