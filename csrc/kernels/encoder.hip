@@ -493,12 +493,12 @@ int enc_ln_gemm(int np, const float* parts, const uint16_t* pbias, const uint16_
 #define ELN(RW_)                             \
     if (M <= GW * RW_) {                     \
         if (K <= 512 && np == 1) EL(RW_, 1, 1); \
-        if (K <= 512 && np == 2) EL(RW_, 1, 2); \
-        if (K <= 512) EL(RW_, 1, 4);         \
+        if (K <= 512) EL(RW_, 1, MP);        \
         if (np == 1) EL(RW_, 2, 1);          \
-        if (np == 2) EL(RW_, 2, 2);          \
-        EL(RW_, 2, 4);                       \
+        EL(RW_, 2, MP);                      \
     }
+    constexpr int MP = OUT == ENC_ACT ? enc_parts(1 << 20) : 2;  // behind the down product; behind the output product of heads' parts up to 16 rows
+    if ((np != 1 && np != MP) || K > 1024) return (int)hipErrorInvalidValue;
     ELN(1) ELN(2)
 #undef ELN
 #undef EL
@@ -516,14 +516,13 @@ int enc_attn_gemm(const uint16_t* qkv, const int* klen, float scale, int heads, 
         enc_attn_gemm_kernel<MT_, NS_, F16><<<dim3(H / 16, 1, parts), 64 * GW, enc_fused_lds<MT_>(K), st>>>(qkv, klen, scale, heads, W, y, M, H); \
         return (int)hipGetLastError();                                                                                                 \
     } while (0)
-#define EAM(MT_)                      \
-    if (M <= 16 * MT_) {              \
-        if (K <= 256) EA(MT_, 1);     \
-        if (K <= 512) EA(MT_, 2);     \
-        EA(MT_, 4);                   \
-    }
-    EAM(1) EAM(2) EAM(3) EAM(4)
-#undef EAM
+    // (of at most 16 heads: two parts of up to eight to 16 rows, above four parts or two pairs)
+    if (K > (M <= 16 ? 512 : 256)) return (int)hipErrorInvalidValue;
+    if (M <= 16 && K > 256) EA(1, 2);
+    if (M <= 16) EA(1, 1);
+    if (M <= 32) EA(2, 1);
+    if (M <= 48) EA(3, 1);
+    if (M <= 64) EA(4, 1);
 #undef EA
     return (int)hipErrorInvalidValue;
 }
