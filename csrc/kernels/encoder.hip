@@ -2,13 +2,16 @@
 //
 // A layer is four GEMMs, attention (attention_dense.hip) and two LayerNorms. Batches of few rows are bound by launches
 // and by the time a workgroup waits for its first loads, large ones by the GEMMs and by the passes between them; so
-//   - few rows run whole layers from one call (mxk_enc_layers), with a GEMM that splits K over the waves of a workgroup
+//   - up to 64 rows the layers run from one call (mxk_enc_layers), with a GEMM that splits K over the waves of a workgroup
 //     and applies bias and GELU to its fp32 sums, and with what lies before a product done inside it where that is cheaper
 //     than a launch: attention of one text up to 64 rows, the norms up to 16;
-//   - above, the caller multiplies with the library and the passes between are one kernel each, over 16-bit rows.
+//   - above, and for wider layers below, they run from one call too (mxk_enc_layers_tiled), on dense16.hip's tiles with bias and GELU in the
+//     up product's epilogue, the narrow products' sums in fp32 parts that the LayerNorm adds up, or 16 bits;
+//   - widths that are no whole 64s: the first up to ops/dense.py small_rows, beyond that the caller multiplies with the library and the passes
+//     between are one kernel each, over 16-bit rows.
 // Measured on BERT-base, against padded rows with fp32 copies around each LayerNorm and a library call per operation: one
-// text of 19 tokens 2019 -> 375 us (75 launches of 4-5 us; 8 tokens 275, 51 launches), 48 texts of 23-401 tokens (6428 rows of 19248 padded) 7147 ->
-// 2278: LayerNorm + casts 74 -> 8.3 us (30 MB: 3.6 TB/s), GELU 40 -> 16 (79 MB: 4.9 TB/s).
+// text of 19 tokens 2019 -> 345 us (75 launches of 4-5 us; 8 tokens 275, 51 launches), 48 texts of 23-401 tokens (6428 rows of 19248 padded) 7147 ->
+// 2041 on tiles (2278 with the library's products): LayerNorm + casts 74 -> 8.3 us (30 MB: 3.6 TB/s), GELU 40 -> 16 (79 MB: 4.9 TB/s) and then none.
 #include "dense16.h"
 #include "mx_common.h"
 

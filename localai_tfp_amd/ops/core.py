@@ -453,7 +453,8 @@ def flash_plan(T: int, n_seqs: int, Hq: int, Hkv: int, D: int, block_size: int, 
     One sequence's chunk behind a context known to be 64 key tiles or more and four times its rows goes to 8 waves in as many
     parts as still run at once: half the staging per product (32 / 8 x 128, us with 4 / 8: 416 rows behind 12000 keys 119 / 110,
     in fp8 136 / 114, behind 6000 73 / 68, 1000 behind 12000 238 / 215, 2048 457 / 433). Not chunks of fewer than two blocks (64
-    rows behind 30000 81 / 101), nor shorter contexts (289 behind 2000 41 / 50, whole prompts of 1500 42 / 48).
+    rows behind 30000 81 / 101), nor shorter contexts (289 behind 2000 41 / 50, whole prompts of 1500 42 / 48). Only steps launched eagerly and
+    callers that capture one sequence know such a context: the engine's graphs have four sequences and know contexts up to 1280 keys.
     Contexts of one key tile are the 16-row kernel's where its smaller workgroups wait less (us here / there, D 128): few of
     them 8.6 / 7.4 (33 rows), sequences that its row tiles hold whole 9.4 / 7.4 (64 x 1), 27 / 19 (200 x 1), 17.4 / 14.4 (100 x
     10), with a soft cap 9.4 / 7.5 (33 rows); not 11.7 / 17.3 (64 x 17), nor beyond what the chip holds at once with more than 4

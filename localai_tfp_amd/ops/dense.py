@@ -26,9 +26,10 @@ def to_dev(a, device, dtype) -> torch.Tensor:
 
 
 def few_rows_parts(M: int, N: int, K: int) -> int:
-    """Parts of K that csrc/kernels/lin16.hip sums for M rows, or 0 where the library multiplies.
+    """Parts of K that csrc/kernels/lin16.hip sums for M rows, or 0 where the library multiplies. It is asked after dense16.hip (takes_dense16), so
+    what comes here is f16, and of bf16 long K with fewer than 2^24 weights, K that is no whole 64s, and rows of `out` off 16 bytes.
 
-    Measured with weights in no cache (bf16, f16 alike; us, here / library): long K and few columns, where the library's choice
+    Measured with weights in no cache, against the library (bf16, f16 alike; us, here / library): long K and few columns, where the library's choice
     degrades beyond K = 16384: 4096 x 17408 0.75 of the library's time at one row, 0.34-0.4 beyond 32, x 28672 0.96 and 0.4-0.47,
     3072 0.65-0.9 and 0.3-0.6, 2048 0.25-0.6, 1024 0.22-0.7, 128-512 0.22-1.0; but 64 x 49152 1.06-1.4 beyond 32 rows, 5120 x
     20480 49-56 / 50-53 to 16 rows, 8192 x 20480 66-89 / 59-65 to 32. Many columns and up to 8 rows: 24576-32768 x 512-2304
@@ -147,10 +148,11 @@ ENC_SMALL_ROWS = 448  # where tiles do not take the widths
 
 
 def small_rows(hidden: int, ffn: int) -> int:
-    """Packed rows up to which the layers run on encoder.hip's 16-column GEMMs rather than the library's (they read a layer's weights once
-    per 64 rows, so rows x weights decide; beyond 64 M weights a layer the library's tiles win at any row count).
+    """Packed rows up to which encoder.hip's 16-column GEMMs are faster than the library's (they read a layer's weights once per 64 rows, so rows
+    x weights decide; beyond 64 M weights a layer the library's tiles win at any row count). They run the layers up to here where dense16.hip's
+    tiles do not take the widths (no whole 64s), and up to 64 rows where they do; the tiles' undivided products keep their fp32 sums up to here.
 
-    Whole embed calls, us, one call / library GEMMs issued from Python (110 us a layer at least): 384 x 1536, 12 layers, 448 rows
+    Whole embed calls, us, one call / library GEMMs issued from Python (110 us a layer at least), all widths by these two: 384 x 1536, 12 layers, 448 rows
     679 / 1433; 768 x 3072, 12 layers, 64 rows 657 / 1374, 384 1161 / 1363, 512 1275 / 1356, 640 1488 / 1354; 1024 x 4096, 24
     layers, 64 rows 1428 / 2631, 256 2263 / 2605, 320 2857 / 2624; 1280 x 5120, 8 layers, 128 rows 828 / 910, 192 940 / 906; 1536 x
     6144, 8 layers, 96 rows 813 / 958, 128 994 / 952; 2048 x 8192, 8 layers, 48 rows 899 / 963, 128 1388 / 947; 3072 x 12288, 4
