@@ -436,6 +436,7 @@ ATTN_VMODE = int(__import__("os").environ.get("MX_ATTN_VMODE", "0"))
 
 CU_COUNT = 256
 FLASH_SPLIT_KEYS = 2048  # contexts from which a grid that leaves compute units idle splits its keys
+FLASH_MIN_TILES = 16  # fewest 64-key tiles of a part that is not a block's last (attention_flash.hip MIN_TILES)
 
 
 def flash_plan(T: int, n_seqs: int, Hq: int, Hkv: int, D: int, block_size: int, table_width: int, window: int,
@@ -450,11 +451,15 @@ def flash_plan(T: int, n_seqs: int, Hq: int, Hkv: int, D: int, block_size: int, 
     A grid of fewer than two workgroups per compute unit is split over its keys where the context is long: 416 rows behind
     12000 keys 275 -> 140 us, 289 behind 2000 58 -> 41; the merge launch costs 1.5-2 us where it has nothing to merge, so
     contexts that are known to be short (else what the block tables can hold) do not ask for it.
-    One sequence's chunk behind a context known to be 64 key tiles or more and four times its rows goes to 8 waves in as many
-    parts as still run at once: half the staging per product (32 / 8 x 128, us with 4 / 8: 416 rows behind 12000 keys 119 / 110,
-    in fp8 136 / 114, behind 6000 73 / 68, 1000 behind 12000 238 / 215, 2048 457 / 433). Not chunks of fewer than two blocks (64
-    rows behind 30000 81 / 101), nor shorter contexts (289 behind 2000 41 / 50, whole prompts of 1500 42 / 48). Only steps launched eagerly and
-    callers that capture one sequence know such a context: the engine's graphs have four sequences and know contexts up to 1280 keys.
+    One sequence's chunk of two blocks or more behind a context known to be 64 key tiles or more and four times its rows may go to 8
+    waves in as many parts as still run at once: half the staging per product. Such a workgroup takes about as long for a tile as two of 4
+    waves that share a compute unit (32 / 8 x 128, us with 4 / 8: 416 rows behind 12000 keys 115 / 108, 1000 240 / 221, 2000 behind 30000
+    1061 / 998; 320 rows of 128 / 8 x 128 in q8_0 behind 7000 257 / 221), but 1.2 times as long as one alone (128 rows behind 4096 39 / 49, 256
+    41 / 46, 512 of 8 / 8 behind 7000 42 / 51). So it is taken where the 4-wave plan has more whole parts than compute units (a last one of three
+    quarters counts) and its own parts are not 1.2 times as long, or where its parts are shorter by a tenth (512 rows of 64 / 8 behind
+    30000, one part / two, 605 / 487). Over 484 shapes (12 head counts, 128 to 2100 rows behind 4096 to 30000, bf16, fp8, q8_0) the pick is 0.01 %
+    slower than the better of the two on average and 2.4 % at most. Only steps launched eagerly and callers that capture one sequence know
+    such a context: the engine's graphs have four sequences and know contexts up to 1280 keys.
     Contexts of one key tile are the 16-row kernel's where its smaller workgroups wait less (us here / there, D 128): few of
     them 8.6 / 7.4 (33 rows), sequences that its row tiles hold whole 9.4 / 7.4 (64 x 1), 27 / 19 (200 x 1), 17.4 / 14.4 (100 x
     10), with a soft cap 9.4 / 7.5 (33 rows); not 11.7 / 17.3 (64 x 17), nor beyond what the chip holds at once with more than 4
@@ -474,13 +479,17 @@ def flash_plan(T: int, n_seqs: int, Hq: int, Hkv: int, D: int, block_size: int, 
     blocks = lambda waves: T // (32 * waves // G) + min(n_seqs, T)  # noqa: E731
     if D == 128 and T >= 4096 * n_seqs and T // (256 // G) * Hkv >= 2 * CU_COUNT:
         return (8, 1) if blocks(8) <= 65535 else None
-    rows8 = 256 // G
-    wide = -(-T // rows8) * Hkv
-    if n_seqs == 1 and ctx_lens_host and window <= 0 and longest >= max(4096, 4 * T) and T >= 2 * rows8 and wide <= CU_COUNT:
-        return 8, min(16, CU_COUNT // wide)
     base = blocks(4) * Hkv
     keys = min(longest, window + 32 * 4 // G) if window > 0 else longest
     parts = max(1, min(16, 2 * CU_COUNT // base)) if keys >= FLASH_SPLIT_KEYS else 1
+    rows8, tiles64 = 256 // G, -(-longest // 64)
+    wide = -(-T // rows8) * Hkv
+    if n_seqs == 1 and ctx_lens_host and window <= 0 and longest >= max(4096, 4 * T) and T >= 2 * rows8 and wide <= CU_COUNT:
+        parts8 = min(16, CU_COUNT // wide)
+        per4, per8 = (max(FLASH_MIN_TILES, -(-tiles64 // p)) for p in (parts, parts8))
+        whole = -(-T // (128 // G)) * Hkv * ((tiles64 + per4 // 4) // per4)
+        if 10 * per8 <= 9 * per4 or whole > CU_COUNT and 10 * per8 <= 12 * per4:
+            return 8, parts8
     return (4, parts) if blocks(4) <= 65535 else None
 
 

@@ -159,12 +159,24 @@ def test_pages_and_rising_scores(bs, D, waves, rise, monkeypatch):
 
 
 def test_plan_of_chunks_behind_long_contexts():
-    """8 waves for one sequence's chunk of two blocks or more where 64 key tiles and four times its rows are known to lie before it."""
+    """8 waves for one sequence's chunk of two blocks or more where 64 key tiles and four times its rows are known to lie before it, and 4 waves
+    would share most compute units or leave parts longer; not where each would have a compute unit to itself."""
     p = lambda T, ctx, n=1, H=32, window=0: K.flash_plan(T, n, H, 8, 128, 16, 2048, window, ctx)  # noqa: E731
-    assert p(416, [12416]) == (8, 4) and p(128, [4096]) == (8, 16) and p(1024, [4096]) == (8, 2) and p(2048, [14048]) == (8, 1)
+    assert p(416, [12416]) == (8, 4) and p(128, [12288]) == (8, 16) and p(1024, [4096]) == (8, 2) and p(2048, [14048]) == (8, 1)
     assert p(127, [4096])[0] == 4 and p(416, [4095])[0] == 4 and p(1025, [4096])[0] == 4 and p(2049, [14048])[0] == 4
     assert p(416, None)[0] == 4 and p(416, [12416] * 2, 2)[0] == 4 and p(416, [12416], window=512)[0] == 4
     assert p(64, [9000], H=64) == (8, 16) and p(63, [9000], H=64)[0] == 4
+    assert p(128, [4096])[0] == p(256, [4352])[0] == p(200, [4300])[0] == 4 and p(512, [30512], H=64) == (8, 2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("waves,parts", [(4, 1), (4, 2), (8, 1), (8, 2)])
+@pytest.mark.parametrize("blocks", [[1], [2], [4], [1, 1], [1.0, 1.0, 0.0], [2.0, 0.0, 1.0, 0.0]])
+def test_grids_hold_the_most_blocks_that_sequences_have(blocks, waves, parts, monkeypatch):
+    """Whole blocks (given as whole numbers) and one row more of each (given as floats, 0.0 one row), which is the most blocks for their
+    rows: every row is written."""
+    rows = [int(b) * 8 * waves + isinstance(b, float) for b in blocks]
+    _check(8, 2, 128, rows, [1100] * len(rows), plan=(waves, parts), monkeypatch=monkeypatch)
 
 
 @pytest.mark.gpu
