@@ -52,8 +52,11 @@ MX_DEV float lanes_sum(float v) {
     return v;
 }
 
-// grid (column blocks, H, sequences from s0 on); block = 256 threads = 256 / LPC columns. ONE: rounds of one token
-template <int NPL, int LPC, bool DELTA, bool CHD, bool ONE>
+// what a round of tokens is: one token; up to TB with a test between steps; or whole rounds in a body of their own without that test
+enum { ROUND_ONE = 0, ROUND_ANY = 1, ROUND_WHOLE = 2 };
+
+// grid (column blocks, H, sequences from s0 on); block = 256 threads = 256 / LPC columns
+template <int NPL, int LPC, bool DELTA, bool CHD, int ROUND>
 __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk, const float* q, int ldq,
                                                          const float* v, int ldv, const float* decay, int ldd,
                                                          const float* coef, int ldc, int coef_sigmoid,
@@ -62,6 +65,7 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk
                                                          int ldo, int H, int G, int N, int P, float q_scale,
                                                          float* nout, int s0) {
     static_assert(LPC == 4 || LPC == 16, "a column's lanes are a quad or a DPP row");
+    constexpr bool ONE = ROUND == ROUND_ONE;
     constexpr int NT = 256;
     constexpr int NP = NPL * LPC;  // padded N
     constexpr int COLS = NT / LPC;
@@ -155,17 +159,14 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk
             st_ac = *src;
         }
     };
-    // which vector and number of it, and which column, a thread stages: the same in every group where groups are whole tokens
-    constexpr int KC = NT % (NW * NP) ? KQ_PT : 1, VC = NT % COLS ? V_PT : 1;
-    float st_mul[KC];
-    bool st_on[KC];
+    // which vector and number of it, and which column, a thread stages: the same in every group where groups are whole tokens. (With channel decays
+    // they are not, and an entry for each of up to 24 groups took so many registers that one block ran on a compute unit for two: 30 chunks of 250
+    // rows, 32 heads of 128 x 128 1081 -> 1704 us. There they are worked out where they are needed.)
+    constexpr bool SAME = !ONE && NT % (NW * NP) == 0;
+    constexpr int VC = NT % COLS ? V_PT : 1;
+    const float st_mul = (threadIdx.x / NP) % NW == 1 ? q_scale : 1.f;
+    const bool st_on = threadIdx.x % NP < N;
     int st_col[VC];
-#pragma unroll
-    for (int i = 0; i < KC; ++i) {
-        const int idx = threadIdx.x + i * NT;
-        st_mul[i] = (idx / NP) % NW == 1 ? q_scale : 1.f;
-        st_on[i] = idx % NP < N;
-    }
 #pragma unroll
     for (int i = 0; i < VC; ++i) st_col[i] = blockIdx.x * COLS + (threadIdx.x + i * NT) % COLS;
     auto publish = [&](int b) {
@@ -173,8 +174,8 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk
         for (int i = 0; i < KQ_PT; ++i) {
             const int idx = threadIdx.x + i * NT;
             if (ONE && idx >= TB * NW * NP) continue;
-            if constexpr (ONE) (&kq[b][0][0][0])[idx] = idx % NP < N ? ((idx / NP) % NW == 1 ? st_kq[i] * q_scale : st_kq[i]) : 0.f;
-            else (&kq[b][0][0][0])[idx] = st_on[i % KC] ? st_kq[i] * st_mul[i % KC] : 0.f;
+            if constexpr (SAME) (&kq[b][0][0][0])[idx] = st_on ? st_kq[i] * st_mul : 0.f;
+            else (&kq[b][0][0][0])[idx] = idx % NP < N ? ((idx / NP) % NW == 1 ? st_kq[i] * q_scale : st_kq[i]) : 0.f;
         }
 #pragma unroll
         for (int i = 0; i < V_PT; ++i)
@@ -256,7 +257,7 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk
             }
         };
         if constexpr (ONE) steps(std::true_type{});
-        else if (nt == TB) steps(std::true_type{});
+        else if (ROUND == ROUND_WHOLE && nt == TB) steps(std::true_type{});
         else steps(std::false_type{});
         auto put = [&](int tt, float o) {
             if (tt >= nt || !live) return;
@@ -403,14 +404,21 @@ extern "C" int mxh_state_scan(const float* k, int ldk, const float* q, int ldq, 
     const int few = N > 64 ? (!channel ? 4 : n_pf < 8 ? 12 : 16) : channel ? 4 : 3;
     const bool one = T - n_dec <= (long)few * n_pf, apart = !one && (long)grid.x * H * n_dec >= 4096;
     const dim3 grid_dec(grid.x, H, n_dec), grid_pf(grid.x, H, apart ? n_pf : n_seqs);
+    // Whole rounds take a fifth less time (one chunk of 2900 rows 644 -> 512 us) and more registers, so fewer blocks run on a compute unit: chunks of
+    // less than a round gain nothing (20 of 9 rows, 32 heads of 128 x 128 30.1 -> 35.0, 100 decode rows beside 18 rows in three chunks, 24 heads
+    // of 32 x 32 11.9 -> 14.0), and with channel decays and N 65 to 128 one block runs where two did, so only grids that leave it alone anyway
+    // gain (one chunk of 1111 rows 277 -> 238, three of 301 to 1111 365 -> 428, 30 of 64 338 -> 523).
+    const long blocks_pf = (long)grid_pf.x * H * grid_pf.z;
+    const bool whole = T - n_dec >= 16l * n_pf && !(channel && N > 64 && N <= 128 && blocks_pf > 256);
 #define GO2(NPL, LPC, D_, C_)              \
     do {                                   \
         if (one) {                         \
-            GO3(NPL, LPC, D_, C_, true, grid, 0); \
+            GO3(NPL, LPC, D_, C_, ROUND_ONE, grid, 0); \
             break;                         \
         }                                  \
-        if (apart) GO3(NPL, LPC, D_, C_, true, grid_dec, 0); \
-        GO3(NPL, LPC, D_, C_, false, grid_pf, apart ? n_dec : 0); \
+        if (apart) GO3(NPL, LPC, D_, C_, ROUND_ONE, grid_dec, 0); \
+        if (whole) GO3(NPL, LPC, D_, C_, ROUND_WHOLE, grid_pf, apart ? n_dec : 0); \
+        else GO3(NPL, LPC, D_, C_, ROUND_ANY, grid_pf, apart ? n_dec : 0); \
     } while (0)
 #define GO3(NPL, LPC, D_, C_, O_, GRID, S0)                                                                                  \
     state_scan_kernel<NPL, LPC, D_, C_, O_><<<GRID, threads, 0, st>>>(k, ldk, q, ldq, v, ldv, decay, ldd, coef, ldc,      \

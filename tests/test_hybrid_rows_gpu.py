@@ -73,6 +73,28 @@ def test_short_chunks_and_rows_apart(H, N, P, n_dec, chunks, delta, channel):
         assert (a - b).abs().max() <= 2e-5 * b.abs().max()
 
 
+@pytest.mark.parametrize("n_dec,chunks", [(1, [33, 16, 5, 40]), (2, [15, 9, 15, 8])])
+@pytest.mark.parametrize("N,P", [(128, 64), (65, 64), (64, 130)])
+@pytest.mark.parametrize("delta,channel", [(True, False), (False, True), (True, True)])
+def test_rounds_of_full_grids(N, P, n_dec, chunks, delta, channel):
+    """Grids of more workgroups than compute units, whose whole rounds run with the others in one body where decays are per channel, and chunks of
+    less than a round each; the bound of test_rounds_of_tokens."""
+    g = torch.Generator().manual_seed(N + n_dec)
+    H, T, slots = 16, n_dec + sum(chunks), list(range(n_dec + len(chunks)))
+    k, q, v = torch.randn(T, 2 * N, generator=g) * N ** -0.5, torch.randn(T, 2 * N, generator=g), torch.randn(T, H * P, generator=g)
+    decay, coef = torch.rand(T, H * N if channel else H, generator=g), torch.rand(T, H, generator=g)
+    at = [(i * 3) % 5 for i in range(len(slots))]
+    start = torch.randn(len(slots), H, P, N, generator=g)
+    got = {}
+    for dev in ("cpu", "cuda"):
+        state, out = start.clone().to(dev), torch.zeros(T, H * P, device=dev)
+        HY.state_scan(k.to(dev), q.to(dev), v.to(dev), decay.to(dev), coef.to(dev), None, state, _rag(n_dec, chunks, at, slots, dev), out,
+                      H, 2, N, P, delta, channel, 0.5, False, None)
+        got[dev] = [out.cpu(), state.cpu()]
+    for a, b in zip(got["cuda"], got["cpu"]):
+        assert (a - b).abs().max() <= 2e-5 * b.abs().max()
+
+
 @pytest.mark.parametrize("F,group,off", [(4, 4, 0), (260, 4, 0), (2048, 256, 0), (1023, 1023, 0), (1024, 2, 0), (1024, 1024, 1)])
 @pytest.mark.parametrize("act", ["silu", "gelu_tanh", "relu2", "clamped", "gelu"])
 def test_glu_widths(F, group, off, act):
