@@ -40,13 +40,14 @@ MX_DEV float block_sum_dyn(float v, float* red) {
     return s;
 }
 
-// grid (T, C / (NT V)): V numbers a thread, four where rows and tables lie on 16 bytes (8 for 16-bit ones). A loop over a row waited for each of
-// its stores' aliases: 33 rows of 4096 took 9.8 us in a profile, now 4.7 (an empty launch shows 3 to 4)
+// grid (T, C / (4 NT)): four numbers a thread, neighbours (V = 4) where rows and tables lie on 16 bytes (8 for 16-bit ones), else NT apart. A
+// loop over a row waited for each of its stores' aliases: 33 rows of 4096 took 9.8 us in a profile, now 4.7 (an empty launch shows 3 to 4). One
+// number a thread was bound by its workgroups: 30000 rows of 4098 in bf16 167 us by the loop, 307 so, now 170.
 template <bool B16, int V>
 __global__ __launch_bounds__(NT) void embed_rows_kernel(const void* __restrict__ table, int rows, const int* tokens, float* out,
                                                         int ldo, int accumulate, int C, bf16_t* o16, int ld16,
                                                         float scale) {
-    const int t = blockIdx.x, c = (blockIdx.y * NT + threadIdx.x) * V;
+    const int t = blockIdx.x, c = V == 4 ? (blockIdx.y * NT + threadIdx.x) * 4 : blockIdx.y * (4 * NT) + threadIdx.x;
     if (c >= C) return;
     int tok = tokens[t];
     if (tok < 0 || tok >= rows) tok = 0;
@@ -70,10 +71,22 @@ __global__ __launch_bounds__(NT) void embed_rows_kernel(const void* __restrict__
         *(float4*)o = make_float4(v[0], v[1], v[2], v[3]);
         if (o16) *(uint2*)(o16 + (long)t * ld16 + c) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
     } else {
-        float v = ld_elem<B16>(table, at) * scale;
-        if (accumulate) v += *o;
-        *o = v;
-        if (o16) o16[(long)t * ld16 + c] = f32_to_bf16(v);
+        float v[4], old[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int i = min(e * NT, C - 1 - c);  // (past the end: the last one again, not stored)
+            v[e] = ld_elem<B16>(table, at + i);
+            old[e] = accumulate ? o[i] : 0.f;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[e] *= scale;
+            if (accumulate) v[e] += old[e];
+            if (c + e * NT < C) {
+                o[e * NT] = v[e];
+                if (o16) o16[(long)t * ld16 + c + e * NT] = f32_to_bf16(v[e]);
+            }
+        }
     }
 }
 
@@ -763,9 +776,8 @@ extern "C" int mxh_embed_rows(const void* table, int is16, int V, const int* tok
     MXH_CHECK(table && tokens && out && C > 0 && V > 0 && ldo >= C && (!o16 || ld16 >= C));
     const bool four = C % 4 == 0 && ldo % 4 == 0 && (!o16 || ld16 % 4 == 0) && ((uintptr_t)out & 15) == 0 && ((uintptr_t)table & (is16 ? 7 : 15)) == 0 &&
                       ((uintptr_t)o16 & 7) == 0;
-    const long wide = four ? 4 * NT : NT;
-    MXH_CHECK((C + wide - 1) / wide <= 65535 && T <= (1 << 24) - 1);
-    const dim3 grid(T, (unsigned)((C + wide - 1) / wide));
+    MXH_CHECK((C + 4 * NT - 1) / (4 * NT) <= 65535 && T <= (1 << 24) - 1);
+    const dim3 grid(T, (unsigned)((C + 4 * NT - 1) / (4 * NT)));
 #define GO(B_, V_) embed_rows_kernel<B_, V_><<<grid, NT, 0, st>>>(table, V, tokens, out, ldo, accumulate, C, o16, ld16, scale)
     if (is16 && four) GO(true, 4);
     else if (is16) GO(true, 1);

@@ -95,6 +95,24 @@ def test_rounds_of_full_grids(N, P, n_dec, chunks, delta, channel):
         assert (a - b).abs().max() <= 2e-5 * b.abs().max()
 
 
+@pytest.mark.parametrize("C,off", [(1, 0), (255, 0), (256, 1), (257, 0), (1023, 0), (1024, 1), (1025, 0), (2050, 3), (4098, 0), (4096, 0)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_embedding_rows_of_any_width(C, off, dtype):
+    """Widths around a workgroup's numbers, rows that lie on 16 bytes and not, tokens out of the table (row 0). A scale of 2 rounds nothing, and the
+    sum with the old number is rounded once on either side: the same bits."""
+    g = torch.Generator().manual_seed(C)
+    table, ids = torch.randn(9, C, generator=g).to(dtype), torch.tensor([3, 8, 0, -1, 9, 3], dtype=torch.int32)
+    old = torch.randn(6, C + off + 5, generator=g)
+    want = table.float()[ids.where((ids >= 0) & (ids < 9), torch.zeros_like(ids)).long()] * 2
+    for acc in (False, True):
+        buf, o16 = old.clone().cuda(), torch.zeros(6, C + off + 3, dtype=torch.bfloat16, device="cuda")
+        HY.embed_rows(table.cuda(), ids.cuda(), buf[:, off:off + C], accumulate=acc, out16=o16[:, off:off + C], scale=2.0)
+        w = want + old[:, off:off + C] if acc else want
+        assert torch.equal(buf[:, off:off + C].cpu(), w) and torch.equal(o16[:, off:off + C].cpu(), w.bfloat16())
+        buf[:, off:off + C] = old[:, off:off + C].cuda()
+        assert torch.equal(buf.cpu(), old) and not o16[:, :off].any() and not o16[:, off + C:].any()
+
+
 @pytest.mark.parametrize("F,group,off", [(4, 4, 0), (260, 4, 0), (2048, 256, 0), (1023, 1023, 0), (1024, 2, 0), (1024, 1024, 1)])
 @pytest.mark.parametrize("act", ["silu", "gelu_tanh", "relu2", "clamped", "gelu"])
 def test_glu_widths(F, group, off, act):
