@@ -555,7 +555,8 @@ __global__ __launch_bounds__(256) void attn_chunk_mfma_kernel(const bf16_t* __re
 // as attn_chunk_mfma_kernel does, 32 at a time (key fragments straight from the pages, values staged in LDS by the
 // wave itself, the next tile requested ahead). With one
 // partition it writes the result, otherwise (max, sum, unnormalised output) for attn_merge_kernel; the running maximum
-// is kept in base 2 and handed over in base e.
+// is kept in base 2 and handed over in base e. Partitions are made for the longest context that the step may have, so
+// most may be empty: those behind a context write their sum, 0, alone.
 template <int DK, int DV, bool O16, bool P2>
 __global__ __launch_bounds__(64) void attn_decode_mfma_kernel(const bf16_t* __restrict__ q, int ldq,
                                                               const bf16_t* __restrict__ kc,
@@ -581,6 +582,10 @@ __global__ __launch_bounds__(64) void attn_decode_mfma_kernel(const bf16_t* __re
     int v_begin = 0, v_end = qpos + 1 - kr.gap;  // visible keys [v_begin, v_end)
     if (parts > 1) {
         v_begin = z * part_len;
+        if (z > 0 && v_begin >= v_end) {
+            if (lane < rep) part_ml[(((size_t)s * H + kvh * rep + lane) * parts + z) * 2 + 1] = 0.f;
+            return;
+        }
         v_end = min(v_end, v_begin + part_len);
         sink = 0;  // joins in the merge
     }
@@ -763,7 +768,7 @@ __global__ __launch_bounds__(64) void attn_decode_mfma_kernel(const bf16_t* __re
 #undef STORE_TILE
 
 // grid (rows, H): combines the partitions of a row (at most 64: lane z holds partition z's maximum and sum) in a fixed
-// order; an empty partition has sum 0
+// order; an empty partition has sum 0, and none behind the last that has keys is read
 template <bool O16>
 __global__ __launch_bounds__(64) void attn_merge_kernel(const float* part_ml, const float* part_o, int parts, int H,
                                                         int dv, int sink, float out_scale, int row_base, void* out,
@@ -773,6 +778,7 @@ __global__ __launch_bounds__(64) void attn_merge_kernel(const float* part_ml, co
     const long p0 = ((long)r * H + h) * parts;
     const int zc = min(lane, parts - 1);
     const float mz = part_ml[(p0 + zc) * 2], lz = lane < parts ? part_ml[(p0 + zc) * 2 + 1] : 0.f;
+    const int used = 64 - __builtin_clzll(__ballot(lz > 0.f) | 1);
     float M = wave_max(lz > 0.f ? mz : -INFINITY);
     const float s0 = sink_score(ex, h);
     if (sink) M = fmaxf(M, s0);
@@ -786,12 +792,12 @@ __global__ __launch_bounds__(64) void attn_merge_kernel(const float* part_ml, co
         if (u * 64 < dv) {
             const int cc = min(c, dv - 1);
             float a = 0.f;
-            for (int z0 = 0; z0 < parts; z0 += 8) {  // eight partitions' numbers requested together
+            for (int z0 = 0; z0 < used; z0 += 8) {  // eight partitions' numbers requested together
                 float x[8];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) x[e] = part_o[(p0 + min(z0 + e, parts - 1)) * dv + cc];
+                for (int e = 0; e < 8; ++e) x[e] = part_o[(p0 + min(z0 + e, used - 1)) * dv + cc];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) a += x[e] * __shfl(w, min(z0 + e, 63), 64) * (z0 + e < parts ? 1.f : 0.f);
+                for (int e = 0; e < 8; ++e) a += x[e] * __shfl(w, min(z0 + e, 63), 64) * (z0 + e < used ? 1.f : 0.f);
             }
             if (c < dv) {
                 const float v = a * (inv * gate_factor(ex, row_base + r, h, c));

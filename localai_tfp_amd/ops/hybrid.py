@@ -480,6 +480,8 @@ def decode_part_len(n_dec: int, heads: int, visible: int, waves: int | None = No
     """Keys per partition of the decode rows: one wave walks a (row, head, partition), so few sequences with long
     visible ranges are split finely (down to one 64-key tile) and large batches coarsely."""
     want = max(1, (DECODE_WAVES if waves is None else waves) // max(1, n_dec * heads))
+    if waves is not None and want < 3:
+        want = 1
     per = -(-max(1, visible) // want)
     return max(64, -(-per // 64) * 64)
 
@@ -488,7 +490,10 @@ def decode_waves_mfma() -> int:
     """Waves to aim for on the matrix-core route, whose wave serves all query heads of a key / value head: 32 a compute unit, since a wave
     waits 3 us for each tile of 32 keys. us with 8 / 16 / 32 / 64 a unit (kernel and merge, H 32, G 8, heads of 128): 33 rows of contexts
     101-4001 under chunks of 2048 72.8 (3 a unit) / 42.9 / 30.9 / 35.2, plain 256 / 122 (7 partitions) / 54 / 55, 64 rows of 65-1021 62 / 40 / 39 / 39, of 1000-8000 452 / 292 /
-    237 / 244, 9 rows of 64-2000 25.9 / 21.8 / 18.8 / 18.8; G 16, heads of 64: 33 rows 215 / 156 / 58 / 42; G 2: 33 rows 58 / 39 / 25 / 25."""
+    237 / 244, 9 rows of 64-2000 25.9 / 21.8 / 18.8 / 18.8; G 16, heads of 64: 33 rows 215 / 156 / 58 / 42; G 2: 33 rows 58 / 39 / 25 / 25.
+    Two parts are one (decode_part_len): they gain nothing where a unit has 12 waves without (200 rows, G 16, contexts 500-4000 in one part / two 432 / 437,
+    30-300 under 1024 34 / 37). Contexts that are all far shorter than the step's bound pay 3 to 5 us for the merge's launch where one part would do
+    (under 8192, 33 rows of 30-200, G 16 14.8 / 17.4, 200 of 50-500, G 8 62 / 68); longer ones gain what stands above."""
     return 2 * DECODE_WAVES
 
 

@@ -18,6 +18,33 @@ def test_partitions_fit_their_workspace():
         assert plen % 64 == 0 and (parts == 1 or nd * G * group * parts <= HY.partition_rows(seqs, G * group, group))
 
 
+def test_two_partitions_are_one():
+    waves = HY.decode_waves_mfma()
+    for nd, G, want in ((waves // 24, 8, 3), (waves // 24 + 1, 8, 1), (waves // 16, 16, 1), (1, 1, 128)):
+        assert -(-8192 // HY.decode_part_len(nd, G, 8192, waves)) == want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,H,G", [(9, 16, 4), (600, 16, 16)])
+def test_partitions_behind_short_contexts(rows, H, G):
+    """Contexts of one to 70 keys in a step whose bound asks for many partitions (one for so many rows): a workspace of NaN shows that what no
+    key fills is not read. Against the same rows without partitions, within the bound of test_partitions_match_one_walk."""
+    gen = torch.Generator().manual_seed(rows)
+    lens = [1 + (i * 23) % 70 for i in range(rows)]
+    d = dict(device="cuda", dtype=torch.int32)
+    tab = torch.zeros(rows, 512, **d)
+    tab[:, :5] = torch.randint(0, 40, (rows, 5), generator=gen).to(**d)
+    ctx = torch.tensor(lens, **d)
+    rag = types.SimpleNamespace(n_dec=rows, n_pf=0, dec_bt=tab, dec_lens=ctx, dec_max_len=8192, positions=ctx - 1)
+    q, kc, vc = (torch.randn(s, generator=gen).bfloat16().cuda() for s in ((rows, H * 64), (40, 16, G * 64), (40, 16, G * 64)))
+    n = HY.partition_rows(rows, H, H // G)
+    ws = torch.full((n, 2), float("nan"), device="cuda"), torch.full((n, 64), float("nan"), device="cuda")
+    got, want, mag = (torch.empty(rows, H * 64, device="cuda", dtype=torch.bfloat16) for _ in range(3))
+    for out, v, w in ((got, vc, ws), (want, vc, None), (mag, vc.abs(), None)):
+        HY.masked_attention(q, kc, v, rag, H, G, 64, 64, 0.125, out, sink=True, workspace=w)
+    assert ((got.float() - want.float()).abs() <= 2 ** -8 * want.float().abs() + 2 ** -8 * 1.02 * mag.float() + 1e-5).all()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("H,G,dk,dv,chunk", [(32, 8, 128, 128, 2048), (16, 16, 64, 64, 0), (24, 2, 128, 64, 500)])
 def test_partitions_match_one_walk(H, G, dk, dv, chunk):
