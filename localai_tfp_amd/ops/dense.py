@@ -27,7 +27,8 @@ def to_dev(a, device, dtype) -> torch.Tensor:
 
 def few_rows_parts(M: int, N: int, K: int) -> int:
     """Parts of K that csrc/kernels/lin16.hip sums for M rows, or 0 where the library multiplies. It is asked after dense16.hip (takes_dense16), so
-    what comes here is f16, and of bf16 long K with fewer than 2^24 weights, K that is no whole 64s, and rows of `out` off 16 bytes.
+    what comes here is f16, and of bf16 long K with few columns or fewer than 2^24 weights, many columns by short K, K that is no whole 64s, and rows of
+    `out` off 16 bytes.
 
     Measured with weights in no cache, against the library (bf16, f16 alike; us, here / library): long K and few columns, where the library's choice
     degrades beyond K = 16384: 4096 x 17408 0.75 of the library's time at one row, 0.34-0.4 beyond 32, x 28672 0.96 and 0.4-0.47,
@@ -189,13 +190,29 @@ def takes_dense16(M: int, N_: int, K: int) -> bool:
     at 121 / 891 20 / 17, 43 / 36 (75 rows 15.4 / 16.4). Many columns by up to 64 rows: 28672 x 4096 at 5 / 33 rows 60 / 45, 50 / 46, 32000 60 / 53, 65536
     119 / 101, 123 / 103, 128256 187 / 181, 208 / 191, 50304 x 2048 48 / 40, 50 / 42, 151936 x 1536 161 / 89, 112 / 105; by up to 16 rows also 24576 x
     3072 49 / 30 (33 rows 32.2 / 32.3) and 25000 x 5120 69 / 47 (33 rows 50 / 52). The rest is the library's: 2048 x 2048 .. 4096 x 4096 are 5 to
-    20 % slower here, 8192 x 8192 0.84 to 1.17, wide matrices by 65 to 300 rows 0.8 to 1.0, by more rows 0.9 to 1.5 as its choice falls."""
+    20 % slower here, 8192 x 8192 0.84 to 1.17, wide matrices by 65 to 300 rows 0.8 to 1.0, by more rows 0.9 to 1.5 as its choice falls.
+    Where the lines lie within these, here against there (lin16.hip for few rows): few rows by 2048 columns and fewer 1.01 to 1.16 (2048 x 20480
+    at 1 / 33 / 48 rows 1.16, 1.00, 0.96; 3072 x 49152 at 8 / 12 1.02, 0.98), 128 x 131072 at 128 rows 1.20, 1024 x 16384 at 64 1.09; more than 900 rows by K
+    up to 8960 0.83 to 1.12, 0.99 on average; one round of 256 x 192 tiles 0.96 to 1.15 (1800 x 5120 x 13824 1.10; three of 32 0.57), all other
+    tiles of 216 products of more rows and longer K 0.86 on average, 1.05 at most; many columns by K of 1024 and less 1.0 to 1.28 beyond 32000
+    columns (100352 x 512 at 16 rows 1.16), by 1280 and more than 16 rows 1.04 to 1.07."""
     if K % 64 or N_ % 4 or M <= 0 or K < 64:
         return False
     if K >= 2 * N_:
-        return M >= (1 if K > 16384 else 64) and N_ * K >= 1 << 24 or M >= 96 and N_ * K >= 12 << 20
+        if M < 96 and N_ * K < 1 << 24 or N_ * K < 12 << 20 or N_ < 256:
+            return False
+        if M < 64:
+            return K > 16384 and (M >= 40 or N_ >= 3072 and (K <= 32768 or M > 8))
+        if M < 96:
+            return K > 16384 or N_ > 1024
+        if M <= 900:
+            return True
+        mi, nj, whole, parts = dense16_plan(M, N_, K)
+        return K >= 9216 and not (mi == 8 and nj == 6 and parts == 1 and -(-M // 256) * -(-N_ // 192) <= CU_COUNT)
     if N_ >= 24576 and M <= 64:
-        return K <= 2048 or K <= 4096 and N_ >= 28672 or K <= 5120 and M <= 16
+        if K <= 2048:
+            return K >= (1280 if M <= 16 else 1536) or N_ <= 32000 and 576 <= K <= 1024
+        return K <= 4096 and N_ >= 28672 or K <= 5120 and M <= 16
     return False
 
 
@@ -203,8 +220,16 @@ def takes_gated16(M: int, N_: int, K: int, Fn: int) -> bool:
     """Whether a projection's N_ plain columns and its gated unit of Fn features run as one launch of dense16.hip. us, the library's product
     and the gating kernel / here: 12320 + 2 x 14336 columns x 4096 at 1 / 33 / 112 / 322 / 703 / 2062 rows 76 / 64, 78 / 67, 92 / 88, 214 / 143, 334 / 227,
     733 / 641, 6176 + 2 x 8192 x 2048 at 5 / 33 / 310 / 1693 / 3557 38 / 22, 29 / 23, 50 / 47, 197 / 158, 407 / 307 (184 rows 41 / 42), 9000 + 2 x 20000 x
-    6144 134 / 111, 145 / 110, 194 / 165 (239 rows); 3000 + 2 x 5632 x 2048 even up to 64 rows (20 / 20 and 20.6 / 21.5), 465 rows 52 / 40."""
-    return M > 0 and K % 64 == 0 and K >= 512 and N_ > 0 and N_ % 4 == 0 and Fn % 8 == 0 and Fn > 0 and (N_ + 2 * Fn) * K >= (1 << 22 if M > 64 else 1 << 25)
+    6144 134 / 111, 145 / 110, 194 / 165 (239 rows); 3000 + 2 x 5632 x 2048 even up to 64 rows (20 / 20 and 20.6 / 21.5), 465 rows 52 / 40.
+    Fewer gated columns than plain ones are left apart between 64 and 1000 rows from K = 2048 on (twelve such of 48 widths and heights 1.02 to 1.27 of
+    the two launches, 0.98 on average; narrower K 0.6 to 0.95), and so are up to 64 rows by fewer than 16384 columns (3840 + 2 x 5120 x 2560 1.17 to
+    1.28). Of 1244 products beyond 64 rows that are taken 2 % are slower by more than 1.05, 768 + 2 x 24576 x 3072 at 80 rows by 1.14; 0.85 on average."""
+    if M <= 0 or K % 64 or K < 512 or N_ <= 0 or N_ % 4 or Fn % 8 or Fn <= 0:
+        return False
+    n = N_ + 2 * Fn
+    if M <= 64:
+        return n >= 16384 and n * K >= 1 << 25
+    return n * K >= 1 << 22 and (2 * Fn >= N_ or K < 2048 or M > 1000)
 
 
 def _dense16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, acc: bool, bias, gated=None) -> bool:

@@ -27,6 +27,17 @@ def test_rules():
     assert not (g(100, 352, 256, 512) or g(8, 1600, 1024, 2816) or g(8, 12320, 4096, 14338) or g(8, 12322, 4096, 14336) or g(0, 12320, 4096, 14336))
 
 
+def test_rules_leave_to_others_what_they_are_faster_at():
+    """Few rows by few columns, many columns by short K, large products of short K or one round of 192-column tiles, gated units that are the smaller part."""
+    t, g = D.takes_dense16, D.takes_gated16
+    assert t(40, 2048, 20480) and t(1, 3072, 20480) and t(9, 3072, 49152) and t(64, 1024, 16448) and t(96, 256, 65536) and t(900, 2048, 8192)
+    assert not (t(39, 2048, 20480) or t(8, 3072, 49152) or t(64, 1024, 16384) or t(128, 128, 131072) or t(901, 2048, 8192) or t(1024, 1536, 8960))
+    assert D.dense16_plan(1800, 5120, 13824)[:2] == (8, 6) and not t(1800, 5120, 13824) and t(1400, 5120, 13824) and t(4000, 5120, 13824)
+    assert t(16, 100352, 1280) and t(64, 100352, 1536) and t(33, 32000, 576) and not (t(16, 100352, 1024) or t(17, 100352, 1280) or t(33, 32000, 512) or t(8, 32004, 1024))
+    assert g(1, 4608, 3072, 6144) and g(65, 3840, 2560, 5120) and g(1001, 9216, 3072, 3072) and g(80, 4608, 1536, 1536)
+    assert not (g(64, 3840, 2560, 5120) or g(1000, 9216, 3072, 3072) or g(65, 6144, 2048, 2048))
+
+
 def _run(epi, tile, x, w, out, whole, parts, bias=None, gated=None):
     from localai_tfp_amd import _native as Nv
     M, K = x.shape
