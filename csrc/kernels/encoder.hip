@@ -2,9 +2,9 @@
 //
 // A layer is four GEMMs, attention (attention_dense.hip) and two LayerNorms. Batches of few rows are bound by launches
 // and by the time a workgroup waits for its first loads, large ones by the GEMMs and by the passes between them; so
-//   - up to 64 rows the layers run from one call (mxk_enc_layers), with a GEMM that splits K over the waves of a workgroup
+//   - up to 64 rows, more of narrow layers (models/bert.py few_rows), they run from one call (mxk_enc_layers), with a GEMM that splits K over the waves of a workgroup
 //     and applies bias and GELU to its fp32 sums, and with what lies before a product done inside it where that is cheaper
-//     than a launch: attention of one text up to 64 rows, the norms up to 16;
+//     than a launch: attention of one text up to 64 rows, the norms up to 16 (8 of several texts beyond 512 columns);
 //   - above, and for wider layers below, they run from one call too (mxk_enc_layers_tiled), on dense16.hip's tiles with bias and GELU in the
 //     up product's epilogue, the narrow products' sums in fp32 parts that the LayerNorm adds up, or 16 bits;
 //   - widths that are no whole 64s: the first up to ops/dense.py small_rows, beyond that the caller multiplies with the library and the passes
@@ -624,7 +624,8 @@ extern "C" int mxk_enc_layers(const void* const* w, int n_layers, uint16_t* x, i
     static_assert(enc_parts(32) == 1 && enc_parts(1 << 20) == 4, "parts");
     const int np = enc_parts(F);
     const bool one = B == 1 && H / heads == 64 && rows <= ENC_ATTN_ROWS && H <= ENC_FUSED_H;
-    const bool norms = rows <= ENC_NORM_ROWS && H <= ENC_FUSED_H;
+    // (layers alone, captured, 2 x 8 rows, us, norms apart / inside: 512 x 2048, 4 layers, 90 / 84, 640 x 2560 103 / 107)
+    const bool norms = rows <= (one || H <= 512 ? ENC_NORM_ROWS : 8) && H <= ENC_FUSED_H;
     uint16_t* xm = norms ? (uint16_t*)(parts + (size_t)4 * rows * H) : x;  // the rows between a layer's halves: where none is read and written at once
     for (int l = 0; l < n_layers; ++l, w += 12) {
         auto at = [&](int i) { return (const uint16_t*)w[i]; };

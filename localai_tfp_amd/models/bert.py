@@ -33,6 +33,16 @@ from ..ops.linear import ACT_DTYPE
 # 600 / 1700 / 6428 / 12000 rows 1378 / 640, 1392 / 1036, 2450 / 2191, 4233 / 3602; 1024 x 4096 1000 / 6428 927 / 617, 2288 / 2232; 2048 x 8192, 4 layers, 100 /
 # 1700 / 12000 492 / 352, 1043 / 924, 5407 / 4938 (6428 rows 2769 / 2837).
 ENC_FEW_ROWS = 64
+# layers of fewer weights than this run on them up to as many more rows. The layers alone, captured, us, these / tiles: 4 of 128 x 512 at 447 rows 106 / 121, 256 x
+# 1024 at 128 / 300 / 400 rows 114 / 119, 136 / 140, 154 / 154, 512 x 2048 at 65 / 128 / 200 120 / 139, 124 / 144, 165 / 158, 640 x 2560 at 65 / 100 157 / 159, 165 /
+# 162; 6 of 384 x 1536 at 65 / 128 / 200 196 / 198, 201 / 203, 233 / 224, 768 x 3072 at 64 / 65 225 / 217, 264 / 243
+ENC_FEW_WEIGHTS = 6_400_000
+
+
+def few_rows(hidden: int, ffn: int) -> int:
+    """Packed rows up to which the layers run on encoder.hip's 16-column GEMMs where dense16.hip's tiles take the widths too."""
+    weights = 4 * hidden * hidden + 2 * hidden * ffn
+    return min(small_rows(hidden, ffn), ENC_FEW_ROWS * max(weights, ENC_FEW_WEIGHTS) // weights)
 
 
 @dataclass
@@ -210,7 +220,7 @@ class BertModel:
         st = N.stream_ptr()
         N.kcall("mxk_enc_embed", img.data_ptr(), R, *ptrs[:5], H, float(cfg.eps), x.data_ptr(), st)
         scale = 1.0 / math.sqrt(H // cfg.n_heads)
-        if H % 64 == 0 and Fd % 64 == 0 and (R > ENC_FEW_ROWS or R > small_rows(H, Fd)):
+        if H % 64 == 0 and Fd % 64 == 0 and R > few_rows(H, Fd):
             plan, keep = encoder_plan(R, H, Fd), R <= small_rows(H, Fd)
             plan = [n if i not in (2, 5) or n > 1 or keep else 0 for i, n in enumerate(plan)]  # 0 parts: 16-bit sums
             most = max(plan[2], plan[5])

@@ -108,6 +108,13 @@ def test_one_call_layers_are_chosen_by_rows_and_width():
     assert rows(3072, 12288) == rows(4096, 16384) == 0
 
 
+def test_narrow_layers_stay_in_one_call():
+    """Layers of few weights leave the 16-column products later than others, at most where any does; wide ones where they leave them for the library."""
+    assert BM.few_rows(64, 256) == BM.few_rows(128, 512) == BM.few_rows(256, 1024) == BM.ENC_SMALL_ROWS and 128 <= BM.few_rows(512, 2048) < 192
+    assert 128 <= BM.few_rows(384, 1536) < 256 and BM.few_rows(768, 3072) == BM.few_rows(1024, 4096) == BM.ENC_FEW_ROWS and BM.few_rows(2048, 8192) == BM.small_rows(2048, 8192) < 64
+    assert BM.few_rows(4096, 16384) == 0
+
+
 @pytest.mark.gpu
 def test_bert_gpu_matches_fp32():
     """GPU path (hipBLASLt GEMMs + attention_dense.hip + norm.hip LayerNorm) vs the fp32 encoder."""
@@ -270,9 +277,10 @@ def test_tiled_layers_match_fp32(tile, dtype, monkeypatch):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("hidden,rows", [(64, 65), (128, 300), (384, 448), (512, 200), (640, 300), (768, 400), (832, 350)])
-def test_sums_stay_in_fp32_until_the_norm(hidden, rows):
+def test_sums_stay_in_fp32_until_the_norm(hidden, rows, monkeypatch):
     """Biases of 1000, which the norms take away again: an f16 there has steps of 0.5, fp32 of 6e-5, beside rows of order 1. Up to small_rows
     the bound of test_wide_one_call_layers holds all the same; the smallest widths have undivided products throughout."""
+    monkeypatch.setattr(BM, "ENC_FEW_ROWS", 0)
     cfg = BM.BertConfig(vocab=400, hidden=hidden, n_layers=2, n_heads=hidden // 64, ffn=4 * hidden, max_pos=300, name="t")
     src = BM.synthetic_bert(cfg, 5)
 
@@ -297,6 +305,7 @@ def test_parts_that_do_not_fit_are_done_without(small, monkeypatch):
     get = BM.synthetic_bert(cfg, 5)
     g, c = BM.BertModel.load(cfg, get, "cuda:0"), BM.BertModel.load(cfg, get, "cpu")
     monkeypatch.setattr(BM, "small_rows", lambda H, F: small)
+    monkeypatch.setattr(BM, "ENC_FEW_ROWS", 0)
     monkeypatch.setattr(BM, "encoder_plan", lambda R, H, F: (36, 68, 3, 36, 40, 8))
     ids = [list(range(10, 10 + n)) for n in (200, 57)]
     want, refused, real = c.embed(ids), [], torch.empty
