@@ -118,14 +118,15 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(float* __restrict__ qkv, c
 // KVF_Q8_0: eight consecutive lanes hold a block of 32, rounded to bf16 as the staged rows of the other block formats are, and store its
 // codes themselves: the rows' trip through a staging buffer was a second launch a layer (and one for its slots), 584 -> 559 us for a
 // four-layer step of 9 rows.
-template <int D, bool NEOX, bool HAS_BIAS, bool ZERO, int KVF, bool QKN = false>
+// AHEAD: the slot and a thread's one load of the values are asked for with its first unit; behind the barrier they are waits of their own. With
+// more loads than one, or so many rows that others hide the wait, it costs more than it gives (1000 rows of 16 / 16 heads of 128 6.7 -> 7.4 us).
+template <int D, bool NEOX, bool HAS_BIAS, bool ZERO, int KVF, bool QKN, bool AHEAD>
 __global__ __launch_bounds__(256) void rope_kv4_kernel(float* __restrict__ qkv, const float* __restrict__ bias,
                                                        const int* __restrict__ pos, const int* __restrict__ slots,
                                                        const float* __restrict__ inv_freq, float attn_factor, int Hq,
                                                        int Hkv, bf16_t* __restrict__ qo, void* __restrict__ kc,
                                                        void* __restrict__ vc, int block_size,
-                                                       const float* __restrict__ qn = nullptr,
-                                                       const float* __restrict__ kn = nullptr, float eps = 0.f) {
+                                                       const float* __restrict__ qn, const float* __restrict__ kn, float eps) {
     constexpr int HALF = D / 2;
     constexpr int UPH = NEOX ? D / 8 : D / 4;  // work units per head
     constexpr int USH = UPH == 8 ? 3 : UPH == 16 ? 4 : 5;
@@ -157,9 +158,12 @@ __global__ __launch_bounds__(256) void rope_kv4_kernel(float* __restrict__ qkv, 
     }
     const int vi = v_lo * (D / 4) + threadIdx.x;
     float4 v0 = {0.f, 0.f, 0.f, 0.f};
-    if (vi < v_hi * (D / 4)) v0 = *(const float4*)(row + (Hq + Hkv) * D + 4 * vi);
-    const int p = pos[t], slot = slots[t];  // (behind the barrier the slot and the values were waits of their own)
-    const int blk = slot >= 0 ? slot / block_size : 0, off = slot >= 0 ? slot % block_size : 0;
+    int slot = 0;
+    if constexpr (AHEAD) {
+        if (vi < v_hi * (D / 4)) v0 = *(const float4*)(row + (Hq + Hkv) * D + 4 * vi);
+        slot = slots[t];
+    }
+    const int p = pos[t];
     for (int i = threadIdx.x; i < HALF; i += 256) {
         float sv, cv;
         sincosf((float)p * inv_freq[i], &sv, &cv);
@@ -167,6 +171,8 @@ __global__ __launch_bounds__(256) void rope_kv4_kernel(float* __restrict__ qkv, 
         sn[i] = sv * attn_factor;
     }
     __syncthreads();
+    if constexpr (!AHEAD) slot = slots[t];
+    const int blk = slot >= 0 ? slot / block_size : 0, off = slot >= 0 ? slot % block_size : 0;
     auto put = [&](void* pool, int kh, int d, float4 y) {
         const size_t r = ((size_t)blk * Hkv + kh) * block_size + off;
         if constexpr (KVF == KVF_Q8_0) {
@@ -246,7 +252,8 @@ __global__ __launch_bounds__(256) void rope_kv4_kernel(float* __restrict__ qkv, 
     for (int idx = vi; idx < v_hi * (D / 4); idx += 256) {
         const int kh = idx / (D / 4), d = (idx % (D / 4)) * 4;
         if (slot >= 0) {
-            float4 v = idx == vi ? v0 : *(const float4*)(vr + kh * D + d);
+            float4 v = v0;
+            if (!AHEAD || idx != vi) v = *(const float4*)(vr + kh * D + d);
             if (HAS_BIAS) {
                 const float4 b = *(const float4*)(bias + (Hq + Hkv) * D + kh * D + d);
                 v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w;
@@ -271,13 +278,15 @@ extern "C" int mxk_rope_kv(float* qkv, const float* bias, const int* pos, const 
     const dim3 grid(T, ng);
     if (rot_dim == D && (D == 64 || D == 128) && !(((uintptr_t)qkv) & 15) && !(((uintptr_t)bias) & 15) &&
         (!qkn || (!(((uintptr_t)qn) & 15) && !(((uintptr_t)kn) & 15)))) {
-#define RK4(D_, N_, B_, Z_, K8_)                                                                                         \
-    do {                                                                                                                 \
-        if (qkn) rope_kv4_kernel<D_, N_, B_, Z_, K8_, true><<<grid, 256, 0, st>>>(qkv, bias, pos, slots, inv_freq,       \
-                                                                                  attn_factor, Hq, Hkv, qo, kc, vc,      \
-                                                                                  block_size, qn, kn, eps);              \
-        else rope_kv4_kernel<D_, N_, B_, Z_, K8_><<<grid, 256, 0, st>>>(qkv, bias, pos, slots, inv_freq, attn_factor,    \
-                                                                        Hq, Hkv, qo, kc, vc, block_size);                \
+        const bool ahead = T <= 2048 && (Hkv + ng - 1) / ng * (D / 4) <= 256;
+#define RK4A(D_, N_, B_, Z_, K8_, Q_, A_)                                                                                 \
+    rope_kv4_kernel<D_, N_, B_, Z_, K8_, Q_, A_><<<grid, 256, 0, st>>>(qkv, bias, pos, slots, inv_freq, attn_factor, Hq, Hkv, qo, kc, vc, block_size, qn, kn, eps)
+#define RK4(D_, N_, B_, Z_, K8_)                             \
+    do {                                                     \
+        if (qkn && ahead) RK4A(D_, N_, B_, Z_, K8_, true, true);   \
+        else if (qkn) RK4A(D_, N_, B_, Z_, K8_, true, false);      \
+        else if (ahead) RK4A(D_, N_, B_, Z_, K8_, false, true);    \
+        else RK4A(D_, N_, B_, Z_, K8_, false, false);              \
     } while (0)
 #define RK4F(D_, N_, B_, Z_)                              \
     {                                                     \
@@ -293,6 +302,7 @@ extern "C" int mxk_rope_kv(float* qkv, const float* bias, const int* pos, const 
 #undef RK4Z
 #undef RK4F
 #undef RK4
+#undef RK4A
         MXK_CHECK_LAUNCH();
     }
 #define RKZ(N_, B_, Q_, K8_) { if (zero_after) rope_kv_kernel<N_, B_, Q_, true, K8_><<<grid, 256, 0, st>>>(qkv, bias, pos, slots, inv_freq, attn_factor, Hq, Hkv, D, rot_dim, qo, kc, vc, block_size, qn, kn, eps); \

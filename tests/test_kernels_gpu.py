@@ -196,6 +196,31 @@ def test_rope_kv(neox, D, rot, qkn):
         assert rel(b, a) < 1e-2
 
 
+@pytest.mark.parametrize("T,Hq,Hkv,D", [(2049, 4, 2, 128), (2050, 4, 2, 64), (600, 16, 16, 128), (513, 33, 33, 64)])
+@pytest.mark.parametrize("neox,zero,qkn", [(False, False, False), (True, True, False), (False, True, True), (True, False, True)])
+def test_rope_kv_of_many_rows_and_value_heads(T, Hq, Hkv, D, neox, zero, qkn):
+    """Rows whose slot and values are read behind the rotation's table, against the same rows in calls of 100 whose are read ahead of it: the same
+    arithmetic, the same bits, in each cache format that the kernel stores itself."""
+    nb, bs = -(-T // 16) + 1, 16
+    qkv, pos, slots = (t.to(DEV) for t in _rope_setup(T, Hq, Hkv, D, nb, bs))
+    bias = (torch.randn((Hq + 2 * Hkv) * D) * 0.1).to(DEV) if zero else None
+    inv, af = K.rope_inv_freq(D, 500000.0)
+    w = (1 + 0.3 * torch.randn(D)).to(DEV)
+    for dt, cols in ((torch.bfloat16, D), (torch.float8_e4m3fn, D), (torch.uint8, D + D // 16)):
+        got = []
+        for step in (T, 100):
+            x, q = qkv.clone(), torch.zeros(T, Hq, D, dtype=torch.bfloat16, device=DEV)
+            kc, vc = torch.zeros(nb, Hkv, bs, cols, device=DEV).to(dt), torch.zeros(nb, Hkv, bs, cols, device=DEV).to(dt)
+            if dt == torch.uint8:
+                kc.kvf = vc.kvf = 2
+            for i in range(0, T, step):
+                K.rope_kv(x[i:i + step], bias, pos[i:i + step], slots[i:i + step], inv.to(DEV), af, Hq, Hkv, D, D, neox, q[i:i + step], kc, vc, bs,
+                          qk_norm=(w, w, 1e-6) if qkn else None, zero_after=zero)
+            assert torch.equal(x, torch.zeros_like(x) if zero else qkv)
+            got.append([t.view(torch.uint8) for t in (q, kc, vc)])
+        assert all(torch.equal(a, b) for a, b in zip(*got)) and got[0][2].any()
+
+
 def _paged_kv(nb, Hkv, bs, D, seed):
     g = torch.Generator().manual_seed(seed)
     kc = (torch.randn(nb, Hkv, bs, D, generator=g)).bfloat16()
