@@ -497,8 +497,9 @@ int enc_ln_gemm(int np, const float* parts, const uint16_t* pbias, const uint16_
     if (M <= GW * RW_) {                     \
         if (K <= 512 && np == 1) EL(RW_, 1, 1); \
         if (K <= 512) EL(RW_, 1, MP);        \
-        if (np == 1) EL(RW_, 2, 1);          \
-        EL(RW_, 2, MP);                      \
+        if constexpr (RW_ == 1 || OUT == ENC_ACT) /* (9 to 16 rows so wide are one text's, whose output product has two parts) */ \
+            if (np == 1) EL(RW_, 2, 1);      \
+        if (np == MP) EL(RW_, 2, MP);        \
     }
     constexpr int MP = OUT == ENC_ACT ? enc_parts(1 << 20) : 2;  // behind the down product; behind the output product of heads' parts up to 16 rows
     if ((np != 1 && np != MP) || K > 1024) return (int)hipErrorInvalidValue;

@@ -233,6 +233,19 @@ def test_few_rows_with_norms_and_attention_inside_the_products(hidden, heads, ff
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("hidden,heads,ffn", [(512, 8, 2048), (576, 9, 2080), (1024, 16, 2048), (1024, 8, 160)])
+def test_norms_of_several_texts(hidden, heads, ffn):
+    """Norms inside the products of several texts: up to 16 rows of 512 columns, up to 8 beyond; apart from there on. The bound of
+    test_packed_rows_match_fp32."""
+    cfg = BM.BertConfig(vocab=400, hidden=hidden, n_layers=3, n_heads=heads, ffn=ffn, max_pos=64, name="t")
+    get = BM.synthetic_bert(cfg, 5)
+    g, c = BM.BertModel.load(cfg, get, "cuda:0"), BM.BertModel.load(cfg, get, "cpu")
+    for lens in ([1, 1], [3, 5], [0, 7], [4, 5], [7, 1, 8], [9, 8]):
+        ids = [list(range(10, 10 + n)) for n in lens]
+        assert (g.embed(ids).cpu() - c.embed(ids)).abs().max() < 5e-3, lens
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("pooling", ["mean", "cls", "last"])
 def test_empty_texts_match_the_padded_batch(pooling):
     """An empty text has a row too: nothing for the mean, its first row, or the batch's last position."""
