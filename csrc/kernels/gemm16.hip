@@ -153,7 +153,6 @@ __global__ __launch_bounds__(256) void t32_expand_kernel(const uint8_t* __restri
     }
     auto tile = [&](auto q_c) {
         constexpr int Q = decltype(q_c)::value;
-        b[Q].template prep<Q>();
         *(f16x8*)(o + 64 * Q) = b[Q].template frag<Q, 0>();
         *(f16x8*)(o + 64 * Q + 16) = b[Q].template frag<Q, 1>();
         *(f16x8*)(o + 64 * Q + 32) = b[Q].template frag<Q, 2>();

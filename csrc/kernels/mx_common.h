@@ -39,6 +39,17 @@ MX_DEV void mx_lds_dma4(const void* g, const MX_LDS void* lds) {
     asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "{m0}"(m0) : "memory");
 }
 
+// the same from a wave-uniform base and a 32-bit byte offset a lane: no 64-bit vector addition for each. `m0`: uniform LDS address.
+MX_DEV uint32_t mx_lds_addr(const void* p) { return (uint32_t)(uintptr_t)(const MX_LDS char*)p; }
+MX_DEV void mx_lds_dma16(const void* base, uint32_t off, uint32_t m0) {
+    m0 = __builtin_amdgcn_readfirstlane(m0);
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(m0) : "memory");
+}
+MX_DEV void mx_lds_dma4(const void* base, uint32_t off, uint32_t m0) {
+    m0 = __builtin_amdgcn_readfirstlane(m0);
+    asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "{m0}"(m0) : "memory");
+}
+
 MX_DEV float bf16_to_f32(bf16_t v) { return __uint_as_float(((uint32_t)v) << 16); }
 
 // round-to-nearest-even; NaN stays NaN (the plain cast lowers to v_cvt_pk_bf16_f32 on gfx950).

@@ -27,19 +27,6 @@
 // Reference parity: llama.cpp's MMQ path for these formats (reached via backend/cpp/llama/grpc-server.cpp:2002
 // llama_decode); numerics = f16 dequantised weights x f16 activations, fp32 accumulation.
 #include "qmm2_impl.h"
-int g_qmm2_rot = 0;
-
-extern "C" int mxk_qmm2_set_rot(int r) {
-    g_qmm2_rot = r;
-    return 0;
-}
-
-// isolation builds of the Q4_K SwiGLU kernel ((wm, ks, wn) = (8, 1, 1), (4, 2, 1), (4, 1, 2), (2, 2, 2); no split),
-// see DBG above
-extern "C" int mxk_qmm2_dbg(int dbg, int wm, int ks, int wn, const uint16_t* A, int lda, const uint8_t* W, int M, int N,
-                            int K, void* C, int ldc, hipStream_t st) {
-    return qmm2_dbg_q4k(dbg, wm, ks, wn, A, lda, W, M, N, K, C, ldc, st);
-}
 
 // A f16 [M, K] (lda % 8 == 0, 16-B aligned), W t32 Q4_K / Q5_K / Q6_K / Q3_K / Q2_K / Q8_0 / MX4F / MX5F [N, K] (N % 32 == 0, K % 256 == 0).
 // epi: 0 fp32 store, 1 f16 store, 2 fp32 accumulate (split-K via atomics when splits > 1), 3/4 SwiGLU /

@@ -2,8 +2,6 @@
 #pragma once
 #include "qmm2_fmt.h"
 
-extern int g_qmm2_rot;  // k-order rotation multiplier per column tile (0: natural order), mxk_qmm2_set_rot
-
 // RMSNorm fused across two GEMMs (M > 4 dense layers: o_proj -> gate|up, down -> next qkv). rmsnorm(x) W^T =
 // diag(1 / rms(x)) ((x * g) W^T), so the norm splits into
 //   mode 1, the producer (E16_ADD_F32 into the fp32 residual): once a 32-row x 32-column block of the residual is
@@ -86,7 +84,7 @@ struct Q2Geom {
     static constexpr int A_BYTES = BM * 128;          // one 64-k tile of A
     static constexpr int STAGE = A_BYTES + NG * F::QB; // A + the column groups' quant bytes
     static constexpr int HSZ = NG * F::HB;            // one super-block header slot (NG groups)
-    static constexpr int NH = NS >= 6 ? 3 : 2;         // header slots: super-blocks live at once (stages kt .. kt+NS-1)
+    static constexpr int NH = 2;                      // header slots (a wave keeps the header of its super-block in registers)
     static constexpr int LDS = NS * STAGE + NH * HSZ;
     // A LDS-DMA instructions per wave per stage (rounded up: with BM / 8 not a multiple of NT the last wave's spare
     // instructions re-load the tile's last 8-row block into its own slot, identical bytes)
@@ -98,9 +96,15 @@ struct Q2Geom {
 };
 
 
-// per-k-step issue schedule: each MFMA followed by one LDS read (the first NDS) and up to NV VALU, so the next
-// k-step's fragment reads leave early and the dequant VALU fills the MFMA shadows
-constexpr int Q2_VPM = 5;
+template <int I, int N, class FN>
+MX_DEV void q2_static_for(FN&& fn) {
+    if constexpr (I < N) {
+        fn(std::integral_constant<int, I>{});
+        q2_static_for<I + 1, N>(fn);
+    }
+}
+
+// four-wave tiles, one wave a SIMD: each product followed by one LDS read (the first NDS) and up to NV vector instructions
 template <int I, int NM, int NDS, int NV>
 MX_DEV void q2_interleave() {
     if constexpr (I < NM) {
@@ -108,22 +112,6 @@ MX_DEV void q2_interleave() {
         if constexpr (I < NDS) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         __builtin_amdgcn_sched_group_barrier(0x002, NV, 0);
         q2_interleave<I + 1, NM, NDS, NV>();
-    }
-}
-
-// Q2_AEARLY 1: the next k-step's A fragments are read at the TOP of a k-step (all WM reads back to back, then the
-// k-step's MFMAs with the dequant VALU in their shadows) instead of one read after each MFMA (0, default). Same-box
-// A/B with the asm LDS-DMA (counted lgkmcnt waits either way): within 1 % on every projection, and 0 needs 20
-// fewer VGPRs (profiles/r6_qmm2_asm_dma.md)
-#ifndef Q2_AEARLY
-#define Q2_AEARLY 0
-#endif
-template <int I, int NM, int NV>
-MX_DEV void q2_interleave_mfma() {
-    if constexpr (I < NM) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, NV, 0);
-        q2_interleave_mfma<I + 1, NM, NV>();
     }
 }
 
@@ -155,13 +143,12 @@ struct Q2Group {
 };
 
 
-// DBG (isolation builds, tools/prof_qmm.py --q2dbg): 1 no MFMA, 2 no dequant VALU, 4 no A loads, 8 no weight loads
-template <int QT, int WM, int KS, int WN, int EPI, int DBG = 0, int NS = 4, int NG = 4, int GPW = 1, bool GR = false,
+template <int QT, int WM, int KS, int WN, int EPI, int NS = 4, int NG = 4, int GPW = 1, bool GR = false,
           bool FU = false>
 __global__ __launch_bounds__(NG == 8 ? 512 / GPW : 256 * KS) void qmm2_kernel(const uint16_t* __restrict__ A, int lda,
                                                         const uint8_t* __restrict__ W, int M, int N, int K,
                                                         int n_mt, int splits, int sbps, void* __restrict__ Cv,
-                                                        int ldc, int rot_mul, Q2Group grp, Q2Fuse fu = Q2Fuse{}) {
+                                                        int ldc, Q2Group grp, Q2Fuse fu = Q2Fuse{}) {
     using G = Q2Geom<QT, WM, KS, WN, NS, NG, GPW>;
     using F = Q2F<QT>;
     constexpr int BM = G::BM, WA = G::WA, STAGE = G::STAGE, A_BYTES = G::A_BYTES;
@@ -171,15 +158,10 @@ __global__ __launch_bounds__(NG == 8 ? 512 / GPW : 256 * KS) void qmm2_kernel(co
     static_assert(WA >= 1 && WA * 8 * G::NT >= BM && (WA - 1) * 8 * G::NT < BM, "A tile split");
     static_assert(G::LDS <= 160 * 1024, "LDS");
     static_assert((NS - 2) * G::template cnt<0, true>() <= 63, "vmcnt range");
-    // LDS-DMA instructions per stage as issued (the isolation builds drop some)
-    constexpr int WAI = (DBG & 4) ? 0 : WA, QII = (DBG & 8) ? 0 : GPW * F::QI, HII = (DBG & 8) ? 0 : GPW * F::HI;
-    auto cnt = [](auto jq_c, auto wl_c) constexpr {
-        return WAI + (decltype(wl_c)::value ? QII + (decltype(jq_c)::value == 0 ? HII : 0) : 0);
-    };
+    constexpr int QII = GPW * F::QI, HII = GPW * F::HI;  // LDS-DMA instructions of a stage's weights
     extern __shared__ __attribute__((aligned(16))) char smem[];
     char* const hdr_lds = smem + NS * STAGE;
-    // ring slot of k-tile ki = ki % NS; header slot of super-block v = v % NH
-    auto hslot_of = [](int v) { return G::NH == 3 ? v % 3 : v & 1; };
+    // ring slot of k-tile ki = ki % NS; header slot of super-block v = v & 1
 
     // wave index as a scalar: every LDS-DMA destination (M0) and weight pointer below is then SGPR math
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -238,7 +220,7 @@ __global__ __launch_bounds__(NG == 8 ? 512 / GPW : 256 * KS) void qmm2_kernel(co
         if constexpr (GR) {
             if (grp.stok) row = grp.stok[row];
         }
-        aoff[i] = (uint32_t)(row * lda + 16 * s + 8 * hh);
+        aoff[i] = 2 * (uint32_t)(row * lda + 16 * s + 8 * hh);
     }
     // per-lane fragment read bases (byte offsets within a stage)
     const int rb = col >> 3;
@@ -246,23 +228,23 @@ __global__ __launch_bounds__(NG == 8 ? 512 / GPW : 256 * KS) void qmm2_kernel(co
     const uint32_t b_rd = (uint32_t)(A_BYTES + nw * WN * F::QB);  // + j * QB for the wave's group j
     const int hg = nw * WN * F::HB;                                 // header offset of group nw * WN
 
-    // stage issue: the A rows of k-tile `kta` and (weight waves) the quant bytes of super-block `sbw`,
-    // quarter JQ, into ring slot `slot`; JQ == 0 stages also bring that super-block's header into header slot
-    // `hslot`. Dummy stages past the end pass clamped (valid, never consumed) sources.
-    auto issue = [&](int kta, int sbw, int slot, int hslot, auto jq_c, auto wl_c) {
-        constexpr int JQ = decltype(jq_c)::value;
-        char* sb = smem + slot * STAGE;
-        const uint16_t* ak = A + (size_t)kta * 64;
-#pragma unroll
-        for (int i = 0; i < WAI; ++i)
-            q2_dma((const void*)(ak + aoff[i]), (MX_LDS void*)(sb + min(wave * WA + i, BM / 8 - 1) * 1024), 16);
-        if constexpr (decltype(wl_c)::value && QII > 0) {
-            const uint8_t* u = wg + (size_t)sbw * F::UNIT;
-            q2_stage_weights<QT, JQ>(u, sb + A_BYTES + GPW * cg * F::QB, hdr_lds + hslot * G::HSZ + GPW * cg * F::HB,
-                                     lane);
-            if constexpr (GPW == 2)
-                q2_stage_weights<QT, JQ>(wg2 + (size_t)sbw * F::UNIT, sb + A_BYTES + (2 * cg + 1) * F::QB,
-                                         hdr_lds + hslot * G::HSZ + (2 * cg + 1) * F::HB, lane);
+    const uint32_t ring = mx_lds_addr(smem), hring = ring + NS * STAGE;
+    // a stage's issue: the A rows of a k-tile and (weight waves) its quant bytes into a ring slot; stages of a super-block's
+    // first quarter also bring its header into a header slot. In WA + 1 pieces: an A instruction each, then the weights'.
+    struct Stage {
+        const uint16_t* a;
+        const uint8_t* u;
+        const uint8_t* u2;
+        uint32_t lds, hd;
+    };
+    auto issue = [&](const Stage& st, auto d_c, auto jq_c) {
+        constexpr int D = decltype(d_c)::value, JQ = decltype(jq_c)::value;
+        if constexpr (D < WA) {
+            mx_lds_dma16(st.a, aoff[D], st.lds + min(wave * WA + D, BM / 8 - 1) * 1024);
+        } else {
+            const uint32_t qd = st.lds + A_BYTES + GPW * cg * F::QB, hd = st.hd + GPW * cg * F::HB;
+            q2_stage_weights<QT, JQ>(st.u, qd, hd, lane);
+            if constexpr (GPW == 2) q2_stage_weights<QT, JQ>(st.u2, qd + F::QB, hd + F::HB, lane);
         }
     };
 
@@ -282,23 +264,26 @@ __global__ __launch_bounds__(NG == 8 ? 512 / GPW : 256 * KS) void qmm2_kernel(co
         using I1 = std::integral_constant<int, 1>;
         using I2 = std::integral_constant<int, 2>;
         using I3 = std::integral_constant<int, 3>;
-        // the split's super-blocks are visited in a rotated order (v -> sb0 + (v + rot) % nv): workgroups that
-        // run side by side on one XCD (consecutive column tiles) then stream different k ranges of the shared
-        // A rows instead of all hitting the same 128-B lines (and L2 channels) at the same time
         const int nv = sb1 - sb0;
-        const int rot = rot_mul ? (int)(((unsigned)ct * (unsigned)rot_mul) % (unsigned)nv) : 0;
-        auto phys = [&](int v) {
-            int p = v + rot;
-            if (p >= nv) p -= nv;
-            return sb0 + p;
-        };
-        // stage ki of the virtual k-tile sequence (ki & 3 == KI & 3, compile-time): past the split's end a dummy
-        // stage re-reads the last real super-block's tile 3 (valid addresses, never consumed)
-        auto issue_stage = [&](int ki, auto jq_c) {
+        // ring offset of a k-tile's slot, moved on tile by tile (with four slots it is the compiler's to know)
+        auto next_slot = [](uint32_t o) { return o == (NS - 1) * STAGE ? 0u : o + STAGE; };
+        // stage ki of the split's k-tiles (ki & 3 == JQ: its quarter) at ring offset `so`; past the split's end a dummy stage
+        // re-reads the last k-tile's rows and the last super-block's weights (valid addresses, never consumed)
+        auto stage = [&](int ki, uint32_t so) {
             const int vi = ki >> 2;
-            const bool real = vi < nv;
-            const int ps = phys(real ? vi : nv - 1);
-            issue(ps * 4 + (real ? (ki & 3) : 3), ps, ki % NS, hslot_of(vi), jq_c, WLc{});
+            Stage st;
+            st.a = A + (size_t)(uint32_t)(sb0 * 4 + min(ki, nv * 4 - 1)) * 64;
+            const uint8_t* const u = wg + (size_t)(uint32_t)(sb0 + min(vi, nv - 1)) * F::UNIT;
+            st.u = u;
+            st.u2 = GPW == 2 ? u + (wg2 - wg) : nullptr;
+            st.lds = ring + so;
+            st.hd = hring + (vi & 1) * G::HSZ;
+            return st;
+        };
+        constexpr int ND = WA + (WL ? 1 : 0);  // pieces of a stage's issue
+        auto issue_stage = [&](int ki, auto jq_c) {
+            const Stage st = stage(ki, ki * STAGE);
+            q2_static_for<0, ND>([&](auto d_c) { issue(st, d_c, jq_c); });
         };
         // prologue: stages 0 .. NS - 2, then stage 0 landed
         issue_stage(0, I0{});
@@ -308,98 +293,104 @@ __global__ __launch_bounds__(NG == 8 ? 512 / GPW : 256 * KS) void qmm2_kernel(co
         if constexpr (NS >= 6) issue_stage(4, I0{});
         if constexpr (NS >= 7) issue_stage(5, I1{});
         if constexpr (NS >= 8) issue_stage(6, I2{});
-        q2_wait_barrier<q2_cnt_run<WAI, QII, HII, WL, 1, NS - 2>()>();
+        q2_wait_barrier<q2_cnt_run<WA, QII, HII, WL, 1, NS - 2>()>();
 
-        // fragment producers (S is a compile-time constant after unrolling)
-        auto bfrag = [&](const Q2B<QT>& b, auto jq_c, int S) -> f16x8 {
-            constexpr int JQ_ = decltype(jq_c)::value;
-            if constexpr (DBG & 2) {
-                const u32x2 r2 = (S & 1) ? b.v1 : b.v0;
-                return __builtin_bit_cast(f16x8, (u32x4){r2[0], r2[1], r2[0] ^ (uint32_t)S, r2[1]});
-            } else {
-                switch (S) {
-                    case 0: return b.template frag<JQ_, 0>();
-                    case 1: return b.template frag<JQ_, 1>();
-                    case 2: return b.template frag<JQ_, 2>();
-                    default: return b.template frag<JQ_, 3>();
-                }
-            }
-        };
+        constexpr int S0 = 2 * KH, S1 = KS == 1 ? 3 : S0 + 1;  // the wave's k-steps of a k-tile: a 32-k sub-block, or both
         Q2B<QT> bw[WN];
         f16x8 af[2][WM], bfc[WN];
 #pragma unroll
         for (int j = 0; j < WN; ++j) {
             bw[j].load_hdr(hdr_lds + hg + j * F::HB, col, h);
             bw[j].load_q(smem + b_rd + j * F::QB, col, h);
-            bw[j].template prep<0>();
-            bfc[j] = bfrag(bw[j], I0{}, KH);
+            bfc[j] = bw[j].template frag<0, S0>();
         }
 #pragma unroll
-        for (int i = 0; i < WM; ++i) af[0][i] = *(const f16x8*)(smem + a_rd + i * 4096 + KH * 256);
+        for (int i = 0; i < WM; ++i) af[0][i] = *(const f16x8*)(smem + a_rd + i * 4096 + S0 * 256);
 
-        // one k-tile (ring slot JQ): the wave's k-steps KH, KH + KS, ...; software-pipelined one k-step deep:
-        // k-step S's MFMAs consume A / B fragments read and dequantised during k-step S - KS, while this
-        // k-step reads and dequantises those of the next one (on the last k-step: the next tile's first, from
-        // ring slot JQ + 1, landed at the top). An explicit per-k-step schedule (q2_interleave) keeps the
-        // compiler from sinking the LDS reads next to their MFMAs, which stalled every k-step on lgkmcnt(0).
-        auto tile = [&](int sb, auto jq_c) {  // sb: virtual super-block index
+        // one k-tile (ring slot JQ): the wave's k-steps S0 .. S1; software-pipelined one k-step deep: a k-step's products
+        // consume A / B fragments read and dequantised during the step before, while this one reads and dequantises those
+        // of the next (on the last k-step: the next tile's first, from ring slot JQ + 1, landed at the top).
+        // Two waves a SIMD (SPREAD): the order is the source's. A wave issues one vector instruction in eight cycles (the SIMD one in
+        // four), so these tiles are bound by the instructions a wave has a k-tile, and what is not spread between the products
+        // is not hidden behind them: the dequantisation in pieces of five or six instructions, the reads where a fragment's
+        // registers are free, and the stage's issue, since a compute unit's 24 to 40 LDS-DMA instructions at once hold its waves at
+        // the address unit for 16 cycles each. 128 x 128 tiles, a wave's instructions a k-tile 100 -> 76: q|k 6144 x 4096 at 416 rows
+        // 32.9 -> 30.4 us, 4096 x 14336 67.7 -> 63.7, 4096 x 4096 at 64-row tiles 25.4 -> 23.4, gate|up 28672 x 4096 at 128 rows 45.5 -> 40.0.
+        // (A ring of six slots, whose addresses are no constants, takes ten instructions more and 20 % longer.)
+        // One wave a SIMD has no other to fill its gaps and is better off with the compiler's order under q2_interleave (34.9 us
+        // against 41.9 on the first of these).
+        constexpr bool SPREAD = G::NT > 4;
+        uint32_t o_cs = 0, o_is = (NS - 1) * STAGE;
+        auto tile = [&](int sb, auto jq_c) {  // sb: super-block index in the split
             constexpr int JQ = decltype(jq_c)::value;
             constexpr int NJ = (JQ + 1) & 3;
             const int kt = sb * 4 + JQ;
-            const int cs = kt % NS, ns = (kt + 1) % NS;  // ring slots of this tile and the next
+            // ring offsets of this tile, the next and the stage issued here
+            const uint32_t cs = NS == 4 ? JQ * STAGE : o_cs, ns = NS == 4 ? NJ * STAGE : next_slot(cs);
+            const uint32_t is = NS == 4 ? ((JQ + 3) & 3) * STAGE : o_is;
+            if constexpr (NS != 4) {
+                o_cs = ns;
+                o_is = next_slot(is);
+            }
             // stage kt+1 landed (stages kt+2 .. kt+NS-2 may still be in flight); every wave is past tile kt-1
-            q2_wait_barrier<q2_cnt_run<WAI, QII, HII, WL, (JQ + 2) & 3, NS - 3>()>();
-            issue_stage(kt + NS - 1, std::integral_constant<int, (JQ + NS - 1) & 3>{});
+            q2_wait_barrier<q2_cnt_run<WA, QII, HII, WL, (JQ + 2) & 3, NS - 3>()>();
+            const Stage st = stage(kt + NS - 1, is);
+            if constexpr (!SPREAD)
+                q2_static_for<0, ND>([&](auto d_c) { issue(st, d_c, std::integral_constant<int, (JQ + NS - 1) & 3>{}); });
             // the next tile's quant bytes (and, at a super-block edge, header): slot NJ landed at the wait above
             Q2B<QT> bn[WN];
 #pragma unroll
             for (int j = 0; j < WN; ++j) {
                 bn[j] = bw[j];
-                if constexpr (NJ == 0) bn[j].load_hdr(hdr_lds + hslot_of(sb + 1) * G::HSZ + hg + j * F::HB, col, h);
-                bn[j].load_q(smem + ns * STAGE + b_rd + j * F::QB, col, h);
+                if constexpr (NJ == 0) bn[j].load_hdr(hdr_lds + ((sb + 1) & 1) * G::HSZ + hg + j * F::HB, col, h);
+                bn[j].load_q(smem + ns + b_rd + j * F::QB, col, h);
             }
-            constexpr int NSTEP = 4 / KS;
-#pragma unroll
-            for (int t = 0; t < NSTEP; ++t) {
+            q2_static_for<S0, S1 + 1>([&](auto s_c) {
+                constexpr int S = decltype(s_c)::value, cur = S & 1;
+                constexpr bool LAST = S == S1;
+                constexpr int SN = LAST ? S0 : S + 1, JN = LAST ? NJ : JQ;  // the fragments made here
+                const char* an = smem + (LAST ? ns : cs) + a_rd + SN * 256;
+                u32x4 bfn[WN];
+                auto piece = [&](auto u_c) {
+                    constexpr int j = decltype(u_c)::value / 3, u = decltype(u_c)::value % 3;
+                    Q2B<QT>& w = LAST ? bn[j] : bw[j];
+                    if constexpr (u == 0) {
+                        w.template prep<JN, SN>();
+                    } else {
+                        const u32x2 x = w.template half<JN, SN, u - 1>();
+                        bfn[j][2 * (u - 1)] = x[0];
+                        bfn[j][2 * (u - 1) + 1] = x[1];
+                    }
+                };
+                constexpr int NM = WM * WN, NP = 3 * WN;  // products and pieces of this step, and the stage's pieces in it
+                constexpr int NSTEP = S1 - S0 + 1, D0 = ND * (S - S0) / NSTEP, D1 = ND * (S - S0 + 1) / NSTEP;
                 __builtin_amdgcn_sched_barrier(0);
-                const int S = KH + KS * t;  // compile-time after unrolling
-                const int cur = t & 1;
-                f16x8 bfn[WN];
-                if (t + 1 < NSTEP) {
-#pragma unroll
-                    for (int i = 0; i < WM; ++i)
-                        af[cur ^ 1][i] = *(const f16x8*)(smem + cs * STAGE + a_rd + i * 4096 + (S + KS) * 256);
-#pragma unroll
-                    for (int j = 0; j < WN; ++j) bfn[j] = bfrag(bw[j], jq_c, S + KS);
+                if constexpr (SPREAD) {
+                    q2_static_for<0, NM>([&](auto m_c) {
+                        constexpr int m = decltype(m_c)::value, i = m / WN, j = m % WN;
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[cur][i], bfc[j], acc[i][j], 0, 0, 0);
+                        if constexpr (j == WN - 1) af[cur ^ 1][i] = *(const f16x8*)(an + i * 4096);
+                        __builtin_amdgcn_sched_barrier(0);
+                        q2_static_for<m * NP / NM, (m + 1) * NP / NM>(piece);
+                        q2_static_for<D0 + (D1 - D0) * m / NM, D0 + (D1 - D0) * (m + 1) / NM>(
+                            [&](auto d_c) { issue(st, d_c, std::integral_constant<int, (JQ + NS - 1) & 3>{}); });
+                        __builtin_amdgcn_sched_barrier(0);
+                    });
                 } else {
 #pragma unroll
-                    for (int i = 0; i < WM; ++i)
-                        af[cur ^ 1][i] = *(const f16x8*)(smem + ns * STAGE + a_rd + i * 4096 + KH * 256);
+                    for (int i = 0; i < WM; ++i) af[cur ^ 1][i] = *(const f16x8*)(an + i * 4096);
+                    q2_static_for<0, NP>(piece);
 #pragma unroll
-                    for (int j = 0; j < WN; ++j) {
-                        bn[j].template prep<NJ>();
-                        bfn[j] = bfrag(bn[j], std::integral_constant<int, NJ>{}, KH);
-                    }
+                    for (int j = 0; j < WN; ++j)
+#pragma unroll
+                        for (int i = 0; i < WM; ++i)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[cur][i], bfc[j], acc[i][j], 0, 0, 0);
+                    q2_interleave<0, NM, WM, 5>();
                 }
 #pragma unroll
-                for (int j = 0; j < WN; ++j)
-#pragma unroll
-                    for (int i = 0; i < WM; ++i) {
-                        if constexpr (DBG & 1) asm volatile("" ::"v"(af[cur][i]), "v"(bfc[j]));
-                        else acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[cur][i], bfc[j], acc[i][j], 0, 0, 0);
-                    }
-                if constexpr (!(DBG & 1)) {
-                    if constexpr (Q2_AEARLY) {
-                        __builtin_amdgcn_sched_group_barrier(0x100, WM, 0);  // the next k-step's A reads first
-                        q2_interleave_mfma<0, WM * WN, Q2_VPM>();
-                    } else {
-                        q2_interleave<0, WM * WN, WM, Q2_VPM>();
-                    }
-                }
-#pragma unroll
-                for (int j = 0; j < WN; ++j) bfc[j] = bfn[j];
-            }
-            // NSTEP is even: the next tile's first fragments are in af[0]
+                for (int j = 0; j < WN; ++j) bfc[j] = __builtin_bit_cast(f16x8, bfn[j]);
+            });
+            // S1 is odd: the next tile's first fragments are in af[0]
 #pragma unroll
             for (int j = 0; j < WN; ++j) bw[j] = bn[j];
         };
@@ -560,17 +551,23 @@ __global__ __launch_bounds__(NG == 8 ? 512 / GPW : 256 * KS) void qmm2_kernel(co
             continue;
         }
         if constexpr (EPI == E16_SWIGLU || EPI == E16_GEGLU) {
-            // W rows interleaved in 16-row groups: tile columns 0..15 gate, 16..31 up of the same features
+            // W rows interleaved in 16-row groups: tile columns 0..15 gate, 16..31 up of the same features. Two rows' values
+            // trade their halves, after which one register holds both rows' gates and the other their ups: every lane
+            // has an output of its own (16 lanes' shuffles and half the lanes idle took 10-18 % of a 200-row GEMM)
 #pragma unroll
-            for (int i = 0; i < WM; ++i)
+            for (int i = 0; i < WM; ++i) {
+                if (mb + i * 32 >= M) break;
+                uint16_t* const cr = (uint16_t*)Cv + (size_t)(mb + i * 32 + 4 * h + (col >> 4)) * ldc + (nt >> 1) + (col & 15);
+                const bool full = mb + i * 32 + 32 <= M;
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const float v = acc[i][j][r];
-                    const float up = __shfl_xor(v, 16);
-                    const int m = mb + i * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-                    if (col < 16 && m < M)
-                        ((uint16_t*)Cv)[(size_t)m * ldc + (nt >> 1) + col] = f32_to_act<true>(glu_gate_f<EPI>(v) * up);
+                for (int r = 0; r < 16; r += 2) {
+                    const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[i][j][r]), __float_as_uint(acc[i][j][r + 1]),
+                                                                    false, false);
+                    const uint16_t o = f32_to_act<true>(glu_gate_f<EPI>(__uint_as_float(x[0])) * __uint_as_float(x[1]));
+                    const int rr = 8 * (r >> 2) + (r & 3);
+                    if (full || mb + i * 32 + 4 * h + (col >> 4) + rr < M) cr[(size_t)rr * ldc] = o;
                 }
+            }
             continue;
         }
 #pragma unroll
@@ -689,12 +686,12 @@ static int launch_qmm2(const uint16_t* A, int lda, const uint8_t* W, int M, int 
     if (nwg <= 0 || nwg > 0x7fffffff) return (int)hipErrorInvalidValue;
     static bool attr_set = false;
     if (!attr_set) {
-        (void)hipFuncSetAttribute((const void*)qmm2_kernel<QT, WM, KS, WN, EPI, 0, NS, NG, GPW, false, FU>,
+        (void)hipFuncSetAttribute((const void*)qmm2_kernel<QT, WM, KS, WN, EPI, NS, NG, GPW, false, FU>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS);
         attr_set = true;
     }
-    qmm2_kernel<QT, WM, KS, WN, EPI, 0, NS, NG, GPW, false, FU><<<dim3((unsigned)nwg), 64 * G::NT, G::LDS, st>>>(
-        A, lda, W, M, N, K, n_mt, splits, sbps, C, ldc, g_qmm2_rot, Q2Group{}, fu);
+    qmm2_kernel<QT, WM, KS, WN, EPI, NS, NG, GPW, false, FU><<<dim3((unsigned)nwg), 64 * G::NT, G::LDS, st>>>(
+        A, lda, W, M, N, K, n_mt, splits, sbps, C, ldc, Q2Group{}, fu);
     MXK_CHECK_LAUNCH();
 }
 
@@ -710,12 +707,12 @@ static int launch_qmm2_grouped(const uint16_t* A, int lda, const int* stok, cons
     if (nwg <= 0 || nwg > 0x7fffffff) return (int)hipErrorInvalidValue;
     static bool attr_set = false;
     if (!attr_set) {
-        (void)hipFuncSetAttribute((const void*)qmm2_kernel<QT, WM, KS, 1, EPI, 0, 4, 4, 1, true>,
+        (void)hipFuncSetAttribute((const void*)qmm2_kernel<QT, WM, KS, 1, EPI, 4, 4, 1, true>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS);
         attr_set = true;
     }
-    qmm2_kernel<QT, WM, KS, 1, EPI, 0, 4, 4, 1, true><<<dim3((unsigned)nwg), 64 * G::NT, G::LDS, st>>>(
-        A, lda, W, P, N, K, n_mt, 1, K >> 8, C, ldc, 0, Q2Group{tiles, off, stok, E, otok, owt}, Q2Fuse{});
+    qmm2_kernel<QT, WM, KS, 1, EPI, 4, 4, 1, true><<<dim3((unsigned)nwg), 64 * G::NT, G::LDS, st>>>(
+        A, lda, W, P, N, K, n_mt, 1, K >> 8, C, ldc, Q2Group{tiles, off, stok, E, otok, owt}, Q2Fuse{});
     MXK_CHECK_LAUNCH();
 }
 
@@ -784,41 +781,6 @@ static int dispatch_qmm2(int wm, int ks, int wn, const uint16_t* A, int lda, con
     return (int)hipErrorInvalidValue;
 }
 
-template <int DBG>
-static int launch_dbg(int wm, int ks, int wn, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, void* C, int ldc,
-                      hipStream_t st) {
-    constexpr int QT = MXQ_Q4_K, EPI = E16_SWIGLU;
-    auto go = [&](auto kern, int bm, int ks, int lds, int ng = 4) {
-        (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        const int n_ct = (N + 32 * ng - 1) / (32 * ng), n_mt = (M + bm - 1) / bm;
-        kern<<<dim3(n_ct * n_mt), ng == 8 ? 512 : 256 * ks, lds, st>>>(A, lda, W, M, N, K, n_mt, 1, K >> 8, C, ldc,
-                                                                      g_qmm2_rot, Q2Group{}, Q2Fuse{});
-        return (int)hipGetLastError();
-    };
-    // ks 17: the wide tiles (8 column groups)
-    if (wm == 6 && ks == 17 && wn == 1)
-        return go(qmm2_kernel<QT, 6, 1, 1, EPI, DBG, 4, 8>, 192, 1, Q2Geom<QT, 6, 1, 1, 4, 8>::LDS, 8);
-    if (wm == 4 && ks == 17 && wn == 1)
-        return go(qmm2_kernel<QT, 4, 1, 1, EPI, DBG, 4, 8>, 128, 1, Q2Geom<QT, 4, 1, 1, 4, 8>::LDS, 8);
-    if (wm == 3 && ks == 17 && wn == 2)
-        return go(qmm2_kernel<QT, 3, 1, 2, EPI, DBG, 4, 8>, 192, 1, Q2Geom<QT, 3, 1, 2, 4, 8>::LDS, 8);
-    if (wm == 6 && ks == 18 && wn == 2 && QT == MXQ_Q4_K) {
-        auto k4 = qmm2_kernel<QT, 6, 1, 2, EPI, DBG, 4, 8, 2>;
-        (void)hipFuncSetAttribute((const void*)k4, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  Q2Geom<QT, 6, 1, 2, 4, 8, 2>::LDS);
-        const int n_ct = (N + 255) / 256, n_mt = (M + 191) / 192;
-        k4<<<dim3(n_ct * n_mt), 256, Q2Geom<QT, 6, 1, 2, 4, 8, 2>::LDS, st>>>(A, lda, W, M, N, K, n_mt, 1, K >> 8, C, ldc,
-                                                                            g_qmm2_rot, Q2Group{}, Q2Fuse{});
-        return (int)hipGetLastError();
-    }
-    if (wm == 8 && ks == 1 && wn == 1) return go(qmm2_kernel<QT, 8, 1, 1, EPI, DBG>, 256, 1, Q2Geom<QT, 8, 1, 1>::LDS);
-    if (wm == 4 && ks == 2 && wn == 1) return go(qmm2_kernel<QT, 4, 2, 1, EPI, DBG>, 128, 2, Q2Geom<QT, 4, 2, 1>::LDS);
-    if (wm == 4 && ks == 1 && wn == 2) return go(qmm2_kernel<QT, 4, 1, 2, EPI, DBG>, 256, 1, Q2Geom<QT, 4, 1, 2>::LDS);
-    if (wm == 2 && ks == 2 && wn == 2) return go(qmm2_kernel<QT, 2, 2, 2, EPI, DBG>, 128, 2, Q2Geom<QT, 2, 2, 2>::LDS);
-    return (int)hipErrorInvalidValue;
-}
-
-
 // all epilogues of one block format (each format's instances live in their own translation unit, qmm2_q*.hip)
 template <int QT>
 static int qmm2_run(int epi, int wm, int ks, int wn, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, int splits, void* C, int ldc, hipStream_t st, const Q2Fuse& fu) {
@@ -859,4 +821,3 @@ int qmm2_grouped_q4k(int epi, int wm, const uint16_t* A, int lda, const int* sto
 int qmm2_grouped_q5k(int epi, int wm, const uint16_t* A, int lda, const int* stok, const uint8_t* W, int P, int E, int N, int K, const int* tiles, const int* off, void* C, int ldc, const int* otok, const float* owt, hipStream_t st);
 int qmm2_grouped_q6k(int epi, int wm, const uint16_t* A, int lda, const int* stok, const uint8_t* W, int P, int E, int N, int K, const int* tiles, const int* off, void* C, int ldc, const int* otok, const float* owt, hipStream_t st);
 int qmm2_grouped_q80(int epi, int wm, const uint16_t* A, int lda, const int* stok, const uint8_t* W, int P, int E, int N, int K, const int* tiles, const int* off, void* C, int ldc, const int* otok, const float* owt, hipStream_t st);
-int qmm2_dbg_q4k(int dbg, int wm, int ks, int wn, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, void* C, int ldc, hipStream_t st);

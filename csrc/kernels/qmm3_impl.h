@@ -79,12 +79,12 @@ __global__ __launch_bounds__(512) void qmm3_kernel(const uint16_t* __restrict__ 
             if constexpr (!(DBG & 4)) {
 #pragma unroll
                 for (int i = 0; i < WA; ++i)
-                    q2_dma((const void*)(ak + aoff[i]), (MX_LDS void*)(as + (p * WA + i) * 1024), 16);
+                    mx_lds_dma16(ak, 2 * aoff[i], mx_lds_addr(as + (p * WA + i) * 1024));
             }
             if constexpr (DBG & 8) return;
             const uint8_t* u = wg + (size_t)sb * F::UNIT;
-            q2_stage_weights<QT, JQ>(u, smem + G::OFF_Q + slot * G::QSZ + p * F::QB,
-                                     smem + G::OFF_H + ((t >> 2) & 1) * G::HSZ + p * F::HB, lane);
+            q2_stage_weights<QT, JQ>(u, mx_lds_addr(smem + G::OFF_Q + slot * G::QSZ + p * F::QB),
+                                     mx_lds_addr(smem + G::OFF_H + ((t >> 2) & 1) * G::HSZ + p * F::HB), lane);
         };
         // dequant of tile t (its bytes landed) into f16 B buffer t & 1
         Q2B<QT> bq;
@@ -93,7 +93,6 @@ __global__ __launch_bounds__(512) void qmm3_kernel(const uint16_t* __restrict__ 
             if constexpr (DBG & 2) return;
             if constexpr (JQ == 0) bq.load_hdr(smem + G::OFF_H + ((t >> 2) & 1) * G::HSZ + p * F::HB, col, h);
             bq.load_q(smem + G::OFF_Q + slot * G::QSZ + p * F::QB, col, h);
-            bq.template prep<JQ>();
             char* bd = smem + G::OFF_B + (t & 1) * G::B16 + p * 1024 + lane * 16;
             *(f16x8*)(bd + 0 * 4096) = bq.template frag<JQ, 0>();
             *(f16x8*)(bd + 1 * 4096) = bq.template frag<JQ, 1>();

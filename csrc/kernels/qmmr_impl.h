@@ -103,7 +103,6 @@ __global__ __launch_bounds__(64 * GW * KW) void qmmr_kernel(const uint16_t* __re
                     const char* as = smem + (t & 1) * G::SLOT + a_rd;
                     auto quarter = [&](auto q_c) {
                         constexpr int q = decltype(q_c)::value, JQ = Q0 + q;
-                        b[u][q].template prep<JQ>();
                         auto step = [&](auto s_c) {
                             constexpr int S = decltype(s_c)::value;
                             f16x8 af[WM];
