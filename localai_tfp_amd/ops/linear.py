@@ -326,7 +326,7 @@ def row_chunks(M: int, chunk: int | None = None) -> list[tuple[int, int]]:
 def run_plan(plan: tuple, W: QWeight, x: torch.Tensor, epi: int, out: torch.Tensor, out_zeroed: bool,
              fuse: "NormFuse | None" = None):
     """Launch one GEMM plan (ops/autotune.py): ("q3", wm, splits) | ("q2", wm, ks, wn, splits) |
-    ("qr", wm, gw, kw, splits) | ("rows", chunk) | ("x16", columns, plan)."""
+    ("qr", wm, gw, kw, splits) | ("q4", blocks, 1) | ("rows", chunk) | ("x16", columns, plan)."""
     M = x.shape[0]
     kind = plan[0]
     if fuse is not None and kind != "q2":
@@ -346,6 +346,9 @@ def run_plan(plan: tuple, W: QWeight, x: torch.Tensor, epi: int, out: torch.Tens
     if kind == "q3":
         N.kcall("mxk_qmm3", int(W.qtype), e, plan[1], x.data_ptr(), x.stride(0), W.data.data_ptr(), M, W.N, W.K,
                 splits, out.data_ptr(), out.stride(0), N.stream_ptr())
+    elif kind == "q4":
+        N.kcall("mxk_qmm4", int(W.qtype), e, plan[1], x.data_ptr(), x.stride(0), W.data.data_ptr(), M, W.N, W.K, out.data_ptr(),
+                out.stride(0), N.stream_ptr())
     elif kind == "qr":
         N.kcall("mxk_qmmr", int(W.qtype), e, plan[1], plan[2], plan[3], x.data_ptr(), x.stride(0), W.data.data_ptr(),
                 M, W.N, W.K, splits, out.data_ptr(), out.stride(0), N.stream_ptr())
@@ -412,6 +415,8 @@ def _t32_plan(W: QWeight, M: int, epi: int, out_zeroed: bool, dtype=torch.float1
             plan = _gemm_pick(M, W.N, W.K, int(W.qtype), can_split)
             if M >= X16_MIN_M and not forced and not (NORM_FUSE or ROPE_FUSE) and dtype == torch.float16:
                 plan = _expanded_plan(M, W.N, W.K, int(W.qtype), can_split, epi in GLU_EPIS) or plan
+            if epi != EPI_ADD_F32 and not forced and not (NORM_FUSE or ROPE_FUSE) and dtype == torch.float16:
+                plan = _wide_plan(plan, M, W.N, W.K, int(W.qtype), can_split, epi in GLU_EPIS)
     return plan
 
 
@@ -652,6 +657,8 @@ QMM2_QTYPES = (int(QType.Q4_K), int(QType.Q6_K), int(QType.Q3_K), int(QType.Q2_K
 # qmmr.hip (wm, gw, kw): 32 wm rows x 32 gw columns a workgroup, kw waves over each super-block of K
 QMMR_CONFIGS = ((1, 4, 4), (1, 2, 4), (1, 1, 4), (1, 4, 2), (1, 2, 2), (2, 2, 4), (2, 4, 2))
 QMMR_MAX_M = 192  # rows up to which the tuner times them (weights are decoded once per row tile)
+QMM4_BLOCKS = (8, 10, 12, 14)  # qmm4.hip: 16-row blocks a row tile (x 256 columns) may have
+QMM4_MIN_M = 97  # rows from which the tuner times it
 QMM2_MIN_M = int(os.environ.get("MX_QMM2_MIN_M", "16"))
 
 
@@ -674,6 +681,16 @@ _STAGE_BYTES = {int(QType.Q4_K): (1024, 512), int(QType.Q5_K): (1024, 1536), int
                 int(QType.MX5F): (1280, 1024), int(QType.Q8_0): (2176, 0)}
 
 
+def _rounds(workgroups: int) -> float:
+    """Rounds of one workgroup a compute unit; a last one that is r full counts 0.6 + 0.4 r (a half-empty chip clocks and feeds faster)."""
+    full, rem = divmod(workgroups, CU_COUNT)
+    return full + (0.6 + 0.4 * rem / CU_COUNT if rem else 0.0)
+
+
+def _tiles_us(M: int, N_: int, K: int, bm: int, bn: int, c: float, s: int = 1) -> float:
+    return 6.6 + _rounds(-(-M // bm) * -(-N_ // bn) * s) * bm * bn * K * c * 1e-6
+
+
 @functools.lru_cache(maxsize=4096)
 def _large_best(M: int, N_: int, K: int, qtype: int, can_split: bool):
     """(estimate, plan): the qmm2 plan of a GEMM of more than LARGE_M rows: the least of
@@ -689,10 +706,7 @@ def _large_best(M: int, N_: int, K: int, qtype: int, can_split: bool):
     qb, hb = _STAGE_BYTES[qtype]
 
     def cost(wm, ks, wn, c, s):
-        bm, ng = 32 * wm * wn, 8 if ks == 17 else 4
-        full, rem = divmod(-(-M // bm) * -(-N_ // (32 * ng)) * s, CU_COUNT)
-        rounds = full + (0.6 + 0.4 * rem / CU_COUNT if rem else 0.0)
-        t = 6.6 + rounds * bm * 32 * ng * 256 * -(-(K // 256) // s) * c * 1e-6
+        t = _tiles_us(M, N_, 256 * -(-(K // 256) // s), 32 * wm * wn, 256 if ks == 17 else 128, c, s)
         return t + 2.4e-6 * M * N_ * s if s > 1 else t
     square = next(t for t in _LARGE_TILES if t[:3] == (4, 2, 1))
     splits = 1 if N_ < 16384 and K < 8192 else _split_for(-(-M // 128) * -(-N_ // 128), K, can_split)
@@ -730,14 +744,57 @@ def _expanded_plan(M: int, N_: int, K: int, qtype: int, can_split: bool, glu: bo
     238. Weights in two pieces leave half a round each: 8192 x 28672 Q4_K at 2048 rows 904 / 1155, at 4096 1791 / 1911, at 8191 3591 / 3259;
     57344 x 8192 at 2304 2021 / 2162, at 4096 3603 / 2992."""
     t, plan = _large_best(M, N_, K, qtype, can_split)
-    cols = max(256, X16_SCRATCH // (K * 512) * 256)
-    us = 0.62e-6 * N_ * K
-    for n0 in range(0, N_, cols):
-        full, rem = divmod(-(-M // 256) * -(-min(cols, N_ - n0) // 256), CU_COUNT)
-        us += 11.0 + (full + (0.6 + 0.4 * rem / CU_COUNT if rem else 0.0)) * (1.45 * K / 64 + (5.0 if glu else 12.0))
+    us, cols = _expanded_us(M, N_, K, glu)
     if us < t * (1.12 if glu else 1.05) * (0.98 if qtype == int(QType.MX4F) else 1.0):
         return ("x16", cols, plan)
     return None
+
+
+def _expanded_us(M: int, N_: int, K: int, glu: bool):
+    cols = max(256, X16_SCRATCH // (K * 512) * 256)
+    us = 0.62e-6 * N_ * K
+    for n0 in range(0, N_, cols):
+        us += 11.0 + _rounds(-(-M // 256) * -(-min(cols, N_ - n0) // 256)) * (1.45 * K / 64 + (5.0 if glu else 12.0))
+    return us, cols
+
+
+# qmm4.hip: largest row tile in 16-row blocks (where the ring fits the LDS), whether odd numbers of blocks are compiled, and what a
+# format's decoding costs beside Q4_K's
+_QMM4_TILES = {int(QType.Q4_K): (14, 1, 1.0), int(QType.Q5_K): (13, 1, 1.13), int(QType.Q6_K): (12, 1, 1.06), int(QType.Q8_0): (11, 1, 1.03),
+               int(QType.Q3_K): (12, 2, 1.0), int(QType.Q2_K): (14, 2, 0.95), int(QType.MX4F): (14, 2, 0.95), int(QType.MX5F): (12, 2, 1.05)}
+
+
+@functools.lru_cache(maxsize=4096)
+def _wide_best(M: int, N_: int, K: int, qtype: int):
+    """(estimate, ("q4", blocks, 1)): qmm4.hip's best cut of M rows. Within 6 % of 117 measurements (Q4_K and Q6_K, 6144 x 4096 .. 57344 x 8192,
+    520 to 8191 rows) and 12 % of 35 in the other formats; small tiles cost more a flop, since every workgroup dequantises its 256 columns."""
+    top, step, q = _QMM4_TILES[qtype]
+    best = None
+    for nb in range(8, top + 1, step):
+        blocks = -(-M // 16)
+        ni = -(-blocks // -(-blocks // nb))
+        ni = max(8, -(-ni // step) * step)
+        t = _tiles_us(M, N_, K, 16 * ni, 256, (0.30 + 1.35 / ni) * q)
+        if best is None or t < best[0]:
+            best = (t, ("q4", nb, 1))
+    return best
+
+
+def _wide_plan(plan: tuple, M: int, N_: int, K: int, qtype: int, can_split: bool, glu: bool):
+    """qmm4's plan instead of `plan`, what an untuned product that does not accumulate would run, where its estimate is the lower one.
+    _large_best is 7 % low against these measurements for gated products and even for others, so qmm4 is taken up to 5 % above it there;
+    expanded weights stay up to 3 % above it. Up to 512 rows only of 16384 columns and more, beyond 256 rows, where `plan` is the 128-row tile: fewer leave
+    compute units idle. us, before / qmm4: gate|up 28672 x 4096 Q4_K at 384 / 700 / 1300 / 2048 rows 97 / 76, 184 / 158, 301 / 269, 440
+    (expanded) / 405, Q6_K at 1300 340 / 330; 57344 x 8192 Q4_K at 1100 968 / 863, at 4096 2921 (expanded, kept) / 3124; 6144 x 4096 at 2048 104 / 91, at 900
+    52 (kept) / 61; 8192 x 2048 at 1100 45 / 39."""
+    if M <= 256 or M <= LARGE_M and N_ < 16384:
+        return plan
+    t, wide = _wide_best(M, N_, K, qtype)
+    if plan[0] == "x16":
+        return plan if _expanded_us(M, N_, K, glu)[0] < 1.03 * t else wide
+    if M <= LARGE_M:
+        return wide if t < 0.97 * _tiles_us(M, N_, K, 128, 128, 0.526) else plan
+    return wide if t < (1.055 if glu else 1.0) * _large_best(M, N_, K, qtype, can_split)[0] else plan
 
 
 # super-blocks of a qmmr workgroup up to which it is the faster one, at 5 to 15 and 16 to 32 rows
