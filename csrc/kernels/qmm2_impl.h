@@ -143,12 +143,10 @@ struct Q2Group {
 };
 
 
-template <int QT, int WM, int KS, int WN, int EPI, int NS = 4, int NG = 4, int GPW = 1, bool GR = false,
-          bool FU = false>
-__global__ __launch_bounds__(NG == 8 ? 512 / GPW : 256 * KS) void qmm2_kernel(const uint16_t* __restrict__ A, int lda,
-                                                        const uint8_t* __restrict__ W, int M, int N, int K,
-                                                        int n_mt, int splits, int sbps, void* __restrict__ Cv,
-                                                        int ldc, Q2Group grp, Q2Fuse fu = Q2Fuse{}) {
+// (workgroup `bid` of the `nwg` that share the product)
+template <int QT, int WM, int KS, int WN, int EPI, int NS = 4, int NG = 4, int GPW = 1, bool GR = false, bool FU = false>
+MX_DEV void qmm2_body(const int nwg, const int bid, const uint16_t* __restrict__ A, int lda, const uint8_t* __restrict__ W, int M, int N, int K,
+                      int n_mt, int splits, int sbps, void* __restrict__ Cv, int ldc, Q2Group grp, Q2Fuse fu) {
     using G = Q2Geom<QT, WM, KS, WN, NS, NG, GPW>;
     using F = Q2F<QT>;
     constexpr int BM = G::BM, WA = G::WA, STAGE = G::STAGE, A_BYTES = G::A_BYTES;
@@ -172,7 +170,6 @@ __global__ __launch_bounds__(NG == 8 ? 512 / GPW : 256 * KS) void qmm2_kernel(co
     const int nw = cg % NW, mw = cg / NW;
 
     // XCD-aware bijective remap: consecutive logical ids (q2_tile_of) run on one XCD and share its L2
-    const int nwg = gridDim.x, bid = blockIdx.x;
     const int xcd = bid & 7, q8 = nwg >> 3, r8 = nwg & 7;
     const int lid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (bid >> 3);
     int mt, rest;
@@ -671,6 +668,13 @@ __global__ __launch_bounds__(NG == 8 ? 512 / GPW : 256 * KS) void qmm2_kernel(co
             }
         }
     }
+}
+
+template <int QT, int WM, int KS, int WN, int EPI, int NS = 4, int NG = 4, int GPW = 1, bool GR = false, bool FU = false>
+__global__ __launch_bounds__(NG == 8 ? 512 / GPW : 256 * KS) void qmm2_kernel(const uint16_t* __restrict__ A, int lda, const uint8_t* __restrict__ W,
+                                                                              int M, int N, int K, int n_mt, int splits, int sbps,
+                                                                              void* __restrict__ Cv, int ldc, Q2Group grp, Q2Fuse fu = Q2Fuse{}) {
+    qmm2_body<QT, WM, KS, WN, EPI, NS, NG, GPW, GR, FU>(gridDim.x, blockIdx.x, A, lda, W, M, N, K, n_mt, splits, sbps, Cv, ldc, grp, fu);
 }
 
 template <int QT, int WM, int KS, int WN, int EPI, int NS = 4, int NG = 4, int GPW = 1, bool FU = false>

@@ -16,11 +16,10 @@ struct QrGeom {
     static constexpr int AP = BM * 32 / NT;                 // 16-byte pieces of A a thread stages per super-block
 };
 
+// (workgroup `bid` of the `nwg` that share the product)
 template <int QT, int WM, int GW, int KW, int EPI>
-__global__ __launch_bounds__(64 * GW * KW) void qmmr_kernel(const uint16_t* __restrict__ A, int lda,
-                                                            const uint8_t* __restrict__ W, int M, int N, int K,
-                                                            int n_mt, int splits, int sbps, void* __restrict__ Cv,
-                                                            int ldc) {
+MX_DEV void qmmr_body(const int nwg, const int bid, const uint16_t* __restrict__ A, int lda, const uint8_t* __restrict__ W, int M, int N, int K,
+                      int n_mt, int splits, int sbps, void* __restrict__ Cv, int ldc) {
     using G = QrGeom<WM, GW, KW>;
     using F = Q2F<QT>;
     constexpr int BM = G::BM, AP = G::AP, NQ = 4 / KW;
@@ -34,7 +33,6 @@ __global__ __launch_bounds__(64 * GW * KW) void qmmr_kernel(const uint16_t* __re
     const int gw = wave % GW, kw = wave / GW;
 
     // consecutive logical ids run on one XCD (q2_tile_of)
-    const int nwg = gridDim.x, bid = blockIdx.x;
     const int xcd = bid & 7, q8 = nwg >> 3, r8 = nwg & 7;
     const int lid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (bid >> 3);
     int mt, rest;
@@ -176,6 +174,12 @@ __global__ __launch_bounds__(64 * GW * KW) void qmmr_kernel(const uint16_t* __re
             }
         }
     }
+}
+
+template <int QT, int WM, int GW, int KW, int EPI>
+__global__ __launch_bounds__(64 * GW * KW) void qmmr_kernel(const uint16_t* __restrict__ A, int lda, const uint8_t* __restrict__ W, int M, int N,
+                                                            int K, int n_mt, int splits, int sbps, void* __restrict__ Cv, int ldc) {
+    qmmr_body<QT, WM, GW, KW, EPI>(gridDim.x, blockIdx.x, A, lda, W, M, N, K, n_mt, splits, sbps, Cv, ldc);
 }
 
 template <int QT, int WM, int GW, int KW, int EPI>

@@ -40,6 +40,7 @@ KERNEL_SIGS = {
     "mxk_qmm2_fused": [I, I, I, I, I, P, I, P, I, I, I, I, P, I, I, P, P, P, P, I, P, P, F, F, P],
     "mxk_qmm2_rope": [I, I, I, I, I, P, I, P, I, I, I, I, P, I, I, P, F, F, P, P, P, P, P, P, P, I, I, I, I, I, P],
     "mxk_qmm3": [I, I, I, P, I, P, I, I, I, I, P, I, P],
+    "mxk_qmm_pair": [I, I, I, I, I, I, I, P, I, P, I, P, I, I, I, I, P, I, P],
     "mxk_qmm4": [I, I, I, P, I, P, I, I, I, P, I, P],
     "mxk_qmmr": [I, I, I, I, I, P, I, P, I, I, I, I, P, I, P],
     "mxk_t32_expand": [I, P, I, I, P, P],

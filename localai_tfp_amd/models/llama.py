@@ -37,7 +37,7 @@ from ..ops import core as K
 from ..ops import quant as Q
 from ..ops.linear import (ACT_DTYPE, EPI_ADD_F32, EPI_BF16, EPI_F32, EPI_GEGLU, EPI_SWIGLU, QWeight, concat_rows,
                           _fp32_out_ok, dense_min_m, interleave_gate_up, glu_interleaved, qmatmul, qmv_fusable, qmv_rope_ok,
-                          qmv_fused, qmv_rope_fused, qmv_rope_pair_fused, NormFuse, norm_fusable)
+                          qmatmul_pair, qmv_fused, qmv_rope_fused, qmv_rope_pair_fused, NormFuse, norm_fusable)
 from ..ops import linear as _LIN
 from ..ops import autotune as _AT
 from ..ops.moe import MoEWeights, moe_ffn
@@ -416,6 +416,8 @@ class LlamaModel:
         for L in self.layers:
             for w in L.qkv_parts:
                 yield w, EPI_F32, True
+            if len(L.qkv_parts) == 2:
+                yield tuple(L.qkv_parts), EPI_F32, True
             for w in (L.wo, L.wd):
                 if w is not None:
                     yield (w, EPI_BF16, False) if tp else (w, EPI_ADD_F32, True)
@@ -694,6 +696,9 @@ class LlamaModel:
                                           sk=(ws.sk_ws, ws.sk_cnt)):
                         raise RuntimeError("qkv RoPE fusion applied to some parts only")
                     o2 += w.N
+            if (off == 0 and len(L.qkv_parts) == 2 and not (gemv or rope_ep or nf_qkv is not None)
+                    and qkv.is_cuda and qmatmul_pair(L.qkv_parts, xb, qkv)):
+                off = qkv.shape[1]
             for w in (L.qkv_parts if off == 0 and not rope_fused else ()):
                 sl = qkv[:, off:off + w.N] if len(L.qkv_parts) > 1 else qkv
                 if fuse_qkv:

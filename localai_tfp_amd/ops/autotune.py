@@ -30,6 +30,7 @@ BUCKETS = (16, 32, 64, 96, 128, 160, 192, 224, 256, 320, 384, 448, 512)
 SPLITS = (1, 2, 4, 8)
 # (N, K, qtype, epi, can_split) -> [(bucket, plan)] sorted by bucket
 TUNED: dict[tuple, list] = {}
+TUNED_PAIRS: dict[tuple, list] = {}  # (Na, Nb, K, qa, qb) -> [(bucket, plan of qmmp.hip, () where two launches are faster)]
 TIMES: dict[tuple, list] = {}  # key -> [(bucket, plan, us)] of the plans tuned in this process (reports)
 ENABLED = os.environ.get("MX_GEMM_TUNE", "1") != "0"
 
@@ -44,6 +45,14 @@ def lookup(N: int, K: int, qtype: int, epi: int, can_split: bool, M: int):
     if not ent:
         return None
     for b, plan in ent:
+        if M <= b:
+            return plan
+    return None
+
+
+def lookup_pair(Na: int, Nb: int, K: int, qa: int, qb: int, M: int):
+    """Tuned plan of two weights in one launch, () where two launches won, or None (untuned, or M beyond the largest bucket)."""
+    for b, plan in TUNED_PAIRS.get((int(Na), int(Nb), int(K), int(qa), int(qb)), ()):
         if M <= b:
             return plan
     return None
@@ -130,6 +139,36 @@ def tune_weight(W, epi: int, can_split: bool, buckets=BUCKETS, iters: int = 8) -
     return res
 
 
+def tune_pair(a, b, buckets=BUCKETS, iters: int = 8) -> list:
+    """Time the plans of two weights in one launch beside a launch each by their own plans; -> [(bucket, plan or ())]."""
+    from . import linear as L
+    dev, Mmax = a.data.device, max(buckets)
+    x = (torch.randn(Mmax, a.K, device=dev) * 0.5).to(torch.float16)
+    out = torch.zeros(Mmax, a.N + b.N, device=dev, dtype=torch.float32)
+    res = []
+    for m in sorted(buckets):
+        xb, ob = x[:m], out[:m]
+
+        def apart():
+            L.qmatmul(a, xb, L.EPI_F32, ob[:, :a.N], out_zeroed=True)
+            L.qmatmul(b, xb, L.EPI_F32, ob[:, a.N:], out_zeroed=True)
+        apart()
+        best, best_t = (), min(_time(apart, iters), _time(apart, iters))
+        for p in L.PAIR_PLANS:
+            if 32 * p[1] > 2 * max(m, 32) or p[0] == "qr" and m > L.QMMR_MAX_M:
+                continue
+            for s in (s for s in SPLITS if s == 1 or a.K // 256 // s >= 2):
+                def run(plan=(*p, s)):
+                    L.run_pair(plan, a, b, xb, ob)
+                run()
+                t = min(_time(run, iters), _time(run, iters))
+                if t < best_t:
+                    best, best_t = (*p, s), t
+        res.append((m, best))
+        log.debug("tune pair %s M=%d -> %s %.1f us", (a.N, b.N, a.K), m, best, best_t)
+    return res
+
+
 def report() -> list[dict]:
     """The plans tuned in this process with their times (bench / profiles)."""
     return [{"N": k[0], "K": k[1], "qtype": k[2], "epi": k[3], "split": k[4],
@@ -199,7 +238,12 @@ def tune_gemms(specs, buckets=BUCKETS) -> float:
     cache = load_cache()
     new = {}
     seen = set()
+    pairs = {}
     for W, epi, can_split in specs:
+        if isinstance(W, tuple):  # two weights by the same rows, tuned when each of them is
+            if L.pair_ok(W):
+                pairs.setdefault((W[0].N, W[1].N, W[0].K, int(W[0].qtype), int(W[1].qtype)), W)
+            continue
         if (not isinstance(W, L.QWeight) or W.layout != "t32" or not W.data.is_cuda
                 or int(W.qtype) not in L.QMM2_QTYPES):
             continue
@@ -216,6 +260,13 @@ def tune_gemms(specs, buckets=BUCKETS) -> float:
             new[ck] = [(b, list(p)) for b, p in res]
         else:
             log.warning("gemm autotune: no plan ran for %s; the untuned fallback rule serves it", key)
+    for key, (a, b) in pairs.items():
+        ck = "pair," + ",".join(map(str, key)) + "|" + ",".join(map(str, buckets))
+        if ck in cache:
+            TUNED_PAIRS[key] = [(b_, tuple(p)) for b_, p in cache[ck]]
+            continue
+        TUNED_PAIRS[key] = tune_pair(a, b, buckets)
+        new[ck] = [(b_, list(p)) for b_, p in TUNED_PAIRS[key]]
     if new:
         save_cache(new)
     dt = time.time() - t0

@@ -485,6 +485,49 @@ def _qmatmul_t32(W: QWeight, x, epi: int, out, xq, xds, M: int, out_zeroed: bool
     return run_plan(plan, W, x, epi, out, out_zeroed)
 
 
+# qmmp.hip: two weights by the same rows in one launch, formats and (kind, wm | wm, ks | gw, wn | kw) compiled
+PAIR_QTYPES = {(int(QType.Q4_K), int(QType.Q6_K)), (int(QType.Q5_K), int(QType.Q6_K)), (int(QType.Q3_K), int(QType.Q5_K))}
+PAIR_PLANS = (("q2", 4, 2, 1), ("q2", 2, 2, 1), ("qr", 1, 1, 4), ("qr", 1, 2, 4), ("qr", 1, 4, 4), ("qr", 2, 2, 4))
+
+
+def pair_ok(parts) -> bool:
+    """Two t32 weights of formats that qmmp.hip is built for, on one GPU, without dense copies."""
+    return (len(parts) == 2 and all(isinstance(w, QWeight) and w.layout == "t32" and w.data.is_cuda and w.bf16_cache is None for w in parts)
+            and parts[0].K == parts[1].K and (int(parts[0].qtype), int(parts[1].qtype)) in PAIR_QTYPES
+            and not (NORM_FUSE or ROPE_FUSE or QMM2 or QMM3 or QMM2_FORCE is not None or QMM3_FORCE is not None))
+
+
+def _pair_plan(a: QWeight, b: QWeight, M: int):
+    """Plan of qmmp.hip for M rows into a zeroed output: what the load-time tuner found, else the rule's plan of as many columns where it is
+    compiled for pairs. None: two launches."""
+    tuned = _AT.lookup_pair(a.N, b.N, a.K, int(a.qtype), int(b.qtype), M)
+    if tuned is not None:
+        return tuned or None
+    plan = _gemm_pick(M, a.N + b.N, a.K, int(a.qtype), True)
+    return plan if plan[:-1] in PAIR_PLANS else None
+
+
+def run_pair(plan: tuple, a: QWeight, b: QWeight, x: torch.Tensor, out: torch.Tensor):
+    kind, p0, p1, p2, splits = plan
+    N.kcall("mxk_qmm_pair", int(a.qtype), int(b.qtype), EPI_ADD_F32 if splits > 1 else EPI_F32, 2 if kind == "q2" else 0, p0, p1, p2, x.data_ptr(),
+            x.stride(0), a.data.data_ptr(), a.N, b.data.data_ptr(), b.N, x.shape[0], a.K, splits, out.data_ptr(), out.stride(0), N.stream_ptr())
+
+
+def qmatmul_pair(parts, x: torch.Tensor, out: torch.Tensor) -> bool:
+    """out = x [a; b]^T for two weights of different block formats in one launch; out: fp32 [M, a.N + b.N], zero (K may be split over atomics).
+    False: not applicable, nothing launched."""
+    if x.dtype != torch.float16 or x.stride(-1) != 1 or out.dtype != torch.float32 or out.stride(-1) != 1 or not pair_ok(parts):
+        return False
+    a, b = parts
+    if out.shape != (x.shape[0], a.N + b.N) or x.shape[1] != a.K or x.shape[0] == 0 or not x.is_cuda or not out.is_cuda:
+        return False
+    plan = _pair_plan(a, b, x.shape[0])
+    if plan is None:
+        return False
+    run_pair(plan, a, b, x, out)
+    return True
+
+
 QMV_FUSE = os.environ.get("MX_QMV_FUSE", "1") != "0"
 
 
