@@ -17,9 +17,10 @@ struct Q4Geom {
     static constexpr int WA = (2 * NI + 7) / 8;          // A LDS-DMA instructions of a wave a stage (spare ones re-load the last block)
 };
 
+// splits > 1 (fp32 out alone): sbps super-blocks of K a workgroup, the sums of part p to Cv [p][M][ldc]
 template <int QT, int NI, int EPI>
 __global__ __launch_bounds__(512) void qmm4_kernel(const uint16_t* __restrict__ A, int lda, const uint8_t* __restrict__ W,
-                                                   int M, int N, int K, int n_mt, void* __restrict__ Cv, int ldc) {
+                                                   int M, int N, int K, int n_mt, int splits, int sbps, void* __restrict__ Cv, int ldc) {
     using G = Q4Geom<QT, NI>;
     using F = Q2F<QT>;
     using B = Q2B<QT, 32>;
@@ -38,13 +39,23 @@ __global__ __launch_bounds__(512) void qmm4_kernel(const uint16_t* __restrict__ 
     // XCD-aware bijective remap: consecutive logical ids (q2_tile_of) run on one XCD and share its L2
     const int nwg = gridDim.x, bid = blockIdx.x;
     const int xcd = bid & 7, q8 = nwg >> 3, r8 = nwg & 7;
-    const int lid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (bid >> 3);
-    int mt, ct;
-    q2_tile_of(lid, n_mt, nwg / n_mt, mt, ct);
-    const int nsb = K >> 8;
+    int lid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (bid >> 3);
+    int mt, ct, tiles = nwg, nsb = K >> 8, sb0 = 0;
+    const size_t col_bytes = (size_t)nsb * F::UNIT;  // of a column group
+    if constexpr (EPI == E16_F32) {
+        // the tiles of a part of K follow one another: they read the same k of A, and its L2 holds that
+        tiles = nwg / splits;
+        const int p = lid / tiles;
+        lid -= p * tiles;
+        sb0 = p * sbps;
+        nsb = min(sbps, nsb - sb0);
+        Cv = (float*)Cv + (size_t)p * M * ldc;
+    }
+    q2_tile_of(lid, n_mt, tiles / n_mt, mt, ct);
     const int m_base = mt * BM, ngrp = N >> 5;
     // (groups past N re-read the last, never stored)
-    const uint8_t* wg = W + (size_t)min(ct * NG + wave, ngrp - 1) * ((size_t)nsb * F::UNIT);
+    const uint8_t* wg = W + (size_t)min(ct * NG + wave, ngrp - 1) * col_bytes + (size_t)sb0 * F::UNIT;
+    A += (size_t)sb0 * 256;
 
     // A LDS-DMA sources and image as qmm2's: 8-row block j, lane p writes image slot (16-k step p >> 4, row (p >> 1) & 7, half
     // (p & 1) ^ (j & 1)) from 16 B of that row
@@ -205,18 +216,22 @@ __global__ __launch_bounds__(512) void qmm4_kernel(const uint16_t* __restrict__ 
     }
 }
 
+// super-blocks of K in each of `splits` parts (the last one may have fewer; none is empty)
+static int qmm4_part_blocks(int K, int splits) { return ((K >> 8) + splits - 1) / splits; }
+
 template <int QT, int NI, int EPI>
-static int launch_qmm4(const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, void* C, int ldc, hipStream_t st) {
+static int launch_qmm4(const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, int splits, void* C, int ldc, hipStream_t st) {
     using G = Q4Geom<QT, NI>;
-    const int n_ct = (N + 255) / 256, n_mt = (M + G::BM - 1) / G::BM;
-    const long nwg = (long)n_ct * n_mt;
+    const int n_ct = (N + 255) / 256, n_mt = (M + G::BM - 1) / G::BM, sbps = qmm4_part_blocks(K, splits);
+    splits = ((K >> 8) + sbps - 1) / sbps;
+    const long nwg = (long)n_ct * n_mt * splits;
     if (nwg <= 0 || nwg > 0x7fffffff) return (int)hipErrorInvalidValue;
     static bool attr_set = false;
     if (!attr_set) {
         (void)hipFuncSetAttribute((const void*)qmm4_kernel<QT, NI, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS);
         attr_set = true;
     }
-    qmm4_kernel<QT, NI, EPI><<<dim3((unsigned)nwg), 512, G::LDS, st>>>(A, lda, W, M, N, K, n_mt, C, ldc);
+    qmm4_kernel<QT, NI, EPI><<<dim3((unsigned)nwg), 512, G::LDS, st>>>(A, lda, W, M, N, K, n_mt, splits, sbps, C, ldc);
     MXK_CHECK_LAUNCH();
 }
 
@@ -228,7 +243,7 @@ constexpr int qmm4_max_ni() {  // largest tile whose ring fits the LDS
 // `nb`: 16-row blocks a tile may have, 8 .. 14. The fewest row tiles that hold M rows, as even as blocks allow: 416 rows run as 2 x 208,
 // 333 as 2 x 176. (The formats of few checkpoints have tiles of an even number of blocks alone, to halve what is compiled.)
 template <int QT, int EPI>
-static int dispatch_qmm4(int nb, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, void* C, int ldc, hipStream_t st) {
+static int dispatch_qmm4(int nb, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, int splits, void* C, int ldc, hipStream_t st) {
     constexpr int MAX = qmm4_max_ni<QT>();
     constexpr bool ODD = QT == MXQ_Q4_K || QT == MXQ_Q5_K || QT == MXQ_Q6_K || QT == MXQ_Q8_0;
     static_assert(Q4Geom<QT, MAX>::LDS <= 160 * 1024, "LDS");
@@ -236,7 +251,7 @@ static int dispatch_qmm4(int nb, const uint16_t* A, int lda, const uint8_t* W, i
     const int blocks = (M + 15) / 16, tiles = (blocks + nb - 1) / nb, ni = (blocks + tiles - 1) / tiles;
 #define Q4_CASE(NI_)                                                                                  \
     if constexpr (NI_ <= MAX && (ODD || NI_ % 2 == 0))                                                \
-        if (ni <= NI_) return launch_qmm4<QT, NI_, EPI>(A, lda, W, M, N, K, C, ldc, st);
+        if (ni <= NI_) return launch_qmm4<QT, NI_, EPI>(A, lda, W, M, N, K, splits, C, ldc, st);
     Q4_CASE(8) Q4_CASE(9) Q4_CASE(10) Q4_CASE(11) Q4_CASE(12) Q4_CASE(13) Q4_CASE(14)
 #undef Q4_CASE
     return (int)hipErrorInvalidValue;
@@ -244,23 +259,23 @@ static int dispatch_qmm4(int nb, const uint16_t* A, int lda, const uint8_t* W, i
 
 // the epilogues of one block format (each format's instances live in their own translation unit, qmm4_q*.hip)
 template <int QT>
-static int qmm4_run(int epi, int nb, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, void* C, int ldc, hipStream_t st) {
+static int qmm4_run(int epi, int nb, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, int splits, void* C, int ldc, hipStream_t st) {
     switch (epi) {
-        case E16_F32: return dispatch_qmm4<QT, E16_F32>(nb, A, lda, W, M, N, K, C, ldc, st);
-        case E16_ACT: return dispatch_qmm4<QT, E16_ACT>(nb, A, lda, W, M, N, K, C, ldc, st);
-        case E16_SWIGLU: return dispatch_qmm4<QT, E16_SWIGLU>(nb, A, lda, W, M, N, K, C, ldc, st);
-        case E16_GEGLU: return dispatch_qmm4<QT, E16_GEGLU>(nb, A, lda, W, M, N, K, C, ldc, st);
+        case E16_F32: return dispatch_qmm4<QT, E16_F32>(nb, A, lda, W, M, N, K, splits, C, ldc, st);
+        case E16_ACT: return dispatch_qmm4<QT, E16_ACT>(nb, A, lda, W, M, N, K, splits, C, ldc, st);
+        case E16_SWIGLU: return dispatch_qmm4<QT, E16_SWIGLU>(nb, A, lda, W, M, N, K, splits, C, ldc, st);
+        case E16_GEGLU: return dispatch_qmm4<QT, E16_GEGLU>(nb, A, lda, W, M, N, K, splits, C, ldc, st);
     }
     return (int)hipErrorInvalidValue;
 }
 
 }  // namespace
 
-int qmm4_run_q4k(int epi, int nb, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, void* C, int ldc, hipStream_t st);
-int qmm4_run_q5k(int epi, int nb, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, void* C, int ldc, hipStream_t st);
-int qmm4_run_q6k(int epi, int nb, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, void* C, int ldc, hipStream_t st);
-int qmm4_run_q3k(int epi, int nb, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, void* C, int ldc, hipStream_t st);
-int qmm4_run_q2k(int epi, int nb, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, void* C, int ldc, hipStream_t st);
-int qmm4_run_q80(int epi, int nb, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, void* C, int ldc, hipStream_t st);
-int qmm4_run_mx4(int epi, int nb, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, void* C, int ldc, hipStream_t st);
-int qmm4_run_mx5(int epi, int nb, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, void* C, int ldc, hipStream_t st);
+int qmm4_run_q4k(int epi, int nb, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, int splits, void* C, int ldc, hipStream_t st);
+int qmm4_run_q5k(int epi, int nb, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, int splits, void* C, int ldc, hipStream_t st);
+int qmm4_run_q6k(int epi, int nb, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, int splits, void* C, int ldc, hipStream_t st);
+int qmm4_run_q3k(int epi, int nb, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, int splits, void* C, int ldc, hipStream_t st);
+int qmm4_run_q2k(int epi, int nb, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, int splits, void* C, int ldc, hipStream_t st);
+int qmm4_run_q80(int epi, int nb, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, int splits, void* C, int ldc, hipStream_t st);
+int qmm4_run_mx4(int epi, int nb, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, int splits, void* C, int ldc, hipStream_t st);
+int qmm4_run_mx5(int epi, int nb, const uint16_t* A, int lda, const uint8_t* W, int M, int N, int K, int splits, void* C, int ldc, hipStream_t st);

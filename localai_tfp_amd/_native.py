@@ -42,6 +42,7 @@ KERNEL_SIGS = {
     "mxk_qmm3": [I, I, I, P, I, P, I, I, I, I, P, I, P],
     "mxk_qmm_pair": [I, I, I, I, I, I, I, P, I, P, I, P, I, I, I, I, P, I, P],
     "mxk_qmm4": [I, I, I, P, I, P, I, I, I, P, I, P],
+    "mxk_qmm4_parts": [I, I, I, P, I, P, I, I, I, P, P, I, P],
     "mxk_qmmr": [I, I, I, I, I, P, I, P, I, I, I, I, P, I, P],
     "mxk_t32_expand": [I, P, I, I, P, P],
     "mxk_gemm16": [I, P, I, P, I, I, I, I, P, I, P],

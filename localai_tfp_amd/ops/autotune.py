@@ -6,7 +6,7 @@ badly between its breakpoints (qkv 6144 x 4096: 55 us at M = 384 against 41 us a
 profiles/r5_gemm_curve.md). Instead, every distinct (N, K, block format, epilogue class) of a loaded model is
 timed on the GPU it runs on, for each M bucket the engine produces, over every compiled tile / split
 candidate; the fastest plan per bucket is kept in TUNED and ops/linear.py dispatches from it. A plan is
-("q2", wm, ks, wn, splits) | ("q3", wm, splits) | ("qr", wm, gw, kw, splits) | ("q4", blocks, 1) | ("rows", chunk) (row chunks of
+("q2", wm, ks, wn, splits) | ("q3", wm, splits) | ("qr", wm, gw, kw, splits) | ("q4", blocks, splits) | ("rows", chunk) (row chunks of
 `chunk`, each dispatched by its own bucket). Only kernel choice is tuned: every candidate computes the same product
 (the GPU tests check every tile / split / epilogue against the fp32 reference).
 
@@ -75,9 +75,12 @@ def candidates(M: int, N: int, K: int, qtype: int, can_split: bool) -> list[tupl
                 continue
             for s in sp:
                 out.append(("q3", wm, s))
-    if M >= L.QMM4_MIN_M and not (L.NORM_FUSE or L.ROPE_FUSE):  # (nor has qmm4; it refuses accumulating products)
-        tiles = {-(-(-(-M // 16)) // b): b for b in sorted(L.QMM4_BLOCKS, reverse=True)}  # the fewest blocks for each number of tiles
+    if M >= L.QMM4_MIN_M and not (L.NORM_FUSE or L.ROPE_FUSE):  # (nor has qmm4; it refuses accumulating products in one part)
+        top, step, _ = L._QMM4_TILES[qtype]
+        tiles = {-(-(-(-M // 16)) // b): b for b in range(top // step * step, 7, -step)}  # the fewest blocks for each number of tiles
         out += [("q4", b, 1) for b in tiles.values()]
+        if can_split:  # parts that make one round of workgroups
+            out += [("q4", b, s) for t, b in tiles.items() if (s := min(L.CU_COUNT // (t * -(-N // 256)), nsb // 2)) >= 2 and s * M * N <= L.QMM4_PARTS]
     if M <= L.QMMR_MAX_M and not (L.NORM_FUSE or L.ROPE_FUSE):  # (qmmr has no fused instances)
         for wm, gw, kw in L.QMMR_CONFIGS:
             if 32 * wm <= max(32, M):

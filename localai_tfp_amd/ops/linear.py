@@ -326,7 +326,7 @@ def row_chunks(M: int, chunk: int | None = None) -> list[tuple[int, int]]:
 def run_plan(plan: tuple, W: QWeight, x: torch.Tensor, epi: int, out: torch.Tensor, out_zeroed: bool,
              fuse: "NormFuse | None" = None):
     """Launch one GEMM plan (ops/autotune.py): ("q3", wm, splits) | ("q2", wm, ks, wn, splits) |
-    ("qr", wm, gw, kw, splits) | ("q4", blocks, 1) | ("rows", chunk) | ("x16", columns, plan)."""
+    ("qr", wm, gw, kw, splits) | ("q4", blocks, splits) | ("rows", chunk) | ("x16", columns, plan)."""
     M = x.shape[0]
     kind = plan[0]
     if fuse is not None and kind != "q2":
@@ -346,6 +346,15 @@ def run_plan(plan: tuple, W: QWeight, x: torch.Tensor, epi: int, out: torch.Tens
     if kind == "q3":
         N.kcall("mxk_qmm3", int(W.qtype), e, plan[1], x.data_ptr(), x.stride(0), W.data.data_ptr(), M, W.N, W.K,
                 splits, out.data_ptr(), out.stride(0), N.stream_ptr())
+    elif kind == "q4" and splits > 1:
+        if e != EPI_ADD_F32:
+            raise ValueError(f"plan {plan}: K is split into fp32 sums alone")
+        try:
+            part = torch.empty(splits, M, W.N, dtype=torch.float32, device=x.device)
+        except torch.cuda.OutOfMemoryError:  # (qmm2 adds its parts up in place)
+            return run_plan(_gemm_pick(M, W.N, W.K, int(W.qtype), True), W, x, epi, out, out_zeroed)
+        N.kcall("mxk_qmm4_parts", int(W.qtype), plan[1], splits, x.data_ptr(), x.stride(0), W.data.data_ptr(), M, W.N, W.K, part.data_ptr(),
+                out.data_ptr(), out.stride(0), N.stream_ptr())
     elif kind == "q4":
         N.kcall("mxk_qmm4", int(W.qtype), e, plan[1], x.data_ptr(), x.stride(0), W.data.data_ptr(), M, W.N, W.K, out.data_ptr(),
                 out.stride(0), N.stream_ptr())
@@ -417,6 +426,8 @@ def _t32_plan(W: QWeight, M: int, epi: int, out_zeroed: bool, dtype=torch.float1
                 plan = _expanded_plan(M, W.N, W.K, int(W.qtype), can_split, epi in GLU_EPIS) or plan
             if epi != EPI_ADD_F32 and not forced and not (NORM_FUSE or ROPE_FUSE) and dtype == torch.float16:
                 plan = _wide_plan(plan, M, W.N, W.K, int(W.qtype), can_split, epi in GLU_EPIS)
+            if can_split and plan[0] == "q2" and not forced and not (NORM_FUSE or ROPE_FUSE) and dtype == torch.float16:
+                plan = _parts_plan(M, W.N, W.K, int(W.qtype)) or plan
     return plan
 
 
@@ -700,8 +711,8 @@ QMM2_QTYPES = (int(QType.Q4_K), int(QType.Q6_K), int(QType.Q3_K), int(QType.Q2_K
 # qmmr.hip (wm, gw, kw): 32 wm rows x 32 gw columns a workgroup, kw waves over each super-block of K
 QMMR_CONFIGS = ((1, 4, 4), (1, 2, 4), (1, 1, 4), (1, 4, 2), (1, 2, 2), (2, 2, 4), (2, 4, 2))
 QMMR_MAX_M = 192  # rows up to which the tuner times them (weights are decoded once per row tile)
-QMM4_BLOCKS = (8, 10, 12, 14)  # qmm4.hip: 16-row blocks a row tile (x 256 columns) may have
 QMM4_MIN_M = 97  # rows from which the tuner times it
+QMM4_PARTS = 1 << 24  # fp32 sums of its parts of K, 64 MB
 QMM2_MIN_M = int(os.environ.get("MX_QMM2_MIN_M", "16"))
 
 
@@ -838,6 +849,32 @@ def _wide_plan(plan: tuple, M: int, N_: int, K: int, qtype: int, can_split: bool
     if M <= LARGE_M:
         return wide if t < 0.97 * _tiles_us(M, N_, K, 128, 128, 0.526) else plan
     return wide if t < (1.055 if glu else 1.0) * _large_best(M, N_, K, qtype, can_split)[0] else plan
+
+
+@functools.lru_cache(maxsize=4096)
+def _parts_plan(M: int, N_: int, K: int, qtype: int):
+    """("q4", blocks, parts of K) for an untuned product of long K that may be split: qmm4's tiles, K in as many parts as make one round of them, their
+    fp32 sums added up by a second kernel (7.7 us and 0.41 a million of them); None where _large_best's plan is the faster one. Its estimate is
+    12 % above what its 128 x 128 tile takes by such matrices and 3 to 5 % above the others', hence the factors: of 147 products of 520 to 1700 rows by 2048 x
+    8192 .. 8192 x 28672 in Q4_K, Q5_K, Q6_K and Q8_0 the picks take 0.90 of its plan's time on average, 3 of 84 more than 1.02, 1.08 at most (K below
+    8192 mostly lost: 4096 x 4096 Q4_K at 600 rows 32.4 / 37.1). us, before / here: 4096 x 14336 Q4_K at 520 / 700 / 1100 / 1700 rows 95 / 78, 111 / 85,
+    149 / 125, 208 / 181, Q6_K at 700 110 / 92; 5120 x 13824 at 777 147 / 114; 8192 x 28672 at 600 328 / 260."""
+    top, step, q = _QMM4_TILES[qtype]
+    if M <= LARGE_M or K < 8192 or step != 1:
+        return None
+    t, plan = _large_best(M, N_, K, qtype, True)
+    best = (t * (0.84 if plan[1:4] == (4, 2, 1) else 0.92), None)
+    blocks = -(-M // 16)
+    for nb in range(8, top + 1):
+        tiles = -(-blocks // nb)
+        s = min(CU_COUNT // (tiles * -(-N_ // 256)), K // 512)
+        if s < 2 or s * M * N_ > QMM4_PARTS:
+            continue
+        ni = max(8, -(-blocks // tiles))
+        t = _tiles_us(M, N_, 256 * -(-(K // 256) // s), 16 * ni, 256, (0.30 + 1.35 / ni) * q, s) + 7.7 + 0.41e-6 * M * N_ * s
+        if t < best[0]:
+            best = (t, ("q4", nb, s))
+    return best[1]
 
 
 # super-blocks of a qmmr workgroup up to which it is the faster one, at 5 to 15 and 16 to 32 rows

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from localai_tfp_amd.formats.gguf import QType
+from localai_tfp_amd.ops import autotune as A
 from localai_tfp_amd.ops import linear as L
 from localai_tfp_amd.ops import quant as Q
 
@@ -31,6 +32,48 @@ def test_rule_takes_wide_products_that_do_not_accumulate():
     W.layout = "t32"
     kinds = {e: L._t32_plan(W, 700, e, False)[0] for e in (L.EPI_F32, L.EPI_BF16, L.EPI_SWIGLU, L.EPI_GEGLU, L.EPI_ADD_F32)}
     assert kinds.pop(L.EPI_ADD_F32) == "q2" and set(kinds.values()) == {"q4"}
+
+
+def test_rule_splits_long_products():
+    q4, q6 = int(QType.Q4_K), int(QType.Q6_K)
+    for m in (513, 700, 1100, 1700, 8191):
+        for n, k, qt in ((4096, 14336, q4), (4096, 14336, q6), (8192, 28672, q4), (5120, 13824, int(QType.Q5_K)), (32, 8192, q4)):
+            p = L._parts_plan(m, n, k, qt)
+            assert p is None or p[0] == "q4" and 2 <= p[2] <= k // 512 and 8 <= p[1] <= L._QMM4_TILES[qt][0] and p[2] * m * n <= L.QMM4_PARTS
+    assert L._parts_plan(700, 4096, 14336, q4) and not L._parts_plan(512, 4096, 14336, q4) and not L._parts_plan(700, 4096, 4096, q4)
+    for m in (128, 333, 416, 512):
+        for c in (c for c in A.candidates(m, 4096, 14336, q6, True) if c[0] == "q4"):
+            assert c[1] <= 12 and (c[2] == 1 or c[2] * m * 4096 <= L.QMM4_PARTS)
+        assert all(c[2] == 1 for c in A.candidates(m, 4096, 14336, q6, False) if c[0] == "q4")
+    W = L.QWeight(4096, 14336, q4, torch.empty(0))
+    W.layout = "t32"
+    assert L._t32_plan(W, 700, L.EPI_ADD_F32, False)[0] == L._t32_plan(W, 700, L.EPI_F32, True)[0] == "q4"
+    assert L._t32_plan(W, 700, L.EPI_F32, False)[-1] == L._t32_plan(W, 700, L.EPI_BF16, False)[-1] == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("qt", FORMATS)
+@pytest.mark.parametrize("M,nb,n,k,splits", [(1, 8, 32, 512, 2), (129, 14, 288, 1280, 2), (333, 12, 544, 2816, 11), (417, 14, 256, 2560, 9)])
+def test_parts_of_k(qt, M, nb, n, k, splits):
+    """Parts of one super-block and of several, a last part with fewer, fewer parts than asked for (9 of ten super-blocks: five of two), more than one turn
+    of the sum's loads, columns past the last whole 256; outputs off 16 bytes; nothing outside the output changes."""
+    raw = Q.random_quantized(np.random.default_rng(M + n), int(qt), n, k).reshape(n, -1)
+    W = L.QWeight.from_ggml(raw, int(qt), n, k, "cuda", t32=True)
+    dense = torch.from_numpy(Q.dequantize(raw.reshape(-1), int(qt), (k, n)).reshape(n, k).copy()).double()
+    assert W.to_t32()
+    x = (torch.randn(M, k, generator=torch.Generator().manual_seed(M)) * 0.5).half()
+    old = torch.randn(M, n, generator=torch.Generator().manual_seed(M + 1))
+    want = x.double() @ dense.t()
+    for epi, zeroed in ((L.EPI_ADD_F32, False), (L.EPI_F32, True)):
+        for off in (0, 1):
+            buf = torch.full((M + 1, n + 4 + 3 * off), -7.0, device="cuda")
+            out = buf[:M, off:off + n]
+            out.copy_(old if epi == L.EPI_ADD_F32 else torch.zeros_like(old))
+            L.run_plan(("q4", nb, splits), W, x.cuda(), epi, out, zeroed)
+            got = out.cpu().double() - (old.double() if epi == L.EPI_ADD_F32 else 0)
+            # weights are rounded to f16 once (2^-11), products and parts summed in fp32
+            assert float((got - want).norm() / want.norm()) < 2 ** -10
+            assert (buf[M:] == -7).all() and (buf[:, off + n:] == -7).all() and (not off or (buf[:, 0] == -7).all())
 
 
 @pytest.mark.gpu
@@ -68,3 +111,5 @@ def test_qmm4_refuses_what_it_does_not_do():
     x = torch.zeros(8, 256, device="cuda", dtype=torch.float16)
     with pytest.raises(RuntimeError):
         L.run_plan(("q4", 8, 1), W, x, L.EPI_ADD_F32, torch.zeros(8, 64, device="cuda"), False)
+    with pytest.raises(ValueError):
+        L.run_plan(("q4", 8, 2), W, x, L.EPI_BF16, torch.zeros(8, 64, device="cuda", dtype=torch.float16), False)
