@@ -2,7 +2,7 @@
 // state_scan). Per sequence and head, over the step's rows in order:
 //     S <- a_t S;   u = c_t (v_t - S^T k_t)  [delta]   or   u = c_t v_t;   S <- S + k_t u^T;   o_t = S^T q_t (+ D v_t)
 // S has N numbers for each of the head's P value columns, fp32, stored column-major: state [slots, H, P, N]. The
-// columns never mix, so a column belongs to LPC neighbouring lanes (4, or the 16 of one DPP row) that each keep NPL of its
+// columns never mix, so a column belongs to LPC neighbouring lanes (4, or the 16 of one DPP row or the 32 of two) that each keep NPL of its
 // numbers (every LPC-th quadruple) in registers for the whole chunk. k_t and q_t are the same for every column of a head: the
 // block stages them in LDS together with the tokens' decays, write strengths and values, 8 or 16 tokens at a time in two
 // buffers; the next tokens' numbers are requested from memory before the current ones are worked on and wait in registers
@@ -40,33 +40,43 @@ template <int CTRL>
 MX_DEV float dpp_move(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
 }
-// sum over the LPC (4 or 16) neighbouring lanes of a column, returned to each of them
+// sum over the DPP rows 2 r and 2 r + 1 (32 lanes), lane by lane, returned to both
+MX_DEV float row_pair_sum(float v) {
+    const u32x2 x = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false));
+    return __uint_as_float(x[0]) + __uint_as_float(x[1]);
+}
+// sum over the LPC (4, 16 or 32) neighbouring lanes of a column, returned to each of them
 template <int LPC>
 MX_DEV float lanes_sum(float v) {
     v = dpp_add<0xB1>(v);  // quad_perm [1, 0, 3, 2]
     v = dpp_add<0x4E>(v);  // quad_perm [2, 3, 0, 1]
-    if constexpr (LPC == 16) {
+    if constexpr (LPC >= 16) {
         v = dpp_add<0x124>(v);  // row_ror 4
         v = dpp_add<0x128>(v);  // row_ror 8
     }
+    if constexpr (LPC == 32) v = row_pair_sum(v);
     return v;
 }
+
+MX_DEV float chains_sum(const float (&c)[1]) { return c[0]; }
+MX_DEV float chains_sum(const float (&c)[2]) { return c[0] + c[1]; }
+MX_DEV float chains_sum(const float (&c)[4]) { return (c[0] + c[1]) + (c[2] + c[3]); }
 
 // what a round of tokens is: one token; up to TB with a test between steps; or whole rounds in a body of their own without that test
 enum { ROUND_ONE = 0, ROUND_ANY = 1, ROUND_WHOLE = 2 };
 
-// grid (column blocks, H, sequences from s0 on); block = 256 threads = 256 / LPC columns
+// grid (column blocks, H, sequences from s0 on); block = 256 threads (512 of 32 lanes a column) = 256 / LPC (16) columns
 template <int NPL, int LPC, bool DELTA, bool CHD, int ROUND>
-__global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk, const float* q, int ldq,
+__global__ __launch_bounds__(LPC == 32 ? 512 : 256) void state_scan_kernel(const float* k, int ldk, const float* q, int ldq,
                                                          const float* v, int ldv, const float* decay, int ldd,
                                                          const float* coef, int ldc, int coef_sigmoid,
                                                          const float* skip, float* state, const int* seq_state,
                                                          const int* positions, int n_dec, const int* pf_cu, float* out,
                                                          int ldo, int H, int G, int N, int P, float q_scale,
                                                          float* nout, int s0) {
-    static_assert(LPC == 4 || LPC == 16, "a column's lanes are a quad or a DPP row");
+    static_assert(LPC == 4 || LPC == 16 || LPC == 32, "a column's lanes are a quad, a DPP row or two");
     constexpr bool ONE = ROUND == ROUND_ONE;
-    constexpr int NT = 256;
+    constexpr int NT = LPC == 32 ? 512 : 256;
     constexpr int NP = NPL * LPC;  // padded N
     constexpr int COLS = NT / LPC;
     constexpr int TB = ONE ? 1 : NP <= 128 ? 16 : 8;  // tokens staged together
@@ -218,6 +228,10 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk
                 if constexpr (CHD) *(float4*)(x.d + j) = *(const float4*)&kq[b][tt][NW - 1][j * LPC + part * 4];
             }
         };
+        // a lane's products are summed in chains of four (quads of lanes: in four chains, 2 % slower)
+        constexpr int NC = LPC == 4 ? 4 : NPL / 4;
+        auto chain = [](int j) { return LPC == 4 ? j & 3 : j >> 2; };
+        auto head = [](int j) { return LPC == 4 ? j & 3 : j & ~3; };  // the first of j's chain
         // whole rounds without a test between steps: those cost nine register moves a step beside the branch
         auto steps = [&](auto whole_c) {
             constexpr bool ALL = decltype(whole_c)::value;
@@ -237,22 +251,22 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk
 #pragma unroll
                         for (int j = 0; j < NPL; ++j) S[j] *= ab[j];
                     }
-                    float d[4] = {0.f, 0.f, 0.f, 0.f};  // four chains of dependent adds
+                    float d[NC];
 #pragma unroll
-                    for (int j = 0; j < NPL; ++j) d[j & 3] += S[j] * kb[j];
-                    const float dk = lanes_sum<LPC>((d[0] + d[1]) + (d[2] + d[3]));
+                    for (int j = 0; j < NPL; ++j) d[chain(j)] = j != head(j) ? fmaf(S[j], kb[j], d[chain(j)]) : S[j] * kb[j];
+                    const float dk = lanes_sum<LPC>(chains_sum(d));
                     u = cf * (CHD ? vv - dk : vv - a * dk);  // (one decay for all rows: taken out of the sum)
                 } else {
                     u = cf * vv;
                 }
-                float o[4] = {0.f, 0.f, 0.f, 0.f};
+                float o[NC];
 #pragma unroll
                 for (int j = 0; j < NPL; ++j) {
                     if constexpr (!(DELTA && CHD)) S[j] *= CHD ? ab[CHD ? j : 0] : a;
                     S[j] += kb[j] * u;
-                    o[j & 3] += S[j] * qb[j];
+                    o[chain(j)] = j != head(j) ? fmaf(S[j], qb[j], o[chain(j)]) : S[j] * qb[j];
                 }
-                os[tt] = (o[0] + o[1]) + (o[2] + o[3]);
+                os[tt] = chains_sum(o);
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
@@ -274,7 +288,7 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk
             const float e0 = a0 + dpp_move<0xB1>(b0), e1 = a1 + dpp_move<0xB1>(b1);  // quad_perm [1, 0, 3, 2]
             const float f0 = part & 2 ? e1 : e0, f1 = part & 2 ? e0 : e1;
             o4[j] = f0 + dpp_move<0x4E>(f1);                                          // quad_perm [2, 3, 0, 1]
-            if constexpr (LPC == 16) {
+            if constexpr (LPC >= 16) {
                 o4[j] = dpp_add<0x124>(o4[j]);  // row_ror 4
                 o4[j] = dpp_add<0x128>(o4[j]);  // row_ror 8
             }
@@ -282,11 +296,12 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const float* k, int ldk
         if constexpr (ONE) {
             const float o = lanes_sum<LPC>(os[0]);
             if (part == 0) put(0, o);
-        } else if constexpr (LPC == 16) {
+        } else if constexpr (LPC >= 16) {
             float o = o4[0];
 #pragma unroll
-            for (int j = 1; j < TB / 4; ++j) o = (part >> 2) == j ? o4[j] : o;
-            put(part, o);
+            for (int j = 1; j < TB / 4; ++j) o = (part >> 2 & 3) == j ? o4[j] : o;
+            if constexpr (LPC == 32) o = row_pair_sum(o);
+            if (part < 16) put(part, o);
         } else {
 #pragma unroll
             for (int j = 0; j < TB / 4; ++j) put(4 * j + part, o4[j]);
@@ -391,9 +406,7 @@ extern "C" int mxh_state_scan(const float* k, int ldk, const float* q, int ldq, 
     const int ldd = decay_rows ? H : 0;
     MXH_CHECK(H > 0 && G > 0 && H % G == 0 && N > 0 && N <= 256 && P > 0 && H <= 65535 && n_seqs <= 65535);
     MXH_CHECK(ldk >= G * N && ldq >= G * N && ldv >= H * P && ldo >= H * P);
-    const int lpc = N <= 32 ? 4 : 16;
-    const int threads = 256;
-    const int cols = threads / lpc;
+    const int cols = N <= 32 ? 64 : 16;  // of a block
     const dim3 grid((P + (nout ? 1 : 0) + cols - 1) / cols, H, n_seqs);
     // Short prompt chunks step token by token as decode rows do (ONE): staging 8 or 16 tokens and reading them ahead costs registers,
     // which are what keeps states in flight. us, staged / one by one: 8 heads of 128 x 256 with channel decays, 64 chunks of 3
@@ -406,24 +419,17 @@ extern "C" int mxh_state_scan(const float* k, int ldk, const float* q, int ldq, 
     const dim3 grid_dec(grid.x, H, n_dec), grid_pf(grid.x, H, apart ? n_pf : n_seqs);
     // Whole rounds take a fifth less time (one chunk of 2900 rows 644 -> 512 us) and more registers, so fewer blocks run on a compute unit: chunks of
     // less than a round gain nothing (20 of 9 rows, 32 heads of 128 x 128 30.1 -> 35.0, 100 decode rows beside 18 rows in three chunks, 24 heads
-    // of 32 x 32 11.9 -> 14.0), and with channel decays and N 65 to 128 one block runs where two did, so only grids that leave it alone anyway
-    // gain (one chunk of 1111 rows 277 -> 238, three of 301 to 1111 365 -> 428, 30 of 64 338 -> 523).
+    // of 32 x 32 11.9 -> 14.0), and with channel decays and N 65 to 128 one block of 16 lanes a column runs where two did, so only grids that leave it
+    // alone anyway gain (one chunk of 1111 rows 277 -> 238, three of 301 to 1111 365 -> 428, 30 of 64 338 -> 523).
     const long blocks_pf = (long)grid_pf.x * H * grid_pf.z;
-    const bool whole = T - n_dec >= 16l * n_pf && !(channel && N > 64 && N <= 128 && blocks_pf > 256);
-#define GO2(NPL, LPC, D_, C_)              \
-    do {                                   \
-        if (one) {                         \
-            GO3(NPL, LPC, D_, C_, ROUND_ONE, grid, 0); \
-            break;                         \
-        }                                  \
-        if (apart) GO3(NPL, LPC, D_, C_, ROUND_ONE, grid_dec, 0); \
-        if (whole) GO3(NPL, LPC, D_, C_, ROUND_WHOLE, grid_pf, apart ? n_dec : 0); \
-        else GO3(NPL, LPC, D_, C_, ROUND_ANY, grid_pf, apart ? n_dec : 0); \
-    } while (0)
-#define GO3(NPL, LPC, D_, C_, O_, GRID, S0)                                                                                  \
-    state_scan_kernel<NPL, LPC, D_, C_, O_><<<GRID, threads, 0, st>>>(k, ldk, q, ldq, v, ldv, decay, ldd, coef, ldc,      \
-                                                                  coef_sigmoid, skip, state, seq_state, positions,    \
-                                                                  n_dec, pf_cu, out, ldo, H, G, N, P, q_scale, nout, S0)
+    // Columns over 32 lanes in blocks of 512 threads: twice the waves with fewer instructions each, since a wave alone on its SIMD issues one
+    // in nine cycles. It wins until the chunks' blocks bring more than two such waves to a SIMD. us, 16 / 32 lanes: one chunk of 1111 rows, 16 heads of 128 x
+    // 128 with the delta rule 190 / 168, without 149 / 110, with channel decays 231 / 192 and 189 / 145; three of 301 to 1111, delta rule 199 / 189 (384
+    // blocks), 64 heads of 128 x 64 without 173 / 166, with it 223 / 244 (768 blocks); four of 200, 16 heads of 128 x 128 (512 blocks) 45.4 / 50.7 and 35.0 /
+    // 35.5, with channel decays 64.9 / 77.7 and 55.6 / 60.7. N above 128 always: 16 numbers a lane leave one block a compute unit (8 heads of 256 x 256, one
+    // chunk of 1111 328 / 271, 30 of 64 rows with channel decays 443 / 336, eight of 250 without 182 / 186).
+    const bool wide = N > 128 || (N > 64 && (long)grid.x * H * n_pf <= (delta || channel ? 384 : 768));
+    const bool full = T - n_dec >= 16l * n_pf, whole = full && !(channel && blocks_pf > 256);
 #define GO(NPL, LPC)                              \
     do {                                          \
         if (delta && channel) GO2(NPL, LPC, true, true); \
@@ -431,6 +437,29 @@ extern "C" int mxh_state_scan(const float* k, int ldk, const float* q, int ldq, 
         else if (channel) GO2(NPL, LPC, false, true); \
         else GO2(NPL, LPC, false, false);         \
     } while (0)
+#define GO2(NPL, LPC, D_, C_)                                                                          \
+    do {                                                                                               \
+        if (one) {                                                                                     \
+            GO3(NPL, LPC, D_, C_, ROUND_ONE, grid, 0);                                                 \
+            break;                                                                                     \
+        }                                                                                              \
+        if (apart) GO3(NPL, LPC, D_, C_, ROUND_ONE, grid_dec, 0);                                      \
+        if constexpr (NPL * LPC > 64) {                                                                \
+            if (NPL == 16 || wide) {                                                                   \
+                if (full) GO3(NPL / 2, 32, D_, C_, ROUND_WHOLE, grid_pf, apart ? n_dec : 0);           \
+                else GO3(NPL / 2, 32, D_, C_, ROUND_ANY, grid_pf, apart ? n_dec : 0);                  \
+                break;                                                                                 \
+            }                                                                                          \
+        }                                                                                              \
+        if constexpr (NPL < 16) {                                                                      \
+            if (NPL * LPC > 64 ? whole : full) GO3(NPL, LPC, D_, C_, ROUND_WHOLE, grid_pf, apart ? n_dec : 0); \
+            else GO3(NPL, LPC, D_, C_, ROUND_ANY, grid_pf, apart ? n_dec : 0);                         \
+        }                                                                                              \
+    } while (0)
+#define GO3(NPL, LPC, D_, C_, O_, GRID, S0)                                                                                  \
+    state_scan_kernel<NPL, LPC, D_, C_, O_><<<GRID, LPC == 32 ? 512 : 256, 0, st>>>(k, ldk, q, ldq, v, ldv, decay, ldd, coef, ldc, \
+                                                                  coef_sigmoid, skip, state, seq_state, positions,    \
+                                                                  n_dec, pf_cu, out, ldo, H, G, N, P, q_scale, nout, S0)
     if (N <= 16) GO(4, 4);
     else if (N <= 32) GO(8, 4);
     else if (N <= 64) GO(4, 16);

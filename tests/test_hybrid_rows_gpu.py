@@ -296,3 +296,25 @@ def test_chunks_of_many_sequences(chunk, window):
         HY.masked_attention(q.to(dev), kc.to(dev), vc.to(dev), rag, H, G, D, D, D ** -0.5, out, chunk=chunk, window=window)
         got[dev] = out.float().cpu()
     assert (got["cuda"] - got["cpu"]).abs().max() <= 2 ** -6 and (got["cuda"] - got["cpu"]).norm() <= 2 ** -8 * got["cpu"].norm()
+
+
+@pytest.mark.parametrize("H,P,chunks", [(48, 64, [33, 16]), (49, 64, [20, 17]), (64, 64, [33, 16, 5, 40]), (7, 300, [15, 1, 31]), (8, 256, [40, 17, 8])])
+@pytest.mark.parametrize("N", [65, 128])
+@pytest.mark.parametrize("delta,channel", [(True, False), (False, True), (False, False), (True, True)])
+def test_lanes_of_a_column(H, P, chunks, N, delta, channel):
+    """Grids around the size where a column's numbers move from 32 lanes to 16 (384 blocks; 768 without delta rule and channel decays) and well beyond
+    it; the bound of test_rounds_of_tokens."""
+    g = torch.Generator().manual_seed(N + H)
+    T, slots = 1 + sum(chunks), list(range(1 + len(chunks)))
+    k, q, v = torch.randn(T, N, generator=g) * N ** -0.5, torch.randn(T, N, generator=g), torch.randn(T, H * P, generator=g)
+    decay, coef = torch.rand(T, H * N if channel else H, generator=g), torch.rand(T, H, generator=g)
+    at = [(i * 3) % 5 for i in range(len(slots))]
+    start = torch.randn(len(slots), H, P, N, generator=g)
+    got = {}
+    for dev in ("cpu", "cuda"):
+        state, out = start.clone().to(dev), torch.zeros(T, H * P, device=dev)
+        HY.state_scan(k.to(dev), q.to(dev), v.to(dev), decay.to(dev), coef.to(dev), None, state, _rag(1, chunks, at, slots, dev), out,
+                      H, 1, N, P, delta, channel, 0.5, False, None)
+        got[dev] = [out.cpu(), state.cpu()]
+    for a, b in zip(got["cuda"], got["cpu"]):
+        assert (a - b).abs().max() <= 2e-5 * b.abs().max()
