@@ -26,14 +26,6 @@ struct D16Args {
     int part_rows;
 };
 
-// x / (1 + exp(-x)): the exponent in two parts (x log2 e and what its rounding left), the reciprocal to 1 ulp. Largest relative error
-// 2.6e-7 over -87 .. 87 (x / (1.f + expf(-x)) has 4.5e-7 over -8 .. 8, 1.4e-6 over -30 .. 30); infinities and NaN as there. 10 instructions
-// for some 30: a gated 256 x 256 tile has 128 of these a lane, and nothing runs beside them.
-MX_DEV float d16_silu(float x) {
-    const float y = fminf(x, 128.f), m = y * -1.44269504f, lo = fmaf(y, -1.925963033e-8f, fmaf(y, -1.44269504f, -m));
-    return x * __builtin_amdgcn_rcpf(fmaf(__builtin_amdgcn_exp2f(m), fmaf(lo, 0.69314718f, 1.f), 1.f));
-}
-
 template <int EPI, bool F16, int MI, int NJ>
 __global__ __launch_bounds__(256, 1) void dense16_kernel(D16Args a) {
     using T = G16T<MI, NJ>;
@@ -99,7 +91,7 @@ __global__ __launch_bounds__(256, 1) void dense16_kernel(D16Args a) {
 #pragma unroll
                     for (int e = 0; e < FL; ++e) {
                         const int j = q * (FL / 2) + (e >> 2) * 2;
-                        v[e] = d16_silu(acc[i][j][e & 3] + gb[e]) * (acc[i][j + 1][e & 3] + ub[e]);
+                        v[e] = silu_gate_f(acc[i][j][e & 3] + gb[e]) * (acc[i][j + 1][e & 3] + ub[e]);
                     }
 #pragma unroll
                     for (int e = 0; e < FL; e += 2) w[e / 2] = pack_act2<F16>(v[e], v[e + 1]);
