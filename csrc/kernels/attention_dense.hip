@@ -213,13 +213,15 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dense_t_kernel(const uint16_t
                                                               int Hkv, const int* __restrict__ qlen_b,
                                                               const int* __restrict__ klen_b, int causal, float scale,
                                                               int kv_rows, const float* __restrict__ rbias, int rb_ld,
-                                                              const int* __restrict__ cu) {
+                                                              const int* __restrict__ cu, const int* __restrict__ blocks) {
     constexpr int FT = AT_KEYS, IMG = FT * D * 2;
     constexpr int NCH = FT * D / 8 / (64 * NW);  // 16-byte chunks of an image per thread
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int h = lane >> 5, col = lane & 31;
-    const int b = blockIdx.z, head = blockIdx.y, kvh = head / (Hq / Hkv), q0 = blockIdx.x * (32 * NW);
+    // `blocks`: the (sequence, first query) of a block, in the order they are to start
+    const int b = blocks ? blocks[2 * blockIdx.y] : blockIdx.z, head = blocks ? blockIdx.x : blockIdx.y, kvh = head / (Hq / Hkv);
+    const int q0 = blocks ? blocks[2 * blockIdx.y + 1] : blockIdx.x * (32 * NW);
     // ragged batches: sequence b's rows are cu[b] .. cu[b + 1], keys and queries alike
     const size_t q_row = cu ? (size_t)cu[b] : (size_t)b * Sq, k_row = cu ? (size_t)cu[b] : (size_t)b * kv_rows;
     const int qlen = cu ? cu[b + 1] - cu[b] : qlen_b ? qlen_b[b] : Sq;
@@ -347,9 +349,10 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dense_t_kernel(const uint16_t
 template <int D, int NW, bool F16>
 static int launch_dense_t(const uint16_t* q, int q_stride, const uint16_t* k, int k_stride, const uint16_t* v, int v_stride,
                           uint16_t* o, int o_stride, int B, int Sq, int Sk, int Hq, int Hkv, const int* qlen, const int* klen,
-                          int causal, float scale, int kv_rows, const float* rbias, int rb_ld, const int* cu, hipStream_t st) {
+                          int causal, float scale, int kv_rows, const float* rbias, int rb_ld, const int* cu, const int* blocks, int n_blocks,
+                          hipStream_t st) {
     constexpr int LDS = 4 * 64 * D * 2;
-    const dim3 grid((Sq + 32 * NW - 1) / (32 * NW), Hq, B);
+    const dim3 grid = blocks ? dim3(Hq, n_blocks) : dim3((Sq + 32 * NW - 1) / (32 * NW), Hq, B);
 #define DT(GEN_)                                                                                                              \
     do {                                                                                                                      \
         static const hipError_t once = hipFuncSetAttribute((const void*)attn_dense_t_kernel<D, NW, F16, GEN_>,                \
@@ -357,7 +360,7 @@ static int launch_dense_t(const uint16_t* q, int q_stride, const uint16_t* k, in
         if (once != hipSuccess) return (int)once;                                                                             \
         attn_dense_t_kernel<D, NW, F16, GEN_><<<grid, 64 * NW, LDS, st>>>(q, q_stride, k, k_stride, v, v_stride, o, o_stride, \
                                                                           Sq, Sk, Hq, Hkv, qlen, klen, causal, scale, kv_rows, \
-                                                                          rbias, rb_ld, cu);                                  \
+                                                                          rbias, rb_ld, cu, blocks);                          \
     } while (0)
     if (rbias || !(scale > 0.f)) DT(true);
     else DT(false);
@@ -367,13 +370,13 @@ static int launch_dense_t(const uint16_t* q, int q_stride, const uint16_t* k, in
 
 static int dense_t(const uint16_t* q, int q_stride, const uint16_t* k, int k_stride, const uint16_t* v, int v_stride, uint16_t* o,
                    int o_stride, int B, int Sq, int Sk, int Hq, int Hkv, int D, const int* qlen, const int* klen, int causal,
-                   float scale, int kv_rows, const float* rbias, int rb_ld, const int* cu, hipStream_t st) {
+                   float scale, int kv_rows, const float* rbias, int rb_ld, const int* cu, const int* blocks, int n_blocks, hipStream_t st) {
     // two waves for ragged heads of 64, where the last block of each sequence is part empty (48 texts of 23-401 rows, 12 heads:
     // 23.7 us against 29.8; at 401 rows each 80 against 69); four waves elsewhere, whatever the grid (1500 rows, 20 heads:
     // 32.6 against 40.5; 4500 rows of 24 heads of 128: 343 against 515)
     int rc = 0;
 #define DTL(D_, NW_) launch_dense_t<D_, NW_, F16>(q, q_stride, k, k_stride, v, v_stride, o, o_stride, B, Sq, Sk, Hq, Hkv, qlen, \
-                                                  klen, causal, scale, kv_rows, rbias, rb_ld, cu, st)
+                                                  klen, causal, scale, kv_rows, rbias, rb_ld, cu, blocks, n_blocks, st)
     MX_ACT_DISPATCH(rc = D == 128 ? DTL(128, 4) : cu ? DTL(64, 2) : DTL(64, 4));
 #undef DTL
     return rc;
@@ -393,20 +396,22 @@ extern "C" int mxk_attn_dense(const uint16_t* q, int q_stride, const uint16_t* k
     if ((q_stride | k_stride | v_stride) & 7) return (int)hipErrorInvalidValue;
     if (D != 512)
         return dense_t(q, q_stride, k, k_stride, v, v_stride, o, o_stride, B, Sq, Sk, Hq, Hkv, D, qlen, klen, causal, scale,
-                       kv_rows, rbias, rb_ld, nullptr, st);
+                       kv_rows, rbias, rb_ld, nullptr, nullptr, 0, st);
     MX_ACT_DISPATCH((attn_dense_kernel<512, F16><<<dim3((Sq + 63) / 64, Hq, B), 256, 0, st>>>(
         q, q_stride, k, k_stride, v, v_stride, o, o_stride, Sq, Sk, Hq, Hkv, qlen, klen, causal, scale, kv_rows, rbias, rb_ld)));
     MXK_CHECK_LAUNCH();
 }
 
 // Rows packed without padding (BERT): sequence b of B has rows cu[b] .. cu[b + 1] (at most Smax) of q, k, v and o, and sees
-// its first klen[b] keys; D in {64, 128}.
+// its first klen[b] keys; D in {64, 128}. blocks (or null): n_blocks pairs (b, first query), one for every 64 (D 64) or 128 queries that a sequence
+// has, in the order they start. A block's time is its keys', so the longest come first: in the order of 48 texts of 23 to 401 rows from the
+// shortest, 12 heads, the last ones' seven key tiles ran after all else (24.5 us).
 extern "C" int mxk_attn_dense_ragged(const uint16_t* q, int q_stride, const uint16_t* k, int k_stride, const uint16_t* v,
                                      int v_stride, uint16_t* o, int o_stride, int B, int Smax, int H, int D, const int* cu,
-                                     const int* klen, float scale, hipStream_t st) {
+                                     const int* klen, float scale, const int* blocks, int n_blocks, hipStream_t st) {
     if (B <= 0 || Smax <= 0) return 0;
-    if ((D != 64 && D != 128) || B > 65535 || !cu || !klen) return (int)hipErrorInvalidValue;
+    if ((D != 64 && D != 128) || B > 65535 || !cu || !klen || (blocks && (n_blocks <= 0 || n_blocks > 65535))) return (int)hipErrorInvalidValue;
     if ((q_stride | k_stride | v_stride) & 7) return (int)hipErrorInvalidValue;
     return dense_t(q, q_stride, k, k_stride, v, v_stride, o, o_stride, B, Smax, Smax, H, H, D, nullptr, klen, 0, scale, 0, nullptr,
-                   0, cu, st);
+                   0, cu, blocks, n_blocks, st);
 }

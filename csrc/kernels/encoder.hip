@@ -567,7 +567,7 @@ bool enc_width_ok(int H) { return H > 0 && H % 8 == 0 && H <= 4096; }
 
 extern "C" int mxk_attn_dense_ragged(const uint16_t* q, int q_stride, const uint16_t* k, int k_stride, const uint16_t* v,
                                      int v_stride, uint16_t* o, int o_stride, int B, int Smax, int H, int D, const int* cu,
-                                     const int* klen, float scale, hipStream_t st);
+                                     const int* klen, float scale, const int* blocks, int n_blocks, hipStream_t st);
 
 extern "C" int mxk_enc_embed(const int* ids, int rows, const float* tok, const float* pos, const float* typ, const float* g,
                              const float* b, int H, float eps, uint16_t* x, hipStream_t st) {
@@ -641,7 +641,7 @@ extern "C" int mxk_enc_layers(const void* const* w, int n_layers, uint16_t* x, i
         if (!rc && one) {
             MX_ACT_DISPATCH((rc = enc_attn_gemm<F16>(qkv, klen, scale, heads, at(2), parts, rows, H, st)));
         } else if (!rc) {
-            rc = mxk_attn_dense_ragged(qkv, 3 * H, qkv + H, 3 * H, qkv + 2 * H, 3 * H, attn, H, B, Smax, heads, H / heads, cu, klen, scale, st);
+            rc = mxk_attn_dense_ragged(qkv, 3 * H, qkv + H, 3 * H, qkv + 2 * H, 3 * H, attn, H, B, Smax, heads, H / heads, cu, klen, scale, nullptr, 0, st);
             if (!rc) MX_ACT_DISPATCH((rc = enc_gemm<F16, ENC_PART>(attn, at(2), nullptr, parts, rows, H, H, st)));
         }
         if (!rc && norms) {
@@ -659,10 +659,10 @@ extern "C" int mxk_enc_layers(const void* const* w, int n_layers, uint16_t* x, i
 
 // The same layers by dense16.hip's tiles. plan: tile of the qkv product; tile and parts of K of the output product; tile of the up product; tile and
 // parts of the down product: 1, 2, 3, 4 or 8 parts of fp32 sums, or 0: stored in 16 bits with its bias. H and F multiples of 64; parts
-// [most parts][rows][H] where there are any.
+// [most parts][rows][H] where there are any. blocks: as mxk_attn_dense_ragged takes them.
 extern "C" int mxk_enc_layers_tiled(const void* const* w, int n_layers, uint16_t* x, int rows, int B, int Smax, const int* cu, const int* klen, int H,
                                     int heads, int F, float scale, float eps, uint16_t* qkv, uint16_t* attn, float* parts, uint16_t* up,
-                                    const int* plan, hipStream_t st) {
+                                    const int* plan, const int* blocks, int n_blocks, hipStream_t st) {
     if (rows <= 0 || n_layers <= 0) return 0;
     if (!enc_width_ok(H) || H % 64 || F <= 0 || F % 64 || heads <= 0 || H % heads) return (int)hipErrorInvalidValue;
     for (int l = 0; l < n_layers; ++l, w += 12) {
@@ -677,7 +677,7 @@ extern "C" int mxk_enc_layers_tiled(const void* const* w, int n_layers, uint16_t
             return rc ? rc : enc_parts_ln(np, parts, at(i + 1), x, x, rows, g, b, H, eps, st);
         };
         int rc = mx_dense16_enc(D16_ACT, plan[0], x, H, at(0), rows, 3 * H, H, at(1), qkv, 3 * H, 1, nullptr, st);
-        if (!rc) rc = mxk_attn_dense_ragged(qkv, 3 * H, qkv + H, 3 * H, qkv + 2 * H, 3 * H, attn, H, B, Smax, heads, H / heads, cu, klen, scale, st);
+        if (!rc) rc = mxk_attn_dense_ragged(qkv, 3 * H, qkv + H, 3 * H, qkv + 2 * H, 3 * H, attn, H, B, Smax, heads, H / heads, cu, klen, scale, blocks, n_blocks, st);
         if (!rc) rc = add_ln(attn, H, plan[1], plan[2], 2);
         if (!rc) rc = mx_dense16_enc(D16_GELU, plan[3], x, H, at(6), rows, F, H, at(7), up, F, 1, nullptr, st);
         if (!rc) rc = add_ln(up, F, plan[4], plan[5], 8);

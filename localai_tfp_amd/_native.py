@@ -66,8 +66,8 @@ KERNEL_SIGS = {
     "mxk_enc_gelu": [P, C.c_longlong, P],
     "mxk_enc_pool": [P, P, P, I, I, I, I, P, P],
     "mxk_enc_layers": [P, I, P, I, I, I, P, P, I, I, I, F, F, P, P, P, P, P],
-    "mxk_enc_layers_tiled": [P, I, P, I, I, I, P, P, I, I, I, F, F, P, P, P, P, P, P],
-    "mxk_attn_dense_ragged": [P, I, P, I, P, I, P, I, I, I, I, I, P, P, F, P],
+    "mxk_enc_layers_tiled": [P, I, P, I, I, I, P, P, I, I, I, F, F, P, P, P, P, P, P, I, P],
+    "mxk_attn_dense_ragged": [P, I, P, I, P, I, P, I, I, I, I, I, P, P, F, P, I, P],
     "mxk_qgemv": [I, I, P, P, P, P, I, I, I, P, I, P],
     "mxk_dequant_rows": [I, P, P, P, I, I, P, P, I, P],
     "mxk_rope_kv": [P, P, P, P, P, F, I, I, I, I, I, I, P, P, P, I, P, P, F, I, I, P],

@@ -77,6 +77,17 @@ BERT_BASE = BertConfig()
 BERT_TINY = BertConfig(vocab=400, hidden=128, n_layers=2, n_heads=2, ffn=512, max_pos=128, name="bert-tiny")
 
 
+def attn_blocks(rows: np.ndarray, queries: int) -> np.ndarray | None:
+    """The attention's blocks of `queries` rows of each text, [blocks, 2] = (text, first row), the longest texts' first. None: more than a grid
+    takes (they run in the texts' order)."""
+    order = np.argsort(-rows, kind="stable")
+    n = -(-rows[order] // queries)
+    first = np.cumsum(n) - n
+    if first[-1] + n[-1] > 65535:
+        return None
+    return np.stack([np.repeat(order, n), (np.arange(n.sum()) - np.repeat(first, n)) * queries], 1).astype(np.int32)
+
+
 class BertModel:
     def __init__(self, cfg: BertConfig, device="cpu"):
         self.cfg = cfg
@@ -189,7 +200,10 @@ class BertModel:
         cu = np.zeros(B + 1, np.int64)
         np.cumsum(rows, out=cu[1:])
         R, S = int(cu[-1]), int(rows.max())
-        img = np.zeros(3 * R + 2 * B + 1, np.int32)
+        tiled = H % 64 == 0 and Fd % 64 == 0 and R > few_rows(H, Fd)
+        blocks = attn_blocks(rows, 64 if H // cfg.n_heads == 64 else 128) if tiled and B > 1 else None
+        nb = 0 if blocks is None else blocks.shape[0]
+        img = np.zeros(3 * R + 2 * B + 1 + 2 * nb, np.int32)
         tok, pos, typ = img[:R], img[R:2 * R], img[2 * R:3 * R]
         pos[:] = np.arange(R) - np.repeat(cu[:-1], rows)
         if last:
@@ -211,16 +225,18 @@ class BertModel:
         if S > positions.shape[0]:
             raise IndexError(f"text of {S} tokens, {positions.shape[0]} positions")
         img[3 * R:3 * R + B + 1] = cu
-        img[3 * R + B + 1:] = lens
+        img[3 * R + B + 1:3 * R + 2 * B + 1] = lens
+        if nb:
+            img[3 * R + 2 * B + 1:] = blocks.reshape(-1)
         img = torch.from_numpy(img).to(dev)
-        cu_d, len_d = img[3 * R:3 * R + B + 1], img[3 * R + B + 1:]
+        cu_d, len_d = img[3 * R:3 * R + B + 1], img[3 * R + B + 1:3 * R + 2 * B + 1]
         x = torch.empty(R, H, dtype=self.dtype, device=dev)
         attn = torch.empty(R, H, dtype=self.dtype, device=dev)
         N.ensure_act(self.dtype)
         st = N.stream_ptr()
         N.kcall("mxk_enc_embed", img.data_ptr(), R, *ptrs[:5], H, float(cfg.eps), x.data_ptr(), st)
         scale = 1.0 / math.sqrt(H // cfg.n_heads)
-        if H % 64 == 0 and Fd % 64 == 0 and R > few_rows(H, Fd):
+        if tiled:
             plan, keep = encoder_plan(R, H, Fd), R <= small_rows(H, Fd)
             plan = [n if i not in (2, 5) or n > 1 or keep else 0 for i, n in enumerate(plan)]  # 0 parts: 16-bit sums
             most = max(plan[2], plan[5])
@@ -231,7 +247,8 @@ class BertModel:
                 plan[2] = plan[5] = int(keep)
                 parts = torch.empty(R, H, dtype=torch.float32, device=dev) if keep else None
             N.kcall("mxk_enc_layers_tiled", (ctypes.c_void_p * (12 * cfg.n_layers))(*ptrs[5:]), cfg.n_layers, x.data_ptr(), R, B, S, cu_d.data_ptr(), len_d.data_ptr(), H,
-                    cfg.n_heads, Fd, scale, float(cfg.eps), qkv.data_ptr(), attn.data_ptr(), N.ptr(parts), up.data_ptr(), (ctypes.c_int * 6)(*plan), st)
+                    cfg.n_heads, Fd, scale, float(cfg.eps), qkv.data_ptr(), attn.data_ptr(), N.ptr(parts), up.data_ptr(), (ctypes.c_int * 6)(*plan),
+                    img.data_ptr() + 4 * (3 * R + 2 * B + 1) if nb else None, nb, st)
             return x, cu_d, len_d
         if R <= small_rows(H, Fd):
             parts = torch.empty(5, R, H, dtype=torch.float32, device=dev)  # fp32 sums of up to four parts of K, and a norm's rows
@@ -250,7 +267,7 @@ class BertModel:
             qkv = linear(x, wq, bq)
             q = qkv.data_ptr()
             N.kcall("mxk_attn_dense_ragged", q, 3 * H, q + 2 * H, 3 * H, q + 4 * H, 3 * H, attn.data_ptr(), H, B, S,
-                    cfg.n_heads, H // cfg.n_heads, cu_d.data_ptr(), len_d.data_ptr(), scale, st)
+                    cfg.n_heads, H // cfg.n_heads, cu_d.data_ptr(), len_d.data_ptr(), scale, None, 0, st)
             add_ln(linear(attn, wo, bo), g1, b1)
             up = linear(x, wu, bu)
             N.kcall("mxk_enc_gelu", up.data_ptr(), up.numel(), st)

@@ -3,6 +3,7 @@ micro-batching, and the HTTP surface (/v1/embeddings, /v1/rerank) — reference 
 core/http/app_test.go embeddings + rerank cases, backend/python/rerankers/test.py."""
 import math
 
+import numpy as np
 import pytest
 import torch
 import yaml
@@ -286,6 +287,31 @@ def test_tiled_layers_match_fp32(tile, dtype, monkeypatch):
         ids = [list(range(10, 10 + n)) for n in lens]
         got, want = g.embed(ids).cpu(), c.embed(ids)
         assert "mxk_enc_layers_tiled" in used and (got - want).abs().max() < (5e-3 if dtype == torch.float16 else 4e-2), (lens, po, pd)
+
+
+def test_attention_blocks_cover_each_row_once():
+    for rows in ([1], [64, 65, 63, 1], [5, 300, 300, 128, 129], [1] * 70):
+        for q in (64, 128):
+            b = BM.attn_blocks(np.array(rows), q)
+            assert sorted(map(tuple, b.tolist())) == sorted((i, f) for i, n in enumerate(rows) for f in range(0, n, q))
+            assert (np.diff(np.array(rows)[b[:, 0]]) <= 0).all() and b.dtype == np.int32
+    assert BM.attn_blocks(np.full(65535, 1), 64).shape == (65535, 2) and BM.attn_blocks(np.array([64] * 65535 + [1]), 64) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads", [2, 4])
+def test_texts_of_blocks_edges_in_any_order(heads, monkeypatch):
+    """Heads of 128 and 64: texts of no token, of one, around whole blocks of 64 and 128 rows; the bound of test_packed_rows_match_fp32."""
+    cfg = BM.BertConfig(vocab=400, hidden=256, n_layers=2, n_heads=heads, ffn=512, max_pos=300, name="t")
+    get = BM.synthetic_bert(cfg, 5)
+    g, c = BM.BertModel.load(cfg, get, "cuda:0"), BM.BertModel.load(cfg, get, "cpu")
+    monkeypatch.setattr(BM, "ENC_FEW_ROWS", 0)
+    batches = [[1, 63, 64, 65, 128, 129, 257], [129, 0, 2], [64, 64], [300, 1, 127], [65]]
+    ids = [[[(7 * i + j) % 390 + 5 for j in range(n)] for i, n in enumerate(lens)] for lens in batches]
+    got = [g.embed(x) for x in ids]
+    for e, x in zip(got, ids):
+        want = c.embed(x)
+        assert (e.cpu() - want)[[i for i, t in enumerate(x) if t]].abs().max() < 5e-3
 
 
 @pytest.mark.gpu
