@@ -15,12 +15,13 @@
 // With parts > 1 (decode rows of long contexts) grid.z splits a row's visible keys into partitions whose
 // (max, sum, unnormalised output) go to a workspace; attn_merge_kernel combines them in a fixed order and adds the sink.
 //
-// bf16 pools with head sizes of 64 / 128 (or 96 for both) run on the matrix cores instead: attn_chunk_mfma_kernel for
+// bf16 pools with head sizes of 64 / 128 (or 96 for both) run on the matrix cores instead: attn_chunk_t_kernel and attn_chunk_mfma_kernel for
 // prompt chunks, attn_decode_mfma_kernel for single new tokens (both further down, with their fragment layouts).
 //
 // Other long prompt chunks take another route (ops/hybrid.py): kv_gather_kernel copies the chunk's visible keys and values
 // from the pages into head-major matrices, head_transpose_kernel does the same for the queries, the library computes
 // the score and value products, and masked_softmax_kernel turns raw scores into masked, sink-normalised weights.
+#include "../attn_tile.h"
 #include "../mx_common.h"
 
 namespace {
@@ -548,6 +549,178 @@ __global__ __launch_bounds__(256) void attn_chunk_mfma_kernel(const bf16_t* __re
     }
 }
 
+// attn_chunk_t_kernel: the same chunks where neither bias, kept tokens, P2 nor fewer value heads ask for more (heads of 64 or 128 both), on
+// attn_tile.h's tiles: 128 columns a workgroup, column = query * (H / G) + query head of one key / value head, 32 of them a wave, so that a key or
+// value fragment read from LDS serves 32 columns where it served 16 rows, a column's softmax is one lane's but for one exchange, and the
+// weights never pass through LDS. Tiles are double-buffered, the next one stored and the one after it requested beside the products; page
+// numbers are looked up a tile before the rows. Key heads are the grid's first dimension: with eight of them each has an XCD's L2 to itself.
+// Chunks of 301 / 578 / 1111 rows, 32 / 8 heads of 128: 116 -> 38 us, bound by the longest's chain of 18 tiles; errors against 64 bits are the same
+// to four digits.
+template <int D, bool O16>
+__global__ __launch_bounds__(256, 2) void attn_chunk_t_kernel(const bf16_t* __restrict__ q, int ldq, const bf16_t* __restrict__ kc,
+                                                              const bf16_t* __restrict__ vc, int bs, int bs_sh, const int* __restrict__ table,
+                                                              int bt_stride, AttnSeqs sq, void* __restrict__ out, int ldo, int H, int G,
+                                                              float scale, int chunk, int window, int sink, float out_scale, AttnExtra ex) {
+    constexpr int FT = AT_KEYS, IMG = FT * D * 2, NCH = FT * D / 8 / 256;
+    constexpr float LOG2E_ = 1.4426950408889634f;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    int s = 0;
+    while (s + 1 < sq.count && sq.first[s + 1] <= (int)blockIdx.y) ++s;
+    const int p0 = sq.p0[s], n = sq.n[s], last = sq.first[s + 1] - 1;
+    table += (size_t)sq.bt[s] * bt_stride;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int h = lane >> 5, col = lane & 31;
+    const int rep = H / G, RQ = 128 / rep, kvh = blockIdx.x;
+    const int q0 = (last - (int)blockIdx.y) * RQ;  // (a chunk's last rows see the most keys: first)
+    const int r = wave * 32 + col, qi = q0 + r / rep, hq = kvh * rep + r % rep;
+    const bool real = r < RQ * rep && qi < n;
+    auto lo_of = [&](int pos) { return chunk > 0 ? pos / chunk * chunk : window > 0 ? max(0, pos - window + 1) : 0; };
+    const int kv_end = p0 + min(n, q0 + RQ), kt_begin = lo_of(p0 + q0);
+    const int n_tiles = (kv_end - kt_begin + FT - 1) / FT;
+    const int qpos = p0 + qi, lo = lo_of(qpos);
+    const int wq0 = p0 + min(q0 + wave * 32 / rep, n - 1), wq1 = p0 + min(q0 + min(RQ - 1, (wave * 32 + 31) / rep), n - 1);  // the wave's rows
+    const int wlo0 = lo_of(wq0), wlo1 = lo_of(wq1);
+
+    u32x4 qf[D / 16];  // Q^T as B operand: lane = column (past the end a real row, not stored), 8 dims 16 ks + 8 h
+    {
+        const bf16_t* qp = q + (size_t)(sq.row[s] + min(qi, n - 1)) * ldq + (size_t)hq * D + 8 * h;
+#pragma unroll
+        for (int ks = 0; ks < D / 16; ++ks) qf[ks] = *(const u32x4*)(qp + 16 * ks);
+    }
+    f32x16 o[D / 32];
+#pragma unroll
+    for (int i = 0; i < D / 32; ++i)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) o[i][j] = 0.f;
+    // the sink starts the maximum and the sum (one of a column's two lanes)
+    float m_run = sink ? sink_score(ex, hq) * LOG2E_ : -INFINITY, l_run = sink && h == 0 ? 1.f : 0.f;
+    const float qs = scale * LOG2E_, cap = ex.softcap * LOG2E_, cap_k = ex.softcap > 0.f ? 2.f * qs / ex.softcap : 0.f;
+
+    // a tile's chunks: the page and the row in it a tile before the numbers, the numbers a tile before they are stored; rows past the last
+    // key repeat it, no column sees them
+    u32x4 kr[NCH], vr[NCH];
+    int blk[NCH], off[NCH];
+    auto find_rows = [&](int t) {
+        int bi[NCH];
+#pragma unroll
+        for (int j = 0; j < NCH; ++j) {
+            off[j] = min(kt_begin + t * FT + (int)(threadIdx.x + j * 256) / (D / 8), kv_end - 1);
+            bi[j] = bs_sh >= 0 ? off[j] >> bs_sh : off[j] / bs;
+        }
+#pragma unroll
+        for (int j = 0; j < NCH; ++j) {
+            blk[j] = table[bi[j]];
+            off[j] -= bi[j] * bs;
+        }
+    };
+    auto load_chunk = [&](int j) {
+        const size_t at = (((size_t)blk[j] * bs + off[j]) * G + kvh) * D + threadIdx.x % (D / 8) * 8;
+        kr[j] = *(const u32x4*)(kc + at);
+        vr[j] = *(const u32x4*)(vc + at);
+    };
+    auto store_k = [&](int buf, int j) {
+        const int id = threadIdx.x + j * 256;
+        *(u32x4*)(smem + buf * (2 * IMG) + at_k_off<D>(id / (D / 8), id % (D / 8))) = kr[j];
+    };
+    auto store_v = [&](int buf, int j) {
+        const int id = threadIdx.x + j * 256, c = id % (D / 8);
+        *(u32x4*)(smem + buf * (2 * IMG) + IMG + at_v_off<D>(id / (D / 8), c >> 1) + 16 * (c & 1)) = vr[j];
+    };
+    int vo[D / 32];
+    at_v_lane<D>(lane, vo);
+    auto piece = [&](int t, int i) {  // tile t + 1 to the other buffer, tile t + 2 requested
+        if (i >= 2 * NCH) return;
+        if (i % 2 == 0) store_k((t + 1) & 1, i / 2);
+        else {
+            store_v((t + 1) & 1, i / 2);
+            load_chunk(i / 2);
+        }
+    };
+    auto work = [&](int t, auto more) {
+        const char* kb = smem + (t & 1) * (2 * IMG);
+        const char* vb = kb + IMG;
+        const int kt0 = kt_begin + t * FT;
+        f32x16 sc[2];
+        if constexpr (decltype(more)::value) at_scores<D, false, D / 64>(kb, h, col, qf, sc, [&](int ks) { piece(t, ks); });
+        else at_scores<D, false, D / 64>(kb, h, col, qf, sc);
+        if (kt0 > wq1 || kt0 + FT - 1 < wlo0) return;  // (uniform per wave) none of its rows sees the tile
+        u32x4 vf[4][D / 32];
+        __builtin_amdgcn_sched_barrier(0);
+        at_read_v<D>(vb, vo, 0, vf);
+        __builtin_amdgcn_sched_barrier(0);
+        if (ex.softcap > 0.f) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int j = 0; j < 16; ++j) sc[u][j] = capped_log2(sc[u][j], cap, cap_k);
+        }
+        if (kt0 + FT - 1 > wq0 || kt0 < wlo1) {
+            const int d = qpos - kt0 - 4 * h, dl = lo - kt0 - 4 * h;
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int j = 0; j < 16; ++j) {
+                    const int kp = 32 * u + 8 * (j >> 2) + (j & 3);
+                    if (kp > d || kp < dl) sc[u][j] = -INFINITY;
+                }
+        }
+        at_softmax_v<D, false>(vb, vo, sc, ex.softcap > 0.f ? 1.f : qs, vf, o, m_run, l_run);
+    };
+    find_rows(0);
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) load_chunk(j);
+    find_rows(min(1, n_tiles - 1));
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) {
+        store_k(0, j);
+        store_v(0, j);
+    }
+    if (n_tiles > 1) {
+#pragma unroll
+        for (int j = 0; j < NCH; ++j) load_chunk(j);
+        find_rows(min(2, n_tiles - 1));
+    }
+    __syncthreads();
+    for (int t = 0; t < n_tiles - 1; ++t) {
+        // the other buffer was last read while tile t - 1 was worked on, before the barrier that ended that round
+        work(t, std::true_type{});
+        find_rows(min(t + 3, n_tiles - 1));
+        __syncthreads();
+    }
+    work(n_tiles - 1, std::false_type{});
+
+    l_run = at_half_sum(l_run);
+    if (!real) return;
+    const float inv = l_run > 0.f ? out_scale / l_run : 0.f;
+    const size_t orow = (size_t)(sq.row[s] + qi), at = orow * ldo + (size_t)hq * D + 4 * h;
+    const bool wide = !(((uintptr_t)out & (O16 ? 7 : 15)) | (ldo & 3));
+#pragma unroll
+    for (int mt = 0; mt < D / 32; ++mt)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            f32x4 v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = o[mt][4 * g + e] * (inv * gate_factor(ex, (long)orow, hq, 32 * mt + 8 * g + 4 * h + e));
+            if constexpr (O16) {
+                bf16_t* p = (bf16_t*)out + at + 32 * mt + 8 * g;
+                if (wide) {
+                    *(u32x2*)p = (u32x2){pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) p[e] = f32_to_bf16(v[e]);
+                }
+            } else {
+                float* p = (float*)out + at + 32 * mt + 8 * g;
+                if (wide) {
+                    *(f32x4*)p = v;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) p[e] = v[e];
+                }
+            }
+        }
+}
+
 // attn_decode_mfma_kernel: single new tokens on the matrix cores (bf16 pools, head sizes as above, up to 16 query heads
 // per key / value head). grid (sequences, G, partitions), one wave per workgroup: the 16 rows of its tile are the
 // query heads that share key / value head blockIdx.y (rows beyond H / G are zero), all at the sequence's newest
@@ -1004,6 +1177,14 @@ extern "C" int mxh_attention_mfma(const void* q, int ldq, const void* kc, const 
     const int GW = rep % 4 == 0 ? 4 : rep % 2 == 0 ? 2 : 1;
     const int RT = 4 / GW;
     MXH_CHECK(H / GW <= 65535);
+    // attn_chunk_t_kernel takes what it can: of 90 shapes (six head layouts, 16 to 2000 rows, up to 4000 keys) it is the faster one or even, us, 16 rows a
+    // wave / here: 32 / 8 heads of 128 333 rows 27.3 / 15.8, 1111 82.7 / 36.3, 2000 216 / 62, 416 behind 3584 keys 120 / 52, four of 200 22.9 / 14.3; up to
+    // 64 keys even
+    long rows = 0;
+    for (int i = 0; i < count; ++i) rows += seqs[4 * i + 2];
+    const bool tiles = dk == dv && dk != 96 && !bias && !p2 && gv == G && (!keep || !window) && rep <= 32 && scale > 0.f &&
+                       rows / (128 / rep) + count <= 65535;
+    const int RQ = tiles ? 128 / rep : RT * 16;  // rows of a workgroup
     for (int i = 0; i < count; ++i) MXH_CHECK(seqs[4 * i] >= 0 && seqs[4 * i + 1] >= 0 && seqs[4 * i + 2] >= 0 && seqs[4 * i + 3] >= 0);
     for (int i0 = 0; i0 < count; i0 += ATTN_SEQS) {
         const int some = min(count - i0, ATTN_SEQS);
@@ -1024,11 +1205,28 @@ extern "C" int mxh_attention_mfma(const void* q, int ldq, const void* kc, const 
             sq.p0[k] = c[1];
             sq.n[k] = c[2];
             sq.row[k] = c[3];
-            blocks += (c[2] + RT * 16 - 1) / (RT * 16);
+            blocks += (c[2] + RQ - 1) / RQ;
             MXH_CHECK(blocks <= 0x7fffffff);
             sq.first[k + 1] = (int)blocks;
         }
         if (blocks == 0) continue;
+        if (tiles) {
+            const dim3 gt(G, (unsigned)blocks);
+            const int sh = bs & (bs - 1) ? -1 : __builtin_ctz(bs);
+#define GO(D_, O_)                                                                                                                             \
+    do {                                                                                                                                       \
+        static const hipError_t attr = hipFuncSetAttribute((const void*)attn_chunk_t_kernel<D_, O_>, hipFuncAttributeMaxDynamicSharedMemorySize, 512 * D_); \
+        if (attr != hipSuccess) return (int)attr;                                                                                              \
+        attn_chunk_t_kernel<D_, O_><<<gt, 256, 512 * D_, st>>>((const bf16_t*)q, ldq, (const bf16_t*)kc, (const bf16_t*)vc, bs, sh, table,     \
+                                                               bt_stride, sq, out, ldo, H, G, scale, chunk, window, sink, out_scale, ex);      \
+    } while (0)
+            if (dk == 64 && o16) GO(64, true);
+            else if (dk == 64) GO(64, false);
+            else if (o16) GO(128, true);
+            else GO(128, false);
+#undef GO
+            continue;
+        }
         const dim3 grid((unsigned)blocks, H / GW);
 #define GO3(K_, V_, O_, P_)                                                                                       \
     attn_chunk_mfma_kernel<K_, V_, O_, P_><<<grid, 256, 0, st>>>((const bf16_t*)q, ldq, (const bf16_t*)kc,             \

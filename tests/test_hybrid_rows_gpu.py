@@ -318,3 +318,43 @@ def test_lanes_of_a_column(H, P, chunks, N, delta, channel):
         got[dev] = [out.cpu(), state.cpu()]
     for a, b in zip(got["cuda"], got["cpu"]):
         assert (a - b).abs().max() <= 2e-5 * b.abs().max()
+
+
+@pytest.mark.parametrize("lens,pre,H,G,D,bs,kw", [
+    ([33], [0], 8, 2, 128, 16, {}), ([100, 17], [30, 283], 6, 2, 64, 10, dict(sink=True)), ([70], [430], 4, 4, 128, 16, dict(chunk=128, sink=True)),
+    ([150], [250], 12, 1, 64, 16, dict(window=70)), ([64, 65, 16], [0, 135, 1], 32, 1, 128, 8, dict(window=33, softcap=5.0, sink="each")),
+    ([200], [60], 3, 1, 128, 16, dict(chunk=50)), ([40, 0, 63], [0, 0, 65], 8, 8, 64, 16, dict(gate=1)),
+    ([90], [0], 8, 4, 128, 16, dict(gate=128, softcap=20.0, dtype=torch.float32)), ([128, 129], [1, 62], 5, 1, 64, 4, dict(dtype=torch.float32))])
+@pytest.mark.parametrize("off", [0, 1])
+def test_chunks_on_key_tiles(lens, pre, H, G, D, bs, kw, off):
+    """Query heads that fill a workgroup's columns and that do not, key counts around whole tiles, chunk borders and window edges inside a tile, pages
+    that are no power of two, sinks, caps, gates, outputs that allow wide stores and that do not. bf16 weights (and outputs): 2^-8 of numbers of order 1."""
+    g, T, kw = torch.Generator().manual_seed(D + H), sum(lens), dict(kw)
+    dt = kw.pop("dtype", torch.bfloat16)
+    need = [-(-(p + n) // bs) for p, n in zip(pre, lens)]
+    order = torch.randperm(sum(need), generator=g).tolist()
+    tables, at = torch.zeros(len(lens), max(need), dtype=torch.int32), 0
+    for i, n in enumerate(need):
+        tables[i, :n] = torch.tensor(order[at:at + n], dtype=torch.int32)
+        at += n
+    q = torch.randn(T, H * D, generator=g).bfloat16()
+    kc, vc = (torch.randn(sum(need), bs, G * D, generator=g).bfloat16() for _ in range(2))
+    if kw.get("sink") == "each":
+        kw["sink"] = torch.randn(H, generator=g)
+    if "gate" in kw:
+        kw["gate"] = torch.randn(T, H * kw["gate"], generator=g)
+    cu, ctx = [sum(lens[:i]) for i in range(len(lens) + 1)], [p + n for p, n in zip(pre, lens)]
+    i32 = lambda x, dev: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    got = {}
+    for dev in ("cpu", "cuda"):
+        rag = HY.Ragged(types.SimpleNamespace(T=T, n_decode=0, positions=i32([0] * T, dev), seq_state=None, slots=None, pf_cu_q=i32(cu, dev),
+                                              pf_q_lens_host=lens, pf_ctx_lens_host=ctx, pf_block_tables=tables.to(dev), pf_ctx_lens=i32(ctx, dev),
+                                              dec_block_tables=None, dec_seq_lens=None, dec_max_len=0))
+        # (the reference in fp32 throughout)
+        x = [t.float() if dev == "cpu" else t.to(dev) for t in (q, kc, vc)]
+        buf = torch.full((T + 1, H * D + 4 + 3 * off), 7.0, device=dev, dtype=torch.float32 if dev == "cpu" else dt)
+        HY.masked_attention(*x, rag, H, G, D, D, D ** -0.5, buf[:T, off:off + H * D], out_scale=0.7,
+                            **{k: v.to(dev) if torch.is_tensor(v) else v for k, v in kw.items()})
+        got[dev] = buf[:T, off:off + H * D].float().cpu()
+        assert (buf[T] == 7).all() and (buf[:, off + H * D:] == 7).all() and (not off or (buf[:, 0] == 7).all())
+    assert (got["cuda"] - got["cpu"]).norm() <= 2 ** -8 * got["cpu"].norm() and (got["cuda"] - got["cpu"]).abs().max() <= 2 ** -6
