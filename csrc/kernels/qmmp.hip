@@ -9,7 +9,7 @@
 #include "qmmp_impl.h"
 
 // qa, qb: Q4_K + Q6_K, Q5_K + Q6_K, Q3_K + Q5_K. epi 0 or 2 as mxk_qmm2 (splits 1 for 0). kind 2: qmm2 tiles (p0, p1, p2) = (wm, ks, wn),
-// (4, 2, 1) or (2, 2, 1); kind 0: qmmr tiles (wm, gw, kw), (1, 1, 4), (1, 2, 4), (1, 4, 4) or (2, 2, 4). C 4-byte aligned.
+// (4, 2, 1), (3, 2, 1) or (2, 2, 1); kind 0: qmmr tiles (wm, gw, kw), (1, 1, 4), (1, 2, 4), (1, 4, 4) or (2, 2, 4). C 4-byte aligned.
 extern "C" int mxk_qmm_pair(int qa, int qb, int epi, int kind, int p0, int p1, int p2, const uint16_t* A, int lda, const uint8_t* Wa, int Na,
                             const uint8_t* Wb, int Nb, int M, int K, int splits, float* C, int ldc, hipStream_t st) {
     if (M <= 0) return 0;

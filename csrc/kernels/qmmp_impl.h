@@ -68,7 +68,7 @@ static int dispatch_qmmp(int kind, int p0, int p1, int p2, const QpArgs& a, hipS
         static bool once = false;                                                                                                     \
         return launch_qmmp(qmmpr_kernel<QA, QB, WM_, GW_, KW_, EPI>, 64 * GW_ * KW_, 32 * GW_, 32 * WM_, QrGeom<WM_, GW_, KW_>::LDS, once, a, st); \
     }
-    QP2(4, 2) QP2(2, 2) QPR(1, 1, 4) QPR(1, 2, 4) QPR(1, 4, 4) QPR(2, 2, 4)
+    QP2(4, 2) QP2(3, 2) QP2(2, 2) QPR(1, 1, 4) QPR(1, 2, 4) QPR(1, 4, 4) QPR(2, 2, 4)
 #undef QP2
 #undef QPR
     return (int)hipErrorInvalidValue;

@@ -498,7 +498,7 @@ def _qmatmul_t32(W: QWeight, x, epi: int, out, xq, xds, M: int, out_zeroed: bool
 
 # qmmp.hip: two weights by the same rows in one launch, formats and (kind, wm | wm, ks | gw, wn | kw) compiled
 PAIR_QTYPES = {(int(QType.Q4_K), int(QType.Q6_K)), (int(QType.Q5_K), int(QType.Q6_K)), (int(QType.Q3_K), int(QType.Q5_K))}
-PAIR_PLANS = (("q2", 4, 2, 1), ("q2", 2, 2, 1), ("qr", 1, 1, 4), ("qr", 1, 2, 4), ("qr", 1, 4, 4), ("qr", 2, 2, 4))
+PAIR_PLANS = (("q2", 4, 2, 1), ("q2", 3, 2, 1), ("q2", 2, 2, 1), ("qr", 1, 1, 4), ("qr", 1, 2, 4), ("qr", 1, 4, 4), ("qr", 2, 2, 4))
 
 
 def pair_ok(parts) -> bool:
