@@ -73,7 +73,7 @@ __global__ __launch_bounds__(LPC == 32 ? 512 : 256) void state_scan_kernel(const
                                                          const float* skip, float* state, const int* seq_state,
                                                          const int* positions, int n_dec, const int* pf_cu, float* out,
                                                          int ldo, int H, int G, int N, int P, float q_scale,
-                                                         float* nout, int s0) {
+                                                         float* nout, int s0, int n_pf, int rows_pf) {
     static_assert(LPC == 4 || LPC == 16 || LPC == 32, "a column's lanes are a quad, a DPP row or two");
     constexpr bool ONE = ROUND == ROUND_ONE;
     constexpr int NT = LPC == 32 ? 512 : 256;
@@ -99,6 +99,11 @@ __global__ __launch_bounds__(LPC == 32 ? 512 : 256) void state_scan_kernel(const
         n = pf_cu[i + 1] - pf_cu[i];
     }
     if (n <= 0) return;
+    // the longest chunks end the launch, so chunks above the mean issue before the others' waves of a SIMD: 301 / 578 / 1111 rows, 16 heads of 128 x 128
+    // with the delta rule 202 -> 177 us, 64 of 128 x 64 without 184 -> 169
+    if constexpr (!ONE) {
+        if ((long)n * n_pf > rows_pf) __builtin_amdgcn_s_setprio(2);
+    }
     const int slot = seq_state[s];
     const bool fresh = positions[row0] == 0 || slot < 0;
     const int PT = P + (nout ? 1 : 0);  // state columns of a head
@@ -425,7 +430,7 @@ extern "C" int mxh_state_scan(const float* k, int ldk, const float* q, int ldq, 
     // Columns over 32 lanes in blocks of 512 threads: twice the waves with fewer instructions each, since a wave alone on its SIMD issues one
     // in nine cycles. It wins until the chunks' blocks bring more than two such waves to a SIMD. us, 16 / 32 lanes: one chunk of 1111 rows, 16 heads of 128 x
     // 128 with the delta rule 190 / 168, without 149 / 110, with channel decays 231 / 192 and 189 / 145; three of 301 to 1111, delta rule 199 / 189 (384
-    // blocks), 64 heads of 128 x 64 without 173 / 166, with it 223 / 244 (768 blocks); four of 200, 16 heads of 128 x 128 (512 blocks) 45.4 / 50.7 and 35.0 /
+    // blocks), 64 heads of 128 x 64 without 173 / 166, with it 223 / 244 (768 blocks; these before chunks had priorities); four of 200, 16 heads of 128 x 128 (512 blocks) 45.4 / 50.7 and 35.0 /
     // 35.5, with channel decays 64.9 / 77.7 and 55.6 / 60.7. N above 128 always: 16 numbers a lane leave one block a compute unit (8 heads of 256 x 256, one
     // chunk of 1111 328 / 271, 30 of 64 rows with channel decays 443 / 336, eight of 250 without 182 / 186).
     const bool wide = N > 128 || (N > 64 && (long)grid.x * H * n_pf <= (delta || channel ? 384 : 768));
@@ -459,7 +464,7 @@ extern "C" int mxh_state_scan(const float* k, int ldk, const float* q, int ldq, 
 #define GO3(NPL, LPC, D_, C_, O_, GRID, S0)                                                                                  \
     state_scan_kernel<NPL, LPC, D_, C_, O_><<<GRID, LPC == 32 ? 512 : 256, 0, st>>>(k, ldk, q, ldq, v, ldv, decay, ldd, coef, ldc, \
                                                                   coef_sigmoid, skip, state, seq_state, positions,    \
-                                                                  n_dec, pf_cu, out, ldo, H, G, N, P, q_scale, nout, S0)
+                                                                  n_dec, pf_cu, out, ldo, H, G, N, P, q_scale, nout, S0, n_pf, T - n_dec)
     if (N <= 16) GO(4, 4);
     else if (N <= 32) GO(8, 4);
     else if (N <= 64) GO(4, 16);
