@@ -358,3 +358,30 @@ def test_chunks_on_key_tiles(lens, pre, H, G, D, bs, kw, off):
         got[dev] = buf[:T, off:off + H * D].float().cpu()
         assert (buf[T] == 7).all() and (buf[:, off + H * D:] == 7).all() and (not off or (buf[:, 0] == 7).all())
     assert (got["cuda"] - got["cpu"]).norm() <= 2 ** -8 * got["cpu"].norm() and (got["cuda"] - got["cpu"]).abs().max() <= 2 ** -6
+
+
+@pytest.mark.parametrize("groups,group", [(3, 16), (5, 60), (2, 64), (3, 68), (16, 128), (1, 256), (2, 260), (1, 512), (3, 516), (1, 2048), (1, 2052), (2, 4096), (1, 4100), (1, 8192)])
+@pytest.mark.parametrize("T,gate_first,act,den,dtype", [(33, True, "silu", False, torch.bfloat16), (5, False, "silu", True, torch.float32),
+                                                       (7, False, "sigmoid", False, torch.bfloat16), (1, True, "sigmoid", True, torch.float32)])
+def test_group_norms_of_quadruples(groups, group, T, gate_first, act, den, dtype):
+    """Groups around each number of threads, rows whose groups end inside a block, weights of a group and of a row; aligned rows and rows a number off
+    (the scalar form). fp32 sums of up to 8192 squares in another order: below 2^-17 of the result; bf16 outputs, of eight
+    significant bits, round by up to half of 2^-7 of it more."""
+    g, C = torch.Generator().manual_seed(group), groups * group
+    y, gate = torch.randn(T, C, generator=g), 3 * torch.randn(T, C, generator=g)
+    gate[0, :4] = torch.tensor([-200.0, 200.0, 0.0, -90.0])
+    dn = dict(den=torch.randn(T, groups, generator=g), den_min=torch.rand(T, groups, generator=g) + 0.1, den_eps=1e-3) if den else {}
+    for off in (0, 1):
+        for wlen in (group, C):
+            w = torch.rand(wlen, generator=g) + 0.5
+            got = {}
+            for dev in ("cpu", "cuda"):
+                yb, gb = (torch.zeros(T, C + 8, device=dev) for _ in range(2))
+                yb[:, off:off + C], gb[:, off:off + C] = y.to(dev), gate.to(dev)
+                out = torch.full((T + 1, C + 8), 7.0, device=dev, dtype=torch.float32 if dev == "cpu" else dtype)
+                HY.gated_group_norm(yb[:, off:off + C], gb[:, off:off + C], w.to(dev), 1e-6, group, out[:T, off:off + C], gate_first=gate_first, out_scale=0.7,
+                                    act=act, **{k: v.to(dev) if torch.is_tensor(v) else v for k, v in dn.items()})
+                got[dev] = out[:T, off:off + C].float().cpu()
+                assert (out[T] == 7).all() and (out[:, off + C:] == 7).all() and (not off or (out[:, 0] == 7).all())
+            bound = 2 ** -17 + (2 ** -8 if dtype == torch.bfloat16 else 0)
+            assert ((got["cuda"] - got["cpu"]).abs() <= bound * got["cpu"].abs() + 1e-7).all()
