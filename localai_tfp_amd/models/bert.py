@@ -204,7 +204,7 @@ class BertModel:
         blocks = attn_blocks(rows, 64 if H // cfg.n_heads == 64 else 128) if tiled and B > 1 else None
         nb = 0 if blocks is None else blocks.shape[0]
         # pinned, so that the copy is queued and the host goes on to the next call while this one runs (one text of 19 tokens after
-        # another 365 us a call before, when each copy waited for the call before it). A capture refuses pageable memory as it did: its
+        # another 374 -> 347 us a call: before, each copy waited for the call before it). A capture refuses pageable memory as it did: its
         # graph would read the image again.
         queued = not torch.cuda.is_current_stream_capturing()
         host = torch.zeros(3 * R + 2 * B + 1 + 2 * nb, dtype=torch.int32, pin_memory=queued)

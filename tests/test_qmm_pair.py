@@ -33,6 +33,35 @@ def test_rule_and_tuned_plans():
     assert not L.qmatmul_pair((a, b), torch.zeros(8, 4096), torch.zeros(8, 6144))
 
 
+def test_pairs_that_are_expanded():
+    q4, q6 = int(QType.Q4_K), int(QType.Q6_K)
+    take = lambda m, na=5120, nb=1024, k=4096: L._pair_expands(na, nb, k, q4, q6, m)  # noqa: E731
+    assert take(8191) and take(5000) and not take(2600) and not take(L.X16_MIN_M - 1) and not take(512) and not take(1040)
+    assert not take(8191, 32768, 8192) and take(8191, 9216, 1024, 8192)  # (scratch)
+
+
+@pytest.mark.gpu
+def test_expanded_pair(monkeypatch):
+    """Both weights in one launch, rows and columns off its tiles, nothing outside; what cannot be expanded is left to two launches."""
+    M, na, nb, k = 300, 160, 96, 512
+    ws, dense = [], []
+    for i, (qt, n) in enumerate(zip(PAIRS[1], (na, nb))):
+        raw = Q.random_quantized(np.random.default_rng(i), int(qt), n, k).reshape(n, -1)
+        w = L.QWeight.from_ggml(raw, int(qt), n, k, "cuda", t32=True)
+        assert w.to_t32()
+        ws.append(w)
+        dense.append(torch.from_numpy(Q.dequantize(raw.reshape(-1), int(qt), (k, n)).reshape(n, k).copy()).double())
+    x = (torch.randn(M, k, generator=torch.Generator().manual_seed(M)) * 0.5).half()
+    want = x.double() @ torch.cat(dense).t()
+    monkeypatch.setattr(L, "_pair_expands", lambda *a: True)
+    buf = torch.full((M + 1, na + nb + 8), -7.0, device="cuda")
+    assert L.qmatmul_pair(ws, x.cuda(), buf[:M, :na + nb])
+    # weights are rounded to f16 once (2^-11), products summed in fp32
+    assert float((buf[:M, :na + nb].cpu().double() - want).norm() / want.norm()) < 2 ** -10
+    assert (buf[M:] == -7).all() and (buf[:, na + nb:] == -7).all()
+    assert not L.qmatmul_pair(ws, x.cuda(), torch.zeros(M, na + nb + 1, device="cuda")[:, 1:])
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("pair", PAIRS)
 @pytest.mark.parametrize("M", [5, 33, 64, 129, 300])
