@@ -564,8 +564,8 @@ def qmatmul_pair(parts, x: torch.Tensor, out: torch.Tensor) -> bool:
     a, b = parts
     if out.shape != (x.shape[0], a.N + b.N) or x.shape[1] != a.K or x.shape[0] == 0 or not x.is_cuda or not out.is_cuda:
         return False
-    if _pair_expands(a.N, b.N, a.K, int(a.qtype), int(b.qtype), x.shape[0]):
-        return _run_pair_x16(a, b, x, out)
+    if _pair_expands(a.N, b.N, a.K, int(a.qtype), int(b.qtype), x.shape[0]) and _run_pair_x16(a, b, x, out):
+        return True
     plan = _pair_plan(a, b, x.shape[0])
     if plan is None:
         return False

@@ -42,7 +42,7 @@ def test_pairs_that_are_expanded():
 
 @pytest.mark.gpu
 def test_expanded_pair(monkeypatch):
-    """Both weights in one launch, rows and columns off its tiles, nothing outside; what cannot be expanded is left to two launches."""
+    """Both weights in one launch, rows and columns off its tiles, nothing outside; rows off 16 bytes run as they did."""
     M, na, nb, k = 300, 160, 96, 512
     ws, dense = [], []
     for i, (qt, n) in enumerate(zip(PAIRS[1], (na, nb))):
@@ -59,7 +59,9 @@ def test_expanded_pair(monkeypatch):
     # weights are rounded to f16 once (2^-11), products summed in fp32
     assert float((buf[:M, :na + nb].cpu().double() - want).norm() / want.norm()) < 2 ** -10
     assert (buf[M:] == -7).all() and (buf[:, na + nb:] == -7).all()
-    assert not L.qmatmul_pair(ws, x.cuda(), torch.zeros(M, na + nb + 1, device="cuda")[:, 1:])
+    off = torch.zeros(M, na + nb + 1, device="cuda")[:, 1:]
+    assert not L._run_pair_x16(*ws, x.cuda(), off) and L.qmatmul_pair(ws, x.cuda(), off)
+    assert float((off.cpu().double() - want).norm() / want.norm()) < 2 ** -10
 
 
 @pytest.mark.gpu
